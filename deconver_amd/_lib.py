@@ -389,3 +389,20 @@ def get_library() -> NdcLibrary:
                 if os.environ.get("DECONVER_NDC_MATRIX", "0") == "1":
                     _library.matrix_kernels(True)
     return _library
+
+
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
+_native = None
+
+
+def get_native():
+    """The compiled autograd nodes (``csrc/ndc_torch.cpp``), on top of :func:`get_library`'s HIP
+    library; raises if either has not been built."""
+    global _native
+    if _native is None:
+        get_library()
+        if not os.path.exists(NATIVE_PATH):
+            raise NdcError(f"{NATIVE_PATH} is missing: build it with `python -m deconver_amd.build`.")
+        from . import _native as module
+        _native = module
+    return _native

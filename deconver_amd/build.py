@@ -1,6 +1,6 @@
 """In-tree build of the HIP library (and, on request, of the host checker).
 
-    python -m deconver_amd.build            # libdeconver_ndc.so for gfx950
+    python -m deconver_amd.build            # libdeconver_ndc.so for gfx950, _native.so (autograd nodes)
     python -m deconver_amd.build --hostcheck  # + libndc_hostcheck.so (CPU test-suite)
 """
 
@@ -42,6 +42,26 @@ def build_hip(extra_flags=()) -> str:
     return out
 
 
+def build_native() -> str:
+    """The autograd nodes (``csrc/ndc_torch.cpp``): host code against PyTorch and the HIP library,
+    which it finds next to itself."""
+    import sysconfig
+
+    import torch
+
+    out = os.path.join(_HERE, "_native.so")
+    base = os.path.dirname(torch.__file__)
+    include = [os.path.join(base, "include"), os.path.join(base, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    libs = ["c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python"]
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-w", "-DTORCH_EXTENSION_NAME=_native",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+          *["-isystem" + d for d in include], os.path.join(CSRC, "ndc_torch.cpp"), "-o", out,
+          "-L" + _HERE, "-ldeconver_ndc", "-L" + os.path.join(base, "lib"), *["-l" + n for n in libs],
+          "-Wl,-rpath,$ORIGIN"])
+    return out
+
+
 def build_hostcheck(sanitize: bool = False) -> str:
     out = os.path.join(_HERE, "libndc_hostcheck.so")
     flags = ["-O1", "-g", "-fsanitize=address,undefined"] if sanitize else ["-O2"]
@@ -57,6 +77,7 @@ def main(argv=None) -> None:
     args = ap.parse_args(argv)
     if not args.no_hip:
         print(build_hip())
+        print(build_native())
     if args.hostcheck:
         print(build_hostcheck())
 

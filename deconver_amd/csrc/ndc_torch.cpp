@@ -1,0 +1,987 @@
+// The autograd nodes of the package, natively: shape checks, output allocation, the calls into
+// libdeconver_ndc.so and the backward formulas of the NDC update, the 1x1 projections, the MLP,
+// the norms and the 2-tap regrouping (deconver/deconvolution/functional.py:97-207 and
+// deconver/layers of the reference are what these nodes stand for).
+//
+// Why native: a step of these networks is some 600 kernel launches, and on small tensors it is
+// bound by what the host does between them.  With the nodes written in Python (an autograd
+// Function each, its operands marshalled through ctypes) a launch cost about 20 us of host time:
+// a training step on one 32^3 volume took 12.7 ms for 5.7 ms of kernels, one forward + backward
+// of a 32-channel 64^2 layer 0.48 ms for 0.15 ms of kernels.  The arithmetic stays behind the C
+// ABI of include/deconver_ndc.h; nothing here computes on tensors except through it, the
+// library GEMMs of shapes the streaming GEMM does not take, and a few float32 sums of partial
+// results.
+#include <torch/extension.h>
+
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
+
+#include "../../include/deconver_ndc.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ---------------------------------------------------------------------------- helpers
+
+void check(int status, const char *what)
+{
+    TORCH_CHECK(status == 0, what, " failed: ", ndc_status_string(status), " (status ", status, ")");
+}
+
+int dtype_tag(const Tensor &t)
+{
+    if (t.scalar_type() == at::kFloat) return NDC_F32;
+    if (t.scalar_type() == at::kBFloat16) return NDC_BF16;
+    TORCH_CHECK_TYPE(false, "NDC kernels store activations as float32 or bfloat16, got ", t.scalar_type());
+}
+
+// What every node works under: the device of its tensors current, autocast off (operands are
+// already in the dtype the node computes in), and no autograd recording inside.
+struct Scope {
+    c10::OptionalDeviceGuard device;
+    c10::impl::ExcludeDispatchKeyGuard autocast;
+    at::AutoDispatchBelowADInplaceOrView below;
+    void *stream;
+    explicit Scope(const Tensor &t)
+        : device(t.device()), autocast(c10::autocast_dispatch_keyset),
+          stream((void *)c10::hip::getCurrentHIPStream(t.device().index()).stream())
+    {
+        TORCH_CHECK(t.is_cuda(), "the HIP kernels run on GPU tensors only");
+    }
+};
+
+const void *ptr(const Tensor &t) { return t.defined() ? t.const_data_ptr() : nullptr; }
+void *out_ptr(const Tensor &t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
+const float *fptr(const Tensor &t) { return (const float *)ptr(t); }
+float *out_fptr(const Tensor &t) { return (float *)out_ptr(t); }
+
+Tensor f32_vector(const OptTensor &t)
+{
+    if (!t || !t->defined()) return Tensor();
+    return t->detach().to(at::kFloat).contiguous();
+}
+
+Tensor empty(at::IntArrayRef size, const Tensor &like) { return at::empty(size, like.options()); }
+Tensor empty_f32(at::IntArrayRef size, const Tensor &like)
+{
+    return at::empty(size, like.options().dtype(at::kFloat));
+}
+
+bool wants_grad(const Tensor &t) { return t.defined() && t.requires_grad(); }
+bool wants_grad(const OptTensor &t) { return t && wants_grad(*t); }
+
+// Which gradients the engine asks for, by forward argument.  (The engine counts only the
+// arguments that are tensors.)
+struct Needs {
+    std::vector<int> edge;
+    int count = 0;
+    void arg(bool defined) { edge.push_back(defined ? count++ : -1); }
+    std::vector<bool> ask(AutogradContext *ctx) const
+    {
+        std::vector<bool> out(edge.size());
+        for (size_t i = 0; i < edge.size(); ++i) out[i] = edge[i] >= 0 && ctx->needs_input_grad(edge[i]);
+        return out;
+    }
+};
+
+// Gradients of a node that is differentiable once: under create_graph they come back attached
+// to a node that refuses the second differentiation instead of silently dropping its terms.
+variable_list once(variable_list grads, bool recording, const variable_list &gouts)
+{
+    if (!recording) return grads;
+    bool any = false;
+    for (auto &g : gouts) any = any || wants_grad(g);
+    if (!any) return grads;
+    auto err = std::make_shared<torch::autograd::DelayedError>(
+        "trying to differentiate twice a function that was marked with @once_differentiable", (int64_t)grads.size());
+    variable_list marked;
+    for (auto &g : grads) marked.push_back(g.defined() ? g.detach().requires_grad_(true) : g);
+    return (*err)(std::move(marked));
+}
+
+// ---------------------------------------------------------------------------- layouts
+
+bool channels_last(const Tensor &t)
+{
+    if ((t.dim() != 4 && t.dim() != 5) || t.is_contiguous()) return false;
+    return t.is_contiguous(t.dim() == 4 ? at::MemoryFormat::ChannelsLast : at::MemoryFormat::ChannelsLast3d);
+}
+
+int64_t voxels(const Tensor &t)
+{
+    int64_t n = 1;
+    for (int64_t d = 2; d < t.dim(); ++d) n *= t.size(d);
+    return n;
+}
+
+Tensor channel_first(const Tensor &t, void *stream)
+{
+    if (t.is_contiguous()) return t;
+    if (!channels_last(t)) return t.contiguous();
+    Tensor out = empty(t.sizes(), t);
+    check(ndc_relayout(ptr(t), out_ptr(out), t.size(0), t.size(1), voxels(t), dtype_tag(t), 0, stream), "ndc_relayout");
+    return out;
+}
+
+Tensor to_channels_last(const Tensor &t, void *stream)
+{
+    Tensor out = at::empty(t.sizes(), t.options().memory_format(
+                                          t.dim() == 4 ? at::MemoryFormat::ChannelsLast : at::MemoryFormat::ChannelsLast3d));
+    check(ndc_relayout(ptr(t), out_ptr(out), t.size(0), t.size(1), voxels(t), dtype_tag(t), 1, stream), "ndc_relayout");
+    return out;
+}
+
+// ---------------------------------------------------------------------------- projections
+
+// The matrix W (cout x cin) of a 1x1 projection as it lies in memory: rows of W, or rows of its
+// transpose (a transposed convolution's weight).  Any floating dtype.
+struct Matrix {
+    Tensor m;
+    bool transposed;
+    Matrix(const Tensor &w, bool t) : m(w.detach()), transposed(t)
+    {
+        if (m.dim() != 2) m = m.reshape({m.size(0), -1});
+        if (!m.is_contiguous()) m = m.contiguous();
+    }
+    int64_t cout() const { return m.size(transposed ? 1 : 0); }
+    int64_t cin() const { return m.size(transposed ? 0 : 1); }
+    // (rows of W, columns of W) as a dense operand of a library GEMM, in `dtype`
+    Tensor dense(at::ScalarType dtype, bool transpose) const
+    {
+        Tensor w = m.to(dtype);
+        return transpose != transposed ? w.t() : w;
+    }
+};
+
+bool streaming_gemm(const Tensor &x, int64_t cout, bool act_or_keep)
+{
+    if (x.scalar_type() != at::kBFloat16 || (x.size(1) > 256 && act_or_keep)) return false;
+    return ndc_pointwise_gemm_supported(x.size(1), cout, x.size(2), NDC_BF16) != 0;
+}
+
+// W (or W^T) in the order the streaming GEMM reads it
+Tensor pack(const Matrix &w, bool transpose, const Tensor &like, void *stream)
+{
+    Tensor m = w.m;
+    if (m.scalar_type() != at::kFloat && m.scalar_type() != at::kBFloat16) m = m.to(at::kBFloat16);
+    const int64_t cin = transpose ? w.cout() : w.cin(), cout = transpose ? w.cin() : w.cout();
+    Tensor frag = at::empty({cin * cout}, like.options().dtype(at::kBFloat16));
+    check(ndc_pointwise_pack(ptr(m), dtype_tag(m), transpose != w.transposed, out_ptr(frag), cin, cout, stream),
+          "ndc_pointwise_pack");
+    return frag;
+}
+
+Tensor batched(const Tensor &w, int64_t B) { return w.unsqueeze(0).expand({B, w.size(0), w.size(1)}); }
+
+// W x per sample
+Tensor project(const Matrix &w, const Tensor &x, void *stream)
+{
+    const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
+    Tensor z = empty({B, cout, n}, x);
+    if (streaming_gemm(x, cout, false)) {
+        Tensor frag = pack(w, false, x, stream);
+        check(ndc_pointwise_gemm(ptr(x), ptr(frag), nullptr, nullptr, out_ptr(z), nullptr, B, w.cin(), cout, n, NDC_ACT_NONE,
+                                 NDC_BF16, stream), "ndc_pointwise_gemm");
+        return z;
+    }
+    // one batched GEMM, the weight shared by the samples through a zero stride
+    at::bmm_out(z, batched(w.dense(x.scalar_type(), false), B), x);
+    return z;
+}
+
+// W^T gz per sample, onto `accumulate` if given (which may be overwritten), zero where mask <= 0
+Tensor project_back(const Matrix &w, const Tensor &gz, Tensor accumulate, const Tensor &mask, void *stream)
+{
+    const int64_t B = gz.size(0), n = gz.size(2), cin = w.cin(), cout = w.cout();
+    Tensor gx;
+    if (cout == 1) {
+        // an outer product, i.e. a broadcast multiplication at the memory rate (as a GEMM it ran
+        // at a fifth of it)
+        gx = at::mul(gz, w.m.reshape({1, -1, 1}).to(gz.scalar_type()));
+        if (accumulate.defined()) gx = accumulate.add_(gx);
+    } else if (streaming_gemm(gz, cin, false)) {
+        Tensor frag = pack(w, true, gz, stream);
+        gx = empty({B, cin, n}, gz);
+        if (mask.defined())
+            check(ndc_pointwise_gemm_masked(ptr(gz), ptr(frag), nullptr, ptr(accumulate), ptr(mask), out_ptr(gx), B, cout, cin,
+                                            n, NDC_BF16, stream), "ndc_pointwise_gemm_masked");
+        else
+            check(ndc_pointwise_gemm(ptr(gz), ptr(frag), nullptr, ptr(accumulate), out_ptr(gx), nullptr, B, cout, cin, n,
+                                     NDC_ACT_NONE, NDC_BF16, stream), "ndc_pointwise_gemm");
+        return gx;
+    } else {
+        Tensor wt = batched(w.dense(gz.scalar_type(), true), B);
+        if (accumulate.defined()) {
+            gx = accumulate.baddbmm_(wt, gz);
+        } else {
+            gx = empty({B, cin, n}, gz);
+            at::bmm_out(gx, wt, gz);
+        }
+    }
+    return mask.defined() ? gx.mul_(mask.gt(0)) : gx;
+}
+
+// Equal chunks the voxel axis is cut into for the weight-gradient GEMM: a power of two that
+// divides n, chunks of at least `least` voxels, at most 128 GEMMs in the batch.
+int64_t weight_grad_chunks(int64_t batch, int64_t n, int64_t least)
+{
+    int64_t s = 1;
+    while (s < 64 && n % (2 * s) == 0 && n / (2 * s) >= least && batch * 2 * s <= 128) s *= 2;
+    return s;
+}
+
+// Chunk counts from timings with batch 2 in bfloat16 (64 chunks at 128^3; 32 at 64^3, where 64
+// cost 0.05 ms more on the 128 x 128 result; 16 at 32^3: 0.056 ms against 0.11-0.13 ms unchunked;
+// none at 16^3) and batch 8 in float32 (none up to 256^2 voxels: there every chunked form was
+// slower).
+int64_t weight_grad_plan(int64_t batch, int64_t n, bool half)
+{
+    if (half) return n < (1 << 15) ? 1 : weight_grad_chunks(batch, n, n < (1 << 17) ? 2048 : 8192);
+    return n < (1 << 17) ? 1 : weight_grad_chunks(batch, n, 2048);
+}
+
+// sum_b gz[b] x[b]^T: the weight gradient, (cout, cin) -- or (cin, cout) for a weight stored
+// transposed --, added up in float32.  Long rows are cut into equal chunks of the voxel axis that
+// become batch entries (strided views, no copies); bfloat16 operands hand out their float32
+// accumulators.
+Tensor weight_grad(const Tensor &gz, const Tensor &x, const Matrix &w, at::IntArrayRef shape, at::ScalarType dtype)
+{
+    const Tensor &a = w.transposed ? x : gz, &c = w.transposed ? gz : x;
+    const int64_t B = a.size(0), n = a.size(2), rows = a.size(1), cols = c.size(1);
+    const bool half = a.scalar_type() == at::kBFloat16;
+    const int64_t s = weight_grad_plan(B, n, half);
+    Tensor parts;
+    if (s == 1) {
+        parts = half ? at::bmm(a, c.transpose(1, 2), at::kFloat) : at::bmm(a, c.transpose(1, 2));
+    } else {
+        parts = empty_f32({B * s, rows, cols}, a);
+        for (int64_t b = 0; b < B; ++b) {
+            Tensor ab = a.select(0, b).view({rows, s, n / s}).transpose(0, 1);
+            Tensor cb = c.select(0, b).view({cols, s, n / s}).permute({1, 2, 0});
+            Tensor to = parts.narrow(0, b * s, s);
+            if (half) at::bmm_out(to, ab, cb, at::kFloat);
+            else at::bmm_out(to, ab, cb);
+        }
+    }
+    return parts.sum(at::IntArrayRef{0}, false, at::kFloat).to(dtype).view(shape);
+}
+
+// sum over batch and voxels, float32, one value per channel
+Tensor channel_sums(const Tensor &g, void *stream)
+{
+    const int64_t B = g.size(0), C = g.size(1), n = g.size(2);
+    const int64_t parts = ndc_bias_act_parts(B * C, n);
+    Tensor partial = empty_f32({B, C, parts}, g);
+    check(ndc_row_sums(ptr(g), out_fptr(partial), B * C, n, dtype_tag(g), stream), "ndc_row_sums");
+    return partial.sum(at::IntArrayRef{0, 2});
+}
+
+// ---------------------------------------------------------------------------- the update
+
+struct UpdateConfig {
+    int64_t groups, m, sc;
+    double eps;
+    bool relu_input, save_ratio;
+};
+
+ndc_geom geom_for(const Tensor &x, const Tensor &h, const UpdateConfig &c, int path)
+{
+    ndc_geom g;
+    const int rank = (int)x.dim() - 2;
+    TORCH_CHECK_VALUE(rank >= 1 && rank <= 3 && h.dim() - 2 == rank, "unsupported spatial rank ", rank, " / kernel rank ",
+                      h.dim() - 2);
+    g.batch = (int32_t)x.size(0);
+    g.groups = (int32_t)c.groups;
+    g.m = (int32_t)c.m;
+    g.sc = (int32_t)c.sc;
+    for (int a = 0; a < 3; ++a) {
+        const int d = a - (3 - rank);
+        g.size[a] = d < 0 ? 1 : (int32_t)x.size(2 + d);
+        g.kernel[a] = d < 0 ? 1 : (int32_t)h.size(2 + d);
+    }
+    g.dtype = dtype_tag(x);
+    g.relu_input = c.relu_input ? 1 : 0;
+    g.path = path;
+    g.eps = (float)c.eps;
+    return g;
+}
+
+void check_update(const Tensor &x, const Tensor &z, const Tensor &h, const Tensor &bias, const UpdateConfig &c)
+{
+    TORCH_CHECK_VALUE(x.dim() >= 3 && x.dim() <= 5, "expected a (B, C, *S) tensor with 1-3 spatial dims, got ", x.sizes());
+    TORCH_CHECK_VALUE(x.size(1) == c.groups * c.m, "x has ", x.size(1), " channels, expected groups*m = ", c.groups * c.m);
+    bool same = z.dim() == x.dim() && z.size(0) == x.size(0) && z.size(1) == c.groups * c.sc;
+    for (int64_t d = 2; same && d < x.dim(); ++d) same = z.size(d) == x.size(d);
+    TORCH_CHECK_VALUE(same, "z has shape ", z.sizes(), ", expected the extents of x ", x.sizes(), " with ", c.groups * c.sc,
+                      " channels");
+    TORCH_CHECK_VALUE(h.dim() == x.dim() && h.size(0) * h.size(1) == c.groups * c.m * c.sc, "filter of shape ", h.sizes(),
+                      " does not match groups=", c.groups, ", m=", c.m, ", sc=", c.sc);
+    TORCH_CHECK_TYPE(x.scalar_type() == z.scalar_type(), "x (", x.scalar_type(), ") and z (", z.scalar_type(),
+                     ") must share a dtype");
+    TORCH_CHECK_TYPE(h.scalar_type() == at::kFloat && (!bias.defined() || bias.scalar_type() == at::kFloat),
+                     "filter and bias must be float32");
+    for (const Tensor *t : {&x, &z, &h, &bias})
+        TORCH_CHECK_VALUE(!t->defined() || (t->device() == x.device() && t->is_contiguous()),
+                          "all tensors must be contiguous and on one device");
+    TORCH_CHECK_VALUE(!bias.defined() || bias.numel() == c.groups * c.sc, "bias has ", bias.numel(), " entries, expected ",
+                      c.groups * c.sc);
+}
+
+// a 256-byte aligned slice of a fresh buffer
+Tensor scratch(size_t bytes, const Tensor &like)
+{
+    Tensor buf = at::empty({(int64_t)bytes + 256}, like.options().dtype(at::kByte));
+    const int64_t off = (256 - (int64_t)((uintptr_t)buf.const_data_ptr() & 255)) & 255;
+    return buf.narrow(0, off, (int64_t)bytes);
+}
+
+// the filter table the kernels of this geometry read instead of h, or undefined
+Tensor prepare_taps(const ndc_geom &g, const Tensor &h, void *stream)
+{
+    const size_t bytes = ndc_taps_bytes(&g);
+    if (!bytes) return Tensor();
+    Tensor taps = scratch(bytes, h);
+    check(ndc_prepare_taps(&g, fptr(h), out_ptr(taps), bytes, stream), "ndc_prepare_taps");
+    return taps;
+}
+
+struct UpdateForward {
+    Tensor x, z, t1, h, s_over_den, ratio, taps;   // what the backward reads (h: contiguous)
+    int path;
+    bool x_last, z_last;                           // x / z came in channels-last
+};
+
+// Forward of an update.  `grad`: a backward will follow.
+Tensor update_forward(Tensor x, Tensor z, const Tensor &h, const Tensor &bias, Tensor taps, const UpdateConfig &c, bool grad,
+                      UpdateForward &f, void *stream)
+{
+    // channels-last tensors come in through the library's tiled transposition, and the results
+    // go back out the same way, in the layout of the tensor they belong to
+    f.x_last = channels_last(x);
+    f.z_last = channels_last(z);
+    x = channel_first(x, stream);
+    z = channel_first(z, stream);
+    Tensor hc = h.contiguous();
+    check_update(x, z, hc, bias, c);
+    // The kernel family is read once, here, and named in both calls of this node: backward runs
+    // on an autograd thread, possibly after the process default has changed.
+    ndc_geom g = geom_for(x, hc, c, NDC_PATH_AUTO);
+    const bool fused = ndc_fused_supported(&g) != 0;
+    if (fused) g.path = ndc_matrix_kernels(-1) ? NDC_PATH_FUSED_MATRIX : NDC_PATH_FUSED_VECTOR;
+    f.path = g.path;
+    // (kept only where the backward kernels of this geometry read them)
+    const bool keep = grad && c.save_ratio && ndc_backward_uses_saved(&g);
+    // packed once here, used by the forward kernel and again by the backward's
+    if (!taps.defined()) taps = prepare_taps(g, hc, stream);
+    Tensor out = at::empty_like(z);
+    if (grad || !fused) f.t1 = at::empty_like(x);
+    if (keep) {
+        f.s_over_den = at::empty_like(z);
+        f.ratio = at::empty_like(z);
+    }
+    if (taps.defined()) {
+        check(ndc_forward_taps(&g, ptr(x), ptr(z), fptr(hc), ptr(taps), fptr(bias), out_ptr(out), out_ptr(f.t1),
+                               out_ptr(f.s_over_den), out_ptr(f.ratio), stream), "ndc_forward_taps");
+    } else {
+        const size_t bytes = ndc_forward_workspace_bytes(&g);
+        Tensor ws = bytes ? scratch(bytes, x) : Tensor();
+        check(ndc_forward(&g, ptr(x), ptr(z), fptr(hc), fptr(bias), out_ptr(out), out_ptr(f.t1), out_ptr(f.s_over_den),
+                          out_ptr(f.ratio), out_ptr(ws), bytes, stream), "ndc_forward");
+    }
+    f.x = x;
+    f.z = z;
+    f.h = hc;
+    f.taps = taps;
+    return f.z_last ? to_channels_last(out, stream) : out;
+}
+
+void refuse_double_backward(bool recording)
+{
+    // The gradients come from kernels autograd cannot see through, so a second differentiation
+    // would silently drop terms: refuse it, as the reference does.
+    TORCH_CHECK(!recording, "double backward through the fused Deconv update is not supported; construct the layer with a "
+                            "convolution keyword argument (e.g. stride=1) to force the general path, which is plain PyTorch "
+                            "and doubly differentiable");
+}
+
+struct UpdateGrads {
+    Tensor gx, gz, gh, gb;
+};
+
+UpdateGrads update_backward(const UpdateForward &f, const Tensor &bias, Tensor gout, const UpdateConfig &c, bool need_x,
+                            bool need_z, bool need_h, bool need_b, void *stream)
+{
+    const Tensor &x = f.x, &z = f.z;
+    if (gout.scalar_type() != z.scalar_type()) gout = gout.to(z.scalar_type());
+    gout = channel_first(gout, stream);
+    TORCH_CHECK_VALUE(gout.sizes() == z.sizes(), "the gradient has shape ", gout.sizes(), ", expected ", z.sizes());
+    need_b = need_b && bias.defined();
+    const ndc_geom g = geom_for(x, f.h, c, f.path);
+    UpdateGrads r;
+    if (need_x) r.gx = at::empty_like(x);
+    if (need_z) r.gz = at::empty_like(z);
+    if (need_h) r.gh = at::empty_like(f.h);
+    if (need_b) r.gb = empty_f32({c.groups * c.sc}, x);
+    const size_t bytes = ndc_backward_workspace_bytes(&g, need_x, need_z, need_h, need_b);
+    Tensor ws = scratch(bytes ? bytes : 1, x);
+    if (f.taps.defined())
+        check(ndc_backward_taps(&g, ptr(x), ptr(z), ptr(f.t1), ptr(f.s_over_den), ptr(f.ratio), fptr(f.h), ptr(f.taps),
+                                fptr(bias), ptr(gout), out_ptr(r.gx), out_ptr(r.gz), out_fptr(r.gh), out_fptr(r.gb),
+                                out_ptr(ws), bytes, stream), "ndc_backward_taps");
+    else
+        check(ndc_backward(&g, ptr(x), ptr(z), ptr(f.t1), ptr(f.s_over_den), ptr(f.ratio), fptr(f.h), fptr(bias), ptr(gout),
+                           out_ptr(r.gx), out_ptr(r.gz), out_fptr(r.gh), out_fptr(r.gb), out_ptr(ws), bytes, stream),
+              "ndc_backward");
+    return r;
+}
+
+void save_config(AutogradContext *ctx, const UpdateConfig &c, const UpdateForward &f)
+{
+    ctx->saved_data["cfg"] = std::vector<int64_t>{c.groups, c.m, c.sc, c.relu_input, f.path, f.x_last, f.z_last};
+    ctx->saved_data["eps"] = c.eps;
+}
+
+void load_config(AutogradContext *ctx, UpdateConfig &c, UpdateForward &f)
+{
+    const auto v = ctx->saved_data["cfg"].toIntVector();
+    c = UpdateConfig{v[0], v[1], v[2], ctx->saved_data["eps"].toDouble(), v[3] != 0, false};
+    f.path = (int)v[4];
+    f.x_last = v[5] != 0;
+    f.z_last = v[6] != 0;
+}
+
+// out = relu?(z + b) * (A(x) + eps) / (A(K(relu?(z + b))) + eps)
+struct Update : public torch::autograd::Function<Update> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &z, const Tensor &h, const OptTensor &bias,
+                          const OptTensor &taps, const UpdateConfig &c)
+    {
+        Scope scope(x);
+        UpdateForward f;
+        const Tensor b = bias ? *bias : Tensor();
+        Tensor out = update_forward(x, z, h, b, taps ? *taps : Tensor(), c, true, f, scope.stream);
+        save_config(ctx, c, f);
+        ctx->save_for_backward({f.x, f.z, f.t1, f.h, b, f.s_over_den, f.ratio, f.taps});
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        refuse_double_backward(at::GradMode::is_enabled());
+        UpdateConfig c;
+        UpdateForward f;
+        load_config(ctx, c, f);
+        const auto v = ctx->get_saved_variables();
+        f.x = v[0], f.z = v[1], f.t1 = v[2], f.h = v[3], f.s_over_den = v[5], f.ratio = v[6], f.taps = v[7];
+        Scope scope(f.x);
+        Needs n;
+        n.arg(true), n.arg(true), n.arg(true), n.arg(v[4].defined());
+        const auto need = n.ask(ctx);
+        UpdateGrads r = update_backward(f, v[4], gouts[0], c, need[0], need[1], need[2], need[3], scope.stream);
+        if (f.x_last && r.gx.defined()) r.gx = to_channels_last(r.gx, scope.stream);
+        if (f.z_last && r.gz.defined()) r.gz = to_channels_last(r.gz, scope.stream);
+        return {r.gx, r.gz, r.gh, r.gb, Tensor(), Tensor()};
+    }
+};
+
+Tensor update(const Tensor &x, const Tensor &z, const Tensor &h, const OptTensor &bias, int64_t groups, int64_t m, int64_t sc,
+              double eps, bool relu_input, const OptTensor &taps, bool save_ratio)
+{
+    const UpdateConfig c{groups, m, sc, eps, relu_input, save_ratio};
+    if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(z) || wants_grad(h) || wants_grad(bias)))
+        return Update::apply(x, z, h, bias, taps, c);
+    Scope scope(x);
+    UpdateForward f;
+    return update_forward(x, z, h, bias ? *bias : Tensor(), taps ? *taps : Tensor(), c, false, f, scope.stream);
+}
+
+// The layer's first update together with the 1x1 projection that makes its source
+// (deconv.py:157-165 with layers/linear.py:53-58 of the reference): z = W x per sample, then the
+// update of (x, z) with the projection's bias and the ReLU applied where the kernels load z.  One
+// node because x feeds both: as two nodes their input gradients are two tensors that autograd
+// adds in a pass of its own; here the projection's input-gradient GEMM accumulates onto the
+// update's gx.  With `rectify` the node takes the filter parameter itself and rectifies it (the
+// filter's relu and its backward are then no nodes of their own).
+struct Projected : public torch::autograd::Function<Projected> {
+    static Tensor run(const Tensor &x, const Tensor &weight, const Tensor &h, const Tensor &bias, const Tensor &taps,
+                      const UpdateConfig &c, bool grad, bool rectify, UpdateForward &f, void *stream)
+    {
+        const Matrix w(weight, false);
+        auto size = x.sizes().vec();
+        Tensor z = project(w, x.flatten(2), stream);
+        size[1] = w.cout();
+        return update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
+    }
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight, const Tensor &h, const OptTensor &bias,
+                          const OptTensor &taps, const UpdateConfig &c, bool rectified_input, bool rectify)
+    {
+        Scope scope(x);
+        UpdateForward f;
+        const Tensor b = bias ? *bias : Tensor();
+        Tensor out = run(x, weight, h, b, taps ? *taps : Tensor(), c, true, rectify, f, scope.stream);
+        save_config(ctx, c, f);
+        ctx->saved_data["flags"] = std::vector<int64_t>{rectified_input, rectify};
+        ctx->save_for_backward({f.x, f.z, f.t1, f.h, b, f.s_over_den, f.ratio, f.taps, weight});
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        refuse_double_backward(at::GradMode::is_enabled());
+        UpdateConfig c;
+        UpdateForward f;
+        load_config(ctx, c, f);
+        const auto flags = ctx->saved_data["flags"].toIntVector();
+        const auto v = ctx->get_saved_variables();
+        f.x = v[0], f.z = v[1], f.t1 = v[2], f.h = v[3], f.s_over_den = v[5], f.ratio = v[6], f.taps = v[7];
+        Scope scope(f.x);
+        Needs n;
+        n.arg(true), n.arg(true), n.arg(true), n.arg(v[4].defined());
+        const auto need = n.ask(ctx);
+        UpdateGrads r =
+            update_backward(f, v[4], gouts[0], c, need[0], need[0] || need[1], need[2], need[3], scope.stream);
+        const Tensor x = f.x.flatten(2);
+        const Matrix w(v[8], false);
+        Tensor gw, gx;
+        if (need[1]) gw = weight_grad(r.gz.flatten(2), x, w, v[8].sizes(), v[8].scalar_type());
+        if (need[0]) {
+            gx = project_back(w, r.gz.flatten(2), r.gx.flatten(2), flags[0] ? x : Tensor(), scope.stream).view(f.x.sizes());
+            if (f.x_last) gx = to_channels_last(gx, scope.stream);
+        }
+        if (flags[1] && r.gh.defined()) r.gh = at::threshold_backward(r.gh, f.h, 0);
+        return {gx, gw, r.gh, r.gb, Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+Tensor projected_update(const Tensor &x, const Tensor &weight, const Tensor &h, const OptTensor &bias, int64_t groups,
+                        int64_t m, int64_t sc, double eps, const OptTensor &taps, bool rectified_input, bool rectify,
+                        bool save_ratio)
+{
+    const UpdateConfig c{groups, m, sc, eps, true, save_ratio};
+    if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(h) || wants_grad(bias)))
+        return Projected::apply(x, weight, h, bias, taps, c, rectified_input, rectify);
+    Scope scope(x);
+    UpdateForward f;
+    return Projected::run(x, weight, h, bias ? *bias : Tensor(), taps ? *taps : Tensor(), c, false, rectify, f, scope.stream);
+}
+
+// ---------------------------------------------------------------------------- projection with its tail
+
+// y[b] = act(W x[b] + bias) + residual[b] on channel-first (B, C, n) tensors.  keep: the
+// activation's gradient will want the product (gelu, or relu under a residual sum)
+struct Linear : public torch::autograd::Function<Linear> {
+    static Tensor run(const Tensor &x, const Matrix &w, const Tensor &bias, int64_t act, const Tensor &res, bool keep, Tensor &z,
+                      void *stream)
+    {
+        const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
+        Tensor y;
+        if (streaming_gemm(x, cout, act != NDC_ACT_NONE || keep)) {
+            // product, bias, activation and residual in one kernel that reads x once and writes
+            // the result (and z where it is kept) once
+            Tensor frag = pack(w, false, x, stream);
+            y = empty({B, cout, n}, x);
+            if (keep) z = empty({B, cout, n}, x);
+            check(ndc_pointwise_gemm(ptr(x), ptr(frag), fptr(bias), ptr(res), out_ptr(y), out_ptr(z), B, w.cin(), cout, n,
+                                     (int)act, NDC_BF16, stream), "ndc_pointwise_gemm");
+            return y;
+        }
+        y = project(w, x, stream);
+        if (!bias.defined() && act == NDC_ACT_NONE && !res.defined()) return y;
+        if (keep) z = y, y = empty({B, cout, n}, x);
+        check(ndc_bias_act(ptr(keep ? z : y), fptr(bias), ptr(res), out_ptr(y), B, cout, n, (int)act, dtype_tag(x), stream),
+              "ndc_bias_act");
+        return y;
+    }
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight, const OptTensor &bias, int64_t act,
+                          const OptTensor &residual, bool premasked, bool transposed)
+    {
+        Scope scope(x);
+        const Matrix w(weight, transposed);
+        const Tensor b = f32_vector(bias), res = residual ? *residual : Tensor();
+        // relu alone needs only the sign of its output
+        const bool keep = act == NDC_ACT_GELU || (act == NDC_ACT_RELU && res.defined());
+        Tensor z;
+        Tensor y = run(x, w, b, act, res, keep, z, scope.stream);
+        ctx->save_for_backward({x, weight, keep ? z : act == NDC_ACT_RELU ? y : Tensor(), keep ? b : Tensor()});
+        // (premasked: every gradient that arrives is already zero where the result is)
+        ctx->saved_data["cfg"] = std::vector<int64_t>{
+            act, bias.has_value() && bias->defined(), res.defined(), premasked && act == NDC_ACT_RELU && !res.defined(), transposed,
+            bias.has_value() && bias->defined() ? (int64_t)bias->scalar_type() : 0};
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const bool recording = at::GradMode::is_enabled();
+        at::NoGradGuard no_grad;
+        const auto cfg = ctx->saved_data["cfg"].toIntVector();
+        const int act = (int)cfg[0];
+        const auto v = ctx->get_saved_variables();
+        const Tensor &x = v[0], &kept = v[2], &bias = v[3];
+        Scope scope(x);
+        const Matrix w(v[1], cfg[4] != 0);
+        Needs n;
+        n.arg(true), n.arg(true), n.arg(cfg[1]), n.arg(cfg[2]);
+        const auto need = n.ask(ctx);
+        const Tensor gy = gouts[0].contiguous();
+        Tensor gz = gy, gx, gw, gb;
+        if (act == NDC_ACT_NONE || cfg[3]) {
+            if (need[2]) gb = channel_sums(gy, scope.stream);
+        } else {
+            const int64_t B = gy.size(0), C = gy.size(1), nv = gy.size(2);
+            gz = at::empty_like(gy);
+            Tensor part;
+            if (need[2]) part = empty_f32({B, C, ndc_bias_act_parts(B * C, nv)}, gy);
+            check(ndc_bias_act_backward(ptr(gy), ptr(kept), fptr(bias), out_ptr(gz), out_fptr(part), B, C, nv, act, dtype_tag(gy),
+                                        scope.stream), "ndc_bias_act_backward");
+            if (need[2]) gb = part.sum(at::IntArrayRef{0, 2});
+        }
+        if (need[0]) gx = project_back(w, gz, Tensor(), Tensor(), scope.stream);
+        if (need[1]) gw = weight_grad(gz, x, w, v[1].sizes(), v[1].scalar_type());
+        if (gb.defined()) gb = gb.to((at::ScalarType)cfg[5]);
+        return once({gx, gw, gb, Tensor(), need[3] ? gy : Tensor(), Tensor(), Tensor()}, recording, gouts);
+    }
+};
+
+Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, int64_t act, const OptTensor &residual,
+              bool premasked, bool transposed)
+{
+    const Tensor xc = x.contiguous();
+    OptTensor res = residual;
+    if (res && res->defined()) {
+        if (res->scalar_type() != xc.scalar_type()) res = res->to(xc.scalar_type());
+        res = res->contiguous();
+    }
+    if (at::GradMode::is_enabled() && (wants_grad(xc) || wants_grad(weight) || wants_grad(bias) || wants_grad(res)))
+        return Linear::apply(xc, weight, bias, act, res, premasked, transposed);
+    Scope scope(xc);
+    Tensor z;
+    return Linear::run(xc, Matrix(weight, transposed), f32_vector(bias), act, res ? *res : Tensor(), false, z, scope.stream);
+}
+
+// W2 gelu(W1 x + b1) + b2 + residual on contiguous bfloat16 (B, C, n) tensors, on the streaming
+// GEMM (layers/mlp.py:40-63 with the block's sum, deconver.py:60-64): two launches forward (the
+// GELU and the kept pre-activation leave the first, bias and residual ride on the second), and a
+// backward in which the input gradient of the second projection comes out already multiplied by
+// the GELU's derivative, with the first bias's gradient summed in the same kernel.
+struct Mlp : public torch::autograd::Function<Mlp> {
+    static Tensor run(const Tensor &x, const Matrix &w1, const Tensor &b1, const Matrix &w2, const Tensor &b2, const Tensor &res,
+                      bool keep, Tensor &z, Tensor &a, void *stream)
+    {
+        const int64_t B = x.size(0), n = x.size(2), hidden = w1.cout(), cout = w2.cout();
+        Tensor f1 = pack(w1, false, x, stream), f2 = pack(w2, false, x, stream);
+        a = empty({B, hidden, n}, x);
+        if (keep) z = empty({B, hidden, n}, x);
+        check(ndc_pointwise_gemm(ptr(x), ptr(f1), fptr(b1), nullptr, out_ptr(a), out_ptr(z), B, w1.cin(), hidden, n, NDC_ACT_GELU,
+                                 NDC_BF16, stream), "ndc_pointwise_gemm");
+        Tensor y = empty({B, cout, n}, x);
+        check(ndc_pointwise_gemm(ptr(a), ptr(f2), fptr(b2), ptr(res), out_ptr(y), nullptr, B, hidden, cout, n, NDC_ACT_NONE,
+                                 NDC_BF16, stream), "ndc_pointwise_gemm");
+        return y;
+    }
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor &w2,
+                          const OptTensor &b2, const OptTensor &residual)
+    {
+        Scope scope(x);
+        Tensor z, a;
+        const Tensor b1f = f32_vector(b1);
+        Tensor y = run(x, Matrix(w1, false), b1f, Matrix(w2, false), f32_vector(b2), residual ? *residual : Tensor(), true, z, a,
+                       scope.stream);
+        ctx->save_for_backward({x, z, a, w1, w2, b1f});
+        ctx->saved_data["cfg"] = std::vector<int64_t>{b1.has_value(), b2.has_value(), residual.has_value(),
+                                                      b1 ? (int64_t)b1->scalar_type() : 0, b2 ? (int64_t)b2->scalar_type() : 0};
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const bool recording = at::GradMode::is_enabled();
+        at::NoGradGuard no_grad;
+        const auto cfg = ctx->saved_data["cfg"].toIntVector();
+        const auto v = ctx->get_saved_variables();
+        const Tensor &x = v[0], &z = v[1], &a = v[2], &b1 = v[5];
+        Scope scope(x);
+        const Matrix w1(v[3], false), w2(v[4], false);
+        Needs n;
+        n.arg(true), n.arg(true), n.arg(cfg[0]), n.arg(true), n.arg(cfg[1]), n.arg(cfg[2]);
+        const auto need = n.ask(ctx);
+        const Tensor gy = gouts[0].contiguous();
+        const int64_t B = x.size(0), nv = x.size(2), hidden = w1.cout();
+        Tensor gx, gw1, gb1, gw2, gb2;
+        if (need[4]) gb2 = channel_sums(gy, scope.stream).to((at::ScalarType)cfg[4]);
+        if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type());
+        if (need[0] || need[1] || need[2]) {
+            Tensor frag = pack(w2, true, gy, scope.stream), gz = at::empty_like(z), part;
+            if (need[2]) part = empty_f32({ndc_pointwise_gemm_parts(), hidden}, gy);
+            check(ndc_pointwise_gemm_actgrad(ptr(gy), ptr(frag), fptr(b1), ptr(z), out_ptr(gz), out_fptr(part), B, w2.cout(), hidden,
+                                             nv, NDC_ACT_GELU, NDC_BF16, scope.stream), "ndc_pointwise_gemm_actgrad");
+            if (need[2]) gb1 = part.sum(0).to((at::ScalarType)cfg[3]);
+            if (need[1]) gw1 = weight_grad(gz, x, w1, v[3].sizes(), v[3].scalar_type());
+            if (need[0]) gx = project_back(w1, gz, Tensor(), Tensor(), scope.stream);
+        }
+        return once({gx, gw1, gb1, gw2, gb2, need[5] ? gy : Tensor()}, recording, gouts);
+    }
+};
+
+// whether mlp() takes these shapes: bfloat16, all four products on the streaming GEMM
+bool mlp_applies(const Tensor &x, int64_t hidden, int64_t cout)
+{
+    const int64_t c = x.size(1), n = voxels(x);
+    auto ok = [n](int64_t ci, int64_t co) { return ndc_pointwise_gemm_supported(ci, co, n, NDC_BF16) != 0; };
+    return x.is_cuda() && ok(c, hidden) && ok(hidden, cout) && ok(cout, hidden) && ok(hidden, c);
+}
+
+Tensor mlp(const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor &w2, const OptTensor &b2,
+           const OptTensor &residual)
+{
+    const Tensor xc = x.contiguous();
+    OptTensor res = residual;
+    if (res && res->defined()) {
+        if (res->scalar_type() != xc.scalar_type()) res = res->to(xc.scalar_type());
+        res = res->contiguous();
+    }
+    if (at::GradMode::is_enabled() && (wants_grad(xc) || wants_grad(w1) || wants_grad(b1) || wants_grad(w2) || wants_grad(b2) ||
+                                       wants_grad(res)))
+        return Mlp::apply(xc, w1, b1, w2, b2, res);
+    Scope scope(xc);
+    Tensor z, a;
+    return Mlp::run(xc, Matrix(w1, false), f32_vector(b1), Matrix(w2, false), f32_vector(b2), res ? *res : Tensor(), false, z, a,
+                    scope.stream);
+}
+
+// ---------------------------------------------------------------------------- norms
+
+Tensor row_workspace(int64_t rows, int64_t n, const Tensor &like)
+{
+    return empty_f32({std::max<int64_t>((int64_t)ndc_rownorm_workspace_bytes(rows, n) / 4, 2)}, like);
+}
+
+Tensor row_norm_forward(const Tensor &x, double eps, Tensor &stats, void *stream)
+{
+    const int64_t rows = x.size(0) * x.size(1), n = voxels(x);
+    Tensor y = at::empty_like(x);
+    stats = empty_f32({rows, 2}, x);
+    Tensor ws = row_workspace(rows, n, x);
+    check(ndc_rownorm_forward(ptr(x), out_ptr(y), out_fptr(stats), rows, n, dtype_tag(x), (float)eps, out_ptr(ws), ws.numel() * 4,
+                              stream), "ndc_rownorm_forward");
+    return y;
+}
+
+Tensor row_norm_backward(const Tensor &gy, const Tensor &y, const Tensor &stats, const Tensor &addend, void *stream)
+{
+    const int64_t rows = stats.size(0), n = voxels(y);
+    Tensor gx = at::empty_like(y), ws = row_workspace(rows, n, y);
+    check(ndc_rownorm_backward(ptr(gy), ptr(y), fptr(stats), ptr(addend), out_ptr(gx), rows, n, dtype_tag(y), out_ptr(ws),
+                               ws.numel() * 4, stream), "ndc_rownorm_backward");
+    return gx;
+}
+
+struct RowNorm : public torch::autograd::Function<RowNorm> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, double eps)
+    {
+        Scope scope(x);
+        Tensor stats, y = row_norm_forward(x.contiguous(), eps, stats, scope.stream);
+        ctx->save_for_backward({y, stats});
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const bool recording = at::GradMode::is_enabled();
+        at::NoGradGuard no_grad;
+        const auto v = ctx->get_saved_variables();
+        Scope scope(v[0]);
+        return once({row_norm_backward(gouts[0].contiguous(), v[0], v[1], Tensor(), scope.stream), Tensor()}, recording, gouts);
+    }
+};
+
+// (norm(x), x) for a pre-norm residual block x + f(norm(x)): in backward the gradient that
+// arrives for the second output is summed into the norm's own input gradient by the kernel that
+// writes it, instead of by a separate addition
+struct RowNormSkip : public torch::autograd::Function<RowNormSkip> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, double eps)
+    {
+        Scope scope(x);
+        Tensor stats, y = row_norm_forward(x.contiguous(), eps, stats, scope.stream);
+        ctx->save_for_backward({y, stats});
+        ctx->set_materialize_grads(false);   // an unused output's gradient arrives undefined
+        return {y, x.view_as(x)};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const bool recording = at::GradMode::is_enabled();
+        at::NoGradGuard no_grad;
+        const auto v = ctx->get_saved_variables();
+        if (!gouts[0].defined()) return {gouts[1], Tensor()};
+        Scope scope(v[0]);
+        Tensor skip = gouts[1];
+        if (skip.defined()) skip = skip.to(v[0].scalar_type()).contiguous();
+        return once({row_norm_backward(gouts[0].contiguous(), v[0], v[1], skip, scope.stream), Tensor()}, recording, gouts);
+    }
+};
+
+Tensor row_norm(const Tensor &x, double eps)
+{
+    if (at::GradMode::is_enabled() && wants_grad(x)) return RowNorm::apply(x, eps);
+    Scope scope(x);
+    Tensor stats;
+    return row_norm_forward(x.contiguous(), eps, stats, scope.stream);
+}
+
+std::pair<Tensor, Tensor> row_norm_skip(const Tensor &x, double eps)
+{
+    if (!at::GradMode::is_enabled() || !wants_grad(x)) return {row_norm(x, eps), x};
+    auto r = RowNormSkip::apply(x, eps);
+    return {r[0], r[1]};
+}
+
+// nn.LayerNorm over the channel axis of a channel-first (B, C, n) tensor: lanes along the
+// voxels, a loop over the channels, nothing transposed
+struct ChannelNorm : public torch::autograd::Function<ChannelNorm> {
+    static Tensor run(const Tensor &x, const Tensor &w, const Tensor &b, double eps, Tensor &stats, void *stream)
+    {
+        const int64_t B = x.size(0), C = x.size(1), n = x.size(2);
+        Tensor y = at::empty_like(x);
+        stats = empty_f32({B, 2, n}, x);
+        check(ndc_chnorm_forward(ptr(x), fptr(w), fptr(b), out_ptr(y), out_fptr(stats), B, C, n, dtype_tag(x), (float)eps, stream),
+              "ndc_chnorm_forward");
+        return y;
+    }
+    static Tensor forward(AutogradContext *ctx, const Tensor &x_, const OptTensor &weight, const OptTensor &bias, double eps)
+    {
+        Scope scope(x_);
+        const Tensor x = x_.contiguous(), w = f32_vector(weight), b = f32_vector(bias);
+        Tensor stats, y = run(x, w, b, eps, stats, scope.stream);
+        ctx->save_for_backward({x, stats, w});
+        ctx->saved_data["cfg"] = std::vector<int64_t>{weight.has_value(), bias.has_value(),
+                                                      weight ? (int64_t)weight->scalar_type() : 0,
+                                                      bias ? (int64_t)bias->scalar_type() : 0};
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const bool recording = at::GradMode::is_enabled();
+        at::NoGradGuard no_grad;
+        const auto cfg = ctx->saved_data["cfg"].toIntVector();
+        const auto v = ctx->get_saved_variables();
+        const Tensor &x = v[0];
+        Scope scope(x);
+        Needs nd;
+        nd.arg(true), nd.arg(cfg[0]), nd.arg(cfg[1]);
+        const auto need = nd.ask(ctx);
+        const Tensor gy = gouts[0].to(x.scalar_type()).contiguous();
+        const int64_t B = x.size(0), C = x.size(1), n = x.size(2);
+        Tensor gx = at::empty_like(x), partial, gw, gb;
+        const bool affine = need[1] || need[2];
+        if (affine) partial = empty_f32({ndc_chnorm_parts(B, n, dtype_tag(x)), C, 2}, x);
+        check(ndc_chnorm_backward(ptr(gy), ptr(x), fptr(v[1]), fptr(v[2]), out_ptr(gx), out_fptr(partial), B, C, n, dtype_tag(x),
+                                  scope.stream), "ndc_chnorm_backward");
+        if (affine) {
+            const Tensor sums = partial.sum(0);
+            if (need[1]) gw = sums.select(1, 0).to((at::ScalarType)cfg[2]).contiguous();
+            if (need[2]) gb = sums.select(1, 1).to((at::ScalarType)cfg[3]).contiguous();
+        }
+        return once({need[0] ? gx : Tensor(), gw, gb, Tensor()}, recording, gouts);
+    }
+};
+
+Tensor channel_norm(const Tensor &x, const OptTensor &weight, const OptTensor &bias, double eps)
+{
+    if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(bias)))
+        return ChannelNorm::apply(x, weight, bias, eps);
+    Scope scope(x);
+    Tensor stats;
+    return ChannelNorm::run(x.contiguous(), f32_vector(weight), f32_vector(bias), eps, stats, scope.stream);
+}
+
+// ---------------------------------------------------------------------------- regrouping
+
+// 2 x 2 (x 2) windows of the grid <-> 2^nd channels per window; each direction's gradient is the
+// other direction.  On the way back to the grid a per-channel bias can be added in the same pass.
+Tensor regroup_run(const Tensor &x, bool to_channels, const Tensor &bias, void *stream)
+{
+    const int64_t B = x.size(0), nd = x.dim() - 2, win = int64_t(1) << nd;
+    auto size = x.sizes().vec();
+    size[1] = to_channels ? x.size(1) * win : x.size(1) / win;
+    for (int64_t d = 0; d < nd; ++d) size[2 + d] = to_channels ? x.size(2 + d) / 2 : x.size(2 + d) * 2;
+    Tensor out = empty(size, x);
+    const auto fine = to_channels ? x.sizes() : out.sizes();
+    const int64_t C = fine[1], D = nd == 3 ? fine[2] : 1;
+    check(ndc_regroup(ptr(x), out_ptr(out), fptr(bias), B * C, C, D, fine[nd], fine[nd + 1], nd == 3, dtype_tag(x), to_channels,
+                      stream), "ndc_regroup");
+    return out;
+}
+
+struct Regroup : public torch::autograd::Function<Regroup> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, bool to_channels, const OptTensor &bias)
+    {
+        Scope scope(x);
+        ctx->saved_data["cfg"] = std::vector<int64_t>{to_channels, bias.has_value() && bias->defined(),
+                                                      bias && bias->defined() ? (int64_t)bias->scalar_type() : 0};
+        return regroup_run(x, to_channels, f32_vector(bias), scope.stream);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const bool recording = at::GradMode::is_enabled();
+        at::NoGradGuard no_grad;
+        const auto cfg = ctx->saved_data["cfg"].toIntVector();
+        const Tensor g = gouts[0].contiguous();
+        Scope scope(g);
+        Needs n;
+        n.arg(true), n.arg(cfg[1]);
+        const auto need = n.ask(ctx);
+        Tensor gb;
+        if (!cfg[0] && need[1]) gb = channel_sums(g.flatten(2), scope.stream).to((at::ScalarType)cfg[2]);
+        return once({regroup_run(g, !cfg[0], Tensor(), scope.stream), Tensor(), gb}, recording, gouts);
+    }
+};
+
+Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
+{
+    if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(bias))) return Regroup::apply(x, to_channels, bias);
+    Scope scope(x);
+    return regroup_run(x, to_channels, f32_vector(bias), scope.stream);
+}
+
+OptTensor taps_for(const Tensor &x, const Tensor &h, int64_t groups, int64_t m, int64_t sc)
+{
+    Scope scope(x);
+    const ndc_geom g = geom_for(x, h, UpdateConfig{groups, m, sc, 0.0, true, false}, NDC_PATH_AUTO);
+    Tensor taps = prepare_taps(g, h, scope.stream);
+    return taps.defined() ? OptTensor(taps) : OptTensor();
+}
+
+// the name Python shows for a node (type(y.grad_fn))
+template <class F> void name_node(const char *name)
+{
+    static PyTypeObject type{};
+    torch::autograd::_initFunctionPyTypeObject(type, name, nullptr, nullptr);
+    torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<F>), &type);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
+{
+    name_node<Update>("DeconvUpdateBackward");
+    name_node<Projected>("ProjectedUpdateBackward");
+    name_node<Linear>("_PointwiseLinearBackward");
+    name_node<Mlp>("_FusedMLPBackward");
+    name_node<RowNorm>("_RowNormBackward");
+    name_node<RowNormSkip>("_RowNormSkipBackward");
+    name_node<ChannelNorm>("_ChannelNormBackward");
+    name_node<Regroup>("_RegroupBackward");
+    m.def("update", &update);
+    m.def("projected_update", &projected_update);
+    m.def("prepare_taps", &taps_for);
+    m.def("linear", &linear);
+    m.def("mlp", &mlp);
+    m.def("mlp_applies", &mlp_applies);
+    m.def("row_norm", &row_norm);
+    m.def("row_norm_skip", &row_norm_skip);
+    m.def("channel_norm", &channel_norm);
+    m.def("regroup", &regroup);
+    m.def("weight_grad_chunks", &weight_grad_chunks);
+    m.def("weight_grad_plan", &weight_grad_plan);
+}

@@ -23,182 +23,24 @@ def _wgrad_chunks(batch: int, n: int, min_chunk: int = 2048) -> int:
     """Number of equal chunks the voxel axis is cut into for the weight-gradient GEMM: a power
     of two that divides ``n``, leaves chunks of at least ``min_chunk`` voxels and at most 128
     GEMMs in the batch."""
-    s = 1
-    while s < 64 and n % (2 * s) == 0 and n // (2 * s) >= min_chunk and batch * 2 * s <= 128:
-        s *= 2
-    return s
+    return _lib.get_native().weight_grad_chunks(batch, n, min_chunk)
 
 
 def _wgrad_plan(batch: int, n: int, dtype: torch.dtype) -> int:
-    """The chunk count ``projection_weight_grad`` uses, from timings on an MI355X with batch 2
-    in bfloat16 (64 chunks at 128^3; 32 at 64^3, where 64 cost 0.05 ms more on the 128 x 128
-    result; 16 at 32^3: 0.056 ms against 0.11-0.13 ms unchunked; none at 16^3) and batch 8 in
-    float32 (none up to 256^2 voxels: there every chunked form was slower)."""
-    if dtype == torch.bfloat16:
-        return 1 if n < (1 << 15) else _wgrad_chunks(batch, n, 2048 if n < (1 << 17) else 8192)
-    return 1 if n < (1 << 17) else _wgrad_chunks(batch, n)
+    """The chunk count of a projection's weight gradient (see ``csrc/ndc_torch.cpp``)."""
+    return _lib.get_native().weight_grad_plan(batch, n, dtype == torch.bfloat16)
 
 
-def projection_weight_grad(gz: torch.Tensor, x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """``sum_b gz[b] x[b]^T`` for ``gz`` of shape ``(B, Cout, N)`` and ``x`` of shape
-    ``(B, Cin, N)``: the weight gradient of a 1x1 projection, a ``Cout x Cin`` result summed
-    over all voxels.  Short rows (the 2-D network's levels) take one batched GEMM and a sum over
-    the batch; long rows are cut into equal chunks of the voxel axis that become batch entries
-    (strided views, no copies).  The partial results -- float32 also for bfloat16 operands -- are
-    added in float32, in one reduction."""
-    B, cout, n = gz.shape
-    cin = x.shape[1]
-    s = _wgrad_plan(B, n, gz.dtype)
-    # bfloat16 operands: the GEMMs hand out their float32 accumulators (same speed, and the
-    # partial results are then not rounded to bfloat16 before they are added)
-    f32 = {"out_dtype": torch.float32} if gz.is_cuda and gz.dtype == torch.bfloat16 else {}
-    if s == 1:
-        parts = torch.bmm(gz, x.transpose(1, 2), **f32)
-    else:
-        parts = gz.new_empty(B * s, cout, cin, dtype=torch.float32 if f32 else gz.dtype)
-        for b in range(B):
-            a = gz[b].view(cout, s, n // s).transpose(0, 1)
-            c = x[b].view(cin, s, n // s).permute(1, 2, 0)
-            torch.bmm(a, c, out=parts[b * s:(b + 1) * s], **f32)
-    return parts.sum(0, dtype=torch.float32).to(dtype)
-
-
-def project(weight: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """``W x`` per sample for contiguous ``x`` of shape ``(B, Cin, N)`` and ``weight`` of shape
-    ``(Cout, Cin)`` in any floating dtype (used in ``x``'s): the library's streaming GEMM where
-    it applies, else one batched hipBLASLt GEMM with the weight shared through a zero stride."""
-    lib = _lib.get_library()
-    if ops.pointwise_gemm_applies(lib, x, weight.shape[0]):
-        with torch.cuda.device(x.device):
-            return ops.pointwise_gemm(lib, x, ops.pointwise_pack(lib, weight.contiguous()), weight.shape[0])[0]
-    z = x.new_empty(x.shape[0], weight.shape[0], x.shape[2])
-    torch.bmm(weight.to(x.dtype).unsqueeze(0).expand(x.shape[0], -1, -1), x, out=z)
-    return z
-
-
-def project_back(weight: torch.Tensor, gz: torch.Tensor, accumulate: Optional[torch.Tensor] = None,
-                 mask: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``W^T gz`` per sample (the input gradient of a 1x1 projection with ``weight`` of shape
-    ``(Cout, Cin)``), plus ``accumulate`` if given (a tensor of the result's shape, which may
-    be overwritten), and zero wherever ``mask <= 0`` if a mask of the result's shape is given
-    (the gradient taken through the rectifier whose output the projection read).  The
-    library's streaming GEMM where it applies -- the weight is packed as it lies, no transposed
-    copy --, else one batched hipBLASLt GEMM."""
-    B, cout, n = gz.shape
-    if cout == 1:
-        # one output channel (the network's head): the product is an outer product, i.e. a
-        # broadcast multiplication at the memory rate (as a GEMM it ran at a fifth of it)
-        gx = gz * weight.reshape(1, -1, 1).to(gz.dtype)
-        gx = gx if accumulate is None else accumulate.add_(gx)
-    else:
-        lib = _lib.get_library()
-        if gz.is_contiguous() and ops.pointwise_gemm_applies(lib, gz, weight.shape[1]):
-            with torch.cuda.device(gz.device):
-                wfrag = ops.pointwise_pack(lib, weight.contiguous(), transposed=True)
-                return ops.pointwise_gemm(lib, gz, wfrag, weight.shape[1], residual=accumulate, mask=mask)[0]
-        wt = weight.to(gz.dtype).t().unsqueeze(0).expand(B, -1, -1)
-        if accumulate is not None:
-            gx = accumulate.baddbmm_(wt, gz)
-        else:
-            gx = gz.new_empty(B, weight.shape[1], n)
-            torch.bmm(wt, gz, out=gx)
-    return gx if mask is None else gx.mul_(mask > 0)
-
-
-class _PointwiseLinear(torch.autograd.Function):
-    """``y[b] = act(W x[b] + bias) + residual[b]`` for ``x`` of shape ``(B, Cin, N)``: the 1x1
-    projection as plain GEMMs on the channel-first layout (hipBLASLt through ``torch.bmm``),
-    then ONE pass of the HIP library over the result for bias, activation and residual sum
-    (``ndc_bias_act``).
-
-    The same map as ``nn.Conv1d(kernel_size=1)`` (layers/linear.py:53-58) followed by the
-    activation and the ``x + ...`` of the block (layers/mlp.py:40-63, deconver.py:60-64).  The
-    library convolution reaches its GEMM through layout transposes of input and output and a
-    separate weight-gradient kernel; here forward and input gradient are one GEMM each on
-    the tensors as they lie, and the weight gradient (a ``Cout x Cin`` result summed over
-    millions of voxels) is a batch of GEMMs over equal chunks of the voxel axis whose
-    partial results are added in float32: 0.54 ms instead of 0.89 ms for forward + backward
-    of the 128 -> 512 projection at 2 x 64^3 in bf16."""
-
-    @staticmethod
-    def forward(ctx, x, weight, bias, act, residual, grad_premasked=False):
-        lib = _lib.get_library()
-        # one batched GEMM on the tensors as they lie, the weight shared by the batch entries
-        # through a zero stride (no copy; the same bits as one GEMM per sample, in one launch)
-        # (the weight arrives in its own dtype -- float32 under autocast -- and is cast here, so
-        # that its gradient leaves backward as the float32 sum it is, not rounded to bf16 first)
-        B = x.shape[0]
-        w = weight.detach()
-        bias32 = None if bias is None else bias.detach().float().contiguous()
-        # the activation's gradient needs z + bias: gelu keeps z; relu alone needs only the
-        # sign of its output, which may then overwrite z
-        keep_z = act == "gelu" or (act == "relu" and residual is not None)
-        keep_z = keep_z and any(ctx.needs_input_grad)     # (nothing is kept for a forward-only call)
-        if ops.pointwise_gemm_applies(lib, x, w.shape[0], act, keep_z):
-            # the library's streaming GEMM: product, bias, activation and residual in one
-            # kernel that reads x once and writes the result (and z where it is kept) once
-            with torch.cuda.device(x.device):
-                y, z = ops.pointwise_gemm(lib, x, ops.pointwise_pack(lib, w.contiguous()),
-                                          w.shape[0], bias32, residual, act, keep_z=keep_z)
-            # (the packing reads the weight in its own dtype, and so does the backward's: no
-            # cast copy of it is made or kept)
-        else:
-            w = w.to(x.dtype)
-            z = x.new_empty(B, w.shape[0], x.shape[2])
-            torch.bmm(w.unsqueeze(0).expand(B, -1, -1), x, out=z)
-            y = z
-            if bias is not None or act is not None or residual is not None:
-                with torch.cuda.device(x.device):
-                    y = ops.bias_act(lib, z, bias32, residual, act, inplace=not keep_z)
-        kept = z if keep_z else y if act == "relu" else None
-        ctx.save_for_backward(x, w, kept, bias32 if keep_z else None)
-        ctx.weight_dtype = weight.dtype
-        ctx.has_bias = bias is not None
-        ctx.act = act
-        # a ReLU whose consumer hands back a gradient that is already zero where the output is
-        # (``project_back(mask=...)``): the backward then has no pass of its own for it
-        ctx.premasked = bool(grad_premasked) and act == "relu" and residual is None
-        return y
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, gy):
-        x, weight, kept, bias32 = ctx.saved_tensors
-        gy = gy.contiguous()
-        gx = gw = gb = None
-        gres = gy if ctx.needs_input_grad[4] else None
-        want_gb = ctx.has_bias and ctx.needs_input_grad[2]
-        gz = gy
-        if ctx.premasked:
-            if want_gb:
-                with torch.cuda.device(gy.device):
-                    gb = ops.channel_sums(_lib.get_library(), gy)
-        elif ctx.act is not None:
-            with torch.cuda.device(gy.device):
-                gz, gb = ops.bias_act_backward(_lib.get_library(), gy, kept, bias32, ctx.act,
-                                               need_bias_grad=want_gb)
-        elif want_gb:
-            # per-row partial sums by the library (at the copy rate), then the few per-sample
-            # sums: PyTorch's one-call reduction of a (B, C, N) tensor over B and N runs at a
-            # tenth of the memory bandwidth, its row sums at two thirds
-            with torch.cuda.device(gy.device):
-                gb = ops.channel_sums(_lib.get_library(), gy)
-        if ctx.needs_input_grad[0]:
-            gx = project_back(weight, gz)
-        if ctx.needs_input_grad[1]:
-            gw = projection_weight_grad(gz, x, ctx.weight_dtype)
-        return gx, gw, gb, None, gres, None
-
-
+_ACT_TAGS = {None: _lib.ACT_NONE, "relu": _lib.ACT_RELU, "gelu": _lib.ACT_GELU}
 _ACT_FUNCTIONS = {None: lambda t: t, "relu": torch.relu, "gelu": torch.nn.functional.gelu}
 
 
 def pointwise_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                      act: Optional[str] = None, residual: Optional[torch.Tensor] = None,
-                     grad_premasked: bool = False) -> torch.Tensor:
+                     grad_premasked: bool = False, transposed: bool = False) -> torch.Tensor:
     """``act(W x + bias) + residual``: the 1x1 projection ``(B, Cin, N) -> (B, Cout, N)`` with
-    ``weight`` of shape ``(Cout, Cin)`` or ``(Cout, Cin, 1)``, optionally followed by an
-    activation (``"relu"`` or ``"gelu"``, the exact one) and the sum with a tensor of the
+    ``weight`` of shape ``(Cout, Cin)`` or ``(Cout, *)`` with ``Cin`` elements per row (with
+    ``transposed``: the ``(Cin, Cout)`` storage of it), optionally followed by an activation (``"relu"`` or ``"gelu"``, the exact one) and the sum with a tensor of the
     output's shape.  bfloat16 (stored or under autocast) and float32 tensors on the GPU run as
     batched GEMMs on the channel-first layout plus one pass of the HIP library over the result;
     everything else as the reference's ``conv1d`` followed by PyTorch's activation and sum.
@@ -207,20 +49,17 @@ def pointwise_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     caller guarantees that every gradient reaching the result is already zero where the result
     is -- its only consumer took it through the rectifier (``project_back(mask=...)``) --, so the
     backward skips the rectifier's pass."""
-    w2 = weight.squeeze(-1) if weight.dim() == 3 else weight
     dtype = x.dtype
     if x.is_cuda and torch.is_autocast_enabled(x.device.type):
         dtype = torch.get_autocast_dtype(x.device.type)
     # (2-D network in float32, batch 8: 16.6 ms per step this way against 20.8 ms with the
     # GEMM left to the library's conv1d, whose weight gradient goes through layout transposes)
     if not x.is_cuda or x.dim() != 3 or dtype not in (torch.bfloat16, torch.float32):
-        y = _ACT_FUNCTIONS[act](torch.nn.functional.conv1d(x, w2.unsqueeze(-1), bias))
+        w = weight.t() if transposed else weight.flatten(1)
+        y = _ACT_FUNCTIONS[act](torch.nn.functional.conv1d(x, w.unsqueeze(-1), bias))
         return y if residual is None else residual + y
-    x = x.to(dtype)
-    if residual is not None:
-        residual = residual.to(dtype).contiguous()
-    with torch.autocast(x.device.type, enabled=False):
-        return _PointwiseLinear.apply(x.contiguous(), w2, bias, act, residual, grad_premasked)
+    return _lib.get_native().linear(x if x.dtype == dtype else x.to(dtype), weight, bias, _ACT_TAGS[act], residual,
+                                    grad_premasked, transposed)
 
 
 def _gemm_route(x: torch.Tensor) -> bool:
@@ -276,35 +115,6 @@ def channels_to_patches(y: torch.Tensor, k, coarse) -> torch.Tensor:
     return y.permute(order).reshape(B, C, *[c * v for c, v in zip(coarse, k)])
 
 
-class _Regroup2(torch.autograd.Function):
-    """2 x 2 (x 2) windows of the grid <-> 2^nd channels per window on the HIP kernel
-    (``ndc_regroup``); each direction's gradient is the other direction.  On the way back to
-    the grid a per-channel bias can be added in the same pass."""
-
-    @staticmethod
-    def forward(ctx, x, to_channels, bias):
-        lib = _lib.get_library()
-        ctx.to_channels = to_channels
-        ctx.has_bias = bias is not None
-        with torch.cuda.device(x.device):
-            if to_channels:
-                return ops.windows_to_channels(lib, x)
-            return ops.channels_to_windows(lib, x, None if bias is None else bias.detach().float().contiguous())
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, g):
-        lib = _lib.get_library()
-        g = g.contiguous()
-        gb = None
-        with torch.cuda.device(g.device):
-            if ctx.to_channels:
-                return ops.channels_to_windows(lib, g), None, None
-            if ctx.has_bias and ctx.needs_input_grad[2]:
-                gb = ops.channel_sums(lib, g.flatten(2))
-            return ops.windows_to_channels(lib, g), None, gb
-
-
 def _regroup_on_hip(fine_shape, dtype, k, *tensors) -> bool:
     """2-windows in every dimension and GPU buffers the kernel takes (``tensors``: the ones
     that exist already)."""
@@ -321,10 +131,10 @@ def patch_conv(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
         x = x.to(torch.get_autocast_dtype(x.device.type))     # before the regrouping, not after
     xc = x.contiguous()
     if _regroup_on_hip(xc.shape, xc.dtype, k, xc):
-        cols = _Regroup2.apply(xc, True, None).flatten(2)
+        cols = _lib.get_native().regroup(xc, True, None).flatten(2)
     else:
         cols = patches_to_channels(x, k)
-    y = pointwise_linear(cols, weight.flatten(1), bias)
+    y = pointwise_linear(cols, weight, bias)
     return y.view(x.shape[0], -1, *coarse)
 
 
@@ -334,21 +144,21 @@ def patch_conv_transpose(x: torch.Tensor, weight: torch.Tensor,
     ``Cout * prod(k)`` channels, then every column spread over its window of the finer grid."""
     k = tuple(weight.shape[2:])
     # weight (Cin, Cout, *k): row (cout, offset) of the projection is weight[:, cout, offset]
-    w = weight.flatten(1).t()
+    w = weight.flatten(1)
     fine = (x.shape[0], weight.shape[1], *[s * v for s, v in zip(x.shape[2:], k)])
     dtype = x.dtype
     if x.is_cuda and torch.is_autocast_enabled(x.device.type):
         dtype = torch.get_autocast_dtype(x.device.type)
     if x.is_cuda and _regroup_on_hip(fine, dtype, k):
         # the bias rides on the regrouping pass
-        y = pointwise_linear(x.flatten(2), w, None).contiguous()
+        y = pointwise_linear(x.flatten(2), w, None, transposed=True).contiguous()
         if _regroup_on_hip(fine, y.dtype, k, y):
-            return _Regroup2.apply(y.view(x.shape[0], -1, *x.shape[2:]), False, bias)
+            return _lib.get_native().regroup(y.view(x.shape[0], -1, *x.shape[2:]), False, bias)
         y = channels_to_patches(y, k, x.shape[2:])
         return y if bias is None else y + bias.to(y.dtype).view(1, -1, *([1] * len(k)))
     if bias is not None:
         bias = bias.repeat_interleave(math.prod(k))
-    return channels_to_patches(pointwise_linear(x.flatten(2), w, bias), k, x.shape[2:])
+    return channels_to_patches(pointwise_linear(x.flatten(2), w, bias, transposed=True), k, x.shape[2:])
 
 
 class _PatchConvMixin:
@@ -390,7 +200,7 @@ def unfold_conv(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
         shifts = [t + (o,) for t in shifts for o in range(v)]
     cols = torch.stack([xp[(slice(None), slice(None), *[slice(o, o + n) for o, n in zip(t, size)])]
                         for t in shifts], dim=2)
-    y = pointwise_linear(cols.flatten(1, 2).flatten(2), weight.flatten(1), bias)
+    y = pointwise_linear(cols.flatten(1, 2).flatten(2), weight, bias)
     return y.view(x.shape[0], -1, *size)
 
 
@@ -479,58 +289,21 @@ class Linear(nn.Module):
         return y.view(shape[0], -1, *shape[2:])
 
 
-class _FusedMLP(torch.autograd.Function):
-    """``W2 gelu(W1 x + b1) + b2 + residual`` on contiguous bfloat16 ``(B, C, N)`` tensors as ONE
-    autograd node on the library's streaming GEMM (layers/mlp.py:40-63 with the block's sum,
-    deconver.py:60-64): two launches forward (the GELU and the kept pre-activation leave the
-    first, bias and residual ride on the second), and a backward in which the input gradient
-    of the second projection comes out already multiplied by the GELU's derivative, with the
-    first bias's gradient summed in the same kernel -- the hidden tensor's gradient is written
-    once and never read back by an activation pass."""
+class _FusedMLP:
+    """``W2 gelu(W1 x + b1) + b2 + residual`` as ONE autograd node on the library's streaming GEMM
+    (layers/mlp.py:40-63 with the block's sum, deconver.py:60-64), compiled in
+    ``csrc/ndc_torch.cpp``: the hidden tensor's gradient is written once and never read back by an
+    activation pass."""
 
     @staticmethod
     def applies(lib, x: torch.Tensor, hidden: int, cout: int) -> bool:
-        B, c, n = x.shape
-        ok = lambda cin, co: lib.pointwise_gemm_supported(cin, co, n, _lib.NDC_BF16)   # noqa: E731
-        return (x.is_cuda and x.dtype == torch.bfloat16 and ok(c, hidden) and ok(hidden, cout)
-                and ok(cout, hidden) and ok(hidden, c))
+        """Whether it takes ``x`` (B, C, *): bfloat16 on the GPU, all four products of forward and
+        backward in the streaming GEMM's shapes."""
+        return x.dtype == torch.bfloat16 and _lib.get_native().mlp_applies(x, hidden, cout)
 
     @staticmethod
-    def forward(ctx, x, w1, b1, w2, b2, residual):
-        lib = _lib.get_library()
-        hidden, cout = w1.shape[0], w2.shape[0]
-        b1f = None if b1 is None else b1.detach().float().contiguous()
-        b2f = None if b2 is None else b2.detach().float().contiguous()
-        with torch.cuda.device(x.device):
-            a, z = ops.pointwise_gemm(lib, x, ops.pointwise_pack(lib, w1.detach().contiguous()), hidden, b1f,
-                                      None, "gelu", keep_z=any(ctx.needs_input_grad))
-            y, _ = ops.pointwise_gemm(lib, a, ops.pointwise_pack(lib, w2.detach().contiguous()), cout, b2f,
-                                      residual, None)
-        ctx.save_for_backward(x, z, a, w1.detach(), w2.detach(), b1f)
-        ctx.dtypes = (w1.dtype, w2.dtype)
-        return y
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, gy):
-        x, z, a, w1, w2, b1f = ctx.saved_tensors
-        lib = _lib.get_library()
-        gy = gy.contiguous()
-        need_x, need_w1, need_b1, need_w2, need_b2, need_res = ctx.needs_input_grad
-        gx = gw1 = gb1 = gw2 = gb2 = None
-        with torch.cuda.device(gy.device):
-            if need_b2:
-                gb2 = ops.channel_sums(lib, gy)
-            if need_w2:
-                gw2 = projection_weight_grad(gy, a, ctx.dtypes[1])
-            if need_x or need_w1 or need_b1:
-                gz, gb1 = ops.pointwise_gemm_actgrad(lib, gy, ops.pointwise_pack(lib, w2.contiguous(), transposed=True),
-                                                     w2.shape[1], z, b1f, "gelu", need_bias_grad=need_b1)
-                if need_w1:
-                    gw1 = projection_weight_grad(gz, x, ctx.dtypes[0])
-                if need_x:
-                    gx = project_back(w1, gz)
-        return gx, gw1, gb1, gw2, gb2, (gy if need_res else None)
+    def apply(x, w1, b1, w2, b2, residual):
+        return _lib.get_native().mlp(x, w1, b1, w2, b2, residual)
 
 
 class MLP(nn.Module):
@@ -572,45 +345,15 @@ class MLP(nn.Module):
         dtype = torch.get_autocast_dtype(x.device.type) if torch.is_autocast_enabled(x.device.type) else x.dtype
         if dtype != torch.bfloat16:
             return None
-        flat = x.flatten(2).to(dtype).contiguous()
-        w1, w2 = first.linear.weight.squeeze(-1), second.linear.weight.squeeze(-1)
-        if not _FusedMLP.applies(_lib.get_library(), flat, w1.shape[0], w2.shape[0]):
+        w1, w2 = first.linear.weight, second.linear.weight
+        flat = x.flatten(2)
+        if flat.dtype != dtype:
+            flat = flat.to(dtype)
+        if not _FusedMLP.applies(None, flat, w1.shape[0], w2.shape[0]):
             return None
-        res = None if residual is None else residual.flatten(2).to(dtype).contiguous()
-        with torch.autocast(x.device.type, enabled=False):
-            y = _FusedMLP.apply(flat, w1, first.linear.bias, w2, second.linear.bias, res)
-        return y.view(x.shape[0], -1, *x.shape[2:])
-
-
-class _ChannelNorm(torch.autograd.Function):
-    """``nn.LayerNorm`` over the channel axis of a channel-first ``(B, C, n)`` tensor on the HIP
-    kernels (``ndc_chnorm_forward`` / ``_backward``): lanes along the voxels, a loop over the
-    channels, nothing transposed."""
-
-    @staticmethod
-    def forward(ctx, x, weight, bias, eps):
-        lib = _lib.get_library()
-        x = x.contiguous()
-        w32 = None if weight is None else weight.detach().float().contiguous()
-        b32 = None if bias is None else bias.detach().float().contiguous()
-        with torch.cuda.device(x.device):
-            y, stats = ops.chnorm_forward(lib, x, w32, b32, eps)
-        ctx.save_for_backward(x, stats, w32)
-        ctx.dtypes = (None if weight is None else weight.dtype, None if bias is None else bias.dtype)
-        return y
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, gy):
-        x, stats, w32 = ctx.saved_tensors
-        gy = gy.to(x.dtype).contiguous()
-        affine = any(ctx.needs_input_grad[1:3])
-        with torch.cuda.device(x.device):
-            gx, gw, gb = ops.chnorm_backward(_lib.get_library(), gy, x, stats, w32, need_affine_grads=affine)
-        wd, bd = ctx.dtypes
-        return (gx if ctx.needs_input_grad[0] else None,
-                gw.to(wd) if affine and ctx.needs_input_grad[1] and wd is not None else None,
-                gb.to(bd) if affine and ctx.needs_input_grad[2] and bd is not None else None, None)
+        y = _FusedMLP.apply(flat, w1, first.linear.bias, w2, second.linear.bias,
+                            None if residual is None else residual.flatten(2))
+        return y.view(x.shape)
 
 
 _CHNORM_MIN_VOXELS = 32768
@@ -637,7 +380,6 @@ class LayerNorm(nn.Module):
                 and x.shape[0] * x[0, 0].numel() >= _CHNORM_MIN_VOXELS):
             t = x.float() if torch.is_autocast_enabled(x.device.type) else x
             if t.dtype in (torch.float32, torch.bfloat16):
-                with torch.autocast(x.device.type, enabled=False):
-                    y = _ChannelNorm.apply(t.flatten(2), self.norm.weight, self.norm.bias, float(self.norm.eps))
+                y = _lib.get_native().channel_norm(t.flatten(2), self.norm.weight, self.norm.bias, float(self.norm.eps))
                 return y.view(x.shape)
         return self.norm(x.movedim(1, -1)).movedim(-1, 1)

@@ -19,64 +19,9 @@ from __future__ import annotations
 import torch
 from torch import Tensor, nn
 
-from . import _lib, ops
+from . import _lib
 
 __all__ = ["InstanceNorm1d", "InstanceNorm2d", "InstanceNorm3d", "instance_norm", "native_norm"]
-
-
-class _RowNorm(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x: Tensor, eps: float) -> Tensor:
-        lib = _lib.get_library()
-        x = x.contiguous()
-        rows = x.shape[0] * x.shape[1]
-        with torch.cuda.device(x.device):
-            y, stats = ops.rownorm_forward(lib, x.view(rows, -1), eps)
-        ctx.save_for_backward(y, stats)
-        ctx.shape = x.shape
-        return y.view(x.shape)
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, gy: Tensor):
-        y, stats = ctx.saved_tensors
-        lib = _lib.get_library()
-        gy = gy.contiguous().view(y.shape)
-        with torch.cuda.device(y.device):
-            gx = ops.rownorm_backward(lib, gy, y, stats)
-        return gx.view(ctx.shape), None
-
-
-class _RowNormSkip(torch.autograd.Function):
-    """``(norm(x), x)``: the norm and the tensor it was taken of, for a pre-norm residual block
-    ``x + f(norm(x))``.  In backward the gradient that arrives for the second output (the
-    residual branch's) is summed into the norm's own input gradient by the kernel that writes
-    it, instead of by a separate addition."""
-
-    @staticmethod
-    def forward(ctx, x: Tensor, eps: float):
-        lib = _lib.get_library()
-        xc = x.contiguous()
-        rows = xc.shape[0] * xc.shape[1]
-        with torch.cuda.device(xc.device):
-            y, stats = ops.rownorm_forward(lib, xc.view(rows, -1), eps)
-        ctx.save_for_backward(y, stats)
-        ctx.shape = xc.shape
-        ctx.set_materialize_grads(False)     # an unused output's gradient arrives as None
-        return y.view(xc.shape), x.view_as(x)
-
-    @staticmethod
-    @torch.autograd.function.once_differentiable
-    def backward(ctx, gy, gskip):
-        y, stats = ctx.saved_tensors
-        if gy is None:
-            return gskip, None
-        gy = gy.contiguous().view(y.shape)
-        if gskip is not None:
-            gskip = gskip.to(gy.dtype).contiguous().view(y.shape)
-        with torch.cuda.device(y.device):
-            gx = ops.rownorm_backward(_lib.get_library(), gy, y, stats, addend=gskip)
-        return gx.view(ctx.shape), None
 
 
 def hip_norm_applies(x: Tensor) -> bool:
@@ -89,8 +34,7 @@ def instance_norm(x: Tensor, eps: float = 1e-5) -> Tensor:
     HIP kernels; ``x`` is ``(B, C, *S)`` on the GPU, float32 or bfloat16."""
     if not hip_norm_applies(x):
         raise ValueError("instance_norm runs on GPU tensors (B, C, *S) in float32 or bfloat16")
-    shape = x.shape
-    return _RowNorm.apply(x, float(eps)).view(shape)
+    return _lib.get_native().row_norm(x, float(eps))
 
 
 class _HipInstanceNorm:
@@ -111,7 +55,7 @@ class _HipInstanceNorm:
         if not self._on_hip(x) or not x.requires_grad:
             return self(x), x
         self._check_input_dim(x)
-        return _RowNormSkip.apply(x, float(self.eps))
+        return _lib.get_native().row_norm_skip(x, float(self.eps))
 
 
 class InstanceNorm1d(_HipInstanceNorm, nn.InstanceNorm1d):
