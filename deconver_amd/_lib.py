@@ -57,6 +57,9 @@ EXPORTS = (
     "ndc_pointwise_gemm_parts",
     "ndc_pointwise_gemm_actgrad",
     "ndc_pointwise_gemm_masked",
+    "ndc_gemm",
+    "ndc_weight_grad_workspace_bytes",
+    "ndc_weight_grad",
 )
 
 
@@ -155,6 +158,11 @@ class NdcLibrary:
         d.ndc_pointwise_gemm_parts.argtypes = []
         d.ndc_pointwise_gemm_actgrad.argtypes = [vp, vp, vp, vp, vp, vp, ctypes.c_int64, ctypes.c_int64,
                                                  ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, vp]
+        i64 = ctypes.c_int64
+        d.ndc_gemm.argtypes = [vp, fp, ctypes.c_int, fp, vp, vp, vp, vp, i64, i64, i64, i64, ctypes.c_int, ctypes.c_int, vp]
+        d.ndc_weight_grad_workspace_bytes.restype = ctypes.c_size_t
+        d.ndc_weight_grad_workspace_bytes.argtypes = [i64, i64, i64, i64, ctypes.c_int]
+        d.ndc_weight_grad.argtypes = [vp, vp, fp, fp, i64, i64, i64, i64, ctypes.c_int, vp, ctypes.c_size_t, vp]
         d.ndc_regroup.argtypes = [vp, vp, vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                    ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]
         d.ndc_taps_bytes.restype = ctypes.c_size_t
@@ -342,6 +350,21 @@ class NdcLibrary:
         """``gz = (W gy) * act'(z + bias)`` with per-wavefront sums of ``gz`` in ``gpart``."""
         self._check(self._dll.ndc_pointwise_gemm_actgrad(gy, wfrag, bias, z, gz, gpart, batch, cin, cout, n,
                                                          act, dtype, stream), "ndc_pointwise_gemm_actgrad")
+
+    def gemm(self, x: int, w: int, transposed: bool, bias: Optional[int], residual: Optional[int], mask: Optional[int],
+             y: int, zkeep: Optional[int], batch: int, cin: int, cout: int, n: int, mode: int, dtype: int, stream) -> None:
+        """``y = epilogue(W x)`` on channel-first ``(batch, c, n)`` tensors of any size (see the header)."""
+        self._check(self._dll.ndc_gemm(x, w, int(transposed), bias, residual, mask, y, zkeep, batch, cin, cout, n, mode,
+                                       dtype, stream), "ndc_gemm")
+
+    def weight_grad_workspace_bytes(self, batch: int, rows: int, cols: int, n: int, dtype: int) -> int:
+        return int(self._dll.ndc_weight_grad_workspace_bytes(batch, rows, cols, n, dtype))
+
+    def weight_grad(self, gz: int, x: int, gw: int, gb: Optional[int], batch: int, rows: int, cols: int, n: int, dtype: int,
+                    workspace: Optional[int], workspace_bytes: int, stream) -> None:
+        """``gw = sum_b gz[b] x[b]^T`` and ``gb`` the row sums of ``gz``, float32."""
+        self._check(self._dll.ndc_weight_grad(gz, x, gw, gb, batch, rows, cols, n, dtype, workspace, workspace_bytes,
+                                              stream), "ndc_weight_grad")
 
     def chnorm_parts(self, batch: int, n: int, dtype: int) -> int:
         return int(self._dll.ndc_chnorm_parts(batch, n, dtype))

@@ -7,15 +7,17 @@
 from __future__ import annotations
 
 import argparse
+import concurrent.futures
 import os
 import subprocess
 import sys
+import tempfile
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-ffp-contract=fast",
     # packed-fp32 VALU forms are kept out of the generated code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -35,10 +37,17 @@ def _run(cmd):
     return out
 
 
-def build_hip(extra_flags=()) -> str:
-    out = os.path.join(_HERE, "libdeconver_ndc.so")
+HIP_SOURCES = ("ndc_capi.hip", "ndc_fused_bf16.hip", "ndc_fused_f32.hip", "ndc_gemm.hip")
+
+
+def build_hip(extra_flags=(), out: str = os.path.join(_HERE, "libdeconver_ndc.so"), csrc: str = CSRC) -> str:
+    """The HIP library: its translation units side by side, then one link."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-    _run([hipcc, *HIPCC_FLAGS, *extra_flags, "-o", out, os.path.join(CSRC, "ndc_capi.hip")])
+    with tempfile.TemporaryDirectory() as tmp, concurrent.futures.ThreadPoolExecutor() as pool:
+        objects = [os.path.join(tmp, name + ".o") for name in HIP_SOURCES]
+        list(pool.map(lambda so: _run([hipcc, *HIPCC_FLAGS, *extra_flags, "-c", os.path.join(csrc, so[0]), "-o", so[1]]),
+                      zip(HIP_SOURCES, objects)))
+        _run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", out, *objects])
     return out
 
 

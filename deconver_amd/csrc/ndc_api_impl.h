@@ -525,7 +525,7 @@ int ndc_pointwise_gemm_supported(int64_t cin, int64_t cout, int64_t n, int dtype
     if (dtype != NDC_BF16) return 0;
     // up to 256 input channels held whole in registers, any width of output; or many input
     // channels in chunks of 64 with the accumulators of at most 128 output channels
-    const bool whole = cin == 64 || cin == 128 || cin == 256;
+    const bool whole = cin == 32 || cin == 64 || cin == 128 || cin == 256;
     const bool deep = cin > 256 && cin % 64 == 0 && cin <= 4096 && cout <= 128;
     if (!whole && !deep) return 0;
     if (cout < 32 || cout % 32 || cout > 4096) return 0;
@@ -607,6 +607,108 @@ int ndc_pointwise_gemm_actgrad(const void *gy, const void *wfrag, const float *b
         return NDC_ERR_WORKSPACE;
     if (gz == gy || gz == z) return NDC_ERR_GEOMETRY;
     return ndc::Backend::pwgemm(gy, wfrag, bias, z, gz, nullptr, gpart, nullptr, batch, (int)cin, (int)cout, n, act + 2, stream);
+}
+
+// ---- the tiled GEMMs (ndc_gemm.h)
+
+static int gemm_check(long long batch, long long cin, long long cout, long long n, int dtype)
+{
+    if (dtype != NDC_F32 && dtype != NDC_BF16) return NDC_ERR_DTYPE;
+    if (batch < 1 || cin < 1 || cout < 1 || n < 1 || cin > (1 << 20) || cout > (1 << 20) || batch > (1 << 20)) return NDC_ERR_GEOMETRY;
+    if ((long double)batch * (cin > cout ? cin : cout) * n > 9.0e15L || n > (1 << 24)) return NDC_ERR_GEOMETRY;
+    return NDC_OK;
+}
+
+// Tile and split of a weight gradient.  The tile holds as much of the result as one workgroup's
+// registers take (each operand is read once per tile that shares it), unless the voxels are too
+// few to give 256 such tiles and splits, where 64 x 64 tiles spread the work wider.  The voxel
+// axis is split until the launch has 512 workgroups (256 with the largest tiles over long rows:
+// 0.55 ms against 0.56-0.68 for the 256 x 64 result over 2 x 128^3), in chunks of at least 256 voxels,
+// so that partial results stay small next to the operands.  Rows of half a million voxels and
+// more are read 16 granules at a time (see the kernel), shorter ones 8.
+static ndc::WgradPlan wgrad_plan(long long batch, long long rows, long long cols, long long n, int esz)
+{
+    ndc::WgradPlan w;
+    if (rows >= 192 && cols <= 64) w.bm = 256, w.bn = 64;
+    else if (cols >= 192 && rows <= 64) w.bm = 64, w.bn = 256;
+    else if (rows > 64 && cols > 64) w.bm = w.bn = 128;
+    else if (cols <= 32 && rows > 64) w.bm = 128, w.bn = 32;
+    else if (rows <= 32 && cols > 64) w.bm = 32, w.bn = 128;
+    else w.bm = w.bn = 64;
+    const long long most = n / 256 > 0 ? n / 256 : 1;             // splits of a sample
+    auto tiles_of = [&] { return ((rows + w.bm - 1) / w.bm) * ((cols + w.bn - 1) / w.bn); };
+    // (lane offsets within a tile are 32-bit: fewer rows per tile on enormous grids)
+    if (tiles_of() * most * batch < 256 || (long double)(w.bm > w.bn ? w.bm : w.bn) * n * esz > 4.0e9L) w.bm = w.bn = 64;
+    w.depth = esz == 2 && n >= (1 << 19) ? 16 : 8;
+    const long long stage = 16 / esz * w.depth, tiles = tiles_of();   // voxels per stage
+    const long long want = w.bm + w.bn == 320 && n >= (1 << 19) ? 256 : 512;
+    long long per = (want + tiles * batch - 1) / (tiles * batch);
+    if (per > most) per = most;
+    w.chunk = ((n + per - 1) / per + stage - 1) / stage * stage;
+    w.per_sample = (int)((n + w.chunk - 1) / w.chunk);
+    return w;
+}
+
+size_t ndc_weight_grad_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int64_t n, int dtype)
+{
+    if (gemm_check(batch, cols, rows, n, dtype)) return 0;
+    const ndc::WgradPlan w = wgrad_plan(batch, rows, cols, n, dtype == NDC_BF16 ? 2 : 4);
+    const long long splits = batch * w.per_sample;
+    return splits == 1 ? 0 : (size_t)splits * (size_t)(rows * cols + rows) * 4;
+}
+
+int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t batch, int64_t rows, int64_t cols,
+                    int64_t n, int dtype, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!gz || !x || !gw) return NDC_ERR_NULL;
+    int st = gemm_check(batch, cols, rows, n, dtype);
+    if (st) return st;
+    const size_t need = ndc_weight_grad_workspace_bytes(batch, rows, cols, n, dtype);
+    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15u))) return NDC_ERR_WORKSPACE;
+    const int esz = dtype == NDC_BF16 ? 2 : 4;
+    if (((uintptr_t)gz | (uintptr_t)x) & (uintptr_t)(esz - 1)) return NDC_ERR_WORKSPACE;
+    const ndc::WgradPlan w = wgrad_plan(batch, rows, cols, n, esz);
+    const long long splits = batch * w.per_sample, out = rows * cols;
+    const long long blocks = ((splits + 7) / 8 * 8) * ((rows + w.bm - 1) / w.bm) * ((cols + w.bn - 1) / w.bn);
+    if (blocks > 0x7fffffffLL || out + rows > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
+    float *part = need ? (float *)workspace : nullptr;
+    st = ndc::Backend::wgrad(gz, x, gw, gb, part, batch, (int)rows, (int)cols, n, esz, w, stream);
+    if (st || !part) return st;
+    const int total = (int)(out + (gb ? rows : 0)), nout = (int)out;
+    const long long stride = out + rows;
+    return ndc::Backend::strided_sum(total, (int)splits, stream,
+                                     [=] NDC_LAMBDA(int o, float v) { if (o < nout) gw[o] = v; else gb[o - nout] = v; },
+                                     [=] NDC_LAMBDA(int o, int s) { return part[s * stride + o]; });
+}
+
+int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, const void *residual, const void *mask,
+             void *y, void *zkeep, int64_t batch, int64_t cin, int64_t cout, int64_t n, int mode, int dtype,
+             void *stream)
+{
+    if (!x || !w || !y) return NDC_ERR_NULL;
+    int st = gemm_check(batch, cin, cout, n, dtype);
+    if (st) return st;
+    if (mode < NDC_ACT_NONE || mode > NDC_GEMM_GELU_GRAD || mode == 3) return NDC_ERR_GEOMETRY;
+    const bool grad = mode == NDC_GEMM_GELU_GRAD, act = mode == NDC_ACT_RELU || mode == NDC_ACT_GELU;
+    if (grad && !residual) return NDC_ERR_NULL;
+    if (mask && mode != NDC_ACT_NONE) return NDC_ERR_GEOMETRY;
+    if (zkeep && !act) return NDC_ERR_GEOMETRY;
+    if ((act && transposed) || (grad && !transposed)) return NDC_ERR_GEOMETRY;   // forms no caller has
+    const uintptr_t all = (uintptr_t)x | (uintptr_t)y | (uintptr_t)residual | (uintptr_t)mask | (uintptr_t)zkeep;
+    if (all & (uintptr_t)((dtype == NDC_BF16 ? 2 : 4) - 1) || ((uintptr_t)w & 3u) || ((uintptr_t)bias & 3u)) return NDC_ERR_WORKSPACE;
+    if (y == x || zkeep == x || (zkeep && zkeep == y)) return NDC_ERR_GEOMETRY;
+    // Small grids -- at most four workgroups of 32 rows x 64 voxels per CU -- take the form that
+    // slices the channels over the wavefronts (waves = 0): 128 -> 512 channels over 4096 voxels in
+    // bf16 8.1 us against 10.2 tiled, over 32 768 (4096 workgroups) 24 against 11.5.  Otherwise as
+    // many output rows per workgroup (32 per wavefront) as still leave two workgroups per CU.
+    const int esz = dtype == NDC_BF16 ? 2 : 4;
+    const long long vt = batch * ((n + 127) / 128), small = batch * ((n + 63) / 64) * ((cout + 31) / 32);
+    int waves = 4;
+    while (waves > 1 && (cout <= 32 * (waves / 2) || vt * ((cout + 32 * waves - 1) / (32 * waves)) < 512)) waves /= 2;
+    if (small <= 1024 && cin % (16 / esz) == 0 && n >= 2) waves = 0;
+    if ((vt + 8) * 2 * ((cout + 31) / 32 + 8) > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
+    return ndc::Backend::tile_gemm(x, w, transposed != 0, bias, residual, mask, y, zkeep, batch, (int)cin, (int)cout, n,
+                                   mode, esz, waves, stream);
 }
 
 static int chnorm_check(long long B, long long C, long long n, int dtype)

@@ -308,7 +308,7 @@ template <class BE> static int prepare_taps(const KGeom &q, const float *h, floa
 }
 
 template <class BE, typename T>
-static int forward(const KGeom &q, const T *x, const T *z, const float *h, const float *bias,
+int forward(const KGeom &q, const T *x, const T *z, const float *h, const float *bias,
                    T *out, T *t1, T *s_over_den, T *ratio, const float *taps, void *ws,
                    void *stream)
 {
@@ -358,7 +358,7 @@ static int forward(const KGeom &q, const T *x, const T *z, const float *h, const
 }
 
 template <class BE, typename T>
-static int backward(const KGeom &q, const T *x, const T *z, const T *t1, const T *s_over_den,
+int backward(const KGeom &q, const T *x, const T *z, const T *t1, const T *s_over_den,
                     const T *ratio, const float *h, const float *bias, const T *gout, T *gx,
                     T *gz, float *gh, float *gb, const float *taps, void *ws, void *stream,
                     float *pass_ms = nullptr)
@@ -485,6 +485,14 @@ static int backward(const KGeom &q, const T *x, const T *z, const T *t1, const T
     tm.finish(pass_ms, 3);
     return NDC_OK;
 }
+
+// the two above for one backend and storage type, to declare (`extern template`) or instantiate
+#define NDC_FUSED_ENTRY_POINTS(KIND, T)                                                            \
+    KIND int forward<Backend, T>(const KGeom &, const T *, const T *, const float *, const float *, \
+                                 T *, T *, T *, T *, const float *, void *, void *);               \
+    KIND int backward<Backend, T>(const KGeom &, const T *, const T *, const T *, const T *,        \
+                                  const T *, const float *, const float *, const T *, T *, T *,     \
+                                  float *, float *, const float *, void *, void *, float *);
 
 }  // namespace fused
 }  // namespace ndc

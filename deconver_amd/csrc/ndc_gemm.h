@@ -1,0 +1,629 @@
+// The remaining GEMMs of the 1x1 projections on channel-first tensors, float32 and bf16:
+//
+//   tile_kernel    y[b] = epilogue(W x[b])        (forward and input gradient, layers/linear.py:53-58
+//                                                  of the reference with its callers' tails)
+//   wgrad_kernel   gw = sum_b gz[b] x[b]^T,       (weight gradient, with the bias gradient
+//                  gb = row sums of gz             sum_{b,v} gz from the same pass)
+//
+// What the streaming GEMM of ndc_pwgemm.h does not take ends up here: float32 storage, the wide
+// levels whose weights do not fit LDS, odd voxel counts, small grids.  Both kernels are ordinary
+// LDS-tiled matrix-instruction GEMMs; what is particular to them:
+//
+//   * Unit of staging is a 16-byte granule: 8 bf16 or 4 float32 values of consecutive k for one
+//     row (one column) of the operand, which is what a lane hands v_mfma_f32_32x32x16_bf16, or,
+//     element after element, four v_mfma_f32_32x32x2_f32.  A stage is 8 granules deep (64 bf16 or
+//     32 float32 k-values); granule (row r, depth q) sits at slot q * rows + (r ^ q), so that
+//     neither its writer (8 lanes along q, for operands contiguous in k) nor its readers (32 lanes
+//     along r) meet a bank twice.
+//   * Whatever order the instruction takes its k-values in, both operands are filled by one rule
+//     (lane half kb, element e <-> k = (2 step + kb) * E + e), so the products pair up.
+//   * The weight comes in as it lies (float32, rows of W or of its transpose): no packing launch
+//     and no cast copy.
+//   * Voxel counts of any size and tensors of any alignment: ragged ends are filled with zeros
+//     element by element, rows that are not 16-byte aligned are read with unaligned vector loads.
+//
+// Sums are float32 in a fixed order (partial results of the split voxel axis are added in order
+// by a second launch): results are reproducible.  Device code only.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+#include <type_traits>
+#include "ndc_common.h"
+#include "ndc_epilogue.h"
+
+namespace ndc {
+namespace gemm {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// the same at any element alignment
+typedef u32x4 u32x4_a2 __attribute__((aligned(2), may_alias));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2), may_alias));
+
+static const int kDepth = 8;              // granules per stage along k
+
+template <typename T> struct Gran;        // E elements of consecutive k in 16 bytes
+template <> struct Gran<float> {
+    static constexpr int E = 4;
+    static __device__ u32x4 pack(const float (&v)[4])
+    {
+        u32x4 r = {__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])};
+        return r;
+    }
+    static __device__ float sum(u32x4 g)
+    {
+        return (__uint_as_float(g[0]) + __uint_as_float(g[1])) + (__uint_as_float(g[2]) + __uint_as_float(g[3]));
+    }
+    static __device__ f32x16 mma(u32x4 a, u32x4 b, f32x16 acc)
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a[j]), __uint_as_float(b[j]), acc, 0, 0, 0);
+        return acc;
+    }
+};
+template <> struct Gran<bf16_t> {
+    static constexpr int E = 8;
+    static __device__ u32x4 pack(const float (&v)[8])
+    {
+        u32x4 r = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+        return r;
+    }
+    static __device__ float sum(u32x4 g)
+    {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s += __uint_as_float(g[i] << 16) + __uint_as_float(g[i] & 0xffff0000u);
+        return s;
+    }
+    static __device__ f32x16 mma(u32x4 a, u32x4 b, f32x16 acc)
+    {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+    }
+};
+
+// Granule slot.  Rows of a stage: a multiple of 32.
+__device__ inline int slot(int rows, int q, int r) { return q * rows + (r ^ q); }
+
+// E elements from `p` of which the first `have` exist (the rest read as zero)
+template <typename T> __device__ inline u32x4 ragged(const T *p, int have)
+{
+    constexpr int E = Gran<T>::E;
+    float v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = e < have ? Elem<T>::load(p + e) : 0.f;
+    return Gran<T>::pack(v);
+}
+
+// ---------------------------------------------------------------------------- weight gradient
+
+struct WgradParams {
+    const void *a, *b;      // (batch, rows, n) and (batch, cols, n)
+    float *part;            // split results: (splits, rows * cols + rows), or null with one split
+    float *gw, *gb;         // (rows, cols); (rows) or null.  Written here when there is one split
+    long long n, chunk;     // voxels per sample; voxels per split, a multiple of a stage's depth
+    int rows, cols, tiles_m, tiles_n;
+    int per_sample, splits; // splits of a sample; batch * per_sample
+};
+
+// Tile of 32 WM RT rows x 32 WN CT columns, WM x WN wavefronts of RT x CT matrix tiles each; a
+// stage is D granules deep.  Bound by memory: a 64 x 64 gradient over 2 x 128^3 voxels in bf16 takes
+// 0.19 ms (5.6 TB/s on both operands; 0.27 ms as a batch of library GEMMs plus the sum of their
+// results), a 64 x 64 one over 183 645 voxels 0.02 ms, a 256 x 64 one 0.04 ms (0.26 ms: the library
+// does not split that axis).  What decides is how the loads fall on memory: rows lie megabytes
+// apart, so few workgroups with long runs per row (D = 16: 256 bytes) beat many with short ones --
+// 512 workgroups, D 16: 192 us; 2048, D 8: 351 us.
+template <typename T, int WM, int WN, int RT, int CT, int D>
+__global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
+{
+    typedef Gran<T> G;
+    constexpr int NT = 64 * WM * WN, BM = 32 * WM * RT, BN = 32 * WN * CT, E = G::E, BK = D * E;
+    constexpr int NA = BM * D / NT, NB = BN * D / NT;   // granules a thread stages
+    static_assert(NA * NT == BM * D && NB * NT == BN * D, "whole granules per thread");
+    __shared__ __attribute__((aligned(16))) u32x4 lds[(BM + BN) * D];
+    // all tiles of a split run on one XCD one after the other (workgroups go round-robin over the
+    // eight XCDs), so that what they share of the operands comes out of that XCD's L2
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
+    const int tile = pos % tiles, split = (pos / tiles) * 8 + xcd;
+    if (split >= p.splits) return;
+    const int m0 = (tile / p.tiles_n) * BM, n0 = (tile % p.tiles_n) * BN;
+    const int sample = __builtin_amdgcn_readfirstlane(split / p.per_sample);
+    const long long k_lo = (long long)(split % p.per_sample) * p.chunk;
+    const long long k_hi = k_lo + p.chunk < p.n ? k_lo + p.chunk : p.n;
+    const int tid = threadIdx.x, q = tid % D, r0 = tid / D;
+    const T *A = (const T *)p.a + ((long long)sample * p.rows + m0) * p.n;   // (uniform)
+    const T *B = (const T *)p.b + ((long long)sample * p.cols + n0) * p.n;
+    const bool want_sums = p.gb != nullptr && n0 == 0;
+    u32x4 ra[NA], rb[NB];
+    float sums[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) sums[i] = 0.f;
+
+    // Rows past the end repeat the last one: what they contribute is never stored.  Addresses are a
+    // uniform pointer plus a 32-bit lane offset (the caller keeps a tile's rows below 4 GiB): as
+    // 64-bit lane addresses they took the registers of a third resident wavefront.
+    uint32_t off_a[NA], off_b[NB];
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+        off_a[i] = ((uint32_t)min(r0 + i * (NT / D), p.rows - 1 - m0) * (uint32_t)p.n + q * E) * (uint32_t)sizeof(T);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+        off_b[i] = ((uint32_t)min(r0 + i * (NT / D), p.cols - 1 - n0) * (uint32_t)p.n + q * E) * (uint32_t)sizeof(T);
+    auto fetch = [&](long long k0) {
+        const char *a = (const char *)(A + k0), *b = (const char *)(B + k0);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) ra[i] = *(const u32x4_a2 *)(a + off_a[i]);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) rb[i] = *(const u32x4_a2 *)(b + off_b[i]);
+    };
+    auto fetch_ragged = [&](long long k0) {
+        const char *a = (const char *)(A + k0), *b = (const char *)(B + k0);
+        const long long rest = k_hi - k0 - (long long)q * E;
+        const int have = rest < 0 ? 0 : rest < E ? (int)rest : E;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) ra[i] = ragged<T>((const T *)(a + off_a[i]), have);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) rb[i] = ragged<T>((const T *)(b + off_b[i]), have);
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            lds[slot(BM, q, r0 + i * (NT / D))] = ra[i];
+            if (want_sums) sums[i] += G::sum(ra[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) lds[BM * D + slot(BN, q, r0 + i * (NT / D))] = rb[i];
+    };
+
+    const int lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN, l32 = lane & 31, kb = lane >> 5;
+    f32x16 acc[RT][CT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) acc[i][j] = f32x16{};
+    auto multiply = [&]() {
+#pragma unroll
+        for (int s = 0; s < D / 2; ++s) {
+            u32x4 fa[RT], fb[CT];
+            const int d = 2 * s + kb;
+#pragma unroll
+            for (int i = 0; i < RT; ++i) fa[i] = lds[slot(BM, d, 32 * (wm * RT + i) + l32)];
+#pragma unroll
+            for (int j = 0; j < CT; ++j) fb[j] = lds[BM * D + slot(BN, d, 32 * (wn * CT + j) + l32)];
+#pragma unroll
+            for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int j = 0; j < CT; ++j) acc[i][j] = G::mma(fa[i], fb[j], acc[i][j]);
+        }
+    };
+    // Whole stages in a loop without conditions: the next stage's loads are in flight while this
+    // one multiplies.  (A branch between the two forms of fetch inside the loop made every stage
+    // wait for its loads before it multiplied.)
+    const int stages = (int)((k_hi - k_lo) / BK);
+    if (stages > 0) fetch(k_lo);
+    for (int s = 0; s < stages; ++s) {
+        put();
+        __syncthreads();
+        fetch(k_lo + (long long)(s + 1 < stages ? s + 1 : s) * BK);
+        multiply();
+        __syncthreads();
+    }
+    if (k_lo + (long long)stages * BK < k_hi) {
+        fetch_ragged(k_lo + (long long)stages * BK);
+        put();
+        __syncthreads();
+        multiply();
+    }
+    const long long out_size = (long long)p.rows * p.cols;
+    float *gw = p.part ? p.part + split * (out_size + p.rows) : p.gw;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            const int col = n0 + 32 * (wn * CT + j) + l32;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = m0 + 32 * (wm * RT + i) + 8 * (e / 4) + 4 * kb + e % 4;
+                if (row < p.rows && col < p.cols) gw[(long long)row * p.cols + col] = acc[i][j][e];
+            }
+        }
+    if (want_sums) {
+        float *gb = p.part ? p.part + split * (out_size + p.rows) + out_size : p.gb;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            float s = sums[i];
+#pragma unroll
+            for (int o = 1; o < D; o *= 2) s += __shfl_xor(s, o);
+            const int row = m0 + r0 + i * (NT / D);
+            if (q == 0 && row < p.rows) gb[row] = s;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------- y = epilogue(W x)
+
+struct TileParams {
+    const void *x;           // (batch, cin, n)
+    const float *w;          // W (cout, cin), or (cin, cout) storage of it
+    const float *bias;       // cout values or null
+    const void *res;         // (batch, cout, n) or null: added to y; with a gradient mode the
+                             // pre-activation whose derivative (at res + bias) multiplies the product
+    const void *mask;        // (batch, cout, n) or null: y is zero where mask <= 0
+    void *y, *zkeep;         // (batch, cout, n); zkeep or null: the product before bias and activation
+    long long n;
+    int cin, cout, tiles_m, tiles_n, batch;
+};
+
+// modes: epilogue::kNone / kRelu / kGelu, and the product times the GELU's derivative
+enum { kGeluGrad = 4 };
+
+template <typename T> struct Quad;   // 4 voxels of one row
+template <> struct Quad<float> {
+    f32x4 v;
+    __device__ float get(int i) const { return v[i]; }
+    __device__ void load(const float *p) { v = __builtin_bit_cast(f32x4, *(const u32x4_a2 *)p); }
+    __device__ void store(float *p) const { *(u32x4_a2 *)p = __builtin_bit_cast(u32x4, v); }
+    __device__ void set(const float (&f)[4]) { v = f32x4{f[0], f[1], f[2], f[3]}; }
+};
+template <> struct Quad<bf16_t> {
+    u32x2 v;
+    __device__ float get(int i) const
+    {
+        const uint32_t w = v[i >> 1];
+        return __uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16));
+    }
+    __device__ void load(const bf16_t *p) { v = *(const u32x2_a2 *)p; }
+    __device__ void store(bf16_t *p) const { *(u32x2_a2 *)p = v; }
+    __device__ void set(const float (&f)[4]) { v = u32x2{pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3])}; }
+};
+
+template <typename T> __device__ inline Quad<T> load_quad(const T *p, int have)
+{
+    Quad<T> r;
+    if (have >= 4) {
+        r.load(p);
+    } else {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = i < have ? Elem<T>::load(p + i) : 0.f;
+        r.set(v);
+    }
+    return r;
+}
+template <typename T> __device__ inline void store_quad(T *p, const float (&f)[4], int have)
+{
+    if (have >= 4) {
+        Quad<T> r;
+        r.set(f);
+        r.store(p);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (i < have) Elem<T>::store(p + i, f[i]);
+    }
+}
+
+// (E rows of k) x (4 voxels) -> four granules
+template <typename T> __device__ inline void transpose(const Quad<T> (&in)[Gran<T>::E], u32x4 (&out)[4])
+{
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[c][e] = __float_as_uint(in[e].v[c]);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int pr = 0; pr < 4; ++pr) {
+                out[2 * h][pr] = __builtin_amdgcn_perm(in[2 * pr + 1].v[h], in[2 * pr].v[h], 0x05040100u);
+                out[2 * h + 1][pr] = __builtin_amdgcn_perm(in[2 * pr + 1].v[h], in[2 * pr].v[h], 0x07060302u);
+            }
+    }
+}
+
+// The epilogue of NR consecutive rows of four voxels: z the products, `have` of the four voxels
+// exist (`whole`: all of them, in every lane).  What it reads is requested ahead of its stores.
+template <typename T, int MODE, int NR>
+__device__ inline void finish(const TileParams &p, const float (&z)[NR][4], int row0, long long base, int have, bool whole)
+{
+    auto run = [&](auto tag) {
+        constexpr bool WHOLE = decltype(tag)::value;
+        Quad<T> rq[NR], mq[NR];
+        float bias[NR];
+#pragma unroll
+        for (int e = 0; e < NR; ++e) {
+            const int row = min(row0 + e, p.cout - 1);
+            const long long at = base + (long long)row * p.n;
+            bias[e] = p.bias ? p.bias[row] : 0.f;
+            if (p.res) rq[e] = load_quad<T>((const T *)p.res + at, WHOLE ? 4 : have);
+            if (p.mask) mq[e] = load_quad<T>((const T *)p.mask + at, WHOLE ? 4 : have);
+        }
+#pragma unroll
+        for (int e = 0; e < NR; ++e) {
+            if (row0 + e >= p.cout) continue;
+            const long long at = base + (long long)(row0 + e) * p.n;
+            float y[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (MODE == kGeluGrad) {
+                    y[j] = z[e][j] * epilogue::act_grad<epilogue::kGelu>(rq[e].get(j) + bias[e]);
+                } else {
+                    y[j] = epilogue::act_fwd<MODE>(z[e][j] + bias[e]);
+                    if (p.res) y[j] += rq[e].get(j);
+                    if (p.mask) y[j] = mq[e].get(j) > 0.f ? y[j] : 0.f;
+                }
+            }
+            if constexpr (MODE == epilogue::kRelu || MODE == epilogue::kGelu)
+                if (p.zkeep) store_quad<T>((T *)p.zkeep + at, z[e], WHOLE ? 4 : have);
+            store_quad<T>((T *)p.y + at, y, WHOLE ? 4 : have);
+        }
+    };
+    if (whole) run(std::true_type{});
+    else run(std::false_type{});
+}
+
+// A workgroup of WAVES wavefronts makes a tile of 32 WAVES output rows x 128 voxels.  Voxel
+// v of the tile is column v / 4 of matrix tile v % 4, so that a lane ends up with four
+// consecutive voxels of a row: stores (and the loads of residual, mask and kept product) are 8
+// or 16 bytes per lane, 32 lanes contiguous.
+template <typename T, bool WT, int WAVES, int MODE>
+__global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
+{
+    typedef Gran<T> G;
+    constexpr int NT = 64 * WAVES, BM = 32 * WAVES, BN = 128, E = G::E, BK = kDepth * E;
+    constexpr int NA = BM * kDepth / NT;             // weight granules a thread stages
+    constexpr int NB = 32 * kDepth / NT;             // voxel quads a thread stages
+    static_assert(NA * NT == BM * kDepth && NB * NT == 32 * kDepth, "whole granules per thread");
+    __shared__ __attribute__((aligned(16))) u32x4 lds[(BM + BN) * kDepth];
+    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
+    const int tile_m = pos % p.tiles_m, vt = (pos / p.tiles_m) * 8 + xcd;   // a voxel tile stays on one XCD
+    if (vt >= p.tiles_n * p.batch) return;
+    const int sample = vt / p.tiles_n, m0 = tile_m * BM;
+    const long long v0 = (long long)(vt % p.tiles_n) * BN;
+    const int tid = threadIdx.x;
+    const T *X = (const T *)p.x + (long long)sample * p.cin * p.n + v0;
+    const float *W = p.w;
+    const int left = (int)(p.n - v0 < BN ? p.n - v0 : BN);   // voxels of this tile
+
+    float rw[NA][E];
+    Quad<T> rx[NB][E];
+    auto weight_at = [&](int i, int &r, int &q) {   // granule i of this thread
+        const int g = tid + i * NT;
+        if (WT) r = g % BM, q = g / BM;             // lanes along the rows of W, contiguous in W^T
+        else r = g >> 3, q = g & 7;
+    };
+    // Whole granules and quads (all but the narrow first layers and the last voxel tile of an odd
+    // count): loads without conditions, and nothing done to their values before `put`, so that a
+    // stage's loads stay in flight while the stage before it multiplies.  Rows and quads past the
+    // end repeat the last one -- their results are never stored --, depths past the end are zeroed.
+    const bool whole = p.cin % E == 0 && left % 4 == 0;
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            int r, q;
+            weight_at(i, r, q);
+            const int m = min(m0 + r, p.cout - 1), k = min(k0 + q * E, p.cin - E);
+            if constexpr (WT) {
+#pragma unroll
+                for (int e = 0; e < E; ++e) rw[i][e] = W[(long long)(k + e) * p.cout + m];
+            } else {
+#pragma unroll
+                for (int h = 0; h < E / 4; ++h) {
+                    Quad<float> t;
+                    t.load(W + (long long)m * p.cin + k + 4 * h);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rw[i][4 * h + e] = t.get(e);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int u = tid + i * NT, c = min(u & 31, left / 4 - 1), k = min(k0 + (u >> 5) * E, p.cin - E);
+            const T *src = X + (long long)k * p.n + 4 * c;
+#pragma unroll
+            for (int e = 0; e < E; ++e) rx[i][e].load(src + (long long)e * p.n);
+        }
+    };
+    auto fetch_ragged = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            int r, q;
+            weight_at(i, r, q);
+            const int m = m0 + r, k = k0 + q * E, have = m < p.cout ? p.cin - k : 0;
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                rw[i][e] = e < have ? W[WT ? (long long)(k + e) * p.cout + m : (long long)m * p.cin + k + e] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int u = tid + i * NT, c = u & 31, k = k0 + (u >> 5) * E;
+            const T *src = X + (long long)k * p.n + 4 * c;
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                rx[i][e] = load_quad<T>(src + (long long)e * p.n, k + e < p.cin ? left - 4 * c : 0);
+        }
+    };
+    auto put = [&](int k0) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            int r, q;
+            weight_at(i, r, q);
+            const uint32_t keep = k0 + q * E < p.cin ? ~0u : 0u;
+            u32x4 g = G::pack(rw[i]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) g[e] &= keep;
+            lds[slot(BM, q, r)] = g;
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int u = tid + i * NT, c = u & 31, q = u >> 5;
+            const uint32_t keep = k0 + q * E < p.cin ? ~0u : 0u;
+            u32x4 g[4];
+            transpose<T>(rx[i], g);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) g[j][e] &= keep;
+                lds[BM * kDepth + slot(BN, q, 32 * j + c)] = g[j];
+            }
+        }
+    };
+
+    const int lane = tid & 63, wave = tid >> 6, l32 = lane & 31, kb = lane >> 5;
+    f32x16 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = f32x16{};
+    auto multiply = [&](int k0) {
+        const int steps = p.cin - k0 >= BK ? kDepth / 2 : (p.cin - k0 + 2 * E - 1) / (2 * E);
+        for (int s = 0; s < steps; ++s) {
+            const int d = 2 * s + kb;
+            const u32x4 fa = lds[slot(BM, d, 32 * wave + l32)];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j] = G::mma(fa, lds[BM * kDepth + slot(BN, d, 32 * j + l32)], acc[j]);
+        }
+    };
+    if (whole) {
+        fetch(0);
+        for (int k0 = 0; k0 < p.cin; k0 += BK) {
+            put(k0);
+            __syncthreads();
+            if (k0 + BK < p.cin) fetch(k0 + BK);
+            multiply(k0);
+            __syncthreads();
+        }
+    } else {
+        for (int k0 = 0; k0 < p.cin; k0 += BK) {
+            fetch_ragged(k0);
+            put(k0);
+            __syncthreads();
+            multiply(k0);
+            __syncthreads();
+        }
+    }
+    const int have = left - 4 * l32;
+    if (have <= 0) return;
+    const long long base = (long long)sample * p.cout * p.n + v0 + 4 * l32;
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+        float z[4][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) z[e][j] = acc[j][4 * h + e];
+        finish<T, MODE, 4>(p, z, m0 + 32 * wave + 8 * h + 4 * kb, base, have, whole);
+    }
+}
+
+// ---------------------------------------------------------------------------- small grids
+
+// A grid of a few thousand voxels leaves the tiled kernel a handful of workgroups that walk the
+// channels one stage after the other, each stage waiting for memory (2048 -> 512 channels over
+// 64 voxels: 32 stages, 195 us).  Here the channels are split over the wavefronts of a workgroup
+// instead: a tile is 32 output rows x 64 voxels, wavefront w takes its share of the channels
+// straight from memory into the operand registers (kAhead steps requested together, no staging,
+// no barrier), and the wavefronts' partial tiles are added through LDS, in order.  Lanes hold
+// voxel pairs: pair c is column c of an even-voxel and an odd-voxel matrix tile.
+static const int kMaxSlices = 8;
+
+template <typename T, bool WT, int MODE>
+__global__ void __launch_bounds__(64 * kMaxSlices) sliced_kernel(TileParams p)
+{
+    typedef Gran<T> G;
+    constexpr int E = G::E, kAhead = 4;              // steps whose operands are in flight
+    __shared__ __attribute__((aligned(16))) float part[kMaxSlices][32][64];
+    // the voxel tiles of a row tile run on one XCD: they read the same rows of W
+    const int vts = p.tiles_n * p.batch;
+    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
+    const int tile_m = (pos / vts) * 8 + xcd, vt = pos % vts;
+    if (tile_m >= p.tiles_m) return;
+    const int sample = vt / p.tiles_n, m0 = tile_m * 32;
+    const int v0 = (vt % p.tiles_n) * 64, left = min((int)p.n - v0, 64);
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, kb = lane >> 5, slices = blockDim.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const T *X = (const T *)p.x + (long long)sample * p.cin * p.n + v0;
+    const int m = min(m0 + l32, p.cout - 1);
+    // pairs past the end repeat the last one; the half pair at the end of an odd count is the
+    // second element of the pair before it
+    const bool half = 2 * l32 + 1 == left;
+    const int c = min(2 * l32, left - 2);   // (-1 in a tile of one voxel: n >= 2)
+    const int steps = (p.cin + 2 * E - 1) / (2 * E), per = (steps + slices - 1) / slices;
+    const int s_lo = wave * per, s_hi = min(s_lo + per, steps);
+    typedef typename std::conditional<sizeof(T) == 2, uint32_t, u32x2>::type Pair;   // two voxels
+    typedef Pair Pair_a2 __attribute__((aligned(2), may_alias));
+    float w[kAhead][E];
+    Pair xv[kAhead][E];
+    auto request = [&](int a, int s) {
+        const int k = min((2 * s + kb) * E, p.cin - E);   // (the caller has checked cin % E == 0, n >= 2)
+        if constexpr (WT) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) w[a][e] = p.w[(long long)(k + e) * p.cout + m];
+        } else {
+#pragma unroll
+            for (int h = 0; h < E / 4; ++h) {
+                Quad<float> t;
+                t.load(p.w + (long long)m * p.cin + k + 4 * h);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[a][4 * h + e] = t.get(e);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) xv[a][e] = *(const Pair_a2 *)(X + (long long)(k + e) * p.n + c);
+    };
+    f32x16 acc0 = {}, acc1 = {};
+    const uint32_t second = half ? ~0u : 0u;
+    auto multiply = [&](int a, int s) {
+        // (masks instead of selects: a condition here becomes a branch around the loads' first use)
+        const uint32_t keep = (2 * s + kb) * E < p.cin ? ~0u : 0u;
+        u32x4 gw = G::pack(w[a]), g0, g1;
+        if constexpr (sizeof(T) == 2) {
+#pragma unroll
+            for (int pr = 0; pr < 4; ++pr) {
+                const uint32_t e0 = xv[a][2 * pr] >> (second & 16u), e1 = xv[a][2 * pr + 1] >> (second & 16u);
+                g0[pr] = __builtin_amdgcn_perm(e1, e0, 0x05040100u) & keep;
+                g1[pr] = __builtin_amdgcn_perm(xv[a][2 * pr + 1], xv[a][2 * pr], 0x07060302u) & keep;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                g0[e] = ((xv[a][e][0] & ~second) | (xv[a][e][1] & second)) & keep;
+                g1[e] = xv[a][e][1] & keep;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) gw[e] &= keep;
+        acc0 = G::mma(gw, g0, acc0);
+        acc1 = G::mma(gw, g1, acc1);
+    };
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a)
+        if (s_lo + a < s_hi) request(a, s_lo + a);
+    for (int s0 = s_lo; s0 < s_hi; s0 += kAhead) {
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) {
+            if (s0 + a < s_hi) multiply(a, s0 + a);
+            if (s0 + a + kAhead < s_hi) request(a, s0 + a + kAhead);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+        *reinterpret_cast<float2 *>(&part[wave][8 * (j / 4) + 4 * kb + j % 4][2 * l32]) = make_float2(acc0[j], acc1[j]);
+    __syncthreads();
+    for (int t = tid; t < 32 * 16; t += blockDim.x) {
+        const int row = t >> 4, q = t & 15, have = left - 4 * q;
+        if (m0 + row >= p.cout || have <= 0) continue;
+        float z[1][4] = {{0.f, 0.f, 0.f, 0.f}};
+        for (int w = 0; w < slices; ++w) {
+            const float4 v = *reinterpret_cast<const float4 *>(&part[w][row][4 * q]);
+            z[0][0] += v.x, z[0][1] += v.y, z[0][2] += v.z, z[0][3] += v.w;
+        }
+        finish<T, MODE, 1>(p, z, m0 + row, (long long)sample * p.cout * p.n + v0 + 4 * q, have, false);
+    }
+}
+
+}  // namespace gemm
+}  // namespace ndc

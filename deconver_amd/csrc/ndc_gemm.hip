@@ -1,0 +1,85 @@
+// Launches of the tiled GEMMs; see ndc_gemm.h.
+#include <hip/hip_runtime.h>
+
+#include "ndc_gemm.h"
+#include "ndc_gemm_host.h"
+
+namespace ndc {
+namespace gemm {
+
+// the tile of a weight gradient's workgroup: rows x columns, by what the result holds
+template <typename T, int WM, int WN, int RT, int CT, int D>
+static void wgrad_launch(WgradParams p, void *stream)
+{
+    const unsigned blocks = 8u * (unsigned)((p.splits + 7) / 8) * (unsigned)(p.tiles_m * p.tiles_n);
+    hipLaunchKernelGGL((wgrad_kernel<T, WM, WN, RT, CT, D>), dim3(blocks), dim3(64 * WM * WN), 0,
+                       (hipStream_t)stream, p);
+}
+template <typename T, int D> static void wgrad_t(const WgradParams &p, int bm, int bn, void *stream)
+{
+    if (bm == 256) wgrad_launch<T, 4, 1, 2, 2, D>(p, stream);
+    else if (bn == 256) wgrad_launch<T, 1, 4, 2, 2, D>(p, stream);
+    else if (bm == 128 && bn == 128) wgrad_launch<T, 2, 2, 2, 2, D>(p, stream);
+    else if (bm == 128) wgrad_launch<T, 4, 1, 1, 1, D>(p, stream);
+    else if (bn == 128) wgrad_launch<T, 1, 4, 1, 1, D>(p, stream);
+    else wgrad_launch<T, 2, 2, 1, 1, D>(p, stream);
+}
+int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long long batch, int rows, int cols,
+                 long long n, int esz, const WgradPlan &plan, void *stream)
+{
+    WgradParams p;
+    p.a = a, p.b = b, p.part = part, p.gw = gw, p.gb = gb, p.n = n, p.chunk = plan.chunk, p.rows = rows, p.cols = cols;
+    p.tiles_m = (rows + plan.bm - 1) / plan.bm, p.tiles_n = (cols + plan.bn - 1) / plan.bn;
+    p.per_sample = plan.per_sample, p.splits = (int)batch * plan.per_sample;
+    if (esz == 4) wgrad_t<float, 8>(p, plan.bm, plan.bn, stream);
+    else if (plan.depth == 16) wgrad_t<bf16_t, 16>(p, plan.bm, plan.bn, stream);
+    else wgrad_t<bf16_t, 8>(p, plan.bm, plan.bn, stream);
+    return 0;
+}
+
+template <typename T, bool WT, int MODE> static void tile_gemm_w(TileParams p, int waves, void *stream)
+{
+    if (waves == 0) {   // small grid: channels sliced over the wavefronts
+        constexpr int step = 2 * Gran<T>::E;
+        int slices = (p.cin + step - 1) / step;
+        if (slices > kMaxSlices) slices = kMaxSlices;
+        p.tiles_m = (p.cout + 31) / 32;
+        p.tiles_n = (int)((p.n + 63) / 64);
+        hipLaunchKernelGGL((sliced_kernel<T, WT, MODE>), dim3(8u * (unsigned)((p.tiles_m + 7) / 8) * (unsigned)(p.tiles_n * p.batch)),
+                           dim3(64 * slices), 0, (hipStream_t)stream, p);
+        return;
+    }
+    const int rows = 32 * waves;   // 32, 64 or 128 output rows per workgroup
+    p.tiles_m = (p.cout + rows - 1) / rows;
+    p.tiles_n = (int)((p.n + 127) / 128);
+    const dim3 grid(8u * (unsigned)((p.tiles_n * p.batch + 7) / 8) * (unsigned)p.tiles_m);
+    if (waves == 4) hipLaunchKernelGGL((tile_kernel<T, WT, 4, MODE>), grid, dim3(256), 0, (hipStream_t)stream, p);
+    else if (waves == 2) hipLaunchKernelGGL((tile_kernel<T, WT, 2, MODE>), grid, dim3(128), 0, (hipStream_t)stream, p);
+    else hipLaunchKernelGGL((tile_kernel<T, WT, 1, MODE>), grid, dim3(64), 0, (hipStream_t)stream, p);
+}
+template <typename T>
+static int tile_gemm_t(const TileParams &p, int transposed, int mode, int waves, void *stream)
+{
+    // (an activation follows a projection, whose weight lies as W; its derivative an input
+    // gradient, whose weight lies as the transpose of what is applied)
+    if (mode == epilogue::kNone && !transposed) tile_gemm_w<T, false, epilogue::kNone>(p, waves, stream);
+    else if (mode == epilogue::kNone) tile_gemm_w<T, true, epilogue::kNone>(p, waves, stream);
+    else if (mode == epilogue::kRelu && !transposed) tile_gemm_w<T, false, epilogue::kRelu>(p, waves, stream);
+    else if (mode == epilogue::kGelu && !transposed) tile_gemm_w<T, false, epilogue::kGelu>(p, waves, stream);
+    else if (mode == kGeluGrad && transposed) tile_gemm_w<T, true, kGeluGrad>(p, waves, stream);
+    else return -2;
+    return 0;
+}
+int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res,
+                     const void *mask, void *y, void *zkeep, long long batch, int cin, int cout, long long n,
+                     int mode, int esz, int waves, void *stream)
+{
+    TileParams p;
+    p.x = x, p.w = w, p.bias = bias, p.res = res, p.mask = mask, p.y = y, p.zkeep = zkeep, p.n = n, p.cin = cin;
+    p.cout = cout, p.batch = (int)batch;
+    return esz == 2 ? tile_gemm_t<bf16_t>(p, transposed, mode, waves, stream)
+                    : tile_gemm_t<float>(p, transposed, mode, waves, stream);
+}
+
+}  // namespace gemm
+}  // namespace ndc

@@ -7,6 +7,7 @@
 
 #include "ndc_common.h"
 #include "ndc_exec.h"
+#include "ndc_gemm_host.h"
 
 #define NDC_LAMBDA
 
@@ -355,6 +356,68 @@ struct Backend {
 
     // put(o, sum_p term(o, p)) in the association of the HIP build (kSumSlices interleaved
     // partial sums, then those in order)
+    template <typename T>
+    static void wgrad_t(const T *a, const T *b, float *gw, float *gb, float *part, long long batch, int rows, int cols,
+                        long long n, const WgradPlan &w)
+    {
+        const long long out = (long long)rows * cols;
+        for (long long s = 0; s < batch * w.per_sample; ++s) {
+            const long long at = s / w.per_sample, lo = s % w.per_sample * w.chunk, hi = std::min(n, lo + w.chunk);
+            float *ow = part ? part + s * (out + rows) : gw, *ob = part ? ow + out : gb;
+            for (int r = 0; r < rows; ++r) {
+                float sum = 0.f;
+                for (long long v = lo; v < hi; ++v) sum += Elem<T>::load(a + (at * rows + r) * n + v);
+                if (gb) ob[r] = sum;
+                for (int c = 0; c < cols; ++c) {
+                    float acc = 0.f;
+                    for (long long v = lo; v < hi; ++v)
+                        acc += Elem<T>::load(a + (at * rows + r) * n + v) * Elem<T>::load(b + (at * cols + c) * n + v);
+                    ow[(long long)r * cols + c] = acc;
+                }
+            }
+        }
+    }
+    static int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long long batch, int rows, int cols,
+                     long long n, int esz, const WgradPlan &w, void *)
+    {
+        if (esz == 2) wgrad_t<bf16_t>((const bf16_t *)a, (const bf16_t *)b, gw, gb, part, batch, rows, cols, n, w);
+        else wgrad_t<float>((const float *)a, (const float *)b, gw, gb, part, batch, rows, cols, n, w);
+        return 0;
+    }
+
+    template <typename T>
+    static void tile_gemm_t(const T *x, const float *w, int transposed, const float *bias, const T *res, const T *mask, T *y,
+                            T *zkeep, long long batch, int cin, int cout, long long n, int mode)
+    {
+        for (long long b = 0; b < batch; ++b)
+            for (int co = 0; co < cout; ++co)
+                for (long long v = 0; v < n; ++v) {
+                    float acc = 0.f;
+                    for (int k = 0; k < cin; ++k) {
+                        float wv = w[transposed ? (long long)k * cout + co : (long long)co * cin + k];
+                        if (sizeof(T) == 2) wv = bf16_to_float(float_to_bf16(wv));
+                        acc += wv * Elem<T>::load(x + (b * cin + k) * n + v);
+                    }
+                    const long long at = (b * cout + co) * n + v;
+                    const float bv = bias ? bias[co] : 0.f, rv = res ? Elem<T>::load(res + at) : 0.f;
+                    float out = mode == 4 ? acc * act_value(2, rv + bv, true) : act_value(mode, acc + bv, false) + rv;
+                    if (mask && !(Elem<T>::load(mask + at) > 0.f)) out = 0.f;
+                    if (zkeep) Elem<T>::store(zkeep + at, acc);
+                    Elem<T>::store(y + at, out);
+                }
+    }
+    static int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res, const void *mask,
+                         void *y, void *zkeep, long long batch, int cin, int cout, long long n, int mode, int esz, int, void *)
+    {
+        if (esz == 2)
+            tile_gemm_t<bf16_t>((const bf16_t *)x, w, transposed, bias, (const bf16_t *)res, (const bf16_t *)mask, (bf16_t *)y,
+                                (bf16_t *)zkeep, batch, cin, cout, n, mode);
+        else
+            tile_gemm_t<float>((const float *)x, w, transposed, bias, (const float *)res, (const float *)mask, (float *)y,
+                               (float *)zkeep, batch, cin, cout, n, mode);
+        return 0;
+    }
+
     template <class P, class F> static int strided_sum(int nout, int nparts, void *, P put, F term)
     {
         for (int o = 0; o < nout; ++o) {

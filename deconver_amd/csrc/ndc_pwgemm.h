@@ -244,11 +244,12 @@ __global__ void __launch_bounds__(THREADS) gemm_kernel(Params p)
                         constexpr int A = ACT == kGeluGrad ? epilogue::kGelu : epilogue::kRelu;
                         y0 = z0 * epilogue::act_grad<A>(lo_bf16(rw[j]) + bq[jj]);
                         y1 = z1 * epilogue::act_grad<A>(hi_bf16(rw[j]) + bq[jj]);
-                        // the channel's sum over the tile's 64 voxels: the 32 lanes of this half
-                        float t = y0 + y1;
+                        if (p.gpart) {   // the channel's sum over the tile's 64 voxels: the 32 lanes of this half
+                            float t = y0 + y1;
 #pragma unroll
-                        for (int m = 1; m < 32; m <<= 1) t += __shfl_xor(t, m);
-                        if (p.gpart && n32 == 0) gs[32 * c + 8 * q + 4 * kb + jj] += t;
+                            for (int m = 1; m < 32; m <<= 1) t += __shfl_xor(t, m);
+                            if (n32 == 0) gs[32 * c + 8 * q + 4 * kb + jj] += t;
+                        }
                     } else if constexpr (ACT == kMasked) {
                         y0 = z0 + bq[jj], y1 = z1 + bq[jj];
                         if constexpr (RES) y0 += lo_bf16(rw[j]), y1 += hi_bf16(rw[j]);

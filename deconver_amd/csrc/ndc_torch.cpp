@@ -160,10 +160,29 @@ struct Matrix {
     }
 };
 
-bool streaming_gemm(const Tensor &x, int64_t cout, bool act_or_keep)
+// Which GEMM makes a 1x1 projection (or an input gradient), by what was measured on an MI355X:
+//   kStream   the streaming GEMM (ndc_pointwise_gemm): bf16 in its channel counts, from 2048 of its
+//             64-voxel tiles on (below, filling its weight table costs more than the product: 128 ->
+//             512 channels over 4096 voxels 45 us against 8 us tiled);
+//   kTiled    the tiled GEMM (ndc_gemm): small products -- a library GEMM costs the host 15-19 us a
+//             call, as much as the product --, and larger ones whose tail (bias, activation,
+//             residual, mask) it takes along: float32 always, bf16 with at most 32 K weights (256
+//             -> 1024 channels over 2 x 32^3 voxels: 85 us against 59 us by the library, which then
+//             pays for one more pass over the result);
+//   kLibrary  the rest.
+enum Gemm { kStream, kTiled, kLibrary };
+
+Gemm choose_gemm(const Tensor &x, int64_t cout, bool act_or_keep, bool tail)
 {
-    if (x.scalar_type() != at::kBFloat16 || (x.size(1) > 256 && act_or_keep)) return false;
-    return ndc_pointwise_gemm_supported(x.size(1), cout, x.size(2), NDC_BF16) != 0;
+    const int64_t B = x.size(0), cin = x.size(1), n = x.size(2);
+    const bool half = x.scalar_type() == at::kBFloat16;
+    const bool stream = half && !(cin > 256 && act_or_keep) && ndc_pointwise_gemm_supported(cin, cout, n, NDC_BF16);
+    if (stream && B * n >= 2048 * 64) return kStream;
+    if (n > (1 << 24)) return stream ? kStream : kLibrary;
+    const double flops = 2.0 * (double)B * (double)n * (double)cin * (double)cout;
+    if (flops < (half ? 4e9 : 2e9)) return kTiled;
+    if (tail && (!half || cin * cout <= 32 * 1024)) return kTiled;
+    return stream ? kStream : kLibrary;
 }
 
 // W (or W^T) in the order the streaming GEMM reads it
@@ -180,19 +199,31 @@ Tensor pack(const Matrix &w, bool transpose, const Tensor &like, void *stream)
 
 Tensor batched(const Tensor &w, int64_t B) { return w.unsqueeze(0).expand({B, w.size(0), w.size(1)}); }
 
+// y = epilogue(W x) or epilogue(W^T x) by the tiled GEMM
+void tiled(const Matrix &w, bool transpose, const Tensor &x, const Tensor &bias, const Tensor &res, const Tensor &mask,
+           const Tensor &y, const Tensor &z, int mode, void *stream)
+{
+    const Tensor m = w.m.scalar_type() == at::kFloat ? w.m : w.m.to(at::kFloat);
+    check(ndc_gemm(ptr(x), fptr(m), transpose != w.transposed, fptr(bias), ptr(res), ptr(mask), out_ptr(y), out_ptr(z), x.size(0),
+                   x.size(1), y.size(1), x.size(2), mode, dtype_tag(x), stream), "ndc_gemm");
+}
+
 // W x per sample
-Tensor project(const Matrix &w, const Tensor &x, void *stream)
+Tensor project(const Matrix &w, const Tensor &x, bool library, void *stream)
 {
     const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
     Tensor z = empty({B, cout, n}, x);
-    if (streaming_gemm(x, cout, false)) {
+    const Gemm by = library ? kLibrary : choose_gemm(x, cout, false, false);
+    if (by == kStream) {
         Tensor frag = pack(w, false, x, stream);
         check(ndc_pointwise_gemm(ptr(x), ptr(frag), nullptr, nullptr, out_ptr(z), nullptr, B, w.cin(), cout, n, NDC_ACT_NONE,
                                  NDC_BF16, stream), "ndc_pointwise_gemm");
-        return z;
+    } else if (by == kTiled) {
+        tiled(w, false, x, Tensor(), Tensor(), Tensor(), z, Tensor(), NDC_ACT_NONE, stream);
+    } else {
+        // one batched GEMM, the weight shared by the samples through a zero stride
+        at::bmm_out(z, batched(w.dense(x.scalar_type(), false), B), x);
     }
-    // one batched GEMM, the weight shared by the samples through a zero stride
-    at::bmm_out(z, batched(w.dense(x.scalar_type(), false), B), x);
     return z;
 }
 
@@ -200,32 +231,37 @@ Tensor project(const Matrix &w, const Tensor &x, void *stream)
 Tensor project_back(const Matrix &w, const Tensor &gz, Tensor accumulate, const Tensor &mask, void *stream)
 {
     const int64_t B = gz.size(0), n = gz.size(2), cin = w.cin(), cout = w.cout();
-    Tensor gx;
     if (cout == 1) {
         // an outer product, i.e. a broadcast multiplication at the memory rate (as a GEMM it ran
         // at a fifth of it)
-        gx = at::mul(gz, w.m.reshape({1, -1, 1}).to(gz.scalar_type()));
+        Tensor gx = at::mul(gz, w.m.reshape({1, -1, 1}).to(gz.scalar_type()));
         if (accumulate.defined()) gx = accumulate.add_(gx);
-    } else if (streaming_gemm(gz, cin, false)) {
-        Tensor frag = pack(w, true, gz, stream);
-        gx = empty({B, cin, n}, gz);
-        if (mask.defined())
-            check(ndc_pointwise_gemm_masked(ptr(gz), ptr(frag), nullptr, ptr(accumulate), ptr(mask), out_ptr(gx), B, cout, cin,
-                                            n, NDC_BF16, stream), "ndc_pointwise_gemm_masked");
-        else
-            check(ndc_pointwise_gemm(ptr(gz), ptr(frag), nullptr, ptr(accumulate), out_ptr(gx), nullptr, B, cout, cin, n,
-                                     NDC_ACT_NONE, NDC_BF16, stream), "ndc_pointwise_gemm");
-        return gx;
-    } else {
-        Tensor wt = batched(w.dense(gz.scalar_type(), true), B);
+        return mask.defined() ? gx.mul_(mask.gt(0)) : gx;
+    }
+    const Gemm by = choose_gemm(gz, cin, false, accumulate.defined() || mask.defined());
+    if (by == kLibrary) {
+        Tensor wt = batched(w.dense(gz.scalar_type(), true), B), gx;
         if (accumulate.defined()) {
             gx = accumulate.baddbmm_(wt, gz);
         } else {
             gx = empty({B, cin, n}, gz);
             at::bmm_out(gx, wt, gz);
         }
+        return mask.defined() ? gx.mul_(mask.gt(0)) : gx;
     }
-    return mask.defined() ? gx.mul_(mask.gt(0)) : gx;
+    Tensor gx = empty({B, cin, n}, gz);
+    if (by == kTiled) {
+        tiled(w, true, gz, Tensor(), accumulate, mask, gx, Tensor(), NDC_ACT_NONE, stream);
+        return gx;
+    }
+    Tensor frag = pack(w, true, gz, stream);
+    if (mask.defined())
+        check(ndc_pointwise_gemm_masked(ptr(gz), ptr(frag), nullptr, ptr(accumulate), ptr(mask), out_ptr(gx), B, cout, cin, n,
+                                        NDC_BF16, stream), "ndc_pointwise_gemm_masked");
+    else
+        check(ndc_pointwise_gemm(ptr(gz), ptr(frag), nullptr, ptr(accumulate), out_ptr(gx), nullptr, B, cout, cin, n, NDC_ACT_NONE,
+                                 NDC_BF16, stream), "ndc_pointwise_gemm");
+    return gx;
 }
 
 // Equal chunks the voxel axis is cut into for the weight-gradient GEMM: a power of two that
@@ -247,32 +283,6 @@ int64_t weight_grad_plan(int64_t batch, int64_t n, bool half)
     return n < (1 << 17) ? 1 : weight_grad_chunks(batch, n, 2048);
 }
 
-// sum_b gz[b] x[b]^T: the weight gradient, (cout, cin) -- or (cin, cout) for a weight stored
-// transposed --, added up in float32.  Long rows are cut into equal chunks of the voxel axis that
-// become batch entries (strided views, no copies); bfloat16 operands hand out their float32
-// accumulators.
-Tensor weight_grad(const Tensor &gz, const Tensor &x, const Matrix &w, at::IntArrayRef shape, at::ScalarType dtype)
-{
-    const Tensor &a = w.transposed ? x : gz, &c = w.transposed ? gz : x;
-    const int64_t B = a.size(0), n = a.size(2), rows = a.size(1), cols = c.size(1);
-    const bool half = a.scalar_type() == at::kBFloat16;
-    const int64_t s = weight_grad_plan(B, n, half);
-    Tensor parts;
-    if (s == 1) {
-        parts = half ? at::bmm(a, c.transpose(1, 2), at::kFloat) : at::bmm(a, c.transpose(1, 2));
-    } else {
-        parts = empty_f32({B * s, rows, cols}, a);
-        for (int64_t b = 0; b < B; ++b) {
-            Tensor ab = a.select(0, b).view({rows, s, n / s}).transpose(0, 1);
-            Tensor cb = c.select(0, b).view({cols, s, n / s}).permute({1, 2, 0});
-            Tensor to = parts.narrow(0, b * s, s);
-            if (half) at::bmm_out(to, ab, cb, at::kFloat);
-            else at::bmm_out(to, ab, cb);
-        }
-    }
-    return parts.sum(at::IntArrayRef{0}, false, at::kFloat).to(dtype).view(shape);
-}
-
 // sum over batch and voxels, float32, one value per channel
 Tensor channel_sums(const Tensor &g, void *stream)
 {
@@ -281,6 +291,39 @@ Tensor channel_sums(const Tensor &g, void *stream)
     Tensor partial = empty_f32({B, C, parts}, g);
     check(ndc_row_sums(ptr(g), out_fptr(partial), B * C, n, dtype_tag(g), stream), "ndc_row_sums");
     return partial.sum(at::IntArrayRef{0, 2});
+}
+
+// Weight gradient sum_b gz[b] x[b]^T, (cout, cin) -- or (cin, cout) for a weight stored
+// transposed --, and the bias gradient, the sums of gz, from the same pass.  Rows beyond the
+// kernel's reach (2^24 voxels) are cut into chunks that become batch entries of a library GEMM.
+Tensor weight_grad(const Tensor &gz, const Tensor &x, const Matrix &w, at::IntArrayRef shape, at::ScalarType dtype, Tensor *gb,
+                   void *stream)
+{
+    const Tensor &a = w.transposed ? x : gz, &c = w.transposed ? gz : x;
+    const int64_t B = a.size(0), n = a.size(2), rows = a.size(1), cols = c.size(1);
+    if (n <= (1 << 24)) {
+        const bool sums = gb && !w.transposed;
+        Tensor gw = empty_f32({rows, cols}, a);
+        if (sums) *gb = empty_f32({rows}, a);
+        const int64_t bytes = (int64_t)ndc_weight_grad_workspace_bytes(B, rows, cols, n, dtype_tag(a));
+        Tensor ws = bytes ? at::empty({bytes}, a.options().dtype(at::kByte)) : Tensor();
+        check(ndc_weight_grad(ptr(a), ptr(c), out_fptr(gw), sums ? out_fptr(*gb) : nullptr, B, rows, cols, n, dtype_tag(a),
+                              out_ptr(ws), bytes, stream), "ndc_weight_grad");
+        if (gb && !sums) *gb = channel_sums(gz, stream);
+        return gw.to(dtype).view(shape);
+    }
+    if (gb) *gb = channel_sums(gz, stream);
+    const bool half = a.scalar_type() == at::kBFloat16;
+    const int64_t s = weight_grad_plan(B, n, half);
+    Tensor parts = empty_f32({B * s, rows, cols}, a);
+    for (int64_t b = 0; b < B; ++b) {
+        Tensor ab = a.select(0, b).view({rows, s, n / s}).transpose(0, 1);
+        Tensor cb = c.select(0, b).view({cols, s, n / s}).permute({1, 2, 0});
+        Tensor to = parts.narrow(0, b * s, s);
+        if (half) at::bmm_out(to, ab, cb, at::kFloat);
+        else at::bmm_out(to, ab, cb);
+    }
+    return parts.sum(at::IntArrayRef{0}, false, at::kFloat).to(dtype).view(shape);
 }
 
 // ---------------------------------------------------------------------------- the update
@@ -513,7 +556,8 @@ struct Projected : public torch::autograd::Function<Projected> {
     {
         const Matrix w(weight, false);
         auto size = x.sizes().vec();
-        Tensor z = project(w, x.flatten(2), stream);
+        // (float32: the library's product, whose bits decide which source units are on)
+        Tensor z = project(w, x.flatten(2), x.scalar_type() == at::kFloat, stream);
         size[1] = w.cout();
         return update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
     }
@@ -547,7 +591,7 @@ struct Projected : public torch::autograd::Function<Projected> {
         const Tensor x = f.x.flatten(2);
         const Matrix w(v[8], false);
         Tensor gw, gx;
-        if (need[1]) gw = weight_grad(r.gz.flatten(2), x, w, v[8].sizes(), v[8].scalar_type());
+        if (need[1]) gw = weight_grad(r.gz.flatten(2), x, w, v[8].sizes(), v[8].scalar_type(), nullptr, scope.stream);
         if (need[0]) {
             gx = project_back(w, r.gz.flatten(2), r.gx.flatten(2), flags[0] ? x : Tensor(), scope.stream).view(f.x.sizes());
             if (f.x_last) gx = to_channels_last(gx, scope.stream);
@@ -578,22 +622,28 @@ struct Linear : public torch::autograd::Function<Linear> {
                       void *stream)
     {
         const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
-        Tensor y;
-        if (streaming_gemm(x, cout, act != NDC_ACT_NONE || keep)) {
+        const bool tail = bias.defined() || act != NDC_ACT_NONE || res.defined();
+        // (an activation's tile form reads W as rows; a bare float32 product is the library's, as in
+        // Projected: the two give the same bits)
+        const bool library = (w.transposed && act != NDC_ACT_NONE) || (!tail && x.scalar_type() == at::kFloat);
+        const Gemm by = library ? kLibrary : choose_gemm(x, cout, act != NDC_ACT_NONE || keep, tail);
+        Tensor y = empty({B, cout, n}, x);
+        if (keep) z = empty({B, cout, n}, x);
+        if (by == kStream) {
             // product, bias, activation and residual in one kernel that reads x once and writes
             // the result (and z where it is kept) once
             Tensor frag = pack(w, false, x, stream);
-            y = empty({B, cout, n}, x);
-            if (keep) z = empty({B, cout, n}, x);
             check(ndc_pointwise_gemm(ptr(x), ptr(frag), fptr(bias), ptr(res), out_ptr(y), out_ptr(z), B, w.cin(), cout, n,
                                      (int)act, NDC_BF16, stream), "ndc_pointwise_gemm");
-            return y;
+        } else if (by == kTiled) {
+            tiled(w, false, x, bias, res, Tensor(), y, z, (int)act, stream);
+        } else {
+            Tensor &product = keep ? z : y;
+            at::bmm_out(product, batched(w.dense(x.scalar_type(), false), B), x);
+            if (tail)
+                check(ndc_bias_act(ptr(product), fptr(bias), ptr(res), out_ptr(y), B, cout, n, (int)act, dtype_tag(x), stream),
+                      "ndc_bias_act");
         }
-        y = project(w, x, stream);
-        if (!bias.defined() && act == NDC_ACT_NONE && !res.defined()) return y;
-        if (keep) z = y, y = empty({B, cout, n}, x);
-        check(ndc_bias_act(ptr(keep ? z : y), fptr(bias), ptr(res), out_ptr(y), B, cout, n, (int)act, dtype_tag(x), stream),
-              "ndc_bias_act");
         return y;
     }
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight, const OptTensor &bias, int64_t act,
@@ -628,19 +678,14 @@ struct Linear : public torch::autograd::Function<Linear> {
         const auto need = n.ask(ctx);
         const Tensor gy = gouts[0].contiguous();
         Tensor gz = gy, gx, gw, gb;
-        if (act == NDC_ACT_NONE || cfg[3]) {
-            if (need[2]) gb = channel_sums(gy, scope.stream);
-        } else {
-            const int64_t B = gy.size(0), C = gy.size(1), nv = gy.size(2);
+        if (act != NDC_ACT_NONE && !cfg[3]) {
             gz = at::empty_like(gy);
-            Tensor part;
-            if (need[2]) part = empty_f32({B, C, ndc_bias_act_parts(B * C, nv)}, gy);
-            check(ndc_bias_act_backward(ptr(gy), ptr(kept), fptr(bias), out_ptr(gz), out_fptr(part), B, C, nv, act, dtype_tag(gy),
-                                        scope.stream), "ndc_bias_act_backward");
-            if (need[2]) gb = part.sum(at::IntArrayRef{0, 2});
+            check(ndc_bias_act_backward(ptr(gy), ptr(kept), fptr(bias), out_ptr(gz), nullptr, gy.size(0), gy.size(1), gy.size(2), act,
+                                        dtype_tag(gy), scope.stream), "ndc_bias_act_backward");
         }
         if (need[0]) gx = project_back(w, gz, Tensor(), Tensor(), scope.stream);
-        if (need[1]) gw = weight_grad(gz, x, w, v[1].sizes(), v[1].scalar_type());
+        if (need[1]) gw = weight_grad(gz, x, w, v[1].sizes(), v[1].scalar_type(), need[2] ? &gb : nullptr, scope.stream);
+        else if (need[2]) gb = channel_sums(gz, scope.stream);
         if (gb.defined()) gb = gb.to((at::ScalarType)cfg[5]);
         return once({gx, gw, gb, Tensor(), need[3] ? gy : Tensor(), Tensor(), Tensor()}, recording, gouts);
     }
@@ -662,25 +707,17 @@ Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, int6
     return Linear::run(xc, Matrix(weight, transposed), f32_vector(bias), act, res ? *res : Tensor(), false, z, scope.stream);
 }
 
-// W2 gelu(W1 x + b1) + b2 + residual on contiguous bfloat16 (B, C, n) tensors, on the streaming
-// GEMM (layers/mlp.py:40-63 with the block's sum, deconver.py:60-64): two launches forward (the
-// GELU and the kept pre-activation leave the first, bias and residual ride on the second), and a
-// backward in which the input gradient of the second projection comes out already multiplied by
-// the GELU's derivative, with the first bias's gradient summed in the same kernel.
+// W2 gelu(W1 x + b1) + b2 + residual on contiguous (B, C, n) tensors (layers/mlp.py:40-63 with the
+// block's sum, deconver.py:60-64): the GELU and the kept pre-activation leave the first product,
+// bias and residual ride on the second, and in backward the input gradient of the second comes
+// out already multiplied by the GELU's derivative where one of the library's own GEMMs makes it.
 struct Mlp : public torch::autograd::Function<Mlp> {
     static Tensor run(const Tensor &x, const Matrix &w1, const Tensor &b1, const Matrix &w2, const Tensor &b2, const Tensor &res,
                       bool keep, Tensor &z, Tensor &a, void *stream)
     {
-        const int64_t B = x.size(0), n = x.size(2), hidden = w1.cout(), cout = w2.cout();
-        Tensor f1 = pack(w1, false, x, stream), f2 = pack(w2, false, x, stream);
-        a = empty({B, hidden, n}, x);
-        if (keep) z = empty({B, hidden, n}, x);
-        check(ndc_pointwise_gemm(ptr(x), ptr(f1), fptr(b1), nullptr, out_ptr(a), out_ptr(z), B, w1.cin(), hidden, n, NDC_ACT_GELU,
-                                 NDC_BF16, stream), "ndc_pointwise_gemm");
-        Tensor y = empty({B, cout, n}, x);
-        check(ndc_pointwise_gemm(ptr(a), ptr(f2), fptr(b2), ptr(res), out_ptr(y), nullptr, B, hidden, cout, n, NDC_ACT_NONE,
-                                 NDC_BF16, stream), "ndc_pointwise_gemm");
-        return y;
+        Tensor unused;
+        a = Linear::run(x, w1, b1, NDC_ACT_GELU, Tensor(), keep, z, stream);
+        return Linear::run(a, w2, b2, NDC_ACT_NONE, res, false, unused, stream);
     }
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor &w2,
                           const OptTensor &b2, const OptTensor &residual)
@@ -710,28 +747,31 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         const Tensor gy = gouts[0].contiguous();
         const int64_t B = x.size(0), nv = x.size(2), hidden = w1.cout();
         Tensor gx, gw1, gb1, gw2, gb2;
-        if (need[4]) gb2 = channel_sums(gy, scope.stream).to((at::ScalarType)cfg[4]);
-        if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type());
+        if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type(), need[4] ? &gb2 : nullptr, scope.stream);
+        else if (need[4]) gb2 = channel_sums(gy, scope.stream);
         if (need[0] || need[1] || need[2]) {
-            Tensor frag = pack(w2, true, gy, scope.stream), gz = at::empty_like(z), part;
-            if (need[2]) part = empty_f32({ndc_pointwise_gemm_parts(), hidden}, gy);
-            check(ndc_pointwise_gemm_actgrad(ptr(gy), ptr(frag), fptr(b1), ptr(z), out_ptr(gz), out_fptr(part), B, w2.cout(), hidden,
-                                             nv, NDC_ACT_GELU, NDC_BF16, scope.stream), "ndc_pointwise_gemm_actgrad");
-            if (need[2]) gb1 = part.sum(0).to((at::ScalarType)cfg[3]);
-            if (need[1]) gw1 = weight_grad(gz, x, w1, v[3].sizes(), v[3].scalar_type());
+            Tensor gz = at::empty_like(z);
+            const Gemm by = choose_gemm(gy, hidden, true, true);
+            if (by == kStream) {
+                Tensor frag = pack(w2, true, gy, scope.stream);
+                check(ndc_pointwise_gemm_actgrad(ptr(gy), ptr(frag), fptr(b1), ptr(z), out_ptr(gz), nullptr, B, w2.cout(), hidden, nv,
+                                                 NDC_ACT_GELU, NDC_BF16, scope.stream), "ndc_pointwise_gemm_actgrad");
+            } else if (by == kTiled) {
+                tiled(w2, true, gy, b1, z, Tensor(), gz, Tensor(), NDC_GEMM_GELU_GRAD, scope.stream);
+            } else {
+                Tensor ga = project_back(w2, gy, Tensor(), Tensor(), scope.stream);
+                check(ndc_bias_act_backward(ptr(ga), ptr(z), fptr(b1), out_ptr(gz), nullptr, B, hidden, nv, NDC_ACT_GELU, dtype_tag(gy),
+                                            scope.stream), "ndc_bias_act_backward");
+            }
+            if (need[1]) gw1 = weight_grad(gz, x, w1, v[3].sizes(), v[3].scalar_type(), need[2] ? &gb1 : nullptr, scope.stream);
+            else if (need[2]) gb1 = channel_sums(gz, scope.stream);
             if (need[0]) gx = project_back(w1, gz, Tensor(), Tensor(), scope.stream);
         }
+        if (gb1.defined()) gb1 = gb1.to((at::ScalarType)cfg[3]);
+        if (gb2.defined()) gb2 = gb2.to((at::ScalarType)cfg[4]);
         return once({gx, gw1, gb1, gw2, gb2, need[5] ? gy : Tensor()}, recording, gouts);
     }
 };
-
-// whether mlp() takes these shapes: bfloat16, all four products on the streaming GEMM
-bool mlp_applies(const Tensor &x, int64_t hidden, int64_t cout)
-{
-    const int64_t c = x.size(1), n = voxels(x);
-    auto ok = [n](int64_t ci, int64_t co) { return ndc_pointwise_gemm_supported(ci, co, n, NDC_BF16) != 0; };
-    return x.is_cuda() && ok(c, hidden) && ok(hidden, cout) && ok(cout, hidden) && ok(hidden, c);
-}
 
 Tensor mlp(const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor &w2, const OptTensor &b2,
            const OptTensor &residual)
@@ -977,7 +1017,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("prepare_taps", &taps_for);
     m.def("linear", &linear);
     m.def("mlp", &mlp);
-    m.def("mlp_applies", &mlp_applies);
     m.def("row_norm", &row_norm);
     m.def("row_norm_skip", &row_norm_skip);
     m.def("channel_norm", &channel_norm);

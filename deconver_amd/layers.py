@@ -290,16 +290,15 @@ class Linear(nn.Module):
 
 
 class _FusedMLP:
-    """``W2 gelu(W1 x + b1) + b2 + residual`` as ONE autograd node on the library's streaming GEMM
-    (layers/mlp.py:40-63 with the block's sum, deconver.py:60-64), compiled in
-    ``csrc/ndc_torch.cpp``: the hidden tensor's gradient is written once and never read back by an
-    activation pass."""
+    """``W2 gelu(W1 x + b1) + b2 + residual`` as ONE autograd node (layers/mlp.py:40-63 with the
+    block's sum, deconver.py:60-64), compiled in ``csrc/ndc_torch.cpp``: the hidden tensor's gradient
+    is written once and, where the library's own GEMMs make it, never read back by an activation
+    pass."""
 
     @staticmethod
     def applies(lib, x: torch.Tensor, hidden: int, cout: int) -> bool:
-        """Whether it takes ``x`` (B, C, *): bfloat16 on the GPU, all four products of forward and
-        backward in the streaming GEMM's shapes."""
-        return x.dtype == torch.bfloat16 and _lib.get_native().mlp_applies(x, hidden, cout)
+        """Whether it takes ``x`` (B, C, n): bfloat16 or float32 on the GPU."""
+        return x.is_cuda and x.dim() == 3 and x.dtype in (torch.bfloat16, torch.float32)
 
     @staticmethod
     def apply(x, w1, b1, w2, b2, residual):
@@ -338,13 +337,11 @@ class MLP(nn.Module):
 
     @staticmethod
     def _fused(first: "Linear", second: "Linear", x: torch.Tensor, residual: Optional[torch.Tensor]):
-        """The block as one node on the streaming GEMM where all four of its products fit it
-        (bfloat16, stored or under autocast; e.g. 64 -> 256 -> 64 channels), else None."""
+        """The block as one node for bfloat16 (stored or under autocast) and float32 tensors on the
+        GPU, else None."""
         if not _gemm_route(x):
             return None
         dtype = torch.get_autocast_dtype(x.device.type) if torch.is_autocast_enabled(x.device.type) else x.dtype
-        if dtype != torch.bfloat16:
-            return None
         w1, w2 = first.linear.weight, second.linear.weight
         flat = x.flatten(2)
         if flat.dtype != dtype:

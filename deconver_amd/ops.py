@@ -360,6 +360,46 @@ def pointwise_gemm_actgrad(lib: _lib.NdcLibrary, gy: Tensor, wfrag: Tensor, cout
     return gz, (gpart.sum(0) if need_bias_grad else None)
 
 
+def gemm(lib: _lib.NdcLibrary, x: Tensor, w: Tensor, bias: Optional[Tensor] = None, residual: Optional[Tensor] = None,
+         act: Optional[str] = None, keep_z: bool = False, mask: Optional[Tensor] = None, transposed: bool = False):
+    """``act(W x + bias) + residual`` (zero where ``mask <= 0``) for contiguous ``x`` (B, cin, n) and
+    float32 ``w`` (cout, cin), or its (cin, cout) storage with ``transposed``; ``act="gelu_grad"``:
+    ``(W x) * gelu'(residual + bias)``.  Returns ``(y, z)``, ``z`` the product with ``keep_z``."""
+    if x.dim() != 3 or not x.is_contiguous() or w.dim() != 2 or not w.is_contiguous() or w.dtype != torch.float32:
+        raise ValueError("gemm wants a contiguous (B, cin, n) tensor and a contiguous float32 matrix")
+    B, cin, n = x.shape
+    cout = w.shape[1 if transposed else 0]
+    if w.shape[0 if transposed else 1] != cin:
+        raise ValueError("the matrix does not belong to this tensor")
+    for t in (residual, mask):
+        if t is not None and (t.shape != (B, cout, n) or t.dtype != x.dtype or not t.is_contiguous()):
+            raise ValueError("residual and mask must be contiguous, of the output's shape and dtype")
+    if bias is not None and (bias.dtype != torch.float32 or bias.numel() != cout or not bias.is_contiguous()):
+        raise ValueError("bias must be float32 with one entry per output channel")
+    y = x.new_empty(B, cout, n)
+    z = x.new_empty(B, cout, n) if keep_z else None
+    mode = 4 if act == "gelu_grad" else ACTS[act]
+    lib.gemm(_ptr(x), _ptr(w), transposed, _ptr(bias), _ptr(residual), _ptr(mask), _ptr(y), _ptr(z), B, cin, cout, n, mode,
+             dtype_tag(x.dtype), _stream_of(x))
+    return y, z
+
+
+def weight_grad(lib: _lib.NdcLibrary, gz: Tensor, x: Tensor, need_bias_grad: bool = False):
+    """``(sum_b gz[b] x[b]^T, row sums of gz or None)``, float32, for contiguous (B, rows, n) and
+    (B, cols, n) tensors of one dtype."""
+    if gz.dim() != 3 or gz.dtype != x.dtype or gz.shape[::2] != x.shape[::2] or not (gz.is_contiguous() and x.is_contiguous()):
+        raise ValueError("weight_grad wants contiguous (B, C, n) tensors of one dtype, batch and voxel count")
+    B, rows, n = gz.shape
+    cols = x.shape[1]
+    gw = torch.empty(rows, cols, dtype=torch.float32, device=x.device)
+    gb = torch.empty(rows, dtype=torch.float32, device=x.device) if need_bias_grad else None
+    nbytes = lib.weight_grad_workspace_bytes(B, rows, cols, n, dtype_tag(x.dtype))
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
+    lib.weight_grad(_ptr(gz), _ptr(x), _ptr(gw), _ptr(gb), B, rows, cols, n, dtype_tag(x.dtype), _ptr(ws), nbytes,
+                    _stream_of(x))
+    return gw, gb
+
+
 def regroup2_applies(fine_shape, dtype, *ptrs) -> bool:
     """Whether ``ndc_regroup`` takes a fine-grid tensor ``(B, C, [D,] H, W)``: float32 or
     bfloat16, even extents, rows of whole 16-byte vectors, 16-byte aligned buffers."""

@@ -320,7 +320,7 @@ int ndc_bias_act_backward(const void *gy, const void *z, const float *bias, void
  * deconver/deconver.py:41-46, 60-64 and deconver/layers/mlp.py:40-63 apply to its output).
  * A streaming kernel on the matrix units: x is read once, y written once, float32 accumulation,
  * one rounding of the result.
- *   ndc_pointwise_gemm_supported  1 where the kernel applies: NDC_BF16; cin 64, 128 or 256, or a
+ *   ndc_pointwise_gemm_supported  1 where the kernel applies: NDC_BF16; cin 32, 64, 128 or 256, or a
  *                  larger multiple of 64 with cout <= 128; cout a multiple of 32;
  *                  cin * cout * 2 <= 128 KiB; n a multiple of 64; else 0 (callers then use a
  *                  library GEMM and ndc_bias_act)
@@ -408,6 +408,35 @@ int ndc_chnorm_backward(const void *gy, const void *x, const float *stats, const
  */
 int ndc_regroup(const void *src, void *dst, const float *bias, int64_t rows, int64_t channels, int64_t D,
                  int64_t H, int64_t W, int depth2, int dtype, int to_channels, void *stream);
+
+/*
+ * The 1x1 projections and their input gradients as a tiled GEMM, for the tensors
+ * ndc_pointwise_gemm does not take (float32, any channel and voxel count, any alignment to the
+ * element): on channel-first (batch, c, n) tensors
+ *     NDC_ACT_NONE:          y = (W x + bias + residual), zero where mask <= 0 if a mask is given
+ *     NDC_ACT_RELU / GELU:   y = act(W x + bias) + residual; zkeep (or null) receives W x
+ *     NDC_GEMM_GELU_GRAD:    y = (W x) * gelu'(residual + bias)
+ * Replaces nn.Conv1d(kernel_size=1) and what follows it (deconver/layers/linear.py:53-58,
+ * deconver/layers/mlp.py:40-63, deconver/deconver.py:60-64), as ndc_pointwise_gemm does.
+ *   w           float32, (cout, cin), or with `transposed` its (cin, cout) storage; read as it
+ *               lies (activations need transposed = 0, the gradient mode transposed = 1)
+ *   bias, residual, mask   optional; residual and mask of y's shape and dtype
+ */
+#define NDC_GEMM_GELU_GRAD 4
+int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, const void *residual,
+             const void *mask, void *y, void *zkeep, int64_t batch, int64_t cin, int64_t cout, int64_t n,
+             int mode, int dtype, void *stream);
+
+/*
+ * Weight gradient of a 1x1 projection and the sums its bias gradient is, in one pass:
+ *     gw = sum_b gz[b] x[b]^T  (rows, cols) float32,   gb = sum_{b,v} gz[b][.][v]  (rows) or null
+ * for gz (batch, rows, n) and x (batch, cols, n), float32 or bfloat16.  The voxel axis is split over
+ * workgroups; their float32 partial results (workspace, 16-byte aligned, may be null when the
+ * size is 0) are added in a fixed order.
+ */
+size_t ndc_weight_grad_workspace_bytes(int64_t batch, int64_t rows, int64_t cols, int64_t n, int dtype);
+int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t batch, int64_t rows,
+                    int64_t cols, int64_t n, int dtype, void *workspace, size_t workspace_bytes, void *stream);
 
 #ifdef __cplusplus
 }

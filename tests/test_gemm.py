@@ -1,0 +1,88 @@
+"""The tiled GEMMs of the projections (ndc_gemm: forward and input gradient with their tails;
+ndc_weight_grad: weight and bias gradient in one pass) against float64 products of the same
+operands, at the sizes where tiles, stages and splits have ends."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from deconver_amd import _lib, ops
+from tests.helpers import hostcheck_library
+
+# (B, cin, cout, n): one element; a voxel past a tile; ragged depth and rows; tiny grids over many
+# channels (channels sliced over the wavefronts); an odd row length; a tile of one voxel pair
+SHAPES = [(1, 1, 1, 1), (2, 64, 32, 129), (3, 130, 70, 77), (1, 54, 64, 1000), (2, 1048, 96, 105), (1, 64, 33, 4099),
+          (2, 8, 40, 2), (1, 512, 160, 64)]
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
+DTYPES = [(torch.float32, 2e-6), (torch.bfloat16, 4e-3)]
+
+
+def _setup(device, shape, dtype):
+    lib = hostcheck_library() if device == "cpu" else _lib.get_library()
+    B, cin, cout, n = shape
+    gen = torch.Generator().manual_seed(cin + cout)
+    rn = lambda *s: torch.randn(*s, generator=gen)   # noqa: E731
+    x, res, mask, g = rn(B, cin, n), rn(B, cout, n), rn(B, cout, n), rn(B, cout, n)
+    w, bias = rn(cout, cin) / cin ** 0.5, rn(cout)
+    return lib, [t.to(device=device, dtype=dtype) for t in (x, res, mask, g)], w.to(device), bias.to(device)
+
+
+def _rel(a, ref):
+    ref = ref.double()
+    return float((a.double() - ref).norm() / ref.norm().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize("dtype,tol", DTYPES)
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("device", DEVICES)
+def test_products_with_their_tails(device, shape, dtype, tol):
+    lib, (x, res, mask, _), w, bias = _setup(device, shape, dtype)
+    wt = w.t().contiguous()
+    z = torch.matmul(w.to(dtype).double(), x.double())
+    u = z + bias.double()[:, None]
+    y, _ = ops.gemm(lib, x, w)
+    assert _rel(y, z) < tol
+    y, zk = ops.gemm(lib, x, w, bias, res, "gelu", keep_z=True)
+    assert _rel(y, F.gelu(u) + res.double()) < tol and _rel(zk, z) < tol
+    y, _ = ops.gemm(lib, x, w, bias, None, "relu")
+    assert _rel(y, u.clamp_min(0)) < tol
+    y, _ = ops.gemm(lib, x, wt, bias, res, mask=mask, transposed=True)
+    assert _rel(y, torch.where(mask.double() > 0, u + res.double(), 0.0)) < tol
+    v = (res.double() + bias.double()[:, None]).requires_grad_(True)
+    F.gelu(v).sum().backward()
+    y, _ = ops.gemm(lib, x, wt, bias, res, "gelu_grad", transposed=True)
+    assert _rel(y, z * v.grad) < tol
+
+
+@pytest.mark.parametrize("dtype,tol", DTYPES)
+@pytest.mark.parametrize("shape", SHAPES + [(1, 32, 256, 3000), (2, 300, 48, 2100), (2, 96, 128, 1537)])
+@pytest.mark.parametrize("device", DEVICES)
+def test_weight_and_bias_gradient(device, shape, dtype, tol):
+    lib, (x, _, _, g), _, _ = _setup(device, shape, dtype)
+    gw, gb = ops.weight_grad(lib, g, x, need_bias_grad=True)
+    assert _rel(gw, torch.matmul(g.double(), x.double().transpose(1, 2)).sum(0)) < 4e-6
+    assert _rel(gb, g.double().sum((0, 2))) < 4e-6
+    again, none = ops.weight_grad(lib, g, x)
+    assert torch.equal(again, gw) and none is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(256, 64), (64, 54)])
+def test_weight_gradient_over_long_rows(rows, cols):
+    """Rows long enough for the deep stages, with a ragged end."""
+    lib, n = _lib.get_library(), (1 << 19) + 21
+    torch.manual_seed(0)
+    g, x = (torch.randn(1, c, n, device="cuda").bfloat16() for c in (rows, cols))
+    gw, gb = ops.weight_grad(lib, g, x, need_bias_grad=True)
+    assert _rel(gw, g[0].double() @ x[0].double().t()) < 1e-5 and _rel(gb, g.double().sum((0, 2))) < 1e-5
+
+
+def test_refused_arguments():
+    lib = hostcheck_library()
+    x, w = torch.zeros(1, 8, 4), torch.zeros(6, 8)
+    with pytest.raises(_lib.NdcError):      # an activation reads W as rows
+        ops.gemm(lib, x, w.t().contiguous(), act="relu", transposed=True)
+    with pytest.raises(_lib.NdcError):      # the gradient mode reads its transpose
+        ops.gemm(lib, x, w, residual=torch.zeros(1, 6, 4), act="gelu_grad")
+    with pytest.raises(_lib.NdcError):      # and needs the pre-activation
+        ops.gemm(lib, x, w.t().contiguous(), act="gelu_grad", transposed=True)
