@@ -47,8 +47,15 @@ def dice_bce_loss(logits: Tensor, target: Tensor) -> Tensor:
 
 def make_optimizer(model: nn.Module, capturable: bool = False) -> torch.optim.Optimizer:
     """AdamW as above; ``capturable`` keeps its step counters on the device, which
-    ``GraphedTrainStep`` needs."""
-    return torch.optim.AdamW(model.parameters(), lr=1e-3, weight_decay=1e-2, capturable=capturable)
+    ``GraphedTrainStep`` needs.
+
+    On the GPU the update is the fused form: one pass over parameter, gradient and moments in a
+    few launches (28 bytes a parameter), where the default form reads and writes them once per
+    operation -- with the step counters on the device in some 280 launches, most of them on one
+    counter each.  Parameters on the CPU keep the default form."""
+    params = list(model.parameters())
+    fused = bool(params) and all(p.is_cuda and p.is_floating_point() for p in params)
+    return torch.optim.AdamW(params, lr=1e-3, weight_decay=1e-2, capturable=capturable, fused=fused or None)
 
 
 def _gaussian_blur(t: Tensor, sigma: float) -> Tensor:
