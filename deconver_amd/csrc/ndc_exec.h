@@ -90,19 +90,35 @@ template <class State> struct DeviceExec {
     // every global load this thread has issued has returned (s_waitcnt vmcnt(0))
     NDC_D void wait_loads() const { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-    // Sum N per-thread values over the workgroup: butterfly inside each wavefront, one LDS
-    // row per wavefront, then thread i < N adds the rows in a fixed order and hands the sum
-    // to `put`.  Reuses LDS from offset 0 (callers are done with their tiles by then).
+    // the sum of `v` over the wavefront, in lane 63: adds whose second operand comes through the
+    // vector unit's own lane network (shifts inside rows of 16 lanes, then row to row)
+    static NDC_D float wave_sum(float v)
+    {
+#define NDC_DPP_ADD(CTRL, ROWS)                                                                               \
+    v += __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, true))
+        NDC_DPP_ADD(0x111, 0xf);   // row_shr:1
+        NDC_DPP_ADD(0x112, 0xf);   // row_shr:2
+        NDC_DPP_ADD(0x114, 0xf);   // row_shr:4
+        NDC_DPP_ADD(0x118, 0xf);   // row_shr:8
+        NDC_DPP_ADD(0x142, 0xa);   // row_bcast:15 into rows 1 and 3
+        NDC_DPP_ADD(0x143, 0xc);   // row_bcast:31 into rows 2 and 3
+#undef NDC_DPP_ADD
+        return v;
+    }
+
+    // Sum N per-thread values over the workgroup: inside each wavefront on the vector unit (six
+    // adds a value; a butterfly of __shfl_xor goes through the LDS unit of the CU six times a
+    // value, 650 times a wavefront for the 108 sums of a 3x3x3 filter), one LDS row per
+    // wavefront, then thread i < N adds the rows in a fixed order and hands the sum to `put`.
+    // Reuses LDS from offset 0 (callers are done with their tiles by then).
     template <int N, class Get, class Put> NDC_D void block_reduce(Get get, Put put)
     {
         __syncthreads();
         const int lane = tid & 63, wave = tid >> 6, nw = nthreads >> 6;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            float v = get(st, i);
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            if (lane == 0) lds[wave * N + i] = v;
+            const float v = wave_sum(get(st, i));
+            if (lane == 63) lds[wave * N + i] = v;
         }
         __syncthreads();
         for (int i = tid; i < N; i += nthreads) {
