@@ -67,6 +67,39 @@ static inline int choose_path(const ndc_geom *g, const KGeom &q)
 
 // ------------------------------------------------------------------ direct path
 
+template <typename TI, typename TO>
+static int direct_gconv(const KGeom &q, const TI *in, const float *h, const float *bias,
+                        int adjoint, TO *out, void *stream)
+{
+    const int rectify = bias != nullptr || q.relu, cout = adjoint ? q.sc : q.m;
+    return direct::with_form(q, cout, [&](auto form) {
+        typedef decltype(form) F;
+        const int blocks = (cout + F::nb - 1) / F::nb;
+        const long long units = (long long)q.B * q.G * blocks;
+        if (adjoint) {
+            const direct::GConv<TI, TO, true, F::nb, F::kwb, typename F::off> op = {q, in, h, bias, rectify, out, blocks};
+            return Backend::per_unit(units, q.SP, stream, op);
+        }
+        const direct::GConv<TI, TO, false, F::nb, F::kwb, typename F::off> op = {q, in, h, bias, rectify, out, blocks};
+        return Backend::per_unit(units, q.SP, stream, op);
+    });
+}
+
+// n = A(x) + eps, d = A(t1) + eps and what STAGE makes of them (ndc_direct.h)
+template <typename T, int STAGE>
+static int direct_ratio(const KGeom &q, const T *x, const T *t1, const T *z, const T *gout, const float *gt1,
+                        const float *h, const float *bias, T *out, T *s_over_den, T *ratio, float *gn, float *gd,
+                        void *stream)
+{
+    return direct::with_form(q, q.sc, [&](auto form) {
+        typedef decltype(form) F;
+        const int blocks = (q.sc + F::nb - 1) / F::nb;
+        const direct::Ratio<T, STAGE, F::nb, F::kwb, typename F::off> op = {
+            q, x, t1, z, gout, gt1, h, bias, out, s_over_den, ratio, gn, gd, blocks};
+        return Backend::per_unit((long long)q.B * q.G * blocks, q.SP, stream, op);
+    });
+}
+
 template <typename T>
 static int direct_forward(const KGeom &q, const T *x, const T *z, const float *h,
                           const float *bias, T *out, T *t1, T *s_over_den, T *ratio, void *stream)
@@ -74,22 +107,21 @@ static int direct_forward(const KGeom &q, const T *x, const T *z, const float *h
     // t1 = K(relu(z + b)) lands in the caller's t1; without one there is nowhere to put
     // it, so the direct path asks for it (the fused path does not need it)
     if (!t1) return NDC_ERR_NULL;
-    const long long n_x = (long long)q.B * q.C() * q.SP, n_s = (long long)q.B * q.CS() * q.SP;
-    int st = Backend::elementwise(n_x, stream, [=] NDC_LAMBDA(long long idx) {
-        direct::gconv<T, T, false>(idx, q, z, h, bias, true, t1);
-    });
+    int st = direct_gconv<T, T>(q, z, h, bias, 0, t1, stream);
     if (st) return st;
-    return Backend::elementwise(n_s, stream, [=] NDC_LAMBDA(long long idx) {
-        direct::fwd<T>(idx, q, x, t1, z, h, bias, out, s_over_den, ratio);
-    });
+    return direct_ratio<T, direct::FWD>(q, x, t1, z, nullptr, nullptr, h, bias, out, s_over_den, ratio, nullptr,
+                                        nullptr, stream);
 }
 
 static inline size_t direct_backward_ws(const KGeom &q)
 {
     const size_t n_x = (size_t)q.B * q.C() * q.SP, n_s = (size_t)q.B * q.CS() * q.SP;
-    return align_up(n_s * 4, 256) * 2 + align_up(n_x * 4, 256);
+    const size_t sums = (size_t)q.G * q.m * q.sc * q.KT + q.CS();
+    return align_up(n_s * 4, 256) * 2 + align_up(n_x * 4, 256) +
+           align_up((size_t)direct::reduce_chunks(q) * sums * 4, 256);
 }
 
+// scratch: gn | gd | gt1 (all float) | partial sums of gh and gb, [chunk][gh, gb]
 template <typename T>
 static int direct_backward(const KGeom &q, const T *x, const T *z, const T *t1, const float *h,
                            const float *bias, const T *gout, T *gx, T *gz, float *gh, float *gb,
@@ -102,63 +134,55 @@ static int direct_backward(const KGeom &q, const T *x, const T *z, const T *t1, 
     float *gd = (float *)w;
     w += align_up((size_t)n_s * 4, 256);
     float *gt1 = (float *)w;
+    w += align_up((size_t)n_x * 4, 256);
+    float *part = (float *)w;
+    const int n_gh = q.G * q.m * q.sc * q.KT, nchunk = direct::reduce_chunks(q);
+    const long long stride = (long long)n_gh + q.CS();
     KGeom qn = q;  // gn/gd/gt1 are plain tensors: no bias, no rectification on load
     qn.relu = 0;
-    int st = Backend::elementwise(n_s, stream, [=] NDC_LAMBDA(long long idx) {
-        direct::bwd_gn_gd<T>(idx, q, x, t1, z, gout, h, bias, gn, gd);
-    });
+    int st = direct_ratio<T, direct::GRAD>(q, x, t1, z, gout, nullptr, h, bias, nullptr, nullptr, nullptr, gn, gd,
+                                           stream);
     if (st) return st;
-    st = Backend::elementwise(n_x, stream, [=] NDC_LAMBDA(long long idx) {
-        direct::gconv<float, float, false>(idx, qn, gd, h, nullptr, false, gt1);
-    });
-    if (st) return st;
-    if (gx) {
-        st = Backend::elementwise(n_x, stream, [=] NDC_LAMBDA(long long idx) {
-            direct::gconv<float, T, false>(idx, qn, gn, h, nullptr, false, gx);
+    if (!gx) {
+        st = direct_gconv<float, float>(qn, gd, h, nullptr, 0, gt1, stream);
+    } else {
+        st = direct::with_form(q, q.m, [&](auto form) {
+            typedef decltype(form) F;
+            const int blocks = (q.m + F::nb - 1) / F::nb;
+            const direct::GradPair<T, F::nb, F::kwb, typename F::off> op = {q, gn, gd, h, gx, gt1, blocks};
+            return Backend::per_unit((long long)q.B * q.G * blocks, q.SP, stream, op);
         });
-        if (st) return st;
     }
+    if (st) return st;
     if (gh) {
-        st = Backend::block_reduce(q.G * q.m * q.sc * q.KT, stream, gh,
-                                   [=] NDC_LAMBDA(int o, int tid, int nt) {
-                                       return direct::gh_partial<T>(o, tid, nt, q, x, t1, z, bias,
-                                                                    gn, gd, gt1);
-                                   });
+        st = direct::with_grad_form(q, [&](auto form) {
+            typedef decltype(form) F;
+            const int ob = (q.m + F::mb - 1) / F::mb, ib = (q.sc + F::sb - 1) / F::sb, wb = q.kW / F::kwb;
+            const direct::FilterGrad<T, F::mb, F::sb, F::kwb, typename F::off> op = {
+                q, x, t1, z, bias, gn, gd, gt1, part, stride, nchunk, ob, ib, wb};
+            return Backend::unit_sums((long long)q.G * ob * ib * q.kD * q.kH * wb * nchunk, stream, op);
+        });
         if (st) return st;
     }
     if (gz || gb) {
         // gz is needed to form gb; when the caller does not want gz it goes to the gn
         // scratch (gn is dead by now), typed as T
         T *gz_out = gz ? gz : (T *)gn;
-        st = Backend::elementwise(n_s, stream, [=] NDC_LAMBDA(long long idx) {
-            direct::bwd_gz<T>(idx, q, x, t1, z, gout, gt1, h, bias, gz_out);
-        });
+        st = direct_ratio<T, direct::SOURCE>(q, x, t1, z, gout, gt1, h, bias, gz_out, nullptr, nullptr, nullptr,
+                                             nullptr, stream);
         if (st) return st;
         if (gb) {
-            st = Backend::block_reduce(q.CS(), stream, gb, [=] NDC_LAMBDA(int o, int tid, int nt) {
-                return direct::gb_partial<T>(o, tid, nt, q, gz_out);
-            });
+            const direct::BiasGrad<T> op = {q, gz_out, part + n_gh, stride, nchunk};
+            st = Backend::unit_sums((long long)q.CS() * nchunk, stream, op);
             if (st) return st;
         }
     }
-    return NDC_OK;
-}
-
-template <typename TI, typename TO>
-static int direct_gconv(const KGeom &q, const TI *in, const float *h, const float *bias,
-                        int adjoint, TO *out, void *stream)
-{
-    const bool rectify = (bias != nullptr) || q.relu;
-    if (adjoint) {
-        const long long n = (long long)q.B * q.CS() * q.SP;
-        return Backend::elementwise(n, stream, [=] NDC_LAMBDA(long long idx) {
-            direct::gconv<TI, TO, true>(idx, q, in, h, bias, rectify, out);
-        });
-    }
-    const long long n = (long long)q.B * q.C() * q.SP;
-    return Backend::elementwise(n, stream, [=] NDC_LAMBDA(long long idx) {
-        direct::gconv<TI, TO, false>(idx, q, in, h, bias, rectify, out);
-    });
+    // the chunks' sums, added in order (no atomics: results are reproducible)
+    const int lo = gh ? 0 : n_gh, n = (gh ? n_gh : 0) + (gb ? q.CS() : 0);
+    if (!n) return NDC_OK;
+    return Backend::strided_sum(n, nchunk, stream, [=] NDC_LAMBDA(int o, float v) {
+        if (lo + o < n_gh) gh[o] = v; else gb[lo + o - n_gh] = v;
+    }, [=] NDC_LAMBDA(int o, int p) { return part[p * stride + lo + o]; });
 }
 
 }  // namespace ndc

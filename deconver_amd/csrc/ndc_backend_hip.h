@@ -26,18 +26,32 @@ __global__ void __launch_bounds__(256) elementwise_kernel(long long n, F f)
         f(idx);
 }
 
+// f(unit, position): the unit is the same for a whole workgroup, lanes run along the positions
 template <class F>
-__global__ void __launch_bounds__(256) block_reduce_kernel(float *out, F partial)
+__global__ void __launch_bounds__(128) per_unit_kernel(unsigned blocks, long long npos, F f)
 {
-    __shared__ float buf[256];
-    const int tid = threadIdx.x;
-    buf[tid] = partial((int)blockIdx.x, tid, 256);
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) buf[tid] += buf[tid + s];
-        __syncthreads();
+    const unsigned u = blockIdx.x / blocks;
+    const long long pos = (long long)(blockIdx.x - u * blocks) * 128 + threadIdx.x;
+    if (pos < npos) f((int)u, pos);
+}
+
+// F::N sums over the threads of a workgroup, one workgroup per unit: f.sums gives a thread's
+// own, f.put takes the totals
+template <class F> __global__ void __launch_bounds__(256) unit_sums_kernel(F f)
+{
+    struct None {};
+    __shared__ float lds[4 * F::N];
+    const int u = (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    float acc[F::N];
+    f.sums(u, tid, 256, acc);
+#pragma unroll
+    for (int i = 0; i < F::N; ++i) {
+        const float v = DeviceExec<None>::wave_sum(acc[i]);
+        if (lane == 63) lds[wave * F::N + i] = v;
     }
-    if (tid == 0) out[blockIdx.x] = buf[0];
+    __syncthreads();
+    for (int i = tid; i < F::N; i += 256)
+        f.put(u, i, ((lds[i] + lds[F::N + i]) + lds[2 * F::N + i]) + lds[3 * F::N + i]);
 }
 
 // put(o, sum over p < nparts of term(o, p)) for o < nout.  A workgroup sums 32 outputs:
@@ -615,11 +629,21 @@ struct Backend {
         return check();
     }
 
-    template <class F> static int block_reduce(int nout, void *stream, float *out, F partial)
+    template <class F> static int per_unit(long long units, long long npos, void *stream, F f)
     {
-        if (nout <= 0) return 0;
-        hipLaunchKernelGGL(block_reduce_kernel<F>, dim3((unsigned)nout), dim3(256), 0,
-                           (hipStream_t)stream, out, partial);
+        const long long blocks = (npos + 127) / 128;
+        if (units <= 0 || npos <= 0) return 0;
+        if (blocks > 0x7fffffffLL / units) return -2;
+        hipLaunchKernelGGL(per_unit_kernel<F>, dim3((unsigned)(units * blocks)), dim3(128), 0, (hipStream_t)stream,
+                           (unsigned)blocks, npos, f);
+        return check();
+    }
+
+    template <class F> static int unit_sums(long long units, void *stream, F f)
+    {
+        if (units <= 0) return 0;
+        if (units > 0x7fffffffLL) return -2;
+        hipLaunchKernelGGL(unit_sums_kernel<F>, dim3((unsigned)units), dim3(256), 0, (hipStream_t)stream, f);
         return check();
     }
 };

@@ -432,14 +432,22 @@ struct Backend {
         return 0;
     }
 
-    template <class F> static int block_reduce(int nout, void *, float *out, F partial)
+    template <class F> static int per_unit(long long units, long long npos, void *, F f)
     {
-        float buf[256];
-        for (int o = 0; o < nout; ++o) {
-            for (int tid = 0; tid < 256; ++tid) buf[tid] = partial(o, tid, 256);
-            for (int s = 128; s > 0; s >>= 1)
-                for (int tid = 0; tid < s; ++tid) buf[tid] += buf[tid + s];
-            out[o] = buf[0];
+        for (long long u = 0; u < units; ++u)
+            for (long long p = 0; p < npos; ++p) f((int)u, p);
+        return 0;
+    }
+
+    template <class F> static int unit_sums(long long units, void *, F f)
+    {
+        for (long long u = 0; u < units; ++u) {
+            float total[F::N] = {0.f}, acc[F::N];
+            for (int tid = 0; tid < 256; ++tid) {
+                f.sums((int)u, tid, 256, acc);
+                for (int i = 0; i < F::N; ++i) total[i] += acc[i];
+            }
+            for (int i = 0; i < F::N; ++i) f.put((int)u, i, total[i]);
         }
         return 0;
     }
