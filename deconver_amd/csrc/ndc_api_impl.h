@@ -768,7 +768,7 @@ int ndc_chnorm_forward(const void *x, const float *weight, const float *bias, vo
     const int esz = dtype == NDC_BF16 ? 2 : 4;
     const bool vec = chnorm_wide(batch, n, esz) && aligned16(x) && aligned16(y);
     st = ndc::Backend::chnorm(false, nullptr, x, stats, weight, bias, y, nullptr, batch, (int)channels, n, esz, vec,
-                              eps, stream);
+                              ndc_chnorm_parts(batch, n, dtype), eps, stream);
     return st == -2 ? (int)NDC_ERR_GEOMETRY : st;
 }
 
@@ -785,7 +785,7 @@ int ndc_chnorm_backward(const void *gy, const void *x, const float *stats, const
     // the partial rows are laid out for the path ndc_chnorm_parts counted
     if (partial && fits && !vec) return NDC_ERR_WORKSPACE;
     st = ndc::Backend::chnorm(true, gy, x, stats, weight, nullptr, gx, partial, batch, (int)channels, n, esz, vec,
-                              0.f, stream);
+                              ndc_chnorm_parts(batch, n, dtype), 0.f, stream);
     return st == -2 ? (int)NDC_ERR_GEOMETRY : st;
 }
 

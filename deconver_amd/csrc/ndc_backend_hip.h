@@ -347,12 +347,52 @@ struct Backend {
             hipLaunchKernelGGL((chnorm::forward_kernel<T, VEC>), grid, block, 0, (hipStream_t)stream, (const T *)x,
                                weight, bias, (T *)out, const_cast<float *>(stats), sh, eps);
     }
+    // up to 256 channels: see held_forward_kernel.  Workgroups walk the voxels, 2048 of them in all
+    // (two rounds of the chip at four a CU), never more than `partial` has rows.
+    template <typename T, int LV, int CPT>
+    static void chnorm_held_launch(bool bwd, const void *a, const void *x, const float *stats, const float *weight,
+                                   const float *bias, void *out, float *partial, long long B, int C, long long n,
+                                   long long parts, float eps, void *stream)
+    {
+        const long long tiles = (n / LV + 63) / 64, most = parts / B, want = (2048 + B - 1) / B;
+        long long groups = tiles < want ? tiles : want;
+        if (groups > most) groups = most;
+        const chnorm::HeldShape sh = {n, C, (int)groups, tiles, parts};
+        const dim3 grid((unsigned)(B * groups)), block(chnorm::kHeldThreads);
+        if (bwd)
+            hipLaunchKernelGGL((chnorm::held_backward_kernel<T, LV, CPT>), grid, block, 0, (hipStream_t)stream,
+                               (const T *)a, (const T *)x, stats, weight, (T *)out, partial, sh);
+        else
+            hipLaunchKernelGGL((chnorm::held_forward_kernel<T, LV, CPT>), grid, block, 0, (hipStream_t)stream,
+                               (const T *)x, weight, bias, (T *)out, const_cast<float *>(stats), sh, eps);
+    }
+    template <typename T, int LV>
+    static void chnorm_held(bool bwd, const void *a, const void *x, const float *stats, const float *weight,
+                            const float *bias, void *out, float *partial, long long B, int C, long long n,
+                            long long parts, float eps, void *stream)
+    {
+        const int cpt = (C + chnorm::kSlices - 1) / chnorm::kSlices;
+        if (cpt <= 4) chnorm_held_launch<T, LV, 4>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+        else if (cpt <= 8) chnorm_held_launch<T, LV, 8>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+        else if (cpt <= 16) chnorm_held_launch<T, LV, 16>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+        else chnorm_held_launch<T, LV, 32>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+    }
+
+    // parts: rows of `partial` (ndc_chnorm_parts)
     static int chnorm(bool bwd, const void *a, const void *x, const float *stats, const float *weight,
                       const float *bias, void *out, float *partial, long long B, int C, long long n, int esz,
-                      bool vec, float eps, void *stream)
+                      bool vec, long long parts, float eps, void *stream)
     {
         if (B <= 0 || C <= 0 || n <= 0) return 0;
         if (B * chnorm_blocks(n, esz, vec) > 0x7fffffffLL) return -2;
+        if (C <= chnorm::kHeldChannels) {
+            const bool pairs = n % 2 == 0 && (((uintptr_t)a | (uintptr_t)x | (uintptr_t)out) & (uintptr_t)(2 * esz - 1)) == 0;
+            if (esz == 2 && pairs) chnorm_held<bf16_t, 2>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+            else if (esz == 2) chnorm_held<bf16_t, 1>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+            else if (pairs) chnorm_held<float, 2>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+            else chnorm_held<float, 1>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, parts, eps, stream);
+            return check();
+        }
         if (esz == 2) {
             if (vec) chnorm_launch<bf16_t, true>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, eps, stream);
             else chnorm_launch<bf16_t, false>(bwd, a, x, stats, weight, bias, out, partial, B, C, n, eps, stream);

@@ -215,7 +215,7 @@ struct Backend {
     }
     static int chnorm(bool bwd, const void *a, const void *x, const float *stats, const float *weight,
                       const float *bias, void *out, float *partial, long long B, int C, long long n, int esz,
-                      bool vec, float eps, void *)
+                      bool vec, long long, float eps, void *)
     {
         if (esz == 2)
             chnorm_t<bf16_t>(bwd, (const bf16_t *)a, (const bf16_t *)x, const_cast<float *>(stats), weight, bias,

@@ -369,14 +369,35 @@ class LayerNorm(nn.Module):
         super().__init__()
         self.norm = nn.LayerNorm(dim, **kwargs)
 
+    def _hip(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The normalised ``x`` from the HIP kernels, in its own type, or None if they do not take it."""
+        if not (x.is_cuda and x.dim() >= 3 and len(self.norm.normalized_shape) == 1 and x.numel() > 0
+                and x.shape[1] == self.norm.normalized_shape[0] and x.dtype in (torch.float32, torch.bfloat16)):
+            return None
+        y = _lib.get_native().channel_norm(x.flatten(2), self.norm.weight, self.norm.bias, float(self.norm.eps))
+        return y.view(x.shape)
+
+    def _widened(self, x: torch.Tensor) -> torch.Tensor:
+        return x.float() if x.is_cuda and torch.is_autocast_enabled(x.device.type) else x
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        # (small grids stay with the reference form: below 32 768 voxels in all the kernels'
-        # one-thread-per-voxel launch does not fill the chip, and PyTorch's takes 0.06 ms)
-        if (x.is_cuda and x.dim() >= 3 and len(self.norm.normalized_shape) == 1
-                and x.shape[1] == self.norm.normalized_shape[0]
-                and x.shape[0] * x[0, 0].numel() >= _CHNORM_MIN_VOXELS):
-            t = x.float() if torch.is_autocast_enabled(x.device.type) else x
-            if t.dtype in (torch.float32, torch.bfloat16):
-                y = _lib.get_native().channel_norm(t.flatten(2), self.norm.weight, self.norm.bias, float(self.norm.eps))
-                return y.view(x.shape)
-        return self.norm(x.movedim(1, -1)).movedim(-1, 1)
+        # (below 32 768 voxels in all a caller gets the reference's form, a view of a channels-last result)
+        y = None
+        if x.is_cuda and x.dim() >= 3 and x.shape[0] * x[0, 0].numel() >= _CHNORM_MIN_VOXELS:
+            y = self._hip(self._widened(x))
+        return self.norm(x.movedim(1, -1)).movedim(-1, 1) if y is None else y
+
+    def for_projection(self, x: torch.Tensor, consumer: nn.Module) -> torch.Tensor:
+        """``forward(x)`` for a caller that hands it to the projection ``consumer``, which wants it
+        channel-first and, under bfloat16 autocast, rounded to bfloat16: the kernels at every size,
+        and bfloat16 values under bfloat16 autocast normalised (in float32 arithmetic) and rounded
+        in one pass -- the bits that widening, normalising and rounding in three passes over twice
+        the bytes give, in both directions.  Hooks see what ``forward`` makes."""
+        y = None
+        if type(self) is LayerNorm and _gemm_route(x) and not (
+                self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
+                or self._backward_pre_hooks or consumer._forward_pre_hooks):
+            narrow = (x.dtype == torch.bfloat16 and torch.is_autocast_enabled(x.device.type)
+                      and torch.get_autocast_dtype(x.device.type) == torch.bfloat16)
+            y = self._hip(x if narrow else self._widened(x))
+        return self(x) if y is None else y

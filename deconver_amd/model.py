@@ -90,10 +90,20 @@ class DeconverBlock(nn.Module):
 
     def forward(self, x: Tensor) -> Tensor:
         # (norm(x), x): on the HIP norm the residual's gradient is summed in the norm's backward
-        y, x = self.norm1.with_skip(x) if hasattr(self.norm1, "with_skip") else (self.norm1(x), x)
+        y, x = self._normed(self.norm1, x, self.dcm, self.dcm.in_proj)
         x = self.dcm(y, residual=x)
-        y, x = self.norm2.with_skip(x) if hasattr(self.norm2, "with_skip") else (self.norm2(x), x)
+        y, x = self._normed(self.norm2, x, self.mlp, self.mlp.block[0])
         return self.mlp(y, residual=x)
+
+    @staticmethod
+    def _normed(norm: nn.Module, x: Tensor, consumer: nn.Module, projection: nn.Module):
+        if hasattr(norm, "with_skip"):
+            return norm.with_skip(x)
+        # (the channel norm's result is rounded as the projection that reads it would round it)
+        if (type(norm) is LayerNorm and type(consumer) in (DeconvMixer, layers.MLP)
+                and type(projection) is Linear and not consumer._forward_pre_hooks):
+            return norm.for_projection(x, projection), x
+        return norm(x), x
 
 
 class DeconverStage(nn.Module):
