@@ -722,14 +722,16 @@ int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, c
     if (all & (uintptr_t)((dtype == NDC_BF16 ? 2 : 4) - 1) || ((uintptr_t)w & 3u) || ((uintptr_t)bias & 3u)) return NDC_ERR_WORKSPACE;
     if (y == x || zkeep == x || (zkeep && zkeep == y)) return NDC_ERR_GEOMETRY;
     // Small grids -- at most four workgroups of 32 rows x 64 voxels per CU -- take the form that
-    // slices the channels over the wavefronts (waves = 0): 128 -> 512 channels over 4096 voxels in
-    // bf16 8.1 us against 10.2 tiled, over 32 768 (4096 workgroups) 24 against 11.5.  Otherwise as
+    // slices the channels over the wavefronts (waves <= 0): 128 -> 512 channels over 4096 voxels in
+    // bf16 8.1 us against 10.2 tiled, over 32 768 (4096 workgroups) 24 against 11.5 --, at most one
+    // per CU in tiles of 16 rows x 32 voxels (waves = -1; 288 of the larger tiles, 256 -> 64 channels
+    // over 9152 voxels in float32, 10 us against 11.5 in the smaller).  Otherwise as
     // many output rows per workgroup (32 per wavefront) as still leave two workgroups per CU.
     const int esz = dtype == NDC_BF16 ? 2 : 4;
     const long long vt = batch * ((n + 127) / 128), small = batch * ((n + 63) / 64) * ((cout + 31) / 32);
     int waves = 4;
     while (waves > 1 && (cout <= 32 * (waves / 2) || vt * ((cout + 32 * waves - 1) / (32 * waves)) < 512)) waves /= 2;
-    if (small <= 1024 && cin % (16 / esz) == 0 && n >= 2) waves = 0;
+    if (small <= 1024 && cin % (16 / esz) == 0 && n >= 2) waves = small <= 256 ? -1 : 0;
     if ((vt + 8) * 2 * ((cout + 31) / 32 + 8) > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
     return ndc::Backend::tile_gemm(x, w, transposed != 0, bias, residual, mask, y, zkeep, batch, (int)cin, (int)cout, n,
                                    mode, esz, waves, stream);

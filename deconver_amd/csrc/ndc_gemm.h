@@ -57,6 +57,13 @@ template <> struct Gran<float> {
     {
         return (__uint_as_float(g[0]) + __uint_as_float(g[1])) + (__uint_as_float(g[2]) + __uint_as_float(g[3]));
     }
+    static __device__ f32x4 mma(u32x4 a, u32x4 b, f32x4 acc)
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), __uint_as_float(b[j]), acc, 0, 0, 0);
+        return acc;
+    }
     static __device__ f32x16 mma(u32x4 a, u32x4 b, f32x16 acc)
     {
 #pragma unroll
@@ -78,6 +85,10 @@ template <> struct Gran<bf16_t> {
 #pragma unroll
         for (int i = 0; i < 4; ++i) s += __uint_as_float(g[i] << 16) + __uint_as_float(g[i] & 0xffff0000u);
         return s;
+    }
+    static __device__ f32x4 mma(u32x4 a, u32x4 b, f32x4 acc)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
     }
     static __device__ f32x16 mma(u32x4 a, u32x4 b, f32x16 acc)
     {
@@ -524,41 +535,50 @@ __global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
 // A grid of a few thousand voxels leaves the tiled kernel a handful of workgroups that walk the
 // channels one stage after the other, each stage waiting for memory (2048 -> 512 channels over
 // 64 voxels: 32 stages, 195 us).  Here the channels are split over the wavefronts of a workgroup
-// instead: a tile is 32 output rows x 64 voxels, wavefront w takes its share of the channels
-// straight from memory into the operand registers (kAhead steps requested together, no staging,
+// instead: a tile is R output rows x 2 R voxels, wavefront w takes its share of the channels
+// straight from memory into the operand registers (AHEAD steps requested together, no staging,
 // no barrier), and the wavefronts' partial tiles are added through LDS, in order.  Lanes hold
 // voxel pairs: pair c is column c of an even-voxel and an odd-voxel matrix tile.
+// R = 16 where 32 x 64 tiles would leave CUs without one: what bounds such a launch is the matrix
+// work and the round trips to memory of the few workgroups there are (2048 -> 512 channels over 143
+// voxels in float32: 48 tiles of 14 us of matrix instructions each), so four times the tiles, each
+// with a quarter of the products and half as many round trips.  (The 2-D network's projections over
+// 143 and 572 voxels: 13-23 -> 9-13 us.)
 static const int kMaxSlices = 8;
 
-template <typename T, bool WT, int MODE>
+template <typename T, bool WT, int MODE, int R>
 __global__ void __launch_bounds__(64 * kMaxSlices) sliced_kernel(TileParams p)
 {
     typedef Gran<T> G;
-    constexpr int E = G::E, kAhead = 4;              // steps whose operands are in flight
-    __shared__ __attribute__((aligned(16))) float part[kMaxSlices][32][64];
-    // the voxel tiles of a row tile run on one XCD: they read the same rows of W
-    const int vts = p.tiles_n * p.batch;
-    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
-    const int tile_m = (pos / vts) * 8 + xcd, vt = pos % vts;
-    if (tile_m >= p.tiles_m) return;
-    const int sample = vt / p.tiles_n, m0 = tile_m * 32;
-    const int v0 = (vt % p.tiles_n) * 64, left = min((int)p.n - v0, 64);
-    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, kb = lane >> 5, slices = blockDim.x >> 6;
+    typedef typename std::conditional<R == 16, f32x4, f32x16>::type Acc;
+    constexpr int E = G::E, KB = 64 / R;             // granules of a step
+    constexpr int kAhead = R == 16 && E == 4 ? 8 : 4;   // steps whose operands are in flight
+    __shared__ __attribute__((aligned(16))) float part[kMaxSlices][R][2 * R];
+    // an eighth of the tiles per XCD, consecutive ones, so that the voxel tiles of a row tile, which
+    // read the same rows of W, share an L2 (whole row tiles dealt to the XCDs leave all but a few of
+    // them idle where there are fewer than eight: 128 -> 32 channels over 36 608 voxels 45 us, 10 here)
+    const int vts = p.tiles_n * p.batch, tiles = p.tiles_m * vts, share = (tiles + 7) / 8;
+    const int index = (int)(blockIdx.x & 7) * share + (int)(blockIdx.x >> 3);
+    if (index >= tiles || (int)(blockIdx.x >> 3) >= share) return;
+    const int tile_m = index / vts, vt = index % vts;
+    const int sample = vt / p.tiles_n, m0 = tile_m * R;
+    const int v0 = (vt % p.tiles_n) * 2 * R, left = min((int)p.n - v0, 2 * R);
+    const int tid = threadIdx.x, lane = tid & 63, col = lane % R, kb = lane / R, slices = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T *X = (const T *)p.x + (long long)sample * p.cin * p.n + v0;
-    const int m = min(m0 + l32, p.cout - 1);
+    const int m = min(m0 + col, p.cout - 1);
     // pairs past the end repeat the last one; the half pair at the end of an odd count is the
     // second element of the pair before it
-    const bool half = 2 * l32 + 1 == left;
-    const int c = min(2 * l32, left - 2);   // (-1 in a tile of one voxel: n >= 2)
-    const int steps = (p.cin + 2 * E - 1) / (2 * E), per = (steps + slices - 1) / slices;
+    const bool half = 2 * col + 1 == left;
+    const int c = min(2 * col, left - 2);   // (-1 in a tile of one voxel: n >= 2)
+    const int steps = (p.cin + KB * E - 1) / (KB * E), per = (steps + slices - 1) / slices;
     const int s_lo = wave * per, s_hi = min(s_lo + per, steps);
     typedef typename std::conditional<sizeof(T) == 2, uint32_t, u32x2>::type Pair;   // two voxels
     typedef Pair Pair_a2 __attribute__((aligned(2), may_alias));
     float w[kAhead][E];
     Pair xv[kAhead][E];
     auto request = [&](int a, int s) {
-        const int k = min((2 * s + kb) * E, p.cin - E);   // (the caller has checked cin % E == 0, n >= 2)
+        const int k = min((KB * s + kb) * E, p.cin - E);   // (the caller has checked cin % E == 0, n >= 2)
         if constexpr (WT) {
 #pragma unroll
             for (int e = 0; e < E; ++e) w[a][e] = p.w[(long long)(k + e) * p.cout + m];
@@ -574,11 +594,11 @@ __global__ void __launch_bounds__(64 * kMaxSlices) sliced_kernel(TileParams p)
 #pragma unroll
         for (int e = 0; e < E; ++e) xv[a][e] = *(const Pair_a2 *)(X + (long long)(k + e) * p.n + c);
     };
-    f32x16 acc0 = {}, acc1 = {};
+    Acc acc0 = {}, acc1 = {};
     const uint32_t second = half ? ~0u : 0u;
     auto multiply = [&](int a, int s) {
         // (masks instead of selects: a condition here becomes a branch around the loads' first use)
-        const uint32_t keep = (2 * s + kb) * E < p.cin ? ~0u : 0u;
+        const uint32_t keep = (KB * s + kb) * E < p.cin ? ~0u : 0u;
         u32x4 gw = G::pack(w[a]), g0, g1;
         if constexpr (sizeof(T) == 2) {
 #pragma unroll
@@ -610,11 +630,11 @@ __global__ void __launch_bounds__(64 * kMaxSlices) sliced_kernel(TileParams p)
         }
     }
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-        *reinterpret_cast<float2 *>(&part[wave][8 * (j / 4) + 4 * kb + j % 4][2 * l32]) = make_float2(acc0[j], acc1[j]);
+    for (int j = 0; j < R * R / 64; ++j)   // (a lane has runs of four rows, 4 KB rows apart)
+        *reinterpret_cast<float2 *>(&part[wave][4 * KB * (j / 4) + 4 * kb + j % 4][2 * col]) = make_float2(acc0[j], acc1[j]);
     __syncthreads();
-    for (int t = tid; t < 32 * 16; t += blockDim.x) {
-        const int row = t >> 4, q = t & 15, have = left - 4 * q;
+    for (int t = tid; t < R * R / 2; t += blockDim.x) {
+        const int row = t / (R / 2), q = t % (R / 2), have = left - 4 * q;
         if (m0 + row >= p.cout || have <= 0) continue;
         float z[1][4] = {{0.f, 0.f, 0.f, 0.f}};
         for (int w = 0; w < slices; ++w) {

@@ -39,14 +39,15 @@ int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long 
 
 template <typename T, bool WT, int MODE> static void tile_gemm_w(TileParams p, int waves, void *stream)
 {
-    if (waves == 0) {   // small grid: channels sliced over the wavefronts
-        constexpr int step = 2 * Gran<T>::E;
+    if (waves <= 0) {   // small grid: channels sliced over the wavefronts, tiles of 32 or 16 rows
+        const int rows = waves ? 16 : 32, step = 64 / rows * Gran<T>::E;
         int slices = (p.cin + step - 1) / step;
         if (slices > kMaxSlices) slices = kMaxSlices;
-        p.tiles_m = (p.cout + 31) / 32;
-        p.tiles_n = (int)((p.n + 63) / 64);
-        hipLaunchKernelGGL((sliced_kernel<T, WT, MODE>), dim3(8u * (unsigned)((p.tiles_m + 7) / 8) * (unsigned)(p.tiles_n * p.batch)),
-                           dim3(64 * slices), 0, (hipStream_t)stream, p);
+        p.tiles_m = (p.cout + rows - 1) / rows;
+        p.tiles_n = (int)((p.n + 2 * rows - 1) / (2 * rows));
+        const dim3 grid(8u * (unsigned)((p.tiles_m * p.tiles_n * p.batch + 7) / 8));
+        if (waves) hipLaunchKernelGGL((sliced_kernel<T, WT, MODE, 16>), grid, dim3(64 * slices), 0, (hipStream_t)stream, p);
+        else hipLaunchKernelGGL((sliced_kernel<T, WT, MODE, 32>), grid, dim3(64 * slices), 0, (hipStream_t)stream, p);
         return;
     }
     const int rows = 32 * waves;   // 32, 64 or 128 output rows per workgroup
