@@ -11,7 +11,7 @@ namespace gemm {
 template <typename T, int WM, int WN, int RT, int CT, int D>
 static void wgrad_launch(WgradParams p, void *stream)
 {
-    const unsigned blocks = 8u * (unsigned)((p.splits + 7) / 8) * (unsigned)(p.tiles_m * p.tiles_n);
+    const unsigned blocks = 8u * (((unsigned)p.splits * (unsigned)(p.tiles_m * p.tiles_n) + 7u) / 8u);
     hipLaunchKernelGGL((wgrad_kernel<T, WM, WN, RT, CT, D>), dim3(blocks), dim3(64 * WM * WN), 0,
                        (hipStream_t)stream, p);
 }
