@@ -119,6 +119,11 @@ static inline std::atomic<int> &matrix_default()
 #endif
 static const long long kSplitWavesF = NDC_SPLIT_F, kSplitWavesB = NDC_SPLIT_B;
 
+#ifndef NDC_HELD_WAVES
+#define NDC_HELD_WAVES 2048
+#endif
+static const long long kHeldWaves = NDC_HELD_WAVES;   // two wavefronts on each of the 1024 SIMDs
+
 struct Plan {
     Variant v;
     March m;
@@ -348,7 +353,12 @@ int forward(const KGeom &q, const T *x, const T *z, const float *h, const float 
         }
         return Dot2Launch<BE, T>::fwd(p, pl, stream);
     }
+    // (two wavefronts per SIMD and no more: see FwdKernel)
+    const bool held = (long long)pl.nblk_f * (pl.tf.NT / 64) <= kHeldWaves;
 #define X(kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_)                                          \
+    if (NDC_IS_VARIANT(pl, kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_) && kh_ == 1 && rwf_ == 1 && held) \
+        return BE::template block_kernel<FwdKernel<kd_, kh_, kw_, sc_, rhf_, rwf_, T, kh_ == 1 && rwf_ == 1>>( \
+            p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);                                         \
     if (NDC_IS_VARIANT(pl, kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_))                        \
         return BE::template block_kernel<FwdKernel<kd_, kh_, kw_, sc_, rhf_, rwf_, T>>(        \
             p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);
