@@ -382,7 +382,8 @@ NDC_HD Lane make_lane(int tid, const Tile &t, int RW)
 // waits for latencies: a rolled tap loop takes nine trips through a scalar load and an LDS read per
 // row step, each one after the other, five times as long as its arithmetic.  With more wavefronts
 // the other form's smaller register count is worth as much (4096 wavefronts: the two are level).
-// 32 channels of 64^2 28.7 -> 23.8 us, 64 channels of 104 x 88 42 -> 31, 512 of 13 x 11 41 -> 34.
+// 32 channels of 64^2 28.7 -> 23.8 us, 64 channels of 104 x 88 42 -> 31, 512 of 13 x 11 41 -> 34 (21,
+// 26 and 32 with the loads of a plane left in flight, see load_plane).
 template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool HELD_ = false> struct FwdKernel {
     static constexpr bool HELD = HELD_;
     static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_;
@@ -444,50 +445,26 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
         const int d0 = id.d0, d1 = id.d1;
         const int k_first = d0 - 2 * PD > 0 ? d0 - 2 * PD : 0, k_end = d1 + 2 * PD;
 
-        // global -> registers: plane k of s (bias / ReLU applied) and plane k - PD of x.
-        // Rows outside the image read a clamped address and are zeroed by a select.
+        // global -> registers: plane k of z and plane k - PD of x as they lie in memory (planes past
+        // an end: the last one; rows outside the image: a clamped address).  Bias, rectifier and the
+        // zero of a plane outside the volume are applied when they are staged: an instruction on a
+        // value here would wait for it ahead of the gather that is to hide its latency (8 x 32 channels
+        // of 256^2 in float32 338 -> 315 us, 512 of 13 x 11 34 -> 32, 128 of 52 x 44 30 -> 25).
         auto load_plane = [&](State &st, int k) NDC_LAMBDA {
             if (!st.ln.active) return;
-            if (k < D) {
-                const T *zk = zg + (long long)k * plane;
-                NDC_UNROLL
-                for (int n = 0; n < NZR; ++n) {
-                    NDC_UNROLL
-                    for (int i = 0; i < SC; ++i) {
-                        float v[RW];
-                        IO::load(zk + i * cplane + st.zoff[n], v);
-                        NDC_UNROLL
-                        for (int c = 0; c < RW; ++c) {
-                            float s = v[c] + st.bv[i];
-                            s = floor_f(s, floor_);
-                            st.pz[i][n][c] = s;
-                        }
-                    }
-                }
-            } else {
-                NDC_UNROLL
-                for (int n = 0; n < NZR; ++n)
-                    NDC_UNROLL
-                    for (int i = 0; i < SC; ++i)
-                        NDC_UNROLL
-                        for (int c = 0; c < RW; ++c) st.pz[i][n][c] = 0.f;
-            }
-            // planes outside the volume: load a clamped plane and select zero (a store in each
-            // arm of a branch would push the staging registers into private memory)
-            const int kx = k - PD;
-            const bool xlive = kx >= 0 && kx < D;
-            const T *xk = xg + (long long)clampi(kx, 0, D - 1) * plane;
+            const T *zk = zg + (long long)clampi(k, 0, D - 1) * plane;
             NDC_UNROLL
-            for (int n = 0; n < NXR; ++n) {
-                float v[RW];
-                IO::load(xk + st.xoff[n], v);
+            for (int n = 0; n < NZR; ++n)
                 NDC_UNROLL
-                for (int c = 0; c < RW; ++c) st.px[n][c] = xlive ? v[c] : 0.f;
-            }
+                for (int i = 0; i < SC; ++i) IO::load(zk + i * cplane + st.zoff[n], st.pz[i][n]);
+            const T *xk = xg + (long long)clampi(k - PD, 0, D - 1) * plane;
+            NDC_UNROLL
+            for (int n = 0; n < NXR; ++n) IO::load(xk + st.xoff[n], st.px[n]);
         };
 
         auto store_plane = [&](State &st, int k) NDC_LAMBDA {
             if (!st.ln.active) return;
+            const bool live = k < D;
             // rows outside the image are never written: they keep the zeros of the set-up
             NDC_UNROLL
             for (int n = 0; n < NZR; ++n) {
@@ -496,7 +473,8 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
                     for (int i = 0; i < SC; ++i)
                         NDC_UNROLL
                         for (int c = 0; c < RW; ++c)
-                            ex.st_(st.so + (off_s + (i * RS + n * S) * P) + c, st.pz[i][n][c]);
+                            ex.st_(st.so + (off_s + (i * RS + n * S) * P) + c,
+                                   live ? floor_f(st.pz[i][n][c] + st.bv[i], floor_) : 0.f);
                 }
             }
         };
@@ -504,12 +482,13 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
         // gather that last read that slot, which is what lets KD slots do.
         auto store_x_plane = [&](State &st, int k) NDC_LAMBDA {
             const int slot = wrap((k - PD) % XR, XR);
+            const bool live = k - PD >= 0 && k - PD < D;
             NDC_UNROLL
             for (int n = 0; n < NXR; ++n) {
                 if ((st.xok >> n) & 1u) {
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c)
-                        ex.st_(st.so + (off_x + (slot * RX + n * S) * P) + c, st.px[n][c]);
+                        ex.st_(st.so + (off_x + (slot * RX + n * S) * P) + c, live ? st.px[n][c] : 0.f);
                 }
             }
         };
@@ -637,13 +616,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
                 for (int r = 0; r < RH; ++r)
                     NDC_UNROLL
                     for (int i = 0; i < SC; ++i) {
-                        IO::load(zk + i * cplane + st.ooff[r], sv[i][r]);
-                        NDC_UNROLL
-                        for (int c = 0; c < RW; ++c) {
-                            float s = sv[i][r][c] + st.bv[i];
-                            s = floor_f(s, floor_);
-                            sv[i][r][c] = s;
-                        }
+                        IO::load(zk + i * cplane + st.ooff[r], sv[i][r]);   // (rectified after the gather)
                     }
                 float acc[2][SC][RH][RW];
                 NDC_UNROLL
@@ -679,6 +652,12 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
                         a_plane<KH, KW, KT, SC, RH, RW, 2>(ex, base, P, wt, acc);
                     }
                 }
+                NDC_UNROLL
+                for (int r = 0; r < RH; ++r)
+                    NDC_UNROLL
+                    for (int i = 0; i < SC; ++i)
+                        NDC_UNROLL
+                        for (int c = 0; c < RW; ++c) sv[i][r][c] = floor_f(sv[i][r][c] + st.bv[i], floor_);
                 T *ok_ = og + (long long)j0 * plane;
                 T *dk_ = p.s_over_den ? p.s_over_den + (og - p.out) + (long long)j0 * plane : nullptr;
                 T *rk_ = p.ratio ? p.ratio + (og - p.out) + (long long)j0 * plane : nullptr;
@@ -723,6 +702,9 @@ struct Bwd1Kernel {
     static constexpr int NXR = RH + (PH > 0 ? 2 : 0);   // rows of x/t1 a thread stages
     static constexpr int XR = KD + 1;
     static constexpr int NRED = SC * KT;
+    // own rows of the kept tensors requested a phase ahead, where the registers for it are there (the
+    // 2 x 2 tile of a 3-D filter would spill 17)
+    static constexpr bool AHEAD = SAVED && (KH_ == 1 || RH_ * RW_ < 4);
     typedef BwdParams<T> Params;
     typedef VecIO<T, RW> IO;
 
@@ -740,6 +722,7 @@ struct Bwd1Kernel {
         float accx[KD][RH][RW];      // pending planes of gx
         float acct[KD][RH][RW];      // pending planes of gt1
         float px[NXR][RW], pt[NXR][RW];
+        float qg[AHEAD ? SC : 1][RH][RW], qd[AHEAD ? SC : 1][RH][RW], qr[AHEAD ? SC : 1][RH][RW];
     };
 
     // tile rows: x / t1 have TH + 4*PH (row j = image r0 - 2*PH + j); gn / gd have
@@ -783,24 +766,17 @@ struct Bwd1Kernel {
 
         auto load_plane = [&](State &st, int k) NDC_LAMBDA {
             if (!st.ln.active) return;
-            // planes past the end: load the last plane and select zero (a store in each arm of
-            // a branch would push the staging registers into private memory)
-            const bool live = k < D;
+            // (planes past the end: the last one, staged as zero; see FwdKernel for why not here)
             const long long ko = (long long)clampi(k, 0, D - 1) * plane;
             NDC_UNROLL
             for (int n = 0; n < NXR; ++n) {
-                float vx[RW], vt[RW];
-                IO::load(xg + ko + st.xoff[n], vx);
-                IO::load(t1g + ko + st.xoff[n], vt);
-                NDC_UNROLL
-                for (int c = 0; c < RW; ++c) {
-                    st.px[n][c] = live ? vx[c] : 0.f;
-                    st.pt[n][c] = live ? vt[c] : 0.f;
-                }
+                IO::load(xg + ko + st.xoff[n], st.px[n]);
+                IO::load(t1g + ko + st.xoff[n], st.pt[n]);
             }
         };
         auto store_plane = [&](State &st, int k) NDC_LAMBDA {
             if (!st.ln.active) return;
+            const bool live = k < D;
             const int slot = wrap(k % XR, XR);
             // rows outside the image are never written: they keep the zeros of the set-up
             NDC_UNROLL
@@ -809,19 +785,34 @@ struct Bwd1Kernel {
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) {
                         const int o = st.so + (slot * RX + n * S) * P + c;
-                        ex.st_(off_x + o, st.px[n][c]);
-                        ex.st_(off_t + o, st.pt[n][c]);
+                        ex.st_(off_x + o, live ? st.px[n][c] : 0.f);
+                        ex.st_(off_t + o, live ? st.pt[n][c] : 0.f);
                     }
                 }
             }
+        };
+        // SAVED: gout, s/d, n/d of the own rows of plane j, requested a phase before they are used (8 x 32
+        // channels of 256^2 in float32 291 -> 271 us, 64 channels of 45 x 53 x 77 in bfloat16 489 -> 467)
+        auto load_saved = [&](State &st, int j) NDC_LAMBDA {
+            if (!st.ln.active) return;
+            const long long ko = (long long)clampi(j, 0, D - 1) * plane;
+            NDC_UNROLL
+            for (int r = 0; r < (AHEAD ? RH : 0); ++r)
+                NDC_UNROLL
+                for (int i = 0; i < SC; ++i) {
+                    IO::load(gg + i * cplane + ko + st.ooff[r], st.qg[i][r]);
+                    IO::load(dg + i * cplane + ko + st.ooff[r], st.qd[i][r]);
+                    IO::load(rg + i * cplane + ko + st.ooff[r], st.qr[i][r]);
+                }
         };
 
         // gn, gd of NR rows starting at gn/gd tile row j (image row r0 - PH + j): computed,
         // published to LDS, and returned in acc[0] / acc[1]
         // lo: LDS word offset of (tile row j, first own column) inside a plane
-        auto gn_gd_rows = [&](State &st, int j1, int j, int lo, auto nr_tag,
+        auto gn_gd_rows = [&](State &st, int j1, int j, int lo, auto nr_tag, auto own_tag,
                               float (&acc)[2][SC][decltype(nr_tag)::value][RW]) NDC_LAMBDA {
             constexpr int NR = decltype(nr_tag)::value;
+            constexpr bool OWN = decltype(own_tag)::value != 0;   // the thread's own rows
             float sv[SC][NR][RW], gv[SC][NR][RW];
             const long long ko = (long long)j1 * plane;
             NDC_UNROLL
@@ -831,13 +822,22 @@ struct Bwd1Kernel {
                 const int o = clampi(row, 0, H - 1) * W + st.ln.c0;
                 NDC_UNROLL
                 for (int i = 0; i < SC; ++i) {
-                    IO::load(gg + i * cplane + ko + o, gv[i][r]);
-                    if (SAVED) {
-                        // sv <- s/d, acc[0] <- n/d (as saved by the forward)
-                        IO::load(dg + i * cplane + ko + o, sv[i][r]);
-                        IO::load(rg + i * cplane + ko + o, acc[0][i][r]);
+                    if constexpr (AHEAD && OWN) {
+                        NDC_UNROLL
+                        for (int c = 0; c < RW; ++c) {
+                            gv[i][r][c] = st.qg[i][r][c];
+                            sv[i][r][c] = st.qd[i][r][c];
+                            acc[0][i][r][c] = st.qr[i][r][c];
+                        }
                     } else {
-                        IO::load(zg + i * cplane + ko + o, sv[i][r]);
+                        IO::load(gg + i * cplane + ko + o, gv[i][r]);
+                        if (SAVED) {
+                            // sv <- s/d, acc[0] <- n/d (as saved by the forward)
+                            IO::load(dg + i * cplane + ko + o, sv[i][r]);
+                            IO::load(rg + i * cplane + ko + o, acc[0][i][r]);
+                        } else {
+                            IO::load(zg + i * cplane + ko + o, sv[i][r]);
+                        }
                     }
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) {
@@ -924,6 +924,7 @@ struct Bwd1Kernel {
                     for (int c = 0; c < RW; ++c) st.accx[a][r][c] = st.acct[a][r][c] = 0.f;
             for (int i = tid; i < total; i += nthreads) ex.st_(i, 0.f);
             load_plane(st, k_first);
+            if constexpr (AHEAD) load_saved(st, k_first - PD);
         });
         ex.sync();
         ex.each([&](State &st, int) NDC_LAMBDA { store_plane(st, k_first); });
@@ -943,7 +944,7 @@ struct Bwd1Kernel {
                 {
                     float acc[2][SC][RH][RW];
                     const int j = PH + st.ln.strip * RH;
-                    gn_gd_rows(st, j1, j, st.ob + (PW + PH * P), IntTag<RH>(), acc);
+                    gn_gd_rows(st, j1, j, st.ob + (PW + PH * P), IntTag<RH>(), IntTag<1>(), acc);
                     if (need_gh && own1) {
                         // own rows: A-side filter-gradient terms, re-reading the x / t1 windows
                         // (read ahead: for the 2x2 float32 tile this costs two spilled registers
@@ -981,7 +982,7 @@ struct Bwd1Kernel {
                 }
                 if (XT && st.ln.strip < 2 * PH) {
                     float acc[2][SC][1][RW];
-                    gn_gd_rows(st, j1, halo_row(st.ln.strip, PH, TH), st.ho, IntTag<1>(), acc);
+                    gn_gd_rows(st, j1, halo_row(st.ln.strip, PH, TH), st.ho, IntTag<1>(), IntTag<0>(), acc);
                 }
             });
             ex.sync();
@@ -990,6 +991,7 @@ struct Bwd1Kernel {
             ex.each([&](State &st, int) NDC_LAMBDA {
                 if (!st.ln.active) return;
                 load_plane(st, k + 1);
+                if constexpr (AHEAD) load_saved(st, j1 + 1);
                 if (live1) {
                     NDC_ROLLED
                     for (int ii = 0; ii < SC; ++ii) {
@@ -1098,28 +1100,20 @@ struct Bwd2Kernel {
 
         auto load_plane = [&](State &st, int k) NDC_LAMBDA {
             if (!st.ln.active) return;
-            // planes past the end: load the last plane and select zero (a store in each arm of
-            // a branch would push the staging registers into private memory)
-            const bool live = k < D;
+            // (planes past the end: the last one, staged as zero; see FwdKernel for why not here)
             const long long ko = (long long)clampi(k, 0, D - 1) * plane;
             NDC_UNROLL
             for (int n = 0; n < NXR; ++n) {
-                float vx[RW], vt[RW], vg[RW];
                 if (!SAVED) {
-                    IO::load(xg + ko + st.xoff[n], vx);
-                    IO::load(t1g + ko + st.xoff[n], vt);
+                    IO::load(xg + ko + st.xoff[n], st.px[n]);
+                    IO::load(t1g + ko + st.xoff[n], st.pt[n]);
                 }
-                IO::load(gt1g + ko + st.xoff[n], vg);
-                NDC_UNROLL
-                for (int c = 0; c < RW; ++c) {
-                    st.px[n][c] = (!SAVED && live) ? vx[c] : 0.f;
-                    st.pt[n][c] = (!SAVED && live) ? vt[c] : 0.f;
-                    st.pg[n][c] = live ? vg[c] : 0.f;
-                }
+                IO::load(gt1g + ko + st.xoff[n], st.pg[n]);
             }
         };
         auto store_plane = [&](State &st, int k) NDC_LAMBDA {
             if (!st.ln.active) return;
+            const bool live = k < D;
             const int slot = wrap(k % XR, XR);
             NDC_UNROLL
             for (int n = 0; n < NXR; ++n) {
@@ -1128,10 +1122,10 @@ struct Bwd2Kernel {
                     for (int c = 0; c < RW; ++c) {
                         const int o = st.so + (slot * RX + n * S) * P + c;
                         if (!SAVED) {
-                            ex.st_(off_x + o, st.px[n][c]);
-                            ex.st_(off_t + o, st.pt[n][c]);
+                            ex.st_(off_x + o, live ? st.px[n][c] : 0.f);
+                            ex.st_(off_t + o, live ? st.pt[n][c] : 0.f);
                         }
-                        ex.st_(off_g + o, st.pg[n][c]);
+                        ex.st_(off_g + o, live ? st.pg[n][c] : 0.f);
                     }
                 }
             }
@@ -1180,7 +1174,6 @@ struct Bwd2Kernel {
                 const long long ko = (long long)j0 * plane;
                 NDC_UNROLL
                 for (int r = 0; r < RH; ++r) {
-                    const bool ok = (st.ook >> r) & 1u;
                     NDC_UNROLL
                     for (int i = 0; i < SC; ++i) {
                         IO::load(zg + i * cplane + ko + st.ooff[r], sv[i][r]);
@@ -1190,14 +1183,6 @@ struct Bwd2Kernel {
                         } else {
                             NDC_UNROLL
                             for (int c = 0; c < RW; ++c) rv[i][r][c] = 0.f;
-                        }
-                        NDC_UNROLL
-                        for (int c = 0; c < RW; ++c) {
-                            // with the ReLU on, s <= 0 marks a masked element
-                            float s = sv[i][r][c] + st.bv[i];
-                            s = floor_f(s, floor_);
-                            sv[i][r][c] = ok ? s : 0.f;
-                            gv[i][r][c] = ok ? gv[i][r][c] : 0.f;
                         }
                     }
                 }
@@ -1224,6 +1209,19 @@ struct Bwd2Kernel {
                         base[NA > 1 ? 1 : 0] = off_t + ob;
                     }
                     a_plane<KH, KW, KT, SC, RH, RW, NA, (KH > 1 && SAVED)>(ex, base, P, wt, acc);
+                }
+                NDC_UNROLL
+                for (int r = 0; r < RH; ++r) {
+                    const bool ok = (st.ook >> r) & 1u;
+                    NDC_UNROLL
+                    for (int i = 0; i < SC; ++i)
+                        NDC_UNROLL
+                        for (int c = 0; c < RW; ++c) {
+                            // with the ReLU on, s <= 0 marks a masked element
+                            const float s = floor_f(sv[i][r][c] + st.bv[i], floor_);
+                            sv[i][r][c] = ok ? s : 0.f;
+                            gv[i][r][c] = ok ? gv[i][r][c] : 0.f;
+                        }
                 }
                 if (need_gh) {
                     // K-side filter-gradient term: re-read the gt1 window
