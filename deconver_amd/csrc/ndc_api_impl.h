@@ -648,7 +648,9 @@ static int gemm_check(long long batch, long long cin, long long cout, long long 
 // few to give 256 such tiles and splits, where 64 x 64 tiles spread the work wider.  The voxel
 // axis is split until the launch has 512 workgroups (256 with the largest tiles over long rows:
 // 0.55 ms against 0.56-0.68 for the 256 x 64 result over 2 x 128^3), in chunks of at least 256 voxels,
-// so that partial results stay small next to the operands.  Rows of half a million voxels and
+// so that partial results stay small next to the operands; of at least 64 where that leaves CUs
+// without a workgroup, whose stages each wait for memory (128 x 32 over 16 384 voxels in float32, 64
+// splits, 9.8 us, 256 of them 6.0).  Rows of half a million voxels and
 // more are read 16 granules at a time (see the kernel), shorter ones 8.
 static ndc::WgradPlan wgrad_plan(long long batch, long long rows, long long cols, long long n, int esz)
 {
@@ -659,13 +661,14 @@ static ndc::WgradPlan wgrad_plan(long long batch, long long rows, long long cols
     else if (cols <= 32 && rows > 64) w.bm = 128, w.bn = 32;
     else if (rows <= 32 && cols > 64) w.bm = 32, w.bn = 128;
     else w.bm = w.bn = 64;
-    const long long most = n / 256 > 0 ? n / 256 : 1;             // splits of a sample
+    long long most = n / 256 > 0 ? n / 256 : 1;                   // splits of a sample
     auto tiles_of = [&] { return ((rows + w.bm - 1) / w.bm) * ((cols + w.bn - 1) / w.bn); };
     // (lane offsets within a tile are 32-bit: fewer rows per tile on enormous grids)
     if (tiles_of() * most * batch < 256 || (long double)(w.bm > w.bn ? w.bm : w.bn) * n * esz > 4.0e9L) w.bm = w.bn = 64;
     w.depth = esz == 2 && n >= (1 << 19) ? 16 : 8;
     const long long stage = 16 / esz * w.depth, tiles = tiles_of();   // voxels per stage
     const long long want = w.bm + w.bn == 320 && n >= (1 << 19) ? 256 : 512;
+    if (tiles * most * batch < 256 && n >= 128) most = n / 64;
     long long per = (want + tiles * batch - 1) / (tiles * batch);
     if (per > most) per = most;
     w.chunk = ((n + per - 1) / per + stage - 1) / stage * stage;
