@@ -1,9 +1,10 @@
 """Channel-first helper layers around the NDC update (``deconver/layers`` of the reference):
 ``Linear`` (1x1 projection, parameters held by an ``nn.Conv1d`` as there), ``MLP``,
 ``LayerNorm``, and the network's resampling convolutions, head and stem as subclasses of the
-``torch.nn`` convolutions.  On the GPU the projections are batched channel-first GEMMs
-(hipBLASLt through ``torch.bmm``) followed by one pass of the HIP library for bias, activation
-and residual sum; the strided convolutions are a regrouping copy in front of the same
+``torch.nn`` convolutions.  On the GPU the projections are channel-first GEMMs
+with bias, activation and residual sum in their epilogues (the HIP library's streaming and tiled
+ones; the library GEMM through ``torch.bmm`` where it is ahead);
+the strided convolutions are a regrouping copy in front of the same
 projection.  Parameter names and shapes match the reference, so its checkpoints load
 unchanged."""
 
