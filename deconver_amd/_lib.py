@@ -46,6 +46,7 @@ EXPORTS = (
     "ndc_bias_act",
     "ndc_bias_act_backward",
     "ndc_regroup",
+    "ndc_columns",
     "ndc_row_sums",
     "ndc_chnorm_parts",
     "ndc_chnorm_forward",
@@ -163,6 +164,8 @@ class NdcLibrary:
         d.ndc_weight_grad_workspace_bytes.restype = ctypes.c_size_t
         d.ndc_weight_grad_workspace_bytes.argtypes = [i64, i64, i64, i64, ctypes.c_int]
         d.ndc_weight_grad.argtypes = [vp, vp, fp, fp, i64, i64, i64, i64, ctypes.c_int, vp, ctypes.c_size_t, vp]
+        d.ndc_columns.argtypes = [vp, vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int,
+                                  ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]
         d.ndc_regroup.argtypes = [vp, vp, vp, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                    ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, vp]
         d.ndc_taps_bytes.restype = ctypes.c_size_t
@@ -382,6 +385,9 @@ class NdcLibrary:
 
     def row_sums(self, x: int, partial: int, rows: int, n: int, dtype: int, stream) -> None:
         self._check(self._dll.ndc_row_sums(x, partial, rows, n, dtype, stream), "ndc_row_sums")
+
+    def columns(self, src: int, dst: int, rows: int, D: int, H: int, W: int, k, dtype: int, stream) -> None:
+        self._check(self._dll.ndc_columns(src, dst, rows, D, H, W, *k, dtype, stream), "ndc_columns")
 
     def regroup2(self, src: int, dst: int, bias: Optional[int], rows: int, channels: int, D: int, H: int,
                  W: int, depth2: bool, dtype: int, to_channels: bool, stream) -> None:

@@ -7,6 +7,7 @@
 
 #include "../../include/deconver_ndc.h"
 #include "ndc_common.h"
+#include "ndc_columns.h"
 #include "ndc_direct.h"
 #include "ndc_fused_api.h"
 
@@ -823,6 +824,38 @@ int ndc_regroup(const void *src, void *dst, const float *bias, int64_t rows, int
     const int st = ndc::Backend::regroup2(src, dst, bias, rows, (int)channels, (int)D, (int)H, (int)W,
                                           depth2 ? 1 : 0, esz, to_channels ? 1 : 0, stream);
     return st == -2 ? (int)NDC_ERR_GEOMETRY : st;
+}
+
+}  // extern "C"
+
+template <typename E, int V>
+static int columns_launch(const ndc::KGeom &q, const void *src, void *dst, long long rows, void *stream)
+{
+    const ndc::Columns<E, V> op = {q, (const E *)src, (E *)dst};
+    return ndc::Backend::per_unit(rows * q.KT, q.SP / V, stream, op);
+}
+
+extern "C" {
+
+int ndc_columns(const void *src, void *dst, int64_t rows, int64_t D, int64_t H, int64_t W, int kD, int kH, int kW,
+                int dtype, void *stream)
+{
+    if (!src || !dst) return NDC_ERR_NULL;
+    if (rows < 1 || rows > 0x7fffffffLL || D < 1 || H < 1 || W < 1 || D > 0x7fffffffLL || H > 0x7fffffffLL ||
+        W > 0x7fffffffLL || (long double)D * H * W >= 2147483648.0L || src == dst)
+        return NDC_ERR_GEOMETRY;
+    const ndc_geom g = {(int)rows, 1, 1, 1, {(int)D, (int)H, (int)W}, {kD, kH, kW}, dtype, 0, NDC_PATH_DIRECT, 0.f};
+    ndc::KGeom q;
+    const int st = ndc::make_kgeom(&g, q);
+    if (st) return st;
+    if (rows * q.KT > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
+    // 16 bytes per store where rows are made of them
+    const int esz = dtype == NDC_BF16 ? 2 : 4;
+    const bool wide = W % (16 / esz) == 0 && aligned16(dst);
+    int r;
+    if (esz == 2) r = wide ? columns_launch<uint16_t, 8>(q, src, dst, rows, stream) : columns_launch<uint16_t, 1>(q, src, dst, rows, stream);
+    else r = wide ? columns_launch<uint32_t, 4>(q, src, dst, rows, stream) : columns_launch<uint32_t, 1>(q, src, dst, rows, stream);
+    return r == -2 ? (int)NDC_ERR_GEOMETRY : r;
 }
 
 int ndc_gconv(const ndc_geom *g, const void *in, const float *h, const float *bias, int adjoint,

@@ -984,6 +984,23 @@ Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
     return regroup_run(x, to_channels, f32_vector(bias), scope.stream);
 }
 
+// Column matrix of a contiguous (B, C, *S) tensor for odd kernel extents k: (B, C * taps, voxels).
+// Not differentiable: the caller takes it for inputs that need no gradient.
+Tensor columns(const Tensor &x, const std::vector<int64_t> &k)
+{
+    Scope scope(x);
+    const int64_t nd = x.dim() - 2;
+    int64_t size[3] = {1, 1, 1}, ext[3] = {1, 1, 1}, taps = 1, n = 1;
+    for (int64_t d = 0; d < nd; ++d) {
+        size[3 - nd + d] = x.size(2 + d), ext[3 - nd + d] = k[d];
+        taps *= k[d], n *= x.size(2 + d);
+    }
+    Tensor out = empty({x.size(0), x.size(1) * taps, n}, x);
+    check(ndc_columns(ptr(x), out_ptr(out), x.size(0) * x.size(1), size[0], size[1], size[2], (int)ext[0], (int)ext[1],
+                      (int)ext[2], dtype_tag(x), scope.stream), "ndc_columns");
+    return out;
+}
+
 OptTensor taps_for(const Tensor &x, const Tensor &h, int64_t groups, int64_t m, int64_t sc)
 {
     Scope scope(x);
@@ -1021,6 +1038,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("row_norm_skip", &row_norm_skip);
     m.def("channel_norm", &channel_norm);
     m.def("regroup", &regroup);
+    m.def("columns", &columns);
     m.def("weight_grad_chunks", &weight_grad_chunks);
     m.def("weight_grad_plan", &weight_grad_plan);
 }

@@ -189,9 +189,14 @@ class _PatchConvTransposeMixin:
 def unfold_conv(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """``conv(x, weight, bias, stride=1, padding=k // 2)`` for odd kernel sizes ``k`` as a column
     matrix (every tap's shifted copy of the zero-padded input, channel-major then tap: the order
-    of the weight's ``(Cin, *k)`` axes) followed by the 1x1 projection."""
+    of the weight's ``(Cin, *k)`` axes) followed by the 1x1 projection.  An input that needs no
+    gradient -- images -- has the matrix made by one launch."""
     k = tuple(weight.shape[2:])
     size = x.shape[2:]
+    if (x.is_cuda and len(k) <= 3 and x.dtype in (torch.bfloat16, torch.float32) and x.numel() > 0
+            and math.prod(size) < 2 ** 31 and not (torch.is_grad_enabled() and x.requires_grad)):
+        cols = _lib.get_native().columns(x.contiguous(), list(k))
+        return pointwise_linear(cols, weight, bias).view(x.shape[0], -1, *size)
     pad = []
     for v in reversed(k):
         pad += [v // 2, v // 2]

@@ -410,6 +410,16 @@ int ndc_regroup(const void *src, void *dst, const float *bias, int64_t rows, int
                  int64_t H, int64_t W, int depth2, int dtype, int to_channels, void *stream);
 
 /*
+ * Column matrix of a stride-1 convolution with odd kernel (kD, kH, kW) and zero padding k / 2: the
+ * data movement of the reference's stem (deconver/unet.py:175-276) once its arithmetic is the 1x1
+ * projection.  dst[r][tap][d][h][w] = src[r][d + td - kD/2][h + th - kH/2][w + tw - kW/2], zero
+ * outside the grid, tap = (td kH + th) kW + tw.
+ *   rows       batch * channels; D H W below 2^31; src, dst distinct
+ */
+int ndc_columns(const void *src, void *dst, int64_t rows, int64_t D, int64_t H, int64_t W, int kD, int kH,
+                int kW, int dtype, void *stream);
+
+/*
  * The 1x1 projections and their input gradients as a tiled GEMM, for the tensors
  * ndc_pointwise_gemm does not take (float32, any channel and voxel count, any alignment to the
  * element): on channel-first (batch, c, n) tensors
