@@ -77,6 +77,20 @@ Tensor empty_f32(at::IntArrayRef size, const Tensor &like)
 bool wants_grad(const Tensor &t) { return t.defined() && t.requires_grad(); }
 bool wants_grad(const OptTensor &t) { return t && wants_grad(*t); }
 
+// The nodes have no forward-mode rule.  Where autograd records a call its engine says so; a call that
+// it does not record would drop the tangents without a word.
+void no_tangents() {}
+template <class... Rest> void no_tangents(const Tensor &t, const Rest &...rest);
+template <class... Rest> void no_tangents(const OptTensor &t, const Rest &...rest)
+{
+    no_tangents(t ? *t : Tensor(), rest...);
+}
+template <class... Rest> void no_tangents(const Tensor &t, const Rest &...rest)
+{
+    TORCH_CHECK(!t.defined() || !t._fw_grad(0).defined(), "the NDC nodes do not implement forward-mode differentiation");
+    no_tangents(rest...);
+}
+
 // Which gradients the engine asks for, by forward argument.  (The engine counts only the
 // arguments that are tensors.)
 struct Needs {
@@ -535,6 +549,7 @@ struct Update : public torch::autograd::Function<Update> {
 Tensor update(const Tensor &x, const Tensor &z, const Tensor &h, const OptTensor &bias, int64_t groups, int64_t m, int64_t sc,
               double eps, bool relu_input, const OptTensor &taps, bool save_ratio)
 {
+    no_tangents(x, z, h, bias);
     const UpdateConfig c{groups, m, sc, eps, relu_input, save_ratio};
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(z) || wants_grad(h) || wants_grad(bias)))
         return Update::apply(x, z, h, bias, taps, c);
@@ -605,6 +620,7 @@ Tensor projected_update(const Tensor &x, const Tensor &weight, const Tensor &h, 
                         int64_t m, int64_t sc, double eps, const OptTensor &taps, bool rectified_input, bool rectify,
                         bool save_ratio)
 {
+    no_tangents(x, weight, h, bias);
     const UpdateConfig c{groups, m, sc, eps, true, save_ratio};
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(h) || wants_grad(bias)))
         return Projected::apply(x, weight, h, bias, taps, c, rectified_input, rectify);
@@ -694,6 +710,7 @@ struct Linear : public torch::autograd::Function<Linear> {
 Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, int64_t act, const OptTensor &residual,
               bool premasked, bool transposed)
 {
+    no_tangents(x, weight, bias, residual);
     const Tensor xc = x.contiguous();
     OptTensor res = residual;
     if (res && res->defined()) {
@@ -776,6 +793,7 @@ struct Mlp : public torch::autograd::Function<Mlp> {
 Tensor mlp(const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor &w2, const OptTensor &b2,
            const OptTensor &residual)
 {
+    no_tangents(x, w1, b1, w2, b2, residual);
     const Tensor xc = x.contiguous();
     OptTensor res = residual;
     if (res && res->defined()) {
@@ -863,6 +881,7 @@ struct RowNormSkip : public torch::autograd::Function<RowNormSkip> {
 
 Tensor row_norm(const Tensor &x, double eps)
 {
+    no_tangents(x);
     if (at::GradMode::is_enabled() && wants_grad(x)) return RowNorm::apply(x, eps);
     Scope scope(x);
     Tensor stats;
@@ -871,6 +890,7 @@ Tensor row_norm(const Tensor &x, double eps)
 
 std::pair<Tensor, Tensor> row_norm_skip(const Tensor &x, double eps)
 {
+    no_tangents(x);
     if (!at::GradMode::is_enabled() || !wants_grad(x)) return {row_norm(x, eps), x};
     auto r = RowNormSkip::apply(x, eps);
     return {r[0], r[1]};
@@ -928,6 +948,7 @@ struct ChannelNorm : public torch::autograd::Function<ChannelNorm> {
 
 Tensor channel_norm(const Tensor &x, const OptTensor &weight, const OptTensor &bias, double eps)
 {
+    no_tangents(x, weight, bias);
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(bias)))
         return ChannelNorm::apply(x, weight, bias, eps);
     Scope scope(x);
@@ -979,6 +1000,7 @@ struct Regroup : public torch::autograd::Function<Regroup> {
 
 Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
 {
+    no_tangents(x, bias);
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(bias))) return Regroup::apply(x, to_channels, bias);
     Scope scope(x);
     return regroup_run(x, to_channels, f32_vector(bias), scope.stream);
@@ -988,6 +1010,7 @@ Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
 // Not differentiable: the caller takes it for inputs that need no gradient.
 Tensor columns(const Tensor &x, const std::vector<int64_t> &k)
 {
+    no_tangents(x);
     Scope scope(x);
     const int64_t nd = x.dim() - 2;
     int64_t size[3] = {1, 1, 1}, ext[3] = {1, 1, 1}, taps = 1, n = 1;
