@@ -49,11 +49,15 @@ struct Scope {
     c10::impl::ExcludeDispatchKeyGuard autocast;
     at::AutoDispatchBelowADInplaceOrView below;
     void *stream;
-    explicit Scope(const Tensor &t)
-        : device(t.device()), autocast(c10::autocast_dispatch_keyset),
-          stream((void *)c10::hip::getCurrentHIPStream(t.device().index()).stream())
+    static c10::Device on_gpu(const Tensor &t)
     {
         TORCH_CHECK(t.is_cuda(), "the HIP kernels run on GPU tensors only");
+        return t.device();
+    }
+    explicit Scope(const Tensor &t)
+        : device(on_gpu(t)), autocast(c10::autocast_dispatch_keyset),
+          stream((void *)c10::hip::getCurrentHIPStream(t.device().index()).stream())
+    {
     }
 };
 
@@ -72,6 +76,41 @@ Tensor empty(at::IntArrayRef size, const Tensor &like) { return at::empty(size, 
 Tensor empty_f32(at::IntArrayRef size, const Tensor &like)
 {
     return at::empty(size, like.options().dtype(at::kFloat));
+}
+
+// The kernels see pointers and the sizes of one tensor: what the others have to be is checked here,
+// before anything is launched.
+void check_device(const Tensor &t, const Tensor &like, const char *what)
+{
+    TORCH_CHECK(t.device() == like.device(), "expected all tensors on one device, but ", what, " is on ", t.device(),
+                " and the input on ", like.device());
+}
+
+void check_vector(const OptTensor &t, const Tensor &like, int64_t entries, const char *what)
+{
+    if (!t || !t->defined()) return;
+    check_device(*t, like, what);
+    TORCH_CHECK_VALUE(t->numel() == entries, what, " has ", t->numel(), " entries, expected one per channel, ", entries);
+}
+
+// A 1x1 projection of `channels` channels over the voxels of x, (B, ., *S): its weight (rows of W,
+// or with `transposed` of its transpose), bias and residual (B, cout, *S).  Returns cout.
+int64_t check_projection(const Tensor &x, int64_t channels, const Tensor &w, bool transposed, const OptTensor &bias,
+                         const OptTensor &res)
+{
+    TORCH_CHECK_VALUE(w.dim() >= 2, "expected a weight matrix, got ", w.sizes());
+    const int64_t rows = w.size(0), cols = rows ? w.numel() / rows : 0, cout = transposed ? cols : rows;
+    TORCH_CHECK((transposed ? rows : cols) == channels, "weight of shape ", w.sizes(), transposed ? " (transposed)" : "", " takes ",
+                transposed ? rows : cols, " channels, but the input has ", channels);
+    check_device(w, x, "the weight");
+    check_vector(bias, x, cout, "the bias");
+    if (res && res->defined()) {
+        auto size = x.sizes().vec();
+        size[1] = cout;
+        TORCH_CHECK_VALUE(res->sizes() == at::IntArrayRef(size), "the residual has shape ", res->sizes(), ", expected ", size);
+        check_device(*res, x, "the residual");
+    }
+    return cout;
 }
 
 bool wants_grad(const Tensor &t) { return t.defined() && t.requires_grad(); }
@@ -435,6 +474,10 @@ Tensor update_forward(Tensor x, Tensor z, const Tensor &h, const Tensor &bias, T
     f.path = g.path;
     // (kept only where the backward kernels of this geometry read them)
     const bool keep = grad && c.save_ratio && ndc_backward_uses_saved(&g);
+    if (taps.defined()) {
+        check_device(taps, x, "the filter table");
+        TORCH_CHECK_VALUE(taps.is_contiguous() && taps.nbytes() >= ndc_taps_bytes(&g), "the filter table is another geometry's");
+    }
     // packed once here, used by the forward kernel and again by the backward's
     if (!taps.defined()) taps = prepare_taps(g, hc, stream);
     Tensor out = at::empty_like(z);
@@ -621,6 +664,9 @@ Tensor projected_update(const Tensor &x, const Tensor &weight, const Tensor &h, 
                         bool save_ratio)
 {
     no_tangents(x, weight, h, bias);
+    TORCH_CHECK_VALUE(x.dim() >= 3 && x.dim() <= 5, "expected a (B, C, *S) tensor with 1-3 spatial dims, got ", x.sizes());
+    check_projection(x, x.size(1), weight, false, bias, OptTensor());
+    check_device(h, x, "the filter");
     const UpdateConfig c{groups, m, sc, eps, true, save_ratio};
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(h) || wants_grad(bias)))
         return Projected::apply(x, weight, h, bias, taps, c, rectified_input, rectify);
@@ -711,6 +757,8 @@ Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, int6
               bool premasked, bool transposed)
 {
     no_tangents(x, weight, bias, residual);
+    TORCH_CHECK_VALUE(x.dim() == 3, "expected a (B, C, n) tensor, got ", x.sizes());
+    check_projection(x, x.size(1), weight, transposed, bias, residual);
     const Tensor xc = x.contiguous();
     OptTensor res = residual;
     if (res && res->defined()) {
@@ -794,6 +842,9 @@ Tensor mlp(const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor 
            const OptTensor &residual)
 {
     no_tangents(x, w1, b1, w2, b2, residual);
+    TORCH_CHECK_VALUE(x.dim() == 3, "expected a (B, C, n) tensor, got ", x.sizes());
+    const int64_t hidden = check_projection(x, x.size(1), w1, false, b1, OptTensor());
+    check_projection(x, hidden, w2, false, b2, residual);
     const Tensor xc = x.contiguous();
     OptTensor res = residual;
     if (res && res->defined()) {
@@ -949,6 +1000,9 @@ struct ChannelNorm : public torch::autograd::Function<ChannelNorm> {
 Tensor channel_norm(const Tensor &x, const OptTensor &weight, const OptTensor &bias, double eps)
 {
     no_tangents(x, weight, bias);
+    TORCH_CHECK_VALUE(x.dim() == 3, "expected a (B, C, n) tensor, got ", x.sizes());
+    check_vector(weight, x, x.size(1), "the weight");
+    check_vector(bias, x, x.size(1), "the bias");
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(bias)))
         return ChannelNorm::apply(x, weight, bias, eps);
     Scope scope(x);
@@ -1001,6 +1055,11 @@ struct Regroup : public torch::autograd::Function<Regroup> {
 Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
 {
     no_tangents(x, bias);
+    TORCH_CHECK_VALUE((x.dim() == 4 || x.dim() == 5) && x.is_contiguous(),
+                      "expected a contiguous (B, C, *S) tensor with 2-3 spatial dims, got ", x.sizes());
+    const int64_t window = int64_t(1) << (x.dim() - 2);
+    TORCH_CHECK_VALUE(to_channels || x.size(1) % window == 0, "expected a multiple of ", window, " channels, got ", x.sizes());
+    check_vector(bias, x, x.size(1) / window, "the bias");
     if (at::GradMode::is_enabled() && (wants_grad(x) || wants_grad(bias))) return Regroup::apply(x, to_channels, bias);
     Scope scope(x);
     return regroup_run(x, to_channels, f32_vector(bias), scope.stream);
@@ -1011,8 +1070,10 @@ Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
 Tensor columns(const Tensor &x, const std::vector<int64_t> &k)
 {
     no_tangents(x);
-    Scope scope(x);
     const int64_t nd = x.dim() - 2;
+    TORCH_CHECK_VALUE(nd >= 1 && nd <= 3 && (int64_t)k.size() == nd && x.is_contiguous(),
+                      "expected a contiguous (B, C, *S) tensor and one odd extent per spatial dim, got ", x.sizes());
+    Scope scope(x);
     int64_t size[3] = {1, 1, 1}, ext[3] = {1, 1, 1}, taps = 1, n = 1;
     for (int64_t d = 0; d < nd; ++d) {
         size[3 - nd + d] = x.size(2 + d), ext[3 - nd + d] = k[d];
@@ -1026,6 +1087,10 @@ Tensor columns(const Tensor &x, const std::vector<int64_t> &k)
 
 OptTensor taps_for(const Tensor &x, const Tensor &h, int64_t groups, int64_t m, int64_t sc)
 {
+    TORCH_CHECK_TYPE(h.scalar_type() == at::kFloat, "the filter must be float32");
+    TORCH_CHECK_VALUE(h.numel() > 0 && h.dim() >= 3 && h.size(0) * h.size(1) == groups * m * sc && h.is_contiguous(),
+                      "filter of shape ", h.sizes(), " does not match groups=", groups, ", m=", m, ", sc=", sc);
+    check_device(h, x, "the filter");
     Scope scope(x);
     const ndc_geom g = geom_for(x, h, UpdateConfig{groups, m, sc, 0.0, true, false}, NDC_PATH_AUTO);
     Tensor taps = prepare_taps(g, h, scope.stream);
