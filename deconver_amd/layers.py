@@ -356,7 +356,7 @@ class MLP(nn.Module):
             return None
         y = _FusedMLP.apply(flat, w1, first.linear.bias, w2, second.linear.bias,
                             None if residual is None else residual.flatten(2))
-        return y.view(x.shape)
+        return y.view(x.shape[0], w2.shape[0], *x.shape[2:])
 
 
 _CHNORM_MIN_VOXELS = 32768
