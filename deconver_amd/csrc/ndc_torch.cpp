@@ -609,15 +609,19 @@ Tensor update(const Tensor &x, const Tensor &z, const Tensor &h, const OptTensor
 // update's gx.  With `rectify` the node takes the filter parameter itself and rectifies it (the
 // filter's relu and its backward are then no nodes of their own).
 struct Projected : public torch::autograd::Function<Projected> {
-    static Tensor run(const Tensor &x, const Tensor &weight, const Tensor &h, const Tensor &bias, const Tensor &taps,
+    static Tensor run(const Tensor &x_, const Tensor &weight, const Tensor &h, const Tensor &bias, const Tensor &taps,
                       const UpdateConfig &c, bool grad, bool rectify, UpdateForward &f, void *stream)
     {
         const Matrix w(weight, false);
+        // (the GEMMs and the update read rows of voxels: any other layout is turned first)
+        const Tensor x = channel_first(x_, stream);
         auto size = x.sizes().vec();
         // (float32: the library's product, whose bits decide which source units are on)
         Tensor z = project(w, x.flatten(2), x.scalar_type() == at::kFloat, stream);
         size[1] = w.cout();
-        return update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
+        Tensor out = update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
+        f.x_last = channels_last(x_);
+        return out;
     }
     static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight, const Tensor &h, const OptTensor &bias,
                           const OptTensor &taps, const UpdateConfig &c, bool rectified_input, bool rectify)

@@ -118,7 +118,8 @@ def projected_update(x: Tensor, weight: Tensor, h: Tensor, bias: Optional[Tensor
     (``gx += W^T gz``, one rounding instead of two in bfloat16).
 
     Args:
-        x: input ``(B, C, *S)``, contiguous, float32 or bfloat16 on the GPU.
+        x: input ``(B, C, *S)``, float32 or bfloat16 on the GPU, in any layout (channels-last tensors
+            come in through the library's tiled transposition, and their gradient goes back so).
         weight: the projection's weight ``(groups*sc, C)``, any floating dtype (cast to ``x``'s
             for the GEMMs; its gradient comes back in its own dtype).
         h, bias, groups, m, sc, eps, taps: as for ``deconv_update``.

@@ -99,3 +99,40 @@ def test_update_node_takes_channels_last_operands(dtype, ks, sp):
     assert torch.equal(out_cl, out_cf)
     for a, b in zip(grads_cl, grads_cf):
         assert torch.equal(a, b)
+
+
+def _layouts(t):
+    """The same values in other layouts: channels-last, spatial axes swapped in memory, every other
+    voxel of a wider tensor."""
+    yield _cl(t)
+    yield t.transpose(-1, -2).contiguous().transpose(-1, -2)
+    wide = torch.zeros(*t.shape[:-1], 2 * t.shape[-1], dtype=t.dtype, device=t.device)
+    wide[..., ::2] = t
+    yield wide[..., ::2]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rectified", [False, True])
+@pytest.mark.parametrize("size", [(6, 10), (4, 6, 8)])
+def test_projected_update_of_any_layout(size, rectified, dtype):
+    """Values and gradients equal the channel-first call's bit for bit, and the gradient of a
+    channels-last input is channels-last."""
+    from deconver_amd.functional import projected_update
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *s: torch.rand(*s, generator=gen, device="cuda")   # noqa: E731
+    base, g = rand(2, 8, *size).to(dtype), rand(2, 16, *size).to(dtype)
+    w, h, b = rand(16, 8) - 0.3, rand(8, 2, *[3] * len(size)), rand(16)
+
+    def call(x):
+        leaves = [t.detach().requires_grad_(True) for t in (x, w, h, b)]
+        y = projected_update(*leaves, groups=8, m=1, sc=2, eps=1e-8, rectified_input=rectified)
+        y.backward(g)
+        return [y.detach()] + [t.grad for t in leaves], leaves[0].grad
+
+    want, _ = call(base)
+    for x in _layouts(base):
+        assert torch.equal(x, base) and not x.is_contiguous()
+        got, gx = call(x)
+        assert all(torch.equal(a, r) for a, r in zip(got, want))
+        assert not ops.is_channels_last(x) or ops.is_channels_last(gx)
