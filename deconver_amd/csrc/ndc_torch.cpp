@@ -915,11 +915,14 @@ struct RowNorm : public torch::autograd::Function<RowNorm> {
 struct RowNormSkip : public torch::autograd::Function<RowNormSkip> {
     static variable_list forward(AutogradContext *ctx, const Tensor &x, double eps)
     {
+        // (outside the scope: below it a view is an alias without a base and with a version of its own,
+        // whose changes in place autograd would not see)
+        const Tensor skip = x.view_as(x);
         Scope scope(x);
         Tensor stats, y = row_norm_forward(x.contiguous(), eps, stats, scope.stream);
         ctx->save_for_backward({y, stats});
         ctx->set_materialize_grads(false);   // an unused output's gradient arrives undefined
-        return {y, x.view_as(x)};
+        return {y, skip};
     }
     static variable_list backward(AutogradContext *ctx, variable_list gouts)
     {

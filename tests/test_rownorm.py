@@ -172,6 +172,24 @@ def test_norm_with_skip_sums_the_two_gradients(dtype):
 
 
 @pytest.mark.gpu
+def test_the_skip_is_a_tracked_view_of_the_input():
+    """Shares memory and version with x, so that a change in place is refused or seen, never lost."""
+    norm = dc.norm.InstanceNorm3d(4).cuda()
+    x0 = torch.randn(1, 4, 4, 4, 8, device="cuda", requires_grad=True)
+    x = x0 * 1
+    _, skip = norm.with_skip(x)
+    assert skip._base is x and skip.data_ptr() == x.data_ptr()
+    with pytest.raises(RuntimeError, match="is a view and is being modified inplace"):
+        skip.mul_(3.0)
+    square = skip * skip              # keeps skip for its gradient
+    with torch.no_grad():
+        x.mul_(2.0)
+    assert skip._version == x._version == 1
+    with pytest.raises(RuntimeError, match="modified inplace"):
+        square.sum().backward()
+
+
+@pytest.mark.gpu
 def test_hip_rownorm_is_reproducible_and_handles_views():
     x = torch.randn(2, 6, 16, 16, 16, device="cuda")
     a = dc.instance_norm(x)
