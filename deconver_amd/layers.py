@@ -269,6 +269,13 @@ class PatchConvTranspose3d(_PatchConvTransposeMixin, nn.ConvTranspose3d):
     pass
 
 
+def _hooked(*modules: nn.Module) -> bool:
+    """Whether a hook watches a call of one of ``modules`` (or of every module): a caller that runs a
+    module's work inside another call then calls the module instead."""
+    return nn.modules.module._has_any_global_hook() or any(
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+
+
 class Linear(nn.Module):
     """Pointwise linear map over channels for ``(N, C, *)`` inputs (layers/linear.py:34-58).
 
@@ -344,8 +351,10 @@ class MLP(nn.Module):
     @staticmethod
     def _fused(first: "Linear", second: "Linear", x: torch.Tensor, residual: Optional[torch.Tensor]):
         """The block as one node for bfloat16 (stored or under autocast) and float32 tensors on the
-        GPU, else None."""
-        if not _gemm_route(x):
+        GPU, else None: also where the projections are hooked or of a class of their own, which are
+        called as modules."""
+        if not _gemm_route(x) or type(first) is not Linear or type(second) is not Linear or _hooked(
+                first, first.flatten, second, second.flatten):
             return None
         dtype = torch.get_autocast_dtype(x.device.type) if torch.is_autocast_enabled(x.device.type) else x.dtype
         w1, w2 = first.linear.weight, second.linear.weight
@@ -400,9 +409,8 @@ class LayerNorm(nn.Module):
         in one pass -- the bits that widening, normalising and rounding in three passes over twice
         the bytes give, in both directions.  Hooks see what ``forward`` makes."""
         y = None
-        if type(self) is LayerNorm and _gemm_route(x) and not (
-                self._forward_hooks or self._forward_pre_hooks or self._backward_hooks
-                or self._backward_pre_hooks or consumer._forward_pre_hooks):
+        if (type(self) is LayerNorm and type(self.norm) is nn.LayerNorm and _gemm_route(x)
+                and not _hooked(self, self.norm, consumer)):
             narrow = (x.dtype == torch.bfloat16 and torch.is_autocast_enabled(x.device.type)
                       and torch.get_autocast_dtype(x.device.type) == torch.bfloat16)
             y = self._hip(x if narrow else self._widened(x))

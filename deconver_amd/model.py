@@ -101,7 +101,7 @@ class DeconverBlock(nn.Module):
             return norm.with_skip(x)
         # (the channel norm's result is rounded as the projection that reads it would round it)
         if (type(norm) is LayerNorm and type(consumer) in (DeconvMixer, layers.MLP)
-                and type(projection) is Linear and not consumer._forward_pre_hooks):
+                and type(projection) is Linear and not layers._hooked(consumer)):
             return norm.for_projection(x, projection), x
         return norm(x), x
 

@@ -1,0 +1,67 @@
+"""Modules whose work runs inside another call on the GPU are called as modules where a hook watches them
+or their class is not the package's own."""
+
+import copy
+
+import pytest
+import torch
+from torch import nn
+
+import deconver_amd as dc
+from deconver_amd import layers
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(module, x, autocast):
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        y = module(x)
+    y.float().sum().backward()
+    return y
+
+
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("index", [0, 3])
+def test_hooks_on_the_projections_of_an_mlp_fire(index, autocast):
+    mlp = layers.MLP(64).cuda()
+    seen, width = [], 256 if index == 0 else 64
+    linear = mlp.block[index]
+    linear.register_forward_pre_hook(lambda m, a: seen.append("pre"))
+    linear.register_forward_hook(lambda m, a, out: seen.append(out.shape[1]))
+    linear.register_full_backward_hook(lambda m, gi, go: seen.append("back"))
+    _run(mlp, torch.rand(2, 64, 8, 64, device="cuda", requires_grad=True), autocast)
+    assert seen == ["pre", width, "back"]
+
+
+def test_hooks_on_all_modules_see_the_parts_of_a_block():
+    block = dc.DeconverBlock(8, kernel_size=(3, 3)).cuda()
+    seen = []
+    handle = nn.modules.module.register_module_forward_hook(lambda m, a, out: seen.append(m))
+    try:
+        _run(block, torch.rand(1, 8, 8, 8, device="cuda"), True)
+    finally:
+        handle.remove()
+    for module in (block.norm1, block.dcm.in_proj, block.norm2, block.mlp.block[0], block.mlp.block[3]):
+        assert any(m is module for m in seen), module
+
+
+def test_a_projection_of_another_class_is_called():
+    class Doubled(layers.Linear):
+        def forward(self, x, *args, **kwargs):
+            return 2 * super().forward(x, *args, **kwargs)
+
+    mlp = layers.MLP(8).cuda()
+    plain = copy.deepcopy(mlp)
+    second = Doubled(32, 8).cuda()
+    second.load_state_dict(mlp.block[3].state_dict())
+    mlp.block[3] = second
+    x = torch.rand(1, 8, 8, 8, device="cuda")
+    torch.testing.assert_close(mlp(x), 2 * plain(x), rtol=1e-5, atol=1e-5)   # one float32 chain, twice
+
+
+def test_a_hooked_norm_inside_the_layer_norm_is_called():
+    block = dc.DeconverBlock(8, kernel_size=(3, 3)).cuda()
+    seen = []
+    block.norm1.norm.register_forward_hook(lambda m, a, out: seen.append(out.shape))
+    _run(block, torch.rand(1, 8, 8, 8, device="cuda"), True)
+    assert seen == [(1, 8, 8, 8)]
