@@ -57,15 +57,15 @@ class DeconvMixer(nn.Module):
     def forward(self, x: Tensor, residual: Optional[Tensor] = None) -> Tensor:
         """The mixer's output, plus ``residual`` if given (the block's ``x + dcm(...)``, which
         then rides on ``out_proj`` unless dropout is active)."""
-        if type(self.act) is nn.ReLU and not self.act._forward_hooks and layers._gemm_route(x):
+        if type(self.act) is nn.ReLU and layers._gemm_route(x) and not layers._hooked(self.act, self.in_proj):
             # the rectifier rides on the projection (one kernel, or one pass over its output);
-            # a hooked activation module is still called as a module.  Its backward rides on the
+            # a hooked activation or projection is called as the module it is: what a hook sees and
+            # returns is then the projection's own output.  Its backward rides on the
             # layer's input gradient where the layer forms that in one GEMM; x stands in for
             # the projection's output when asking (same batch, grid, device and autocast state,
             # same channel count for the square in_proj of a block)
             premasked = (type(self.deconv) is Deconv and x.shape[1] == self.in_proj.linear.out_channels
-                         and not self.deconv._forward_hooks and not self.deconv._forward_pre_hooks
-                         and self.deconv.takes_rectified_input(x))
+                         and not layers._hooked(self.deconv) and self.deconv.takes_rectified_input(x))
             h = self.in_proj(x, act="relu", grad_premasked=premasked)
             sources = self.deconv(h, rectified_input=True) if premasked else self.deconv(h)
         else:

@@ -41,7 +41,7 @@ def test_hooks_on_all_modules_see_the_parts_of_a_block():
         _run(block, torch.rand(1, 8, 8, 8, device="cuda"), True)
     finally:
         handle.remove()
-    for module in (block.norm1, block.dcm.in_proj, block.norm2, block.mlp.block[0], block.mlp.block[3]):
+    for module in (block.norm1, block.dcm.in_proj, block.dcm.act, block.norm2, block.mlp.block[0], block.mlp.block[3]):
         assert any(m is module for m in seen), module
 
 
@@ -65,3 +65,30 @@ def test_a_hooked_norm_inside_the_layer_norm_is_called():
     block.norm1.norm.register_forward_hook(lambda m, a, out: seen.append(out.shape))
     _run(block, torch.rand(1, 8, 8, 8, device="cuda"), True)
     assert seen == [(1, 8, 8, 8)]
+
+
+def test_a_loss_on_the_hooked_projection_of_a_mixer_reaches_its_input():
+    """The hook sees the projection's own output, and gradients that reach it past the layer count:
+    input and weight gradients against the same mixer in float64 on the CPU."""
+    torch.manual_seed(0)
+    mixer = dc.DeconvMixer(64, 64, kernel_size=(3, 3, 3), ratio=4, groups=-1)
+    with torch.no_grad():
+        mixer.deconv.init.linear.linear.bias.add_(1.0)
+    ref = copy.deepcopy(mixer).double()
+    mixer = mixer.cuda()
+    x0, g0 = torch.randn(2, 64, 8, 8, 64), torch.randn(2, 64, 8, 8, 64)
+
+    def run(module, x, g):
+        kept = []
+        module.in_proj.register_forward_hook(lambda m, a, out: kept.append(out))
+        y = module(x)
+        (y * g).sum().add((kept[0].double() ** 2).sum()).backward()
+        return x.grad.double().cpu(), module.in_proj.linear.weight.grad.double().cpu()
+
+    x = x0.cuda().bfloat16().requires_grad_(True)
+    assert mixer.deconv.takes_rectified_input(x)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got = run(mixer, x, g0.cuda().bfloat16())
+    want = run(ref, x0.bfloat16().double().requires_grad_(True), g0.bfloat16().double())
+    for a, b in zip(got, want):     # (bfloat16 tensors along the way: as the mixer's other test)
+        assert torch.nn.functional.cosine_similarity(a.flatten(), b.flatten(), dim=0) > 0.998
