@@ -59,6 +59,9 @@ EXPORTS = (
     "ndc_pointwise_gemm_actgrad",
     "ndc_pointwise_gemm_masked",
     "ndc_gemm",
+    "ndc_gemm_parts",
+    "ndc_gemm_gelu_grad",
+    "ndc_column_sums",
     "ndc_weight_grad_workspace_bytes",
     "ndc_weight_grad",
 )
@@ -161,6 +164,10 @@ class NdcLibrary:
                                                  ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, vp]
         i64 = ctypes.c_int64
         d.ndc_gemm.argtypes = [vp, fp, ctypes.c_int, fp, vp, vp, vp, vp, i64, i64, i64, i64, ctypes.c_int, ctypes.c_int, vp]
+        d.ndc_gemm_parts.restype = i64
+        d.ndc_gemm_parts.argtypes = [i64, i64, i64, i64, ctypes.c_int]
+        d.ndc_gemm_gelu_grad.argtypes = [vp, fp, fp, vp, vp, fp, i64, i64, i64, i64, ctypes.c_int, vp]
+        d.ndc_column_sums.argtypes = [fp, fp, i64, i64, vp]
         d.ndc_weight_grad_workspace_bytes.restype = ctypes.c_size_t
         d.ndc_weight_grad_workspace_bytes.argtypes = [i64, i64, i64, i64, ctypes.c_int]
         d.ndc_weight_grad.argtypes = [vp, vp, fp, fp, i64, i64, i64, i64, ctypes.c_int, vp, ctypes.c_size_t, vp]
@@ -359,6 +366,19 @@ class NdcLibrary:
         """``y = epilogue(W x)`` on channel-first ``(batch, c, n)`` tensors of any size (see the header)."""
         self._check(self._dll.ndc_gemm(x, w, int(transposed), bias, residual, mask, y, zkeep, batch, cin, cout, n, mode,
                                        dtype, stream), "ndc_gemm")
+
+    def gemm_parts(self, batch: int, cin: int, cout: int, n: int, dtype: int) -> int:
+        return int(self._dll.ndc_gemm_parts(batch, cin, cout, n, dtype))
+
+    def gemm_gelu_grad(self, gy: int, w: int, bias: Optional[int], z: int, gz: int, gpart: Optional[int], batch: int, cin: int,
+                       cout: int, n: int, dtype: int, stream) -> None:
+        """``gz = (W gy) * gelu'(z + bias)`` with per-tile sums of ``gz`` in ``gpart``."""
+        self._check(self._dll.ndc_gemm_gelu_grad(gy, w, bias, z, gz, gpart, batch, cin, cout, n, dtype, stream),
+                    "ndc_gemm_gelu_grad")
+
+    def column_sums(self, partial: int, sums: int, rows: int, cols: int, stream) -> None:
+        """``sums[c] = sum_r partial[r][c]``, float32; ``partial`` is used as scratch."""
+        self._check(self._dll.ndc_column_sums(partial, sums, rows, cols, stream), "ndc_column_sums")
 
     def weight_grad_workspace_bytes(self, batch: int, rows: int, cols: int, n: int, dtype: int) -> int:
         return int(self._dll.ndc_weight_grad_workspace_bytes(batch, rows, cols, n, dtype))

@@ -709,9 +709,29 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
                                      [=] NDC_LAMBDA(int o, int s) { return part[s * stride + o]; });
 }
 
-int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, const void *residual, const void *mask,
-             void *y, void *zkeep, int64_t batch, int64_t cin, int64_t cout, int64_t n, int mode, int dtype,
-             void *stream)
+// How ndc_gemm cuts its work: wavefronts of a workgroup, each 32 output rows of a 128-voxel tile, or
+// one of the small-grid forms.
+// Small grids -- at most four workgroups of 32 rows x 64 voxels per CU -- take the form that
+// slices the channels over the wavefronts (waves <= 0): 128 -> 512 channels over 4096 voxels in
+// bf16 8.1 us against 10.2 tiled, over 32 768 (4096 workgroups) 24 against 11.5 --, at most one
+// per CU in tiles of 16 rows x 32 voxels (waves = -1; 288 of the larger tiles, 256 -> 64 channels
+// over 9152 voxels in float32, 10 us against 11.5 in the smaller).  Otherwise as
+// many output rows per workgroup (32 per wavefront) as still leave two workgroups per CU.
+static int gemm_waves(long long batch, long long cin, long long cout, long long n, int esz)
+{
+    const long long vt = batch * ((n + 127) / 128), small = batch * ((n + 63) / 64) * ((cout + 31) / 32);
+    if (small <= 1024 && cin % (16 / esz) == 0 && n >= 2) return small <= 256 ? -1 : 0;
+    int waves = 4;
+    while (waves > 1 && (cout <= 32 * (waves / 2) || vt * ((cout + 32 * waves - 1) / (32 * waves)) < 512)) waves /= 2;
+    return waves;
+}
+
+// voxels of a tile
+static int gemm_tile(int waves) { return waves > 0 ? 128 : waves ? 32 : 64; }
+
+static int gemm_impl(const void *x, const float *w, int transposed, const float *bias, const void *residual, const void *mask,
+                     void *y, void *zkeep, float *gpart, int64_t batch, int64_t cin, int64_t cout, int64_t n, int mode,
+                     int dtype, void *stream)
 {
     if (!x || !w || !y) return NDC_ERR_NULL;
     int st = gemm_check(batch, cin, cout, n, dtype);
@@ -723,22 +743,57 @@ int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, c
     if (zkeep && !act) return NDC_ERR_GEOMETRY;
     if ((act && transposed) || (grad && !transposed)) return NDC_ERR_GEOMETRY;   // forms no caller has
     const uintptr_t all = (uintptr_t)x | (uintptr_t)y | (uintptr_t)residual | (uintptr_t)mask | (uintptr_t)zkeep;
-    if (all & (uintptr_t)((dtype == NDC_BF16 ? 2 : 4) - 1) || ((uintptr_t)w & 3u) || ((uintptr_t)bias & 3u)) return NDC_ERR_WORKSPACE;
+    if (all & (uintptr_t)((dtype == NDC_BF16 ? 2 : 4) - 1) || ((uintptr_t)w & 3u) || ((uintptr_t)bias & 3u) || ((uintptr_t)gpart & 3u))
+        return NDC_ERR_WORKSPACE;
     if (y == x || zkeep == x || (zkeep && zkeep == y)) return NDC_ERR_GEOMETRY;
-    // Small grids -- at most four workgroups of 32 rows x 64 voxels per CU -- take the form that
-    // slices the channels over the wavefronts (waves <= 0): 128 -> 512 channels over 4096 voxels in
-    // bf16 8.1 us against 10.2 tiled, over 32 768 (4096 workgroups) 24 against 11.5 --, at most one
-    // per CU in tiles of 16 rows x 32 voxels (waves = -1; 288 of the larger tiles, 256 -> 64 channels
-    // over 9152 voxels in float32, 10 us against 11.5 in the smaller).  Otherwise as
-    // many output rows per workgroup (32 per wavefront) as still leave two workgroups per CU.
     const int esz = dtype == NDC_BF16 ? 2 : 4;
-    const long long vt = batch * ((n + 127) / 128), small = batch * ((n + 63) / 64) * ((cout + 31) / 32);
-    int waves = 4;
-    while (waves > 1 && (cout <= 32 * (waves / 2) || vt * ((cout + 32 * waves - 1) / (32 * waves)) < 512)) waves /= 2;
-    if (small <= 1024 && cin % (16 / esz) == 0 && n >= 2) waves = small <= 256 ? -1 : 0;
+    const long long vt = batch * ((n + 127) / 128);
     if ((vt + 8) * 2 * ((cout + 31) / 32 + 8) > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
-    return ndc::Backend::tile_gemm(x, w, transposed != 0, bias, residual, mask, y, zkeep, batch, (int)cin, (int)cout, n,
-                                   mode, esz, waves, stream);
+    return ndc::Backend::tile_gemm(x, w, transposed != 0, bias, residual, mask, y, zkeep, gpart, batch, (int)cin, (int)cout, n,
+                                   mode, esz, gemm_waves(batch, cin, cout, n, esz), stream);
+}
+
+int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, const void *residual, const void *mask,
+             void *y, void *zkeep, int64_t batch, int64_t cin, int64_t cout, int64_t n, int mode, int dtype,
+             void *stream)
+{
+    return gemm_impl(x, w, transposed, bias, residual, mask, y, zkeep, nullptr, batch, cin, cout, n, mode, dtype, stream);
+}
+
+int64_t ndc_gemm_parts(int64_t batch, int64_t cin, int64_t cout, int64_t n, int dtype)
+{
+    if (gemm_check(batch, cin, cout, n, dtype)) return 0;
+    const int tile = gemm_tile(gemm_waves(batch, cin, cout, n, dtype == NDC_BF16 ? 2 : 4));
+    return batch * ((n + tile - 1) / tile);
+}
+
+int ndc_gemm_gelu_grad(const void *gy, const float *w, const float *bias, const void *z, void *gz, float *gpart,
+                       int64_t batch, int64_t cin, int64_t cout, int64_t n, int dtype, void *stream)
+{
+    return gemm_impl(gy, w, 1, bias, z, nullptr, gz, nullptr, gpart, batch, cin, cout, n, NDC_GEMM_GELU_GRAD, dtype, stream);
+}
+
+// Many rows are folded to 256 first, in place (a row r < 256 receives rows r, r + 256, ... and is read
+// by its own sum only): one level over 4096 rows of 256 columns would be 8 workgroups of 64 round
+// trips to memory each.
+int ndc_column_sums(float *partial, float *sums, int64_t rows, int64_t cols, void *stream)
+{
+    if (!partial || !sums) return NDC_ERR_NULL;
+    if (rows < 1 || cols < 1 || cols > (1 << 22) || rows > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
+    if (rows > 512) {
+        const int nc = (int)cols, total = (int)rows;
+        const int st = ndc::Backend::strided_sum(
+            256 * nc, (total + 255) / 256, stream, [=] NDC_LAMBDA(int o, float v) { partial[o] = v; },
+            [=] NDC_LAMBDA(int o, int s) {
+                const int r = s * 256 + o / nc;
+                return r < total ? partial[(long long)r * nc + o % nc] : 0.f;
+            });
+        if (st) return st;
+        rows = 256;
+    }
+    const long long nc = cols;
+    return ndc::Backend::strided_sum((int)cols, (int)rows, stream, [=] NDC_LAMBDA(int o, float v) { sums[o] = v; },
+                                     [=] NDC_LAMBDA(int o, int s) { return partial[s * nc + o]; });
 }
 
 static int chnorm_check(long long B, long long C, long long n, int dtype)

@@ -665,10 +665,10 @@ struct Backend {
         return st ? st : check();
     }
     static int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res,
-                         const void *mask, void *y, void *zkeep, long long batch, int cin, int cout, long long n,
-                         int mode, int esz, int waves, void *stream)
+                         const void *mask, void *y, void *zkeep, float *gpart, long long batch, int cin, int cout,
+                         long long n, int mode, int esz, int waves, void *stream)
     {
-        const int st = gemm::tile_gemm(x, w, transposed, bias, res, mask, y, zkeep, batch, cin, cout, n, mode, esz, waves, stream);
+        const int st = gemm::tile_gemm(x, w, transposed, bias, res, mask, y, zkeep, gpart, batch, cin, cout, n, mode, esz, waves, stream);
         return st ? st : check();
     }
 

@@ -58,6 +58,22 @@ template <int ACT> __device__ inline float act_grad(float u)
     return 1.f;
 }
 
+// The sum of v over each half of the wavefront, in the half's last lane (31, 63): adds whose second
+// operand comes through the vector unit's own lane network (a butterfly of __shfl_xor goes through
+// the CU's one LDS unit instead).
+__device__ inline float half_sum(float v)
+{
+#define NDC_DPP_ADD(CTRL, ROWS)                                                                               \
+    v += __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, true))
+    NDC_DPP_ADD(0x111, 0xf);   // row_shr:1
+    NDC_DPP_ADD(0x112, 0xf);   // row_shr:2
+    NDC_DPP_ADD(0x114, 0xf);   // row_shr:4
+    NDC_DPP_ADD(0x118, 0xf);   // row_shr:8
+    NDC_DPP_ADD(0x142, 0xa);   // row_bcast:15 into rows 1 and 3
+#undef NDC_DPP_ADD
+    return v;
+}
+
 // out = f(a, b) element by element over one part of a row; returns the part's sum of out in
 // thread 0 when SUM
 template <typename T, bool TWO, bool VEC, bool SUM, class F>

@@ -267,6 +267,7 @@ struct TileParams {
                              // pre-activation whose derivative (at res + bias) multiplies the product
     const void *mask;        // (batch, cout, n) or null: y is zero where mask <= 0
     void *y, *zkeep;         // (batch, cout, n); zkeep or null: the product before bias and activation
+    float *gpart;            // kGeluGrad: (voxel tiles, cout) sums of y over a tile's voxels, or null
     long long n;
     int cin, cout, tiles_m, tiles_n, batch;
 };
@@ -341,9 +342,14 @@ template <typename T> __device__ inline void transpose(const Quad<T> (&in)[Gran<
 
 // The epilogue of NR consecutive rows of four voxels: z the products, `have` of the four voxels
 // exist (`whole`: all of them, in every lane).  What it reads is requested ahead of its stores.
+// sums (kGeluGrad): each row's sum over the voxels that exist, of the float32 values before they
+// are stored -- the bias gradient is these, and must not carry the rounding of what is stored.
 template <typename T, int MODE, int NR>
-__device__ inline void finish(const TileParams &p, const float (&z)[NR][4], int row0, long long base, int have, bool whole)
+__device__ inline void finish(const TileParams &p, const float (&z)[NR][4], int row0, long long base, int have, bool whole,
+                              float (&sums)[NR])
 {
+#pragma unroll
+    for (int e = 0; e < NR; ++e) sums[e] = 0.f;
     auto run = [&](auto tag) {
         constexpr bool WHOLE = decltype(tag)::value;
         Quad<T> rq[NR], mq[NR];
@@ -365,6 +371,7 @@ __device__ inline void finish(const TileParams &p, const float (&z)[NR][4], int 
             for (int j = 0; j < 4; ++j) {
                 if constexpr (MODE == kGeluGrad) {
                     y[j] = z[e][j] * epilogue::act_grad<epilogue::kGelu>(rq[e].get(j) + bias[e]);
+                    sums[e] += WHOLE || j < have ? y[j] : 0.f;
                 } else {
                     y[j] = epilogue::act_fwd<MODE>(z[e][j] + bias[e]);
                     if (p.res) y[j] += rq[e].get(j);
@@ -519,7 +526,8 @@ __global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
         }
     }
     const int have = left - 4 * l32;
-    if (have <= 0) return;
+    const bool summed = MODE == kGeluGrad && p.gpart != nullptr;   // (then every lane takes part below)
+    if (have <= 0 && !summed) return;
     const long long base = (long long)sample * p.cout * p.n + v0 + 4 * l32;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
@@ -528,7 +536,16 @@ __global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
         for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int j = 0; j < 4; ++j) z[e][j] = acc[j][4 * h + e];
-        finish<T, MODE, 4>(p, z, m0 + 32 * wave + 8 * h + 4 * kb, base, have, whole);
+        const int row0 = m0 + 32 * wave + 8 * h + 4 * kb;
+        float sums[4] = {0.f, 0.f, 0.f, 0.f};
+        if (have > 0) finish<T, MODE, 4>(p, z, row0, base, have, whole, sums);
+        if (summed) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float s = epilogue::half_sum(sums[e]);   // the 32 lanes of a row
+                if (l32 == 31 && row0 + e < p.cout) p.gpart[(long long)vt * p.cout + row0 + e] = s;
+            }
+        }
     }
 }
 
@@ -635,15 +652,26 @@ __global__ void __launch_bounds__(64 * kMaxSlices) sliced_kernel(TileParams p)
     for (int j = 0; j < R * R / 64; ++j)   // (a lane has runs of four rows, 4 KB rows apart)
         *reinterpret_cast<float2 *>(&part[wave][4 * KB * (j / 4) + 4 * kb + j % 4][2 * col]) = make_float2(acc0[j], acc1[j]);
     __syncthreads();
-    for (int t = tid; t < R * R / 2; t += blockDim.x) {
+    const bool summed = MODE == kGeluGrad && p.gpart != nullptr;
+    for (int t = tid; t < R * R / 2; t += blockDim.x) {   // (whole wavefronts: both counts are multiples of 64)
         const int row = t / (R / 2), q = t % (R / 2), have = left - 4 * q;
-        if (m0 + row >= p.cout || have <= 0) continue;
-        float z[1][4] = {{0.f, 0.f, 0.f, 0.f}};
-        for (int w = 0; w < slices; ++w) {
-            const float4 v = *reinterpret_cast<const float4 *>(&part[w][row][4 * q]);
-            z[0][0] += v.x, z[0][1] += v.y, z[0][2] += v.z, z[0][3] += v.w;
+        const bool mine = m0 + row < p.cout && have > 0;
+        if (!mine && !summed) continue;
+        float sums[1] = {0.f};
+        if (mine) {
+            float z[1][4] = {{0.f, 0.f, 0.f, 0.f}};
+            for (int w = 0; w < slices; ++w) {
+                const float4 v = *reinterpret_cast<const float4 *>(&part[w][row][4 * q]);
+                z[0][0] += v.x, z[0][1] += v.y, z[0][2] += v.z, z[0][3] += v.w;
+            }
+            finish<T, MODE, 1>(p, z, m0 + row, (long long)sample * p.cout * p.n + v0 + 4 * q, have, false, sums);
         }
-        finish<T, MODE, 1>(p, z, m0 + row, (long long)sample * p.cout * p.n + v0 + 4 * q, have, false);
+        if (summed) {
+            float s = sums[0];
+#pragma unroll
+            for (int o = 1; o < R / 2; o *= 2) s += __shfl_xor(s, o);   // the lanes of a row
+            if (q == 0 && m0 + row < p.cout) p.gpart[(long long)vt * p.cout + m0 + row] = s;
+        }
     }
 }
 

@@ -72,11 +72,11 @@ static int tile_gemm_t(const TileParams &p, int transposed, int mode, int waves,
     return 0;
 }
 int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res,
-                     const void *mask, void *y, void *zkeep, long long batch, int cin, int cout, long long n,
+                     const void *mask, void *y, void *zkeep, float *gpart, long long batch, int cin, int cout, long long n,
                      int mode, int esz, int waves, void *stream)
 {
     TileParams p;
-    p.x = x, p.w = w, p.bias = bias, p.res = res, p.mask = mask, p.y = y, p.zkeep = zkeep, p.n = n, p.cin = cin;
+    p.gpart = gpart, p.x = x, p.w = w, p.bias = bias, p.res = res, p.mask = mask, p.y = y, p.zkeep = zkeep, p.n = n, p.cin = cin;
     p.cout = cout, p.batch = (int)batch;
     return esz == 2 ? tile_gemm_t<bf16_t>(p, transposed, mode, waves, stream)
                     : tile_gemm_t<float>(p, transposed, mode, waves, stream);

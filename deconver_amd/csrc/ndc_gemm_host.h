@@ -17,7 +17,8 @@ namespace gemm {
 int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long long batch, int rows, int cols, long long n,
           int esz, const WgradPlan &plan, void *stream);
 int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res, const void *mask, void *y,
-              void *zkeep, long long batch, int cin, int cout, long long n, int mode, int esz, int waves, void *stream);
+              void *zkeep, float *gpart, long long batch, int cin, int cout, long long n, int mode, int esz, int waves,
+              void *stream);
 
 }  // namespace gemm
 }  // namespace ndc

@@ -387,8 +387,11 @@ struct Backend {
 
     template <typename T>
     static void tile_gemm_t(const T *x, const float *w, int transposed, const float *bias, const T *res, const T *mask, T *y,
-                            T *zkeep, long long batch, int cin, int cout, long long n, int mode)
+                            T *zkeep, float *gpart, long long batch, int cin, int cout, long long n, int mode, int tile)
     {
+        const long long tiles = (n + tile - 1) / tile;
+        if (gpart)
+            for (long long i = 0; i < batch * tiles * cout; ++i) gpart[i] = 0.f;
         for (long long b = 0; b < batch; ++b)
             for (int co = 0; co < cout; ++co)
                 for (long long v = 0; v < n; ++v) {
@@ -403,18 +406,21 @@ struct Backend {
                     float out = mode == 4 ? acc * act_value(2, rv + bv, true) : act_value(mode, acc + bv, false) + rv;
                     if (mask && !(Elem<T>::load(mask + at) > 0.f)) out = 0.f;
                     if (zkeep) Elem<T>::store(zkeep + at, acc);
+                    if (gpart) gpart[(b * tiles + v / tile) * cout + co] += out;
                     Elem<T>::store(y + at, out);
                 }
     }
     static int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res, const void *mask,
-                         void *y, void *zkeep, long long batch, int cin, int cout, long long n, int mode, int esz, int, void *)
+                         void *y, void *zkeep, float *gpart, long long batch, int cin, int cout, long long n, int mode, int esz,
+                         int waves, void *)
     {
+        const int tile = waves > 0 ? 128 : waves ? 32 : 64;   // voxels
         if (esz == 2)
             tile_gemm_t<bf16_t>((const bf16_t *)x, w, transposed, bias, (const bf16_t *)res, (const bf16_t *)mask, (bf16_t *)y,
-                                (bf16_t *)zkeep, batch, cin, cout, n, mode);
+                                (bf16_t *)zkeep, gpart, batch, cin, cout, n, mode, tile);
         else
             tile_gemm_t<float>((const float *)x, w, transposed, bias, (const float *)res, (const float *)mask, (float *)y,
-                               (float *)zkeep, batch, cin, cout, n, mode);
+                               (float *)zkeep, gpart, batch, cin, cout, n, mode, tile);
         return 0;
     }
 

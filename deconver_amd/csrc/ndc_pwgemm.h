@@ -245,10 +245,8 @@ __global__ void __launch_bounds__(THREADS) gemm_kernel(Params p)
                         y0 = z0 * epilogue::act_grad<A>(lo_bf16(rw[j]) + bq[jj]);
                         y1 = z1 * epilogue::act_grad<A>(hi_bf16(rw[j]) + bq[jj]);
                         if (p.gpart) {   // the channel's sum over the tile's 64 voxels: the 32 lanes of this half
-                            float t = y0 + y1;
-#pragma unroll
-                            for (int m = 1; m < 32; m <<= 1) t += __shfl_xor(t, m);
-                            if (n32 == 0) gs[32 * c + 8 * q + 4 * kb + jj] += t;
+                            const float t = epilogue::half_sum(y0 + y1);
+                            if (n32 == 31) gs[32 * c + 8 * q + 4 * kb + jj] += t;
                         }
                     } else if constexpr (ACT == kMasked) {
                         y0 = z0 + bq[jj], y1 = z1 + bq[jj];
@@ -267,7 +265,7 @@ __global__ void __launch_bounds__(THREADS) gemm_kernel(Params p)
         }
     }
     if constexpr (GRAD) {
-        // (only this wavefront touched its row; lanes 0 and 32 wrote it, all lanes read it)
+        // (only this wavefront touched its row; lanes 31 and 63 wrote it, all lanes read it)
         if (p.gpart) {
             __builtin_amdgcn_wave_barrier();
             const int g = (int)blockIdx.x * WAVES + wave;

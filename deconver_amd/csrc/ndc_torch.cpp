@@ -346,6 +346,26 @@ Tensor channel_sums(const Tensor &g, void *stream)
     return partial.sum(at::IntArrayRef{0, 2});
 }
 
+// sum over the rows of float32 partial results (rows, channels), which are overwritten
+Tensor column_sums(const Tensor &partial, void *stream)
+{
+    Tensor sums = empty_f32({partial.size(1)}, partial);
+    check(ndc_column_sums(out_fptr(partial), out_fptr(sums), partial.size(0), partial.size(1), stream), "ndc_column_sums");
+    return sums;
+}
+
+// gz = gy * act'(z + bias), and the bias gradient from the values before they are rounded to gz's
+// type (summing what is stored instead put a bf16 rounding into every term)
+void act_backward(const Tensor &gy, const Tensor &z, const Tensor &bias, const Tensor &gz, int act, Tensor *gb, void *stream)
+{
+    const int64_t B = gy.size(0), C = gy.size(1), n = gy.size(2);
+    Tensor partial;
+    if (gb) partial = empty_f32({B, C, ndc_bias_act_parts(B * C, n)}, gy);
+    check(ndc_bias_act_backward(ptr(gy), ptr(z), fptr(bias), out_ptr(gz), out_fptr(partial), B, C, n, act, dtype_tag(gy), stream),
+          "ndc_bias_act_backward");
+    if (gb) *gb = partial.sum(at::IntArrayRef{0, 2});
+}
+
 // Weight gradient sum_b gz[b] x[b]^T, (cout, cin) -- or (cin, cout) for a weight stored
 // transposed --, and the bias gradient, the sums of gz, from the same pass.  Rows beyond the
 // kernel's reach (2^24 voxels) are cut into chunks that become batch entries of a library GEMM.
@@ -746,12 +766,14 @@ struct Linear : public torch::autograd::Function<Linear> {
         Tensor gz = gy, gx, gw, gb;
         if (act != NDC_ACT_NONE && !cfg[3]) {
             gz = at::empty_like(gy);
-            check(ndc_bias_act_backward(ptr(gy), ptr(kept), fptr(bias), out_ptr(gz), nullptr, gy.size(0), gy.size(1), gy.size(2), act,
-                                        dtype_tag(gy), scope.stream), "ndc_bias_act_backward");
+            // (a rectifier's gradient, and float32, are stored as they are: their sums come with the weight's)
+            const bool rounded = act == NDC_ACT_GELU && gy.scalar_type() == at::kBFloat16;
+            act_backward(gy, kept, bias, gz, act, need[2] && rounded ? &gb : nullptr, scope.stream);
         }
+        Tensor *sums = need[2] && !gb.defined() ? &gb : nullptr;
         if (need[0]) gx = project_back(w, gz, Tensor(), Tensor(), scope.stream);
-        if (need[1]) gw = weight_grad(gz, x, w, v[1].sizes(), v[1].scalar_type(), need[2] ? &gb : nullptr, scope.stream);
-        else if (need[2]) gb = channel_sums(gz, scope.stream);
+        if (need[1]) gw = weight_grad(gz, x, w, v[1].sizes(), v[1].scalar_type(), sums, scope.stream);
+        else if (sums) gb = channel_sums(gz, scope.stream);
         if (gb.defined()) gb = gb.to((at::ScalarType)cfg[5]);
         return once({gx, gw, gb, Tensor(), need[3] ? gy : Tensor(), Tensor(), Tensor()}, recording, gouts);
     }
@@ -819,21 +841,30 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type(), need[4] ? &gb2 : nullptr, scope.stream);
         else if (need[4]) gb2 = channel_sums(gy, scope.stream);
         if (need[0] || need[1] || need[2]) {
+            // bf16: the first bias's gradient is summed in the kernels that make gz, before they round
+            // it (what they store carries a rounding in every term); float32: with the weight's
             Tensor gz = at::empty_like(z);
+            const bool rounded = need[2] && gy.scalar_type() == at::kBFloat16;
             const Gemm by = choose_gemm(gy, hidden, true, true);
+            Tensor partial;
             if (by == kStream) {
                 Tensor frag = pack(w2, true, gy, scope.stream);
-                check(ndc_pointwise_gemm_actgrad(ptr(gy), ptr(frag), fptr(b1), ptr(z), out_ptr(gz), nullptr, B, w2.cout(), hidden, nv,
-                                                 NDC_ACT_GELU, NDC_BF16, scope.stream), "ndc_pointwise_gemm_actgrad");
+                if (rounded) partial = empty_f32({ndc_pointwise_gemm_parts(), hidden}, gy);
+                check(ndc_pointwise_gemm_actgrad(ptr(gy), ptr(frag), fptr(b1), ptr(z), out_ptr(gz), out_fptr(partial), B, w2.cout(),
+                                                 hidden, nv, NDC_ACT_GELU, NDC_BF16, scope.stream), "ndc_pointwise_gemm_actgrad");
             } else if (by == kTiled) {
-                tiled(w2, true, gy, b1, z, Tensor(), gz, Tensor(), NDC_GEMM_GELU_GRAD, scope.stream);
+                const Tensor m = w2.m.to(at::kFloat);
+                if (rounded) partial = empty_f32({ndc_gemm_parts(B, w2.cout(), hidden, nv, dtype_tag(gy)), hidden}, gy);
+                check(ndc_gemm_gelu_grad(ptr(gy), fptr(m), fptr(b1), ptr(z), out_ptr(gz), out_fptr(partial), B, w2.cout(), hidden, nv,
+                                         dtype_tag(gy), scope.stream), "ndc_gemm_gelu_grad");
             } else {
                 Tensor ga = project_back(w2, gy, Tensor(), Tensor(), scope.stream);
-                check(ndc_bias_act_backward(ptr(ga), ptr(z), fptr(b1), out_ptr(gz), nullptr, B, hidden, nv, NDC_ACT_GELU, dtype_tag(gy),
-                                            scope.stream), "ndc_bias_act_backward");
+                act_backward(ga, z, b1, gz, NDC_ACT_GELU, rounded ? &gb1 : nullptr, scope.stream);
             }
-            if (need[1]) gw1 = weight_grad(gz, x, w1, v[3].sizes(), v[3].scalar_type(), need[2] ? &gb1 : nullptr, scope.stream);
-            else if (need[2]) gb1 = channel_sums(gz, scope.stream);
+            if (partial.defined()) gb1 = column_sums(partial, scope.stream);
+            Tensor *sums = need[2] && !gb1.defined() ? &gb1 : nullptr;
+            if (need[1]) gw1 = weight_grad(gz, x, w1, v[3].sizes(), v[3].scalar_type(), sums, scope.stream);
+            else if (sums) gb1 = channel_sums(gz, scope.stream);
             if (need[0]) gx = project_back(w1, gz, Tensor(), Tensor(), scope.stream);
         }
         if (gb1.defined()) gb1 = gb1.to((at::ScalarType)cfg[3]);

@@ -384,6 +384,35 @@ def gemm(lib: _lib.NdcLibrary, x: Tensor, w: Tensor, bias: Optional[Tensor] = No
     return y, z
 
 
+def column_sums(lib: _lib.NdcLibrary, partial: Tensor) -> Tensor:
+    """Sum of a contiguous float32 ``(rows, cols)`` matrix over its rows; ``partial`` is overwritten."""
+    if partial.dim() != 2 or partial.dtype != torch.float32 or not partial.is_contiguous():
+        raise ValueError("column_sums wants a contiguous float32 matrix")
+    sums = torch.empty(partial.shape[1], dtype=torch.float32, device=partial.device)
+    lib.column_sums(_ptr(partial), _ptr(sums), partial.shape[0], partial.shape[1], _stream_of(partial))
+    return sums
+
+
+def gemm_gelu_grad(lib: _lib.NdcLibrary, gy: Tensor, w: Tensor, z: Tensor, bias: Optional[Tensor] = None):
+    """``(gz, gbias)`` with ``gz = (W gy) * gelu'(z + bias)`` for contiguous ``gy`` (B, cin, n), ``w`` the float32
+    (cin, cout) storage of W and ``z`` (B, cout, n), and ``gbias`` the sum of ``gz`` over batch and voxels
+    before it is rounded to its storage, float32."""
+    if gy.dim() != 3 or not gy.is_contiguous() or w.dim() != 2 or not w.is_contiguous() or w.dtype != torch.float32:
+        raise ValueError("gemm_gelu_grad wants a contiguous (B, cin, n) tensor and a contiguous float32 matrix")
+    B, cin, n = gy.shape
+    cout = w.shape[1]
+    if w.shape[0] != cin:
+        raise ValueError("the matrix does not belong to this tensor")
+    if z.shape != (B, cout, n) or z.dtype != gy.dtype or not z.is_contiguous():
+        raise ValueError("z must be contiguous, of the output's shape and dtype")
+    if bias is not None and (bias.dtype != torch.float32 or bias.numel() != cout or not bias.is_contiguous()):
+        raise ValueError("bias must be float32 with one entry per output channel")
+    gz, dtype = torch.empty_like(z), dtype_tag(gy.dtype)
+    gpart = torch.empty(lib.gemm_parts(B, cin, cout, n, dtype), cout, dtype=torch.float32, device=gy.device)
+    lib.gemm_gelu_grad(_ptr(gy), _ptr(w), _ptr(bias), _ptr(z), _ptr(gz), _ptr(gpart), B, cin, cout, n, dtype, _stream_of(gy))
+    return gz, column_sums(lib, gpart)
+
+
 def weight_grad(lib: _lib.NdcLibrary, gz: Tensor, x: Tensor, need_bias_grad: bool = False):
     """``(sum_b gz[b] x[b]^T, row sums of gz or None)``, float32, for contiguous (B, rows, n) and
     (B, cols, n) tensors of one dtype."""

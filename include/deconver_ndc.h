@@ -438,6 +438,24 @@ int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, c
              int mode, int dtype, void *stream);
 
 /*
+ * The NDC_GEMM_GELU_GRAD form with the gradient of `bias`: gz = (W gy) * gelu'(z + bias) for w the
+ * (cin, cout) storage of W, and, if gpart is not NULL, gpart[t][c] = the sum of gz over voxel tile t,
+ * float32 and taken before gz is rounded to its storage: ndc_gemm_parts(...) * cout floats, every one
+ * written.  The gradient of `bias` is the sum over the tiles (ndc_column_sums).
+ */
+int64_t ndc_gemm_parts(int64_t batch, int64_t cin, int64_t cout, int64_t n, int dtype);
+int ndc_gemm_gelu_grad(const void *gy, const float *w, const float *bias, const void *z, void *gz,
+                       float *gpart, int64_t batch, int64_t cin, int64_t cout, int64_t n, int dtype,
+                       void *stream);
+
+/*
+ * sums[c] = sum over r of partial[r][c] for a float32 (rows, cols) matrix, in a fixed order: the last
+ * step of a bias gradient from the gpart of ndc_gemm_gelu_grad or ndc_pointwise_gemm_actgrad.
+ * `partial` is used as scratch.
+ */
+int ndc_column_sums(float *partial, float *sums, int64_t rows, int64_t cols, void *stream);
+
+/*
  * Weight gradient of a 1x1 projection and the sums its bias gradient is, in one pass:
  *     gw = sum_b gz[b] x[b]^T  (rows, cols) float32,   gb = sum_{b,v} gz[b][.][v]  (rows) or null
  * for gz (batch, rows, n) and x (batch, cols, n), float32 or bfloat16.  The voxel axis is split over

@@ -66,6 +66,34 @@ def test_weight_and_bias_gradient(device, shape, dtype, tol):
     assert torch.equal(again, gw) and none is None
 
 
+# voxel tiles of 128 (the last two for a ragged depth and a last tile of one voxel), 64 and 32
+@pytest.mark.parametrize("dtype,tol", DTYPES)
+@pytest.mark.parametrize("shape", SHAPES + [(1, 64, 256, 4099), (2, 64, 96, 30001), (3, 30, 120, 257)])
+@pytest.mark.parametrize("device", DEVICES)
+def test_gelu_gradient_with_its_sums(device, shape, dtype, tol):
+    """The sums are of the float32 values: a rounding to bfloat16 in their terms would show as 1e-3."""
+    if device == "cpu" and shape[3] > 5000:
+        pytest.skip("the host build's loops")
+    lib, (x, res, _, _), w, bias = _setup(device, shape, dtype)
+    z = torch.matmul(w.to(dtype).double(), x.double())
+    v = (res.double() + bias.double()[:, None]).requires_grad_(True)
+    F.gelu(v).sum().backward()
+    gz, gb = ops.gemm_gelu_grad(lib, x, w.t().contiguous(), res, bias)
+    want = z * v.grad
+    assert _rel(gz, want) < tol
+    # per term: the product's float32 sums and the derivative's 3e-7; over the terms as their norm grows
+    assert float((gb.double() - want.sum((0, 2))).abs().max()) < 4e-6 * float(want.norm(dim=(0, 2)).max()) + 1e-6
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (7, 33), (512, 5), (513, 40), (4096, 96)])
+@pytest.mark.parametrize("device", DEVICES)
+def test_column_sums(device, rows, cols):
+    lib = hostcheck_library() if device == "cpu" else _lib.get_library()
+    part = torch.randn(rows, cols, generator=torch.Generator().manual_seed(rows)).to(device)
+    want = part.double().sum(0)
+    assert float((ops.column_sums(lib, part) - want).abs().max()) < 2e-6 * max(1.0, rows ** 0.5)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols", [(256, 64), (64, 54)])
 def test_weight_gradient_over_long_rows(rows, cols):

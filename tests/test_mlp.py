@@ -5,7 +5,7 @@ import copy
 import pytest
 import torch
 
-from deconver_amd.layers import MLP
+from deconver_amd.layers import MLP, pointwise_linear
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +32,49 @@ def test_output_of_another_width(out_channels, with_residual, dtype, tol):
     for a, b in pairs:
         a, b = a.detach().double().cpu(), b.detach()
         assert float((a - b).norm() / b.norm()) < tol
+
+
+def _bias_grad_reference(z, b, gz):
+    """float64 sums of gz * gelu'(z + b), each row over batch and voxels, and their terms' norms."""
+    u = (z.double() + b.double()[:, None]).requires_grad_(True)
+    torch.nn.functional.gelu(u).backward(gz.double())
+    return u.grad.sum((0, 2)), u.grad.norm(dim=(0, 2))
+
+
+# by what makes the gradient of the hidden tensor: the streaming GEMM; the tiled one, its channels sliced over the
+# wavefronts (both tile sizes), in whole and in ragged tiles; the library's and a pass
+ROUTES = [(2, 64, 256, 65536), (1, 64, 256, 1000), (1, 64, 256, 4099), (1, 64, 256, 20001), (2, 30, 120, 777),
+          (1, 256, 1024, 8192)]
+
+
+@pytest.mark.parametrize("B,c,hidden,n", ROUTES)
+def test_bias_gradient_behind_the_gelu_is_not_rounded(B, c, hidden, n):
+    """bfloat16, with weights that pick one channel each, so that the hidden tensor and its gradient's
+    product are exact: what is left is the activation's derivative (3e-7) and float32 sums.  Terms
+    rounded to bfloat16 would put 1e-3 of their norm into the result."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")   # noqa: E731
+    mlp = MLP(c, hidden_channels=hidden).cuda()
+    first, second = mlp.block[0].linear, mlp.block[3].linear
+    unit = torch.arange(hidden, device="cuda")
+    with torch.no_grad():
+        first.weight.zero_()[unit, unit % c, 0] = 0.5
+        second.weight.zero_()[(unit * 7) % c, unit, 0] = 2.0
+    x, g = rand(B, c, n).bfloat16(), rand(B, c, n).bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = mlp(x.requires_grad_(True))
+    y.backward(g)
+    want, norm = _bias_grad_reference(0.5 * x.detach().float()[:, unit % c], first.bias.detach(), 2.0 * g.float()[:, (unit * 7) % c])
+    assert float(((first.bias.grad - want).abs() / norm).max()) < 2e-5
+
+
+def test_bias_gradient_of_a_projection_with_its_gelu_is_not_rounded():
+    torch.manual_seed(0)
+    x = torch.randn(2, 16, 4000, device="cuda").bfloat16()
+    w = torch.zeros(48, 16, device="cuda")
+    w[torch.arange(48), torch.arange(48) % 16] = 0.5
+    b = torch.randn(48, device="cuda", requires_grad=True)
+    g = torch.randn(2, 48, 4000, device="cuda").bfloat16()
+    pointwise_linear(x, w, b, act="gelu").backward(g)
+    want, norm = _bias_grad_reference(0.5 * x.float().repeat(1, 3, 1), b.detach(), g)
+    assert float(((b.grad - want).abs() / norm).max()) < 2e-5
