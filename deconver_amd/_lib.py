@@ -12,6 +12,8 @@ import os
 import threading
 from typing import Optional, Sequence
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdeconver_ndc.so")
 
@@ -454,4 +456,7 @@ def get_native():
             raise NdcError(f"{NATIVE_PATH} is missing: build it with `python -m deconver_amd.build`.")
         from . import _native as module
         _native = module
+    if torch._C._get_tracing_state() is not None:
+        from .tracing import RecordedNodes
+        return RecordedNodes(_native)
     return _native

@@ -194,7 +194,8 @@ def unfold_conv(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     k = tuple(weight.shape[2:])
     size = x.shape[2:]
     if (x.is_cuda and len(k) <= 3 and x.dtype in (torch.bfloat16, torch.float32) and x.numel() > 0
-            and math.prod(size) < 2 ** 31 and not (torch.is_grad_enabled() and x.requires_grad)):
+            and math.prod(size) < 2 ** 31 and not (torch.is_grad_enabled() and x.requires_grad)
+            and not torch.jit.is_tracing()):     # (what is traced runs on other inputs)
         cols = _lib.get_native().columns(x.contiguous(), list(k))
         return pointwise_linear(cols, weight, bias).view(x.shape[0], -1, *size)
     pad = []
