@@ -113,6 +113,18 @@ int64_t check_projection(const Tensor &x, int64_t channels, const Tensor &w, boo
     return cout;
 }
 
+// What comes back from a saved-tensor hook need not be what was saved: the tensor as the kernels read
+// it, or an error.
+Tensor check_saved(const Tensor &t, const Tensor &like, at::IntArrayRef size, at::ScalarType type)
+{
+    if (!t.defined()) return t;
+    check_device(t, like, "a saved tensor");
+    TORCH_CHECK_VALUE(t.scalar_type() == type && t.sizes() == size, "a saved tensor came back as ", t.scalar_type(), " ", t.sizes(),
+                      ", expected ", type, " ", size);
+    return t.contiguous();
+}
+Tensor check_saved(const Tensor &t, const Tensor &like) { return check_saved(t, like, like.sizes(), like.scalar_type()); }
+
 bool wants_grad(const Tensor &t) { return t.defined() && t.requires_grad(); }
 bool wants_grad(const OptTensor &t) { return t && wants_grad(*t); }
 
@@ -212,6 +224,16 @@ struct Matrix {
         return transpose != transposed ? w.t() : w;
     }
 };
+
+// the weight of a projection to `cout` channels as a backward finds it (see check_saved)
+Matrix saved_weight(const Tensor &w, bool transposed, int64_t cout, const Tensor &like)
+{
+    check_device(w, like, "a saved weight");
+    TORCH_CHECK_VALUE(w.dim() >= 2 && w.size(0) > 0, "a saved weight came back as ", w.sizes());
+    const Matrix m(w, transposed);
+    TORCH_CHECK_VALUE(m.cout() == cout, "a saved weight came back as ", w.sizes(), ", expected ", cout, " output channels");
+    return m;
+}
 
 // Which GEMM makes a 1x1 projection (or an input gradient), by what was measured on an MI355X:
 //   kStream   the streaming GEMM (ndc_pointwise_gemm): bf16 in its channel counts, from 2048 of its
@@ -468,6 +490,13 @@ Tensor prepare_taps(const ndc_geom &g, const Tensor &h, void *stream)
     return taps;
 }
 
+void check_taps(const Tensor &taps, const Tensor &x, const ndc_geom &g)
+{
+    if (!taps.defined()) return;
+    check_device(taps, x, "the filter table");
+    TORCH_CHECK_VALUE(taps.is_contiguous() && taps.nbytes() >= ndc_taps_bytes(&g), "the filter table is another geometry's");
+}
+
 struct UpdateForward {
     Tensor x, z, t1, h, s_over_den, ratio, taps;   // what the backward reads (h: contiguous)
     int path;
@@ -494,10 +523,7 @@ Tensor update_forward(Tensor x, Tensor z, const Tensor &h, const Tensor &bias, T
     f.path = g.path;
     // (kept only where the backward kernels of this geometry read them)
     const bool keep = grad && c.save_ratio && ndc_backward_uses_saved(&g);
-    if (taps.defined()) {
-        check_device(taps, x, "the filter table");
-        TORCH_CHECK_VALUE(taps.is_contiguous() && taps.nbytes() >= ndc_taps_bytes(&g), "the filter table is another geometry's");
-    }
+    check_taps(taps, x, g);
     // packed once here, used by the forward kernel and again by the backward's
     if (!taps.defined()) taps = prepare_taps(g, hc, stream);
     Tensor out = at::empty_like(z);
@@ -539,6 +565,8 @@ UpdateGrads update_backward(const UpdateForward &f, const Tensor &bias, Tensor g
                             bool need_z, bool need_h, bool need_b, void *stream)
 {
     const Tensor &x = f.x, &z = f.z;
+    check_update(x, z, f.h, bias, c);
+    const Tensor t1 = check_saved(f.t1, x), s_over_den = check_saved(f.s_over_den, z), ratio = check_saved(f.ratio, z);
     if (gout.scalar_type() != z.scalar_type()) gout = gout.to(z.scalar_type());
     gout = channel_first(gout, stream);
     TORCH_CHECK_VALUE(gout.sizes() == z.sizes(), "the gradient has shape ", gout.sizes(), ", expected ", z.sizes());
@@ -551,12 +579,13 @@ UpdateGrads update_backward(const UpdateForward &f, const Tensor &bias, Tensor g
     if (need_b) r.gb = empty_f32({c.groups * c.sc}, x);
     const size_t bytes = ndc_backward_workspace_bytes(&g, need_x, need_z, need_h, need_b);
     Tensor ws = scratch(bytes ? bytes : 1, x);
+    check_taps(f.taps, x, g);
     if (f.taps.defined())
-        check(ndc_backward_taps(&g, ptr(x), ptr(z), ptr(f.t1), ptr(f.s_over_den), ptr(f.ratio), fptr(f.h), ptr(f.taps),
+        check(ndc_backward_taps(&g, ptr(x), ptr(z), ptr(t1), ptr(s_over_den), ptr(ratio), fptr(f.h), ptr(f.taps),
                                 fptr(bias), ptr(gout), out_ptr(r.gx), out_ptr(r.gz), out_fptr(r.gh), out_fptr(r.gb),
                                 out_ptr(ws), bytes, stream), "ndc_backward_taps");
     else
-        check(ndc_backward(&g, ptr(x), ptr(z), ptr(f.t1), ptr(f.s_over_den), ptr(f.ratio), fptr(f.h), fptr(bias), ptr(gout),
+        check(ndc_backward(&g, ptr(x), ptr(z), ptr(t1), ptr(s_over_den), ptr(ratio), fptr(f.h), fptr(bias), ptr(gout),
                            out_ptr(r.gx), out_ptr(r.gz), out_fptr(r.gh), out_fptr(r.gb), out_ptr(ws), bytes, stream),
               "ndc_backward");
     return r;
@@ -671,7 +700,8 @@ struct Projected : public torch::autograd::Function<Projected> {
         UpdateGrads r =
             update_backward(f, v[4], gouts[0], c, need[0], need[0] || need[1], need[2], need[3], scope.stream);
         const Tensor x = f.x.flatten(2);
-        const Matrix w(v[8], false);
+        const Matrix w = saved_weight(v[8], false, f.z.size(1), x);
+        TORCH_CHECK_VALUE(w.cin() == x.size(1), "a saved weight came back as ", v[8].sizes());
         Tensor gw, gx;
         if (need[1]) gw = weight_grad(r.gz.flatten(2), x, w, v[8].sizes(), v[8].scalar_type(), nullptr, scope.stream);
         if (need[0]) {
@@ -756,13 +786,14 @@ struct Linear : public torch::autograd::Function<Linear> {
         const auto cfg = ctx->saved_data["cfg"].toIntVector();
         const int act = (int)cfg[0];
         const auto v = ctx->get_saved_variables();
-        const Tensor &x = v[0], &kept = v[2], &bias = v[3];
-        Scope scope(x);
-        const Matrix w(v[1], cfg[4] != 0);
+        const Tensor gy = gouts[0].contiguous();
+        Scope scope(gy);
+        const Matrix w = saved_weight(v[1], cfg[4] != 0, gy.size(1), gy);
+        const Tensor x = check_saved(v[0], gy, {gy.size(0), w.cin(), gy.size(2)}, gy.scalar_type());
+        const Tensor kept = check_saved(v[2], gy), bias = check_saved(v[3], gy, {w.cout()}, at::kFloat);
         Needs n;
         n.arg(true), n.arg(true), n.arg(cfg[1]), n.arg(cfg[2]);
         const auto need = n.ask(ctx);
-        const Tensor gy = gouts[0].contiguous();
         Tensor gz = gy, gx, gw, gb;
         if (act != NDC_ACT_NONE && !cfg[3]) {
             gz = at::empty_like(gy);
@@ -829,14 +860,16 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         at::NoGradGuard no_grad;
         const auto cfg = ctx->saved_data["cfg"].toIntVector();
         const auto v = ctx->get_saved_variables();
-        const Tensor &x = v[0], &z = v[1], &a = v[2], &b1 = v[5];
-        Scope scope(x);
-        const Matrix w1(v[3], false), w2(v[4], false);
+        const Tensor gy = gouts[0].contiguous();
+        Scope scope(gy);
+        const Matrix w2 = saved_weight(v[4], false, gy.size(1), gy), w1 = saved_weight(v[3], false, w2.cin(), gy);
+        const int64_t B = gy.size(0), nv = gy.size(2), hidden = w1.cout();
+        const Tensor x = check_saved(v[0], gy, {B, w1.cin(), nv}, gy.scalar_type());
+        const Tensor z = check_saved(v[1], gy, {B, hidden, nv}, gy.scalar_type()), a = check_saved(v[2], z);
+        const Tensor b1 = check_saved(v[5], gy, {hidden}, at::kFloat);
         Needs n;
         n.arg(true), n.arg(true), n.arg(cfg[0]), n.arg(true), n.arg(cfg[1]), n.arg(cfg[2]);
         const auto need = n.ask(ctx);
-        const Tensor gy = gouts[0].contiguous();
-        const int64_t B = x.size(0), nv = x.size(2), hidden = w1.cout();
         Tensor gx, gw1, gb1, gw2, gb2;
         if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type(), need[4] ? &gb2 : nullptr, scope.stream);
         else if (need[4]) gb2 = channel_sums(gy, scope.stream);
@@ -913,8 +946,9 @@ Tensor row_norm_forward(const Tensor &x, double eps, Tensor &stats, void *stream
     return y;
 }
 
-Tensor row_norm_backward(const Tensor &gy, const Tensor &y, const Tensor &stats, const Tensor &addend, void *stream)
+Tensor row_norm_backward(const Tensor &gy, const Tensor &saved_y, const Tensor &saved_stats, const Tensor &addend, void *stream)
 {
+    const Tensor y = check_saved(saved_y, gy), stats = check_saved(saved_stats, gy, {gy.size(0) * gy.size(1), 2}, at::kFloat);
     const int64_t rows = stats.size(0), n = voxels(y);
     Tensor gx = at::empty_like(y), ws = row_workspace(rows, n, y);
     check(ndc_rownorm_backward(ptr(gy), ptr(y), fptr(stats), ptr(addend), out_ptr(gx), rows, n, dtype_tag(y), out_ptr(ws),
@@ -935,7 +969,7 @@ struct RowNorm : public torch::autograd::Function<RowNorm> {
         const bool recording = at::GradMode::is_enabled();
         at::NoGradGuard no_grad;
         const auto v = ctx->get_saved_variables();
-        Scope scope(v[0]);
+        Scope scope(gouts[0]);
         return once({row_norm_backward(gouts[0].contiguous(), v[0], v[1], Tensor(), scope.stream), Tensor()}, recording, gouts);
     }
 };
@@ -961,9 +995,9 @@ struct RowNormSkip : public torch::autograd::Function<RowNormSkip> {
         at::NoGradGuard no_grad;
         const auto v = ctx->get_saved_variables();
         if (!gouts[0].defined()) return {gouts[1], Tensor()};
-        Scope scope(v[0]);
+        Scope scope(gouts[0]);
         Tensor skip = gouts[1];
-        if (skip.defined()) skip = skip.to(v[0].scalar_type()).contiguous();
+        if (skip.defined()) skip = skip.to(gouts[0].scalar_type()).contiguous();
         return once({row_norm_backward(gouts[0].contiguous(), v[0], v[1], skip, scope.stream), Tensor()}, recording, gouts);
     }
 };
@@ -1014,17 +1048,18 @@ struct ChannelNorm : public torch::autograd::Function<ChannelNorm> {
         at::NoGradGuard no_grad;
         const auto cfg = ctx->saved_data["cfg"].toIntVector();
         const auto v = ctx->get_saved_variables();
-        const Tensor &x = v[0];
-        Scope scope(x);
+        const Tensor gy = gouts[0].contiguous();
+        Scope scope(gy);
+        const int64_t B = gy.size(0), C = gy.size(1), n = gy.size(2);
+        const Tensor x = check_saved(v[0], gy), stats = check_saved(v[1], gy, {B, 2, n}, at::kFloat);
+        const Tensor weight = check_saved(v[2], gy, {C}, at::kFloat);
         Needs nd;
         nd.arg(true), nd.arg(cfg[0]), nd.arg(cfg[1]);
         const auto need = nd.ask(ctx);
-        const Tensor gy = gouts[0].to(x.scalar_type()).contiguous();
-        const int64_t B = x.size(0), C = x.size(1), n = x.size(2);
         Tensor gx = at::empty_like(x), partial, gw, gb;
         const bool affine = need[1] || need[2];
         if (affine) partial = empty_f32({ndc_chnorm_parts(B, n, dtype_tag(x)), C, 2}, x);
-        check(ndc_chnorm_backward(ptr(gy), ptr(x), fptr(v[1]), fptr(v[2]), out_ptr(gx), out_fptr(partial), B, C, n, dtype_tag(x),
+        check(ndc_chnorm_backward(ptr(gy), ptr(x), fptr(stats), fptr(weight), out_ptr(gx), out_fptr(partial), B, C, n, dtype_tag(x),
                                   scope.stream), "ndc_chnorm_backward");
         if (affine) {
             const Tensor sums = partial.sum(0);
