@@ -339,25 +339,6 @@ Tensor project_back(const Matrix &w, const Tensor &gz, Tensor accumulate, const 
     return gx;
 }
 
-// Equal chunks the voxel axis is cut into for the weight-gradient GEMM: a power of two that
-// divides n, chunks of at least `least` voxels, at most 128 GEMMs in the batch.
-int64_t weight_grad_chunks(int64_t batch, int64_t n, int64_t least)
-{
-    int64_t s = 1;
-    while (s < 64 && n % (2 * s) == 0 && n / (2 * s) >= least && batch * 2 * s <= 128) s *= 2;
-    return s;
-}
-
-// Chunk counts from timings with batch 2 in bfloat16 (64 chunks at 128^3; 32 at 64^3, where 64
-// cost 0.05 ms more on the 128 x 128 result; 16 at 32^3: 0.056 ms against 0.11-0.13 ms unchunked;
-// none at 16^3) and batch 8 in float32 (none up to 256^2 voxels: there every chunked form was
-// slower).
-int64_t weight_grad_plan(int64_t batch, int64_t n, bool half)
-{
-    if (half) return n < (1 << 15) ? 1 : weight_grad_chunks(batch, n, n < (1 << 17) ? 2048 : 8192);
-    return n < (1 << 17) ? 1 : weight_grad_chunks(batch, n, 2048);
-}
-
 // sum over batch and voxels, float32, one value per channel
 Tensor channel_sums(const Tensor &g, void *stream)
 {
@@ -388,37 +369,43 @@ void act_backward(const Tensor &gy, const Tensor &z, const Tensor &bias, const T
     if (gb) *gb = partial.sum(at::IntArrayRef{0, 2});
 }
 
+// ndc_weight_grad on tensors within its reach
+Tensor weight_grad_within(const Tensor &a, const Tensor &c, Tensor *sums, void *stream)
+{
+    const int64_t B = a.size(0), n = a.size(2), rows = a.size(1), cols = c.size(1);
+    Tensor gw = empty_f32({rows, cols}, a);
+    if (sums) *sums = empty_f32({rows}, a);
+    const int64_t bytes = (int64_t)ndc_weight_grad_workspace_bytes(B, rows, cols, n, dtype_tag(a));
+    Tensor ws = bytes ? at::empty({bytes}, a.options().dtype(at::kByte)) : Tensor();
+    check(ndc_weight_grad(ptr(a), ptr(c), out_fptr(gw), sums ? out_fptr(*sums) : nullptr, B, rows, cols, n, dtype_tag(a), out_ptr(ws),
+                          bytes, stream), "ndc_weight_grad");
+    return gw;
+}
+
 // Weight gradient sum_b gz[b] x[b]^T, (cout, cin) -- or (cin, cout) for a weight stored
-// transposed --, and the bias gradient, the sums of gz, from the same pass.  Rows beyond the
-// kernel's reach (2^24 voxels) are cut into chunks that become batch entries of a library GEMM.
+// transposed --, and the bias gradient, the sums of gz, from the same pass.  The kernel's lane offsets
+// reach 2^24 voxels; longer rows go through it slice by slice, copied (the slices of a row lie apart).
 Tensor weight_grad(const Tensor &gz, const Tensor &x, const Matrix &w, at::IntArrayRef shape, at::ScalarType dtype, Tensor *gb,
                    void *stream)
 {
     const Tensor &a = w.transposed ? x : gz, &c = w.transposed ? gz : x;
-    const int64_t B = a.size(0), n = a.size(2), rows = a.size(1), cols = c.size(1);
-    if (n <= (1 << 24)) {
-        const bool sums = gb && !w.transposed;
-        Tensor gw = empty_f32({rows, cols}, a);
-        if (sums) *gb = empty_f32({rows}, a);
-        const int64_t bytes = (int64_t)ndc_weight_grad_workspace_bytes(B, rows, cols, n, dtype_tag(a));
-        Tensor ws = bytes ? at::empty({bytes}, a.options().dtype(at::kByte)) : Tensor();
-        check(ndc_weight_grad(ptr(a), ptr(c), out_fptr(gw), sums ? out_fptr(*gb) : nullptr, B, rows, cols, n, dtype_tag(a),
-                              out_ptr(ws), bytes, stream), "ndc_weight_grad");
-        if (gb && !sums) *gb = channel_sums(gz, stream);
-        return gw.to(dtype).view(shape);
+    const int64_t n = a.size(2), most = int64_t(1) << 24;
+    Tensor gw, *sums = gb && !w.transposed ? gb : nullptr;
+    if (n <= most) {
+        gw = weight_grad_within(a, c, sums, stream);
+    } else {
+        const int64_t slices = (n + most - 1) / most, step = ((n + slices - 1) / slices + 127) / 128 * 128;
+        for (int64_t lo = 0; lo < n; lo += step) {
+            const int64_t len = std::min(step, n - lo);
+            Tensor part;
+            const Tensor g = weight_grad_within(a.narrow(2, lo, len).contiguous(), c.narrow(2, lo, len).contiguous(),
+                                                sums ? &part : nullptr, stream);
+            gw = lo ? gw.add_(g) : g;
+            if (sums) *sums = lo ? sums->add_(part) : part;
+        }
     }
-    if (gb) *gb = channel_sums(gz, stream);
-    const bool half = a.scalar_type() == at::kBFloat16;
-    const int64_t s = weight_grad_plan(B, n, half);
-    Tensor parts = empty_f32({B * s, rows, cols}, a);
-    for (int64_t b = 0; b < B; ++b) {
-        Tensor ab = a.select(0, b).view({rows, s, n / s}).transpose(0, 1);
-        Tensor cb = c.select(0, b).view({cols, s, n / s}).permute({1, 2, 0});
-        Tensor to = parts.narrow(0, b * s, s);
-        if (half) at::bmm_out(to, ab, cb, at::kFloat);
-        else at::bmm_out(to, ab, cb);
-    }
-    return parts.sum(at::IntArrayRef{0}, false, at::kFloat).to(dtype).view(shape);
+    if (gb && !sums) *gb = channel_sums(gz, stream);
+    return gw.to(dtype).view(shape);
 }
 
 // ---------------------------------------------------------------------------- the update
@@ -1200,6 +1187,4 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("channel_norm", &channel_norm);
     m.def("regroup", &regroup);
     m.def("columns", &columns);
-    m.def("weight_grad_chunks", &weight_grad_chunks);
-    m.def("weight_grad_plan", &weight_grad_plan);
 }

@@ -20,18 +20,6 @@ from torch.nn.modules.utils import _pair
 from . import _lib, ops
 
 
-def _wgrad_chunks(batch: int, n: int, min_chunk: int = 2048) -> int:
-    """Number of equal chunks the voxel axis is cut into for the weight-gradient GEMM: a power
-    of two that divides ``n``, leaves chunks of at least ``min_chunk`` voxels and at most 128
-    GEMMs in the batch."""
-    return _lib.get_native().weight_grad_chunks(batch, n, min_chunk)
-
-
-def _wgrad_plan(batch: int, n: int, dtype: torch.dtype) -> int:
-    """The chunk count of a projection's weight gradient (see ``csrc/ndc_torch.cpp``)."""
-    return _lib.get_native().weight_grad_plan(batch, n, dtype == torch.bfloat16)
-
-
 _ACT_TAGS = {None: _lib.ACT_NONE, "relu": _lib.ACT_RELU, "gelu": _lib.ACT_GELU}
 _ACT_FUNCTIONS = {None: lambda t: t, "relu": torch.relu, "gelu": torch.nn.functional.gelu}
 

@@ -5,7 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from deconver_amd.layers import Linear, _wgrad_chunks, _wgrad_plan, pointwise_linear
+from deconver_amd.layers import Linear, pointwise_linear
 
 pytestmark = pytest.mark.gpu
 
@@ -15,10 +15,10 @@ def _rel(a, ref):
 
 
 @pytest.mark.parametrize("B,cin,cout,n,bias", [
-    (2, 32, 128, 64 * 64 * 16, True),    # 16 chunks of the voxel axis in the weight gradient
-    (1, 128, 32, 32 * 32 * 32, False),   # 16 chunks
-    (3, 16, 64, 7 * 9 * 11, True),       # odd voxel count: one chunk
-    (2, 8, 8, 4096, True),               # two chunks
+    (2, 32, 128, 64 * 64 * 16, True),    # many splits of the voxel axis in the weight gradient
+    (1, 128, 32, 32 * 32 * 32, False),
+    (3, 16, 64, 7 * 9 * 11, True),       # odd voxel count
+    (2, 8, 8, 4096, True),
 ])
 def test_pointwise_linear_matches_conv1d(B, cin, cout, n, bias):
     g = torch.Generator().manual_seed(0)
@@ -44,14 +44,20 @@ def test_pointwise_linear_matches_conv1d(B, cin, cout, n, bias):
         assert b.grad.dtype == torch.float32 and _rel(b.grad, br.grad) < 1e-2
 
 
-def test_chunk_rule():
-    assert _wgrad_chunks(2, 64 ** 3) == 64 and _wgrad_chunks(2, 128 ** 3) == 64
-    assert _wgrad_chunks(2, 32 ** 3) == 16 and _wgrad_chunks(3, 7 * 9 * 11) == 1
-    assert _wgrad_chunks(8, 256 * 256) == 16 and _wgrad_chunks(1, 2048) == 1
-    bf16, f32 = torch.bfloat16, torch.float32
-    assert [_wgrad_plan(2, s ** 3, bf16) for s in (16, 32, 64, 128)] == [1, 16, 32, 64]
-    assert [_wgrad_plan(8, s ** 2, f32) for s in (64, 128, 256, 512)] == [1, 1, 1, 16]
-    assert _wgrad_plan(2, 64 ** 3, f32) == 64 and _wgrad_plan(3, 7 * 9 * 11, bf16) == 1
+@pytest.mark.parametrize("dtype,transposed", [(torch.bfloat16, False), (torch.float32, False), (torch.bfloat16, True)])
+def test_rows_beyond_the_reach_of_the_weight_gradient_kernel(dtype, transposed):
+    """More than 2^24 voxels: two slices, the second one shorter and ragged."""
+    n = (1 << 24) + 1001
+    g = torch.Generator(device="cuda").manual_seed(1)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")   # noqa: E731
+    x, gy = rand(1, 4, n).to(dtype), rand(1, 6, n).to(dtype)
+    w = rand(*((4, 6) if transposed else (6, 4))).requires_grad_(True)
+    b = rand(6).requires_grad_(True)
+    pointwise_linear(x, w, b, transposed=transposed).backward(gy)
+    want = gy[0].double() @ x[0].double().t()
+    # (random terms: their float32 sums against the norm of the terms, sqrt(n) of about 1)
+    assert float((w.grad - (want.t() if transposed else want)).abs().max()) < 4e-6 * n ** 0.5
+    assert float((b.grad - gy.double().sum((0, 2))).abs().max()) < 4e-6 * n ** 0.5
 
 
 def test_linear_module_under_autocast_keeps_float32_parameter_gradients():
