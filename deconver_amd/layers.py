@@ -291,22 +291,6 @@ class Linear(nn.Module):
         return y.view(shape[0], -1, *shape[2:])
 
 
-class _FusedMLP:
-    """``W2 gelu(W1 x + b1) + b2 + residual`` as ONE autograd node (layers/mlp.py:40-63 with the
-    block's sum, deconver.py:60-64), compiled in ``csrc/ndc_torch.cpp``: the hidden tensor's gradient
-    is written once and, where the library's own GEMMs make it, never read back by an activation
-    pass."""
-
-    @staticmethod
-    def applies(lib, x: torch.Tensor, hidden: int, cout: int) -> bool:
-        """Whether it takes ``x`` (B, C, n): bfloat16 or float32 on the GPU."""
-        return x.is_cuda and x.dim() == 3 and x.dtype in (torch.bfloat16, torch.float32)
-
-    @staticmethod
-    def apply(x, w1, b1, w2, b2, residual):
-        return _lib.get_native().mlp(x, w1, b1, w2, b2, residual)
-
-
 class MLP(nn.Module):
     """Linear - GELU - Linear on channels, with dropout after each (layers/mlp.py:40-63)."""
 
@@ -339,9 +323,10 @@ class MLP(nn.Module):
 
     @staticmethod
     def _fused(first: "Linear", second: "Linear", x: torch.Tensor, residual: Optional[torch.Tensor]):
-        """The block as one node for bfloat16 (stored or under autocast) and float32 tensors on the
-        GPU, else None: also where the projections are hooked or of a class of their own, which are
-        called as modules."""
+        """The block as one compiled node (the hidden tensor's gradient is written once and, where the
+        library's own GEMMs make it, never read back by an activation pass) for bfloat16 (stored or
+        under autocast) and float32 tensors on the GPU, else None: also where the projections are
+        hooked or of a class of their own, which are called as modules."""
         if not _gemm_route(x) or type(first) is not Linear or type(second) is not Linear or _hooked(
                 first, first.flatten, second, second.flatten):
             return None
@@ -350,10 +335,8 @@ class MLP(nn.Module):
         flat = x.flatten(2)
         if flat.dtype != dtype:
             flat = flat.to(dtype)
-        if not _FusedMLP.applies(None, flat, w1.shape[0], w2.shape[0]):
-            return None
-        y = _FusedMLP.apply(flat, w1, first.linear.bias, w2, second.linear.bias,
-                            None if residual is None else residual.flatten(2))
+        y = _lib.get_native().mlp(flat, w1, first.linear.bias, w2, second.linear.bias,
+                                  None if residual is None else residual.flatten(2))
         return y.view(x.shape[0], w2.shape[0], *x.shape[2:])
 
 

@@ -178,7 +178,7 @@ def test_mlp_as_one_node_matches_float64(with_residual):
     """The 64 -> 256 -> 64 MLP of the network's first level under bf16 autocast: forward, input,
     residual and parameter gradients against the same module in float64 on the CPU."""
     import copy
-    from deconver_amd.layers import MLP, _FusedMLP
+    from deconver_amd.layers import MLP
     torch.manual_seed(6)
     mlp = MLP(64)
     ref = copy.deepcopy(mlp).double()
@@ -187,7 +187,6 @@ def test_mlp_as_one_node_matches_float64(with_residual):
     g0 = torch.randn(2, 64, 8, 8, 64)
     x = x0.cuda().bfloat16().requires_grad_(True)
     r = r0.cuda().bfloat16().requires_grad_(True) if with_residual else None
-    assert _FusedMLP.applies(_lib.get_library(), x.flatten(2), 256, 64)
     with torch.autocast("cuda", dtype=torch.bfloat16):
         y = mlp(x, residual=r)
     assert y.dtype == torch.bfloat16
