@@ -311,11 +311,13 @@ class MLP(nn.Module):
 
     def forward(self, x: torch.Tensor, residual: Optional[torch.Tensor] = None) -> torch.Tensor:
         """``block(x)``, plus ``residual`` if given.  With the exact GELU and no active dropout
-        the activation and the sum ride on the projections (``Linear.forward``)."""
+        the activation and the sum ride on the projections (``Linear.forward``); parts that are hooked
+        or of another class are called one by one."""
         first, act, drop1, second, drop2 = self.block
         idle = lambda d: d.p == 0 or not d.training   # noqa: E731
-        if (isinstance(first, Linear) and isinstance(second, Linear) and type(act) is nn.GELU
-                and act.approximate == "none" and idle(drop1) and idle(drop2)):
+        if (type(first) is Linear and type(second) is Linear and type(act) is nn.GELU
+                and act.approximate == "none" and idle(drop1) and idle(drop2)
+                and not _hooked(self.block, *self.block, first.flatten, second.flatten)):
             fused = self._fused(first, second, x, residual)
             return second(first(x, act="gelu"), residual=residual) if fused is None else fused
         y = self.block(x)
@@ -325,10 +327,8 @@ class MLP(nn.Module):
     def _fused(first: "Linear", second: "Linear", x: torch.Tensor, residual: Optional[torch.Tensor]):
         """The block as one compiled node (the hidden tensor's gradient is written once and, where the
         library's own GEMMs make it, never read back by an activation pass) for bfloat16 (stored or
-        under autocast) and float32 tensors on the GPU, else None: also where the projections are
-        hooked or of a class of their own, which are called as modules."""
-        if not _gemm_route(x) or type(first) is not Linear or type(second) is not Linear or _hooked(
-                first, first.flatten, second, second.flatten):
+        under autocast) and float32 tensors on the GPU, else None."""
+        if not _gemm_route(x):
             return None
         dtype = torch.get_autocast_dtype(x.device.type) if torch.is_autocast_enabled(x.device.type) else x.dtype
         w1, w2 = first.linear.weight, second.linear.weight

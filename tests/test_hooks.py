@@ -33,6 +33,21 @@ def test_hooks_on_the_projections_of_an_mlp_fire(index, autocast):
     assert seen == ["pre", width, "back"]
 
 
+def test_hooks_on_the_parts_of_an_mlp_see_their_own_results():
+    """The first projection's before the GELU, and the GELU's."""
+    mlp, seen = layers.MLP(64).cuda(), {}
+    for index in (0, 1, 4):
+        mlp.block[index].register_forward_hook(lambda m, a, out, index=index: seen.update({index: out}))
+    x = torch.randn(2, 64, 8, 64, device="cuda")
+    y = mlp(x)
+    first = mlp.block[0].linear
+    want = torch.nn.functional.conv1d(x.double().flatten(2), first.weight.detach().double(), first.bias.detach().double())
+    assert float((seen[0].detach().flatten(2) - want).norm() / want.norm()) < 1e-6      # float32 sums of 64 products
+    want = torch.nn.functional.gelu(want)
+    assert float((seen[1].detach().flatten(2) - want).norm() / want.norm()) < 1e-6
+    assert torch.equal(seen[4], y)
+
+
 def test_hooks_on_all_modules_see_the_parts_of_a_block():
     block = dc.DeconverBlock(8, kernel_size=(3, 3)).cuda()
     seen = []
@@ -41,7 +56,7 @@ def test_hooks_on_all_modules_see_the_parts_of_a_block():
         _run(block, torch.rand(1, 8, 8, 8, device="cuda"), True)
     finally:
         handle.remove()
-    for module in (block.norm1, block.dcm.in_proj, block.dcm.act, block.norm2, block.mlp.block[0], block.mlp.block[3]):
+    for module in (block.norm1, block.dcm.in_proj, block.dcm.act, block.norm2, *block.mlp.block):
         assert any(m is module for m in seen), module
 
 
