@@ -9,8 +9,8 @@
 // a training step on one 32^3 volume took 12.7 ms for 5.7 ms of kernels, one forward + backward
 // of a 32-channel 64^2 layer 0.48 ms for 0.15 ms of kernels.  The arithmetic stays behind the C
 // ABI of include/deconver_ndc.h; nothing here computes on tensors except through it, the
-// library GEMMs of shapes the streaming GEMM does not take, and a few float32 sums of partial
-// results.
+// library GEMMs that choose_gemm leaves, the rectifier of a filter, and a few float32 sums of
+// partial results.
 #include <torch/extension.h>
 
 #include <c10/core/DeviceGuard.h>
@@ -652,7 +652,9 @@ struct Projected : public torch::autograd::Function<Projected> {
         // (the GEMMs and the update read rows of voxels: any other layout is turned first)
         const Tensor x = channel_first(x_, stream);
         auto size = x.sizes().vec();
-        // (float32: the library's product, whose bits decide which source units are on)
+        // (float32: the library's product.  Its bits decide which source units are on, and Linear, which
+        // makes this product for the layer's general form, takes the same: the two agree bit for bit
+        // as long as both use one kernel, whichever it is)
         Tensor z = project(w, x.flatten(2), x.scalar_type() == at::kFloat, stream);
         size[1] = w.cout();
         Tensor out = update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
@@ -726,8 +728,7 @@ struct Linear : public torch::autograd::Function<Linear> {
     {
         const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
         const bool tail = bias.defined() || act != NDC_ACT_NONE || res.defined();
-        // (an activation's tile form reads W as rows; a bare float32 product is the library's, as in
-        // Projected: the two give the same bits)
+        // (an activation's tile form reads W as rows; a bare float32 product: as in Projected)
         const bool library = (w.transposed && act != NDC_ACT_NONE) || (!tail && x.scalar_type() == at::kFloat);
         const Gemm by = library ? kLibrary : choose_gemm(x, cout, act != NDC_ACT_NONE || keep, tail);
         Tensor y = empty({B, cout, n}, x);

@@ -31,13 +31,14 @@ def pointwise_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch
     ``weight`` of shape ``(Cout, Cin)`` or ``(Cout, *)`` with ``Cin`` elements per row (with
     ``transposed``: the ``(Cin, Cout)`` storage of it), optionally followed by an activation (``"relu"`` or ``"gelu"``, the exact one) and the sum with a tensor of the
     output's shape.  bfloat16 (stored or under autocast) and float32 tensors on the GPU run as
-    batched GEMMs on the channel-first layout plus one pass of the HIP library over the result;
-    everything else as the reference's ``conv1d`` followed by PyTorch's activation and sum.
+    GEMMs on the channel-first layout, with the tail in the epilogue of the HIP library's own GEMMs or
+    as one pass of it over a library GEMM's result (``choose_gemm`` in ``csrc/ndc_torch.cpp`` says
+    which); everything else as the reference's ``conv1d`` followed by PyTorch's activation and sum.
 
     ``grad_premasked`` (GEMM route, ``act="relu"`` without residual only; ignored elsewhere): the
     caller guarantees that every gradient reaching the result is already zero where the result
-    is -- its only consumer took it through the rectifier (``project_back(mask=...)``) --, so the
-    backward skips the rectifier's pass."""
+    is -- its only consumer took it through the rectifier (``Deconv.forward(rectified_input=True)``)
+    --, so the backward skips the rectifier's pass."""
     dtype = x.dtype
     if x.is_cuda and torch.is_autocast_enabled(x.device.type):
         dtype = torch.get_autocast_dtype(x.device.type)

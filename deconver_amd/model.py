@@ -18,7 +18,9 @@ tree, hence the same parameter names --
 
 Only the network the reference ships as ``Deconver`` is built here (Deconver stages at
 every level); the reference's generic convolutional U-Net blocks are not part of this path.
-Everything except the ``Deconv`` layers runs on PyTorch-ROCm library kernels.
+On the GPU the ``Deconv`` layers, the projections, norms and resampling convolutions run on the HIP
+library's kernels (``layers.py``, ``norm.py``); concatenation, plain sums and the largest bare
+products are PyTorch-ROCm's.
 """
 
 from __future__ import annotations

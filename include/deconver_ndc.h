@@ -322,8 +322,8 @@ int ndc_bias_act_backward(const void *gy, const void *z, const float *bias, void
  * one rounding of the result.
  *   ndc_pointwise_gemm_supported  1 where the kernel applies: NDC_BF16; cin 32, 64, 128 or 256, or a
  *                  larger multiple of 64 with cout <= 128; cout a multiple of 32;
- *                  cin * cout * 2 <= 128 KiB; n a multiple of 64; else 0 (callers then use a
- *                  library GEMM and ndc_bias_act)
+ *                  cin * cout * 2 <= 128 KiB; n a multiple of 64; else 0 (callers then use
+ *                  ndc_gemm, or a library GEMM and ndc_bias_act)
  *   ndc_pointwise_pack  writes W in the order the kernel reads it into wfrag
  *                  (ndc_pointwise_weight_bytes(cin, cout) bytes, 16-byte aligned): the 8 values
  *                  W[32 c + l % 32][16 s + 8 (l / 32) + 0..7], as bf16, at element
