@@ -259,11 +259,18 @@ class PatchConvTranspose3d(_PatchConvTransposeMixin, nn.ConvTranspose3d):
     pass
 
 
+_any_global_hook = nn.modules.module._has_any_global_hook
+
+
 def _hooked(*modules: nn.Module) -> bool:
     """Whether a hook watches a call of one of ``modules`` (or of every module): a caller that runs a
     module's work inside another call then calls the module instead."""
-    return nn.modules.module._has_any_global_hook() or any(
-        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+    if _any_global_hook():
+        return True
+    for m in modules:       # (a loop: twice as fast as any() over a generator, five times in a block's call)
+        if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            return True
+    return False
 
 
 class Linear(nn.Module):
@@ -314,14 +321,15 @@ class MLP(nn.Module):
         """``block(x)``, plus ``residual`` if given.  With the exact GELU and no active dropout
         the activation and the sum ride on the projections (``Linear.forward``); parts that are hooked
         or of another class are called one by one."""
-        first, act, drop1, second, drop2 = self.block
+        block = self.block
+        first, act, drop1, second, drop2 = block
         idle = lambda d: d.p == 0 or not d.training   # noqa: E731
         if (type(first) is Linear and type(second) is Linear and type(act) is nn.GELU
                 and act.approximate == "none" and idle(drop1) and idle(drop2)
-                and not _hooked(self.block, *self.block, first.flatten, second.flatten)):
+                and not _hooked(block, first, act, drop1, second, drop2)):
             fused = self._fused(first, second, x, residual)
             return second(first(x, act="gelu"), residual=residual) if fused is None else fused
-        y = self.block(x)
+        y = block(x)
         return y if residual is None else residual + y
 
     @staticmethod
@@ -375,15 +383,15 @@ class LayerNorm(nn.Module):
             y = self._hip(self._widened(x))
         return self.norm(x.movedim(1, -1)).movedim(-1, 1) if y is None else y
 
-    def for_projection(self, x: torch.Tensor, consumer: nn.Module) -> torch.Tensor:
-        """``forward(x)`` for a caller that hands it to the projection ``consumer``, which wants it
-        channel-first and, under bfloat16 autocast, rounded to bfloat16: the kernels at every size,
-        and bfloat16 values under bfloat16 autocast normalised (in float32 arithmetic) and rounded
-        in one pass -- the bits that widening, normalising and rounding in three passes over twice
-        the bytes give, in both directions.  Hooks see what ``forward`` makes."""
+    def for_projection(self, x: torch.Tensor, *consumers: nn.Module) -> torch.Tensor:
+        """``forward(x)`` for a caller that hands it to a projection (``consumers``: it, and the module
+        around it that is called), which wants it channel-first and, under bfloat16 autocast, rounded to
+        bfloat16: the kernels at every size, and bfloat16 values under bfloat16 autocast normalised (in
+        float32 arithmetic) and rounded in one pass -- the bits that widening, normalising and rounding
+        in three passes over twice the bytes give, in both directions.  Hooks see what ``forward`` makes."""
         y = None
         if (type(self) is LayerNorm and type(self.norm) is nn.LayerNorm and _gemm_route(x)
-                and not _hooked(self, self.norm, consumer)):
+                and not _hooked(self, self.norm, *consumers)):
             narrow = (x.dtype == torch.bfloat16 and torch.is_autocast_enabled(x.device.type)
                       and torch.get_autocast_dtype(x.device.type) == torch.bfloat16)
             y = self._hip(x if narrow else self._widened(x))

@@ -103,8 +103,8 @@ class DeconverBlock(nn.Module):
             return norm.with_skip(x)
         # (the channel norm's result is rounded as the projection that reads it would round it)
         if (type(norm) is LayerNorm and type(consumer) in (DeconvMixer, layers.MLP)
-                and type(projection) is Linear and not layers._hooked(consumer)):
-            return norm.for_projection(x, projection), x
+                and type(projection) is Linear):
+            return norm.for_projection(x, projection, consumer), x
         return norm(x), x
 
 
