@@ -39,7 +39,8 @@ struct Variant {
 struct Tuning {
     int rhf, rwf, rhb, rwb;      // forced register tiles (0: the table's order of preference)
     int threads_f, threads_b;    // workgroup sizes of the FMA kernels, forward / backward
-    int threads_f2, threads_b2;  // ... of the bf16 dot2 kernels
+    int threads_f2, threads_b2;  // ... of the bf16 dot2 kernels, and the other size tried by dot2_tile
+    int threads_f2_wide, threads_b2_narrow;
     int split, dot2;             // march segments on / bf16 dot2 kernels on
     int mfma;                    // bf16 matrix-instruction kernels on (where they cover the geometry)
 };
@@ -56,12 +57,13 @@ static inline const Tuning &tuning()
                              env_int("NDC_TUNE_RHB", 0),  env_int("NDC_TUNE_RWB", 0),
                              env_int("NDC_TUNE_NTF", 256), env_int("NDC_TUNE_NTB", 512),
                              env_int("NDC_TUNE_NTF2", 256), env_int("NDC_TUNE_NTB2", 256),
+                             env_int("NDC_TUNE_NTF2W", 512), env_int("NDC_TUNE_NTB2N", 128),
                              env_int("NDC_TUNE_SPLIT", 1), env_int("NDC_TUNE_DOT2", 1),
                              env_int("NDC_TUNE_MFMA", 1)};
     return t;
 }
 #else
-static inline Tuning tuning() { return Tuning{0, 0, 0, 0, 256, 512, 256, 256, 1, 1, 1}; }
+static inline Tuning tuning() { return Tuning{0, 0, 0, 0, 256, 512, 256, 256, 512, 128, 1, 1, 1}; }
 #endif
 
 // first listed row of this filter geometry that the width / alignment allow (and, in a
@@ -147,6 +149,66 @@ static inline void plan_lds(Plan &pl)
     ((pl).v.KD == kd_ && (pl).v.KH == kh_ && (pl).v.KW == kw_ && (pl).v.SC == sc_ &&            \
      (pl).v.RHF == rhf_ && (pl).v.RWF == rwf_ && (pl).v.RHB == rhb_ && (pl).v.RWB == rwb_)
 
+// What a launch of the bf16 dot2 kernels takes, up to a factor: the wavefronts a SIMD of the
+// busiest CU works through, times the planes a workgroup marches over.
+//   * R workgroups of a CU run at once (LDS and registers; a workgroup's wavefronts go round the
+//     four SIMDs, so six count as eight).  q resident ones take q ceil(w / 4) + 1: a SIMD with one
+//     wavefront waits for half of its time (the 1), with four hardly ever.
+//   * a segment of the march adds the planes its neighbours own (3 more than it keeps), a row band
+//     the two halo rows it computes twice (a fifth of a strip's work each).
+//   * `mixed`: from two full rounds on, workgroups of different rounds overlap and a remainder
+//     costs its share only (the forward, whose four wavefronts per SIMD drift apart).
+// Against the best of 56 launch shapes measured on each of 22 problems (16^3 .. 192^3, widths 14
+// to 192, 32 to 512 channels) the choice is 1 % behind on average and 11 % at worst; the fixed shape it
+// replaced (256 threads, the whole march) took 1.37 (forward) and 1.24 (backward) times as long on
+// average, 2.7 times on 64 channels of 32^3 (115 / 117 / 81 -> 42 / 50 / 34 us).
+static inline double dot2_cost(const Tile &t, const March &m, long long nbc, int lds_floats, int waves_per_simd,
+                               bool mixed)
+{
+    const int w = t.NT / 64;
+    int R = kMaxLdsBytes / (lds_floats * 4);
+    if (R > waves_per_simd * 4 / w) R = waves_per_simd * 4 / w;
+    if (R < 1) R = 1;
+    const double c = (double)(nbc * t.ntile * t.nseg) / 256.0, per = w > 3 ? (w + 3) / 4 : w / 4.0;
+    auto batch = [&](int q) { return q * per + 1.0; };
+    const long long ci = (nbc * t.ntile * t.nseg + 255) / 256;
+    const long long full = ci / R;
+    const int rem = (int)(ci - full * R);
+    double T = full * batch(R) + (rem ? batch(rem) : 0.0);
+    if (mixed && full >= 2) T = c * batch(R) / R + 0.5 * batch(R) / R;
+    const int planes = (t.SEG < m.D ? t.SEG : m.D) + (t.nseg > 1 ? 3 : 1);
+    return planes * (1.0 + 0.4 / t.S) * T;
+}
+
+// The row bands (workgroups of about `targets[i]` threads) and march segments (an even number of
+// planes, six at least) with the smallest cost.  K: the kernel whose LDS need counts.
+template <class K>
+static inline bool dot2_tile(const March &m, int RH, long long nbc, const int (&targets)[2], int min_strips,
+                             int waves_per_simd, bool mixed, Tile &best)
+{
+    static const int parts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
+    double least = 0.0;
+    bool found = false;
+    for (int target : targets) {
+        Tile t;
+        if (!make_tile(m, RH, 2, target, t, min_strips)) continue;
+        const int lds = K::lds_floats(t);
+        if (lds * 4 > kMaxLdsBytes) continue;
+        for (int n : parts) {
+            if (n > 1 && m.D < 6 * n) break;
+            t.SEG = n == 1 ? m.D : round_up((m.D + n - 1) / n, 2);
+            t.nseg = (m.D + t.SEG - 1) / t.SEG;
+            const double cost = dot2_cost(t, m, nbc, lds, waves_per_simd, mixed);
+            if (!found || cost < least) {
+                found = true;
+                least = cost;
+                best = t;
+            }
+        }
+    }
+    return found;
+}
+
 // pairs_ok: every activation pointer of the call is aligned to two elements
 static const int kDot2RH = 2;   // rows per thread of the bf16 dot2 kernels (columns: 2)
 
@@ -176,8 +238,17 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
         (long long)q.sc * q.SP * 2 < (1LL << 31) &&
         pl.m.KH == 3 && pl.m.KW == 3 && tn.dot2) {
         Tile tf, tb;
-        if (make_tile(pl.m, kDot2RH, 2, tn.threads_f2, tf, FwdKernelB<kDot2RH>::kMinStrips) &&
-            make_tile(pl.m, kDot2RH, 2, tn.threads_b2, tb)) {
+        const long long nbc = (long long)q.B * q.G;
+        const int targets_f[2] = {tn.threads_f2, tn.threads_f2_wide}, targets_b[2] = {tn.threads_b2_narrow, tn.threads_b2};
+        // (the matrix-instruction kernels march over whole volumes in one shape)
+        const bool whole = matrix && (FwdKernelM<kDot2RH>::covers(pl.m.W) || Bwd1KernelM<kDot2RH>::covers(pl.m.W) ||
+                                      Bwd2KernelM<kDot2RH>::covers(pl.m.W));
+        const bool fits = whole ? make_tile(pl.m, kDot2RH, 2, tn.threads_f2, tf, FwdKernelB<kDot2RH>::kMinStrips) &&
+                                      make_tile(pl.m, kDot2RH, 2, tn.threads_b2, tb)
+                                : dot2_tile<FwdKernelB<kDot2RH>>(pl.m, kDot2RH, nbc, targets_f,
+                                                                 FwdKernelB<kDot2RH>::kMinStrips, 4, true, tf) &&
+                                      dot2_tile<Bwd1KernelB<kDot2RH, true>>(pl.m, kDot2RH, nbc, targets_b, 0, 2, false, tb);
+        if (fits) {
             const int lf = FwdKernelB<kDot2RH>::lds_floats(tf);
             const int l1 = Bwd1KernelB<kDot2RH>::lds_floats(tb);
             const int l2 = Bwd2KernelB<kDot2RH>::lds_floats(tb);
@@ -243,7 +314,10 @@ static inline size_t backward_ws(const KGeom &q, int dtype, int /*need_gh*/, int
     Plan a, b;
     if (!make_plan(q, a, false, dtype)) return 0;
     const bool has_b = make_plan(q, b, true, dtype);
-    const size_t nblk = has_b && b.nblk_b > a.nblk_b ? b.nblk_b : a.nblk_b;
+    size_t nblk = has_b && b.nblk_b > a.nblk_b ? b.nblk_b : a.nblk_b;
+    // ... and whichever kernel family
+    Plan mx;
+    if (make_plan(q, mx, true, dtype, true) && (size_t)mx.nblk_b > nblk) nblk = mx.nblk_b;
     const size_t esz = dtype == NDC_BF16 ? 2 : 4;
     const size_t n_x = (size_t)q.B * q.G * q.SP;
     const size_t kt = (size_t)q.sc * q.KT;
@@ -273,14 +347,33 @@ template <class BE, typename T> struct Dot2Launch {
     static int bwd2(const BwdParams<T> &, const Plan &, void *, bool) { return NDC_ERR_GEOMETRY; }
 };
 template <class BE> struct Dot2Launch<BE, bf16_t> {
+    template <bool NT> static int fwd_dot2(const FwdParams<bf16_t> &p, const Plan &pl, void *stream)
+    {
+        if (p.s_over_den && p.ratio)
+            return BE::template block_kernel<FwdKernelB<kDot2RH, true, NT>>(p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);
+        return BE::template block_kernel<FwdKernelB<kDot2RH, false, NT>>(p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);
+    }
+    template <bool NT> static int bwd1_dot2(const BwdParams<bf16_t> &p, const Plan &pl, void *stream, bool saved)
+    {
+        typedef Bwd1KernelB<kDot2RH, true, NT> KS;
+        if (saved) return BE::template block_kernel<KS>(p, pl.nblk_b, pl.tb.NT, KS::lds_floats(pl.tb), stream);
+        return BE::template block_kernel<Bwd1KernelB<kDot2RH, false, NT>>(p, pl.nblk_b, pl.tb.NT, pl.lds_b1, stream);
+    }
+    template <bool NT> static int bwd2_dot2(const BwdParams<bf16_t> &p, const Plan &pl, void *stream, bool saved)
+    {
+        typedef Bwd2KernelB<kDot2RH, true, NT> KS;
+        if (saved) return BE::template block_kernel<KS>(p, pl.nblk_b, pl.tb.NT, KS::lds_floats(pl.tb), stream);
+        return BE::template block_kernel<Bwd2KernelB<kDot2RH, false, NT>>(p, pl.nblk_b, pl.tb.NT, pl.lds_b2, stream);
+    }
+    // (rows of whole 128-byte lines: see FwdKernelB)
+    static bool whole_lines(const Plan &pl) { return pl.m.W % 64 == 0; }
+
     static int fwd(const FwdParams<bf16_t> &p, const Plan &pl, void *stream)
     {
         if (pl.mfmaf)
             return BE::template block_kernel<FwdKernelM<kDot2RH>>(p, pl.nblk_f, pl.tf.NT,
                                                                    FwdKernelM<kDot2RH>::lds_floats(pl.tf), stream);
-        if (p.s_over_den && p.ratio)
-            return BE::template block_kernel<FwdKernelB<kDot2RH, true>>(p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);
-        return BE::template block_kernel<FwdKernelB<kDot2RH>>(p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);
+        return whole_lines(pl) ? fwd_dot2<true>(p, pl, stream) : fwd_dot2<false>(p, pl, stream);
     }
     // saved: the call brought the forward's s/d and n/d
     static int bwd1(const BwdParams<bf16_t> &p, const Plan &pl, void *stream, bool saved)
@@ -288,20 +381,14 @@ template <class BE> struct Dot2Launch<BE, bf16_t> {
         if (saved && pl.mfma1)
             return BE::template block_kernel<Bwd1KernelM<kDot2RH>>(
                 p, pl.nblk_b, pl.tb.NT, Bwd1KernelM<kDot2RH>::lds_floats(pl.tb), stream);
-        if (saved)
-            return BE::template block_kernel<Bwd1KernelB<kDot2RH, true>>(
-                p, pl.nblk_b, pl.tb.NT, Bwd1KernelB<kDot2RH, true>::lds_floats(pl.tb), stream);
-        return BE::template block_kernel<Bwd1KernelB<kDot2RH>>(p, pl.nblk_b, pl.tb.NT, pl.lds_b1, stream);
+        return whole_lines(pl) ? bwd1_dot2<true>(p, pl, stream, saved) : bwd1_dot2<false>(p, pl, stream, saved);
     }
     static int bwd2(const BwdParams<bf16_t> &p, const Plan &pl, void *stream, bool saved)
     {
         if (saved && pl.mfma2)
             return BE::template block_kernel<Bwd2KernelM<kDot2RH>>(
                 p, pl.nblk_b, pl.tb.NT, Bwd2KernelM<kDot2RH>::lds_floats(pl.tb), stream);
-        if (saved)
-            return BE::template block_kernel<Bwd2KernelB<kDot2RH, true>>(
-                p, pl.nblk_b, pl.tb.NT, Bwd2KernelB<kDot2RH, true>::lds_floats(pl.tb), stream);
-        return BE::template block_kernel<Bwd2KernelB<kDot2RH>>(p, pl.nblk_b, pl.tb.NT, pl.lds_b2, stream);
+        return whole_lines(pl) ? bwd2_dot2<true>(p, pl, stream, saved) : bwd2_dot2<false>(p, pl, stream, saved);
     }
 };
 

@@ -283,11 +283,17 @@ NDC_D void stream_rows(Exec &ex, Addr addr, Body body, const uint32_t (*first)[N
 
 // =================================================================== forward (bf16, dot2)
 
+// NT (here and in the backward kernels): tensors that are read or written once carry the
+// non-temporal hint.  It pays where an instruction moves whole 128-byte lines (rows of a multiple
+// of 64 columns); elsewhere neighbouring rows share a line, and a line that leaves the L2 between
+// their two accesses is moved twice: 2 x 128 channels of 56^3 900 / 620 / 459 us with the hint
+// (forward with both kept tensors, pass 1, pass 2), 559 / 549 / 385 without; 2 x 64 of 128^3
+// 2521 / 2536 / 1851 with, 2614 / 2494 / 2061 without.
 // KEEP: the call keeps s/d and n/d for backward (both tensors are there); without it the code
 // that forms and stores them is not compiled in (as a run-time condition it cost a branch per
 // row and channel, each reloading a spilled buffer resource).
-template <int RH_, bool KEEP_ = false> struct FwdKernelB {
-    static constexpr bool KEEP = KEEP_;
+template <int RH_, bool KEEP_ = false, bool NT_ = true> struct FwdKernelB {
+    static constexpr bool KEEP = KEEP_, NT = NT_;
     static constexpr int KD = 3, KH = 3, KW = 3, SC = 4, RH = RH_, RW = 2;
     static constexpr int PD = 1, PH = 1, PW = 1, KT = 27;
     // staging slots per thread: thread (strip, lane) stages rows strip, strip + S, ... of the
@@ -348,6 +354,8 @@ template <int RH_, bool KEEP_ = false> struct FwdKernelB {
         const bool have_t1 = p.t1 != nullptr;
         UniformF tab = as_uniform(p.wtab + (long long)id.c * kTabWords);
         const int r0 = id.r0;
+        // planes [d0, d1) are this workgroup's; t1 of plane d0 - 1 takes source planes from d0 - 2 on
+        const int d0 = id.d0, d1 = id.d1, k0 = d0 > 2 * PD ? d0 - 2 * PD : 0;
         const int nthreads = ex.nthreads;
         const float floor_ = p.relu ? 0.f : pass_through_floor();   // floor_f(s, floor_) rectifies or passes through
         const float eps = p.eps;
@@ -455,15 +463,15 @@ template <int RH_, bool KEEP_ = false> struct FwdKernelB {
                     for (int a = 0; a < KD; ++a) st.t1acc[a][r][c] = 0.f;
             }
             for (int i = tid; i < total; i += nthreads) ex.st_(i, 0.f);
-            load_plane(st, 0);
+            load_plane(st, k0);
         });
         ex.sync();
-        ex.each([&](State &st, int) NDC_LAMBDA { store_plane(st, 0); });
+        ex.each([&](State &st, int) NDC_LAMBDA { store_plane(st, k0); });
         ex.sync();
 
         // Two barriers per plane step: the source plane of the NEXT step is staged at the end of
         // the gather phase (nothing reads the source slot there), not in a phase of its own.
-        for (int kk = 0; kk < D + 2; ++kk) {
+        for (int kk = k0; kk < d1 + 2; ++kk) {
             const int k = uniform_int(kk);   // the plane index stays on the scalar unit
 
             // ---- K-scatter of source plane k; t1 plane k - 1
@@ -504,7 +512,7 @@ template <int RH_, bool KEEP_ = false> struct FwdKernelB {
                         ex.st_(off_qt + j * PQ + 1 + (st.ln.c0 >> 1), bits_to_float(vq));
                     }
                     st.t1prev[r] = vq;
-                    if (r < RH && have_t1 && live)
+                    if (r < RH && have_t1 && live && pf >= d0 && pf < d1)
                         buf_st(tb_, st.ooff[r < RH ? r : 0], (unsigned)pf * plane2, vq);
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) {
@@ -521,7 +529,7 @@ template <int RH_, bool KEEP_ = false> struct FwdKernelB {
                 if (!st.ln.active) return;
                 load_plane(st, k + 1);
                 const int j0 = k - 2;
-                if (j0 < 0) {
+                if (j0 < d0) {
                     store_plane(st, k + 1);
                     return;
                 }
@@ -568,10 +576,10 @@ template <int RH_, bool KEEP_ = false> struct FwdKernelB {
                             rt[c] = acc[0][i][r][c] * inv;
                             v[c] = s * rt[c];
                         }
-                        buf_st<true>(ob_, st.ooff[r], oj + i * cplane2, pack_bf16x2(v[0], v[1]));
+                        buf_st<NT>(ob_, st.ooff[r], oj + i * cplane2, pack_bf16x2(v[0], v[1]));
                         if (KEEP) {
-                            buf_st<true>(db_, st.ooff[r], oj + i * cplane2, pack_bf16x2(rd[0], rd[1]));
-                            buf_st<true>(rb_, st.ooff[r], oj + i * cplane2, pack_bf16x2(rt[0], rt[1]));
+                            buf_st<NT>(db_, st.ooff[r], oj + i * cplane2, pack_bf16x2(rd[0], rd[1]));
+                            buf_st<NT>(rb_, st.ooff[r], oj + i * cplane2, pack_bf16x2(rt[0], rt[1]));
                         }
                     }
                 }
@@ -587,8 +595,8 @@ template <int RH_, bool KEEP_ = false> struct FwdKernelB {
 // SAVED: the call brings the forward's s/d and n/d, so gn = g (s/d), gd = -gn (n/d) are
 // elementwise (z is not read) and the plane-pair rings of x and t1 (for re-gathering n and d)
 // are not kept.
-template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
-    static constexpr bool SAVED = SAVED_;
+template <int RH_, bool SAVED_ = false, bool NT_ = true> struct Bwd1KernelB {
+    static constexpr bool SAVED = SAVED_, NT = NT_;
     static constexpr int KD = 3, KH = 3, KW = 3, SC = 4, RH = RH_, RW = 2;
     static constexpr int PD = 1, PH = 1, PW = 1, KT = 27;
     static constexpr int NXR = RH + 2;
@@ -652,6 +660,11 @@ template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
         const bool have_gx = p.gx != nullptr;
         UniformF tab = as_uniform(p.wtab + (long long)id.c * kTabWords);
         const int r0 = id.r0;
+        // planes [d0, d1) are this workgroup's; their gx takes gn of the planes d0 - 1 .. d1, and a
+        // re-gathered gn (x, t1) one plane further
+        const int d0 = id.d0, d1 = id.d1;
+        const int jb = d0 > PD ? d0 - PD : 0;
+        const int k0 = SAVED || jb == 0 ? jb : jb - 1;
         const int nthreads = ex.nthreads;
         const float floor_ = p.relu ? 0.f : pass_through_floor();   // floor_f(s, floor_) rectifies or passes through
         const float eps = p.eps;
@@ -710,9 +723,9 @@ template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
                 const unsigned o = r < RH ? st.ooff[r < RH ? r : 0] : st.hoff;
                 NDC_UNROLL
                 for (int i = 0; i < SC; ++i) {
-                    st.qg[i][r] = buf_ld<true>(gb_, o, jo + i * cplane2);
-                    st.qd[i][r] = buf_ld<true>(db_, o, jo + i * cplane2);
-                    st.qr[i][r] = buf_ld<true>(rb_, o, jo + i * cplane2);
+                    st.qg[i][r] = buf_ld<NT>(gb_, o, jo + i * cplane2);
+                    st.qd[i][r] = buf_ld<NT>(db_, o, jo + i * cplane2);
+                    st.qr[i][r] = buf_ld<NT>(rb_, o, jo + i * cplane2);
                 }
             }
         };
@@ -840,19 +853,19 @@ template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) st.accx[a][r][c] = st.acct[a][r][c] = 0.f;
             for (int i = tid; i < total; i += nthreads) ex.st_(i, 0.f);
-            load_plane(st, 0);
+            load_plane(st, k0);
         });
         ex.sync();
-        ex.each([&](State &st, int) NDC_LAMBDA { store_plane(st, 0); });
+        ex.each([&](State &st, int) NDC_LAMBDA { store_plane(st, k0); });
         ex.sync();
 
         // Two barriers per plane step: the (x, t1) plane of the NEXT step is staged at the end
         // of the scatter phase (the ring slots it overwrites were last read in the phase before).
-        for (int kk = 0; kk < D + 2; ++kk) {
+        for (int kk = k0; kk < d1 + 2; ++kk) {
             const int k = uniform_int(kk);   // the plane index stays on the scalar unit
 
             const int j1 = k - 1;
-            const bool live1 = j1 >= 0 && j1 < D;
+            const bool live1 = j1 >= jb && j1 < D;
             ex.each([&](State &st, int) NDC_LAMBDA {
                 if (!st.ln.active || !live1) return;
                 {
@@ -868,7 +881,7 @@ template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
                     read_row<RW + 2>(ex, xt_row(0), row0);
                     ex.fence();
                     gn_gd_rows(st, j1, j, st.ob + (PW + PH * P), IntTag<RH>(), 0, gg2);
-                    if (need_gh) {
+                    if (need_gh && j1 >= d0 && j1 < d1) {
                         // A-side filter-gradient terms: (gn_i, gd_i) . (x, t1)[neighbour]
                         stream_rows<KD * (RH + 2), RW + 2, true>(
                             ex, xt_row,
@@ -931,8 +944,8 @@ template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
                 const int pf = k - 2;
                 NDC_UNROLL
                 for (int r = 0; r < RH; ++r) {
-                    if (pf >= 0) {   // rows outside the image: the stores go nowhere
-                        if (have_gx) buf_st<true>(gxb_, st.ooff[r], (unsigned)pf * plane2,
+                    if (pf >= d0) {   // rows outside the image: the stores go nowhere
+                        if (have_gx) buf_st<NT>(gxb_, st.ooff[r], (unsigned)pf * plane2,
                                             pack_bf16x2(st.accx[0][r][0], st.accx[0][r][1]));
                         buf_st(gtb_, st.ooff[r], (unsigned)pf * plane2,
                                pack_bf16x2(st.acct[0][r][0], st.acct[0][r][1]));
@@ -964,8 +977,8 @@ template <int RH_, bool SAVED_ = false> struct Bwd1KernelB {
 // =================================================================== backward pass 2 (bf16, dot2)
 
 // SAVED: gz = [s > 0] (g (n/d) + A(gt1)) with the forward's n/d, so only the gt1 ring is kept.
-template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
-    static constexpr bool SAVED = SAVED_;
+template <int RH_, bool SAVED_ = false, bool NT_ = true> struct Bwd2KernelB {
+    static constexpr bool SAVED = SAVED_, NT = NT_;
     static constexpr int NA = SAVED ? 1 : 3;   // gathered operands: (x, t1,) gt1
     static constexpr int KD = 3, KH = 3, KW = 3, SC = 4, RH = RH_, RW = 2;
     static constexpr int PD = 1, PH = 1, PW = 1, KT = 27;
@@ -1031,6 +1044,9 @@ template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
         const BufRef gzb_ = make_buf(p.gz ? p.gz + cbase * SC : nullptr, sbytes);
         UniformF tab = as_uniform(p.wtab + (long long)id.c * kTabWords);
         const int r0 = id.r0;
+        // planes [d0, d1) are this workgroup's (d0 even: the filter-gradient terms pair planes);
+        // their gathers take gt1 of the planes d0 - 1 .. d1
+        const int d0 = id.d0, d1 = id.d1, k0 = d0 > 2 * PD ? d0 - 2 * PD : 0;
         const int nthreads = ex.nthreads;
         const float floor_ = p.relu ? 0.f : pass_through_floor();   // floor_f(s, floor_) rectifies or passes through
         const float eps = p.eps;
@@ -1114,7 +1130,7 @@ template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
                     for (int a = 0; a < 2; ++a) st.qz[a][i][r] = st.qg[a][i][r] = st.qr[a][i][r] = 0u;
             }
             for (int i = tid; i < total; i += nthreads) ex.st_(i, 0.f);
-            load_plane(st, 0);
+            load_plane(st, k0);
         });
         ex.sync();
 
@@ -1138,11 +1154,11 @@ template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
                             gw[i][r] = st.qg[PAR][i][r];
                             rw[i][r] = st.qr[PAR][i][r];
                             st.qz[1 - PAR][i][r] = buf_ld(zb_, st.ooff[r], jn + i * cplane2);
-                            st.qg[1 - PAR][i][r] = buf_ld<true>(gb_, st.ooff[r], jn + i * cplane2);
-                            st.qr[1 - PAR][i][r] = buf_ld<true>(rb_, st.ooff[r], jn + i * cplane2);
+                            st.qg[1 - PAR][i][r] = buf_ld<NT>(gb_, st.ooff[r], jn + i * cplane2);
+                            st.qr[1 - PAR][i][r] = buf_ld<NT>(rb_, st.ooff[r], jn + i * cplane2);
                         }
                 }
-                if (!st.ln.active || j0 < 0) return;
+                if (!st.ln.active || j0 < d0) return;
                 float sv[SC][RH][RW];
                 NDC_UNROLL
                 for (int i = 0; i < SC; ++i)
@@ -1150,7 +1166,7 @@ template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
                     for (int r = 0; r < RH; ++r)
                         NDC_UNROLL
                         for (int c = 0; c < RW; ++c) sv[i][r][c] = 0.f;
-                if (j0 < D) {
+                if (j0 < d1) {
                     const unsigned jo = (unsigned)j0 * plane2;
                     if (!SAVED) {
                         NDC_UNROLL
@@ -1213,11 +1229,11 @@ template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
                             const uint32_t gzw = pack_bf16x2(v[0], v[1]);
                             st.gbacc[i] = dot2_bf16(gzw, st.okw[r], st.gbacc[i]);
                             // (no gz asked for: gzb_ is an empty slice and the store goes nowhere)
-                            buf_st<true>(gzb_, st.ooff[r], jo + i * cplane2, gzw);
+                            buf_st<NT>(gzb_, st.ooff[r], jo + i * cplane2, gzw);
                         }
                     }
                 }
-                if (PAR == 0 && need_gh && j0 <= D) {   // j0 odd
+                if (PAR == 0 && need_gh && j0 <= d1) {   // j0 odd
                     // K-side filter-gradient term for the plane pair (j0 - 1, j0):
                     // (s_i[j0-1], s_i[j0]) . (gt1[m], gt1[m+1])[neighbour], m = j0 - td
                     uint32_t ss[SC][RH][RW];
@@ -1261,7 +1277,7 @@ template <int RH_, bool SAVED_ = false> struct Bwd2KernelB {
                             for (int c = 0; c < RW; ++c) st.sprev[i][r][c] = sv[i][r][c];
                 }
         };
-        for (int kk = 0; kk < D + 2; kk += 2) {
+        for (int kk = k0; kk < d1 + 2; kk += 2) {
             {
                 const int k = uniform_int(kk);   // the plane index stays on the scalar unit
                 ex.each([&](State &st, int) NDC_LAMBDA { store_plane(st, k); });
