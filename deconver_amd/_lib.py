@@ -66,6 +66,10 @@ EXPORTS = (
     "ndc_column_sums",
     "ndc_weight_grad_workspace_bytes",
     "ndc_weight_grad",
+    "ndc_mlp_supported",
+    "ndc_mlp_forward",
+    "ndc_mlp_workspace_bytes",
+    "ndc_mlp_backward",
 )
 
 

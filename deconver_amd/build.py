@@ -37,7 +37,7 @@ def _run(cmd):
     return out
 
 
-HIP_SOURCES = ("ndc_capi.hip", "ndc_fused_bf16.hip", "ndc_fused_f32.hip", "ndc_gemm.hip")
+HIP_SOURCES = ("ndc_capi.hip", "ndc_fused_bf16.hip", "ndc_fused_f32.hip", "ndc_gemm.hip", "ndc_mlp.hip")
 
 
 def build_hip(extra_flags=(), out: str = os.path.join(_HERE, "libdeconver_ndc.so"), csrc: str = CSRC) -> str:

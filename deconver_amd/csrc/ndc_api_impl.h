@@ -10,6 +10,7 @@
 #include "ndc_columns.h"
 #include "ndc_direct.h"
 #include "ndc_fused_api.h"
+#include "ndc_mlp_host.h"
 
 namespace ndc {
 
@@ -632,6 +633,54 @@ int ndc_pointwise_gemm_actgrad(const void *gy, const void *wfrag, const float *b
         return NDC_ERR_WORKSPACE;
     if (gz == gy || gz == z) return NDC_ERR_GEOMETRY;
     return ndc::Backend::pwgemm(gy, wfrag, bias, z, gz, nullptr, gpart, nullptr, batch, (int)cin, (int)cout, n, act + 2, stream);
+}
+
+// ---- the MLP with its hidden tensor on chip (ndc_mlp.h)
+
+int ndc_mlp_supported(int64_t c, int64_t n, int dtype)
+{
+    return dtype == NDC_BF16 && (c == 32 || c == 64) && n >= 64 && n % 64 == 0 && n <= (1LL << 26);
+}
+
+static int mlp_check(int64_t batch, int64_t c, int64_t n, int w_dtype, int dtype)
+{
+    if (dtype != NDC_BF16 || (w_dtype != NDC_F32 && w_dtype != NDC_BF16)) return NDC_ERR_DTYPE;
+    if (batch < 1 || !ndc_mlp_supported(c, n, dtype) || (long double)batch * n > 64.0L * 0x7fffff00LL) return NDC_ERR_GEOMETRY;
+    return NDC_OK;
+}
+
+int ndc_mlp_forward(const void *x, const void *w1, const void *w2, int w_dtype, const float *b1, const float *b2,
+                    const void *residual, void *y, int64_t batch, int64_t c, int64_t n, int dtype, void *stream)
+{
+    if (!x || !w1 || !w2 || !y) return NDC_ERR_NULL;
+    const int st = mlp_check(batch, c, n, w_dtype, dtype);
+    if (st) return st;
+    if (((uintptr_t)x & 3u) || ((uintptr_t)y & 3u) || ((uintptr_t)residual & 3u) || ((uintptr_t)b1 & 3u) || ((uintptr_t)b2 & 3u) ||
+        ((uintptr_t)w1 & 3u) || ((uintptr_t)w2 & 3u))
+        return NDC_ERR_WORKSPACE;
+    if (y == x) return NDC_ERR_GEOMETRY;
+    return ndc::Backend::mlp_forward(x, w1, w2, w_dtype == NDC_BF16, b1, b2, residual, y, batch, (int)c, n, stream);
+}
+
+size_t ndc_mlp_workspace_bytes(int64_t batch, int64_t c, int64_t n)
+{
+    if (batch < 1 || !ndc_mlp_supported(c, n, NDC_BF16)) return 0;
+    return (size_t)ndc::mlp::grad_groups(batch * (n / 64)) * (size_t)ndc::mlp::part_floats((int)c) * 4;
+}
+
+int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *w2, int w_dtype, const float *b1,
+                     void *gx, float *gw1, float *gb1, float *gw2, float *gb2, int64_t batch, int64_t c, int64_t n,
+                     int dtype, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!x || !gy || !w1 || !w2 || !gx || !gw1 || !gw2) return NDC_ERR_NULL;
+    const int st = mlp_check(batch, c, n, w_dtype, dtype);
+    if (st) return st;
+    if (((uintptr_t)x & 15u) || ((uintptr_t)gy & 15u) || ((uintptr_t)gx & 3u) || ((uintptr_t)b1 & 3u) || ((uintptr_t)w1 & 3u) ||
+        ((uintptr_t)w2 & 3u) || !workspace || ((uintptr_t)workspace & 15u) || workspace_bytes < ndc_mlp_workspace_bytes(batch, c, n))
+        return NDC_ERR_WORKSPACE;
+    if (gx == x || gx == gy) return NDC_ERR_GEOMETRY;
+    return ndc::Backend::mlp_backward(x, gy, w1, w2, w_dtype == NDC_BF16, b1, gx, gw1, gb1, gw2, gb2, (float *)workspace, batch, (int)c,
+                                      n, stream);
 }
 
 // ---- the tiled GEMMs (ndc_gemm.h)

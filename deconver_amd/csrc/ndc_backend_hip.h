@@ -13,6 +13,7 @@
 #include "ndc_chnorm.h"
 #include "ndc_pwgemm.h"
 #include "ndc_gemm_host.h"
+#include "ndc_mlp_host.h"
 
 #define NDC_LAMBDA __host__ __device__
 
@@ -669,6 +670,20 @@ struct Backend {
                          long long n, int mode, int esz, int waves, void *stream)
     {
         const int st = gemm::tile_gemm(x, w, transposed, bias, res, mask, y, zkeep, gpart, batch, cin, cout, n, mode, esz, waves, stream);
+        return st ? st : check();
+    }
+
+    static int mlp_forward(const void *x, const void *w1, const void *w2, int w_is_bf16, const float *b1, const float *b2,
+                           const void *res, void *y, long long batch, int c, long long n, void *stream)
+    {
+        const int st = mlp::forward(x, w1, w2, w_is_bf16, b1, b2, res, y, batch, c, n, stream);
+        return st ? st : check();
+    }
+    static int mlp_backward(const void *x, const void *gy, const void *w1, const void *w2, int w_is_bf16, const float *b1,
+                            void *gx, float *gw1, float *gb1, float *gw2, float *gb2, float *part, long long batch, int c,
+                            long long n, void *stream)
+    {
+        const int st = mlp::backward(x, gy, w1, w2, w_is_bf16, b1, gx, gw1, gb1, gw2, gb2, part, batch, c, n, stream);
         return st ? st : check();
     }
 

@@ -8,6 +8,7 @@
 #include "ndc_common.h"
 #include "ndc_exec.h"
 #include "ndc_gemm_host.h"
+#include "ndc_mlp_host.h"
 
 #define NDC_LAMBDA
 
@@ -410,6 +411,18 @@ struct Backend {
                     Elem<T>::store(y + at, out);
                 }
     }
+    // (kernels of matrix instructions throughout, without a sequential form)
+    static int mlp_forward(const void *, const void *, const void *, int, const float *, const float *, const void *, void *,
+                           long long, int, long long, void *)
+    {
+        return -2;
+    }
+    static int mlp_backward(const void *, const void *, const void *, const void *, int, const float *, void *, float *, float *,
+                            float *, float *, float *, long long, int, long long, void *)
+    {
+        return -2;
+    }
+
     static int tile_gemm(const void *x, const float *w, int transposed, const float *bias, const void *res, const void *mask,
                          void *y, void *zkeep, float *gpart, long long batch, int cin, int cout, long long n, int mode, int esz,
                          int waves, void *)

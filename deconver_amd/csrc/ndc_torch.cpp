@@ -817,14 +817,38 @@ Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, int6
     return Linear::run(xc, Matrix(weight, transposed), f32_vector(bias), act, res ? *res : Tensor(), false, z, scope.stream);
 }
 
+// Whether an MLP runs with its hidden tensor on chip (ndc_mlp_forward / _backward) where those kernels
+// apply: with 64 channels from 32 768 voxels on (their kernels take 24 + 30 us there, the projections' 30 +
+// 55; over 16 384 voxels 23 against 20 forward), with 32 from 4096 (10 + 20 against 9 + 26).
+int64_t mlp_least_voxels(int64_t c) { return c == 32 ? 4096 : 32768; }
+
+bool mlp_on_chip(const Tensor &x, const Matrix &w1, const Matrix &w2)
+{
+    const int64_t c = x.size(1), n = x.size(2);
+    auto type = [](const Tensor &t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; };
+    return x.scalar_type() == at::kBFloat16 && w1.cout() == 4 * c && w2.cout() == c && type(w1.m) && w1.m.scalar_type() == w2.m.scalar_type() &&
+           x.size(0) * n >= mlp_least_voxels(c) && ndc_mlp_supported(c, n, NDC_BF16) && ((uintptr_t)ptr(x) & 3) == 0;
+}
+
+// the tensor at an address the kernels' 16-byte accesses take
+Tensor aligned(const Tensor &t) { return ((uintptr_t)ptr(t) & 15) ? t.clone() : t; }
+
 // W2 gelu(W1 x + b1) + b2 + residual on contiguous (B, C, n) tensors (layers/mlp.py:40-63 with the
-// block's sum, deconver.py:60-64): the GELU and the kept pre-activation leave the first product,
-// bias and residual ride on the second, and in backward the input gradient of the second comes
-// out already multiplied by the GELU's derivative where one of the library's own GEMMs makes it.
+// block's sum, deconver.py:60-64).  Where mlp_on_chip says so the hidden tensor never leaves the chip: one
+// kernel forward, and one backward that forms it again from x.  Elsewhere the GELU and the kept
+// pre-activation leave the first product, bias and residual ride on the second, and in backward the
+// input gradient of the second comes out already multiplied by the GELU's derivative where one of the
+// library's own GEMMs makes it.
 struct Mlp : public torch::autograd::Function<Mlp> {
     static Tensor run(const Tensor &x, const Matrix &w1, const Tensor &b1, const Matrix &w2, const Tensor &b2, const Tensor &res,
-                      bool keep, Tensor &z, Tensor &a, void *stream)
+                      bool keep, bool on_chip, Tensor &z, Tensor &a, void *stream)
     {
+        if (on_chip && (!res.defined() || ((uintptr_t)ptr(res) & 3) == 0)) {
+            Tensor y = empty(x.sizes(), x);
+            check(ndc_mlp_forward(ptr(x), ptr(w1.m), ptr(w2.m), dtype_tag(w1.m), fptr(b1), fptr(b2), ptr(res), out_ptr(y), x.size(0),
+                                  x.size(1), x.size(2), NDC_BF16, stream), "ndc_mlp_forward");
+            return y;
+        }
         Tensor unused;
         a = Linear::run(x, w1, b1, NDC_ACT_GELU, Tensor(), keep, z, stream);
         return Linear::run(a, w2, b2, NDC_ACT_NONE, res, false, unused, stream);
@@ -835,9 +859,11 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         Scope scope(x);
         Tensor z, a;
         const Tensor b1f = f32_vector(b1);
-        Tensor y = run(x, Matrix(w1, false), b1f, Matrix(w2, false), f32_vector(b2), residual ? *residual : Tensor(), true, z, a,
-                       scope.stream);
-        ctx->save_for_backward({x, z, a, w1, w2, b1f});
+        const Matrix m1(w1, false), m2(w2, false);
+        // (the one-kernel backward makes all gradients at once: taken where they are all wanted)
+        const bool on_chip = wants_grad(x) && wants_grad(w1) && wants_grad(w2) && mlp_on_chip(x, m1, m2);
+        Tensor y = run(x, m1, b1f, m2, f32_vector(b2), residual ? *residual : Tensor(), true, on_chip, z, a, scope.stream);
+        ctx->save_for_backward({x, z, a, w1, w2, b1f});   // (z, a undefined: the hidden tensor stayed on chip)
         ctx->saved_data["cfg"] = std::vector<int64_t>{b1.has_value(), b2.has_value(), residual.has_value(),
                                                       b1 ? (int64_t)b1->scalar_type() : 0, b2 ? (int64_t)b2->scalar_type() : 0};
         return y;
@@ -853,12 +879,30 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         const Matrix w2 = saved_weight(v[4], false, gy.size(1), gy), w1 = saved_weight(v[3], false, w2.cin(), gy);
         const int64_t B = gy.size(0), nv = gy.size(2), hidden = w1.cout();
         const Tensor x = check_saved(v[0], gy, {B, w1.cin(), nv}, gy.scalar_type());
-        const Tensor z = check_saved(v[1], gy, {B, hidden, nv}, gy.scalar_type()), a = check_saved(v[2], z);
         const Tensor b1 = check_saved(v[5], gy, {hidden}, at::kFloat);
         Needs n;
         n.arg(true), n.arg(true), n.arg(cfg[0]), n.arg(true), n.arg(cfg[1]), n.arg(cfg[2]);
         const auto need = n.ask(ctx);
         Tensor gx, gw1, gb1, gw2, gb2;
+        if (!v[1].defined()) {
+            const Tensor xa = aligned(x), ga = aligned(gy);
+            const bool half = w1.m.scalar_type() == at::kBFloat16 && w2.m.scalar_type() == at::kBFloat16;
+            const Tensor m1 = half ? w1.m : w1.m.to(at::kFloat), m2 = half ? w2.m : w2.m.to(at::kFloat);
+            gx = empty(x.sizes(), x);
+            gw1 = empty_f32(m1.sizes(), x), gw2 = empty_f32(m2.sizes(), x);
+            if (need[2]) gb1 = empty_f32({hidden}, x);
+            if (need[4]) gb2 = empty_f32({w2.cout()}, x);
+            const size_t bytes = ndc_mlp_workspace_bytes(B, x.size(1), nv);
+            Tensor ws = scratch(bytes, x);
+            check(ndc_mlp_backward(ptr(xa), ptr(ga), ptr(m1), ptr(m2), dtype_tag(m1), fptr(b1), out_ptr(gx), out_fptr(gw1), out_fptr(gb1),
+                                   out_fptr(gw2), out_fptr(gb2), B, x.size(1), nv, NDC_BF16, out_ptr(ws), bytes, scope.stream),
+                  "ndc_mlp_backward");
+            if (gb1.defined()) gb1 = gb1.to((at::ScalarType)cfg[3]);
+            if (gb2.defined()) gb2 = gb2.to((at::ScalarType)cfg[4]);
+            return once({gx, gw1.to(v[3].scalar_type()).view(v[3].sizes()), gb1, gw2.to(v[4].scalar_type()).view(v[4].sizes()), gb2,
+                         need[5] ? gy : Tensor()}, recording, gouts);
+        }
+        const Tensor z = check_saved(v[1], gy, {B, hidden, nv}, gy.scalar_type()), a = check_saved(v[2], z);
         if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type(), need[4] ? &gb2 : nullptr, scope.stream);
         else if (need[4]) gb2 = channel_sums(gy, scope.stream);
         if (need[0] || need[1] || need[2]) {
@@ -912,7 +956,8 @@ Tensor mlp(const Tensor &x, const Tensor &w1, const OptTensor &b1, const Tensor 
         return Mlp::apply(xc, w1, b1, w2, b2, res);
     Scope scope(xc);
     Tensor z, a;
-    return Mlp::run(xc, Matrix(w1, false), f32_vector(b1), Matrix(w2, false), f32_vector(b2), res ? *res : Tensor(), false, z, a,
+    const Matrix m1(w1, false), m2(w2, false);
+    return Mlp::run(xc, m1, f32_vector(b1), m2, f32_vector(b2), res ? *res : Tensor(), false, mlp_on_chip(xc, m1, m2), z, a,
                     scope.stream);
 }
 

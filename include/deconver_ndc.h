@@ -466,6 +466,28 @@ size_t ndc_weight_grad_workspace_bytes(int64_t batch, int64_t rows, int64_t cols
 int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t batch, int64_t rows,
                     int64_t cols, int64_t n, int dtype, void *workspace, size_t workspace_bytes, void *stream);
 
+/*
+ * The MLP of a Deconver block with its hidden tensor kept on chip (deconver/layers/mlp.py:40-63 with
+ * the sum of deconver/deconver.py:60-64), on channel-first (batch, c, n) bfloat16 tensors:
+ *     y = W2 gelu(W1 x + b1) + b2 + residual          W1 (4c, c), W2 (c, 4c)
+ * and its gradients from x and gy (the hidden tensor is formed again).
+ *   ndc_mlp_supported  1 where the kernels apply: NDC_BF16, c 32 or 64, n a multiple of 64 up to 2^26
+ *   w1, w2      as they lie, both of dtype w_dtype (NDC_F32 or NDC_BF16); rounded to bfloat16 for the
+ *               products
+ *   b1, b2      float32 or NULL; residual: y's shape, or NULL; y may be residual
+ *   gw1, gw2    float32, shapes of W1 and W2; gb1, gb2 float32, or NULL; gb1 is summed before the
+ *               hidden tensor's gradient is rounded
+ *   workspace   ndc_mlp_workspace_bytes(batch, c, n) bytes, 16-byte aligned
+ *   x, gy, gx   16-byte aligned for the backward, word-aligned for the forward; gx is neither x nor gy
+ */
+int ndc_mlp_supported(int64_t c, int64_t n, int dtype);
+int ndc_mlp_forward(const void *x, const void *w1, const void *w2, int w_dtype, const float *b1, const float *b2,
+                    const void *residual, void *y, int64_t batch, int64_t c, int64_t n, int dtype, void *stream);
+size_t ndc_mlp_workspace_bytes(int64_t batch, int64_t c, int64_t n);
+int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *w2, int w_dtype, const float *b1,
+                     void *gx, float *gw1, float *gb1, float *gw2, float *gb2, int64_t batch, int64_t c, int64_t n,
+                     int dtype, void *workspace, size_t workspace_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

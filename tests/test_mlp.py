@@ -5,6 +5,7 @@ import copy
 import pytest
 import torch
 
+from deconver_amd import _lib
 from deconver_amd.layers import MLP, pointwise_linear
 
 pytestmark = pytest.mark.gpu
@@ -41,9 +42,9 @@ def _bias_grad_reference(z, b, gz):
     return u.grad.sum((0, 2)), u.grad.norm(dim=(0, 2))
 
 
-# by what makes the gradient of the hidden tensor: the streaming GEMM; the tiled one, its channels sliced over the
+# by what makes the gradient of the hidden tensor: the kernel that keeps it on chip; the streaming GEMM; the tiled one, its channels sliced over the
 # wavefronts (both tile sizes), in whole and in ragged tiles; the library's and a pass
-ROUTES = [(2, 64, 256, 65536), (1, 64, 256, 1000), (1, 64, 256, 4099), (1, 64, 256, 20001), (2, 30, 120, 777),
+ROUTES = [(2, 64, 256, 65536), (2, 128, 512, 65536), (1, 64, 256, 1000), (1, 64, 256, 4099), (1, 64, 256, 20001), (2, 30, 120, 777),
           (1, 256, 1024, 8192)]
 
 
@@ -78,3 +79,68 @@ def test_bias_gradient_of_a_projection_with_its_gelu_is_not_rounded():
     pointwise_linear(x, w, b, act="gelu").backward(g)
     want, norm = _bias_grad_reference(0.5 * x.float().repeat(1, 3, 1), b.detach(), g)
     assert float(((b.grad - want).abs() / norm).max()) < 2e-5
+
+
+def _float64_mlp(x, w1, b1, w2, b2, res, g):
+    """Value and gradients in float64 of the operands as bfloat16 holds them (weights rounded, as the
+    products take them)."""
+    leaves = [t.detach().double().requires_grad_(True) if t is not None else None
+              for t in (x, w1.bfloat16(), b1, w2.bfloat16(), b2, res)]
+    xd, w1d, b1d, w2d, b2d, rd = leaves
+    u = w1d @ xd if b1d is None else w1d @ xd + b1d[:, None]
+    y = w2d @ torch.nn.functional.gelu(u)
+    if b2d is not None:
+        y = y + b2d[:, None]
+    if rd is not None:
+        y = y + rd
+    y.backward(g.double())
+    return y.detach(), [t.grad if t is not None else None for t in leaves]
+
+
+# the size the hidden tensor stays on chip from, with 64 and 32 channels; tiles that fill the workgroups of
+# the backward and each workgroup size of the forward evenly, and one over
+@pytest.mark.parametrize("B,c,n", [(1, 64, 32768), (1, 64, 65600), (1, 64, 131072), (3, 64, 43712), (1, 64, 262208), (1, 32, 4096),
+                                   (2, 32, 65600), (1, 32, 196608)])
+@pytest.mark.parametrize("bias,residual,wdtype", [(True, True, torch.float32), (False, False, torch.bfloat16)])
+def test_hidden_tensor_on_chip(B, c, n, bias, residual, wdtype):
+    """Bounds: the result and gx carry one rounding (2^-9) of themselves and of the hidden values they
+    sum (their errors independent, so no more in norm); the weight gradients the hidden roundings only;
+    the bias gradients float32 sums and the derivative's 3e-7."""
+    gen = torch.Generator(device="cuda").manual_seed(c + n)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")   # noqa: E731
+    x, g = rand(B, c, n).bfloat16(), rand(B, c, n).bfloat16()
+    w1, w2 = (rand(4 * c, c) / c ** 0.5).to(wdtype), (rand(c, 4 * c) / (4 * c) ** 0.5).to(wdtype)
+    b1, b2 = (rand(4 * c), rand(c)) if bias else (None, None)
+    res = rand(B, c, n).bfloat16() if residual else None
+    leaves = [t.requires_grad_(True) if t is not None else None for t in (x, w1, b1, w2, b2, res)]
+    native = _lib.get_native()
+    y = native.mlp(*leaves)
+    y.backward(g)
+    with torch.no_grad():
+        assert torch.equal(native.mlp(*leaves), y)
+    want, grads = _float64_mlp(x, w1, b1, w2, b2, res, g)
+    err = lambda a, b: float((a.double() - b).norm() / b.norm())   # noqa: E731
+    assert err(y.detach(), want) < 4e-3
+    for t, ref, tol in zip(leaves, grads, (4e-3, 6e-3, 2e-5, 6e-3, 2e-5, 1e-6)):
+        if t is not None and t.dtype == torch.bfloat16:
+            tol = max(tol, 4e-3)
+        assert t is None or err(t.grad, ref) < tol, (tuple(t.shape), err(t.grad, ref))
+
+
+@pytest.mark.parametrize("frozen", ["x", "w1", "w2"])
+def test_partly_frozen_mlp_gives_the_same_gradients(frozen):
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")   # noqa: E731
+    ops_ = dict(x=rand(1, 32, 131072).bfloat16(), w1=rand(128, 32) / 6, w2=rand(32, 128) / 11)
+    g = rand(1, 32, 131072).bfloat16()
+    got = []
+    for keep in (True, False):
+        t = {k: v.clone().requires_grad_(keep or k != frozen) for k, v in ops_.items()}
+        _lib.get_native().mlp(t["x"], t["w1"], None, t["w2"], None, None).backward(g)
+        got.append(t)
+    for k in ops_:
+        if k == frozen:
+            assert got[1][k].grad is None
+        else:
+            a, b = got[0][k].grad.double(), got[1][k].grad.double()
+            assert float((a - b).norm() / a.norm()) < 1e-2
