@@ -652,9 +652,8 @@ struct Projected : public torch::autograd::Function<Projected> {
         // (the GEMMs and the update read rows of voxels: any other layout is turned first)
         const Tensor x = channel_first(x_, stream);
         auto size = x.sizes().vec();
-        // (float32: the library's product.  Its bits decide which source units are on, and Linear, which
-        // makes this product for the layer's general form, takes the same: the two agree bit for bit
-        // as long as both use one kernel, whichever it is)
+        // (float32: the library's product.  Its bits decide which source units are on, and what else forms
+        // this product -- a check of a network's on/off patterns by torch.bmm -- sees the same units)
         Tensor z = project(w, x.flatten(2), x.scalar_type() == at::kFloat, stream);
         size[1] = w.cout();
         Tensor out = update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
@@ -728,8 +727,11 @@ struct Linear : public torch::autograd::Function<Linear> {
     {
         const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
         const bool tail = bias.defined() || act != NDC_ACT_NONE || res.defined();
-        // (an activation's tile form reads W as rows; a bare float32 product: as in Projected)
-        const bool library = (w.transposed && act != NDC_ACT_NONE) || (!tail && x.scalar_type() == at::kFloat);
+        // An activation's tile form reads W as rows.  A bare float32 product that widens could be a layer's
+        // projection taken apart: the library's product, bit for bit as in Projected.  One that narrows (a
+        // stage's adapter, a downsampling) is nobody's but this node's; the library ran 512 -> 256 channels over
+        // 256 voxels in one workgroup, 123 us against 7 us sliced.
+        const bool library = (w.transposed && act != NDC_ACT_NONE) || (!tail && x.scalar_type() == at::kFloat && w.cin() <= cout);
         const Gemm by = library ? kLibrary : choose_gemm(x, cout, act != NDC_ACT_NONE || keep, tail);
         Tensor y = empty({B, cout, n}, x);
         if (keep) z = empty({B, cout, n}, x);
