@@ -315,17 +315,6 @@ NDC_HD int uniform_int(int v)
 #endif
 }
 
-// Zero, of which the compiler does not know that it is the same in every lane: an address formed
-// with it is loaded from by the vector unit, and what is loaded stays in vector registers.
-NDC_HD int lane_zero()
-{
-    int z = 0;
-#if NDC_DEVICE_BUILD && defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(z));
-#endif
-    return z;
-}
-
 template <int N> struct IntTag {
     static constexpr int value = N;
 };

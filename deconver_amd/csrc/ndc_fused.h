@@ -377,15 +377,7 @@ NDC_HD Lane make_lane(int tid, const Tile &t, int RW)
 
 // =================================================================== forward
 
-// HELD: the taps sit in vector registers for the whole march and the tap loops are unrolled, for
-// 2-D launches of one column per thread that put at most two wavefronts on a SIMD.  Such a launch
-// waits for latencies: a rolled tap loop takes nine trips through a scalar load and an LDS read per
-// row step, each one after the other, five times as long as its arithmetic.  With more wavefronts
-// the other form's smaller register count is worth as much (4096 wavefronts: the two are level).
-// 32 channels of 64^2 28.7 -> 23.8 us, 64 channels of 104 x 88 42 -> 31, 512 of 13 x 11 41 -> 34 (21,
-// 26 and 32 with the loads of a plane left in flight, see load_plane).
-template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool HELD_ = false> struct FwdKernel {
-    static constexpr bool HELD = HELD_;
+template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> struct FwdKernel {
     static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_;
     static constexpr int PD = KD / 2, PH = KH / 2, PW = KW / 2, KT = KD * KH * KW;
     static constexpr int XT = PH > 0 ? 1 : 0;            // one extra halo row for strips < 2*PH
@@ -404,7 +396,6 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
         float t1acc[KD][RHK][RW];
         float pz[SC][NZR][RW];
         float px[NXR][RW];
-        float taps[HELD ? SC : 1][HELD ? KT : 1];
         // LDS word offsets inside a ring slot, formed once: the word (first own row - PH, first
         // own column - PW), the word (row `strip`, first own column) and the word (halo row,
         // first own column - PW).  What is added per access (slot, row, channel) is the same in
@@ -527,13 +518,6 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
                 for (int r = 0; r < RHK; ++r)
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) st.t1acc[a][r][c] = 0.f;
-            if constexpr (HELD) {
-                const float *hl = p.h + (long long)id.c * SC * KT + lane_zero();   // (vector loads)
-                NDC_UNROLL
-                for (int i = 0; i < SC; ++i)
-                    NDC_UNROLL
-                    for (int a = 0; a < KT; ++a) st.taps[i][a] = hl[i * KT + a];
-            }
             for (int i = tid; i < total; i += nthreads) ex.st_(i, 0.f);
             load_plane(st, k_first);
         });
@@ -552,15 +536,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
                 store_x_plane(st, k);
                 const bool extra = XT && st.ln.strip < 2 * PH;
                 const int jx = halo_row(st.ln.strip, PH, TH);
-                if constexpr (HELD) {
-                    static_assert(!HELD || !XT, "no halo rows in this form");
-                    if (k < D) {
-                        NDC_UNROLL
-                        for (int i = 0; i < SC; ++i)
-                            k_rows<KD, KH, KW, RH, RW, RHK>(ex, st.ob + (off_s + (i * RS + PH) * P), P, st.taps[i],
-                                                            st.t1acc, 0);
-                    }
-                } else if (k < D) {
+                if (k < D) {
                     NDC_ROLLED
                     for (int ii = 0; ii < SC; ++ii) {
                         const int i = uniform_int(ii);
@@ -627,30 +603,15 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
                         for (int r = 0; r < RH; ++r)
                             NDC_UNROLL
                             for (int c = 0; c < RW; ++c) acc[a][i][r][c] = 0.f;
-                if constexpr (HELD) {
-                    NDC_UNROLL
-                    for (int td = 0; td < KD; ++td) {
-                        float wt[SC][KH * KW];
-                        NDC_UNROLL
-                        for (int i = 0; i < SC; ++i)
-                            NDC_UNROLL
-                            for (int a = 0; a < KH * KW; ++a) wt[i][a] = st.taps[i][td * KH * KW + a];
-                        const int pl = j0 + PD - td;
-                        const int base[2] = {st.ob + (off_x + wrap(pl % XR, XR) * RX * P),
-                                             st.ob + (off_t + wrap(pl % KD, KD) * RX * P)};
-                        a_plane<KH, KW, KT, SC, RH, RW, 2>(ex, base, P, wt, acc);
-                    }
-                } else {
-                    NDC_ROLLED
-                    for (int tdd = 0; tdd < KD; ++tdd) {
-                        const int td = uniform_int(tdd);
-                        float wt[SC][KH * KW];
-                        load_plane_taps<SC, KT, KH * KW>(hw + td * KH * KW, wt);
-                        const int pl = j0 + PD - td;
-                        const int base[2] = {st.ob + (off_x + wrap(pl % XR, XR) * RX * P),
-                                             st.ob + (off_t + wrap(pl % KD, KD) * RX * P)};
-                        a_plane<KH, KW, KT, SC, RH, RW, 2>(ex, base, P, wt, acc);
-                    }
+                NDC_ROLLED
+                for (int tdd = 0; tdd < KD; ++tdd) {
+                    const int td = uniform_int(tdd);
+                    float wt[SC][KH * KW];
+                    load_plane_taps<SC, KT, KH * KW>(hw + td * KH * KW, wt);
+                    const int pl = j0 + PD - td;
+                    const int base[2] = {st.ob + (off_x + wrap(pl % XR, XR) * RX * P),
+                                         st.ob + (off_t + wrap(pl % KD, KD) * RX * P)};
+                    a_plane<KH, KW, KT, SC, RH, RW, 2>(ex, base, P, wt, acc);
                 }
                 NDC_UNROLL
                 for (int r = 0; r < RH; ++r)

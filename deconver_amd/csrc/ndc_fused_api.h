@@ -7,9 +7,11 @@
 #include <stdlib.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "ndc_fused.h"
 #include "ndc_fused_mfma.h"
+#include "ndc_fused_2d.h"
 
 namespace ndc {
 namespace fused {
@@ -121,10 +123,14 @@ static inline std::atomic<int> &matrix_default()
 #endif
 static const long long kSplitWavesF = NDC_SPLIT_F, kSplitWavesB = NDC_SPLIT_B;
 
-#ifndef NDC_HELD_WAVES
-#define NDC_HELD_WAVES 2048
-#endif
-static const long long kHeldWaves = NDC_HELD_WAVES;   // two wavefronts on each of the 1024 SIMDs
+// 2-D problems of up to so many pixels in all, and of small images up to so many, run tile by tile
+// (ndc_fused_2d.h), forward and backward.  us marching -> in tiles, 5x5, float32 (bf16 within 10 %):
+//   forward   32 x 64^2 18 -> 8, 512 x 8^2 21 -> 8, 32 x 128^2 36 -> 17, 64 x 104 x 88 25 -> 21, 2 x 32 x 150 x 170
+//             (1.6 M) 59 -> 46, 8 x 256 x 32^2 (2.1 M) 76 -> 41; 8 x 128 x 64^2 (4.2 M) 85 -> 85, 8 x 64 x 128^2 129 -> 164
+//   backward  32 x 64^2 48 -> 20, 512 x 13 x 11 73 -> 21, 32 x 128^2 67 -> 49, 4 x 64 x 50 x 70 (0.9 M) 87 -> 84,
+//             8 x 256 x 32^2 (2.1 M) 148 -> 101; 32 x 208 x 176 (1.2 M) 89 -> 95, 8 x 128 x 64^2 175 -> 235
+static const long long kPixelsF = 1700 * 1000, kSmallImagesF = 3000 * 1000;
+static const long long kPixelsB = 900 * 1000, kSmallImagesB = 2500 * 1000;
 
 struct Plan {
     Variant v;
@@ -132,6 +138,9 @@ struct Plan {
     bool dot2;            // bf16 dot2 kernels (3x3x3, SC = 4, even W, aligned pairs)
     bool mfma1, mfma2;    // ... with pass 1 / pass 2 on the matrix instruction when they read the forward's ratios
     bool mfmaf;           // ... with the forward on the matrix instruction
+    bool small_f, small_b;   // one-shot kernels of small images (ndc_fused_2d.h); the backward where it has the ratios
+    Tile t2;                 // ... their tiles
+    int nblk_f2, nblk_b2;
     Tile tf, tb;          // forward / backward launch shapes
     int lds_f, lds_b1, lds_b2;
     int nblk_f, nblk_b;
@@ -279,6 +288,16 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
     if (nf > 0x7fffffffLL || nb > 0x7fffffffLL) return false;
     pl.nblk_f = (int)nf;
     pl.nblk_b = (int)nb;
+    pl.small_f = pl.small_b = false;
+    pl.nblk_f2 = pl.nblk_b2 = 0;
+    if (q.sc == 4 && make_tile_2d(pl.m, nbc, pl.t2)) {
+        const long long image = (long long)pl.m.D * pl.m.W, pixels = nbc * image;
+        pl.small_f = pixels <= kPixelsF || (image <= 64 * 64 && pixels <= kSmallImagesF);
+        pl.small_b = pixels <= kPixelsB || (image <= 32 * 32 && pixels <= kSmallImagesB);
+        pl.t2.PL = pairs_ok && pl.m.W % 2 == 0;   // pixels go in and out by pairs
+        if (pl.small_f) pl.nblk_f2 = (int)(nbc * pl.t2.ntile);
+        if (pl.small_b) pl.nblk_b2 = (int)(nbc * ((pl.t2.ntile + pl.t2.SEG - 1) / pl.t2.SEG));
+    }
     return true;
 }
 
@@ -322,7 +341,9 @@ static inline size_t backward_ws(const KGeom &q, int dtype, int /*need_gh*/, int
     const size_t n_x = (size_t)q.B * q.G * q.SP;
     const size_t kt = (size_t)q.sc * q.KT;
     const size_t tabs = has_b && b.dot2 ? align256((size_t)q.G * kTabWords * 4) : 0;
-    return align256(n_x * esz) + align256(nblk * kt * 4) + align256(nblk * (kt + q.sc) * 4) + tabs;
+    const size_t march = align256(n_x * esz) + align256(nblk * kt * 4) + align256(nblk * (kt + q.sc) * 4) + tabs;
+    const size_t tiles = align256((size_t)a.nblk_b2 * (kt + q.sc) * 4);
+    return march > tiles ? march : tiles;
 }
 
 // bytes of scratch the forward call needs (the packed tap tables of the bf16 dot2 kernels)
@@ -399,6 +420,13 @@ template <class BE> static int prepare_taps(const KGeom &q, const float *h, floa
                            [=] NDC_LAMBDA(long long idx) { prep_tables(idx, h, tab); });
 }
 
+// f(kernel type tag): the instance of a one-shot 2-D kernel for this plan
+template <template <int, int, typename> class Kernel, typename T, class F> static int with_tile_2d(const Plan &pl, F f)
+{
+    if (pl.m.KD == 5) return pl.t2.P == 16 ? f((Kernel<5, 16, T> *)nullptr) : f((Kernel<5, 32, T> *)nullptr);
+    return pl.t2.P == 16 ? f((Kernel<3, 16, T> *)nullptr) : f((Kernel<3, 32, T> *)nullptr);
+}
+
 template <class BE, typename T>
 int forward(const KGeom &q, const T *x, const T *z, const float *h, const float *bias,
                    T *out, T *t1, T *s_over_den, T *ratio, const float *taps, void *ws,
@@ -440,12 +468,14 @@ int forward(const KGeom &q, const T *x, const T *z, const float *h, const float 
         }
         return Dot2Launch<BE, T>::fwd(p, pl, stream);
     }
-    // (two wavefronts per SIMD and no more: see FwdKernel)
-    const bool held = (long long)pl.nblk_f * (pl.tf.NT / 64) <= kHeldWaves;
+    if (pl.small_f) {
+        p.t = pl.t2;
+        return with_tile_2d<Fwd2D, T>(pl, [&](auto *tag) {
+            typedef std::remove_pointer_t<decltype(tag)> KS;
+            return BE::template block_kernel<KS>(p, pl.nblk_f2, pl.t2.NT, KS::lds_floats(pl.t2), stream);
+        });
+    }
 #define X(kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_)                                          \
-    if (NDC_IS_VARIANT(pl, kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_) && kh_ == 1 && rwf_ == 1 && held) \
-        return BE::template block_kernel<FwdKernel<kd_, kh_, kw_, sc_, rhf_, rwf_, T, kh_ == 1 && rwf_ == 1>>( \
-            p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);                                         \
     if (NDC_IS_VARIANT(pl, kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_))                        \
         return BE::template block_kernel<FwdKernel<kd_, kh_, kw_, sc_, rhf_, rwf_, T>>(        \
             p, pl.nblk_f, pl.tf.NT, pl.lds_f, stream);
@@ -506,6 +536,36 @@ int backward(const KGeom &q, const T *x, const T *z, const T *t1, const T *s_ove
     p.t = pl.tb;
 
     int st = NDC_ERR_GEOMETRY;
+    const int C = q.G, SC = q.sc, B = q.B;
+    // (gh and gb in one launch: outputs [0, C kt) are gh, the C SC after them gb)
+    const int n_gh = gh ? C * kt : 0, n_gb = gb ? C * SC : 0;
+    auto put = [=] NDC_LAMBDA(int o, float v) {
+        if (o < n_gh) gh[o] = v; else gb[o - n_gh] = v;
+    };
+    if (pl.small_b && saved) {
+        float *part = (float *)ws;
+        p.t = pl.t2;
+        p.part = part;
+        p.part_stride = kt + SC;
+        st = with_tile_2d<Bwd2D, T>(pl, [&](auto *tag) {
+            typedef std::remove_pointer_t<decltype(tag)> KS;
+            return BE::template block_kernel<KS>(p, pl.nblk_b2, pl.t2.NT, KS::lds_floats(pl.t2), stream);
+        });
+        if (st) return st;
+        tm.mark();
+        tm.mark();
+        if (n_gh + n_gb) {
+            const int ntile = (pl.t2.ntile + pl.t2.SEG - 1) / pl.t2.SEG;
+            st = BE::strided_sum(n_gh + n_gb, B * ntile, stream, put, [=] NDC_LAMBDA(int o, int pi) {
+                const int c = o < n_gh ? o / kt : (o - n_gh) / SC, r = o < n_gh ? o % kt : kt + (o - n_gh) % SC;
+                return part[(((long long)(pi / ntile) * C + c) * ntile + pi % ntile) * (kt + SC) + r];
+            });
+            if (st) return st;
+        }
+        tm.mark();
+        tm.finish(pass_ms, 3);
+        return NDC_OK;
+    }
     p.part = part1;
     p.part_stride = kt;
     if (pl.dot2) {
@@ -560,13 +620,9 @@ int backward(const KGeom &q, const T *x, const T *z, const T *t1, const T *s_ove
     tm.mark();
 
     // combine the per-workgroup partial sums: a fixed association, so results are reproducible
-    const int C = q.G, SC = q.sc, ntile = pl.tb.ntile * pl.tb.nseg, B = q.B;
-    // (gh and gb in one launch: outputs [0, C kt) are gh, the C SC after them gb)
-    const int n_gh = gh ? C * kt : 0, n_gb = gb ? C * SC : 0;
+    const int ntile = pl.tb.ntile * pl.tb.nseg;
     if (n_gh + n_gb) {
-        st = BE::strided_sum(n_gh + n_gb, B * ntile, stream, [=] NDC_LAMBDA(int o, float v) {
-            if (o < n_gh) gh[o] = v; else gb[o - n_gh] = v;
-        }, [=] NDC_LAMBDA(int o, int pi) {
+        st = BE::strided_sum(n_gh + n_gb, B * ntile, stream, put, [=] NDC_LAMBDA(int o, int pi) {
             if (o < n_gh) {
                 const int c = o / kt, r = o % kt;
                 const long long blk = ((long long)(pi / ntile) * C + c) * ntile + pi % ntile;
