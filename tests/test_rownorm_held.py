@@ -1,0 +1,33 @@
+"""Rows held in registers by one workgroup: lengths at and next to every size of workgroup and every
+number of vectors a thread, whole vectors and single elements, the longest such row and the first that
+takes two launches, with and without the addend, against float64.  Bounds as in the other norm tests."""
+
+import pytest
+import torch
+
+from deconver_amd.norm import InstanceNorm2d
+
+pytestmark = pytest.mark.gpu
+
+# in 16-byte vectors; * 4 or 8 elements, and one element more (single elements from there on)
+VECTORS = [1, 127, 128, 129, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192, 8193, 12288, 12289]
+
+
+@pytest.mark.parametrize("vectors", VECTORS)
+@pytest.mark.parametrize("odd", [0, 1])
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("rows", [3, 97])
+def test_lengths(vectors, odd, dtype, tol, rows):
+    n = vectors * (16 // dtype.itemsize) + odd
+    print("case", rows, n, dtype, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x = (torch.randn(1, rows, n, 1, generator=gen, device="cuda") * 3 + 20).to(dtype).requires_grad_(True)
+    g, skip_g = (torch.randn(x.shape, generator=gen, device="cuda").to(dtype) for _ in range(2))
+    norm = InstanceNorm2d(rows)
+    y, skip = norm.with_skip(x)
+    (y * g + skip * skip_g).sum().backward()
+    xd = x.detach().double().requires_grad_(True)
+    yd = torch.nn.functional.instance_norm(xd)
+    (yd * g.double() + xd * skip_g.double()).sum().backward()
+    for a, r in ((y, yd), (x.grad, xd.grad)):
+        assert float((a.detach().double() - r.detach()).abs().max() / r.detach().abs().max()) < tol
