@@ -70,6 +70,9 @@ EXPORTS = (
     "ndc_mlp_forward",
     "ndc_mlp_workspace_bytes",
     "ndc_mlp_backward",
+    "ndc_dice_bce_workspace_bytes",
+    "ndc_dice_bce_forward",
+    "ndc_dice_bce_backward",
 )
 
 

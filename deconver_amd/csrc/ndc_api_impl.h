@@ -683,6 +683,53 @@ int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *
                                       n, stream);
 }
 
+// ---- training loss (ndc_loss.h)
+
+// Parts of a row, a workgroup each: about 2048 in all where a part keeps 2048 elements, and a part has at
+// most 65536 (a thread then sums 256 terms).  One workgroup adds the parts of all rows, a wavefront a row:
+// that is sized for some hundred rows, hence the limit.
+static int dice_split(long long rows, long long n, int &parts, long long &chunk)
+{
+    if (rows < 1 || n < 1 || rows > 1024 || n > (1LL << 36)) return NDC_ERR_GEOMETRY;
+    long long want = (2048 + rows - 1) / rows;
+    if (want > n / 2048) want = n / 2048;
+    if (want < (n + 65535) / 65536) want = (n + 65535) / 65536;
+    chunk = (n + want - 1) / want;
+    parts = (int)((n + chunk - 1) / chunk);
+    return rows * parts < (1LL << 31) ? NDC_OK : NDC_ERR_GEOMETRY;
+}
+
+size_t ndc_dice_bce_workspace_bytes(int64_t rows, int64_t n)
+{
+    int parts;
+    long long chunk;
+    return dice_split(rows, n, parts, chunk) ? 0 : (size_t)rows * parts * 16;
+}
+
+int ndc_dice_bce_forward(const float *logits, const float *target, float *loss, float *coef, int64_t rows, int64_t n,
+                         void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!logits || !target || !loss || !coef || !workspace) return NDC_ERR_NULL;
+    int parts;
+    long long chunk;
+    const int st = dice_split(rows, n, parts, chunk);
+    if (st) return st;
+    if (workspace_bytes < (size_t)rows * parts * 16 || ((uintptr_t)workspace & 15u) || ((uintptr_t)coef & 7u)) return NDC_ERR_WORKSPACE;
+    return ndc::Backend::dice_bce_forward(logits, target, loss, coef, (float *)workspace, (int)rows, n, parts, chunk, stream);
+}
+
+int ndc_dice_bce_backward(const float *logits, const float *target, const float *coef, const float *gloss,
+                          float *glogits, int64_t rows, int64_t n, void *stream)
+{
+    if (!logits || !target || !coef || !gloss || !glogits) return NDC_ERR_NULL;
+    int parts;
+    long long chunk;
+    const int st = dice_split(rows, n, parts, chunk);
+    if (st) return st;
+    if ((uintptr_t)coef & 7u) return NDC_ERR_WORKSPACE;
+    return ndc::Backend::dice_bce_backward(logits, target, coef, gloss, glogits, (int)rows, n, parts, chunk, stream);
+}
+
 // ---- the tiled GEMMs (ndc_gemm.h)
 
 static int gemm_check(long long batch, long long cin, long long cout, long long n, int dtype)

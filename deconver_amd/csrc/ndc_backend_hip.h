@@ -14,6 +14,7 @@
 #include "ndc_pwgemm.h"
 #include "ndc_gemm_host.h"
 #include "ndc_mlp_host.h"
+#include "ndc_loss.h"
 
 #define NDC_LAMBDA __host__ __device__
 
@@ -717,6 +718,23 @@ struct Backend {
     {
         const int st = mlp::backward(x, gy, w1, w2, w_is_bf16, b1, gx, gw1, gb1, gw2, gb2, part, batch, c, n, stream);
         return st ? st : check();
+    }
+
+    static int dice_bce_forward(const float *l, const float *y, float *loss, float *coef, float *partial, int rows, long long n,
+                                int parts, long long chunk, void *stream)
+    {
+        hipLaunchKernelGGL(loss::sums_kernel, dim3((unsigned)(rows * parts)), dim3(loss::kThreads), 0, (hipStream_t)stream, l, y,
+                           (float4 *)partial, n, parts, chunk);
+        hipLaunchKernelGGL(loss::finish_kernel, dim3(1), dim3(loss::kFinish), 0, (hipStream_t)stream, (const float4 *)partial,
+                           (float2 *)coef, loss, rows, parts, 1.f / ((float)rows * (float)n));
+        return check();
+    }
+    static int dice_bce_backward(const float *l, const float *y, const float *coef, const float *g, float *gl, int rows, long long n,
+                                 int parts, long long chunk, void *stream)
+    {
+        hipLaunchKernelGGL(loss::grad_kernel, dim3((unsigned)(rows * parts)), dim3(loss::kThreads), 0, (hipStream_t)stream, l, y,
+                           (const float2 *)coef, g, gl, n, parts, chunk, 1.f / ((float)rows * (float)n));
+        return check();
     }
 
     static constexpr int kSumSlices = 8;

@@ -1173,6 +1173,74 @@ Tensor regroup(const Tensor &x, bool to_channels, const OptTensor &bias)
     return regroup_run(x, to_channels, f32_vector(bias), scope.stream);
 }
 
+// ---------------------------------------------------------------------------- training loss
+
+// Cross-entropy plus Dice loss (ndc_loss.h) of float32 (B, C, *S) logits and targets of their shape.
+struct DiceBce : public torch::autograd::Function<DiceBce> {
+    static Tensor run(const Tensor &l, const Tensor &y, Tensor &coef, void *stream)
+    {
+        const int64_t rows = l.size(0) * l.size(1), n = l.numel() / rows;
+        Tensor loss = empty_f32({}, l);
+        coef = empty_f32({rows, 2}, l);
+        const size_t bytes = ndc_dice_bce_workspace_bytes(rows, n);
+        Tensor ws = empty_f32({(int64_t)(bytes / 4)}, l);
+        check(ndc_dice_bce_forward(fptr(l), fptr(y), out_fptr(loss), out_fptr(coef), rows, n, out_ptr(ws), bytes, stream),
+              "ndc_dice_bce_forward");
+        return loss;
+    }
+    static Tensor forward(AutogradContext *ctx, const Tensor &l, const Tensor &y)
+    {
+        Scope scope(l);
+        Tensor coef, loss = run(l.contiguous(), y.contiguous(), coef, scope.stream);
+        ctx->save_for_backward({l, y, coef});
+        return loss;
+    }
+    // (under create_graph the gradient is made of tensor operations, which can be differentiated again)
+    static Tensor formula(const Tensor &l, const Tensor &y_, const Tensor &g)
+    {
+        const int64_t rows = l.size(0) * l.size(1), n = l.numel() / rows;
+        const Tensor p = l.reshape({rows, n}).sigmoid(), y = y_.reshape({rows, n});
+        const Tensor num = 2 * (p * y).sum(1, true) + 1, den = p.sum(1, true) + y.sum(1, true) + 1;
+        const Tensor dp = (num / (den * den) - 2 * y / den) / (double)rows;
+        return (g * ((p - y) / ((double)rows * (double)n) + p * (1 - p) * dp)).view(l.sizes());
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list gouts)
+    {
+        const auto v = ctx->get_saved_variables();
+        const Tensor &g = gouts[0];
+        check_device(v[0], g, "a saved tensor");
+        const c10::DeviceGuard device(g.device());
+        if (at::GradMode::is_enabled() && (wants_grad(g) || wants_grad(v[0]))) return {formula(v[0], v[1], g), Tensor()};
+        Scope scope(g);
+        TORCH_CHECK_VALUE(v[0].dim() >= 3 && v[0].numel() > 0, "a saved tensor came back as ", v[0].sizes());
+        const int64_t rows = v[0].size(0) * v[0].size(1), n = v[0].numel() / rows;
+        const Tensor l = check_saved(v[0], g, v[0].sizes(), at::kFloat), y = check_saved(v[1], g, l.sizes(), at::kFloat);
+        const Tensor coef = check_saved(v[2], g, {rows, 2}, at::kFloat), gl = at::empty_like(l);
+        check(ndc_dice_bce_backward(fptr(l), fptr(y), fptr(coef), fptr(g.contiguous()), out_fptr(gl), rows, n, scope.stream),
+              "ndc_dice_bce_backward");
+        return {gl, Tensor()};
+    }
+};
+
+// None for tensors that the kernels do not take; the caller has the loss in tensor operations.
+OptTensor dice_bce(const Tensor &l, const Tensor &y)
+{
+    const auto plain = [](const Tensor &t) {
+        return t.is_cuda() && t.scalar_type() == at::kFloat && t.layout() == at::kStrided && !t._fw_grad(0).defined() &&
+               !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                                         c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize}));
+    };
+    if (!plain(l) || !plain(y) || l.device() != y.device() || l.dim() < 3 || l.sizes() != y.sizes() || l.numel() == 0 ||
+        wants_grad(y) || ndc_dice_bce_workspace_bytes(l.size(0) * l.size(1), voxels(l)) == 0)
+        return std::nullopt;
+    if (at::GradMode::is_enabled() && wants_grad(l)) return DiceBce::apply(l, y);
+    Scope scope(l);
+    Tensor coef;
+    return DiceBce::run(l.contiguous(), y.contiguous(), coef, scope.stream);
+}
+
+// ---------------------------------------------------------------------------- columns
+
 // Column matrix of a contiguous (B, C, *S) tensor for odd kernel extents k: (B, C * taps, voxels).
 // Not differentiable: the caller takes it for inputs that need no gradient.
 Tensor columns(const Tensor &x, const std::vector<int64_t> &k)
@@ -1225,6 +1293,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     name_node<RowNormSkip>("_RowNormSkipBackward");
     name_node<ChannelNorm>("_ChannelNormBackward");
     name_node<Regroup>("_RegroupBackward");
+    name_node<DiceBce>("_DiceBceBackward");
     m.def("update", &update);
     m.def("projected_update", &projected_update);
     m.def("prepare_taps", &taps_for);
@@ -1235,4 +1304,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("channel_norm", &channel_norm);
     m.def("regroup", &regroup);
     m.def("columns", &columns);
+    m.def("dice_bce", &dice_bce);
 }

@@ -18,6 +18,9 @@ from typing import Callable, Optional, Sequence, Tuple
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch.utils._python_dispatch import _get_current_dispatch_mode
+
+from . import _lib
 
 __all__ = ["dice_bce_loss", "make_optimizer", "smoothed_noise_masks", "ellipsoid_phantoms",
            "train_step", "GraphedTrainStep"]
@@ -34,10 +37,25 @@ def _voxel_sum(t: Tensor) -> Tensor:
     return t.sum(-1)
 
 
+def _one_node(logits: Tensor) -> bool:
+    return (logits.is_cuda and type(logits) is Tensor and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing() and _get_current_dispatch_mode() is None
+            and not torch._C._are_functorch_transforms_active())
+
+
 def dice_bce_loss(logits: Tensor, target: Tensor) -> Tensor:
-    """Binary cross-entropy on the logits plus soft Dice loss with +1 smoothing, float32."""
+    """Binary cross-entropy on the logits plus soft Dice loss with +1 smoothing, float32.
+
+    On the GPU one compiled node of three launches (two forward, one backward); what it does not
+    take -- the CPU, a target of another shape or one that needs a gradient, forward-mode and
+    functorch transforms, a trace or a dispatch mode that wants to see the operations -- is
+    computed by the tensor operations, some 45 launches forward and backward."""
     logits = logits.float()
     target = target.float()
+    if _one_node(logits):
+        loss = _lib.get_native().dice_bce(logits, target)
+        if loss is not None:
+            return loss
     bce = F.binary_cross_entropy_with_logits(logits, target)
     p = torch.sigmoid(logits).flatten(2)
     y = target.flatten(2)

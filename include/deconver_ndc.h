@@ -488,6 +488,22 @@ int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *
                      void *gx, float *gw1, float *gb1, float *gw2, float *gb2, int64_t batch, int64_t c, int64_t n,
                      int dtype, void *workspace, size_t workspace_bytes, void *stream);
 
+/*
+ * Binary cross-entropy on logits plus soft Dice loss with +1 smoothing, the training loss of the
+ * network's benchmark workloads (the reference ships none), over `rows` = batch * channels rows
+ * (at most 1024) of n, float32:
+ *     loss = mean(bce(l, y)) + mean over rows of 1 - (2 sum(p y) + 1) / (sum(p) + sum(y) + 1)
+ *   logits, target  (rows, n)
+ *   loss        one float; coef 2 * rows floats (8-byte aligned), kept for the backward
+ *   workspace   ndc_dice_bce_workspace_bytes(rows, n) bytes, 16-byte aligned
+ *   gloss       one float on the device; glogits (rows, n)
+ */
+size_t ndc_dice_bce_workspace_bytes(int64_t rows, int64_t n);
+int ndc_dice_bce_forward(const float *logits, const float *target, float *loss, float *coef, int64_t rows, int64_t n,
+                         void *workspace, size_t workspace_bytes, void *stream);
+int ndc_dice_bce_backward(const float *logits, const float *target, const float *coef, const float *gloss,
+                          float *glogits, int64_t rows, int64_t n, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
