@@ -41,7 +41,7 @@ struct Variant {
 struct Tuning {
     int rhf, rwf, rhb, rwb;      // forced register tiles (0: the table's order of preference)
     int threads_f, threads_b;    // workgroup sizes of the FMA kernels, forward / backward
-    int threads_f2, threads_b2;  // ... of the bf16 dot2 kernels, and the other size tried by dot2_tile
+    int threads_f2, threads_b2;  // ... of the bf16 dot2 kernels, and the other size tried by cost_tile
     int threads_f2_wide, threads_b2_narrow;
     int split, dot2;             // march segments on / bf16 dot2 kernels on
     int mfma;                    // bf16 matrix-instruction kernels on (where they cover the geometry)
@@ -146,19 +146,11 @@ struct Plan {
     int nblk_f, nblk_b;
 };
 
-template <int KD, int KH, int KW, int SC, int RHF, int RWF, int RHB, int RWB>
-static inline void plan_lds(Plan &pl)
-{
-    pl.lds_f = FwdKernel<KD, KH, KW, SC, RHF, RWF, float>::lds_floats(pl.tf);
-    pl.lds_b1 = Bwd1Kernel<KD, KH, KW, SC, RHB, RWB, float>::lds_floats(pl.tb);
-    pl.lds_b2 = Bwd2Kernel<KD, KH, KW, SC, RHB, RWB, float>::lds_floats(pl.tb);
-}
-
 #define NDC_IS_VARIANT(pl, kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_)                          \
     ((pl).v.KD == kd_ && (pl).v.KH == kh_ && (pl).v.KW == kw_ && (pl).v.SC == sc_ &&            \
      (pl).v.RHF == rhf_ && (pl).v.RWF == rwf_ && (pl).v.RHB == rhb_ && (pl).v.RWB == rwb_)
 
-// What a launch of the bf16 dot2 kernels takes, up to a factor: the wavefronts a SIMD of the
+// What a launch of the 3-D kernels takes, up to a factor: the wavefronts a SIMD of the
 // busiest CU works through, times the planes a workgroup marches over.
 //   * R workgroups of a CU run at once (LDS and registers; a workgroup's wavefronts go round the
 //     four SIMDs, so six count as eight).  q resident ones take q ceil(w / 4) + 1: a SIMD with one
@@ -167,12 +159,17 @@ static inline void plan_lds(Plan &pl)
 //     the two halo rows it computes twice (a fifth of a strip's work each).
 //   * `mixed`: from two full rounds on, workgroups of different rounds overlap and a remainder
 //     costs its share only (the forward, whose four wavefronts per SIMD drift apart).
-// Against the best of 56 launch shapes measured on each of 22 problems (16^3 .. 192^3, widths 14
-// to 192, 32 to 512 channels) the choice is 1 % behind on average and 11 % at worst; the fixed shape it
-// replaced (256 threads, the whole march) took 1.37 (forward) and 1.24 (backward) times as long on
-// average, 2.7 times on 64 channels of 32^3 (115 / 117 / 81 -> 42 / 50 / 34 us).
-static inline double dot2_cost(const Tile &t, const March &m, long long nbc, int lds_floats, int waves_per_simd,
-                               bool mixed)
+// bf16 dot2 kernels: against the best of 56 launch shapes measured on each of 22 problems (16^3 ..
+// 192^3, widths 14 to 192, 32 to 512 channels) the choice is 1 % behind on average and 11 % at worst;
+// the fixed shape it replaced (256 threads, the whole march) took 1.37 (forward) and 1.24 (backward)
+// times as long on average, 2.7 times on 64 channels of 32^3 (115 / 117 / 81 -> 42 / 50 / 34 us).
+// FMA kernels (float32, odd widths): of up to 60 shapes on 13 problems (15x17x13 .. 128^3, 16 to 128
+// channels) 1 % behind (forward) and 2 % (backward) on average; the fixed 256 and 512 threads, cut into
+// segments until 4096 and 2048 wavefronts were there, left rounds of workgroups part empty: 64 channels
+// of 45x53x77 in bf16 455 / 285 -> 320 / 207 us (the two passes of the backward), 32 of 96^3 in float32
+// 905 / 562 -> 602 / 418, 32 of 95x79x93 617 -> 509 us forward; at worst 3 % slower (32 of 95x79x93, back).
+static inline double launch_cost(const Tile &t, const March &m, long long nbc, int lds_floats, int waves_per_simd,
+                                 bool mixed)
 {
     const int w = t.NT / 64;
     int R = kMaxLdsBytes / (lds_floats * 4);
@@ -189,25 +186,25 @@ static inline double dot2_cost(const Tile &t, const March &m, long long nbc, int
     return planes * (1.0 + 0.4 / t.S) * T;
 }
 
-// The row bands (workgroups of about `targets[i]` threads) and march segments (an even number of
-// planes, six at least) with the smallest cost.  K: the kernel whose LDS need counts.
-template <class K>
-static inline bool dot2_tile(const March &m, int RH, long long nbc, const int (&targets)[2], int min_strips,
-                             int waves_per_simd, bool mixed, Tile &best)
+// The row bands (workgroups of about `targets[i]` threads of RH x RW outputs) and march segments (an
+// even number of planes, `min_planes` at least) with the smallest cost.  K: the kernel whose LDS need counts.
+template <class K, int N>
+static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, const int (&targets)[N], int min_strips,
+                             int min_planes, int waves_per_simd, bool mixed, Tile &best)
 {
     static const int parts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
     double least = 0.0;
     bool found = false;
     for (int target : targets) {
         Tile t;
-        if (!make_tile(m, RH, 2, target, t, min_strips)) continue;
+        if (!make_tile(m, RH, RW, target, t, min_strips)) continue;
         const int lds = K::lds_floats(t);
         if (lds * 4 > kMaxLdsBytes) continue;
         for (int n : parts) {
-            if (n > 1 && m.D < 6 * n) break;
+            if (n > 1 && m.D < min_planes * n) break;
             t.SEG = n == 1 ? m.D : round_up((m.D + n - 1) / n, 2);
             t.nseg = (m.D + t.SEG - 1) / t.SEG;
-            const double cost = dot2_cost(t, m, nbc, lds, waves_per_simd, mixed);
+            const double cost = launch_cost(t, m, nbc, lds, waves_per_simd, mixed);
             if (!found || cost < least) {
                 found = true;
                 least = cost;
@@ -216,6 +213,23 @@ static inline bool dot2_tile(const March &m, int RH, long long nbc, const int (&
         }
     }
     return found;
+}
+
+template <int KD, int KH, int KW, int SC, int RHF, int RWF, int RHB, int RWB>
+static inline void plan_lds(Plan &pl, long long nbc)
+{
+    if constexpr (KD == 3 && KH == 3) {
+        // (153 registers a thread and more forward, 179 and more backward)
+        const Tuning tn = tuning();
+        const int targets_f[4] = {64, 128, tn.threads_f, 512}, targets_b[3] = {128, 256, tn.threads_b};
+        if (tn.split) {
+            cost_tile<FwdKernel<KD, KH, KW, SC, RHF, RWF, float>>(pl.m, RHF, RWF, nbc, targets_f, 0, 4, 3, false, pl.tf);
+            cost_tile<Bwd1Kernel<KD, KH, KW, SC, RHB, RWB, float>>(pl.m, RHB, RWB, nbc, targets_b, 0, 4, 2, false, pl.tb);
+        }
+    }
+    pl.lds_f = FwdKernel<KD, KH, KW, SC, RHF, RWF, float>::lds_floats(pl.tf);
+    pl.lds_b1 = Bwd1Kernel<KD, KH, KW, SC, RHB, RWB, float>::lds_floats(pl.tb);
+    pl.lds_b2 = Bwd2Kernel<KD, KH, KW, SC, RHB, RWB, float>::lds_floats(pl.tb);
 }
 
 // pairs_ok: every activation pointer of the call is aligned to two elements
@@ -232,14 +246,14 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
     const Tuning tn = tuning();
     if (!make_tile(pl.m, pl.v.RHF, pl.v.RWF, tn.threads_f, pl.tf)) return false;
     if (!make_tile(pl.m, pl.v.RHB, pl.v.RWB, tn.threads_b, pl.tb)) return false;
-    if (tn.split) {
-        // the forward keeps four wavefronts per SIMD resident, the backward kernels two
+    if (tn.split && pl.m.KH == 1) {
+        // 2-D: the forward keeps four wavefronts per SIMD resident, the backward kernels two
         split_march(pl.m, (long long)q.B * q.G * pl.tf.ntile, pl.tf, kSplitWavesF);
         split_march(pl.m, (long long)q.B * q.G * pl.tb.ntile, pl.tb, kSplitWavesB);
     }
 #define X(kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_)                                        \
     if (NDC_IS_VARIANT(pl, kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_))                      \
-        plan_lds<kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_>(pl);
+        plan_lds<kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_>(pl, (long long)q.B * q.G);
     NDC_FUSED_VARIANTS(X)
 #undef X
     // (their buffer addressing wants every (sample, channel group) slice below 2^31 bytes)
@@ -254,9 +268,9 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
                                       Bwd2KernelM<kDot2RH>::covers(pl.m.W));
         const bool fits = whole ? make_tile(pl.m, kDot2RH, 2, tn.threads_f2, tf, FwdKernelB<kDot2RH>::kMinStrips) &&
                                       make_tile(pl.m, kDot2RH, 2, tn.threads_b2, tb)
-                                : dot2_tile<FwdKernelB<kDot2RH>>(pl.m, kDot2RH, nbc, targets_f,
-                                                                 FwdKernelB<kDot2RH>::kMinStrips, 4, true, tf) &&
-                                      dot2_tile<Bwd1KernelB<kDot2RH, true>>(pl.m, kDot2RH, nbc, targets_b, 0, 2, false, tb);
+                                : cost_tile<FwdKernelB<kDot2RH>>(pl.m, kDot2RH, 2, nbc, targets_f,
+                                                                 FwdKernelB<kDot2RH>::kMinStrips, 6, 4, true, tf) &&
+                                      cost_tile<Bwd1KernelB<kDot2RH, true>>(pl.m, kDot2RH, 2, nbc, targets_b, 0, 6, 2, false, tb);
         if (fits) {
             const int lf = FwdKernelB<kDot2RH>::lds_floats(tf);
             const int l1 = Bwd1KernelB<kDot2RH>::lds_floats(tb);
