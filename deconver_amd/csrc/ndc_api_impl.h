@@ -770,6 +770,15 @@ static ndc::WgradPlan wgrad_plan(long long batch, long long rows, long long cols
     if (per > most) per = most;
     w.chunk = ((n + per - 1) / per + stage - 1) / stage * stage;
     w.per_sample = (int)((n + w.chunk - 1) / w.chunk);
+    // Few voxels: no splits (per_sample 0, see wgrad_whole_kernel).  us, this and the split form with its
+    // sum, float32 / bf16: 64 x 64 over 256 voxels 6.4 -> 3.6 / 5.4 -> 3.1, over 1024 6.5 -> 6.2 / 5.7 -> 4.4,
+    // over 2048 7.2 -> 9.6 / 6.3 -> 6.1; 512 x 512 over 512 in tiles of 32 13.4 -> 6.7 / 11.7 -> 4.7 (in tiles
+    // of 16 10.7 / 7.4).  Rows that end within 16 bytes read their last turns element by element: 512 x 512
+    // over 500 13.0 -> 7.0 / 10.8 -> 4.3, 64 x 64 over 3 x 343 7.1 -> 4.9 / 8.6 -> 9.8.
+    if (batch * w.per_sample > 1 && batch * n <= (n * esz % 16 ? 512 : 1024)) {
+        w.per_sample = 0, w.bm = w.bn = 16;
+        if (tiles_of() > 256) w.bm = w.bn = 32;
+    }
     return w;
 }
 
@@ -778,7 +787,7 @@ size_t ndc_weight_grad_workspace_bytes(int64_t batch, int64_t rows, int64_t cols
     if (gemm_check(batch, cols, rows, n, dtype)) return 0;
     const ndc::WgradPlan w = wgrad_plan(batch, rows, cols, n, dtype == NDC_BF16 ? 2 : 4);
     const long long splits = batch * w.per_sample;
-    return splits == 1 ? 0 : (size_t)splits * (size_t)(rows * cols + rows) * 4;
+    return splits <= 1 ? 0 : (size_t)splits * (size_t)(rows * cols + rows) * 4;
 }
 
 int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t batch, int64_t rows, int64_t cols,

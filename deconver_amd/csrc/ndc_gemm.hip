@@ -28,6 +28,15 @@ int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long 
                  long long n, int esz, const WgradPlan &plan, void *stream)
 {
     WgradParams p;
+    if (plan.per_sample == 0) {   // all voxels to a workgroup
+        p.a = a, p.b = b, p.part = nullptr, p.gw = gw, p.gb = gb, p.n = n, p.rows = rows, p.cols = cols;
+        p.tiles_m = (rows + plan.bm - 1) / plan.bm, p.tiles_n = (cols + plan.bn - 1) / plan.bn, p.splits = (int)batch;
+        const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * kWholeWaves);
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, p); };
+        if (plan.bm == 32) esz == 4 ? launch(wgrad_whole_kernel<float, 32>) : launch(wgrad_whole_kernel<bf16_t, 32>);
+        else esz == 4 ? launch(wgrad_whole_kernel<float, 16>) : launch(wgrad_whole_kernel<bf16_t, 16>);
+        return 0;
+    }
     p.a = a, p.b = b, p.part = part, p.gw = gw, p.gb = gb, p.n = n, p.chunk = plan.chunk, p.rows = rows, p.cols = cols;
     p.tiles_m = (rows + plan.bm - 1) / plan.bm, p.tiles_n = (cols + plan.bn - 1) / plan.bn;
     p.per_sample = plan.per_sample, p.splits = (int)batch * plan.per_sample;

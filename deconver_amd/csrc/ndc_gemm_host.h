@@ -7,7 +7,7 @@ namespace ndc {
 // how ndc_weight_grad cuts its work: tile of the result per workgroup, stage depth in granules,
 // voxels per split
 struct WgradPlan {
-    int bm, bn, depth, per_sample;
+    int bm, bn, depth, per_sample;   // per_sample 0: all samples and voxels in one workgroup
     long long chunk;
 };
 

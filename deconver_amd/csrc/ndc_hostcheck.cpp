@@ -362,6 +362,22 @@ struct Backend {
                         long long n, const WgradPlan &w)
     {
         const long long out = (long long)rows * cols;
+        if (w.per_sample == 0) {   // no splits
+            for (int r = 0; r < rows; ++r) {
+                float sum = 0.f;
+                for (int c = -1; c < cols; ++c) {
+                    float acc = 0.f;
+                    for (long long at = 0; at < batch; ++at)
+                        for (long long v = 0; v < n; ++v) {
+                            const float av = Elem<T>::load(a + (at * rows + r) * n + v);
+                            if (c < 0) sum += av; else acc += av * Elem<T>::load(b + (at * cols + c) * n + v);
+                        }
+                    if (c >= 0) gw[(long long)r * cols + c] = acc;
+                }
+                if (gb) gb[r] = sum;
+            }
+            return;
+        }
         for (long long s = 0; s < batch * w.per_sample; ++s) {
             const long long at = s / w.per_sample, lo = s % w.per_sample * w.chunk, hi = std::min(n, lo + w.chunk);
             float *ow = part ? part + s * (out + rows) : gw, *ob = part ? ow + out : gb;
