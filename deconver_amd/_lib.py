@@ -73,6 +73,7 @@ EXPORTS = (
     "ndc_dice_bce_workspace_bytes",
     "ndc_dice_bce_forward",
     "ndc_dice_bce_backward",
+    "ndc_adamw",
 )
 
 

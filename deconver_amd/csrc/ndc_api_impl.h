@@ -730,6 +730,23 @@ int ndc_dice_bce_backward(const float *logits, const float *target, const float 
     return ndc::Backend::dice_bce_backward(logits, target, coef, gloss, glogits, (int)rows, n, parts, chunk, stream);
 }
 
+// ---- optimiser step (ndc_adamw.h)
+
+int ndc_adamw(const ndc_adamw_tensor *tensors, int64_t count, double lr, double beta1, double beta2, double eps,
+              double weight_decay, void *stream)
+{
+    if (count < 0 || count > (1 << 24)) return NDC_ERR_GEOMETRY;
+    if (count && !tensors) return NDC_ERR_NULL;
+    for (int64_t i = 0; i < count; ++i) {
+        const ndc_adamw_tensor &t = tensors[i];
+        if (t.n < 0 || t.n > (1LL << 40)) return NDC_ERR_GEOMETRY;
+        if (!t.step || (t.n && (!t.param || !t.grad || !t.m || !t.v))) return NDC_ERR_NULL;
+        if (((uintptr_t)t.param | (uintptr_t)t.grad | (uintptr_t)t.m | (uintptr_t)t.v | (uintptr_t)t.step) & 3u) return NDC_ERR_WORKSPACE;
+    }
+    if (!count) return NDC_OK;
+    return ndc::Backend::adamw(tensors, count, lr, beta1, beta2, eps, weight_decay, stream);
+}
+
 // ---- the tiled GEMMs (ndc_gemm.h)
 
 static int gemm_check(long long batch, long long cin, long long cout, long long n, int dtype)

@@ -15,6 +15,7 @@
 #include "ndc_gemm_host.h"
 #include "ndc_mlp_host.h"
 #include "ndc_loss.h"
+#include "ndc_adamw.h"
 
 #define NDC_LAMBDA __host__ __device__
 
@@ -734,6 +735,35 @@ struct Backend {
     {
         hipLaunchKernelGGL(loss::grad_kernel, dim3((unsigned)(rows * parts)), dim3(loss::kThreads), 0, (hipStream_t)stream, l, y,
                            (const float2 *)coef, g, gl, n, parts, chunk, 1.f / ((float)rows * (float)n));
+        return check();
+    }
+
+    static int adamw(const ndc_adamw_tensor *t, long long count, double lr, double beta1, double beta2, double eps, double decay,
+                     void *stream)
+    {
+        adamw::Params q;
+        q.beta1 = beta1, q.beta2 = beta2, q.lr = lr;
+        q.decay = 1.0 - lr * decay, q.eps = (float)eps;
+        q.count = 0;
+        long long blocks = 0;
+        auto flush = [&] {
+            if (blocks) hipLaunchKernelGGL(adamw::update_kernel, dim3((unsigned)blocks), dim3(adamw::kThreads), 0, (hipStream_t)stream, q);
+            q.count = 0, blocks = 0;
+        };
+        for (long long i = 0; i < count; ++i) {
+            const long long need = (t[i].n + adamw::kChunk - 1) / adamw::kChunk;
+            if (!need) continue;
+            if (q.count == adamw::kTensors || blocks + need > 0x7fffffffLL) flush();
+            q.t[q.count] = t[i], q.first[q.count] = (uint32_t)blocks;
+            ++q.count, blocks += need;
+        }
+        flush();
+        adamw::Steps s;
+        for (long long i = 0; i < count; i += adamw::kSteps) {
+            s.count = (int)(count - i < adamw::kSteps ? count - i : adamw::kSteps);
+            for (int j = 0; j < s.count; ++j) s.step[j] = t[i + j].step;
+            hipLaunchKernelGGL(adamw::count_kernel, dim3((unsigned)((s.count + 63) / 64)), dim3(64), 0, (hipStream_t)stream, s);
+        }
         return check();
     }
 

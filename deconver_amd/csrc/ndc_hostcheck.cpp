@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "ndc_common.h"
+#include "../../include/deconver_ndc.h"
 #include "ndc_exec.h"
 #include "ndc_gemm_host.h"
 #include "ndc_mlp_host.h"
@@ -439,6 +440,8 @@ struct Backend {
         return -2;
     }
 
+    // (elementwise: its oracle is the library's optimiser)
+    static int adamw(const ndc_adamw_tensor *, long long, double, double, double, double, double, void *) { return -2; }
     // (elementwise passes around four sums: their oracle is the loss written in tensor operations)
     static int dice_bce_forward(const float *, const float *, float *, float *, float *, int, long long, int, long long, void *)
     {

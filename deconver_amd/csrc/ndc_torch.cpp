@@ -1239,6 +1239,37 @@ OptTensor dice_bce(const Tensor &l, const Tensor &y)
     return DiceBce::run(l.contiguous(), y.contiguous(), coef, scope.stream);
 }
 
+// ---------------------------------------------------------------------------- optimiser
+
+// One AdamW step in place, or false, with nothing done, where a tensor is not what the kernel takes
+// (dense float32 of one device, the gradient and the moments laid out as the parameter).
+bool adamw(const std::vector<Tensor> &params, const std::vector<Tensor> &grads, const std::vector<Tensor> &m,
+           const std::vector<Tensor> &v, const std::vector<Tensor> &steps, double lr, double beta1, double beta2, double eps,
+           double weight_decay)
+{
+    const size_t count = params.size();
+    if (!count) return true;
+    if (grads.size() != count || m.size() != count || v.size() != count || steps.size() != count) return false;
+    const auto device = params[0].device();
+    const auto plain = [&](const Tensor &t) {
+        return t.defined() && t.device() == device && t.is_cuda() && t.layout() == at::kStrided && t.scalar_type() == at::kFloat &&
+               !t.is_conj() && !t.is_neg() && !t.key_set().has(c10::DispatchKey::Python);
+    };
+    std::vector<ndc_adamw_tensor> list(count);
+    for (size_t i = 0; i < count; ++i) {
+        for (const Tensor *t : {&params[i], &grads[i], &m[i], &v[i]})
+            if (!plain(*t) || !t->is_contiguous() || t->sizes() != params[i].sizes()) return false;
+        if (!plain(steps[i]) || steps[i].numel() != 1) return false;
+    }
+    Scope scope(params[0]);
+    for (size_t i = 0; i < count; ++i) {
+        list[i] = {out_fptr(params[i]), fptr(grads[i]), out_fptr(m[i]), out_fptr(v[i]), out_fptr(steps[i]), params[i].numel()};
+        for (const Tensor *t : {&params[i], &m[i], &v[i], &steps[i]}) t->unsafeGetTensorImpl()->bump_version();
+    }
+    check(ndc_adamw(list.data(), (int64_t)count, lr, beta1, beta2, eps, weight_decay, scope.stream), "ndc_adamw");
+    return true;
+}
+
 // ---------------------------------------------------------------------------- columns
 
 // Column matrix of a contiguous (B, C, *S) tensor for odd kernel extents k: (B, C * taps, voxels).
@@ -1305,4 +1336,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("regroup", &regroup);
     m.def("columns", &columns);
     m.def("dice_bce", &dice_bce);
+    m.def("adamw", &adamw);
 }

@@ -63,17 +63,56 @@ def dice_bce_loss(logits: Tensor, target: Tensor) -> Tensor:
     return bce + (1 - dice).mean()
 
 
+class AdamW(torch.optim.AdamW):
+    """``torch.optim.AdamW`` whose step over float32 parameters on one GPU is the package's kernel
+    (``csrc/ndc_adamw.h``).  State, hooks, schedulers and state dicts are the base class's; what the
+    kernel does not do -- the first step, which makes the state, ``amsgrad``, ``maximize``, tensor
+    learning rates, a gradient scaler's arguments, other types or layouts -- the base class does."""
+
+    def _kernel_step(self) -> bool:
+        if getattr(self, "grad_scale", None) is not None or getattr(self, "found_inf", None) is not None:
+            return False
+        if torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None:
+            return False
+        calls = []
+        for group in self.param_groups:
+            lr, betas = group["lr"], group["betas"]
+            if (not group.get("fused") or group["amsgrad"] or group["maximize"] or group["differentiable"]
+                    or group.get("foreach") or not group.get("decoupled_weight_decay", True)
+                    or isinstance(lr, Tensor) or any(isinstance(b, Tensor) for b in betas)):
+                return False
+            params = [p for p in group["params"] if p.grad is not None]
+            states = [self.state.get(p) for p in params]
+            if not all(states):
+                return False
+            calls.append((params, [p.grad for p in params], [s["exp_avg"] for s in states],
+                          [s["exp_avg_sq"] for s in states], [s["step"] for s in states],
+                          lr, *betas, group["eps"], group["weight_decay"]))
+        # (all or nothing: a second group that is not taken would find the first one's step done)
+        return len(calls) == 1 and _lib.get_native().adamw(*calls[0])
+
+    def step(self, closure=None):
+        if closure is None and not torch.jit.is_tracing():
+            self._cuda_graph_capture_health_check()
+            if self._kernel_step():
+                return None
+        # (the base class's step without the hooks, which belong to this one)
+        base = torch.optim.AdamW.step
+        return (base.__wrapped__ if getattr(base, "hooked", False) else base)(self, closure)
+
+
 def make_optimizer(model: nn.Module, capturable: bool = False) -> torch.optim.Optimizer:
     """AdamW as above; ``capturable`` keeps its step counters on the device, which
     ``GraphedTrainStep`` needs.
 
-    On the GPU the update is the fused form: one pass over parameter, gradient and moments in a
+    On the GPU the update is one pass over parameter, gradient and moments in a
     few launches (28 bytes a parameter), where the default form reads and writes them once per
     operation -- with the step counters on the device in some 280 launches, most of them on one
     counter each.  Parameters on the CPU keep the default form."""
     params = list(model.parameters())
     fused = bool(params) and all(p.is_cuda and p.is_floating_point() for p in params)
-    return torch.optim.AdamW(params, lr=1e-3, weight_decay=1e-2, capturable=capturable, fused=fused or None)
+    kind = AdamW if fused else torch.optim.AdamW
+    return kind(params, lr=1e-3, weight_decay=1e-2, capturable=capturable, fused=fused or None)
 
 
 def _gaussian_blur(t: Tensor, sigma: float) -> Tensor:

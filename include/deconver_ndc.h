@@ -504,6 +504,21 @@ int ndc_dice_bce_forward(const float *logits, const float *target, float *loss, 
 int ndc_dice_bce_backward(const float *logits, const float *target, const float *coef, const float *gloss,
                           float *glogits, int64_t rows, int64_t n, void *stream);
 
+/*
+ * One AdamW step over `count` float32 tensors (the benchmark workloads' optimiser; the reference ships
+ * none): `step` is the tensor's own counter on the device, read as the number of steps before this one
+ * and left one higher.  Tensors of no elements are allowed; no two entries may share memory.
+ */
+typedef struct ndc_adamw_tensor {
+    float *param;
+    const float *grad;
+    float *m, *v;
+    float *step;
+    int64_t n;
+} ndc_adamw_tensor;
+int ndc_adamw(const ndc_adamw_tensor *tensors, int64_t count, double lr, double beta1, double beta2, double eps,
+              double weight_decay, void *stream);
+
 #ifdef __cplusplus
 }
 #endif
