@@ -5,6 +5,7 @@
 
 #include "../../include/deconver_ndc.h"
 #include <stdlib.h>
+#include <string.h>
 
 #include <atomic>
 #include <type_traits>
@@ -320,11 +321,41 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
 // those are what supported() answers for.
 // matrix: the call runs the matrix-instruction family where it covers the geometry (the
 // launch shapes, workspace sizes and table sizes are the same for both families)
-static inline bool make_plan(const KGeom &q, Plan &pl, bool pairs_ok = true, int dtype = NDC_F32,
-                             bool matrix = false)
+static inline bool make_plan_fresh(const KGeom &q, Plan &pl, bool pairs_ok, int dtype, bool matrix)
 {
     if (make_plan_for(q, pl, pairs_ok, dtype, matrix)) return true;
     return pairs_ok && make_plan_for(q, pl, false, dtype, matrix);
+}
+
+// A plan is a function of sizes, and a forward and a backward ask for it some ten times (what is
+// supported, workspace sizes, the launches); the search for a launch shape takes 1-2 us.  Each thread
+// keeps the plans of the last sizes it saw: an update of 64 channels of 32^3 plans for 2 us in all
+// instead of 25, which a small layer waits for.
+static inline bool make_plan(const KGeom &q, Plan &pl, bool pairs_ok = true, int dtype = NDC_F32, bool matrix = false)
+{
+#ifdef NDC_TUNING
+    return make_plan_fresh(q, pl, pairs_ok, dtype, matrix);
+#else
+    static const int kWords = 11, kEntries = 64;
+    const int key[kWords] = {q.B,  q.G,  q.m,  q.sc, q.D, q.H,
+                             q.W, q.kD, q.kH, q.kW, pairs_ok * 4 + matrix * 2 + (dtype == NDC_BF16)};
+    struct Entry {
+        int key[kWords];   // zeros where nothing is kept (a geometry has B >= 1)
+        bool ok;
+        Plan pl;
+    };
+    static thread_local Entry kept[kEntries] = {};
+    unsigned at = 0;
+    for (int k : key) at = at * 31 + (unsigned)k;
+    Entry &e = kept[(at ^ at >> 15) % kEntries];
+    if (memcmp(e.key, key, sizeof(key)) != 0) {
+        e.key[0] = 0;
+        e.ok = make_plan_fresh(q, e.pl, pairs_ok, dtype, matrix);
+        memcpy(e.key, key, sizeof(key));
+    }
+    pl = e.pl;
+    return e.ok;
+#endif
 }
 
 static inline bool supported(const KGeom &q)
