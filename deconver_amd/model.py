@@ -31,10 +31,10 @@ from typing import Any, Optional, Sequence
 import torch
 from torch import Tensor, nn
 
-from . import layers
+from . import _lib, functional, layers
 from .layers import MLP, LayerNorm, Linear
-from .ndc import Deconv
-from .norm import native_norm
+from .ndc import Deconv, Initializer
+from .norm import InstanceNorm1d, InstanceNorm2d, InstanceNorm3d, hip_norm_applies, native_norm
 from .spec import as_tuple, build
 
 __all__ = ["DeconvMixer", "DeconverBlock", "DeconverStage", "Stem", "Deconver"]
@@ -78,6 +78,31 @@ class DeconvMixer(nn.Module):
         return y if residual is None else residual + y
 
 
+_INSTANCE_NORMS = {3: InstanceNorm1d, 4: InstanceNorm2d, 5: InstanceNorm3d}
+
+
+def _stock(module: nn.Module, kind: Optional[type]) -> bool:
+    """Whether a call of ``module`` is ``kind.forward`` and nothing else."""
+    own = module.__dict__
+    return (type(module) is kind and not own["_forward_hooks"] and not own["_forward_pre_hooks"]
+            and not own["_backward_hooks"] and not own["_backward_pre_hooks"] and "forward" not in own
+            and own.get("_compiled_call_impl") is None)
+
+
+def _idle(drop: nn.Module, owner: nn.Module) -> bool:
+    return _stock(drop, nn.Dropout) and (drop.p == 0 or not (drop.training or owner.training))
+
+
+def _weights(linear: Linear):
+    """Weight and bias of a ``Linear`` whose parameters are plain ones, else None."""
+    own = linear._modules
+    conv = own["linear"]
+    if type(conv) is not nn.Conv1d or not _stock(own["flatten"], nn.Flatten):
+        return None
+    own = conv._parameters
+    return None if own.get("weight") is None else (own["weight"], own.get("bias"))
+
+
 class DeconverBlock(nn.Module):
     """Pre-norm residual pair: deconvolution mixer, then channel MLP (deconver.py:49-65)."""
 
@@ -91,11 +116,63 @@ class DeconverBlock(nn.Module):
         self.mlp = MLP(channels, ratio=mlp_ratio, dropout=dropout)
 
     def forward(self, x: Tensor) -> Tensor:
+        done = self._one_call(x)
+        if done is not None:
+            return done
         # (norm(x), x): on the HIP norm the residual's gradient is summed in the norm's backward
         y, x = self._normed(self.norm1, x, self.dcm, self.dcm.in_proj)
         x = self.dcm(y, residual=x)
         y, x = self._normed(self.norm2, x, self.mlp, self.mlp.block[0])
         return self.mlp(y, residual=x)
+
+    def _one_call(self, x: Tensor) -> Optional[Tensor]:
+        """The block as one call of the compiled nodes that its modules' calls come down to, or None
+        unless every module in it is of its stock class, unhooked and takes the HIP route: with an
+        instance norm, one update, the exact GELU, no active dropout.  What is asked here is asked on
+        each call; parameters are read from the modules each time."""
+        if (type(self) is not DeconverBlock or not x.is_cuda or x.dtype not in (torch.float32, torch.bfloat16)
+                or layers._any_global_hook() or torch.jit.is_tracing() or torch.compiler.is_compiling()
+                or torch._C._are_functorch_transforms_active()):
+            return None
+        half = x.dtype == torch.bfloat16
+        if torch.is_autocast_enabled("cuda"):
+            if torch.get_autocast_dtype("cuda") != torch.bfloat16:
+                return None
+            half = True
+        own = self._modules
+        norm1, dcm, norm2, mlp = own["norm1"], own["dcm"], own["norm2"], own["mlp"]
+        kind = _INSTANCE_NORMS.get(x.dim())
+        if not (_stock(norm1, kind) and _stock(norm2, kind) and _stock(dcm, DeconvMixer) and _stock(mlp, MLP)):
+            return None
+        for norm in (norm1, norm2):
+            if norm.affine or norm.track_running_stats or not hip_norm_applies(x):
+                return None
+        own = dcm._modules
+        in_proj, deconv, out_proj, drop = own["in_proj"], own["deconv"], own["out_proj"], own["dropout"]
+        if not (_stock(in_proj, Linear) and _stock(deconv, Deconv) and _stock(own["act"], nn.ReLU) and _stock(out_proj, Linear)
+                and _idle(drop, dcm)):
+            return None
+        inner = mlp._modules["block"]
+        if not _stock(inner, nn.Sequential) or len(inner._modules) != 5:
+            return None
+        first, gelu, drop1, second, drop2 = inner._modules.values()
+        if not (_stock(first, Linear) and _stock(gelu, nn.GELU) and gelu.approximate == "none" and _stock(second, Linear)
+                and _idle(drop1, mlp) and _idle(drop2, mlp)):
+            return None
+        init = deconv._modules["init"]
+        if not (type(init) is Initializer and type(init._modules["linear"]) is Linear and deconv.num_iters == 1
+                and deconv.num_grad_iters >= 1 and len(deconv.kernel_size) == x.dim() - 2 and deconv._regime_allows_hip()):
+            return None
+        if deconv.source_channels >= 16 and deconv.filter_channels >= 4 and not deconv._differentiates(x):
+            return None
+        h0 = init._parameters["h0"]
+        weights = [_weights(m) for m in (in_proj, init._modules["linear"], out_proj, first, second)]
+        if None in weights or h0 is None or h0.dtype != torch.float32:
+            return None
+        (w_in, b_in), (w_source, b_source), (w_out, b_out), (w1, b1), (w2, b2) = weights
+        return _lib.get_native().block(x, half, norm1.eps, norm2.eps, w_in, b_in, h0, w_source, b_source, deconv.groups,
+                                       deconv.filter_channels, deconv.source_channels, deconv.eps, functional._SAVE_RATIO, w_out,
+                                       b_out, w1, b1, w2, b2)
 
     @staticmethod
     def _normed(norm: nn.Module, x: Tensor, consumer: nn.Module, projection: nn.Module):
