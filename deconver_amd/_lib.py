@@ -74,6 +74,9 @@ EXPORTS = (
     "ndc_dice_bce_forward",
     "ndc_dice_bce_backward",
     "ndc_adamw",
+    "ndc_rownorm_stats",
+    "ndc_pointwise_gemm_normed_supported",
+    "ndc_pointwise_gemm_normed",
 )
 
 

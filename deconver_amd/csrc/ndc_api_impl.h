@@ -475,6 +475,23 @@ int ndc_rownorm_forward(const void *x, void *y, float *stats, int64_t rows, int6
                                  chunk, esz, vec, eps, stream);
 }
 
+int ndc_rownorm_stats(const void *x, float *stats, int64_t rows, int64_t n, int dtype, float eps, void *workspace,
+                      size_t workspace_bytes, void *stream)
+{
+    if (!x || !stats || !workspace) return NDC_ERR_NULL;
+    const int st = rownorm_check(rows, n, dtype);
+    if (st) return st;
+    if (!(eps >= 0.f)) return NDC_ERR_GEOMETRY;
+    if (workspace_bytes < ndc_rownorm_workspace_bytes(rows, n) || ((uintptr_t)workspace & 7u) || ((uintptr_t)stats & 7u))
+        return NDC_ERR_WORKSPACE;
+    int nsplit;
+    long long chunk;
+    rownorm_split(rows, n, nsplit, chunk);
+    const int esz = dtype == NDC_BF16 ? 2 : 4;
+    const bool vec = n % (16 / esz) == 0 && aligned16(x);
+    return ndc::Backend::rownorm_stats(x, (float *)workspace, stats, rows, n, nsplit, chunk, esz, vec, eps, stream);
+}
+
 int ndc_rownorm_backward(const void *gy, const void *y, const float *stats, const void *addend, void *gx,
                          int64_t rows, int64_t n, int dtype, void *workspace, size_t workspace_bytes,
                          void *stream)
@@ -597,6 +614,26 @@ int ndc_pointwise_gemm(const void *x, const void *wfrag, const float *bias, cons
                                 stream);
 }
 
+int ndc_pointwise_gemm_normed_supported(int64_t cin, int64_t cout, int64_t n, int act)
+{
+    const bool square = act == NDC_ACT_RELU && cin == cout && (cin == 32 || cin == 64 || cin == 128);
+    const bool hidden = act == NDC_ACT_GELU && cin == 128 && cout == 512;
+    return (square || hidden) && ndc_pointwise_gemm_supported(cin, cout, n, NDC_BF16);
+}
+
+int ndc_pointwise_gemm_normed(const void *x, const float *stats, const void *wfrag, const float *bias, void *y, int64_t batch,
+                              int64_t cin, int64_t cout, int64_t n, int act, int dtype, void *stream)
+{
+    if (!x || !stats || !wfrag || !y) return NDC_ERR_NULL;
+    if (dtype != NDC_BF16) return NDC_ERR_DTYPE;
+    if (batch < 1 || !ndc_pointwise_gemm_normed_supported(cin, cout, n, act)) return NDC_ERR_GEOMETRY;
+    if ((long double)batch * cout * n > 9.0e15L || batch * (n / 64) > 0x7fffff00LL || n > 0x3fffffffLL) return NDC_ERR_GEOMETRY;
+    if (((uintptr_t)x & 3u) || ((uintptr_t)y & 3u) || ((uintptr_t)wfrag & 15u) || ((uintptr_t)bias & 3u) || ((uintptr_t)stats & 15u))
+        return NDC_ERR_WORKSPACE;
+    if (y == x) return NDC_ERR_GEOMETRY;
+    return ndc::Backend::pwgemm_normed(x, stats, wfrag, bias, y, batch, (int)cin, (int)cout, n, act, stream);
+}
+
 int ndc_pointwise_gemm_masked(const void *x, const void *wfrag, const float *bias, const void *residual,
                               const void *mask, void *y, int64_t batch, int64_t cin, int64_t cout, int64_t n,
                               int dtype, void *stream)
@@ -649,17 +686,18 @@ static int mlp_check(int64_t batch, int64_t c, int64_t n, int w_dtype, int dtype
     return NDC_OK;
 }
 
-int ndc_mlp_forward(const void *x, const void *w1, const void *w2, int w_dtype, const float *b1, const float *b2,
+int ndc_mlp_forward(const void *x, const float *stats, const void *w1, const void *w2, int w_dtype, const float *b1, const float *b2,
                     const void *residual, void *y, int64_t batch, int64_t c, int64_t n, int dtype, void *stream)
 {
-    if (!x || !w1 || !w2 || !y) return NDC_ERR_NULL;
+    if (!x || !w1 || !w2 || !y || (stats && !residual)) return NDC_ERR_NULL;
+    if ((uintptr_t)stats & 15u) return NDC_ERR_WORKSPACE;
     const int st = mlp_check(batch, c, n, w_dtype, dtype);
     if (st) return st;
     if (((uintptr_t)x & 3u) || ((uintptr_t)y & 3u) || ((uintptr_t)residual & 3u) || ((uintptr_t)b1 & 3u) || ((uintptr_t)b2 & 3u) ||
         ((uintptr_t)w1 & 3u) || ((uintptr_t)w2 & 3u))
         return NDC_ERR_WORKSPACE;
     if (y == x) return NDC_ERR_GEOMETRY;
-    return ndc::Backend::mlp_forward(x, w1, w2, w_dtype == NDC_BF16, b1, b2, residual, y, batch, (int)c, n, stream);
+    return ndc::Backend::mlp_forward(x, stats, w1, w2, w_dtype == NDC_BF16, b1, b2, residual, y, batch, (int)c, n, stream);
 }
 
 size_t ndc_mlp_workspace_bytes(int64_t batch, int64_t c, int64_t n)

@@ -333,6 +333,24 @@ struct Backend {
                                (float2 *)stats, (T *)out, sp, eps);
     }
 
+    // (mean, rstd) of every row
+    static int rownorm_stats(const void *x, float *partial, float *stats, long long rows, long long n, int nsplit, long long chunk,
+                             int esz, bool vec, float eps, void *stream)
+    {
+        using namespace rownorm;
+        Split sp;
+        sp.n = n, sp.nsplit = nsplit, sp.chunk = chunk;
+        const dim3 grid((unsigned)(rows * nsplit)), block(kThreads);
+        auto reduce = [&](auto kernel, auto *p) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, p, (decltype(p))nullptr, (float2 *)partial, sp);
+        };
+        if (esz == 2) vec ? reduce(reduce_kernel<bf16_t, false, true>, (const bf16_t *)x) : reduce(reduce_kernel<bf16_t, false, false>, (const bf16_t *)x);
+        else vec ? reduce(reduce_kernel<float, false, true>, (const float *)x) : reduce(reduce_kernel<float, false, false>, (const float *)x);
+        hipLaunchKernelGGL(stats_kernel, dim3((unsigned)((rows + kThreads - 1) / kThreads)), block, 0, (hipStream_t)stream,
+                           (const float2 *)partial, (float2 *)stats, rows, sp, eps);
+        return check();
+    }
+
     // Row normalisation, one direction: reduce launch then apply launch on rows * nsplit
     // workgroups.  Forward: a = x, out = y, stats written; backward: a = gy, b = y, stats read,
     // out = gx (+ addend, if given).  `vec`: n is a multiple of 16 bytes of elements and every
@@ -560,10 +578,10 @@ struct Backend {
 
     // persistent workgroups: as many as are resident at once (asked of the runtime once per
     // kernel and LDS size), so that every wavefront walks the same number of tiles
-    template <int CIN, int ACT, bool RES, int THREADS>
+    template <int CIN, int ACT, bool RES, int THREADS, bool NORM = false>
     static int pwgemm_launch(const pwgemm::Params &p, size_t lds, void *stream)
     {
-        void (*entry)(pwgemm::Params) = pwgemm::gemm_kernel<CIN, ACT, RES, THREADS>;
+        void (*entry)(pwgemm::Params) = pwgemm::gemm_kernel<CIN, ACT, RES, THREADS, NORM>;
         static std::atomic<int> resident[3] = {{0}, {0}, {0}};   // by LDS size class
         const int cls = lds <= 40 * 1024 ? 0 : lds <= 80 * 1024 ? 1 : 2;
         int per_cu = resident[cls].load(std::memory_order_relaxed);
@@ -661,7 +679,7 @@ struct Backend {
                       float *gpart, const void *mask, long long batch, int cin, int cout, long long n, int act,
                       void *stream)
     {
-        pwgemm::Params p;
+        pwgemm::Params p = {};
         p.gpart = gpart;
         p.mask = (const uint16_t *)mask;
         p.x = (const uint16_t *)x, p.wfrag = (const uint16_t *)wfrag, p.bias = bias;
@@ -693,6 +711,20 @@ struct Backend {
 #undef NDC_PWGEMM
     }
 
+    // y = act(W normalised(x) + bias): the forms a block has (the caller has checked them)
+    static int pwgemm_normed(const void *x, const float *stats, const void *wfrag, const float *bias, void *y, long long batch,
+                             int cin, int cout, long long n, int act, void *stream)
+    {
+        pwgemm::Params p = {};
+        p.x = (const uint16_t *)x, p.wfrag = (const uint16_t *)wfrag, p.bias = bias, p.y = (uint16_t *)y, p.stats = stats;
+        p.n = n, p.tiles_per_sample = (int)(n / pwgemm::kTileVoxels), p.tiles = (int)(batch * (n / pwgemm::kTileVoxels)), p.cout = cout;
+        const size_t lds = (size_t)cin * cout * 2 + (size_t)cout * 4;
+        if (act == epilogue::kGelu) return pwgemm_launch<128, epilogue::kGelu, false, 1024, true>(p, lds, stream);
+        if (cin == 32) return pwgemm_launch<32, epilogue::kRelu, false, 256, true>(p, lds, stream);
+        if (cin == 64) return pwgemm_launch<64, epilogue::kRelu, false, 256, true>(p, lds, stream);
+        return pwgemm_launch<128, epilogue::kRelu, false, 256, true>(p, lds, stream);
+    }
+
     static int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long long batch, int rows, int cols,
                      long long n, int esz, const WgradPlan &plan, void *stream)
     {
@@ -707,10 +739,10 @@ struct Backend {
         return st ? st : check();
     }
 
-    static int mlp_forward(const void *x, const void *w1, const void *w2, int w_is_bf16, const float *b1, const float *b2,
-                           const void *res, void *y, long long batch, int c, long long n, void *stream)
+    static int mlp_forward(const void *x, const float *stats, const void *w1, const void *w2, int w_is_bf16, const float *b1,
+                           const float *b2, const void *res, void *y, long long batch, int c, long long n, void *stream)
     {
-        const int st = mlp::forward(x, w1, w2, w_is_bf16, b1, b2, res, y, batch, c, n, stream);
+        const int st = mlp::forward(x, stats, w1, w2, w_is_bf16, b1, b2, res, y, batch, c, n, stream);
         return st ? st : check();
     }
     static int mlp_backward(const void *x, const void *gy, const void *w1, const void *w2, int w_is_bf16, const float *b1,

@@ -429,7 +429,15 @@ struct Backend {
                 }
     }
     // (kernels of matrix instructions throughout, without a sequential form)
-    static int mlp_forward(const void *, const void *, const void *, int, const float *, const float *, const void *, void *,
+    static int rownorm_stats(const void *, float *, float *, long long, long long, int, long long, int, bool, float, void *)
+    {
+        return -2;
+    }
+    static int pwgemm_normed(const void *, const float *, const void *, const float *, void *, long long, int, int, long long, int, void *)
+    {
+        return -2;
+    }
+    static int mlp_forward(const void *, const float *, const void *, const void *, int, const float *, const float *, const void *, void *,
                            long long, int, long long, void *)
     {
         return -2;

@@ -29,6 +29,7 @@
 #include "ndc_common.h"
 #include "ndc_epilogue.h"
 #include "ndc_mlp_host.h"
+#include "ndc_pwgemm.h"
 
 namespace ndc {
 namespace mlp {
@@ -40,6 +41,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct Params {
     const uint16_t *x, *gy, *res;   // (B, C, n)
+    const float *stats;             // NORM: (mean, 1 / deviation) of each row of x
     const void *w1, *w2;
     const float *b1, *b2;           // 4C and C values, or null
     uint16_t *y;                    // forward: y; backward: gx
@@ -98,7 +100,8 @@ __device__ inline uint32_t *words(uint16_t *p) { return reinterpret_cast<uint32_
 // C = 64), packed by the workgroup itself from the float32 matrices (twice 64 KB that the L2 holds;
 // a packing launch each costs more).  Workgroups are persistent, twelve wavefronts at C = 64: three per
 // SIMD is what the 168 registers of a wavefront leave.
-template <int C, typename TW, bool RES, int THREADS>
+// NORM: x is normalised as it is loaded, and the residual is the x before that.
+template <int C, typename TW, bool RES, int THREADS, bool NORM>
 __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
 {
     constexpr int H = 4 * C, S = C / 16, HT = H / 32, OT = C / 32, WAVES = THREADS / 64;
@@ -133,6 +136,7 @@ __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) raw[s][e] = words(p.x + at0 + (long long)(16 * s + e) * p.n)[xw];
+            if constexpr (NORM) pwgemm::normalise_words<S>(raw, p.stats + 2 * (long long)b * C, kb);
 #pragma unroll
             for (int s = 0; s < S; ++s) split_words(raw[s], xf[s][0], xf[s][1]);
         }

@@ -17,8 +17,10 @@ static Params params(const void *x, const void *w1, const void *w2, const float 
 template <int C, typename TW, int THREADS> static void forward_launch_t(const Params &p, int per_cu, void *stream)
 {
     const int need = (p.tiles + THREADS / 64 - 1) / (THREADS / 64), blocks = need < 256 * per_cu ? need : 256 * per_cu;
-    if (p.res) hipLaunchKernelGGL((forward_kernel<C, TW, true, THREADS>), dim3(blocks), dim3(THREADS), 0, (hipStream_t)stream, p);
-    else hipLaunchKernelGGL((forward_kernel<C, TW, false, THREADS>), dim3(blocks), dim3(THREADS), 0, (hipStream_t)stream, p);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(THREADS), 0, (hipStream_t)stream, p); };
+    if (p.stats) launch(forward_kernel<C, TW, true, THREADS, true>);
+    else if (p.res) launch(forward_kernel<C, TW, true, THREADS, false>);
+    else launch(forward_kernel<C, TW, false, THREADS, false>);
 }
 // A tile keeps its SIMD's vector unit busy for about 10 us at C = 64 (a third of that at 32), so few tiles go
 // to workgroups small enough to reach all CUs: with twelve wavefronts each, 512 tiles ran 36 us on 43 CUs.
@@ -30,11 +32,11 @@ template <int C, typename TW> static void forward_launch(const Params &p, void *
     else forward_launch_t<C, TW, 768>(p, 1, stream);
 }
 
-int forward(const void *x, const void *w1, const void *w2, int w_is_bf16, const float *b1, const float *b2, const void *res,
-            void *y, long long batch, int c, long long n, void *stream)
+int forward(const void *x, const float *stats, const void *w1, const void *w2, int w_is_bf16, const float *b1, const float *b2,
+            const void *res, void *y, long long batch, int c, long long n, void *stream)
 {
     Params p = params(x, w1, w2, b1, y, batch, n);
-    p.b2 = b2, p.res = (const uint16_t *)res;
+    p.b2 = b2, p.res = (const uint16_t *)res, p.stats = stats;
     if (c == 64) {
         if (w_is_bf16) forward_launch<64, bf16_t>(p, stream);
         else forward_launch<64, float>(p, stream);

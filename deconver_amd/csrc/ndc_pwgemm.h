@@ -68,6 +68,7 @@ struct Params {
     uint16_t *zkeep;         // (B, cout, n) or null: the product before bias and activation
     float *gpart;            // gradient modes: (gridDim.x * waves, cout) sums of y per wavefront, or null
     const uint16_t *mask;    // kMasked: (B, cout, n)
+    const float *stats;      // NORM: (mean, 1 / deviation) of each row of x, (B, cin) pairs
     long long n;             // voxels per sample, a multiple of 64
     int tiles;               // B * n / 64
     int tiles_per_sample;
@@ -164,7 +165,25 @@ __device__ inline void finish_tile(const Params &p, const f32x16 &acc0, const f3
     }
 }
 
-template <int CIN, int ACT, bool RES, int THREADS>
+// The words of a tile normalised, (x - mean) / deviation rounded to bf16 as the row norm's own pass rounds it.
+// stats: the sample's first pair; a lane holds channels 16 s + 8 kb + e.
+template <int S> __device__ inline void normalise_words(uint32_t (&raw)[S][8], const float *stats, int kb)
+{
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const float4 *at = reinterpret_cast<const float4 *>(stats + 2 * (16 * s + 8 * kb));
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            const float4 t = at[e / 2];
+            raw[s][e] = pack_bf16x2((lo_bf16(raw[s][e]) - t.x) * t.y, (hi_bf16(raw[s][e]) - t.x) * t.y);
+            raw[s][e + 1] = pack_bf16x2((lo_bf16(raw[s][e + 1]) - t.z) * t.w, (hi_bf16(raw[s][e + 1]) - t.z) * t.w);
+        }
+    }
+}
+
+// NORM: x is normalised by its rows' statistics as it is loaded.  A norm ahead of a projection is then one
+// pass that reads x instead of one more that reads and writes it.
+template <int CIN, int ACT, bool RES, int THREADS, bool NORM>
 __global__ void __launch_bounds__(THREADS) gemm_kernel(Params p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -202,6 +221,7 @@ __global__ void __launch_bounds__(THREADS) gemm_kernel(Params p)
         {
             uint32_t raw[S][8];
             request_x<S>(p, tile, CIN, xw, raw);
+            if constexpr (NORM) normalise_words<S>(raw, p.stats + 2 * (long long)b * CIN, kb);
             split_x<S>(raw, xf);
         }
         // ---- one 32-channel output tile after the other.  Register j of a lane holds output

@@ -230,6 +230,30 @@ row_sums_kernel(const T *a, float *partial, Split sp)
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// (mean, 1 / sqrt(variance + eps)) of a row: (count, mean, squared deviations) of the parts merged in order
+__device__ inline float2 merge_parts(const float2 *partial, const Split &sp, float eps)
+{
+    float cnt = 0.f, mean = 0.f, m2 = 0.f;
+    for (int p = 0; p < sp.nsplit; ++p) {
+        const float2 q = partial[p];
+        const long long plo = p * sp.chunk, phi = plo + sp.chunk < sp.n ? plo + sp.chunk : sp.n;
+        const float np = (float)(phi - plo), tot = cnt + np, delta = q.x - mean;
+        mean += delta * (np / tot);
+        m2 += q.y + delta * delta * (cnt * np / tot);
+        cnt = tot;
+    }
+    float var = m2 * (1.f / (float)sp.n);
+    var = var > 0.f ? var : 0.f;
+    return make_float2(mean, 1.f / sqrtf(var + eps));
+}
+
+// the statistics alone, a thread a row, for a consumer that normalises what it loads
+static __global__ void __launch_bounds__(kThreads) stats_kernel(const float2 *partial, float2 *stats, long long rows, Split sp, float eps)
+{
+    const long long row = (long long)blockIdx.x * kThreads + threadIdx.x;
+    if (row < rows) stats[row] = merge_parts(partial + row * sp.nsplit, sp, eps);
+}
+
 template <typename T, bool BWD, bool VEC, bool ADD = false>
 __global__ void __launch_bounds__(kThreads)
 apply_kernel(const T *a, const T *b, const T *addend, const float2 *partial, float2 *stats, T *out, Split sp,
@@ -253,22 +277,10 @@ apply_kernel(const T *a, const T *b, const T *addend, const float2 *partial, flo
         c0 = -rstd * s1 * inv_n;
         c2 = -rstd * s2 * inv_n;
     } else {
-        // (count, mean, squared deviations) of the parts merged in order, by every thread
-        float cnt = 0.f, mean = 0.f, m2 = 0.f;
-        for (int p = 0; p < sp.nsplit; ++p) {
-            const float2 q = partial[row * sp.nsplit + p];
-            const long long plo = p * sp.chunk, phi = plo + sp.chunk < sp.n ? plo + sp.chunk : sp.n;
-            const float np = (float)(phi - plo), tot = cnt + np, delta = q.x - mean;
-            mean += delta * (np / tot);
-            m2 += q.y + delta * delta * (cnt * np / tot);
-            cnt = tot;
-        }
-        float var = m2 * inv_n;
-        var = var > 0.f ? var : 0.f;
-        const float rstd = 1.f / sqrtf(var + eps);
-        c1 = rstd;
-        c0 = mean;
-        if (part == 0 && threadIdx.x == 0) stats[row] = make_float2(mean, rstd);
+        const float2 s = merge_parts(partial + row * sp.nsplit, sp, eps);   // (by every thread)
+        c1 = s.y;
+        c0 = s.x;
+        if (part == 0 && threadIdx.x == 0) stats[row] = s;
     }
     if constexpr (VEC) {
         typedef Vec<T> V;

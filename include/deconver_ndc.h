@@ -279,6 +279,10 @@ int ndc_relayout(const void *src, void *dst, int64_t batch, int64_t channels, in
 size_t ndc_rownorm_workspace_bytes(int64_t rows, int64_t n);
 int ndc_rownorm_forward(const void *x, void *y, float *stats, int64_t rows, int64_t n, int dtype,
                         float eps, void *workspace, size_t workspace_bytes, void *stream);
+/* the statistics alone, 2 * rows floats, for a consumer that normalises what it reads (of rows beyond 192 KB
+ * the same bits as the norm's) */
+int ndc_rownorm_stats(const void *x, float *stats, int64_t rows, int64_t n, int dtype, float eps, void *workspace,
+                      size_t workspace_bytes, void *stream);
 int ndc_rownorm_backward(const void *gy, const void *y, const float *stats, const void *addend, void *gx,
                          int64_t rows, int64_t n, int dtype, void *workspace, size_t workspace_bytes,
                          void *stream);
@@ -344,6 +348,16 @@ int ndc_pointwise_pack(const void *w, int w_dtype, int transposed, void *wfrag, 
 int ndc_pointwise_gemm(const void *x, const void *wfrag, const float *bias, const void *residual, void *y,
                        void *zkeep, int64_t batch, int64_t cin, int64_t cout, int64_t n, int act, int dtype,
                        void *stream);
+/*
+ * y = act(W xn + bias) where xn is x normalised by `stats`, (batch, cin) pairs of mean and 1 / deviation
+ * (ndc_rownorm_stats, 16-byte aligned), and rounded to bfloat16: the row norm ahead of a projection
+ * (deconver/deconver.py:60-64) without a pass of its own.  ndc_pointwise_gemm_normed_supported: 1 for the
+ * projections of a block, cin == cout of 32, 64 or 128 with NDC_ACT_RELU and 128 -> 512 with NDC_ACT_GELU.
+ */
+int ndc_pointwise_gemm_normed_supported(int64_t cin, int64_t cout, int64_t n, int act);
+int ndc_pointwise_gemm_normed(const void *x, const float *stats, const void *wfrag, const float *bias, void *y, int64_t batch,
+                              int64_t cin, int64_t cout, int64_t n, int act, int dtype, void *stream);
+
 /*
  * ndc_pointwise_gemm_masked: y = (W x + bias + residual) where mask > 0, else 0; mask of y's shape.
  * The input gradient of a projection whose input is a rectifier's output (mask), with another
@@ -475,14 +489,16 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
  *   w1, w2      as they lie, both of dtype w_dtype (NDC_F32 or NDC_BF16); rounded to bfloat16 for the
  *               products
  *   b1, b2      float32 or NULL; residual: y's shape, or NULL; y may be residual
+ *   stats       NULL, or the (mean, 1 / deviation) pairs of the rows of x (ndc_rownorm_stats, 16-byte
+ *               aligned): the MLP is then of the normalised x; residual is not NULL
  *   gw1, gw2    float32, shapes of W1 and W2; gb1, gb2 float32, or NULL; gb1 is summed before the
  *               hidden tensor's gradient is rounded
  *   workspace   ndc_mlp_workspace_bytes(batch, c, n) bytes, 16-byte aligned
  *   x, gy, gx   16-byte aligned for the backward, word-aligned for the forward; gx is neither x nor gy
  */
 int ndc_mlp_supported(int64_t c, int64_t n, int dtype);
-int ndc_mlp_forward(const void *x, const void *w1, const void *w2, int w_dtype, const float *b1, const float *b2,
-                    const void *residual, void *y, int64_t batch, int64_t c, int64_t n, int dtype, void *stream);
+int ndc_mlp_forward(const void *x, const float *stats, const void *w1, const void *w2, int w_dtype, const float *b1,
+                    const float *b2, const void *residual, void *y, int64_t batch, int64_t c, int64_t n, int dtype, void *stream);
 size_t ndc_mlp_workspace_bytes(int64_t batch, int64_t c, int64_t n);
 int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *w2, int w_dtype, const float *b1,
                      void *gx, float *gw1, float *gb1, float *gw2, float *gb2, int64_t batch, int64_t c, int64_t n,

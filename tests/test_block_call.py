@@ -37,7 +37,11 @@ def _run(block, x, autocast, one_call):
 @pytest.mark.parametrize("nd,channels,size,batch,dtype,autocast", [
     (2, 32, (20, 28), 2, torch.float32, False), (1, 8, (30,), 1, torch.float32, False), (3, 6, (5, 7, 9), 1, torch.float32, False),
     (3, 32, (8, 16, 16), 1, torch.bfloat16, False), (3, 32, (8, 12, 13), 2, torch.float32, True),
-    (3, 64, (32, 32, 32), 1, torch.bfloat16, True), (2, 16, (9, 11), 2, torch.bfloat16, False)])
+    (3, 64, (32, 32, 32), 1, torch.bfloat16, True),
+    # (where no backward follows the norms fold into the projections: from rows of 98 305 voxels)
+    (3, 64, (44, 48, 48), 2, torch.bfloat16, False), (3, 64, (48, 64, 32), 1, torch.bfloat16, False), (3, 64, (48, 48, 60), 1, torch.float32, True), (3, 32, (64, 40, 52), 1, torch.bfloat16, False),
+    (3, 128, (52, 40, 64), 1, torch.bfloat16, False), (3, 32, (50, 46, 43), 2, torch.bfloat16, False),
+    (3, 64, (48, 52, 56), 1, torch.bfloat16, True), (2, 16, (9, 11), 2, torch.bfloat16, False)])
 def test_same_values(nd, channels, size, batch, dtype, autocast):
     print(nd, channels, size, batch, dtype, autocast, flush=True)
     block = _block(nd, channels)
