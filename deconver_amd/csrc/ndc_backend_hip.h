@@ -15,6 +15,7 @@
 #include "ndc_gemm_host.h"
 #include "ndc_mlp_host.h"
 #include "ndc_loss.h"
+#include "ndc_direct.h"
 #include "ndc_adamw.h"
 
 #define NDC_LAMBDA __host__ __device__
@@ -36,6 +37,20 @@ __global__ void __launch_bounds__(128) per_unit_kernel(unsigned blocks, long lon
     const unsigned u = blockIdx.x / blocks;
     const long long pos = (long long)(blockIdx.x - u * blocks) * 128 + threadIdx.x;
     if (pos < npos) f((int)u, pos);
+}
+
+// f.run(unit, position, weights): ... with the unit's weights in LDS
+template <class F, bool STAGED>
+__global__ void __launch_bounds__(128) weighted_unit_kernel(unsigned blocks, long long npos, F f)
+{
+    extern __shared__ __attribute__((aligned(16))) float weights[];
+    const unsigned u = blockIdx.x / blocks;
+    const long long pos = (long long)(blockIdx.x - u * blocks) * 128 + threadIdx.x;
+    if constexpr (STAGED) {
+        f.stage((int)u, weights, threadIdx.x, 128);
+        __syncthreads();
+    }
+    if (pos < npos) f.template run<STAGED>((int)u, pos, weights);
 }
 
 // F::N sums over the threads of a workgroup, one workgroup per unit: f.sums gives a thread's
@@ -815,6 +830,20 @@ struct Backend {
         if (blocks > 0x7fffffffLL / units) return -2;
         hipLaunchKernelGGL(per_unit_kernel<F>, dim3((unsigned)(units * blocks)), dim3(128), 0, (hipStream_t)stream,
                            (unsigned)blocks, npos, f);
+        return check();
+    }
+
+    template <class F> static int weighted_unit(long long units, long long npos, void *stream, F f)
+    {
+        const long long blocks = (npos + 127) / 128;
+        if (units <= 0 || npos <= 0) return 0;
+        if (blocks > 0x7fffffffLL / units) return -2;
+        const dim3 grid((unsigned)(units * blocks)), block(128);
+        const int n = f.weights();
+        if (F::Weights::staged(n, units * blocks * 2))
+            hipLaunchKernelGGL((weighted_unit_kernel<F, true>), grid, block, (size_t)n * 4, (hipStream_t)stream, (unsigned)blocks, npos, f);
+        else
+            hipLaunchKernelGGL((weighted_unit_kernel<F, false>), grid, block, 0, (hipStream_t)stream, (unsigned)blocks, npos, f);
         return check();
     }
 

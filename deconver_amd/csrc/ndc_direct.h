@@ -7,19 +7,24 @@
 //
 // A thread owns one position of one (sample, group) and a block of NB output channels; lanes run
 // along the positions.  A value of a neighbour is loaded once and used for all NB channels, its
-// weights are the same in every lane and come through the scalar unit, and the window's address
+// weights are the same in every lane and come through the scalar unit or, where a launch has the
+// wavefronts (Weights::staged), from a copy in LDS in the order they are used -- each channel's few
+// adjacent weights are a short scalar load of their own, and the scalar cache, which two CUs share,
+// was what large launches waited for --, and the window's address
 // and bounds are formed once per tap row and serve every input channel.  One thread per output
 // element, which this replaces, repeated each load, its 64-bit address and its bounds branch for
 // every output channel.  The filter gradient holds MB x SB x KWB sums (filter channels x source
 // channels x taps of a row) and walks the positions, so that each load feeds three products; one
 // workgroup per single sum loaded two values a product and read the volume m*sc*taps times.
 // What bounds these kernels now is the load path of the CU (a 4-byte load of a wavefront takes
-// four clocks, as a multiply-add of its four SIMDs does); the volumes they serve fit the L2.
+// four clocks, as a multiply-add of its four SIMDs does) and, in small launches, the weights'
+// latency; the volumes they serve fit the L2.
 // Measured (4 groups of 4 filter and 8 source channels, 3x3x3, 2 x 24^3, float32): t1 94 -> 35 us,
 // the forward's ratio 89 -> 25, gn and gd 65 -> 26, gx and gt1 145 -> 26, gh 419 -> 41, gz 151 -> 36,
 // gb 41 -> 5; the layer, forward + backward, 1036 -> 236 us.
 #pragma once
 
+#include "../../include/deconver_ndc.h"
 #include "ndc_common.h"
 
 namespace ndc {
@@ -75,14 +80,74 @@ template <int SIGN, int KWB, typename OFF> struct Window {
     }
 };
 
+// The weights that output channels c0 .. c0 + NB of a group take, in the order accumulate() takes them:
+// [taps by KWB][input channel][output channel][KWB].  A workgroup puts them into LDS where they fit.
+static const int kStagedWeights = 4096;
+template <bool ADJ, int NB, int KWB> struct Weights {
+    // Whether a launch of so many wavefronts takes n weights from LDS (16 KB at most).  us, scalar unit -> LDS,
+    // float32: forwards of 2 groups of 4 -> 16 channels on 64^3 273 -> 161, 8 of 1 -> 8 on 48^3 150 -> 98, 8 of
+    // 1 -> 4 with 7x7 taps on 8 x 128^2 276 -> 216.  With few wavefronts the copy and the LDS's latency show:
+    // A of 4 -> 8 channels on 2 x 24^3 (3456 wavefronts of 4 outputs) 25 -> 34, K 35 -> 31; both of 16 -> 16 on
+    // 24^3 (1728 wavefronts) 73 -> 121.
+    static bool staged(int n, long long waves)
+    {
+        return n <= kStagedWeights && (ADJ ? waves * NB >= 24 * 1024 : waves >= 3 * 1024);
+    }
+    static NDC_HD int count(const KGeom &q) { return (ADJ ? q.m : q.sc) * NB * q.KT; }
+    // the NB x KWB weights of every `step`-th pair (taps, input channel)
+    static NDC_HD void stage(const KGeom &q, const float *hf, int g, int c0, float *to, int first, int step)
+    {
+        const int cin = ADJ ? q.m : q.sc, cout = ADJ ? q.sc : q.m, pairs = q.KT / KWB * cin;
+        const float *hg = hf + (long long)g * q.m * q.sc * q.KT;
+        for (int r = first; r < pairs; r += step) {
+            const int t = r / cin, ci = r - t * cin;
+            float v[NB * KWB];
+#pragma unroll
+            for (int c = 0; c < NB; ++c) {
+                const int k = c0 + c < cout ? c0 + c : cout - 1;
+#pragma unroll
+                for (int j = 0; j < KWB; ++j) v[c * KWB + j] = hg[((ADJ ? ci : k) * q.sc + (ADJ ? k : ci)) * q.KT + t * KWB + j];
+            }
+#pragma unroll
+            for (int i = 0; i < NB * KWB; ++i) to[r * NB * KWB + i] = v[i];
+        }
+    }
+};
+
 // acc[k][c] += the sums of K (ADJ = false, outputs: the m channels) or A (ADJ = true, outputs: the
 // sc channels) at one position for output channels c0 .. c0 + NB of group g and NIN inputs at once.
 // load(k, channel, window, v): the window of input k.  Channels past the last repeat the last.
-template <bool ADJ, int NB, int KWB, int NIN, typename OFF, class Load>
-NDC_HD void accumulate(const KGeom &q, const float *hf, int g, int c0, const Pos<OFF> &p,
+// STAGED: staged holds the weights as Weights has them.
+template <bool ADJ, int NB, int KWB, int NIN, bool STAGED, typename OFF, class Load>
+NDC_HD void accumulate(const KGeom &q, const float *hf, const float *staged, int g, int c0, const Pos<OFF> &p,
                        float (&acc)[NIN][NB], Load load)
 {
     const int cin = ADJ ? q.m : q.sc, cout = ADJ ? q.sc : q.m;
+    if constexpr (STAGED) {
+#pragma unroll
+        for (int k = 0; k < NIN; ++k)
+#pragma unroll
+            for (int c = 0; c < NB; ++c) acc[k][c] = 0.f;
+        const float *w = staged;
+        for (int td = 0; td < q.kD; ++td)
+            for (int th = 0; th < q.kH; ++th)
+                for (int tw0 = 0; tw0 < q.kW; tw0 += KWB) {
+                    const Window<ADJ ? -1 : 1, KWB, OFF> win(q, p, td, th, tw0);
+#pragma unroll 2
+                    for (int ci = 0; ci < cin; ++ci, w += NB * KWB) {
+                        float v[NIN][KWB];
+#pragma unroll
+                        for (int k = 0; k < NIN; ++k) load(k, ci, win, v[k]);
+#pragma unroll
+                        for (int c = 0; c < NB; ++c)
+#pragma unroll
+                            for (int j = 0; j < KWB; ++j)
+#pragma unroll
+                                for (int k = 0; k < NIN; ++k) acc[k][c] += v[k][j] * w[c * KWB + j];
+                    }
+                }
+        return;
+    }
     const UniformF hg = as_uniform(hf + (long long)g * q.m * q.sc * q.KT);
     int chan[NB];
 #pragma unroll
@@ -146,7 +211,14 @@ template <typename TI, typename TO, bool ADJ, int NB, int KWB, typename OFF> str
     int rectify;
     TO *out;
     int blocks;
-    NDC_HD void operator()(int u, long long pos) const
+    typedef direct::Weights<ADJ, NB, KWB> Weights;
+    NDC_HD int weights() const { return Weights::count(q); }
+    NDC_HD void stage(int u, float *to, int first, int step) const
+    {
+        const Unit t(u, q.G, blocks, NB);
+        Weights::stage(q, hf, t.g, t.c0, to, first, step);
+    }
+    template <bool STAGED> NDC_HD void run(int u, long long pos, const float *staged) const
     {
         const Unit t(u, q.G, blocks, NB);
         const int cin = ADJ ? q.m : q.sc, cout = ADJ ? q.sc : q.m;
@@ -154,8 +226,8 @@ template <typename TI, typename TO, bool ADJ, int NB, int KWB, typename OFF> str
         const long long bg = (long long)t.b * q.G + t.g;
         const TI *ig = in + bg * cin * q.SP;
         float acc[1][NB];
-        accumulate<ADJ, NB, KWB, 1, OFF>(q, hf, t.g, t.c0, p, acc,
-                                         [&](int, int ci, const Window<ADJ ? -1 : 1, KWB, OFF> &win, float (&v)[KWB]) {
+        accumulate<ADJ, NB, KWB, 1, STAGED, OFF>(q, hf, staged, t.g, t.c0, p, acc,
+                                                 [&](int, int ci, const Window<ADJ ? -1 : 1, KWB, OFF> &win, float (&v)[KWB]) {
             win.template load<TI>(ig + ci * q.SP, v);
             if (!rectify) return;
             const float bv = bias ? bias[t.g * cin + ci] : 0.f;
@@ -175,14 +247,21 @@ template <typename T, int NB, int KWB, typename OFF> struct GradPair {
     T *gx;
     float *gt1;
     int blocks;
-    NDC_HD void operator()(int u, long long pos) const
+    typedef direct::Weights<false, NB, KWB> Weights;
+    NDC_HD int weights() const { return Weights::count(q); }
+    NDC_HD void stage(int u, float *to, int first, int step) const
+    {
+        const Unit t(u, q.G, blocks, NB);
+        Weights::stage(q, hf, t.g, t.c0, to, first, step);
+    }
+    template <bool STAGED> NDC_HD void run(int u, long long pos, const float *staged) const
     {
         const Unit t(u, q.G, blocks, NB);
         const Pos<OFF> p = position<OFF>(q, (OFF)pos);
         const long long bg = (long long)t.b * q.G + t.g, base = bg * q.sc * q.SP;
         float acc[2][NB];
-        accumulate<false, NB, KWB, 2, OFF>(q, hf, t.g, t.c0, p, acc,
-                                           [&](int k, int ci, const Window<1, KWB, OFF> &win, float (&v)[KWB]) {
+        accumulate<false, NB, KWB, 2, STAGED, OFF>(q, hf, staged, t.g, t.c0, p, acc,
+                                                   [&](int k, int ci, const Window<1, KWB, OFF> &win, float (&v)[KWB]) {
             win.template load<float>((k ? gd : gn) + base + ci * q.SP, v);
         });
 #pragma unroll
@@ -209,15 +288,22 @@ template <typename T, int STAGE, int NB, int KWB, typename OFF> struct Ratio {
     T *out, *s_over_den, *ratio;    // FWD; SOURCE writes gz to `out`
     float *gn, *gd;                 // GRAD
     int blocks;
-    NDC_HD void operator()(int u, long long pos) const
+    typedef direct::Weights<true, NB, KWB> Weights;
+    NDC_HD int weights() const { return Weights::count(q); }
+    NDC_HD void stage(int u, float *to, int first, int step) const
+    {
+        const Unit t(u, q.G, blocks, NB);
+        Weights::stage(q, hf, t.g, t.c0, to, first, step);
+    }
+    template <bool STAGED> NDC_HD void run(int u, long long pos, const float *staged) const
     {
         const Unit t(u, q.G, blocks, NB);
         const Pos<OFF> p = position<OFF>(q, (OFF)pos);
         const long long bg = (long long)t.b * q.G + t.g, base = bg * q.m * q.SP;
         constexpr int NIN = STAGE == SOURCE ? 3 : 2;
         float acc[NIN][NB];
-        accumulate<true, NB, KWB, NIN, OFF>(q, hf, t.g, t.c0, p, acc,
-                                            [&](int k, int ci, const Window<-1, KWB, OFF> &win, float (&v)[KWB]) {
+        accumulate<true, NB, KWB, NIN, STAGED, OFF>(q, hf, staged, t.g, t.c0, p, acc,
+                                                    [&](int k, int ci, const Window<-1, KWB, OFF> &win, float (&v)[KWB]) {
             const long long at = base + ci * q.SP;
             if (k == 2) win.template load<float>(gt1 + at, v);
             else win.template load<T>((k ? t1 : x) + at, v);

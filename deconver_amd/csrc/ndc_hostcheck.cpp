@@ -8,6 +8,7 @@
 #include "ndc_common.h"
 #include "../../include/deconver_ndc.h"
 #include "ndc_exec.h"
+#include "ndc_direct.h"
 #include "ndc_gemm_host.h"
 #include "ndc_mlp_host.h"
 
@@ -492,6 +493,19 @@ struct Backend {
     {
         for (long long u = 0; u < units; ++u)
             for (long long p = 0; p < npos; ++p) f((int)u, p);
+        return 0;
+    }
+
+    template <class F> static int weighted_unit(long long units, long long npos, void *, F f)
+    {
+        const int n = f.weights();
+        const bool staged = F::Weights::staged(n, units * ((npos + 127) / 128) * 2);
+        std::vector<float> w(staged ? n : 0);
+        for (long long u = 0; u < units; ++u) {
+            if (staged) f.stage((int)u, w.data(), 0, 1);
+            for (long long p = 0; p < npos; ++p)
+                staged ? f.template run<true>((int)u, p, w.data()) : f.template run<false>((int)u, p, nullptr);
+        }
         return 0;
     }
 
