@@ -100,7 +100,8 @@ def _weights(linear: Linear):
     if type(conv) is not nn.Conv1d or not _stock(own["flatten"], nn.Flatten):
         return None
     own = conv._parameters
-    return None if own.get("weight") is None else (own["weight"], own.get("bias"))
+    # (a projection without a bias registers it as None; a pruned or plain-tensor bias is not registered)
+    return None if own.get("weight") is None or "bias" not in own else (own["weight"], own["bias"])
 
 
 class DeconverBlock(nn.Module):

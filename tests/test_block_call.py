@@ -6,6 +6,7 @@ import copy
 import pytest
 import torch
 from torch import nn
+from torch.nn.utils import prune
 
 import deconver_amd as dc
 from deconver_amd import model as M
@@ -69,6 +70,12 @@ def test_what_keeps_the_modules_calls():
     def swap(b):
         b.dcm.out_proj.__class__ = OtherLinear
 
+    def plain_bias(b):
+        conv = b.mlp.block[3].linear
+        bias = conv.bias.detach()
+        del conv.bias
+        conv.bias = bias
+
     for change in (lambda b: b.dcm.register_forward_hook(lambda *a: None),
                    lambda b: b.dcm.deconv.register_forward_pre_hook(lambda *a: None),
                    lambda b: b.mlp.register_full_backward_hook(lambda *a: None),
@@ -81,6 +88,7 @@ def test_what_keeps_the_modules_calls():
                    lambda b: setattr(b.mlp, "forward", lambda *a, **k: x),
                    lambda b: setattr(b.norm1, "affine", True),
                    lambda b: torch.nn.utils.parametrizations.weight_norm(b.mlp.block[0].linear),
+                   lambda b: prune.l1_unstructured(b.mlp.block[0].linear, "bias", amount=0.5), plain_bias,
                    swap):
         assert declined(change), change
     assert base.double()._one_call(x.double()) is None and base.float()._one_call(x.cpu()) is None
@@ -92,3 +100,17 @@ def test_what_keeps_the_modules_calls():
     base.eval()
     base.mlp.block[2].p = 0.5
     assert base._one_call(x) is not None
+
+
+@pytest.mark.parametrize("which", ["source", "out", "first", "second"])
+def test_a_pruned_bias_is_added(which):
+    block = _block(2, 8)
+    bare = copy.deepcopy(block)
+    parts = {"source": lambda b: b.dcm.deconv.init.linear, "out": lambda b: b.dcm.out_proj, "first": lambda b: b.mlp.block[0],
+             "second": lambda b: b.mlp.block[3]}
+    conv, other = parts[which](block).linear, parts[which](bare).linear
+    prune.l1_unstructured(conv, "bias", amount=0.5)
+    with torch.no_grad():
+        other.bias.copy_(conv.bias)      # the masked values as a parameter
+        x = torch.randn(1, 8, 6, 6, device="cuda")
+        assert torch.equal(block(x), bare(x))

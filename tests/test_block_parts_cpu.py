@@ -1,0 +1,73 @@
+"""What a block's one call is handed, on the CPU: a recorder stands in for the compiled nodes, and an input
+that says it is on the GPU for one that is.  A part whose tensors are not plain parameters keeps its
+modules' calls, which read attributes."""
+
+import pytest
+import torch
+from torch import nn
+from torch.nn.utils import prune
+
+from deconver_amd import _lib
+from deconver_amd import model as M
+
+
+class _OnGpu(torch.Tensor):
+    is_cuda = property(lambda self: True)
+
+
+class _Recorder:
+    def __init__(self):
+        self.calls = []
+
+    def block(self, *args):
+        self.calls.append(args)
+        return "one call"
+
+
+@pytest.fixture
+def recorder(monkeypatch):
+    r = _Recorder()
+    monkeypatch.setattr(_lib, "get_native", lambda: r)
+    return r
+
+
+def _block():
+    torch.manual_seed(0)
+    return M.DeconverBlock(8, norm=nn.InstanceNorm2d, kernel_size=(5, 5), groups=-1, ratio=4)
+
+
+def _input():
+    return torch.randn(1, 8, 6, 6).as_subclass(_OnGpu)
+
+
+PROJECTIONS = {"source": lambda b: b.dcm.deconv.init.linear, "out": lambda b: b.dcm.out_proj,
+               "first": lambda b: b.mlp.block[0], "second": lambda b: b.mlp.block[3]}
+
+
+def test_stock_block(recorder):
+    block = _block()
+    assert block._one_call(_input()) == "one call"
+    (args,) = recorder.calls
+    conv = block.mlp.block[0].linear
+    assert any(a is conv.weight for a in args) and any(a is conv.bias for a in args)
+    assert args[5] is None      # in_proj has no bias
+
+
+@pytest.mark.parametrize("which", PROJECTIONS)
+@pytest.mark.parametrize("how", ["pruned", "plain attribute"])
+def test_bias_that_is_no_parameter(recorder, which, how):
+    block = _block()
+    conv = PROJECTIONS[which](block).linear
+    if how == "pruned":
+        prune.l1_unstructured(conv, "bias", amount=0.5)
+    else:
+        bias = conv.bias.detach().clone()
+        del conv.bias
+        conv.bias = bias
+    assert torch.is_tensor(conv.bias) and block._one_call(_input()) is None and not recorder.calls
+
+
+def test_projection_without_bias(recorder):
+    block = _block()
+    block.dcm.out_proj = M.Linear(32, 8, bias=False)
+    assert block._one_call(_input()) == "one call"
