@@ -83,10 +83,11 @@ _INSTANCE_NORMS = {3: InstanceNorm1d, 4: InstanceNorm2d, 5: InstanceNorm3d}
 
 def _stock(module: nn.Module, kind: Optional[type]) -> bool:
     """Whether a call of ``module`` is ``kind.forward`` and nothing else."""
+    if type(module) is not kind or kind is None:
+        return False
     own = module.__dict__
-    return (type(module) is kind and not own["_forward_hooks"] and not own["_forward_pre_hooks"]
-            and not own["_backward_hooks"] and not own["_backward_pre_hooks"] and "forward" not in own
-            and own.get("_compiled_call_impl") is None)
+    return (not own["_forward_hooks"] and not own["_forward_pre_hooks"] and not own["_backward_hooks"]
+            and not own["_backward_pre_hooks"] and "forward" not in own and own.get("_compiled_call_impl") is None)
 
 
 def _idle(drop: nn.Module, owner: nn.Module) -> bool:
@@ -96,8 +97,8 @@ def _idle(drop: nn.Module, owner: nn.Module) -> bool:
 def _weights(linear: Linear):
     """Weight and bias of a ``Linear`` whose parameters are plain ones, else None."""
     own = linear._modules
-    conv = own["linear"]
-    if type(conv) is not nn.Conv1d or not _stock(own["flatten"], nn.Flatten):
+    conv = own.get("linear")
+    if type(conv) is not nn.Conv1d or not _stock(own.get("flatten"), nn.Flatten):
         return None
     own = conv._parameters
     # (a projection without a bias registers it as None; a pruned or plain-tensor bias is not registered)
@@ -141,7 +142,8 @@ class DeconverBlock(nn.Module):
                 return None
             half = True
         own = self._modules
-        norm1, dcm, norm2, mlp = own["norm1"], own["dcm"], own["norm2"], own["mlp"]
+        # (get: a part may be a plain attribute that is no module)
+        norm1, dcm, norm2, mlp = own.get("norm1"), own.get("dcm"), own.get("norm2"), own.get("mlp")
         kind = _INSTANCE_NORMS.get(x.dim())
         if not (_stock(norm1, kind) and _stock(norm2, kind) and _stock(dcm, DeconvMixer) and _stock(mlp, MLP)):
             return None
@@ -149,24 +151,24 @@ class DeconverBlock(nn.Module):
             if norm.affine or norm.track_running_stats or not hip_norm_applies(x):
                 return None
         own = dcm._modules
-        in_proj, deconv, out_proj, drop = own["in_proj"], own["deconv"], own["out_proj"], own["dropout"]
-        if not (_stock(in_proj, Linear) and _stock(deconv, Deconv) and _stock(own["act"], nn.ReLU) and _stock(out_proj, Linear)
+        in_proj, deconv, out_proj, drop = own.get("in_proj"), own.get("deconv"), own.get("out_proj"), own.get("dropout")
+        if not (_stock(in_proj, Linear) and _stock(deconv, Deconv) and _stock(own.get("act"), nn.ReLU) and _stock(out_proj, Linear)
                 and _idle(drop, dcm)):
             return None
-        inner = mlp._modules["block"]
+        inner = mlp._modules.get("block")
         if not _stock(inner, nn.Sequential) or len(inner._modules) != 5:
             return None
         first, gelu, drop1, second, drop2 = inner._modules.values()
         if not (_stock(first, Linear) and _stock(gelu, nn.GELU) and gelu.approximate == "none" and _stock(second, Linear)
                 and _idle(drop1, mlp) and _idle(drop2, mlp)):
             return None
-        init = deconv._modules["init"]
-        if not (type(init) is Initializer and type(init._modules["linear"]) is Linear and deconv.num_iters == 1
+        init = deconv._modules.get("init")
+        if not (type(init) is Initializer and type(init._modules.get("linear")) is Linear and deconv.num_iters == 1
                 and deconv.num_grad_iters >= 1 and len(deconv.kernel_size) == x.dim() - 2 and deconv._regime_allows_hip()):
             return None
         if deconv.source_channels >= 16 and deconv.filter_channels >= 4 and not deconv._differentiates(x):
             return None
-        h0 = init._parameters["h0"]
+        h0 = init._parameters.get("h0")     # (absent: pruned, or a replica's plain tensor)
         weights = [_weights(m) for m in (in_proj, init._modules["linear"], out_proj, first, second)]
         if None in weights or h0 is None or h0.dtype != torch.float32:
             return None

@@ -71,3 +71,32 @@ def test_projection_without_bias(recorder):
     block = _block()
     block.dcm.out_proj = M.Linear(32, 8, bias=False)
     assert block._one_call(_input()) == "one call"
+
+
+def test_filter_that_is_no_parameter(recorder):
+    block = _block()
+    prune.l1_unstructured(block.dcm.deconv.init, "h0", amount=0.5)
+    assert block._one_call(_input()) is None and not recorder.calls
+
+
+def _replica(module):
+    """A copy with its parameters as plain attributes, as nn.DataParallel's replicas have them."""
+    new = module._replicate_for_data_parallel()
+    for name, p in module._parameters.items():
+        setattr(new, name, None if p is None else p.detach().clone())
+    for name, child in module._modules.items():
+        setattr(new, name, _replica(child))
+    return new
+
+
+def test_replica(recorder):
+    assert _replica(_block())._one_call(_input()) is None and not recorder.calls
+
+
+@pytest.mark.parametrize("where,name", [("", "norm1"), ("", "norm2"), ("dcm", "act")])
+def test_part_that_is_no_module(recorder, where, name):
+    block = _block()
+    owner = block.get_submodule(where)
+    delattr(owner, name)
+    setattr(owner, name, lambda x: x)
+    assert block._one_call(_input()) is None and not recorder.calls
