@@ -887,6 +887,9 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         const auto need = n.ask(ctx);
         Tensor gx, gw1, gb1, gw2, gb2;
         if (!v[1].defined()) {
+            // (the kernels know the widths by x's channels alone)
+            TORCH_CHECK_VALUE(hidden == 4 * x.size(1) && w2.cout() == x.size(1), "saved weights came back as ", v[3].sizes(), " and ",
+                              v[4].sizes(), " for an MLP of ", x.size(1), " channels with four times as many hidden ones");
             const Tensor xa = aligned(x), ga = aligned(gy);
             const bool half = w1.m.scalar_type() == at::kBFloat16 && w2.m.scalar_type() == at::kBFloat16;
             const Tensor m1 = half ? w1.m : w1.m.to(at::kFloat), m2 = half ? w2.m : w2.m.to(at::kFloat);

@@ -5,7 +5,7 @@ import torch
 from torch import nn
 
 import deconver_amd as dc
-from deconver_amd import layers
+from deconver_amd import _lib, layers
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,17 @@ def test_tensors_that_come_back_as_others_are_refused(unpack, name, autocast):
 def test_tensors_kept_on_the_cpu(name):
     for a, b in zip(_gradients(name, True, lambda t: t.cpu(), lambda t: t.cuda()), _gradients(name, True)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("hidden,cin", [(96, 32), (160, 32), (256, 64), (128, 64)])
+def test_weights_of_another_width_are_refused_by_the_mlp_on_chip(hidden, cin):
+    """Two weights that fit each other and the kept input, but not the widths the kernels are built for."""
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")   # noqa: E731
+    x, w1, w2 = rand(1, 32, 4096).bfloat16(), rand(128, 32), rand(32, 128)
+    other = {(1, 32, 4096): rand(1, cin, 4096).bfloat16(), (128, 32): rand(hidden, cin), (32, 128): rand(32, hidden)}
+    x, w1, w2 = (t.requires_grad_(True) for t in (x, w1, w2))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: other[tuple(t.shape)]):
+        y = _lib.get_native().mlp(x, w1, None, w2, None, None)
+    with pytest.raises(ValueError, match="saved weights came back"):
+        y.backward(torch.ones_like(y))
