@@ -693,8 +693,10 @@ int ndc_mlp_forward(const void *x, const float *stats, const void *w1, const voi
     if ((uintptr_t)stats & 15u) return NDC_ERR_WORKSPACE;
     const int st = mlp_check(batch, c, n, w_dtype, dtype);
     if (st) return st;
+    // (weights are loaded element by element)
+    const uintptr_t wmask = w_dtype == NDC_BF16 ? 1u : 3u;
     if (((uintptr_t)x & 3u) || ((uintptr_t)y & 3u) || ((uintptr_t)residual & 3u) || ((uintptr_t)b1 & 3u) || ((uintptr_t)b2 & 3u) ||
-        ((uintptr_t)w1 & 3u) || ((uintptr_t)w2 & 3u))
+        ((uintptr_t)w1 & wmask) || ((uintptr_t)w2 & wmask))
         return NDC_ERR_WORKSPACE;
     if (y == x) return NDC_ERR_GEOMETRY;
     return ndc::Backend::mlp_forward(x, stats, w1, w2, w_dtype == NDC_BF16, b1, b2, residual, y, batch, (int)c, n, stream);
@@ -713,8 +715,9 @@ int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *
     if (!x || !gy || !w1 || !w2 || !gx || !gw1 || !gw2) return NDC_ERR_NULL;
     const int st = mlp_check(batch, c, n, w_dtype, dtype);
     if (st) return st;
-    if (((uintptr_t)x & 15u) || ((uintptr_t)gy & 15u) || ((uintptr_t)gx & 3u) || ((uintptr_t)b1 & 3u) || ((uintptr_t)w1 & 3u) ||
-        ((uintptr_t)w2 & 3u) || !workspace || ((uintptr_t)workspace & 15u) || workspace_bytes < ndc_mlp_workspace_bytes(batch, c, n))
+    const uintptr_t wmask = w_dtype == NDC_BF16 ? 1u : 3u;
+    if (((uintptr_t)x & 15u) || ((uintptr_t)gy & 15u) || ((uintptr_t)gx & 3u) || ((uintptr_t)b1 & 3u) || ((uintptr_t)w1 & wmask) ||
+        ((uintptr_t)w2 & wmask) || !workspace || ((uintptr_t)workspace & 15u) || workspace_bytes < ndc_mlp_workspace_bytes(batch, c, n))
         return NDC_ERR_WORKSPACE;
     if (gx == x || gx == gy) return NDC_ERR_GEOMETRY;
     return ndc::Backend::mlp_backward(x, gy, w1, w2, w_dtype == NDC_BF16, b1, gx, gw1, gb1, gw2, gb2, (float *)workspace, batch, (int)c,

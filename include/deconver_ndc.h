@@ -486,8 +486,8 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
  *     y = W2 gelu(W1 x + b1) + b2 + residual          W1 (4c, c), W2 (c, 4c)
  * and its gradients from x and gy (the hidden tensor is formed again).
  *   ndc_mlp_supported  1 where the kernels apply: NDC_BF16, c 32 or 64, n a multiple of 64 up to 2^26
- *   w1, w2      as they lie, both of dtype w_dtype (NDC_F32 or NDC_BF16); rounded to bfloat16 for the
- *               products
+ *   w1, w2      as they lie, both of dtype w_dtype (NDC_F32 or NDC_BF16), aligned to an element; rounded to
+ *               bfloat16 for the products
  *   b1, b2      float32 or NULL; residual: y's shape, or NULL; y may be residual
  *   stats       NULL, or the (mean, 1 / deviation) pairs of the rows of x (ndc_rownorm_stats, 16-byte
  *               aligned): the MLP is then of the normalised x; residual is not NULL

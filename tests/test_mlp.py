@@ -144,3 +144,22 @@ def test_partly_frozen_mlp_gives_the_same_gradients(frozen):
         else:
             a, b = got[0][k].grad.double(), got[1][k].grad.double()
             assert float((a - b).norm() / a.norm()) < 1e-2
+
+
+@pytest.mark.parametrize("c,n", [(32, 4096), (64, 32768)])
+def test_weights_at_an_odd_element(c, n):
+    """bfloat16 weights that are views one element into a flat buffer: the same bits as aligned ones."""
+    gen = torch.Generator(device="cuda").manual_seed(c)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")   # noqa: E731
+    x, g = rand(1, c, n).bfloat16(), rand(1, c, n).bfloat16()
+    flat = rand(8 * c * c + 2).bfloat16() / c ** 0.5
+    odd = [flat[1:1 + 4 * c * c].view(4 * c, c), flat[1 + 4 * c * c:1 + 8 * c * c].view(c, 4 * c)]
+    assert all(w.data_ptr() % 4 == 2 for w in odd)
+    got = []
+    for weights in (odd, [w.clone() for w in odd]):
+        leaves = [t.detach().requires_grad_(True) for t in (x, *weights)]
+        y = _lib.get_native().mlp(leaves[0], leaves[1], None, leaves[2], None, None)
+        y.backward(g)
+        got.append([y] + [t.grad for t in leaves])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
