@@ -148,8 +148,10 @@ class DeconverBlock(nn.Module):
         if not (_stock(norm1, kind) and _stock(norm2, kind) and _stock(dcm, DeconvMixer) and _stock(mlp, MLP)):
             return None
         for norm in (norm1, norm2):
-            if norm.affine or norm.track_running_stats or not hip_norm_applies(x):
+            if norm.affine or norm.track_running_stats or "with_skip" in norm.__dict__:
                 return None
+        if not hip_norm_applies(x):
+            return None
         own = dcm._modules
         in_proj, deconv, out_proj, drop = own.get("in_proj"), own.get("deconv"), own.get("out_proj"), own.get("dropout")
         if not (_stock(in_proj, Linear) and _stock(deconv, Deconv) and _stock(own.get("act"), nn.ReLU) and _stock(out_proj, Linear)
@@ -163,10 +165,7 @@ class DeconverBlock(nn.Module):
                 and _idle(drop1, mlp) and _idle(drop2, mlp)):
             return None
         init = deconv._modules.get("init")
-        if not (type(init) is Initializer and type(init._modules.get("linear")) is Linear and deconv.num_iters == 1
-                and deconv.num_grad_iters >= 1 and len(deconv.kernel_size) == x.dim() - 2 and deconv._regime_allows_hip()):
-            return None
-        if deconv.source_channels >= 16 and deconv.filter_channels >= 4 and not deconv._differentiates(x):
+        if not (type(init) is Initializer and type(init._modules.get("linear")) is Linear and deconv._is_one_plain_update(x)):
             return None
         h0 = init._parameters.get("h0")     # (absent: pruned, or a replica's plain tensor)
         weights = [_weights(m) for m in (in_proj, init._modules["linear"], out_proj, first, second)]

@@ -100,3 +100,38 @@ def test_part_that_is_no_module(recorder, where, name):
     delattr(owner, name)
     setattr(owner, name, lambda x: x)
     assert block._one_call(_input()) is None and not recorder.calls
+
+
+ROUTE = ["fast_path_applicable", "takes_rectified_input", "context", "_fit_fast", "_regime_allows_hip", "_hip_is_ahead"]
+
+
+@pytest.mark.parametrize("name", ROUTE)
+@pytest.mark.parametrize("where", ["instance", "class"])
+def test_replaced_method_of_the_layer(recorder, monkeypatch, where, name):
+    """A method that the layer's own call would go through."""
+    block = _block()
+    deconv = block.dcm.deconv
+    own = getattr(deconv, name)
+    replacement = lambda *a, **k: own(*a, **k)      # noqa: E731
+    if where == "instance":
+        setattr(deconv, name, replacement)
+    else:
+        monkeypatch.setattr(type(deconv), name, replacement)
+    assert block._one_call(_input()) is None and not recorder.calls
+
+
+@pytest.mark.parametrize("name", ["norm1", "norm2"])
+def test_replaced_method_of_a_norm(recorder, name):
+    block = _block()
+    getattr(block, name).with_skip = lambda x: (x, x)
+    assert block._one_call(_input()) is None and not recorder.calls
+
+
+def test_forward_only_call_that_the_library_is_ahead_on(recorder):
+    """Many source channels per group: the block's call leaves the choice where the layer makes it."""
+    block = M.DeconverBlock(8, norm=nn.InstanceNorm2d, kernel_size=(3, 3), groups=2, source_channels=16)
+    x = _input()
+    assert block._one_call(x) == "one call"
+    with torch.no_grad():
+        assert block._one_call(x) is None
+    assert len(recorder.calls) == 1
