@@ -295,7 +295,10 @@ struct Backend {
     }
 
     // ... one launch, a row per workgroup (held_kernel), where a row fits: the smallest workgroup that holds
-    // it in a few vectors a thread
+    // it in a few vectors a thread.  Single elements (rows of no whole number of vectors): 8 or 16 a thread, so that
+    // several small workgroups share a CU.  With 2 to 4 of them in 1024 threads a CU had some 8 KB in flight: us,
+    // two launches -> 1024 threads -> as now, float32 forward: 8192 rows of 1025 28.7 -> 57.5 -> 15.6, of 2197 44.9 ->
+    // 58.7 -> 24.1, of 4095 72.1 -> 63.3 -> 43.0; 256 rows of 2197 7.5 -> 4.7 -> 4.3.
     template <typename T, bool BWD, bool VEC, bool ADD, int PER, int NT>
     static bool rownorm_held_launch(const void *a, const void *b, const void *addend, float *stats, void *out, long long rows,
                                     long long n, float eps, void *stream)
@@ -313,10 +316,17 @@ struct Backend {
         if (nv <= 2 * 64) return NDC_HELD(2, 64);
         if (nv <= 2 * 256) return NDC_HELD(2, 256);
         if (nv <= 4 * 256) return NDC_HELD(4, 256);
-        if (nv <= 2 * 1024) return NDC_HELD(2, 1024);
-        if (nv <= 4 * 1024) return NDC_HELD(4, 1024);
         // (two tensors of long rows on few CUs: 64 rows of 32 768 floats 8.6 us against 8.1 in two launches)
-        if (nv <= 8 * 1024 && (!BWD || rows >= 96)) return NDC_HELD(8, 1024);
+        const bool long_rows = nv <= 8 * 1024 && (!BWD || rows >= 96);
+        if constexpr (VEC) {
+            if (nv <= 2 * 1024) return NDC_HELD(2, 1024);
+            if (nv <= 4 * 1024) return NDC_HELD(4, 1024);
+            if (long_rows) return NDC_HELD(8, 1024);
+        } else {
+            if (nv <= 8 * 256) return NDC_HELD(8, 256);
+            if (nv <= 16 * 256) return NDC_HELD(16, 256);
+            if (long_rows) return NDC_HELD(16, 512);
+        }
         if constexpr (!BWD)
             if (nv <= 12 * 1024) return NDC_HELD(12, 1024);
 #undef NDC_HELD

@@ -31,3 +31,11 @@ def test_lengths(vectors, odd, dtype, tol, rows):
     (yd * g.double() + xd * skip_g.double()).sum().backward()
     for a, r in ((y, yd), (x.grad, xd.grad)):
         assert float((a.detach().double() - r.detach()).abs().max() / r.detach().abs().max()) < tol
+
+
+# single elements, at and next to every size
+@pytest.mark.parametrize("n", [127, 129, 511, 513, 1023, 1025, 2047, 2049, 4095, 4097, 8191, 8193, 12287, 12289])
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("rows", [3, 97])
+def test_lengths_in_elements(n, dtype, tol, rows):
+    test_lengths(n // (16 // dtype.itemsize), n % (16 // dtype.itemsize), dtype, tol, rows)
