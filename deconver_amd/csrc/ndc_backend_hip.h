@@ -316,8 +316,13 @@ struct Backend {
         if (nv <= 2 * 64) return NDC_HELD(2, 64);
         if (nv <= 2 * 256) return NDC_HELD(2, 256);
         if (nv <= 4 * 256) return NDC_HELD(4, 256);
-        // (two tensors of long rows on few CUs: 64 rows of 32 768 floats 8.6 us against 8.1 in two launches)
-        const bool long_rows = nv <= 8 * 1024 && (!BWD || rows >= 96);
+        // Long rows in vectors, few of them: one workgroup a row uses few CUs, and two launches read a row again from
+        // the cache.  us, two launches -> held, forward and then forward + backward (the backward in two launches
+        // either way: held it takes 8.6 against 8.1 on 64 rows of 32 768 floats): 64 rows of 24 000 floats 8.3 -> 6.3,
+        // 17.2 -> 17.0; of 32 768 8.4 -> 7.2, 15.8 -> 17.6; 4 rows of 98 304 bf16 values 8.2 -> 8.5, 13.3 -> 14.1;
+        // 96 rows of 65 536 10.3 -> 8.6, 22.0 -> 18.3.
+        const bool few = VEC && rows < 96;
+        const bool long_rows = nv <= (few ? 6 * 1024 : 8 * 1024) && (!BWD || rows >= 96);
         if constexpr (VEC) {
             if (nv <= 2 * 1024) return NDC_HELD(2, 1024);
             if (nv <= 4 * 1024) return NDC_HELD(4, 1024);
@@ -328,7 +333,7 @@ struct Backend {
             if (long_rows) return NDC_HELD(16, 512);
         }
         if constexpr (!BWD)
-            if (nv <= 12 * 1024) return NDC_HELD(12, 1024);
+            if (nv <= 12 * 1024 && !few) return NDC_HELD(12, 1024);
 #undef NDC_HELD
         return false;
     }

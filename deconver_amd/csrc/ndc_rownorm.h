@@ -18,8 +18,9 @@
 // The backward's optional addend is the gradient that reaches x by another way (the residual
 // branch around a pre-norm block): summed here, it saves the separate pass that would add it.
 //
-// Rows of up to 8192 16-byte vectors (12 288 in the forward) take one launch per direction instead:
-// held_kernel keeps a row in the registers of one workgroup, reads it once and needs no partials.
+// Rows of up to 8192 16-byte vectors (12 288 in the forward; Backend::rownorm_held says when) take one launch
+// per direction instead: held_kernel keeps a row in the registers of one workgroup, reads it once and needs no
+// partials.
 //
 // HBM traffic of the two-launch form: forward 2 reads + 1 write of the tensor, backward 4 reads + 1 write.  Sums are
 // float32 whatever the storage type.  Device code only (included by the HIP build).

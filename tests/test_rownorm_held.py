@@ -39,3 +39,11 @@ def test_lengths(vectors, odd, dtype, tol, rows):
 @pytest.mark.parametrize("rows", [3, 97])
 def test_lengths_in_elements(n, dtype, tol, rows):
     test_lengths(n // (16 // dtype.itemsize), n % (16 // dtype.itemsize), dtype, tol, rows)
+
+
+# the longest row of a few that is held, and the fewest rows from which longer ones are
+@pytest.mark.parametrize("vectors", [6144, 6145, 12288])
+@pytest.mark.parametrize("rows", [95, 96])
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)])
+def test_few_long_rows(vectors, rows, dtype, tol):
+    test_lengths(vectors, 0, dtype, tol, rows)
