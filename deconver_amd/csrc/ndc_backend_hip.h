@@ -299,10 +299,12 @@ struct Backend {
     // several small workgroups share a CU.  With 2 to 4 of them in 1024 threads a CU had some 8 KB in flight: us,
     // two launches -> 1024 threads -> as now, float32 forward: 8192 rows of 1025 28.7 -> 57.5 -> 15.6, of 2197 44.9 ->
     // 58.7 -> 24.1, of 4095 72.1 -> 63.3 -> 43.0; 256 rows of 2197 7.5 -> 4.7 -> 4.3.
+    // False, with nothing launched, for rows that do not fit, and past the 2^32 threads of a launch.
     template <typename T, bool BWD, bool VEC, bool ADD, int PER, int NT>
     static bool rownorm_held_launch(const void *a, const void *b, const void *addend, float *stats, void *out, long long rows,
                                     long long n, float eps, void *stream)
     {
+        if (rows > 0xffffffffLL / NT) return false;
         hipLaunchKernelGGL((rownorm::held_kernel<T, BWD, VEC, ADD, PER, NT>), dim3((unsigned)rows), dim3(NT), 0,
                            (hipStream_t)stream, (const T *)a, (const T *)b, (const T *)addend, (float2 *)stats, (T *)out, n, eps);
         return true;
