@@ -719,6 +719,19 @@ Tensor projected_update(const Tensor &x, const Tensor &weight, const Tensor &h, 
 
 // ---------------------------------------------------------------------------- projection with its tail
 
+// Whether a bare float32 product that narrows (a stage's adapter, a downsampling; nobody's but its node's) is
+// the tiled GEMM's.  The library takes a few workgroups for up to some 250 voxels a sample -- 512 -> 256 channels
+// over 256 voxels 119 us against 6 tiled, 512 -> 128 over 8 x 194 69 against 8.5, 384 -> 192 over 241 82 against
+// 5.3 --, above that it is ahead but in small products: 512 -> 256 over 2048 9.1 against 14.7, 384 -> 192 over 2714
+// 8.2 against 13.5, 96 -> 48 over 2 x 2737 5.5 against 6.4; 128 -> 64 over 3295 5.9 against 5.0, 512 -> 256 over 500
+// 7.1 against 6.2.  With 1024 channels it was ahead at every size (over 16 voxels 6.4 against 8.3, 1024 14 against 23).
+bool narrow_is_tiled(int64_t B, int64_t cin, int64_t cout, int64_t n)
+{
+    if (cin <= cout || cin > 768) return false;
+    const double flops = 2.0 * (double)B * (double)n * (double)cin * (double)cout;
+    return (n <= 256 && flops < 0.5e9) || (B * n <= 5000 && flops < 0.1e9);
+}
+
 // y[b] = act(W x[b] + bias) + residual[b] on channel-first (B, C, n) tensors.  keep: the
 // activation's gradient will want the product (gelu, or relu under a residual sum)
 struct Linear : public torch::autograd::Function<Linear> {
@@ -728,10 +741,9 @@ struct Linear : public torch::autograd::Function<Linear> {
         const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
         const bool tail = bias.defined() || act != NDC_ACT_NONE || res.defined();
         // An activation's tile form reads W as rows.  A bare float32 product that widens could be a layer's
-        // projection taken apart: the library's product, bit for bit as in Projected.  One that narrows (a
-        // stage's adapter, a downsampling) is nobody's but this node's; the library ran 512 -> 256 channels over
-        // 256 voxels in one workgroup, 123 us against 7 us sliced.
-        const bool library = (w.transposed && act != NDC_ACT_NONE) || (!tail && x.scalar_type() == at::kFloat && w.cin() <= cout);
+        // projection taken apart: the library's product, bit for bit as in Projected.
+        const bool bare = !tail && x.scalar_type() == at::kFloat;
+        const bool library = (w.transposed && act != NDC_ACT_NONE) || (bare && !narrow_is_tiled(B, w.cin(), cout, n));
         const Gemm by = library ? kLibrary : choose_gemm(x, cout, act != NDC_ACT_NONE || keep, tail);
         Tensor y = empty({B, cout, n}, x);
         if (keep) z = empty({B, cout, n}, x);

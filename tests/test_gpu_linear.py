@@ -76,3 +76,18 @@ def test_linear_module_under_autocast_keeps_float32_parameter_gradients():
     ref = F.conv1d(x.detach().double().flatten(2), lin.linear.weight.double(), lin.linear.bias.double()).view_as(y32)
     assert y32.dtype == torch.float32
     assert float((y32.double() - ref).abs().max() / ref.abs().max()) <= 1e-5
+
+
+# (B, cin, cout, n, by the tiled GEMM): either side of each bound of the rule for bare float32 products that narrow
+NARROW = [(1, 512, 256, 256, True), (1, 768, 384, 131, True), (1, 1024, 512, 64, False), (1, 768, 767, 256, True),
+          (2, 768, 767, 256, False), (1, 128, 64, 5000, True), (1, 128, 64, 5001, False), (2, 64, 8, 2500, True), (2, 64, 8, 2501, False),
+          (1, 512, 256, 381, True), (1, 512, 256, 382, False), (1, 64, 64, 100, False)]
+
+
+@pytest.mark.parametrize("B,cin,cout,n,tiled", NARROW)
+def test_bare_float32_products_that_narrow(B, cin, cout, n, tiled):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, w = torch.randn(B, cin, n, generator=g, device="cuda"), torch.randn(cout, cin, generator=g, device="cuda") / cin ** 0.5
+    y = pointwise_linear(x, w)
+    assert float((y.double() - w.double() @ x.double()).norm() / y.double().norm()) < 2e-6     # float32 sums
+    assert tiled or torch.equal(y, torch.bmm(w.expand(B, cout, cin), x))
