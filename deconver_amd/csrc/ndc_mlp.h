@@ -101,7 +101,9 @@ __device__ inline uint32_t *words(uint16_t *p) { return reinterpret_cast<uint32_
 // a packing launch each costs more).  Workgroups are persistent, twelve wavefronts at C = 64: three per
 // SIMD is what the 168 registers of a wavefront leave.
 // NORM: x is normalised as it is loaded, and the residual is the x before that.
-template <int C, typename TW, bool RES, int THREADS, bool NORM>
+// HALF: a wavefront takes the even or the odd voxels of a tile, and a launch has twice as many: for few tiles,
+// whose time is the GELUs of one wavefront one after the other (see forward_launch).
+template <int C, typename TW, bool RES, int THREADS, bool NORM, bool HALF>
 __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
 {
     constexpr int H = 4 * C, S = C / 16, HT = H / 32, OT = C / 32, WAVES = THREADS / 64;
@@ -125,11 +127,12 @@ __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
     const int lane = threadIdx.x & 63, n32 = lane & 31, kb = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t xw = (uint32_t)(4 * kb) * (uint32_t)p.n + n32, yw = (uint32_t)(2 * kb) * (uint32_t)p.n + n32;
-    const int nwaves = (int)gridDim.x * WAVES;
-    for (int tile = (int)blockIdx.x * WAVES + wave; tile < p.tiles; tile += nwaves) {
+    constexpr int PER = HALF ? 2 : 1, NP = 2 / PER;   // wavefronts to a tile, parities to a wavefront
+    const int nwaves = (int)gridDim.x * WAVES / PER, odd = wave % PER;
+    for (int tile = ((int)blockIdx.x * WAVES + wave) / PER; tile < p.tiles; tile += nwaves) {
         const int b = __builtin_amdgcn_readfirstlane(tile / p.tiles_per_sample);
         const long long at0 = (long long)b * C * p.n + (long long)(tile - b * p.tiles_per_sample) * kTileVoxels;
-        u32x4 xf[S][2];
+        u32x4 xf[S][NP];
         {
             uint32_t raw[S][8];
 #pragma unroll
@@ -138,16 +141,23 @@ __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
                 for (int e = 0; e < 8; ++e) raw[s][e] = words(p.x + at0 + (long long)(16 * s + e) * p.n)[xw];
             if constexpr (NORM) pwgemm::normalise_words<S>(raw, p.stats + 2 * (long long)b * C, kb);
 #pragma unroll
-            for (int s = 0; s < S; ++s) split_words(raw[s], xf[s][0], xf[s][1]);
+            for (int s = 0; s < S; ++s) {
+                u32x4 even_odd[2];
+                split_words(raw[s], even_odd[0], even_odd[1]);
+                if constexpr (HALF) xf[s][0] = odd ? even_odd[1] : even_odd[0];
+                else xf[s][0] = even_odd[0], xf[s][1] = even_odd[1];
+            }
         }
-        f32x16 acc[OT][2];
+        f32x16 acc[OT][NP];
 #pragma unroll
-        for (int o = 0; o < OT; ++o) acc[o][0] = f32x16{}, acc[o][1] = f32x16{};
+        for (int o = 0; o < OT; ++o)
+#pragma unroll
+            for (int par = 0; par < NP; ++par) acc[o][par] = f32x16{};
 #pragma unroll 1
         for (int ct = 0; ct < HT; ++ct) {
             // (the even and the odd voxels one after the other: side by side they spill registers)
 #pragma unroll
-            for (int par = 0; par < 2; ++par) {
+            for (int par = 0; par < NP; ++par) {
                 __builtin_amdgcn_sched_barrier(0);
                 f32x16 u = {};
 #pragma unroll
@@ -184,9 +194,15 @@ __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const float bj = b2l[32 * o + 8 * (j / 4) + 4 * kb + j % 4];
-                float y0 = acc[o][0][j] + bj, y1 = acc[o][1][j] + bj;
-                if constexpr (RES) y0 += lo_bf16(rw[j]), y1 += hi_bf16(rw[j]);
-                words(p.y + at0 + (long long)(32 * o + 8 * (j / 4) + j % 4) * p.n)[yw] = pack_bf16x2(y0, y1);
+                uint32_t *to = words(p.y + at0 + (long long)(32 * o + 8 * (j / 4) + j % 4) * p.n) + yw;
+                float y0 = acc[o][0][j] + bj, y1 = HALF ? 0.f : acc[o][NP - 1][j] + bj;
+                if constexpr (HALF) {
+                    if constexpr (RES) y0 += odd ? hi_bf16(rw[j]) : lo_bf16(rw[j]);
+                    reinterpret_cast<uint16_t *>(to)[odd] = (uint16_t)pack_bf16x2(y0, 0.f);
+                } else {
+                    if constexpr (RES) y0 += lo_bf16(rw[j]), y1 += hi_bf16(rw[j]);
+                    *to = pack_bf16x2(y0, y1);
+                }
             }
         }
     }

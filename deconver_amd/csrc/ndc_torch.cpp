@@ -833,7 +833,7 @@ Tensor linear(const Tensor &x, const Tensor &weight, const OptTensor &bias, int6
 
 // Whether an MLP runs with its hidden tensor on chip (ndc_mlp_forward / _backward) where those kernels
 // apply: with 64 channels from 32 768 voxels on (their kernels take 24 + 30 us there, the projections' 30 +
-// 55; over 16 384 voxels 23 against 20 forward), with 32 from 4096 (10 + 20 against 9 + 26).
+// 55; over 16 384 voxels 23 against 20 forward), with 32 from 4096 (7.5 + 15 against 8.1 + 23).
 int64_t mlp_least_voxels(int64_t c) { return c == 32 ? 4096 : 32768; }
 
 bool mlp_on_chip(const Tensor &x, const Matrix &w1, const Matrix &w2)

@@ -127,6 +127,13 @@ def test_hidden_tensor_on_chip(B, c, n, bias, residual, wdtype):
         assert t is None or err(t.grad, ref) < tol, (tuple(t.shape), err(t.grad, ref))
 
 
+# 32 channels: the tiles that two wavefronts share (an odd number of them, the most) and one more
+@pytest.mark.parametrize("B,n", [(1, 4160), (3, 4160), (1, 32768), (1, 32832)])
+@pytest.mark.parametrize("bias,residual,wdtype", [(True, True, torch.float32), (False, False, torch.bfloat16)])
+def test_tiles_of_two_wavefronts(B, n, bias, residual, wdtype):
+    test_hidden_tensor_on_chip(B, 32, n, bias, residual, wdtype)
+
+
 @pytest.mark.parametrize("frozen", ["x", "w1", "w2"])
 def test_partly_frozen_mlp_gives_the_same_gradients(frozen):
     gen = torch.Generator(device="cuda").manual_seed(1)
