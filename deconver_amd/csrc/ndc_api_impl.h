@@ -712,7 +712,7 @@ int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *
                      void *gx, float *gw1, float *gb1, float *gw2, float *gb2, int64_t batch, int64_t c, int64_t n,
                      int dtype, void *workspace, size_t workspace_bytes, void *stream)
 {
-    if (!x || !gy || !w1 || !w2 || !gx || !gw1 || !gw2) return NDC_ERR_NULL;
+    if (!x || !gy || !w1 || !w2) return NDC_ERR_NULL;
     const int st = mlp_check(batch, c, n, w_dtype, dtype);
     if (st) return st;
     const uintptr_t wmask = w_dtype == NDC_BF16 ? 1u : 3u;
@@ -720,6 +720,7 @@ int ndc_mlp_backward(const void *x, const void *gy, const void *w1, const void *
         ((uintptr_t)w2 & wmask) || !workspace || ((uintptr_t)workspace & 15u) || workspace_bytes < ndc_mlp_workspace_bytes(batch, c, n))
         return NDC_ERR_WORKSPACE;
     if (gx == x || gx == gy) return NDC_ERR_GEOMETRY;
+    if (!gx && !gw1 && !gb1 && !gw2 && !gb2) return NDC_OK;
     return ndc::Backend::mlp_backward(x, gy, w1, w2, w_dtype == NDC_BF16, b1, gx, gw1, gb1, gw2, gb2, (float *)workspace, batch, (int)c,
                                       n, stream);
 }

@@ -223,9 +223,12 @@ __global__ void __launch_bounds__(THREADS) forward_kernel(Params p)
 //     transposition is a product with the identity (exact): its result, packed, is that operand.
 // Two barriers a tile.  The sums a workgroup ends with go to its row of `part`; the caller adds the rows
 // in a fixed order.
-template <int C, typename TW>
+// GX, G1, G2: x's gradient, the first projection's, the second's.  What none of them needs is not compiled in
+// (gx may be null with GX, and is not stored then).
+template <int C, typename TW, bool GX, bool G1, bool G2>
 __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
 {
+    constexpr bool GU = GX || G1;   // the hidden tensor's gradient is formed
     constexpr int H = 4 * C, S = C / 16, WAVES = C / 8, RB = C / 32;
     __shared__ __attribute__((aligned(16))) u32x4 col[2][S][2][64];        // [x, gy][k-step][parity]
     __shared__ __attribute__((aligned(16))) u32x4 row[2][RB][2][2][64];    // [x, gy][32 channels][k-step][parity]
@@ -243,9 +246,9 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         w1f[s] = weight_frag((const TW *)p.w1, [&](int e) { return (h0 + n32) * C + 16 * s + 8 * kb + e; });
-        w2f[s] = weight_frag((const TW *)p.w2, [&](int e) { return (16 * s + 8 * kb + e) * H + h0 + n32; });
+        if constexpr (GU) w2f[s] = weight_frag((const TW *)p.w2, [&](int e) { return (16 * s + 8 * kb + e) * H + h0 + n32; });
     }
-    for (int i = threadIdx.x; i < RB * 2 * WAVES * 64; i += 64 * WAVES) {
+    for (int i = threadIdx.x; GX && i < RB * 2 * WAVES * 64; i += 64 * WAVES) {
         const int l = i & 63, t = (i >> 6) % WAVES, r = (i >> 6) / WAVES, g = l >> 4;
         w1t[r][t][l] = weight_frag((const TW *)p.w1, [&](int e) {
             return (32 * t + 16 * (g >> 1) + result_k(e, g & 1)) * C + 16 * r + (l & 15);
@@ -274,12 +277,15 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
     const uint16_t *src = second ? p.gy : p.x;
     uint32_t cw[8];
     u32x4 rw[2];
+    const bool wants_row = second ? G2 : G1, wants_col = !second || GU;
     auto request = [&](int tile) {
         const int b = __builtin_amdgcn_readfirstlane(tile / p.tiles_per_sample);
         const uint16_t *t0 = src + (long long)b * C * p.n + (long long)(tile - b * p.tiles_per_sample) * kTileVoxels;
+        if (wants_col)
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            cw[e] = words(t0 + (long long)(16 * unit + e) * p.n)[(uint32_t)(4 * kb) * (uint32_t)p.n + n32];
+            for (int e = 0; e < 8; ++e)
+                cw[e] = words(t0 + (long long)(16 * unit + e) * p.n)[(uint32_t)(4 * kb) * (uint32_t)p.n + n32];
+        if (!wants_row) return;
         const uint32_t lo = (uint32_t)n32 * (uint32_t)p.n + 8 * kb;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
@@ -287,9 +293,12 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
     };
     auto stage = [&]() {
         u32x4 even, odd;
-        split_words(cw, even, odd);
-        col[second][unit][0][lane] = even;
-        col[second][unit][1][lane] = odd;
+        if (wants_col) {
+            split_words(cw, even, odd);
+            col[second][unit][0][lane] = even;
+            col[second][unit][1][lane] = odd;
+        }
+        if (!wants_row) return;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -322,7 +331,7 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 u = mfma32(frag(w1f[s]), frag(col[0][s][par][lane]), u);
-                gh = mfma32(frag(w2f[s]), frag(col[1][s][par][lane]), gh);
+                if constexpr (GU) gh = mfma32(frag(w2f[s]), frag(col[1][s][par][lane]), gh);
             }
             u32x4 hf[2], gf[2];
 #pragma unroll
@@ -337,21 +346,22 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
                     const float v = u[j] + bq[jj], cdf = normal_cdf(v, gauss);
                     h[jj] = v * cdf;
                     g[jj] = gh[j] * __builtin_fmaf(v * 0.3989422804014327f, gauss, cdf);
-                    gb1[j] += g[jj];
+                    if constexpr (G1) gb1[j] += g[jj];
                 }
                 hf[q / 2][2 * (q & 1)] = pack_bf16x2(h[0], h[1]);
                 hf[q / 2][2 * (q & 1) + 1] = pack_bf16x2(h[2], h[3]);
                 gf[q / 2][2 * (q & 1)] = pack_bf16x2(g[0], g[1]);
                 gf[q / 2][2 * (q & 1) + 1] = pack_bf16x2(g[2], g[3]);
             }
+            if constexpr (GX)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) gul[2 * wave + s][par][lane] = gf[s];
+                for (int s = 0; s < 2; ++s) gul[2 * wave + s][par][lane] = gf[s];
             // voxels inside the lane, hidden channels along the lanes
             f32x16 ht = {}, gt = {};
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
-                ht = mfma32(frag(hf[s]), frag(ident[s]), ht);
-                gt = mfma32(frag(gf[s]), frag(ident[s]), gt);
+                if constexpr (G2) ht = mfma32(frag(hf[s]), frag(ident[s]), ht);
+                if constexpr (G1) gt = mfma32(frag(gf[s]), frag(ident[s]), gt);
             }
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
@@ -363,13 +373,14 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
                 }
 #pragma unroll
                 for (int i = 0; i < RB; ++i) {
-                    gw1[i] = mfma32(frag(gv), frag(row[0][i][s][par][lane]), gw1[i]);   // hidden x input channel
-                    gw2[i] = mfma32(frag(row[1][i][s][par][lane]), frag(hv), gw2[i]);   // output channel x hidden
+                    if constexpr (G1) gw1[i] = mfma32(frag(gv), frag(row[0][i][s][par][lane]), gw1[i]);   // hidden x input channel
+                    if constexpr (G2) gw2[i] = mfma32(frag(row[1][i][s][par][lane]), frag(hv), gw2[i]);   // output channel x hidden
                 }
             }
         }
         __syncthreads();   // gu of all hidden channels is there; the fragments have been read
         if (next < p.tiles) stage();
+        if (!GX || !p.y) continue;
         f32x4 g0 = {}, g1 = {};
 #pragma unroll
         for (int t = 0; t < WAVES; ++t) {
@@ -386,26 +397,28 @@ __global__ void __launch_bounds__(8 * C, 2) backward_kernel(Params p)
                 pack_bf16x2(g0[j], g1[j]);
     }
 
+    if constexpr (!G1 && !G2) return;
     float *o1 = p.part + (long long)blockIdx.x * part_floats(C), *o2 = o1 + H * C, *ob1 = o2 + H * C, *ob2 = ob1 + H;
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int r = 8 * (j / 4) + 4 * kb + j % 4;
-            o1[(h0 + r) * C + 32 * i + n32] = gw1[i][j];
-            o2[(32 * i + r) * H + h0 + n32] = gw2[i][j];
+            if constexpr (G1) o1[(h0 + r) * C + 32 * i + n32] = gw1[i][j];
+            if constexpr (G2) o2[(32 * i + r) * H + h0 + n32] = gw2[i][j];
         }
+    if constexpr (G1)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const float t = epilogue::half_sum(gb1[j]);
-        if (n32 == 31) ob1[h0 + 8 * (j / 4) + 4 * kb + j % 4] = t;
-    }
-    if (second) ob2[(2 * rs + kb) * C + 32 * rb + n32] = gb2;
+        for (int j = 0; j < 16; ++j) {
+            const float t = epilogue::half_sum(gb1[j]);
+            if (n32 == 31) ob1[h0 + 8 * (j / 4) + 4 * kb + j % 4] = t;
+        }
+    if (G2 && second) ob2[(2 * rs + kb) * C + 32 * rb + n32] = gb2;
 }
 
 // The workgroups' partial results added up: thread (quad, j) of 32 x 8 takes four neighbouring values
 // of the parts j, j + 8, ... in order, eight parts in flight, then the eight sums in order.  (One value a
-// thread, strided_sum_kernel, took 16.5 us for the 34 MB of C = 64.)
+// thread, strided_sum_kernel, took 16.5 us for the 34 MB of C = 64.)  Results that are null are not added up.
 template <int C>
 __global__ void __launch_bounds__(256) sum_kernel(const float *part, int nparts, float *gw1, float *gb1, float *gw2, float *gb2)
 {
@@ -414,8 +427,9 @@ __global__ void __launch_bounds__(256) sum_kernel(const float *part, int nparts,
     __shared__ f32x4 buf[8][32];
     const int qx = threadIdx.x & 31, j = threadIdx.x >> 5;
     const int o = (int)(blockIdx.x * 32 + qx) * 4;
+    float *const base = o < NW ? gw1 : o < 2 * NW ? gw2 : o < first ? gb1 : o < first + C ? gb2 : nullptr;
     f32x4 acc = {};
-    if (o < first) {
+    if (base && o < first) {
         const float *at = part + o;
         int k = j;
         for (; k + 56 < nparts; k += 64) {
@@ -426,7 +440,7 @@ __global__ void __launch_bounds__(256) sum_kernel(const float *part, int nparts,
             for (int i = 0; i < 8; ++i) acc += t[i];
         }
         for (; k < nparts; k += 8) acc += *reinterpret_cast<const f32x4 *>(at + k * stride);
-    } else if (o < first + C) {
+    } else if (base) {
         for (int k = j; k < nparts; k += 8) {
             const float *at = part + o + k * stride;
             f32x4 t[4];
@@ -437,15 +451,13 @@ __global__ void __launch_bounds__(256) sum_kernel(const float *part, int nparts,
     }
     buf[j][qx] = acc;
     __syncthreads();
-    if (j == 0 && o < first + C) {
+    if (j == 0 && base) {
         f32x4 v = buf[0][qx];
 #pragma unroll
         for (int i = 1; i < 8; ++i) v += buf[i][qx];
-        float *out = o < NW ? gw1 + o : o < 2 * NW ? gw2 + (o - NW) : o < first ? (gb1 ? gb1 + (o - 2 * NW) : nullptr)
-                                                                            : (gb2 ? gb2 + (o - first) : nullptr);
-        if (out)
+        float *out = base + (o < NW ? o : o < 2 * NW ? o - NW : o < first ? o - 2 * NW : o - first);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) out[i] = v[i];
+        for (int i = 0; i < 4; ++i) out[i] = v[i];
     }
 }
 

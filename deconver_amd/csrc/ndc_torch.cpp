@@ -874,7 +874,7 @@ struct Mlp : public torch::autograd::Function<Mlp> {
         Tensor z, a;
         const Tensor b1f = f32_vector(b1);
         const Matrix m1(w1, false), m2(w2, false);
-        // (the one-kernel backward makes all gradients at once: taken where they are all wanted)
+        // (the backward forms the hidden tensor again, which pays where all gradients may be wanted)
         const bool on_chip = wants_grad(x) && wants_grad(w1) && wants_grad(w2) && mlp_on_chip(x, m1, m2);
         Tensor y = run(x, m1, b1f, m2, f32_vector(b2), residual ? *residual : Tensor(), true, on_chip, z, a, scope.stream);
         ctx->save_for_backward({x, z, a, w1, w2, b1f});   // (z, a undefined: the hidden tensor stayed on chip)
@@ -905,8 +905,9 @@ struct Mlp : public torch::autograd::Function<Mlp> {
             const Tensor xa = aligned(x), ga = aligned(gy);
             const bool half = w1.m.scalar_type() == at::kBFloat16 && w2.m.scalar_type() == at::kBFloat16;
             const Tensor m1 = half ? w1.m : w1.m.to(at::kFloat), m2 = half ? w2.m : w2.m.to(at::kFloat);
-            gx = empty(x.sizes(), x);
-            gw1 = empty_f32(m1.sizes(), x), gw2 = empty_f32(m2.sizes(), x);
+            if (need[0]) gx = empty(x.sizes(), x);
+            if (need[1]) gw1 = empty_f32(m1.sizes(), x);
+            if (need[3]) gw2 = empty_f32(m2.sizes(), x);
             if (need[2]) gb1 = empty_f32({hidden}, x);
             if (need[4]) gb2 = empty_f32({w2.cout()}, x);
             const size_t bytes = ndc_mlp_workspace_bytes(B, x.size(1), nv);
@@ -916,8 +917,9 @@ struct Mlp : public torch::autograd::Function<Mlp> {
                   "ndc_mlp_backward");
             if (gb1.defined()) gb1 = gb1.to((at::ScalarType)cfg[3]);
             if (gb2.defined()) gb2 = gb2.to((at::ScalarType)cfg[4]);
-            return once({gx, gw1.to(v[3].scalar_type()).view(v[3].sizes()), gb1, gw2.to(v[4].scalar_type()).view(v[4].sizes()), gb2,
-                         need[5] ? gy : Tensor()}, recording, gouts);
+            if (gw1.defined()) gw1 = gw1.to(v[3].scalar_type()).view(v[3].sizes());
+            if (gw2.defined()) gw2 = gw2.to(v[4].scalar_type()).view(v[4].sizes());
+            return once({gx, gw1, gb1, gw2, gb2, need[5] ? gy : Tensor()}, recording, gouts);
         }
         const Tensor z = check_saved(v[1], gy, {B, hidden, nv}, gy.scalar_type()), a = check_saved(v[2], z);
         if (need[3]) gw2 = weight_grad(gy, a, w2, v[4].sizes(), v[4].scalar_type(), need[4] ? &gb2 : nullptr, scope.stream);

@@ -491,8 +491,8 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
  *   b1, b2      float32 or NULL; residual: y's shape, or NULL; y may be residual
  *   stats       NULL, or the (mean, 1 / deviation) pairs of the rows of x (ndc_rownorm_stats, 16-byte
  *               aligned): the MLP is then of the normalised x; residual is not NULL
- *   gw1, gw2    float32, shapes of W1 and W2; gb1, gb2 float32, or NULL; gb1 is summed before the
- *               hidden tensor's gradient is rounded
+ *   gx, gw1, gb1, gw2, gb2   the gradients, each NULL where it is not wanted; gx of x's shape, the others
+ *               float32; gb1 is summed before the hidden tensor's gradient is rounded
  *   workspace   ndc_mlp_workspace_bytes(batch, c, n) bytes, 16-byte aligned
  *   x, gy, gx   16-byte aligned for the backward, word-aligned for the forward; gx is neither x nor gy
  */

@@ -134,6 +134,21 @@ def test_tiles_of_two_wavefronts(B, n, bias, residual, wdtype):
     test_hidden_tensor_on_chip(B, 32, n, bias, residual, wdtype)
 
 
+@pytest.mark.parametrize("c,n", [(32, 4096 + 64), (64, 32768)])
+def test_some_of_the_gradients(c, n):
+    """Where only some are asked for they are the same as among all."""
+    gen = torch.Generator(device="cuda").manual_seed(c)
+    rand = lambda *s: torch.randn(*s, generator=gen, device="cuda")   # noqa: E731
+    leaves = [t.requires_grad_(True) for t in (rand(1, c, n).bfloat16(), rand(4 * c, c) / c ** 0.5, rand(4 * c), rand(c, 4 * c) / c, rand(c))]
+    g = rand(1, c, n).bfloat16()
+    y = _lib.get_native().mlp(*leaves, None)
+    want = torch.autograd.grad(y, leaves, g, retain_graph=True)
+    for some in ((0,), (3,), (4,), (3, 4), (1,), (2,), (1, 2, 3, 4), (0, 1, 2), (0, 4), (0, 3), (1, 3)):
+        print("case", c, some, flush=True)
+        for i, a in zip(some, torch.autograd.grad(y, [leaves[i] for i in some], g, retain_graph=True)):
+            assert torch.equal(a, want[i]), (some, i)
+
+
 @pytest.mark.parametrize("frozen", ["x", "w1", "w2"])
 def test_partly_frozen_mlp_gives_the_same_gradients(frozen):
     gen = torch.Generator(device="cuda").manual_seed(1)
