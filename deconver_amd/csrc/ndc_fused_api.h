@@ -130,8 +130,18 @@ static const long long kSplitWavesF = NDC_SPLIT_F, kSplitWavesB = NDC_SPLIT_B;
 //             (1.6 M) 59 -> 46, 8 x 256 x 32^2 (2.1 M) 76 -> 41; 8 x 128 x 64^2 (4.2 M) 85 -> 85, 8 x 64 x 128^2 129 -> 164
 //   backward  32 x 64^2 48 -> 20, 512 x 13 x 11 73 -> 21, 32 x 128^2 67 -> 49, 4 x 64 x 50 x 70 (0.9 M) 87 -> 84,
 //             8 x 256 x 32^2 (2.1 M) 148 -> 101; 32 x 208 x 176 (1.2 M) 89 -> 95, 8 x 128 x 64^2 175 -> 235
-static const long long kPixelsF = 1700 * 1000, kSmallImagesF = 3000 * 1000;
+// A tile costs the same where it is part empty, so the pixels that tiles cover count too, and a march costs whole
+// wavefronts across a row.  5x5: 8 x 281 x 33 x 34 covers 6.9 M pixels and took 92 -> 112 forward, 8 x 129 x 43 x 66
+// 5.3 M and 111 -> 94.  3x3 marches on fewer products a pixel: tiles up to 0.85 M covered pixels forward and 0.65 M
+// backward, or where they cover clearly fewer than the march has lanes.  us, 3x3, float32, marching -> tiles, with
+// covered pixels / lanes:
+//   forward             80 x 80 x 83 (0.61 M) 19 -> 13, 8 x 49 x 27 x 49 (0.80 M) 17.6 -> 14.0, 8 x 662 x 13 x 17
+//                       (2.4 / 4.4 M) 48 -> 30, 8 x 35 x 58 x 65 (1.4 / 2.1 M) 33 -> 27, 8 x 126 x 51 x 58 (4.1 / 3.3 M) 42 -> 56
+//   forward + backward  184 x 41 x 34 (0.57 M) 46 -> 45, 8 x 91 x 19 x 33 (0.70 / 0.89 M) 63 -> 68,
+//                       8 x 64 x 33 x 33 (1.6 / 1.1 M) 67 -> 81, 8 x 213 x 27 x 34 (2.3 / 2.9 M) 108 -> 143
+static const long long kPixelsF = 1700 * 1000, kSmallImagesF = 3000 * 1000, kCoveredF = 5500 * 1000;
 static const long long kPixelsB = 900 * 1000, kSmallImagesB = 2500 * 1000;
+static const long long kCovered3F = 850 * 1000, kCovered3B = 650 * 1000;
 
 struct Plan {
     Variant v;
@@ -307,8 +317,18 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
     pl.nblk_f2 = pl.nblk_b2 = 0;
     if (q.sc == 4 && make_tile_2d(pl.m, nbc, pl.t2)) {
         const long long image = (long long)pl.m.D * pl.m.W, pixels = nbc * image;
+        const long long covered = nbc * pl.t2.ntile * pl.t2.P * pl.t2.TH;
+        // (a lane takes two columns from 128 on where the width is even; whether the call's pointers allow that
+        // does not count, so that every plan of a geometry agrees)
+        const long long lanes = nbc * pl.m.D * round_up(pl.m.W < 128 || pl.m.W % 2 ? pl.m.W : pl.m.W / 2, 64);
         pl.small_f = pixels <= kPixelsF || (image <= 64 * 64 && pixels <= kSmallImagesF);
         pl.small_b = pixels <= kPixelsB || (image <= 32 * 32 && pixels <= kSmallImagesB);
+        if (pl.m.KW == 3) {
+            pl.small_f = pl.small_f && (covered <= kCovered3F || 100 * covered <= 72 * lanes);
+            pl.small_b = pl.small_b && (covered <= kCovered3B || 100 * covered <= 60 * lanes);
+        } else {
+            pl.small_f = pl.small_f && covered <= kCoveredF;
+        }
         pl.t2.PL = pairs_ok && pl.m.W % 2 == 0;   // pixels go in and out by pairs
         if (pl.small_f) pl.nblk_f2 = (int)(nbc * pl.t2.ntile);
         if (pl.small_b) pl.nblk_b2 = (int)(nbc * ((pl.t2.ntile + pl.t2.SEG - 1) / pl.t2.SEG));
@@ -319,8 +339,8 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
 // The column-pair variants hold more of a row per workgroup: where their LDS need exceeds a
 // workgroup's share (wide rows of a tall image) the one-column variants may still fit, and
 // those are what supported() answers for.
-// matrix: the call runs the matrix-instruction family where it covers the geometry (the
-// launch shapes, workspace sizes and table sizes are the same for both families)
+// matrix: the call runs the matrix-instruction family where it covers the geometry (its launch shapes
+// are its own, the filter's table is the same, and workspace sizes serve both)
 static inline bool make_plan_fresh(const KGeom &q, Plan &pl, bool pairs_ok, int dtype, bool matrix)
 {
     if (make_plan_for(q, pl, pairs_ok, dtype, matrix)) return true;

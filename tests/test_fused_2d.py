@@ -66,6 +66,20 @@ def test_tiles_on_the_gpu(geom, dtype):
     _compare(_lib.get_library(), geom, dtype, True, "cuda")
 
 
+# past the lines that covered pixels and lanes draw, and on this side of them: 3x3 in tiles one way, both ways and
+# neither, 5x5 of many part-empty tiles; even and odd widths that march by pairs and by single columns
+LINES = [(91, (3, 3), (19, 33), 8), (64, (3, 3), (33, 33), 8), (300, (3, 3), (13, 17), 8), (35, (3, 3), (58, 65), 8),
+         (40, (3, 3), (60, 130), 2), (40, (3, 3), (60, 131), 2), (281, (5, 5), (33, 34), 8), (20, (5, 5), (100, 130), 4)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("geom", LINES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_lines_on_the_gpu(geom, dtype):
+    print("case", geom, dtype, flush=True)
+    _compare(_lib.get_library(), geom, dtype, True, "cuda")
+
+
 def test_non_finite_sources_stay_where_they_are():
     """A NaN and an infinity in z at a corner and on a tile's edge reach exactly the entries of every
     result that the oracle's arithmetic carries them to."""
