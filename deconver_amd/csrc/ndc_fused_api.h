@@ -164,35 +164,48 @@ struct Plan {
 // What a launch of the 3-D kernels takes, up to a factor: the wavefronts a SIMD of the
 // busiest CU works through, times the planes a workgroup marches over.
 //   * R workgroups of a CU run at once (LDS and registers; a workgroup's wavefronts go round the
-//     four SIMDs, so six count as eight).  q resident ones take q ceil(w / 4) + 1: a SIMD with one
-//     wavefront waits for half of its time (the 1), with four hardly ever.
+//     four SIMDs, so six count as eight).  q resident ones take q ceil(w / 4) + `alone`: a SIMD with
+//     one wavefront waits for half of its time (1) or more, with four hardly ever.
 //   * a segment of the march adds the planes its neighbours own (3 more than it keeps), a row band
 //     the two halo rows it computes twice (a fifth of a strip's work each).
+//   * behind full rounds a remainder runs into the round before it: `overlap` of it costs its share of
+//     a full round, the rest a round of its own.
 //   * `mixed`: from two full rounds on, workgroups of different rounds overlap and a remainder
-//     costs its share only (the forward, whose four wavefronts per SIMD drift apart).
+//     costs its share only (the dot2 forward, whose four wavefronts per SIMD drift apart).
 // bf16 dot2 kernels: against the best of 56 launch shapes measured on each of 22 problems (16^3 ..
 // 192^3, widths 14 to 192, 32 to 512 channels) the choice is 1 % behind on average and 11 % at worst;
 // the fixed shape it replaced (256 threads, the whole march) took 1.37 (forward) and 1.24 (backward)
 // times as long on average, 2.7 times on 64 channels of 32^3 (115 / 117 / 81 -> 42 / 50 / 34 us).
-// FMA kernels (float32, odd widths): of up to 60 shapes on 13 problems (15x17x13 .. 128^3, 16 to 128
-// channels) 1 % behind (forward) and 2 % (backward) on average; the fixed 256 and 512 threads, cut into
-// segments until 4096 and 2048 wavefronts were there, left rounds of workgroups part empty: 64 channels
-// of 45x53x77 in bf16 455 / 285 -> 320 / 207 us (the two passes of the backward), 32 of 96^3 in float32
-// 905 / 562 -> 602 / 418, 32 of 95x79x93 617 -> 509 us forward; at worst 3 % slower (32 of 95x79x93, back).
-static inline double launch_cost(const Tile &t, const March &m, long long nbc, int lds_floats, int waves_per_simd,
-                                 bool mixed)
+// FMA kernels (float32, odd widths): the fixed 256 and 512 threads, cut into segments until 4096 and 2048
+// wavefronts were there, left rounds of workgroups part empty: 64 channels of 45x53x77 in bf16 455 / 285 ->
+// 320 / 207 us (the two passes of the backward), 32 of 96^3 in float32 905 / 562 -> 602 / 418.  `alone` and
+// `overlap` are fitted to those and the shapes of alone = 1, overlap = 0 on 136 problems (6 to 140 planes, 8 to 512
+// channels, batches of 1 to 4; the ratio of the two predicted within 9 % in the mean, 18 % before), since with
+// those one wavefront a SIMD that marched the whole way looked too cheap: 512 channels of 14x22x17 100 -> 133 us
+// forward, 4 x 128 of 21x15x23 164 -> 201.  On the 136 problems the choice takes 0.92 (forward) and 0.90 (with the
+// backward) of the fixed shapes' time, 1.05 at worst; with alone = 1, overlap = 0 it was 0.95 and 0.92, 1.33 at worst.
+struct CostModel {
+    int waves_per_simd;
+    double alone, overlap;
+    bool mixed;
+};
+static const CostModel kCostDot2F = {4, 1.0, 0.0, true}, kCostDot2B = {2, 1.0, 0.0, false};
+static const CostModel kCostFmaF = {3, 2.0, 0.75, false}, kCostFmaB = {2, 3.0, 0.5, false};
+
+static inline double launch_cost(const Tile &t, const March &m, long long nbc, int lds_floats, const CostModel &c)
 {
     const int w = t.NT / 64;
     int R = kMaxLdsBytes / (lds_floats * 4);
-    if (R > waves_per_simd * 4 / w) R = waves_per_simd * 4 / w;
+    if (R > c.waves_per_simd * 4 / w) R = c.waves_per_simd * 4 / w;
     if (R < 1) R = 1;
-    const double c = (double)(nbc * t.ntile * t.nseg) / 256.0, per = w > 3 ? (w + 3) / 4 : w / 4.0;
-    auto batch = [&](int q) { return q * per + 1.0; };
+    const double share = (double)(nbc * t.ntile * t.nseg) / 256.0, per = w > 3 ? (w + 3) / 4 : w / 4.0;
+    auto batch = [&](int q) { return q * per + c.alone; };
     const long long ci = (nbc * t.ntile * t.nseg + 255) / 256;
     const long long full = ci / R;
     const int rem = (int)(ci - full * R);
-    double T = full * batch(R) + (rem ? batch(rem) : 0.0);
-    if (mixed && full >= 2) T = c * batch(R) / R + 0.5 * batch(R) / R;
+    double T = full * batch(R);
+    if (rem) T += full ? (1.0 - c.overlap) * batch(rem) + c.overlap * batch(R) * rem / R : batch(rem);
+    if (c.mixed && full >= 2) T = share * batch(R) / R + 0.5 * batch(R) / R;
     const int planes = (t.SEG < m.D ? t.SEG : m.D) + (t.nseg > 1 ? 3 : 1);
     return planes * (1.0 + 0.4 / t.S) * T;
 }
@@ -201,9 +214,9 @@ static inline double launch_cost(const Tile &t, const March &m, long long nbc, i
 // even number of planes, `min_planes` at least) with the smallest cost.  K: the kernel whose LDS need counts.
 template <class K, int N>
 static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, const int (&targets)[N], int min_strips,
-                             int min_planes, int waves_per_simd, bool mixed, Tile &best)
+                             int min_planes, const CostModel &model, Tile &best)
 {
-    static const int parts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
+    static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 24, 28, 32};
     double least = 0.0;
     bool found = false;
     for (int target : targets) {
@@ -215,7 +228,7 @@ static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, cons
             if (n > 1 && m.D < min_planes * n) break;
             t.SEG = n == 1 ? m.D : round_up((m.D + n - 1) / n, 2);
             t.nseg = (m.D + t.SEG - 1) / t.SEG;
-            const double cost = launch_cost(t, m, nbc, lds, waves_per_simd, mixed);
+            const double cost = launch_cost(t, m, nbc, lds, model);
             if (!found || cost < least) {
                 found = true;
                 least = cost;
@@ -234,8 +247,8 @@ static inline void plan_lds(Plan &pl, long long nbc)
         const Tuning tn = tuning();
         const int targets_f[4] = {64, 128, tn.threads_f, 512}, targets_b[3] = {128, 256, tn.threads_b};
         if (tn.split) {
-            cost_tile<FwdKernel<KD, KH, KW, SC, RHF, RWF, float>>(pl.m, RHF, RWF, nbc, targets_f, 0, 4, 3, false, pl.tf);
-            cost_tile<Bwd1Kernel<KD, KH, KW, SC, RHB, RWB, float>>(pl.m, RHB, RWB, nbc, targets_b, 0, 4, 2, false, pl.tb);
+            cost_tile<FwdKernel<KD, KH, KW, SC, RHF, RWF, float>>(pl.m, RHF, RWF, nbc, targets_f, 0, 4, kCostFmaF, pl.tf);
+            cost_tile<Bwd1Kernel<KD, KH, KW, SC, RHB, RWB, float>>(pl.m, RHB, RWB, nbc, targets_b, 0, 4, kCostFmaB, pl.tb);
         }
     }
     pl.lds_f = FwdKernel<KD, KH, KW, SC, RHF, RWF, float>::lds_floats(pl.tf);
@@ -280,8 +293,8 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
         const bool fits = whole ? make_tile(pl.m, kDot2RH, 2, tn.threads_f2, tf, FwdKernelB<kDot2RH>::kMinStrips) &&
                                       make_tile(pl.m, kDot2RH, 2, tn.threads_b2, tb)
                                 : cost_tile<FwdKernelB<kDot2RH>>(pl.m, kDot2RH, 2, nbc, targets_f,
-                                                                 FwdKernelB<kDot2RH>::kMinStrips, 6, 4, true, tf) &&
-                                      cost_tile<Bwd1KernelB<kDot2RH, true>>(pl.m, kDot2RH, 2, nbc, targets_b, 0, 6, 2, false, tb);
+                                                                 FwdKernelB<kDot2RH>::kMinStrips, 6, kCostDot2F, tf) &&
+                                      cost_tile<Bwd1KernelB<kDot2RH, true>>(pl.m, kDot2RH, 2, nbc, targets_b, 0, 6, kCostDot2B, tb);
         if (fits) {
             const int lf = FwdKernelB<kDot2RH>::lds_floats(tf);
             const int l1 = Bwd1KernelB<kDot2RH>::lds_floats(tb);
