@@ -790,8 +790,10 @@ struct Backend {
     {
         hipLaunchKernelGGL(loss::sums_kernel, dim3((unsigned)(rows * parts)), dim3(loss::kThreads), 0, (hipStream_t)stream, l, y,
                            (float4 *)partial, n, parts, chunk);
+        int log_width = 0;
+        while ((1 << log_width) < parts && log_width < 6) ++log_width;
         hipLaunchKernelGGL(loss::finish_kernel, dim3(1), dim3(loss::kFinish), 0, (hipStream_t)stream, (const float4 *)partial,
-                           (float2 *)coef, loss, rows, parts, 1.f / ((float)rows * (float)n));
+                           (float2 *)coef, loss, rows, parts, log_width, 1.f / ((float)rows * (float)n));
         return check();
     }
     static int dice_bce_backward(const float *l, const float *y, const float *coef, const float *g, float *gl, int rows, long long n,

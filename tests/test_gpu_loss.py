@@ -44,6 +44,12 @@ def test_loss_and_gradient(shape, dtype):
         assert torch.equal(T.dice_bce_loss(logits, target), loss.detach())
 
 
+# (rows, n): a lane a row, two, four (with one idle), rows past the last trip, a wavefront a row and more parts than lanes
+@pytest.mark.parametrize("shape", [(64, 16, 64), (64, 16, 5000), (100, 1, 6144), (37, 9, 8192), (5, 1, 81920), (1, 3, 160000)])
+def test_parts_of_a_row(shape):
+    test_loss_and_gradient(shape, torch.float32)
+
+
 def test_forms_it_keeps():
     gen = torch.Generator().manual_seed(5)
     logits = torch.randn(2, 3, 10, 12, generator=gen).cuda()
