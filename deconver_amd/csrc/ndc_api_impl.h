@@ -833,8 +833,11 @@ static ndc::WgradPlan wgrad_plan(long long batch, long long rows, long long cols
     // sum, float32 / bf16: 64 x 64 over 256 voxels 6.4 -> 3.6 / 5.4 -> 3.1, over 1024 6.5 -> 6.2 / 5.7 -> 4.4,
     // over 2048 7.2 -> 9.6 / 6.3 -> 6.1; 512 x 512 over 512 in tiles of 32 13.4 -> 6.7 / 11.7 -> 4.7 (in tiles
     // of 16 10.7 / 7.4).  Rows that end within 16 bytes read their last turns element by element: 512 x 512
-    // over 500 13.0 -> 7.0 / 10.8 -> 4.3, 64 x 64 over 3 x 343 7.1 -> 4.9 / 8.6 -> 9.8.
-    if (batch * w.per_sample > 1 && batch * n <= (n * esz % 16 ? 512 : 1024)) {
+    // over 500 13.0 -> 7.0 / 10.8 -> 4.3, 64 x 64 over 3 x 343 7.1 -> 4.9 / 8.6 -> 9.8.  More than 16 samples
+    // spread over the chip by themselves unless the result is large: with the projection itself, over 64 x 16
+    // voxels, 32 x 32 in bf16 10.5 -> 21, 256 x 256 28.5 -> 14.8 / 26.3 -> 23.9, 512 x 512 64 -> 38 / 54 -> 18.
+    const bool ragged = n * esz % 16 != 0;
+    if (batch * w.per_sample > 1 && batch * n <= (ragged ? 512 : 1024) && (batch <= 16 || rows * cols >= 64 * 1024)) {
         w.per_sample = 0, w.bm = w.bn = 16;
         if (tiles_of() > 256) w.bm = w.bn = 32;
     }

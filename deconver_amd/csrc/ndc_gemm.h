@@ -262,8 +262,11 @@ __global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
 // partial results and no second launch to add them: what these sizes cost is launches and the latency of
 // one, and between two launches of a recorded step lie 1-2 us besides.  Tiles of 16 as long as that
 // gives each CU one: it multiplies 1024 voxels of a 32 x 32 tile in float32 in 3.4 us.
+// MANY: the turns of all samples are one count, of which each wavefront has four in flight; one sample after the
+// other, 64 samples of 16 voxels waited 64 times (32 x 32 in bf16, with the projection itself, 94 us; 21 like this).
+// For few samples the plain loops are the shorter code: 32 x 32 over 2 x 250 in float32 7.0 us against 7.8.
 static const int kWholeWaves = 16;
-template <typename T, int TL> __global__ void __launch_bounds__(64 * kWholeWaves) wgrad_whole_kernel(WgradParams p)
+template <typename T, int TL, bool MANY> __global__ void __launch_bounds__(64 * kWholeWaves) wgrad_whole_kernel(WgradParams p)
 {
     typedef Gran<T> G;
     typedef std::conditional_t<TL == 32, f32x16, f32x4> Acc;
@@ -283,23 +286,48 @@ template <typename T, int TL> __global__ void __launch_bounds__(64 * kWholeWaves
         if (want_sums) sum += G::sum(fa);
         acc = G::mma(fa, fb, acc);
     };
-    for (int s = 0; s < p.splits; ++s) {   // samples
-        const T *as = a + (long long)s * p.rows * p.n, *bs = b + (long long)s * p.cols * p.n;
-        int i = wave;
-        for (; i + 3 * NW < full; i += 4 * NW) {
+    if constexpr (MANY) {
+        const int turns = (int)((p.n + Q * E - 1) / (Q * E)), total = p.splits * turns;
+        for (int k = wave; k < total; k += 4 * NW) {
             u32x4 fa[4], fb[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                fa[u] = *(const u32x4_a2 *)(as + (i + u * NW) * Q * E);
-                fb[u] = *(const u32x4_a2 *)(bs + (i + u * NW) * Q * E);
+                const int at = k + u * NW, s = at / turns, i = at - s * turns;
+                fa[u] = fb[u] = u32x4{};
+                if (at >= total) continue;
+                const T *as = a + (long long)s * p.rows * p.n + i * Q * E, *bs = b + (long long)s * p.cols * p.n + i * Q * E;
+                if (i < full) {
+                    fa[u] = *(const u32x4_a2 *)as;
+                    fb[u] = *(const u32x4_a2 *)bs;
+                } else {   // voxels past the whole turns
+                    const int rest = (int)p.n - (i * Q + kb) * E, have = rest < 0 ? 0 : rest < E ? rest : E;
+                    fa[u] = ragged<T>(as, have);
+                    fb[u] = ragged<T>(bs, have);
+                }
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) add(fa[u], fb[u]);
+            for (int u = 0; u < 4; ++u)
+                if (k + u * NW < total) add(fa[u], fb[u]);
         }
-        for (; i < full; i += NW) add(*(const u32x4_a2 *)(as + i * Q * E), *(const u32x4_a2 *)(bs + i * Q * E));
-        if (i == full && p.n % (Q * E)) {   // voxels past the whole turns
-            const int rest = (int)p.n - (i * Q + kb) * E, have = rest < 0 ? 0 : rest < E ? rest : E;
-            add(ragged<T>(as + i * Q * E, have), ragged<T>(bs + i * Q * E, have));
+    } else {
+        for (int s = 0; s < p.splits; ++s) {   // samples
+            const T *as = a + (long long)s * p.rows * p.n, *bs = b + (long long)s * p.cols * p.n;
+            int i = wave;
+            for (; i + 3 * NW < full; i += 4 * NW) {
+                u32x4 fa[4], fb[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    fa[u] = *(const u32x4_a2 *)(as + (i + u * NW) * Q * E);
+                    fb[u] = *(const u32x4_a2 *)(bs + (i + u * NW) * Q * E);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) add(fa[u], fb[u]);
+            }
+            for (; i < full; i += NW) add(*(const u32x4_a2 *)(as + i * Q * E), *(const u32x4_a2 *)(bs + i * Q * E));
+            if (i == full && p.n % (Q * E)) {   // voxels past the whole turns
+                const int rest = (int)p.n - (i * Q + kb) * E, have = rest < 0 ? 0 : rest < E ? rest : E;
+                add(ragged<T>(as + i * Q * E, have), ragged<T>(bs + i * Q * E, have));
+            }
         }
     }
 #pragma unroll

@@ -33,8 +33,15 @@ int wgrad(const void *a, const void *b, float *gw, float *gb, float *part, long 
         p.tiles_m = (rows + plan.bm - 1) / plan.bm, p.tiles_n = (cols + plan.bn - 1) / plan.bn, p.splits = (int)batch;
         const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * kWholeWaves);
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, p); };
-        if (plan.bm == 32) esz == 4 ? launch(wgrad_whole_kernel<float, 32>) : launch(wgrad_whole_kernel<bf16_t, 32>);
-        else esz == 4 ? launch(wgrad_whole_kernel<float, 16>) : launch(wgrad_whole_kernel<bf16_t, 16>);
+        auto by_tile = [&](auto type, auto many) {
+            typedef decltype(type) T;
+            if (plan.bm == 32) launch(wgrad_whole_kernel<T, 32, decltype(many)::value>);
+            else launch(wgrad_whole_kernel<T, 16, decltype(many)::value>);
+        };
+        auto by_samples = [&](auto type) {
+            batch > (n * esz % 16 ? 3 : 8) ? by_tile(type, std::true_type()) : by_tile(type, std::false_type());
+        };
+        if (esz == 4) by_samples(0.f); else by_samples(bf16_t());
         return 0;
     }
     p.a = a, p.b = b, p.part = part, p.gw = gw, p.gb = gb, p.n = n, p.chunk = plan.chunk, p.rows = rows, p.cols = cols;

@@ -31,3 +31,10 @@ def test_weight_gradient_of_few_voxels(rows, cols, batch, n, dtype):
     assert bool(((gb.cpu().double() - g64.sum((0, 2))).abs() <= bound * g64.abs().sum((0, 2)) + 1e-30).all())
     again, none = ops.weight_grad(_lib.get_library(), g, x)
     assert none is None and torch.equal(again, gw)
+
+
+# the most samples of the form without splits, and one more
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch,n", [(8, 64), (9, 64), (2, 27), (3, 27), (4, 27), (5, 27), (64, 16), (128, 1)])
+def test_many_samples(batch, n, dtype):
+    test_weight_gradient_of_few_voxels(17, 33, batch, n, dtype)
