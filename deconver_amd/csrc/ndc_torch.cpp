@@ -720,16 +720,22 @@ Tensor projected_update(const Tensor &x, const Tensor &weight, const Tensor &h, 
 // ---------------------------------------------------------------------------- projection with its tail
 
 // Whether a bare float32 product that narrows (a stage's adapter, a downsampling; nobody's but its node's) is
-// the tiled GEMM's.  The library takes a few workgroups for up to some 250 voxels a sample -- 512 -> 256 channels
-// over 256 voxels 119 us against 6 tiled, 512 -> 128 over 8 x 194 69 against 8.5, 384 -> 192 over 241 82 against
-// 5.3 --, above that it is ahead but in small products: 512 -> 256 over 2048 9.1 against 14.7, 384 -> 192 over 2714
-// 8.2 against 13.5, 96 -> 48 over 2 x 2737 5.5 against 6.4; 128 -> 64 over 3295 5.9 against 5.0, 512 -> 256 over 500
-// 7.1 against 6.2.  With 1024 channels it was ahead at every size (over 16 voxels 6.4 against 8.3, 1024 14 against 23).
+// the tiled GEMM's.  The library has one workgroup for a sample of up to some 250 voxels, whose time grows with
+// them, and is ahead where many samples fill the chip with those while the tiled GEMM's 64-voxel columns are part
+// empty.  us, library / tiled: 512 -> 256 channels over 256 voxels 119 / 6, over 16 x 256 119 / 18, over 128 x 16
+// 22 / 30, over 64 x 4 13 / 17; 384 -> 192 over 241 82 / 5.3; 256 -> 128 over 64 x 16 9.5 / 6.0, over 256 x 16 9.4 / 18.
+// Beyond 256 voxels the tiled GEMM is ahead in small products: 512 -> 256 over 2048 9.1 / 14.7, 384 -> 192 over 2714
+// 8.2 / 13.5, 96 -> 48 over 2 x 2737 5.5 / 6.4; 128 -> 64 over 3295 5.9 / 5.0, 256 -> 128 over 370 5.6 / 4.7.  With 768
+// channels it is only in those (over 131 7.1 / 7.2, 16 x 128 13.6 / 23), with 1024 nowhere (over 16 6.4 / 8.3, 1024 13 / 23).
 bool narrow_is_tiled(int64_t B, int64_t cin, int64_t cout, int64_t n)
 {
     if (cin <= cout || cin > 768) return false;
-    const double flops = 2.0 * (double)B * (double)n * (double)cin * (double)cout;
-    return (n <= 256 && flops < 0.5e9) || (B * n <= 5000 && flops < 0.1e9);
+    const double weights = 2.0 * (double)cin * (double)cout;
+    const bool small = weights * (double)B * (double)n < 0.1e9;
+    if (n > 256) return B * n <= 5000 && small;
+    const int64_t columns = B * ((n + 63) / 64 * 64);
+    if (columns > 4200 + 145 * n) return false;
+    return cin <= 512 ? n >= 16 || weights * (double)columns < 1e9 : small;
 }
 
 // y[b] = act(W x[b] + bias) + residual[b] on channel-first (B, C, n) tensors.  keep: the
