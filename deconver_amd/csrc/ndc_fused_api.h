@@ -216,7 +216,6 @@ template <class K, int N>
 static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, const int (&targets)[N], int min_strips,
                              int min_planes, const CostModel &model, Tile &best)
 {
-    static const int parts[] = {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 24, 28, 32};
     double least = 0.0;
     bool found = false;
     for (int target : targets) {
@@ -224,9 +223,12 @@ static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, cons
         if (!make_tile(m, RH, RW, target, t, min_strips)) continue;
         const int lds = K::lds_floats(t);
         if (lds * 4 > kMaxLdsBytes) continue;
-        for (int n : parts) {
+        int last = 0;
+        for (int n = 1; n <= 32; ++n) {
             if (n > 1 && m.D < min_planes * n) break;
             t.SEG = n == 1 ? m.D : round_up((m.D + n - 1) / n, 2);
+            if (t.SEG == last) continue;
+            last = t.SEG;
             t.nseg = (m.D + t.SEG - 1) / t.SEG;
             const double cost = launch_cost(t, m, nbc, lds, model);
             if (!found || cost < least) {
