@@ -59,6 +59,47 @@ def test_steps(sizes):
         assert scale(p.detach().cpu().double() - q.detach()) <= 20 * 2.0 ** -24 * (scale(q.detach()) + 1)
 
 
+@pytest.mark.parametrize("offset", [1, 2, 3])
+@pytest.mark.parametrize("which", ["param", "grad"])
+def test_views_of_a_flat_buffer(offset, which):
+    """Parameters or gradients that no 16-byte access takes: element by element from the first on, with less
+    than a workgroup's share, exactly one, and one and a part."""
+    sizes = [(4095,), (4096,), (4097,), (33, 300), (1,)]
+    flat = torch.empty(offset + sum(torch.Size(s).numel() for s in sizes) + 4 * len(sizes), device="cuda")
+    views, at = [], offset
+    for s in sizes:
+        n = torch.Size(s).numel()
+        views.append(flat[at:at + n].view(s))
+        at += (n + 3) // 4 * 4        # (all as far from 16 bytes as the first)
+    assert all(v.data_ptr() % 16 == 4 * offset for v in views)
+    bag = _Bag(sizes).cuda()
+    ref = copy.deepcopy(bag).cpu().double()
+    if which == "param":
+        for p, v in zip(bag.p, views):
+            v.copy_(p.detach())
+            p.data = v
+    opt = T.make_optimizer(bag)
+    want = torch.optim.AdamW(ref.parameters(), lr=1e-3, weight_decay=1e-2)
+    for step in range(5):
+        _grads(bag, step), _grads(ref, step)
+        if which == "grad":
+            for p, v in zip(bag.p, views):
+                p.grad = v.copy_(p.grad)
+        if step:
+            assert opt._kernel_step()
+        else:
+            opt.step()
+        want.step()
+    for i, (p, q) in enumerate(zip(bag.p, ref.parameters())):
+        s, r = opt.state[p], want.state[q]
+        assert float(s["step"]) == float(r["step"])
+        # as in test_steps
+        scale = lambda t: float(t.abs().max())      # noqa: E731
+        assert scale(s["exp_avg"].cpu().double() - r["exp_avg"]) <= 20 * 2.0 ** -24 * 10.0 ** (i % 7 - 3) * 5
+        assert scale(s["exp_avg_sq"].cpu().double() - r["exp_avg_sq"]) <= 20 * 2.0 ** -24 * scale(r["exp_avg_sq"])
+        assert scale(p.detach().cpu().double() - q.detach()) <= 20 * 2.0 ** -24 * (scale(q.detach()) + 1)
+
+
 def test_what_the_base_class_does():
     """Forms the kernel declines, and hooks, run once."""
     count = []
