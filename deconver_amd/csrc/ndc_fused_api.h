@@ -143,6 +143,11 @@ static const long long kPixelsF = 1700 * 1000, kSmallImagesF = 3000 * 1000, kCov
 static const long long kPixelsB = 900 * 1000, kSmallImagesB = 2500 * 1000;
 static const long long kCovered3F = 850 * 1000, kCovered3B = 650 * 1000;
 
+// (0 in a host build whose tests send every image down the march)
+#ifndef NDC_TILES_2D
+#define NDC_TILES_2D 1
+#endif
+
 struct Plan {
     Variant v;
     March m;
@@ -330,7 +335,7 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
     pl.nblk_b = (int)nb;
     pl.small_f = pl.small_b = false;
     pl.nblk_f2 = pl.nblk_b2 = 0;
-    if (q.sc == 4 && make_tile_2d(pl.m, nbc, pl.t2)) {
+    if (NDC_TILES_2D && q.sc == 4 && make_tile_2d(pl.m, nbc, pl.t2)) {
         const long long image = (long long)pl.m.D * pl.m.W, pixels = nbc * image;
         const long long covered = nbc * pl.t2.ntile * pl.t2.P * pl.t2.TH;
         // (a lane takes two columns from 128 on where the width is even; whether the call's pointers allow that
@@ -373,7 +378,7 @@ static inline bool make_plan(const KGeom &q, Plan &pl, bool pairs_ok = true, int
 #else
     static const int kWords = 11, kEntries = 64;
     const int key[kWords] = {q.B,  q.G,  q.m,  q.sc, q.D, q.H,
-                             q.W, q.kD, q.kH, q.kW, pairs_ok * 4 + matrix * 2 + (dtype == NDC_BF16)};
+                             q.W, q.kD, q.kH, q.kW, NDC_TILES_2D * 8 + pairs_ok * 4 + matrix * 2 + (dtype == NDC_BF16)};
     struct Entry {
         int key[kWords];   // zeros where nothing is kept (a geometry has B >= 1)
         bool ok;

@@ -523,8 +523,12 @@ struct Backend {
     }
 };
 
+// whether small images run tile by tile, as on the GPU, or march
+static int host_tiles_2d = 1;
+
 }  // namespace ndc
 
+#define NDC_TILES_2D ndc::host_tiles_2d
 #include "ndc_api_impl.h"
 
 // LDS faults (races, out-of-bounds, uninitialised reads) seen by the host execution since
@@ -539,3 +543,6 @@ extern "C" long long ndc_host_faults(char *first, int n)
     f = ndc::HostFaults();
     return total;
 }
+
+// Test hook of the host build only: 0 sends every 2-D problem down the marching kernels.
+extern "C" void ndc_host_tiles_2d(int on) { ndc::host_tiles_2d = on ? 1 : 0; }

@@ -1,5 +1,6 @@
 """Shared helpers of the test-suite."""
 
+import contextlib
 import os
 
 import torch
@@ -45,3 +46,13 @@ def host_faults(lib) -> tuple:
     fn.restype = ctypes.c_longlong
     n = fn(buf, 256)
     return n, buf.value.decode()
+
+
+@contextlib.contextmanager
+def host_march(lib):
+    """The host build with every 2-D problem on the marching kernels, which otherwise serve large images."""
+    lib._dll.ndc_host_tiles_2d(0)
+    try:
+        yield
+    finally:
+        lib._dll.ndc_host_tiles_2d(1)

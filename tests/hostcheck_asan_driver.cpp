@@ -140,19 +140,26 @@ int main()
         {2, 3, 1, 4, 1, 9, 12, 1, 5, 5, NDC_F32, NDC_PATH_FUSED},
         {1, 2, 1, 4, 1, 3, 70, 1, 5, 5, NDC_BF16, NDC_PATH_FUSED},
         {2, 2, 1, 4, 1, 7, 9, 1, 3, 3, NDC_F32, NDC_PATH_FUSED},
+        {1, 1, 1, 4, 1, 40, 49, 1, 5, 5, NDC_F32, NDC_PATH_FUSED},    // several tiles, cut ones; several segments
+        {1, 1, 1, 4, 1, 33, 130, 1, 3, 3, NDC_BF16, NDC_PATH_FUSED},  // column pairs
         {1, 2, 1, 4, 2, 40, 33, 3, 3, 3, NDC_F32, NDC_PATH_FUSED},
         {2, 3, 2, 2, 5, 4, 3, 3, 3, 3, NDC_F32, NDC_PATH_DIRECT},
         {1, 2, 3, 2, 1, 6, 5, 1, 3, 5, NDC_BF16, NDC_PATH_DIRECT},
     };
     int bad = 0;
     for (const Case &c : cases) {
-        const int st = run_case(c);
-        char first[256];
-        const long long faults = ndc_host_faults(first, sizeof first);
-        printf("case B%d G%d m%d sc%d %dx%dx%d k%dx%dx%d dtype%d path%d -> status %d, lds faults %lld %s\n",
-               c.B, c.G, c.m, c.sc, c.D, c.H, c.W, c.kD, c.kH, c.kW, c.dtype, c.path, st, faults, first);
-        if (st || faults) ++bad;
+        // (2-D: in tiles, then down the march of large images)
+        for (int march = 0; march < (c.D == 1 && c.kD == 1 && c.path == NDC_PATH_FUSED ? 2 : 1); ++march) {
+            ndc_host_tiles_2d(!march);
+            const int st = run_case(c);
+            char first[256];
+            const long long faults = ndc_host_faults(first, sizeof first);
+            printf("case B%d G%d m%d sc%d %dx%dx%d k%dx%dx%d dtype%d path%d march%d -> status %d, lds faults %lld %s\n",
+                   c.B, c.G, c.m, c.sc, c.D, c.H, c.W, c.kD, c.kH, c.kW, c.dtype, c.path, march, st, faults, first);
+            if (st || faults) ++bad;
+        }
     }
+    ndc_host_tiles_2d(1);
     if (run_block_level(NDC_F32)) ++bad;
     if (run_block_level(NDC_BF16)) ++bad;
     return bad ? 1 : 0;

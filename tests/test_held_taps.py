@@ -1,6 +1,5 @@
-"""The 2-D forward with its taps in registers (launches of at most two wavefronts per SIMD, one column
-per thread): widths that fill no wavefront, images of few rows, several segments of the march, and a
-launch just past the rule, against the oracle in float64.  Bounds as in the other parity tests."""
+"""2-D forwards of small launches: widths that fill no wavefront, images of few rows, several tiles a row,
+and one of many images, against the oracle in float64.  Bounds as in the other parity tests."""
 
 import pytest
 import torch
@@ -12,7 +11,7 @@ from tests.helpers import hostcheck_library, make_case
 # (C, kernel, spatial, batch)
 GEOMS = [(3, (5, 5), (1, 7), 2), (2, (5, 5), (2, 1), 1), (4, (5, 5), (33, 127), 1), (2, (3, 3), (50, 64), 1),
          (5, (3, 3), (19, 65), 2), (2, (5, 5), (37, 200), 1), (3, (5, 5), (20, 301), 1)]
-PAST = [(520, (5, 5), (64, 30), 1)]          # more than 2048 wavefronts
+PAST = [(520, (5, 5), (64, 30), 1)]          # more workgroups than the chip holds at once
 TOL = {torch.float32: 1e-5, torch.bfloat16: 2e-2}
 
 
