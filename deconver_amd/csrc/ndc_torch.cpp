@@ -720,22 +720,23 @@ Tensor projected_update(const Tensor &x, const Tensor &weight, const Tensor &h, 
 // ---------------------------------------------------------------------------- projection with its tail
 
 // Whether a bare float32 product that narrows (a stage's adapter, a downsampling; nobody's but its node's) is
-// the tiled GEMM's.  The library has one workgroup for a sample of up to some 250 voxels, whose time grows with
+// the tiled GEMM's.  Up to some 250 voxels a sample the library has one workgroup for each, whose time grows with
 // them, and is ahead where many samples fill the chip with those while the tiled GEMM's 64-voxel columns are part
 // empty.  us, library / tiled: 512 -> 256 channels over 256 voxels 119 / 6, over 16 x 256 119 / 18, over 128 x 16
-// 22 / 30, over 64 x 4 13 / 17; 384 -> 192 over 241 82 / 5.3; 256 -> 128 over 64 x 16 9.5 / 6.0, over 256 x 16 9.4 / 18.
-// Beyond 256 voxels the tiled GEMM is ahead in small products: 512 -> 256 over 2048 9.1 / 14.7, 384 -> 192 over 2714
-// 8.2 / 13.5, 96 -> 48 over 2 x 2737 5.5 / 6.4; 128 -> 64 over 3295 5.9 / 5.0, 256 -> 128 over 370 5.6 / 4.7.  With 768
-// channels it is only in those (over 131 7.1 / 7.2, 16 x 128 13.6 / 23), with 1024 nowhere (over 16 6.4 / 8.3, 1024 13 / 23).
+// 22 / 30, over 64 x 4 13 / 17; 384 -> 192 over 241 82 / 5.3; 256 -> 128 over 64 x 16 9.5 / 6.0, over 256 x 16 9.4 / 18;
+// 768 -> 384 over 16 x 128 14 / 23, 1024 -> 512 over 16 6.4 / 8.3.  Beyond that the library is ahead in larger products:
+// 512 -> 256 over 500 7.1 / 6.2, over 1024 7.3 / 8.2, over 2048 9.1 / 14.7; 384 -> 192 over 1840 7.8 / 9.8, over 2714
+// 8.2 / 13.5; 1024 -> 512 over 500 9.9 / 13.4.  2 us more on the GPU (0.3 GFLOP) are less than the 10 us that a call of
+// the library takes the host longer: the 2-D network's forward on one 208 x 176 image, whose four adapters are 0.15
+// GFLOP each, takes 1.34 ms with theirs by the library and 1.23 tiled.
 bool narrow_is_tiled(int64_t B, int64_t cin, int64_t cout, int64_t n)
 {
-    if (cin <= cout || cin > 768) return false;
-    const double weights = 2.0 * (double)cin * (double)cout;
-    const bool small = weights * (double)B * (double)n < 0.1e9;
-    if (n > 256) return B * n <= 5000 && small;
+    if (cin <= cout) return false;
+    const double weights = 2.0 * (double)cin * (double)cout, least = 0.3e9;
+    if (n > 256) return weights * (double)B * (double)n < least;
     const int64_t columns = B * ((n + 63) / 64 * 64);
     if (columns > 4200 + 145 * n) return false;
-    return cin <= 512 ? n >= 16 || weights * (double)columns < 1e9 : small;
+    return weights * (double)columns < least || (cin <= 512 && (n >= 16 || weights * (double)columns < 1e9));
 }
 
 // y[b] = act(W x[b] + bias) + residual[b] on channel-first (B, C, n) tensors.  keep: the

@@ -79,10 +79,11 @@ def test_linear_module_under_autocast_keeps_float32_parameter_gradients():
 
 
 # (B, cin, cout, n, by the tiled GEMM): either side of each bound of the rule for bare float32 products that narrow
-NARROW = [(1, 512, 256, 256, True), (1, 768, 384, 131, True), (1, 1024, 512, 64, False), (1, 768, 384, 256, False),
-          (2, 768, 60, 256, True), (1, 128, 64, 5000, True), (1, 128, 64, 5001, False), (2, 64, 8, 2500, True), (2, 64, 8, 2501, False),
-          (1, 512, 256, 381, True), (1, 512, 256, 382, False), (1, 64, 64, 100, False), (101, 64, 32, 16, True), (102, 64, 32, 16, False),
-          (59, 512, 256, 4, True), (60, 512, 256, 4, False), (70, 256, 128, 4, True), (1024, 128, 64, 1, False)]
+NARROW = [(1, 512, 256, 256, True), (1, 768, 384, 131, True), (1, 1024, 512, 64, True), (1, 1024, 512, 400, False),
+          (2, 768, 60, 256, True), (2, 768, 384, 256, False), (1, 128, 64, 18310, True), (1, 128, 64, 18311, False),
+          (1, 512, 256, 1144, True), (1, 512, 256, 1145, False), (1, 64, 64, 100, False), (101, 64, 32, 16, True),
+          (102, 64, 32, 16, False), (59, 512, 256, 4, True), (60, 512, 256, 4, False), (70, 256, 128, 4, True),
+          (1024, 128, 64, 1, False), (4, 1024, 512, 8, True), (5, 1024, 512, 8, False)]
 
 
 @pytest.mark.parametrize("B,cin,cout,n,tiled", NARROW)
