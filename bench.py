@@ -903,7 +903,7 @@ def block_workload(args) -> int:
 def graphed_workload(args) -> int:
     """Training steps on ONE small sample (a 3-D step on a 32^3 volume under bf16 autocast, a 2-D
     step on a 128^2 image in float32): there a step is bound by the rate at which the host
-    launches its ~600 kernels, and replaying it from a HIP graph (training.GraphedTrainStep)
+    launches its some 300 kernels, and replaying it from a HIP graph (training.GraphedTrainStep)
     removes that bound.  ms per step eager and replayed, same networks as train3d / model2d."""
     import torch
     from torch import nn

@@ -10,8 +10,10 @@
 //
 // Why: as two projections the 4C-channel hidden tensor is written twice (product and GELU) and read
 // once in the forward and written once and read four times in the backward, 39 passes over a C-channel
-// tensor; here the forward moves 3 and the backward 3.  What bounds both is then the GELU on the vector
-// unit (two transcendental and a dozen other instructions per hidden element).
+// tensor; here the forward moves 3 and the backward 3, and its up to 256 workgroups' partial weight
+// gradients, which a second launch adds: 34 MB written and read at C = 64 (a pass over 266 000 voxels), 8.6 at 32.
+// What bounds both is then the GELU on the vector unit (two transcendental and a dozen other instructions per
+// hidden element).
 //
 // Matrix instruction layouts (32x32x16: lane (n, kb) of 32 x 2 holds 8 consecutive-k values of row /
 // column n of its operand; register j of the result is row 8 (j / 4) + 4 kb + j % 4, column n).  The

@@ -1334,7 +1334,7 @@ OptTensor taps_for(const Tensor &x, const Tensor &h, int64_t groups, int64_t m, 
 // order and with the operands of the modules' own calls; None where a layer's geometry is not the kernels'.
 // What a call saves is the modules between the nodes, some 70 us of Python a block where a small block's
 // kernels take as long: the 2-D network's forward on one 208 x 176 image 1.78 -> 1.18 ms, a training step on a
-// 32^3 volume 4.0 -> 3.2-3.6.
+// 32^3 volume, whose pace is the host's, from 4.4-5.2 ms to 2.7-3.9.
 OptTensor block(const Tensor &x_, bool half, double eps1, double eps2, const Tensor &w_in, const OptTensor &b_in, const Tensor &h0,
                 const Tensor &w_source, const OptTensor &b_source, int64_t groups, int64_t m, int64_t sc, double eps, bool save_ratio,
                 const Tensor &w_out, const OptTensor &b_out, const Tensor &w1, const OptTensor &b1, const Tensor &w2,

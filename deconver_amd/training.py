@@ -202,9 +202,9 @@ def train_step(model: nn.Module, optimizer: torch.optim.Optimizer, images: Tenso
 
 class GraphedTrainStep:
     """``train_step`` recorded once into a HIP graph and replayed: for batches small enough that
-    a step is bound by the rate at which the host can launch its ~600 kernels (a 3-D step on
-    one 32^3 volume: 11 ms eager, 7 ms replayed; a 2-D step on one 128^2 image: 14 ms against
-    6 ms on an MI355X), not for the large configurations, whose step keeps the GPU busy.
+    a step is bound by the rate at which the host can launch its some 300 kernels (a 3-D step on
+    one 32^3 volume: 2.7-3.9 ms eager, 2.3 ms replayed; a 2-D step on one 128^2 image: 3.6-4.5 ms against
+    2.0 ms on an MI355X), not for the large configurations, whose step keeps the GPU busy.
 
     The batch shape is fixed at construction.  Construction runs ``warmup`` steps on the given
     batch (the library sizes its launches and the allocator fills its pools on first use),
