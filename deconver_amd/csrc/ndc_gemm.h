@@ -1,12 +1,13 @@
 // The remaining GEMMs of the 1x1 projections on channel-first tensors, float32 and bf16:
 //
 //   tile_kernel    y[b] = epilogue(W x[b])        (forward and input gradient, layers/linear.py:53-58
-//                                                  of the reference with its callers' tails)
+//   parts_kernel                                   of the reference with its callers' tails; bf16 and float32)
+//   sliced_kernel  the same over small grids
 //   wgrad_kernel   gw = sum_b gz[b] x[b]^T,       (weight gradient, with the bias gradient
 //                  gb = row sums of gz             sum_{b,v} gz from the same pass)
 //
 // What the streaming GEMM of ndc_pwgemm.h does not take ends up here: float32 storage, the wide
-// levels whose weights do not fit LDS, odd voxel counts, small grids.  Both kernels are ordinary
+// levels whose weights do not fit LDS, odd voxel counts, small grids.  They are ordinary
 // LDS-tiled matrix-instruction GEMMs; what is particular to them:
 //
 //   * Unit of staging is a 16-byte granule: 8 bf16 or 4 float32 values of consecutive k for one
@@ -15,6 +16,7 @@
 //     32 float32 k-values); granule (row r, depth q) sits at slot q * rows + (r ^ q), so that
 //     neither its writer (8 lanes along q, for operands contiguous in k) nor its readers (32 lanes
 //     along r) meet a bank twice.
+//   * float32 products are made of bf16 parts (see below) where matrix instructions are what a tile waits for.
 //   * Whatever order the instruction takes its k-values in, both operands are filled by one rule
 //     (lane half kb, element e <-> k = (2 step + kb) * E + e), so the products pair up.
 //   * The weight comes in as it lies (float32, rows of W or of its transpose): no packing launch
@@ -30,6 +32,8 @@
 #include <type_traits>
 #include "ndc_common.h"
 #include "ndc_epilogue.h"
+
+#define NDC_INLINE __attribute__((always_inline))
 
 namespace ndc {
 namespace gemm {
@@ -109,6 +113,60 @@ template <typename T> __device__ inline u32x4 ragged(const T *p, int have)
     return Gran<T>::pack(v);
 }
 
+// ---------------------------------------------------------------------------- float32 by bf16 parts
+
+// A float32 is the sum of three bf16: its value rounded, what that leaves rounded, and the rest, which
+// fits.  Six of the nine products of two such triples (all but those of 2^-24 and less) on
+// v_mfma_f32_32x32x16_bf16 take three eighths of the float32 instruction's time for the same k-values
+// (6 x 32 clocks per 16 of them against 8 x 64).  Their sums are nearer to 64 bits, as the accumulator is
+// rounded fewer times: over 32 .. 2048 channels of N(0, 1) values 0.69e-7 .. 7.0e-7 of the result's norm against
+// 1.03e-7 .. 8.1e-7.  Three things are looked after:
+//   * the bf16 instruction drops what it shifts out, which leaves its sums 1e-8 .. 1e-7 of their norm too
+//     low, and that adds up in sums over voxels: half of the results are made with the sign turned (every
+//     other voxel; in weight gradients every other split), so that it cancels;
+//   * infinities, and what rounds to one, leave NaN;
+//   * the parts of numbers below 2^-102 are denormal, which the instruction takes for zero.
+// A tile whose sums are not finite, or not all zero and below 2^-80, is made again by the float32 instruction.
+__device__ inline u32x2 next_part(float (&v)[4])   // four values' next part, which is taken off them
+{
+    const u32x2 r = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        v[2 * h] -= __uint_as_float(r[h] << 16);
+        v[2 * h + 1] -= __uint_as_float(r[h] & 0xffff0000u);
+    }
+    return r;
+}
+// A stage of float32 granules in parts: per part, granules of 8 bf16 (two of the float32 ones), four deep;
+// the rows turned by four per depth, so that a writer's lanes along the depth do not meet a bank twice.
+static const int kPartDepth = 4;
+__device__ inline int part_slot(int rows, int part, int d, int r) { return (part * kPartDepth + d) * rows + (r ^ (4 * d)); }
+__device__ inline void put_parts(u32x4 *lds, int rows, int q, int r, const float (&g)[4])
+{
+    float v[4] = {g[0], g[1], g[2], g[3]};
+    u32x2 *half = reinterpret_cast<u32x2 *>(lds);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) half[2 * part_slot(rows, p, q >> 1, r) + (q & 1)] = next_part(v);
+}
+// granules of 16 bytes per row of a stage of depth D
+template <typename T> constexpr int stage_granules(int depth) { return sizeof(T) == 4 ? 3 * kPartDepth : depth; }
+// whether a wavefront's sums are in the parts' range: 1 some not finite, 2 some not zero, 4 some of 2^-80 and more
+template <int RT, int CT> __device__ inline int range_of(const f32x16 (&acc)[RT][CT])
+{
+    float t = 0.f, most = 0.f;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                t = __builtin_fmaf(acc[i][j][e], 0.f, t);
+                most = __builtin_fmaxf(most, __builtin_fabsf(acc[i][j][e]));
+            }
+    return (__any(t != 0.f) ? 1 : 0) | (__any(most > 0.f) ? 2 : 0) | (__any(most >= 0x1p-80f) ? 4 : 0);
+}
+__device__ inline bool out_of_range(int r) { return (r & 1) || (r & 6) == 2; }
+
 // ---------------------------------------------------------------------------- weight gradient
 
 struct WgradParams {
@@ -127,14 +185,20 @@ struct WgradParams {
 // does not split that axis).  What decides is how the loads fall on memory: rows lie megabytes
 // apart, so few workgroups with long runs per row (D = 16: 256 bytes) beat many with short ones --
 // 512 workgroups, D 16: 192 us; 2048, D 8: 351 us.
+// float32: products of bf16 parts (above), parted as they are staged.  256 x 64 over 8 x 16 384 voxels 55 -> 42 us (one
+// workgroup's matrix instructions next to the other's parting), 512 x 128 over 8 x 4096 48 -> 37, of which the partial
+// results (33 MB written and read) take 14; 32 x 128 over 8 x 65 536, bound by memory, 74 before and after.
 template <typename T, int WM, int WN, int RT, int CT, int D>
-__global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
+__global__ void __launch_bounds__(64 * WM * WN, sizeof(T) == 4 ? 2 : 1) wgrad_kernel(WgradParams p)
 {
     typedef Gran<T> G;
     constexpr int NT = 64 * WM * WN, BM = 32 * WM * RT, BN = 32 * WN * CT, E = G::E, BK = D * E;
     constexpr int NA = BM * D / NT, NB = BN * D / NT;   // granules a thread stages
     static_assert(NA * NT == BM * D && NB * NT == BN * D, "whole granules per thread");
-    __shared__ __attribute__((aligned(16))) u32x4 lds[(BM + BN) * D];
+    constexpr bool F32 = sizeof(T) == 4;
+    static_assert(!F32 || D == 2 * kPartDepth, "a stage in parts");
+    constexpr int LG = stage_granules<T>(D);
+    __shared__ __attribute__((aligned(16))) u32x4 lds[(BM + BN) * LG];
     // an eighth of the launch per XCD (workgroups go round-robin over the eight), the tiles of a split
     // one after the other, so that what they share of the operands comes out of that XCD's L2 (splits
     // dealt to the XCDs whole leave seven of them idle where there is one: 512 x 512 over 64 voxels 8.3
@@ -151,10 +215,9 @@ __global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
     const T *A = (const T *)p.a + ((long long)sample * p.rows + m0) * p.n;   // (uniform)
     const T *B = (const T *)p.b + ((long long)sample * p.cols + n0) * p.n;
     const bool want_sums = p.gb != nullptr && n0 == 0;
+    uint32_t sign = F32 && (split & 1) ? 0x80000000u : 0u;   // (of the products, see above)
     u32x4 ra[NA], rb[NB];
     float sums[NA];
-#pragma unroll
-    for (int i = 0; i < NA; ++i) sums[i] = 0.f;
 
     // Rows past the end repeat the last one: what they contribute is never stored.  Addresses are a
     // uniform pointer plus a 32-bit lane offset (the caller keeps a tile's rows below 4 GiB): as
@@ -166,14 +229,14 @@ __global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
 #pragma unroll
     for (int i = 0; i < NB; ++i)
         off_b[i] = ((uint32_t)min(r0 + i * (NT / D), p.cols - 1 - n0) * (uint32_t)p.n + q * E) * (uint32_t)sizeof(T);
-    auto fetch = [&](long long k0) {
+    auto fetch = [&](long long k0) NDC_INLINE {
         const char *a = (const char *)(A + k0), *b = (const char *)(B + k0);
 #pragma unroll
         for (int i = 0; i < NA; ++i) ra[i] = *(const u32x4_a2 *)(a + off_a[i]);
 #pragma unroll
         for (int i = 0; i < NB; ++i) rb[i] = *(const u32x4_a2 *)(b + off_b[i]);
     };
-    auto fetch_ragged = [&](long long k0) {
+    auto fetch_ragged = [&](long long k0) NDC_INLINE {
         const char *a = (const char *)(A + k0), *b = (const char *)(B + k0);
         const long long rest = k_hi - k0 - (long long)q * E;
         const int have = rest < 0 ? 0 : rest < E ? (int)rest : E;
@@ -182,54 +245,111 @@ __global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
 #pragma unroll
         for (int i = 0; i < NB; ++i) rb[i] = ragged<T>((const T *)(b + off_b[i]), have);
     };
-    auto put = [&]() {
+    auto put = [&](auto parts) NDC_INLINE {
+        auto store = [&](u32x4 *to, int rows, int r, u32x4 g, uint32_t turn) NDC_INLINE {
+            if constexpr (decltype(parts)::value) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(g[e] ^ turn);
+                put_parts(to, rows, q, r, v);
+            } else {
+                to[slot(rows, q, r)] = g;
+            }
+        };
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            lds[slot(BM, q, r0 + i * (NT / D))] = ra[i];
+            store(lds, BM, r0 + i * (NT / D), ra[i], sign);
             if (want_sums) sums[i] += G::sum(ra[i]);
         }
 #pragma unroll
-        for (int i = 0; i < NB; ++i) lds[BM * D + slot(BN, q, r0 + i * (NT / D))] = rb[i];
+        for (int i = 0; i < NB; ++i) store(lds + BM * LG, BN, r0 + i * (NT / D), rb[i], 0u);
     };
 
     const int lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN, l32 = lane & 31, kb = lane >> 5;
     f32x16 acc[RT][CT];
+    auto multiply = [&](auto parts) NDC_INLINE {
+        if constexpr (decltype(parts)::value) {
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
+            for (int s = 0; s < kPartDepth / 2; ++s) {
+                u32x4 fb[CT][3];
+                const int d = 2 * s + kb;
 #pragma unroll
-        for (int j = 0; j < CT; ++j) acc[i][j] = f32x16{};
-    auto multiply = [&]() {
+                for (int o = 0; o < 3; ++o)
 #pragma unroll
-        for (int s = 0; s < D / 2; ++s) {
-            u32x4 fa[RT], fb[CT];
-            const int d = 2 * s + kb;
+                    for (int j = 0; j < CT; ++j) fb[j][o] = lds[BM * LG + part_slot(BN, o, d, 32 * (wn * CT + j) + l32)];
 #pragma unroll
-            for (int i = 0; i < RT; ++i) fa[i] = lds[slot(BM, d, 32 * (wm * RT + i) + l32)];
+                for (int o = 2; o >= 0; --o) {   // the least terms first
+                    u32x4 fa[RT];
 #pragma unroll
-            for (int j = 0; j < CT; ++j) fb[j] = lds[BM * D + slot(BN, d, 32 * (wn * CT + j) + l32)];
+                    for (int i = 0; i < RT; ++i) fa[i] = lds[part_slot(BM, o, d, 32 * (wm * RT + i) + l32)];
 #pragma unroll
-            for (int i = 0; i < RT; ++i)
+                    for (int b = 2 - o; b >= 0; --b)
 #pragma unroll
-                for (int j = 0; j < CT; ++j) acc[i][j] = G::mma(fa[i], fb[j], acc[i][j]);
+                        for (int i = 0; i < RT; ++i)
+#pragma unroll
+                            for (int j = 0; j < CT; ++j) acc[i][j] = Gran<bf16_t>::mma(fa[i], fb[j][b], acc[i][j]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < D / 2; ++s) {
+                u32x4 fa[RT], fb[CT];
+                const int d = 2 * s + kb;
+#pragma unroll
+                for (int i = 0; i < RT; ++i) fa[i] = lds[slot(BM, d, 32 * (wm * RT + i) + l32)];
+#pragma unroll
+                for (int j = 0; j < CT; ++j) fb[j] = lds[BM * LG + slot(BN, d, 32 * (wn * CT + j) + l32)];
+#pragma unroll
+                for (int i = 0; i < RT; ++i)
+#pragma unroll
+                    for (int j = 0; j < CT; ++j) acc[i][j] = G::mma(fa[i], fb[j], acc[i][j]);
+            }
         }
     };
     // Whole stages in a loop without conditions: the next stage's loads are in flight while this
     // one multiplies.  (A branch between the two forms of fetch inside the loop made every stage
     // wait for its loads before it multiplied.)
+    auto clear = [&]() NDC_INLINE {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) sums[i] = 0.f;
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j) acc[i][j] = f32x16{};
+    };
+    auto last = [&](long long k0, auto parts) NDC_INLINE {
+        fetch_ragged(k0);
+        put(parts);
+        __syncthreads();
+        multiply(parts);
+    };
+    clear();
+    const std::bool_constant<F32> parts;
     const int stages = (int)((k_hi - k_lo) / BK);
     if (stages > 0) fetch(k_lo);
     for (int s = 0; s < stages; ++s) {
-        put();
+        put(parts);
         __syncthreads();
         fetch(k_lo + (long long)(s + 1 < stages ? s + 1 : s) * BK);
-        multiply();
+        multiply(parts);
         __syncthreads();
     }
-    if (k_lo + (long long)stages * BK < k_hi) {
-        fetch_ragged(k_lo + (long long)stages * BK);
-        put();
+    if (k_lo + (long long)stages * BK < k_hi) last(k_lo + (long long)stages * BK, parts);
+    if constexpr (F32) {
+        __shared__ int range[WM * WN];
+        if (const int r = range_of(acc); lane == 0) range[wave] = r;
         __syncthreads();
-        multiply();
+        int r = 0;
+#pragma unroll
+        for (int w = 0; w < WM * WN; ++w) r |= range[w];
+        if (out_of_range(r)) {
+            clear();
+            sign = 0u;
+            for (long long k0 = k_lo; k0 < k_hi; k0 += BK) {
+                last(k0, std::false_type());
+                __syncthreads();
+            }
+        }
     }
     const long long out_size = (long long)p.rows * p.cols;
     float *gw = p.part ? p.part + split * (out_size + p.rows) : p.gw;
@@ -241,7 +361,8 @@ __global__ void __launch_bounds__(64 * WM * WN) wgrad_kernel(WgradParams p)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int row = m0 + 32 * (wm * RT + i) + 8 * (e / 4) + 4 * kb + e % 4;
-                if (row < p.rows && col < p.cols) gw[(long long)row * p.cols + col] = acc[i][j][e];
+                if (row < p.rows && col < p.cols)
+                    gw[(long long)row * p.cols + col] = F32 ? __uint_as_float(__float_as_uint(acc[i][j][e]) ^ sign) : acc[i][j][e];
             }
         }
     if (want_sums) {
@@ -415,23 +536,16 @@ template <typename T> __device__ inline void store_quad(T *p, const float (&f)[4
     }
 }
 
-// (E rows of k) x (4 voxels) -> four granules
-template <typename T> __device__ inline void transpose(const Quad<T> (&in)[Gran<T>::E], u32x4 (&out)[4])
+// (8 rows of k) x (4 voxels) -> four granules
+__device__ inline void transpose(const Quad<bf16_t> (&in)[8], u32x4 (&out)[4])
 {
-    if constexpr (sizeof(T) == 4) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) out[c][e] = __float_as_uint(in[e].v[c]);
-    } else {
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int pr = 0; pr < 4; ++pr) {
-                out[2 * h][pr] = __builtin_amdgcn_perm(in[2 * pr + 1].v[h], in[2 * pr].v[h], 0x05040100u);
-                out[2 * h + 1][pr] = __builtin_amdgcn_perm(in[2 * pr + 1].v[h], in[2 * pr].v[h], 0x07060302u);
-            }
-    }
+        for (int pr = 0; pr < 4; ++pr) {
+            out[2 * h][pr] = __builtin_amdgcn_perm(in[2 * pr + 1].v[h], in[2 * pr].v[h], 0x05040100u);
+            out[2 * h + 1][pr] = __builtin_amdgcn_perm(in[2 * pr + 1].v[h], in[2 * pr].v[h], 0x07060302u);
+        }
 }
 
 // The epilogue of NR consecutive rows of four voxels: z the products, `have` of the four voxels
@@ -481,13 +595,14 @@ __device__ inline void finish(const TileParams &p, const float (&z)[NR][4], int 
     else run(std::false_type{});
 }
 
-// A workgroup of WAVES wavefronts makes a tile of 32 WAVES output rows x 128 voxels.  Voxel
+// bf16: a workgroup of WAVES wavefronts makes a tile of 32 WAVES output rows x 128 voxels.  Voxel
 // v of the tile is column v / 4 of matrix tile v % 4, so that a lane ends up with four
 // consecutive voxels of a row: stores (and the loads of residual, mask and kept product) are 8
 // or 16 bytes per lane, 32 lanes contiguous.
-template <typename T, bool WT, int WAVES, int MODE>
+template <bool WT, int WAVES, int MODE>
 __global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
 {
+    typedef bf16_t T;
     typedef Gran<T> G;
     constexpr int NT = 64 * WAVES, BM = 32 * WAVES, BN = 128, E = G::E, BK = kDepth * E;
     constexpr int NA = BM * kDepth / NT;             // weight granules a thread stages
@@ -578,7 +693,7 @@ __global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
             const int u = tid + i * NT, c = u & 31, q = u >> 5;
             const uint32_t keep = k0 + q * E < p.cin ? ~0u : 0u;
             u32x4 g[4];
-            transpose<T>(rx[i], g);
+            transpose(rx[i], g);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -640,6 +755,215 @@ __global__ void __launch_bounds__(64 * WAVES) tile_kernel(TileParams p)
                 if (l32 == 31 && row0 + e < p.cout) p.gpart[(long long)vt * p.cout + row0 + e] = s;
             }
         }
+    }
+}
+
+// float32: a workgroup of four wavefronts makes 32 RT output rows x 128 voxels, each wavefront all of the rows of
+// 32 voxels.  The products are those of bf16 parts (above).  A wavefront's voxels are its own, so x goes from
+// memory to its registers and is parted there, a word per lane and channel; only W, which the wavefronts share,
+// is parted into LDS, in two buffers, one barrier per 32 channels.  (With x through LDS as well, parting and
+// staging took as long as the matrix instructions: 128 -> 512 channels over 8 x 4096 voxels 41 us.)
+// CHAINS: the sums of 32 channels are made apart and then added, which keeps the error of any number of channels
+// below that of the sliced form (2048 channels 1.7e-7 of the result's norm instead of 7.0e-7; slices 2.9e-7).  It
+// takes a wavefront per SIMD: without it 32 -> 128 over 8 x 65 536 takes 77 us instead of 85, 64 -> 256 over
+// 8 x 16 384 43 instead of 49, with 0.69e-7 and 1.1e-7 (the float32 instruction: 1.03e-7, 1.45e-7).
+// Bound by memory to 64 channels (64 -> 256 over 8 x 16 384: 4.0 TB/s), beyond by the matrix instructions,
+// which run at 45 clocks each at the clock that their power leaves, and the vector instructions that part x and W
+// between them: 512 -> 128 over 8 x 4096 78 us by the float32 instruction, 34 like this; 256 -> 1024 over 8 x 1024
+// 45 and 35; 256 -> 64 over 8 x 16 384 50 and 36; 96 -> 64 over 33 333 23 and 11.
+template <bool WT, int RT, bool CHAINS, int MODE>
+__global__ void __launch_bounds__(256, (RT == 2 ? 4 : 5) - CHAINS) parts_kernel(TileParams p)
+{
+    constexpr int BM = 32 * RT, BN = 128, BK = 32;
+    __shared__ __attribute__((aligned(16))) u32x4 lds[2][BM * 3 * kPartDepth];
+    __shared__ __attribute__((aligned(16))) float bias[BM];
+    __shared__ float red[4][BM];
+    const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
+    const int tile_m = pos % p.tiles_m, vt = (pos / p.tiles_m) * 8 + xcd;   // a voxel tile stays on one XCD
+    if (vt >= p.tiles_n * p.batch) return;
+    const int sample = vt / p.tiles_n, m0 = tile_m * BM;
+    const long long v0 = (long long)(vt % p.tiles_n) * BN;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, kb = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int left = (int)(p.n - v0 < BN ? p.n - v0 : BN), mine = 32 * wave + l32;
+    const float *X = (const float *)p.x + (long long)sample * p.cin * p.n + v0;
+    // lanes past the end of a row repeat its last voxel, rows past the end the last row: never stored
+    const uint32_t xoff = ((uint32_t)(8 * kb) * (uint32_t)p.n + (uint32_t)min(mine, left - 1)) * 4u;
+    const uint32_t sign = (uint32_t)(l32 & 1) << 31;
+    float xr[2][8], rw[RT][4];
+    auto weight_at = [&](int i, int &r, int &q) NDC_INLINE {   // granule i of this thread
+        const int g = tid + i * 256;
+        if (WT) r = g % BM, q = g / BM;   // lanes along the rows of W, contiguous in W^T
+        else r = g >> 3, q = g & 7;
+    };
+    auto fetch = [&](int k0) NDC_INLINE {   // (whole stages)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xr[t][e] = *(const float *)((const char *)(X + (long long)(k0 + 16 * t + e) * p.n) + xoff);
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            int r, q;
+            weight_at(i, r, q);
+            const int m = min(m0 + r, p.cout - 1), k = k0 + 4 * q;
+            if constexpr (WT) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rw[i][e] = p.w[(long long)(k + e) * p.cout + m];
+            } else {
+                Quad<float> t;
+                t.load(p.w + (long long)m * p.cin + k);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rw[i][e] = t.get(e);
+            }
+        }
+    };
+    auto fetch_ragged = [&](int k0) NDC_INLINE {   // (depths past the end are zero)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int k = k0 + 16 * t + 8 * kb + e;
+                xr[t][e] = k < p.cin ? X[(long long)k * p.n + min(mine, left - 1)] : 0.f;
+            }
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            int r, q;
+            weight_at(i, r, q);
+            const int m = min(m0 + r, p.cout - 1), k = k0 + 4 * q;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                rw[i][e] = k + e < p.cin ? p.w[WT ? (long long)(k + e) * p.cout + m : (long long)m * p.cin + k + e] : 0.f;
+        }
+    };
+    f32x16 acc[RT][1];
+    u32x4 xp[2][1][3];
+    auto put = [&](u32x4 *to) NDC_INLINE {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+            int r, q;
+            weight_at(i, r, q);
+            put_parts(to, BM, q, r, rw[i]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(__float_as_uint(xr[t][4 * h + e]) ^ sign);
+#pragma unroll
+                for (int o = 0; o < 3; ++o) {
+                    const u32x2 w = next_part(v);
+                    xp[t][0][o][2 * h] = w[0], xp[t][0][o][2 * h + 1] = w[1];
+                }
+            }
+    };
+    auto multiply = [&](const u32x4 *from) NDC_INLINE {
+        f32x16 sum[RT];
+        if constexpr (!CHAINS) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) sum[i] = acc[i][0];
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int o = 2; o >= 0; --o) {   // the least terms first
+                u32x4 fa[RT];
+#pragma unroll
+                for (int i = 0; i < RT; ++i) fa[i] = from[part_slot(BM, o, 2 * t + kb, 32 * i + l32)];
+#pragma unroll
+                for (int b = 2 - o; b >= 0; --b)
+#pragma unroll
+                    for (int i = 0; i < RT; ++i)
+                        sum[i] = Gran<bf16_t>::mma(fa[i], xp[t][0][b], CHAINS && t == 0 && o == 2 ? f32x16{} : sum[i]);
+            }
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[i][0] = CHAINS ? acc[i][0] + sum[i] : sum[i];
+    };
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[i][0] = f32x16{};
+    for (int r = tid; r < BM; r += 256) bias[r] = p.bias && m0 + r < p.cout ? p.bias[m0 + r] : 0.f;
+    const int stages = p.cin / BK;
+    if (stages > 0) fetch(0);
+    for (int s = 0; s < stages; ++s) {
+        put(lds[s & 1]);
+        __syncthreads();
+        if (s + 1 < stages) fetch((s + 1) * BK);
+        multiply(lds[s & 1]);
+    }
+    if (stages * BK < p.cin) {
+        fetch_ragged(stages * BK);
+        put(lds[stages & 1]);
+        __syncthreads();
+        multiply(lds[stages & 1]);
+    }
+    uint32_t turn = sign;
+    if (out_of_range(range_of(acc))) {
+        turn = 0u;
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[i][0] = f32x16{};
+        for (int k0 = 0; k0 < p.cin; k0 += 2) {
+            const int k = k0 + kb;
+            const bool in = k < p.cin;
+            const float b = in ? X[(long long)k * p.n + min(mine, left - 1)] : 0.f;
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const int m = min(m0 + 32 * i + l32, p.cout - 1);
+                const float a = in ? p.w[WT ? (long long)k * p.cout + m : (long long)m * p.cin + k] : 0.f;
+                acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc[i][0], 0, 0, 0);
+            }
+        }
+    }
+    const bool summed = MODE == kGeluGrad && p.gpart != nullptr, exists = mine < left;
+    const long long base = ((long long)sample * p.cout + m0) * p.n + v0;   // (uniform)
+    const uint32_t yoff = ((uint32_t)(4 * kb) * (uint32_t)p.n + (uint32_t)min(mine, left - 1)) * 4u;
+    auto run = [&](auto tag) NDC_INLINE {
+        constexpr bool WHOLE = decltype(tag)::value;   // all rows and voxels of the tile exist
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {   // what eight rows read is requested ahead of their stores
+                float rv[8], mv[8], bv[8];
+                auto row_of = [&](int e) NDC_INLINE { return 32 * i + 16 * h + 8 * (e / 4) + e % 4; };   // (+ 4 kb)
+                auto in = [&](int e) NDC_INLINE { return WHOLE || (exists && m0 + row_of(e) + 4 * kb < p.cout); };
+                auto at = [&](const void *t, int e) NDC_INLINE {
+                    return (float *)((char *)((float *)t + base + (long long)row_of(e) * p.n) + yoff);
+                };
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    bv[e] = bias[row_of(e) + 4 * kb];
+                    if (p.res) rv[e] = in(e) ? *at(p.res, e) : 0.f;
+                    if (p.mask) mv[e] = in(e) ? *at(p.mask, e) : 0.f;
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float z = __uint_as_float(__float_as_uint(acc[i][0][8 * h + e]) ^ turn);
+                    float y;
+                    if constexpr (MODE == kGeluGrad) {
+                        y = z * epilogue::act_grad<epilogue::kGelu>(rv[e] + bv[e]);
+                    } else {
+                        y = epilogue::act_fwd<MODE>(z + bv[e]);
+                        if (p.res) y += rv[e];
+                        if (p.mask) y = mv[e] > 0.f ? y : 0.f;
+                    }
+                    if (in(e)) {
+                        if constexpr (MODE == epilogue::kRelu || MODE == epilogue::kGelu)
+                            if (p.zkeep) *at(p.zkeep, e) = z;
+                        *at(p.y, e) = y;
+                    }
+                    if (summed) {
+                        const float sum = epilogue::half_sum(in(e) ? y : 0.f);   // the 32 lanes of a row
+                        if (l32 == 31) red[wave][row_of(e) + 4 * kb] = sum;
+                    }
+                }
+            }
+    };
+    if (left == BN && m0 + BM <= p.cout) run(std::true_type{});
+    else run(std::false_type{});
+    if (summed) {
+        __syncthreads();
+        if (tid < BM && m0 + tid < p.cout)
+            p.gpart[(long long)vt * p.cout + m0 + tid] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
     }
 }
 

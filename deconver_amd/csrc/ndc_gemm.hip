@@ -70,9 +70,19 @@ template <typename T, bool WT, int MODE> static void tile_gemm_w(TileParams p, i
     p.tiles_m = (p.cout + rows - 1) / rows;
     p.tiles_n = (int)((p.n + 127) / 128);
     const dim3 grid(8u * (unsigned)((p.tiles_n * p.batch + 7) / 8) * (unsigned)p.tiles_m);
-    if (waves == 4) hipLaunchKernelGGL((tile_kernel<T, WT, 4, MODE>), grid, dim3(256), 0, (hipStream_t)stream, p);
-    else if (waves == 2) hipLaunchKernelGGL((tile_kernel<T, WT, 2, MODE>), grid, dim3(128), 0, (hipStream_t)stream, p);
-    else hipLaunchKernelGGL((tile_kernel<T, WT, 1, MODE>), grid, dim3(64), 0, (hipStream_t)stream, p);
+    auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, (hipStream_t)stream, p); };
+    if constexpr (sizeof(T) == 4) {
+        // one chain of sums where it is no less exact than the float32 instruction was there (a grid that used to be
+        // sliced had chains of eight channels)
+        const long long sliced = (long long)p.batch * ((p.n + 63) / 64) * ((p.cout + 31) / 32);
+        const bool one = p.cin <= 32 || (p.cin <= 64 && sliced > 1024);
+        if (waves == 2) one ? launch(parts_kernel<WT, 2, false, MODE>, 256) : launch(parts_kernel<WT, 2, true, MODE>, 256);
+        else one ? launch(parts_kernel<WT, 1, false, MODE>, 256) : launch(parts_kernel<WT, 1, true, MODE>, 256);
+    } else {
+        if (waves == 4) launch(tile_kernel<WT, 4, MODE>, 256);
+        else if (waves == 2) launch(tile_kernel<WT, 2, MODE>, 128);
+        else launch(tile_kernel<WT, 1, MODE>, 64);
+    }
 }
 template <typename T>
 static int tile_gemm_t(const TileParams &p, int transposed, int mode, int waves, void *stream)

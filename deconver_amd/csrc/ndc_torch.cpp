@@ -243,7 +243,11 @@ Matrix saved_weight(const Tensor &w, bool transposed, int64_t cout, const Tensor
 //             call, as much as the product --, and larger ones whose tail (bias, activation,
 //             residual, mask) it takes along: float32 always, bf16 with at most 32 K weights (256
 //             -> 1024 channels over 2 x 32^3 voxels: 85 us against 59 us by the library, which then
-//             pays for one more pass over the result);
+//             pays for one more pass over the result).  In float32 the larger ones without a tail too (us,
+//             library / tiled: 64 -> 256 over 2 x 91 125 voxels 128 / 61, 256 -> 1024 over 2 x 27 000 277 / 212,
+//             512 -> 128 over 8 x 4096 37.7 / 33.9, 128 -> 64 over 8 x 16 384 27.6 / 27.5), but for those from 1024
+//             channels and more between 2 and 12 GFLOP (1024 -> 256 over 8 x 1024 36.9 / 42.2, 2048 -> 512 over
+//             4 x 1000 65 / 82, over 8000, 17 GFLOP, 130 / 118);
 //   kLibrary  the rest.
 enum Gemm { kStream, kTiled, kLibrary };
 
@@ -255,8 +259,9 @@ Gemm choose_gemm(const Tensor &x, int64_t cout, bool act_or_keep, bool tail)
     if (stream && B * n >= 2048 * 64) return kStream;
     if (n > (1 << 24)) return stream ? kStream : kLibrary;
     const double flops = 2.0 * (double)B * (double)n * (double)cin * (double)cout;
-    if (flops < (half ? 4e9 : 2e9)) return kTiled;
-    if (tail && (!half || cin * cout <= 32 * 1024)) return kTiled;
+    if (!half) return !tail && cin >= 1024 && flops >= 2e9 && flops < 12e9 ? kLibrary : kTiled;
+    if (flops < 4e9) return kTiled;
+    if (tail && cin * cout <= 32 * 1024) return kTiled;
     return stream ? kStream : kLibrary;
 }
 

@@ -105,6 +105,54 @@ def test_weight_gradient_over_long_rows(rows, cols):
     assert _rel(gw, g[0].double() @ x[0].double().t()) < 1e-5 and _rel(gb, g.double().sum((0, 2))) < 1e-5
 
 
+# rows of 32 and 64 a workgroup, one chain of sums and several; ragged channels, rows and voxels
+PARTS = [(1, 33, 40, 38501), (2, 100, 130, 9001), (1, 32, 64, 52001), (2, 72, 30, 20003), (1, 1030, 96, 13000)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", PARTS)
+def test_float32_products_of_parts(shape):
+    """float32 products made of bf16 parts, over grids that are not sliced.  The error of a chain of 64 channels is
+    1.1e-7 of the result's norm, that of chains of 32 and their sum 0.7e-7 .. 1.4e-7; the values' mean is off by noise."""
+    print("case", shape, flush=True)
+    lib, (x, res, _, g), w, bias = _setup("cuda", shape, torch.float32)
+    z = torch.matmul(w.double(), x.double())
+    wt = w.t().contiguous()
+    for y in (ops.gemm(lib, x, w)[0], ops.gemm(lib, x, wt, transposed=True)[0]):
+        assert _rel(y, z) < 2e-7
+        assert float((y - z).mean().abs() / z.norm() * z.numel() ** 0.5) < 3e-9
+    y, zk = ops.gemm(lib, x, w, bias, res, "gelu", keep_z=True)
+    assert _rel(zk, z) < 2e-7 and _rel(y, F.gelu(z + bias.double()[:, None]) + res.double()) < 5e-7
+    gw, gb = ops.weight_grad(lib, g, x, need_bias_grad=True)
+    assert _rel(gw, torch.matmul(g.double(), x.double().transpose(1, 2)).sum(0)) < 6e-7
+    assert _rel(gb, g.double().sum((0, 2))) < 4e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-36, 1e-20, 1e30])
+def test_parts_of_small_and_large_values(scale):
+    lib, (x, _, _, g), w, _ = _setup("cuda", (2, 72, 30, 20003), torch.float32)
+    x *= scale
+    assert _rel(ops.gemm(lib, x, w)[0], torch.matmul(w.double(), x.double())) < 4e-7
+    gw, _ = ops.weight_grad(lib, g, x)
+    assert _rel(gw, torch.matmul(g.double(), x.double().transpose(1, 2)).sum(0)) < 1e-6
+
+
+@pytest.mark.gpu
+def test_parts_of_values_that_are_not_finite():
+    """What a float32 product makes of infinities, NaN and values beyond the range of bf16: an infinity's column is
+    infinite by the weight's sign, the rest finite."""
+    lib, (x, _, _, g), w, _ = _setup("cuda", (2, 72, 30, 20003), torch.float32)
+    x[0, 3, 7], x[0, 71, 20002], x[1, 5, 130], x[1, 6, 131] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    for y, want in ((ops.gemm(lib, x, w)[0], torch.matmul(w.double(), x.double())),
+                    (ops.weight_grad(lib, g, x)[0], torch.matmul(g.double(), x.double().transpose(1, 2)).sum(0))):
+        want = want.float()
+        assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isinf(), want.isinf())
+        assert torch.equal(y[y.isinf()], want[want.isinf()])
+        ok = want.isfinite() & (want.abs() < 1e30)
+        assert _rel(y[ok], want[ok]) < 1e-6
+
+
 def test_refused_arguments():
     lib = hostcheck_library()
     x, w = torch.zeros(1, 8, 4), torch.zeros(6, 8)
