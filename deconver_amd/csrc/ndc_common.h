@@ -216,7 +216,7 @@ template <class F> NDC_D uint32_t from_left_lane(uint32_t own, F again)
 }
 
 // N consecutive elements <-> N floats with one memory access (N = 1 or 2; the address must
-// be aligned to N elements)
+// be aligned to N elements; N = -2: two elements at any address of an element)
 template <typename T, int N> struct VecIO;
 template <typename T> struct VecIO<T, 1> {
     static NDC_HD void load(const T *p, float (&v)[1]) { v[0] = Elem<T>::load(p); }
@@ -250,6 +250,38 @@ template <> struct VecIO<bf16_t, 2> {
     static NDC_HD void store(bf16_t *p, const float (&v)[2])
     {
         *reinterpret_cast<uint32_t *>(p) = pack_bf16x2(v[0], v[1]);
+    }
+};
+
+template <> struct VecIO<float, -2> {
+    struct __attribute__((aligned(4), may_alias)) Pair {
+        float a, b;
+    };
+    static NDC_HD void load(const float *p, float (&v)[2])
+    {
+        const Pair q = *reinterpret_cast<const Pair *>(p);
+        v[0] = q.a;
+        v[1] = q.b;
+    }
+    static NDC_HD void store(float *p, const float (&v)[2])
+    {
+        Pair q;
+        q.a = v[0];
+        q.b = v[1];
+        *reinterpret_cast<Pair *>(p) = q;
+    }
+};
+template <> struct VecIO<bf16_t, -2> {
+    typedef uint32_t __attribute__((aligned(2), may_alias)) word_t;
+    static NDC_HD void load(const bf16_t *p, float (&v)[2])
+    {
+        const uint32_t w = *reinterpret_cast<const word_t *>(p);
+        v[0] = bits_to_float(w << 16);
+        v[1] = bits_to_float(w & 0xffff0000u);
+    }
+    static NDC_HD void store(bf16_t *p, const float (&v)[2])
+    {
+        *reinterpret_cast<word_t *>(p) = pack_bf16x2(v[0], v[1]);
     }
 };
 

@@ -34,6 +34,14 @@ template <class State> struct DeviceExec {
     NDC_D void sync() { __syncthreads(); }
     NDC_D float ld(int i) const { return lds[i]; }
     NDC_D void st_(int i, float v) { lds[i] = v; }
+    // a word that another thread may store the same value to in the same phase
+    NDC_D void st_same(int i, float v) { lds[i] = v; }
+    // two consecutive words from any word index (one ds_read2_b32)
+    NDC_D void ld2f(int i, float (&v)[2]) const
+    {
+        v[0] = lds[i];
+        v[1] = lds[i + 1];
+    }
     // two consecutive words from an EVEN word index: one 8-byte read
     NDC_D void ld2(int i, float (&v)[2]) const
     {
@@ -193,6 +201,17 @@ template <class State> struct HostExec {
             r_tid[i] = -2;
         }
         return mem[i];
+    }
+    void ld2f(int i, float (&v)[2])
+    {
+        v[0] = ld(i);
+        v[1] = ld(i + 1);
+    }
+    void st_same(int i, float v)
+    {
+        // (the same bits as the other thread's: its store stands)
+        if (i >= 0 && i < (int)mem.size() && w_epoch[i] == epoch && w_tid[i] != cur && memcmp(&mem[i], &v, 4) == 0) return;
+        st_(i, v);
     }
     void ld2(int i, float (&v)[2])
     {

@@ -91,14 +91,14 @@ static inline int round_up(int v, int a) { return (v + a - 1) / a * a; }
 static const int kMaxThreads = 512;
 static const int kMaxLdsBytes = 160 * 1024;
 
-// S strips of RH rows, RW columns per thread; S >= 2*PH so that the halo rows fit the
-// fixed per-thread bounds
+// S strips of RH rows, RW columns per thread (-2: column pairs of a row of any length, see Lane); S >= 2*PH so
+// that the halo rows fit the fixed per-thread bounds
 static inline bool make_tile(const March &m, int RH, int RW, int target_threads, Tile &t,
                              int min_strips = 0)
 {
     const int PH = m.KH / 2, PW = m.KW / 2;
-    if (m.W % RW) return false;
-    const int cpw = m.W / RW;
+    if (RW < 0 ? m.W < 2 : m.W % RW) return false;
+    const int cpw = RW < 0 ? (m.W + 1) / 2 : m.W / RW;
     if (cpw > kMaxThreads) return false;
     int smin = PH > 0 ? 2 * PH : 1;
     if (smin < min_strips) smin = min_strips;
@@ -115,7 +115,7 @@ static inline bool make_tile(const March &m, int RH, int RW, int target_threads,
     // PW zero words left of column 0: a thread's window (its RW columns and PW either side)
     // then starts at its own first column, an even word when RW = 2
     t.PL = PW;
-    t.P = round_up(t.PL + m.W + PW, RW);
+    t.P = round_up(t.PL + m.W + PW, RW < 0 ? 2 : RW);
     t.nseg = 1;
     t.SEG = m.D;
     return true;
@@ -206,14 +206,15 @@ NDC_HD int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v
 NDC_HD int halo_row(int s, int PH, int TH) { return s < PH ? s : TH + s; }
 
 // NW staged words from `at`.  RW = 2: the window starts at an even word (see make_tile) and
-// is read two words at a time.
-template <int NW, int RW, class Exec> NDC_D void read_window(Exec &ex, int at, float (&v)[NW])
+// is read two words at a time; LOOSE: at any word.
+template <int NW, int RW, bool LOOSE, class Exec> NDC_D void read_window(Exec &ex, int at, float (&v)[NW])
 {
     if constexpr (RW == 2 && NW % 2 == 0) {
         NDC_UNROLL
         for (int u = 0; u < NW; u += 2) {
             float pair[2];
-            ex.ld2(at + u, pair);
+            if constexpr (LOOSE) ex.ld2f(at + u, pair);
+            else ex.ld2(at + u, pair);
             v[u] = pair[0];
             v[u + 1] = pair[1];
         }
@@ -231,23 +232,23 @@ template <int NW, int RW, class Exec> NDC_D void read_window(Exec &ex, int at, f
 // PIPE (here and in a_plane): the LDS words of a row are read one row ahead of the arithmetic
 // that uses them, and a scheduling fence keeps that order; for kernels that run too few
 // wavefronts per SIMD to hide the LDS latency otherwise and have the registers to spare.
-template <int KD, int KH, int KW, int NR, int RW, int STRIDE, bool PIPE = false, class Exec>
+template <int KD, int KH, int KW, int NR, int RW, int STRIDE, bool LOOSE, bool PIPE = false, class Exec>
 NDC_D void k_rows(Exec &ex, int base, int P, const float (&w)[KD * KH * KW],
                   float (*acc)[STRIDE][RW], int r_off)
 {
     constexpr int NW = RW + KW - 1, NROW = NR + KH - 1;
     float vn[NW];
-    if (PIPE) read_window<NW, RW>(ex, base, vn);
+    if (PIPE) read_window<NW, RW, LOOSE>(ex, base, vn);
     NDC_UNROLL
     for (int q = 0; q < NROW; ++q) {
         float v[NW];
         if (PIPE) {
             NDC_UNROLL
             for (int u = 0; u < NW; ++u) v[u] = vn[u];
-            if (q + 1 < NROW) read_window<NW, RW>(ex, base + (q + 1) * P, vn);
+            if (q + 1 < NROW) read_window<NW, RW, LOOSE>(ex, base + (q + 1) * P, vn);
             ex.fence();
         } else {
-            read_window<NW, RW>(ex, base + q * P, v);
+            read_window<NW, RW, LOOSE>(ex, base + q * P, v);
         }
         NDC_UNROLL
         for (int th = 0; th < KH; ++th) {
@@ -268,7 +269,7 @@ NDC_D void k_rows(Exec &ex, int base, int P, const float (&w)[KD * KH * KW],
 // One tap plane of an A-type gather for NT tensors at once over an NR x RW register tile:
 // base[t] addresses, in plane-slot form, the word (first input row, first own column - PW)
 // of tensor t; wt = taps of tap plane td, indexed wt[i][th*KW + tw].
-template <int KH, int KW, int KT, int SC, int NR, int RW, int NTEN, bool PIPE = false, class Exec>
+template <int KH, int KW, int KT, int SC, int NR, int RW, int NTEN, bool LOOSE, bool PIPE = false, class Exec>
 NDC_D void a_plane(Exec &ex, const int (&base)[NTEN], int P, const float (&wt)[SC][KH * KW],
                    float (&acc)[NTEN][SC][NR][RW])
 {
@@ -276,7 +277,7 @@ NDC_D void a_plane(Exec &ex, const int (&base)[NTEN], int P, const float (&wt)[S
     float vn[NTEN][NW];
     if (PIPE) {
         NDC_UNROLL
-        for (int t = 0; t < NTEN; ++t) read_window<NW, RW>(ex, base[t], vn[t]);
+        for (int t = 0; t < NTEN; ++t) read_window<NW, RW, LOOSE>(ex, base[t], vn[t]);
     }
     NDC_UNROLL
     for (int q = 0; q < NROW; ++q) {
@@ -288,12 +289,12 @@ NDC_D void a_plane(Exec &ex, const int (&base)[NTEN], int P, const float (&wt)[S
                 for (int u = 0; u < NW; ++u) v[t][u] = vn[t][u];
             if (q + 1 < NROW) {
                 NDC_UNROLL
-                for (int t = 0; t < NTEN; ++t) read_window<NW, RW>(ex, base[t] + (q + 1) * P, vn[t]);
+                for (int t = 0; t < NTEN; ++t) read_window<NW, RW, LOOSE>(ex, base[t] + (q + 1) * P, vn[t]);
             }
             ex.fence();
         } else {
             NDC_UNROLL
-            for (int t = 0; t < NTEN; ++t) read_window<NW, RW>(ex, base[t] + q * P, v[t]);
+            for (int t = 0; t < NTEN; ++t) read_window<NW, RW, LOOSE>(ex, base[t] + q * P, v[t]);
         }
         NDC_UNROLL
         for (int th = 0; th < KH; ++th) {
@@ -315,13 +316,13 @@ NDC_D void a_plane(Exec &ex, const int (&base)[NTEN], int P, const float (&wt)[S
 
 // NROWS rows of NW staged words of each of NOP operands (row n of operand t at addr(n, t)),
 // handed to body(n, words); PIPE: read one row ahead of the arithmetic (see k_rows).
-template <int NROWS, int NW, int NOP, bool PIPE, int RW, class Exec, class Addr, class Body>
+template <int NROWS, int NW, int NOP, bool PIPE, int RW, bool LOOSE, class Exec, class Addr, class Body>
 NDC_D void stream_rows(Exec &ex, Addr addr, Body body)
 {
     float vn[NOP][NW];
     if (PIPE) {
         NDC_UNROLL
-        for (int t = 0; t < NOP; ++t) read_window<NW, RW>(ex, addr(0, t), vn[t]);
+        for (int t = 0; t < NOP; ++t) read_window<NW, RW, LOOSE>(ex, addr(0, t), vn[t]);
     }
     NDC_UNROLL
     for (int n = 0; n < NROWS; ++n) {
@@ -333,12 +334,12 @@ NDC_D void stream_rows(Exec &ex, Addr addr, Body body)
                 for (int u = 0; u < NW; ++u) v[t][u] = vn[t][u];
             if (n + 1 < NROWS) {
                 NDC_UNROLL
-                for (int t = 0; t < NOP; ++t) read_window<NW, RW>(ex, addr(n + 1, t), vn[t]);
+                for (int t = 0; t < NOP; ++t) read_window<NW, RW, LOOSE>(ex, addr(n + 1, t), vn[t]);
             }
             ex.fence();
         } else {
             NDC_UNROLL
-            for (int t = 0; t < NOP; ++t) read_window<NW, RW>(ex, addr(n, t), v[t]);
+            for (int t = 0; t < NOP; ++t) read_window<NW, RW, LOOSE>(ex, addr(n, t), v[t]);
         }
         body(n, v);
     }
@@ -361,24 +362,40 @@ template <int SC, int KT, int N> NDC_D void load_plane_taps(UniformF src, float 
         for (int a = 0; a < N; ++a) dst[i][a] = src[i * KT + a];
 }
 
-// thread coordinates shared by the three kernels
+// thread coordinates shared by the three kernels.  LOOSE: column pairs of rows of any length.  The last thread
+// of a row of odd length has the last two columns, of which the first is its neighbour's too: both make the same
+// values of it and store them, and the neighbour's count in sums (`twice`: this thread's do not).
 struct Lane {
-    int strip, c0, active;
+    int strip, c0, active, twice;
 };
 
-NDC_HD Lane make_lane(int tid, const Tile &t, int RW)
+template <int RW, bool LOOSE> NDC_HD Lane make_lane(int tid, const Tile &t, int W)
 {
     Lane l;
     l.strip = tid / t.CPW;
     l.c0 = (tid - l.strip * t.CPW) * RW;
     l.active = l.strip < t.S;
+    l.twice = LOOSE && l.c0 + RW > W;
+    if (l.twice) l.c0 = W - RW;
     return l;
+}
+NDC_HD Lane make_lane(int tid, const Tile &t, int RW)
+{
+    return RW == 2 ? make_lane<2, false>(tid, t, 0) : make_lane<1, false>(tid, t, 0);
+}
+
+// a staged word that the threads of a LOOSE row may share
+template <bool LOOSE, class Exec> NDC_D void stage(Exec &ex, int i, float v)
+{
+    if constexpr (LOOSE) ex.st_same(i, v);
+    else ex.st_(i, v);
 }
 
 // =================================================================== forward
 
 template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> struct FwdKernel {
-    static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_;
+    static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_ < 0 ? -RW_ : RW_;
+    static constexpr bool LOOSE = RW_ < 0;   // rows of any length and alignment (see Lane)
     static constexpr int PD = KD / 2, PH = KH / 2, PW = KW / 2, KT = KD * KH * KW;
     static constexpr int XT = PH > 0 ? 1 : 0;            // one extra halo row for strips < 2*PH
     static constexpr int RHK = RH + XT;
@@ -386,7 +403,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
     static constexpr int NXR = RH + (PH > 0 ? 1 : 0);    // rows of x a thread stages
     static constexpr int XR = KD;                        // x ring slots (filled in the scatter phase)
     typedef FwdParams<T> Params;
-    typedef VecIO<T, RW> IO;
+    typedef VecIO<T, RW_> IO;
 
     struct State {
         Lane ln;
@@ -464,7 +481,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
                     for (int i = 0; i < SC; ++i)
                         NDC_UNROLL
                         for (int c = 0; c < RW; ++c)
-                            ex.st_(st.so + (off_s + (i * RS + n * S) * P) + c,
+                            stage<LOOSE>(ex, st.so + (off_s + (i * RS + n * S) * P) + c,
                                    live ? floor_f(st.pz[i][n][c] + st.bv[i], floor_) : 0.f);
                 }
             }
@@ -479,7 +496,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
                 if ((st.xok >> n) & 1u) {
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c)
-                        ex.st_(st.so + (off_x + (slot * RX + n * S) * P) + c, live ? st.px[n][c] : 0.f);
+                        stage<LOOSE>(ex, st.so + (off_x + (slot * RX + n * S) * P) + c, live ? st.px[n][c] : 0.f);
                 }
             }
         };
@@ -487,7 +504,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
         // ---- set-up: thread coordinates, row offsets, zeroed accumulators, zeroed LDS (halo
         //      columns and never-staged rows stay zero for the whole march)
         ex.each([&](State &st, int tid) NDC_LAMBDA {
-            st.ln = make_lane(tid, t, RW);
+            st.ln = make_lane<RW, LOOSE>(tid, t, W);
             st.ob = st.ln.strip * RH * P + PL + st.ln.c0 - PW;
             st.so = st.ln.strip * P + PL + st.ln.c0;
             st.ho = halo_row(st.ln.strip, PH, TH) * P + PL + st.ln.c0 - PW;
@@ -542,9 +559,9 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
                         const int i = uniform_int(ii);
                         float wi[KT];
                         load_taps<KT>(hw + i * KT, wi);
-                        k_rows<KD, KH, KW, RH, RW, RHK>(ex, st.ob + (off_s + (i * RS + PH) * P), P, wi,
+                        k_rows<KD, KH, KW, RH, RW, RHK, LOOSE>(ex, st.ob + (off_s + (i * RS + PH) * P), P, wi,
                                                         st.t1acc, 0);
-                        if (extra) k_rows<KD, KH, KW, 1, RW, RHK>(ex, st.ho + (off_s + i * RS * P), P, wi, st.t1acc, RH);
+                        if (extra) k_rows<KD, KH, KW, 1, RW, RHK, LOOSE>(ex, st.ho + (off_s + i * RS * P), P, wi, st.t1acc, RH);
                     }
                 }
                 // plane k - PD of t1 is complete: publish it (zero outside the volume)
@@ -561,7 +578,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) {
                         v[c] = live ? st.t1acc[0][r][c] : 0.f;
-                        if (mine) ex.st_((r < RH ? st.ob + (tb + (PH + r) * P) : st.ho + tb) + PW + c, v[c]);
+                        if (mine) stage<LOOSE>(ex, (r < RH ? st.ob + (tb + (PH + r) * P) : st.ho + tb) + PW + c, v[c]);
                     }
                     if (r < RH && t1g && live && pf >= d0 && pf < d1)
                         IO::store(t1g + (long long)pf * plane + st.ooff[r < RH ? r : 0], v);
@@ -611,7 +628,7 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
                     const int pl = j0 + PD - td;
                     const int base[2] = {st.ob + (off_x + wrap(pl % XR, XR) * RX * P),
                                          st.ob + (off_t + wrap(pl % KD, KD) * RX * P)};
-                    a_plane<KH, KW, KT, SC, RH, RW, 2>(ex, base, P, wt, acc);
+                    a_plane<KH, KW, KT, SC, RH, RW, 2, LOOSE>(ex, base, P, wt, acc);
                 }
                 NDC_UNROLL
                 for (int r = 0; r < RH; ++r)
@@ -657,7 +674,8 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T> stru
 template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool SAVED_ = false>
 struct Bwd1Kernel {
     static constexpr bool SAVED = SAVED_;
-    static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_;
+    static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_ < 0 ? -RW_ : RW_;
+    static constexpr bool LOOSE = RW_ < 0;   // rows of any length and alignment (see Lane)
     static constexpr int PD = KD / 2, PH = KH / 2, PW = KW / 2, KT = KD * KH * KW;
     static constexpr int XT = PH > 0 ? 1 : 0;
     static constexpr int NXR = RH + (PH > 0 ? 2 : 0);   // rows of x/t1 a thread stages
@@ -665,9 +683,9 @@ struct Bwd1Kernel {
     static constexpr int NRED = SC * KT;
     // own rows of the kept tensors requested a phase ahead, where the registers for it are there (the
     // 2 x 2 tile of a 3-D filter would spill 17)
-    static constexpr bool AHEAD = SAVED && (KH_ == 1 || RH_ * RW_ < 4);
+    static constexpr bool AHEAD = SAVED && (KH_ == 1 || RH_ * RW < 4);
     typedef BwdParams<T> Params;
-    typedef VecIO<T, RW> IO;
+    typedef VecIO<T, RW_> IO;
 
     struct State {
         Lane ln;
@@ -746,8 +764,8 @@ struct Bwd1Kernel {
                     NDC_UNROLL
                     for (int c = 0; c < RW; ++c) {
                         const int o = st.so + (slot * RX + n * S) * P + c;
-                        ex.st_(off_x + o, live ? st.px[n][c] : 0.f);
-                        ex.st_(off_t + o, live ? st.pt[n][c] : 0.f);
+                        stage<LOOSE>(ex, off_x + o, live ? st.px[n][c] : 0.f);
+                        stage<LOOSE>(ex, off_t + o, live ? st.pt[n][c] : 0.f);
                     }
                 }
             }
@@ -828,7 +846,7 @@ struct Bwd1Kernel {
                     const int slot = wrap((j1 + PD - td) % XR, XR);
                     const int ob = lo - PW + slot * RX * P;
                     const int base[2] = {off_x + ob, off_t + ob};
-                    a_plane<KH, KW, KT, SC, NR, RW, 2>(ex, base, P, wt, acc);
+                    a_plane<KH, KW, KT, SC, NR, RW, 2, LOOSE>(ex, base, P, wt, acc);
                 }
             }
             NDC_UNROLL
@@ -846,15 +864,15 @@ struct Bwd1Kernel {
                             gn = gv[i][r][c] * sv[i][r][c] * inv;
                             gd = -(gn * (acc[0][i][r][c] + eps)) * inv;
                         }
-                        ex.st_(lo + (off_g + (i * RG + r) * P) + c, gn);
-                        ex.st_(lo + (off_g + ((SC + i) * RG + r) * P) + c, gd);
+                        stage<LOOSE>(ex, lo + (off_g + (i * RG + r) * P) + c, gn);
+                        stage<LOOSE>(ex, lo + (off_g + ((SC + i) * RG + r) * P) + c, gd);
                         acc[0][i][r][c] = gn;
                         acc[1][i][r][c] = gd;
                     }
         };
 
         ex.each([&](State &st, int tid) NDC_LAMBDA {
-            st.ln = make_lane(tid, t, RW);
+            st.ln = make_lane<RW, LOOSE>(tid, t, W);
             st.ob = st.ln.strip * RH * P + PL + st.ln.c0 - PW;
             st.so = st.ln.strip * P + PL + st.ln.c0;
             st.ho = halo_row(st.ln.strip, PH, TH) * P + PL + st.ln.c0;
@@ -907,11 +925,18 @@ struct Bwd1Kernel {
                     const int j = PH + st.ln.strip * RH;
                     gn_gd_rows(st, j1, j, st.ob + (PW + PH * P), IntTag<RH>(), IntTag<1>(), acc);
                     if (need_gh && own1) {
+                        if constexpr (LOOSE) {
+                            NDC_UNROLL
+                            for (int i = 0; i < SC; ++i)
+                                NDC_UNROLL
+                                for (int r = 0; r < RH; ++r)
+                                    if (st.ln.twice) acc[0][i][r][0] = acc[1][i][r][0] = 0.f;
+                        }
                         // own rows: A-side filter-gradient terms, re-reading the x / t1 windows
                         // (read ahead: for the 2x2 float32 tile this costs two spilled registers
                         // and is still 3 % faster)
                         constexpr int NQ = RH + 2 * PH;
-                        stream_rows<KD * NQ, RW + KW - 1, 2, (KH > 1 && SAVED), RW>(
+                        stream_rows<KD * NQ, RW + KW - 1, 2, (KH > 1 && SAVED), RW, LOOSE>(
                             ex,
                             [&](int n, int t) NDC_LAMBDA {
                                 const int td = n / NQ, q = n % NQ;
@@ -960,8 +985,8 @@ struct Bwd1Kernel {
                         float wi[KT];
                         load_taps<KT>(hw + i * KT, wi);
                         const int gb_ = st.ob + off_g;
-                        k_rows<KD, KH, KW, RH, RW, RH, (KH > 1 && SAVED)>(ex, gb_ + i * RG * P, P, wi, st.accx, 0);
-                        k_rows<KD, KH, KW, RH, RW, RH, (KH > 1 && SAVED)>(ex, gb_ + (SC + i) * RG * P, P, wi, st.acct, 0);
+                        k_rows<KD, KH, KW, RH, RW, RH, LOOSE, (KH > 1 && SAVED)>(ex, gb_ + i * RG * P, P, wi, st.accx, 0);
+                        k_rows<KD, KH, KW, RH, RW, RH, LOOSE, (KH > 1 && SAVED)>(ex, gb_ + (SC + i) * RG * P, P, wi, st.acct, 0);
                     }
                 }
                 const int pf = k - 2 * PD;
@@ -1004,13 +1029,14 @@ template <int KD_, int KH_, int KW_, int SC_, int RH_, int RW_, typename T, bool
 struct Bwd2Kernel {
     static constexpr bool SAVED = SAVED_;
     static constexpr int NA = SAVED ? 1 : 3;   // gathered operands: (x, t1,) gt1
-    static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_;
+    static constexpr int KD = KD_, KH = KH_, KW = KW_, SC = SC_, RH = RH_, RW = RW_ < 0 ? -RW_ : RW_;
+    static constexpr bool LOOSE = RW_ < 0;   // rows of any length and alignment (see Lane)
     static constexpr int PD = KD / 2, PH = KH / 2, PW = KW / 2, KT = KD * KH * KW;
     static constexpr int NXR = RH + (PH > 0 ? 1 : 0);
     static constexpr int XR = KD + 1;
     static constexpr int NRED = SC * KT + SC;
     typedef BwdParams<T> Params;
-    typedef VecIO<T, RW> IO;
+    typedef VecIO<T, RW_> IO;
 
     struct State {
         Lane ln;
@@ -1083,17 +1109,17 @@ struct Bwd2Kernel {
                     for (int c = 0; c < RW; ++c) {
                         const int o = st.so + (slot * RX + n * S) * P + c;
                         if (!SAVED) {
-                            ex.st_(off_x + o, live ? st.px[n][c] : 0.f);
-                            ex.st_(off_t + o, live ? st.pt[n][c] : 0.f);
+                            stage<LOOSE>(ex, off_x + o, live ? st.px[n][c] : 0.f);
+                            stage<LOOSE>(ex, off_t + o, live ? st.pt[n][c] : 0.f);
                         }
-                        ex.st_(off_g + o, live ? st.pg[n][c] : 0.f);
+                        stage<LOOSE>(ex, off_g + o, live ? st.pg[n][c] : 0.f);
                     }
                 }
             }
         };
 
         ex.each([&](State &st, int tid) NDC_LAMBDA {
-            st.ln = make_lane(tid, t, RW);
+            st.ln = make_lane<RW, LOOSE>(tid, t, W);
             st.ob = st.ln.strip * RH * P + PL + st.ln.c0 - PW;
             st.so = st.ln.strip * P + PL + st.ln.c0;
             st.xok = st.ook = 0u;
@@ -1169,7 +1195,7 @@ struct Bwd2Kernel {
                         base[0] = off_x + ob;
                         base[NA > 1 ? 1 : 0] = off_t + ob;
                     }
-                    a_plane<KH, KW, KT, SC, RH, RW, NA, (KH > 1 && SAVED)>(ex, base, P, wt, acc);
+                    a_plane<KH, KW, KT, SC, RH, RW, NA, LOOSE, (KH > 1 && SAVED)>(ex, base, P, wt, acc);
                 }
                 NDC_UNROLL
                 for (int r = 0; r < RH; ++r) {
@@ -1184,10 +1210,17 @@ struct Bwd2Kernel {
                             gv[i][r][c] = ok ? gv[i][r][c] : 0.f;
                         }
                 }
+                auto filter_terms = [&]() NDC_LAMBDA {
                 if (need_gh) {
+                    if constexpr (LOOSE) {
+                        NDC_UNROLL
+                        for (int i = 0; i < SC; ++i)
+                            NDC_UNROLL
+                            for (int r = 0; r < RH; ++r) sv[i][r][0] = st.ln.twice ? 0.f : sv[i][r][0];
+                    }
                     // K-side filter-gradient term: re-read the gt1 window
                     constexpr int NQ = RH + 2 * PH;
-                    stream_rows<KD * NQ, RW + KW - 1, 1, (KH > 1 && SAVED), RW>(
+                    stream_rows<KD * NQ, RW + KW - 1, 1, (KH > 1 && SAVED), RW, LOOSE>(
                         ex,
                         [&](int n, int) NDC_LAMBDA {
                             const int td = n / NQ, q = n % NQ;
@@ -1212,6 +1245,8 @@ struct Bwd2Kernel {
                             }
                         });
                 }
+                };
+                auto write_gz = [&]() NDC_LAMBDA {
                 NDC_UNROLL
                 for (int r = 0; r < RH; ++r) {
                     if (!((st.ook >> r) & 1u)) continue;
@@ -1228,12 +1263,17 @@ struct Bwd2Kernel {
                                           fast_rcp(acc[NA > 1 ? 1 : 0][i][r][c] + eps) +
                                       acc[NA - 1][i][r][c];
                             if (p.relu && sv[i][r][c] <= 0.f) gzv = 0.f;   // a NaN passes
-                            st.gbacc[i] += gzv;
+                            st.gbacc[i] += LOOSE && c == 0 && st.ln.twice ? 0.f : gzv;
                             v[c] = gzv;
                         }
                         if (gzg) IO::store(gzg + i * cplane + ko + st.ooff[r], v);
                     }
                 }
+                };
+                // (LOOSE: the source values that do not count in the sums are zeroed for them)
+                if (LOOSE) write_gz();
+                filter_terms();
+                if (!LOOSE) write_gz();
             });
         }
 

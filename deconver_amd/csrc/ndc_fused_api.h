@@ -21,16 +21,27 @@ namespace fused {
 // (KD, KH, KW, SC, RHF, RWF, RHB, RWB): RHF x RWF is the register tile (rows x columns per
 // thread) of the forward kernel, RHB x RWB that of the two backward kernels.  Rows of one
 // filter geometry are listed in order of preference; a row with RW = 2 needs an even W and
-// tensors aligned to two elements, so every geometry also has an RW = 1 row.
+// tensors aligned to two elements; RW = -2 is the same for any width and alignment; every geometry also has
+// an RW = 1 row.
 #define NDC_FUSED_VARIANTS(X)        \
     X(3, 3, 3, 4, 2, 2, 2, 2)        \
     X(3, 3, 3, 4, 2, 2, 1, 2)        \
+    X(3, 3, 3, 4, 2, -2, 2, -2)      \
+    X(3, 3, 3, 4, 2, -2, 2, 1)       \
     X(3, 3, 3, 4, 4, 1, 2, 1)        \
     X(3, 3, 3, 4, 2, 1, 1, 1)        \
     X(5, 1, 5, 4, 1, 2, 1, 2)        \
+    X(5, 1, 5, 4, 1, -2, 1, -2)      \
+    X(5, 1, 5, 4, 1, 1, 1, -2)       \
     X(5, 1, 5, 4, 1, 1, 1, 1)        \
     X(3, 1, 3, 4, 1, 2, 1, 2)        \
+    X(3, 1, 3, 4, 1, -2, 1, -2)      \
+    X(3, 1, 3, 4, 1, 1, 1, -2)       \
     X(3, 1, 3, 4, 1, 1, 1, 1)
+
+// What a plan may use: one column a thread; in the forward also pairs at any width and alignment; in the backward
+// too; pairs of aligned tensors of an even width.
+enum { kSingles = 0, kLooseForward = 1, kLoosePairs = 2, kPairs = 3 };
 
 struct Variant {
     int KD, KH, KW, SC, RHF, RWF, RHB, RWB;
@@ -71,7 +82,7 @@ static inline Tuning tuning() { return Tuning{0, 0, 0, 0, 256, 512, 256, 256, 51
 
 // first listed row of this filter geometry that the width / alignment allow (and, in a
 // tuning run, that matches the requested register tiles)
-static inline bool find_variant(const KGeom &q, const March &m, bool pairs_ok, Variant &v)
+static inline bool find_variant(const KGeom &q, const March &m, int pairs, Variant &v)
 {
     if (q.m != 1) return false;
     const Tuning tn = tuning();
@@ -79,11 +90,25 @@ static inline bool find_variant(const KGeom &q, const March &m, bool pairs_ok, V
     // 128 columns a lane per column (not per column pair) keeps more of the wavefront busy
     // (measured 16-32 % faster from 16 to 100 columns, 4-15 % slower from 128 on)
     const bool narrow_2d = m.H == 1 && m.W < 128 && !tn.rwf && !tn.rwb;
-    const bool even = pairs_ok && m.W % 2 == 0 && !narrow_2d;
+    const bool even = pairs == kPairs && m.W % 2 == 0 && !narrow_2d;
+    // Loose pairs, where they are ahead of one column a thread (us, float32 / bf16, one column -> pairs).
+    // 3-D: forward 32 channels of 91 x 101 x 87 652 -> 585 / 661 -> 588, of 55 x 61 x 129 557 -> 369 / 556 -> 365, 4 x 128
+    // of 21 x 15 x 23 119 -> 114 / 122 -> 117; backward from 32 columns on (32 of 91 x 101 x 87 1177 -> 1109 / 1117 -> 983,
+    // 64 of 45 x 53 x 77 543 -> 539 / 519 -> 490, 2 x 64 of 33 x 40 x 31 252 -> 256 / 228 -> 241, 512 of 13 x 11 x 9
+    // 72 -> 101).  2-D: backward 8 x 32 of 257 x 255 596 -> 537 / 575 -> 460, 2 x 128 of 301 x 299 1275 -> 996 /
+    // 1342 -> 953; forward up to 256 columns (297 -> 258 / 293 -> 257; 301 x 299 415 -> 431 / 417 -> 443).  3-D rows of more
+    // than 192 leave the backward one workgroup a CU (64 of 30 x 41 x 255 857 -> 1073 / 782 -> 949).
+    // (Rows that one column a thread cannot take stay outside.)
+    const bool plane = m.H == 1;
+    const bool loose_f = pairs >= kLooseForward && !narrow_2d && m.W >= 2 && m.W <= 256;
+    const bool loose_b = pairs >= kLoosePairs && !narrow_2d && m.W >= 32 && m.W <= (plane ? 512 : 192);
+    auto takes = [&](int rwf, int rwb) {
+        return (rwf == 1 || (rwf == 2 ? even : loose_f)) && (rwb == 1 || (rwb == 2 ? even : loose_b));
+    };
     bool found = false;
 #define X(kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_)                                        \
     if (!found && m.KD == kd_ && m.KH == kh_ && m.KW == kw_ && q.sc == sc_ &&                \
-        (even || (rwf_ == 1 && rwb_ == 1)) && (!tn.rhf || tn.rhf == rhf_) &&                 \
+        takes(rwf_, rwb_) && (!tn.rhf || tn.rhf == rhf_) &&                 \
         (!tn.rwf || tn.rwf == rwf_) && (!tn.rhb || tn.rhb == rhb_) &&                        \
         (!tn.rwb || tn.rwb == rwb_)) {                                                       \
         v = Variant{kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_};                             \
@@ -95,7 +120,7 @@ static inline bool find_variant(const KGeom &q, const March &m, bool pairs_ok, V
     // no row matches a tuning request: fall back to the plain order of preference
 #define X(kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_)                                        \
     if (!found && m.KD == kd_ && m.KH == kh_ && m.KW == kw_ && q.sc == sc_ &&                \
-        (even || (rwf_ == 1 && rwb_ == 1))) {                                                \
+        takes(rwf_, rwb_)) {                                                \
         v = Variant{kd_, kh_, kw_, sc_, rhf_, rwf_, rhb_, rwb_};                             \
         found = true;                                                                        \
     }
@@ -263,17 +288,16 @@ static inline void plan_lds(Plan &pl, long long nbc)
     pl.lds_b2 = Bwd2Kernel<KD, KH, KW, SC, RHB, RWB, float>::lds_floats(pl.tb);
 }
 
-// pairs_ok: every activation pointer of the call is aligned to two elements
 static const int kDot2RH = 2;   // rows per thread of the bf16 dot2 kernels (columns: 2)
 
-static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dtype, bool matrix)
+static inline bool make_plan_for(const KGeom &q, Plan &pl, int pairs, int dtype, bool matrix)
 {
     pl.m = march_of(q);
     pl.dot2 = false;
     pl.mfma1 = pl.mfma2 = pl.mfmaf = false;
     // 32-bit offsets inside one (sample, channel) volume
     if ((long long)q.sc * q.SP >= (1LL << 31)) return false;
-    if (!find_variant(q, pl.m, pairs_ok, pl.v)) return false;
+    if (!find_variant(q, pl.m, pairs, pl.v)) return false;
     const Tuning tn = tuning();
     if (!make_tile(pl.m, pl.v.RHF, pl.v.RWF, tn.threads_f, pl.tf)) return false;
     if (!make_tile(pl.m, pl.v.RHB, pl.v.RWB, tn.threads_b, pl.tb)) return false;
@@ -288,7 +312,7 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
     NDC_FUSED_VARIANTS(X)
 #undef X
     // (their buffer addressing wants every (sample, channel group) slice below 2^31 bytes)
-    if (dtype == NDC_BF16 && pairs_ok && pl.m.W % 2 == 0 && q.sc == 4 && pl.m.KD == 3 &&
+    if (dtype == NDC_BF16 && pairs == kPairs && pl.m.W % 2 == 0 && q.sc == 4 && pl.m.KD == 3 &&
         (long long)q.sc * q.SP * 2 < (1LL << 31) &&
         pl.m.KH == 3 && pl.m.KW == 3 && tn.dot2) {
         Tile tf, tb;
@@ -349,7 +373,7 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
         } else {
             pl.small_f = pl.small_f && covered <= kCoveredF;
         }
-        pl.t2.PL = pairs_ok && pl.m.W % 2 == 0;   // pixels go in and out by pairs
+        pl.t2.PL = pairs == kPairs && pl.m.W % 2 == 0;   // pixels go in and out by pairs
         if (pl.small_f) pl.nblk_f2 = (int)(nbc * pl.t2.ntile);
         if (pl.small_b) pl.nblk_b2 = (int)(nbc * ((pl.t2.ntile + pl.t2.SEG - 1) / pl.t2.SEG));
     }
@@ -361,10 +385,12 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, bool pairs_ok, int dt
 // those are what supported() answers for.
 // matrix: the call runs the matrix-instruction family where it covers the geometry (its launch shapes
 // are its own, the filter's table is the same, and workspace sizes serve both)
+// pairs_ok: every activation pointer of the call is aligned to two elements
 static inline bool make_plan_fresh(const KGeom &q, Plan &pl, bool pairs_ok, int dtype, bool matrix)
 {
-    if (make_plan_for(q, pl, pairs_ok, dtype, matrix)) return true;
-    return pairs_ok && make_plan_for(q, pl, false, dtype, matrix);
+    for (int pairs = pairs_ok ? kPairs : kLoosePairs; pairs >= kSingles; --pairs)
+        if (make_plan_for(q, pl, pairs, dtype, matrix)) return true;
+    return false;
 }
 
 // A plan is a function of sizes, and a forward and a backward ask for it some ten times (what is

@@ -377,3 +377,27 @@ def test_autograd_node_names_its_family_once(matrix_switch):
 
     for a, b in zip(run(False), run(True)):
         assert torch.equal(a, b)
+
+
+# column pairs of rows of any length and alignment (W even: at an odd element): one pair a row, either side of where the
+# backward takes them (32 columns), several wavefronts a row; 2-D marches of large images, in the backward only past 256
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("C,ks,sp", [(3, (3, 3, 3), (3, 5, 2)), (3, (3, 3, 3), (6, 7, 31)), (2, (3, 3, 3), (5, 9, 33)),
+                                     (2, (3, 3, 3), (4, 6, 64)), (1, (3, 3, 3), (5, 7, 255)), (64, (5, 5), (150, 201)),
+                                     (48, (3, 3), (160, 301))])
+def test_pairs_of_any_width_and_alignment(C, ks, sp, dtype, tol):
+    print("case", C, ks, sp, dtype, flush=True)
+    lib = _lib.get_library()
+    x, z, h, bias, gout = make_case(C, C, 4, ks, sp, B=1, bias_shift=0.3, dtype=dtype)
+    odd = lambda t: torch.empty(t.numel() + 1, dtype=dtype, device="cuda")[1:].view(t.shape).copy_(t)   # noqa: E731
+    dx, dz, dg = odd(x), odd(z), odd(gout)
+    dh, db = h.cuda(), bias.cuda()
+    kw = dict(groups=C, m=1, sc=4, eps=1e-16, relu_input=True)
+    out, t1, saved = ops.update_forward(lib, dx, dz, dh, db, save_ratio=True, **kw)
+    d = [t.double() for t in (x, z, h, bias, gout)]
+    ro, rt = O.update_grouped(d[0], d[1], d[2], d[3], C, 1, 4, 1e-16, True)
+    refs = [ro, rt, *O.update_backward(d[0], d[1], d[2], d[3], d[4], C, 1, 4, 1e-16, True)]
+    for keep in (saved, None):
+        got = [out, t1, *ops.update_backward(lib, dx, dz, t1, dh, db, dg, saved=keep, **kw)]
+        for a, ref in zip(got, refs):
+            assert O.rel_err(a.double().cpu(), ref) < tol

@@ -6,7 +6,7 @@ import torch
 
 from deconver_amd import _lib, ops
 from oracle import ndc_oracle as O
-from tests.helpers import host_faults, hostcheck_library, make_case
+from tests.helpers import host_faults, host_march, hostcheck_library, make_case
 
 # (C, sc, kernel, spatial, batch)
 FUSED_GEOMS = [
@@ -57,6 +57,43 @@ def _saved_refs(x, z, h, bias, C, sc, eps, relu):
     t1 = O.op_K(s, hd, C, 1, sc)
     den = O.op_A(t1, hd, C, 1, sc) + eps
     return s / den, (O.op_A(xd, hd, C, 1, sc) + eps) / den
+
+
+# column pairs of rows of any length: the last pair of an odd row overlaps the one before it; one pair a row, where
+# the backward takes pairs too (from 32 columns on), 2-D marches with pairs both ways and in the backward only
+LOOSE_GEOMS = [(2, 4, (3, 3, 3), (3, 5, 2), 1), (2, 4, (3, 3, 3), (4, 6, 3), 1), (1, 4, (3, 3, 3), (3, 5, 31), 1),
+               (1, 4, (3, 3, 3), (4, 9, 33), 2), (1, 4, (3, 3, 3), (5, 7, 65), 1), (1, 4, (5, 5), (9, 131), 1),
+               (1, 4, (3, 3), (6, 257), 1)]
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("geom", LOOSE_GEOMS)
+def test_pairs_of_any_width_and_alignment(geom, shift, dtype, tol):
+    """Against the oracle, with tensors at even and odd elements (an even row at an odd element takes these pairs
+    too)."""
+    C, sc, ks, sp, B = geom
+    lib = hostcheck_library()
+    tensors = make_case(C, C, sc, ks, sp, B=B, bias_shift=0.3, dtype=dtype)
+
+    def moved(t):
+        flat = torch.empty(t.numel() + 4, dtype=t.dtype)
+        at = shift + (-(flat.data_ptr() // t.element_size()) % 2)
+        out = flat[at:at + t.numel()].view(t.shape)
+        return out.copy_(t)
+
+    x, z, h, bias, gout = tensors
+    x, z, gout = moved(x), moved(z), moved(gout)
+    kw = dict(groups=C, m=1, sc=sc, eps=1e-16, relu_input=True)
+    host_faults(lib)
+    with host_march(lib):
+        out, t1, saved = ops.update_forward(lib, x, z, h, bias, save_ratio=True, **kw)
+        for keep in (saved, None):
+            got = [out, t1, *ops.update_backward(lib, x, z, t1, h, bias, gout, saved=keep, **kw)]
+            ro, rt, rg = _oracle(x, z, h, bias, gout, C, sc, 1e-16, True)
+            for a, ref in zip(got, [ro, rt, *rg]):
+                assert O.rel_err(a.double(), ref) < tol
+    assert host_faults(lib)[0] == 0
 
 
 @pytest.mark.parametrize("geom", FUSED_GEOMS)
