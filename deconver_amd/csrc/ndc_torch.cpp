@@ -642,6 +642,24 @@ Tensor update(const Tensor &x, const Tensor &z, const Tensor &h, const OptTensor
     return update_forward(x, z, h, bias ? *bias : Tensor(), taps ? *taps : Tensor(), c, false, f, scope.stream);
 }
 
+// Whether a bare float32 product that widens -- a layer's projection, an upsampling -- is the tiled GEMM's: those
+// below half a GFLOP, and up to one from at most 128 channels.  A call of the library takes the host 10-18 us longer,
+// and on the GPU the tiled GEMM is ahead or within 2 us there (us, library / tiled: 32 -> 128 channels over 4096 voxels
+// 5.3 / 4.5, over 36 608 12.9 / 9.1; 64 -> 256 over 9152 10.3 / 8.8; 48 -> 192 over 36 608 37.6 / 15.0; 128 -> 256 over
+// 143 29 / 4.0, over 4096 6.9 / 8.0; 256 -> 1024 over 572 9.0 / 10.0; behind from there on: 512 -> 1024 over 572, 0.6
+// GFLOP, 11.3 / 16.4, 512 -> 2048 17 / 24).  It is nearer to 64 bits too (32 to 512 channels 0.7e-7 to 1.6e-7 of the
+// result's norm, the library 1.0e-7 to 4.1e-7).  Past a GFLOP the library's product stays also where it is behind: its
+// bits decide which source units are on, and what else forms the product of a large network -- a check of its on/off
+// patterns by torch.bmm -- sees the same units.  Samples count with the columns of 64 voxels they fill.
+// One 208 x 176 image through the 2-D network, forward: 1.24 -> 0.95 ms; a layer of 32 channels of 64^2 with its
+// backward 0.180 -> 0.150.
+bool wide_is_tiled(int64_t B, int64_t cin, int64_t cout, int64_t n)
+{
+    if (cin >= cout || B < 1 || n < 1 || B > (1 << 20)) return false;   // (nothing to do, or more than the tiled GEMM takes)
+    const double columns = (double)B * (double)((n + 63) / 64 * 64), flops = 2.0 * (double)cin * (double)cout * columns;
+    return flops < 0.5e9 || (cin <= 128 && flops < 1e9);
+}
+
 // The layer's first update together with the 1x1 projection that makes its source
 // (deconv.py:157-165 with layers/linear.py:53-58 of the reference): z = W x per sample, then the
 // update of (x, z) with the projection's bias and the ReLU applied where the kernels load z.  One
@@ -657,9 +675,9 @@ struct Projected : public torch::autograd::Function<Projected> {
         // (the GEMMs and the update read rows of voxels: any other layout is turned first)
         const Tensor x = channel_first(x_, stream);
         auto size = x.sizes().vec();
-        // (float32: the library's product.  Its bits decide which source units are on, and what else forms
-        // this product -- a check of a network's on/off patterns by torch.bmm -- sees the same units)
-        Tensor z = project(w, x.flatten(2), x.scalar_type() == at::kFloat, stream);
+        const Tensor flat = x.flatten(2);
+        const bool library = x.scalar_type() == at::kFloat && !wide_is_tiled(flat.size(0), w.cin(), w.cout(), flat.size(2));
+        Tensor z = project(w, flat, library, stream);
         size[1] = w.cout();
         Tensor out = update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
         f.x_last = channels_last(x_);
@@ -753,9 +771,10 @@ struct Linear : public torch::autograd::Function<Linear> {
         const int64_t B = x.size(0), n = x.size(2), cout = w.cout();
         const bool tail = bias.defined() || act != NDC_ACT_NONE || res.defined();
         // An activation's tile form reads W as rows.  A bare float32 product that widens could be a layer's
-        // projection taken apart: the library's product, bit for bit as in Projected.
+        // projection taken apart: the same product, bit for bit, as in Projected.
         const bool bare = !tail && x.scalar_type() == at::kFloat;
-        const bool library = (w.transposed && act != NDC_ACT_NONE) || (bare && !narrow_is_tiled(B, w.cin(), cout, n));
+        const bool library = (w.transposed && act != NDC_ACT_NONE) ||
+                             (bare && !narrow_is_tiled(B, w.cin(), cout, n) && !wide_is_tiled(B, w.cin(), cout, n));
         const Gemm by = library ? kLibrary : choose_gemm(x, cout, act != NDC_ACT_NONE || keep, tail);
         Tensor y = empty({B, cout, n}, x);
         if (keep) z = empty({B, cout, n}, x);

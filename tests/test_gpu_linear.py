@@ -93,3 +93,20 @@ def test_bare_float32_products_that_narrow(B, cin, cout, n, tiled):
     y = pointwise_linear(x, w)
     assert float((y.double() - w.double() @ x.double()).norm() / y.double().norm()) < 2e-6     # float32 sums
     assert tiled or torch.equal(y, torch.bmm(w.expand(B, cout, cin), x))
+
+
+# (B, cin, cout, n, by the tiled GEMM): either side of each bound of the rule for those that widen
+WIDE = [(1, 16, 64, 1, True), (3, 18, 75, 77, True), (1, 64, 65, 100, True), (256, 256, 512, 1, False), (7, 512, 1024, 1, True),
+        (8, 512, 1024, 1, False), (1, 256, 1024, 896, True), (1, 256, 1024, 960, False),
+        (2, 128, 512, 3776, True), (2, 128, 512, 3840, False), (1, 136, 512, 3776, False)]
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("B,cin,cout,n,tiled", WIDE)
+def test_bare_float32_products_that_widen(B, cin, cout, n, tiled, transposed):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, w = torch.randn(B, cin, n, generator=g, device="cuda"), torch.randn(cout, cin, generator=g, device="cuda") / cin ** 0.5
+    y = pointwise_linear(x, w.t().contiguous() if transposed else w, transposed=transposed)
+    assert float((y.double() - w.double() @ x.double()).norm() / y.double().norm()) < 2e-6     # float32 sums
+    lib = torch.bmm(w.expand(B, cout, cin), x)
+    assert tiled or (y - lib).abs().max() <= 0 or transposed    # (the library has a kernel of its own for each storage)
