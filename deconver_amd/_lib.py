@@ -36,6 +36,8 @@ EXPORTS = (
     "ndc_prepare_taps",
     "ndc_forward_taps",
     "ndc_backward_taps",
+    "ndc_rectify_filter",
+    "ndc_backward_rectified",
     "ndc_backward_workspace_bytes",
     "ndc_backward",
     "ndc_backward_profiled",
@@ -194,6 +196,8 @@ class NdcLibrary:
         d.ndc_forward_taps.argtypes = [gp, vp, vp, fp, vp, fp, vp, vp, vp, vp, vp]
         d.ndc_backward_taps.argtypes = [gp, vp, vp, vp, vp, vp, fp, vp, fp, vp, vp, vp, fp, fp, vp,
                                         ctypes.c_size_t, vp]
+        d.ndc_rectify_filter.argtypes = [gp, fp, fp, vp, ctypes.c_size_t, vp]
+        d.ndc_backward_rectified.argtypes = d.ndc_backward_taps.argtypes
         # answers of the geometry queries, per geometry: they depend on nothing else, and a
         # layer asks the same few questions on every call
         self._answers = {}
@@ -248,6 +252,18 @@ class NdcLibrary:
     def prepare_taps(self, g: Geom, h: int, taps: int, taps_bytes: int, stream) -> None:
         self._check(self._dll.ndc_prepare_taps(ctypes.byref(g), h, taps, taps_bytes, stream),
                     "ndc_prepare_taps")
+
+    def rectify_filter(self, g: Geom, h0: int, h: int, taps, taps_bytes: int, stream) -> None:
+        self._check(self._dll.ndc_rectify_filter(ctypes.byref(g), h0, h, taps, taps_bytes, stream),
+                    "ndc_rectify_filter")
+
+    def backward_rectified(self, g: Geom, x, z, t1, s_over_den, ratio, h, taps, bias, gout, gx, gz, gh,
+                           gb, ws, ws_bytes, stream) -> None:
+        """``backward_taps`` with ``gh`` the gradient of the filter before its rectifier."""
+        self._check(
+            self._dll.ndc_backward_rectified(ctypes.byref(g), x, z, t1, s_over_den, ratio, h, taps, bias,
+                                             gout, gx, gz, gh, gb, ws, ws_bytes, stream),
+            "ndc_backward_rectified")
 
     def forward_taps(self, g: Geom, x, z, h, taps, bias, out, t1, s_over_den, ratio, stream) -> None:
         """``forward`` with a filter table prepared by ``prepare_taps``: no workspace."""

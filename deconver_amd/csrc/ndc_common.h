@@ -360,6 +360,7 @@ struct KGeom {
     int KT;        // kD*kH*kW
     int relu;      // rectify z (+bias) on load
     int matrix;    // bf16 3x3x3 calls run the matrix-instruction kernel family where it covers them
+    int gate;      // gh is the gradient of the filter before its rectifier: zero where h is not positive
     float eps;
     long long SP;  // D*H*W
 

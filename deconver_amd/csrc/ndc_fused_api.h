@@ -531,6 +531,16 @@ template <class BE> static int prepare_taps(const KGeom &q, const float *h, floa
                            [=] NDC_LAMBDA(long long idx) { prep_tables(idx, h, tab); });
 }
 
+// h = max(h0, 0) and the tables of h, in one launch: a filter of 4 x 27 taps has fewer values than its table words
+template <class BE> static int rectify_and_prepare(const KGeom &q, const float *h0, float *h, float *tab, void *stream)
+{
+    return BE::elementwise((long long)q.G * kTabWords, stream, [=] NDC_LAMBDA(long long idx) {
+        const long long c = idx / kTabWords, e = idx % kTabWords;
+        if (e < 4 * 27) h[c * 4 * 27 + e] = floor_f(h0[c * 4 * 27 + e], 0.f);
+        prep_tables(idx, Rectified{h0}, tab);
+    });
+}
+
 // f(kernel type tag): the instance of a one-shot 2-D kernel for this plan
 template <template <int, int, typename> class Kernel, typename T, class F> static int with_tile_2d(const Plan &pl, F f)
 {
@@ -649,9 +659,9 @@ int backward(const KGeom &q, const T *x, const T *z, const T *t1, const T *s_ove
     int st = NDC_ERR_GEOMETRY;
     const int C = q.G, SC = q.sc, B = q.B;
     // (gh and gb in one launch: outputs [0, C kt) are gh, the C SC after them gb)
-    const int n_gh = gh ? C * kt : 0, n_gb = gb ? C * SC : 0;
+    const int n_gh = gh ? C * kt : 0, n_gb = gb ? C * SC : 0, gate = q.gate;
     auto put = [=] NDC_LAMBDA(int o, float v) {
-        if (o < n_gh) gh[o] = v; else gb[o - n_gh] = v;
+        if (o < n_gh) gh[o] = gate && h[o] <= 0.f ? 0.f : v; else gb[o - n_gh] = v;
     };
     if (pl.small_b && saved) {
         float *part = (float *)ws;

@@ -48,10 +48,17 @@ static const int kTabWK = 0, kTabWA = 54, kTabWQ = 126, kTabWM = 174, kTabWG = 2
 static const int kTabWords = 318;   // packed tap words per channel (54 WK + 72 WA + 48 WQ + 72 WM + 72 WG)
 
 // idx over C * kTabWords
-NDC_HD void prep_tables(long long idx, const float *h, float *tab)
+// (Filter: `const float *`, or a Rectified one, whose table then is the rectified filter's.)
+struct Rectified {
+    const float *h;
+    NDC_HD float operator[](long long i) const { return floor_f(h[i], 0.f); }
+    NDC_HD Rectified operator+(long long i) const { return {h + i}; }
+};
+
+template <class Filter> NDC_HD void prep_tables(long long idx, Filter h, float *tab)
 {
     const int c = (int)(idx / kTabWords), e = (int)(idx % kTabWords);
-    const float *hc = h + (long long)c * 4 * 27;
+    const Filter hc = h + (long long)c * 4 * 27;
     uint32_t w;
     if (e < 54) {
         const int p = e / 27, tau = e % 27;
@@ -62,7 +69,7 @@ NDC_HD void prep_tables(long long idx, const float *h, float *tab)
                    : pack_bf16x2(0.f, hc[i * 27 + t9]);
     } else if (e < kTabWM) {
         const int r = e - kTabWQ, th = r / 16, i = (r % 16) / 4, n = r % 4;
-        const float *ht = hc + i * 27 + th * 3;   // the tap row h[i][0][th][0..2]
+        const Filter ht = hc + (i * 27 + th * 3);   // the tap row h[i][0][th][0..2]
         w = n == 0 ? pack_bf16x2(ht[1], ht[0]) : n == 1 ? pack_bf16x2(0.f, ht[2])
           : n == 2 ? pack_bf16x2(ht[2], ht[1]) : pack_bf16x2(ht[0], 0.f);
     } else if (e < kTabWG) {
@@ -71,7 +78,7 @@ NDC_HD void prep_tables(long long idx, const float *h, float *tab)
         w = m == 3 ? 0u : pack_bf16x2(hc[(2 * half) * 27 + tau], hc[(2 * half + 1) * 27 + tau]);
     } else {
         const int r = e - kTabWG, i = r / 18, t9 = (r % 18) / 2, half = r % 2;
-        const float *ht = hc + i * 27 + t9 * 3;   // the tap row h[i][td][th][0..2]
+        const Filter ht = hc + (i * 27 + t9 * 3);   // the tap row h[i][td][th][0..2]
         w = half == 0 ? pack_bf16x2(ht[2], ht[1]) : pack_bf16x2(ht[0], 0.f);
     }
     tab[idx] = bits_to_float(w);

@@ -9,7 +9,7 @@
 // a training step on one 32^3 volume took 12.7 ms for 5.7 ms of kernels, one forward + backward
 // of a 32-channel 64^2 layer 0.48 ms for 0.15 ms of kernels.  The arithmetic stays behind the C
 // ABI of include/deconver_ndc.h; nothing here computes on tensors except through it, the
-// library GEMMs that choose_gemm leaves, the rectifier of a filter, and a few float32 sums of
+// library GEMMs that choose_gemm leaves, and a few float32 sums of
 // partial results.
 #include <torch/extension.h>
 
@@ -472,6 +472,16 @@ Tensor scratch(size_t bytes, const Tensor &like)
     return buf.narrow(0, off, (int64_t)bytes);
 }
 
+// max(h0, 0), and where no table is given the one the kernels of this geometry read
+Tensor rectify_filter(const ndc_geom &g, const Tensor &h0, Tensor &taps, void *stream)
+{
+    const size_t bytes = taps.defined() ? 0 : ndc_taps_bytes(&g);
+    Tensor h = at::empty_like(h0);
+    if (bytes) taps = scratch(bytes, h0);
+    check(ndc_rectify_filter(&g, fptr(h0), out_fptr(h), bytes ? out_ptr(taps) : nullptr, bytes, stream), "ndc_rectify_filter");
+    return h;
+}
+
 // the filter table the kernels of this geometry read instead of h, or undefined
 Tensor prepare_taps(const ndc_geom &g, const Tensor &h, void *stream)
 {
@@ -495,9 +505,9 @@ struct UpdateForward {
     bool x_last, z_last;                           // x / z came in channels-last
 };
 
-// Forward of an update.  `grad`: a backward will follow.
+// Forward of an update.  `grad`: a backward will follow.  `rectify`: h is the filter before its rectifier.
 Tensor update_forward(Tensor x, Tensor z, const Tensor &h, const Tensor &bias, Tensor taps, const UpdateConfig &c, bool grad,
-                      UpdateForward &f, void *stream)
+                      UpdateForward &f, void *stream, bool rectify = false)
 {
     // channels-last tensors come in through the library's tiled transposition, and the results
     // go back out the same way, in the layout of the tensor they belong to
@@ -517,7 +527,8 @@ Tensor update_forward(Tensor x, Tensor z, const Tensor &h, const Tensor &bias, T
     const bool keep = grad && c.save_ratio && ndc_backward_uses_saved(&g);
     check_taps(taps, x, g);
     // packed once here, used by the forward kernel and again by the backward's
-    if (!taps.defined()) taps = prepare_taps(g, hc, stream);
+    if (rectify) hc = rectify_filter(g, hc, taps, stream);
+    else if (!taps.defined()) taps = prepare_taps(g, hc, stream);
     Tensor out = at::empty_like(z);
     if (grad || !fused) f.t1 = at::empty_like(x);
     if (keep) {
@@ -554,7 +565,7 @@ struct UpdateGrads {
 };
 
 UpdateGrads update_backward(const UpdateForward &f, const Tensor &bias, Tensor gout, const UpdateConfig &c, bool need_x,
-                            bool need_z, bool need_h, bool need_b, void *stream)
+                            bool need_z, bool need_h, bool need_b, void *stream, bool rectify = false)
 {
     const Tensor &x = f.x, &z = f.z;
     check_update(x, z, f.h, bias, c);
@@ -572,7 +583,11 @@ UpdateGrads update_backward(const UpdateForward &f, const Tensor &bias, Tensor g
     const size_t bytes = ndc_backward_workspace_bytes(&g, need_x, need_z, need_h, need_b);
     Tensor ws = scratch(bytes ? bytes : 1, x);
     check_taps(f.taps, x, g);
-    if (f.taps.defined())
+    if (rectify)
+        check(ndc_backward_rectified(&g, ptr(x), ptr(z), ptr(t1), ptr(s_over_den), ptr(ratio), fptr(f.h), ptr(f.taps),
+                                     fptr(bias), ptr(gout), out_ptr(r.gx), out_ptr(r.gz), out_fptr(r.gh), out_fptr(r.gb),
+                                     out_ptr(ws), bytes, stream), "ndc_backward_rectified");
+    else if (f.taps.defined())
         check(ndc_backward_taps(&g, ptr(x), ptr(z), ptr(t1), ptr(s_over_den), ptr(ratio), fptr(f.h), ptr(f.taps),
                                 fptr(bias), ptr(gout), out_ptr(r.gx), out_ptr(r.gz), out_fptr(r.gh), out_fptr(r.gb),
                                 out_ptr(ws), bytes, stream), "ndc_backward_taps");
@@ -679,7 +694,7 @@ struct Projected : public torch::autograd::Function<Projected> {
         const bool library = x.scalar_type() == at::kFloat && !wide_is_tiled(flat.size(0), w.cin(), w.cout(), flat.size(2));
         Tensor z = project(w, flat, library, stream);
         size[1] = w.cout();
-        Tensor out = update_forward(x, z.view(size), rectify ? at::relu(h.detach()) : h, bias, taps, c, grad, f, stream);
+        Tensor out = update_forward(x, z.view(size), rectify ? h.detach() : h, bias, taps, c, grad, f, stream, rectify);
         f.x_last = channels_last(x_);
         return out;
     }
@@ -709,7 +724,7 @@ struct Projected : public torch::autograd::Function<Projected> {
         n.arg(true), n.arg(true), n.arg(true), n.arg(v[4].defined());
         const auto need = n.ask(ctx);
         UpdateGrads r =
-            update_backward(f, v[4], gouts[0], c, need[0], need[0] || need[1], need[2], need[3], scope.stream);
+            update_backward(f, v[4], gouts[0], c, need[0], need[0] || need[1], need[2], need[3], scope.stream, flags[1] != 0);
         const Tensor x = f.x.flatten(2);
         const Matrix w = saved_weight(v[8], false, f.z.size(1), x);
         TORCH_CHECK_VALUE(w.cin() == x.size(1), "a saved weight came back as ", v[8].sizes());
@@ -719,7 +734,6 @@ struct Projected : public torch::autograd::Function<Projected> {
             gx = project_back(w, r.gz.flatten(2), r.gx.flatten(2), flags[0] ? x : Tensor(), scope.stream).view(f.x.sizes());
             if (f.x_last) gx = to_channels_last(gx, scope.stream);
         }
-        if (flags[1] && r.gh.defined()) r.gh = at::threshold_backward(r.gh, f.h, 0);
         return {gx, gw, r.gh, r.gb, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };

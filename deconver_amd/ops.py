@@ -111,6 +111,19 @@ def prepare_taps(lib: _lib.NdcLibrary, x: Tensor, h: Tensor, *, groups: int, m: 
     return taps
 
 
+def rectify_filter(lib: _lib.NdcLibrary, x: Tensor, h0: Tensor, *, groups: int, m: int, sc: int):
+    """``(max(h0, 0), its table)`` for updates of tensors like ``x``, in one launch; the table is ``None``
+    where the kernels read the filter itself."""
+    g = make_geom_for(x, h0, groups, m, sc, 0.0, True)
+    nbytes = lib.taps_bytes(g)
+    h, taps = torch.empty_like(h0), None
+    if nbytes:
+        buf = torch.empty(nbytes + 256, dtype=torch.uint8, device=x.device)
+        taps = buf[-buf.data_ptr() % 256:][:nbytes]   # 256-byte aligned view
+    lib.rectify_filter(g, _ptr(h0), _ptr(h), _ptr(taps), nbytes, _stream_of(x))
+    return h, taps
+
+
 def update_forward(lib: _lib.NdcLibrary, x: Tensor, z: Tensor, h: Tensor,
                    bias: Optional[Tensor], *, groups: int, m: int, sc: int, eps: float,
                    relu_input: bool, need_t1: bool = True, save_ratio: bool = False,
@@ -149,13 +162,15 @@ def update_backward(lib: _lib.NdcLibrary, x: Tensor, z: Tensor, t1: Tensor, h: T
                     need_h: bool = True, need_b: bool = True,
                     path: int = _lib.PATH_AUTO, pass_times: Optional[list] = None,
                     saved: Optional[Tuple[Tensor, Tensor]] = None,
-                    taps: Optional[Tensor] = None):
+                    taps: Optional[Tensor] = None, rectified: bool = False):
     """Gradients ``(gx, gz, gh, gb)`` of the update; entries not asked for are ``None``.
 
     ``saved``: the ``(s_over_den, ratio)`` pair a ``save_ratio`` forward call returned for the
     same inputs.
 
     ``taps``: the table :func:`prepare_taps` made for this ``h`` (skips packing it again).
+
+    ``rectified``: ``gh`` is the gradient of the filter before its rectifier, zero where ``h`` is.
 
     ``pass_times``: a list that, if given, receives the device milliseconds of the three
     backward stages (the call then synchronises)."""
@@ -182,7 +197,9 @@ def update_backward(lib: _lib.NdcLibrary, x: Tensor, z: Tensor, t1: Tensor, h: T
     args = (g, _ptr(x), _ptr(z), _ptr(t1), _ptr(s_over_den), _ptr(ratio), _ptr(h), _ptr(bias),
             _ptr(gout), _ptr(gx),
             _ptr(gz), _ptr(gh), _ptr(gb), ws_ptr, nbytes, _stream_of(x))
-    if taps is not None and pass_times is None:
+    if rectified:
+        lib.backward_rectified(*args[:7], _ptr(taps), *args[7:])
+    elif taps is not None and pass_times is None:
         lib.backward_taps(*args[:7], _ptr(taps), *args[7:])
     elif pass_times is None:
         lib.backward(*args)

@@ -187,6 +187,22 @@ int ndc_backward_taps(const ndc_geom *g, const void *x, const void *z, const voi
                       const float *bias, const void *gout, void *gx, void *gz, float *gh, float *gb,
                       void *workspace, size_t workspace_bytes, void *stream);
 
+/*
+ * A filter that still has its rectifier before it (deconv.py:157-165 of the reference calls relu on
+ * the parameter and differentiates it):
+ *   ndc_rectify_filter      h = max(h0, 0), and its table where `taps` is not null and `g` has one
+ *                           (as ndc_prepare_taps makes of h), in one launch
+ *   ndc_backward_rectified  ndc_backward_taps with gh the gradient of h0: zero where h <= 0.
+ *                           `taps` may be null (then packed here where one is needed)
+ */
+int ndc_rectify_filter(const ndc_geom *g, const float *h0, float *h, void *taps, size_t taps_bytes,
+                       void *stream);
+int ndc_backward_rectified(const ndc_geom *g, const void *x, const void *z, const void *t1,
+                           const void *s_over_den, const void *ratio, const float *h,
+                           const void *taps, const float *bias, const void *gout, void *gx,
+                           void *gz, float *gh, float *gb, void *workspace,
+                           size_t workspace_bytes, void *stream);
+
 /* Bytes of scratch `ndc_backward` needs for `g` with the requested outputs (each flag
  * nonzero when the matching output pointer will be non-null). */
 size_t ndc_backward_workspace_bytes(const ndc_geom *g, int need_gx, int need_gz, int need_gh,

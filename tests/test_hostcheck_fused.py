@@ -399,3 +399,38 @@ def test_prepared_taps_give_the_same_results(dtype, matrix, matrix_switch):
     for a, b in zip(g0, g1):
         assert torch.equal(a, b)
     assert host_faults(lib)[0] == 0
+
+
+@pytest.mark.parametrize("G,m,sc,ks,sp,dtype", [
+    (3, 1, 4, (3, 3, 3), (5, 9, 8), torch.bfloat16),    # packed table
+    (3, 1, 4, (3, 3, 3), (5, 9, 8), torch.float32),     # march
+    (2, 1, 4, (5, 5), (9, 12), torch.float32),          # one-shot tiles
+    (2, 2, 3, (3, 3, 3), (4, 5, 6), torch.float32),     # direct kernels
+])
+def test_filter_rectified_and_its_gradient(G, m, sc, ks, sp, dtype):
+    """ndc_rectify_filter and ndc_backward_rectified against a rectifier before the plain calls and its
+    gradient's mask behind them: bit-equal, the table included; a NaN stays one."""
+    lib = hostcheck_library()
+    x, z, h0, bias, gout = make_case(G * m, G, sc, ks, sp, B=2, dtype=dtype, bias_shift=0.3)
+    h0 = h0 - 0.6 * h0.max()
+    assert 0 < int((h0 <= 0).sum()) < h0.numel()
+    kw = dict(groups=G, m=m, sc=sc)
+    want, (h, taps) = torch.relu(h0), ops.rectify_filter(lib, x, h0, **kw)
+    table = ops.prepare_taps(lib, x, want, **kw)
+    assert torch.equal(h, want) and (taps is None) == (table is None) == (dtype == torch.float32)
+    assert taps is None or torch.equal(taps[:G * 1272], table[:G * 1272])
+    kw.update(eps=1e-2, relu_input=True)    # (windows without a positive tap stay finite)
+    saved = {}
+    if m == 1:
+        _, t1, saved["saved"] = ops.update_forward(lib, x, z, h, bias, save_ratio=True, **kw)
+    else:
+        _, t1 = ops.update_forward(lib, x, z, h, bias, **kw)
+    plain = ops.update_backward(lib, x, z, t1, h, bias, gout, **saved, **kw)
+    for table in {None, taps} if taps is None else (None, taps):
+        got = ops.update_backward(lib, x, z, t1, h, bias, gout, taps=table, rectified=True, **saved, **kw)
+        assert torch.equal(got[2], plain[2].masked_fill(h <= 0, 0.0))
+        for a, b in zip(got[:2] + got[3:], plain[:2] + plain[3:]):
+            assert torch.equal(a, b)
+    h0.view(-1)[5] = float("nan")
+    assert torch.equal(ops.rectify_filter(lib, x, h0, groups=G, m=m, sc=sc)[0].isnan(), h0.isnan())
+    assert host_faults(lib)[0] == 0
