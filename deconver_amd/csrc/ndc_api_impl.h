@@ -8,7 +8,7 @@
 #include "../../include/deconver_ndc.h"
 #include "ndc_common.h"
 #include "ndc_columns.h"
-#include "ndc_direct.h"
+#include "ndc_direct_tile.h"
 #include "ndc_fused_api.h"
 #include "ndc_mlp_host.h"
 
@@ -81,10 +81,10 @@ static int direct_gconv(const KGeom &q, const TI *in, const float *h, const floa
         const long long units = (long long)q.B * q.G * blocks;
         if (adjoint) {
             const direct::GConv<TI, TO, true, F::nb, F::kwb, typename F::off> op = {q, in, h, bias, rectify, out, blocks};
-            return Backend::weighted_unit(units, q.SP, stream, op);
+            return direct::launch<Backend>(op, units, stream);
         }
         const direct::GConv<TI, TO, false, F::nb, F::kwb, typename F::off> op = {q, in, h, bias, rectify, out, blocks};
-        return Backend::weighted_unit(units, q.SP, stream, op);
+        return direct::launch<Backend>(op, units, stream);
     });
 }
 
@@ -99,7 +99,7 @@ static int direct_ratio(const KGeom &q, const T *x, const T *t1, const T *z, con
         const int blocks = (q.sc + F::nb - 1) / F::nb;
         const direct::Ratio<T, STAGE, F::nb, F::kwb, typename F::off> op = {
             q, x, t1, z, gout, gt1, h, bias, out, s_over_den, ratio, gn, gd, blocks};
-        return Backend::weighted_unit((long long)q.B * q.G * blocks, q.SP, stream, op);
+        return direct::launch<Backend>(op, (long long)q.B * q.G * blocks, stream);
     });
 }
 
@@ -153,7 +153,7 @@ static int direct_backward(const KGeom &q, const T *x, const T *z, const T *t1, 
             typedef decltype(form) F;
             const int blocks = (q.m + F::nb - 1) / F::nb;
             const direct::GradPair<T, F::nb, F::kwb, typename F::off> op = {q, gn, gd, h, gx, gt1, blocks};
-            return Backend::weighted_unit((long long)q.B * q.G * blocks, q.SP, stream, op);
+            return direct::launch<Backend>(op, (long long)q.B * q.G * blocks, stream);
         });
     }
     if (st) return st;

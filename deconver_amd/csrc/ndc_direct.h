@@ -21,7 +21,9 @@
 // latency; the volumes they serve fit the L2.
 // Measured (4 groups of 4 filter and 8 source channels, 3x3x3, 2 x 24^3, float32): t1 94 -> 35 us,
 // the forward's ratio 89 -> 25, gn and gd 65 -> 26, gx and gt1 145 -> 26, gh 419 -> 41, gz 151 -> 36,
-// gb 41 -> 5; the layer, forward + backward, 1036 -> 236 us.
+// gb 41 -> 5; the layer, forward + backward, 1036 -> 236 us.  Filters of 3 x 3 and 5 x 5 taps take their
+// convolutions from boxes in LDS since (ndc_direct_tile.h); 1-D ones, those of unequal extents, of 7 taps
+// and volumes from 2^30 positions on are done here.
 #pragma once
 
 #include "../../include/deconver_ndc.h"
@@ -212,6 +214,21 @@ template <typename TI, typename TO, bool ADJ, int NB, int KWB, typename OFF> str
     TO *out;
     int blocks;
     typedef direct::Weights<ADJ, NB, KWB> Weights;
+    static constexpr bool kAdj = ADJ;
+    static constexpr int kNin = 1, kNB = NB, kKWB = KWB;
+    NDC_HD float value(int, const Unit &t, int ci, OFF off) const
+    {
+        const int cin = ADJ ? q.m : q.sc;
+        const float v = load_at<TI, OFF>(in + (((long long)t.b * q.G + t.g) * cin + ci) * q.SP, off);
+        return rectify ? source_of(v, bias ? bias[t.g * cin + ci] : 0.f, q.relu) : v;
+    }
+    NDC_HD void finish(const Unit &t, long long pos, const float (&acc)[1][NB]) const
+    {
+        const int cout = ADJ ? q.sc : q.m;
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+            if (t.c0 + c < cout) Elem<TO>::store(out + (((long long)t.b * q.G + t.g) * cout + t.c0 + c) * q.SP + pos, acc[0][c]);
+    }
     NDC_HD int weights() const { return Weights::count(q); }
     NDC_HD void stage(int u, float *to, int first, int step) const
     {
@@ -221,7 +238,7 @@ template <typename TI, typename TO, bool ADJ, int NB, int KWB, typename OFF> str
     template <bool STAGED> NDC_HD void run(int u, long long pos, const float *staged) const
     {
         const Unit t(u, q.G, blocks, NB);
-        const int cin = ADJ ? q.m : q.sc, cout = ADJ ? q.sc : q.m;
+        const int cin = ADJ ? q.m : q.sc;
         const Pos<OFF> p = position<OFF>(q, (OFF)pos);
         const long long bg = (long long)t.b * q.G + t.g;
         const TI *ig = in + bg * cin * q.SP;
@@ -234,9 +251,7 @@ template <typename TI, typename TO, bool ADJ, int NB, int KWB, typename OFF> str
 #pragma unroll
             for (int j = 0; j < KWB; ++j) v[j] = win.in[j] ? source_of(v[j], bv, q.relu) : 0.f;
         });
-#pragma unroll
-        for (int c = 0; c < NB; ++c)
-            if (t.c0 + c < cout) Elem<TO>::store(out + (bg * cout + t.c0 + c) * q.SP + pos, acc[0][c]);
+        finish(t, pos, acc);
     }
 };
 
@@ -248,6 +263,22 @@ template <typename T, int NB, int KWB, typename OFF> struct GradPair {
     float *gt1;
     int blocks;
     typedef direct::Weights<false, NB, KWB> Weights;
+    static constexpr bool kAdj = false;
+    static constexpr int kNin = 2, kNB = NB, kKWB = KWB;
+    NDC_HD float value(int k, const Unit &t, int ci, OFF off) const
+    {
+        return load_at<float, OFF>((k ? gd : gn) + (((long long)t.b * q.G + t.g) * q.sc + ci) * q.SP, off);
+    }
+    NDC_HD void finish(const Unit &t, long long pos, const float (&acc)[2][NB]) const
+    {
+#pragma unroll
+        for (int c = 0; c < NB; ++c)
+            if (t.c0 + c < q.m) {
+                const long long at = (((long long)t.b * q.G + t.g) * q.m + t.c0 + c) * q.SP + pos;
+                Elem<T>::store(gx + at, acc[0][c]);
+                gt1[at] = acc[1][c];
+            }
+    }
     NDC_HD int weights() const { return Weights::count(q); }
     NDC_HD void stage(int u, float *to, int first, int step) const
     {
@@ -264,13 +295,7 @@ template <typename T, int NB, int KWB, typename OFF> struct GradPair {
                                                    [&](int k, int ci, const Window<1, KWB, OFF> &win, float (&v)[KWB]) {
             win.template load<float>((k ? gd : gn) + base + ci * q.SP, v);
         });
-#pragma unroll
-        for (int c = 0; c < NB; ++c)
-            if (t.c0 + c < q.m) {
-                const long long at = (bg * q.m + t.c0 + c) * q.SP + pos;
-                Elem<T>::store(gx + at, acc[0][c]);
-                gt1[at] = acc[1][c];
-            }
+        finish(t, pos, acc);
     }
 };
 
@@ -289,6 +314,13 @@ template <typename T, int STAGE, int NB, int KWB, typename OFF> struct Ratio {
     float *gn, *gd;                 // GRAD
     int blocks;
     typedef direct::Weights<true, NB, KWB> Weights;
+    static constexpr bool kAdj = true;
+    static constexpr int kNin = STAGE == SOURCE ? 3 : 2, kNB = NB, kKWB = KWB;
+    NDC_HD float value(int k, const Unit &t, int ci, OFF off) const
+    {
+        const long long at = (((long long)t.b * q.G + t.g) * q.m + ci) * q.SP;
+        return k == 2 ? load_at<float, OFF>(gt1 + at, off) : load_at<T, OFF>((k ? t1 : x) + at, off);
+    }
     NDC_HD int weights() const { return Weights::count(q); }
     NDC_HD void stage(int u, float *to, int first, int step) const
     {
@@ -300,14 +332,18 @@ template <typename T, int STAGE, int NB, int KWB, typename OFF> struct Ratio {
         const Unit t(u, q.G, blocks, NB);
         const Pos<OFF> p = position<OFF>(q, (OFF)pos);
         const long long bg = (long long)t.b * q.G + t.g, base = bg * q.m * q.SP;
-        constexpr int NIN = STAGE == SOURCE ? 3 : 2;
-        float acc[NIN][NB];
-        accumulate<true, NB, KWB, NIN, STAGED, OFF>(q, hf, staged, t.g, t.c0, p, acc,
+        float acc[kNin][NB];
+        accumulate<true, NB, KWB, kNin, STAGED, OFF>(q, hf, staged, t.g, t.c0, p, acc,
                                                     [&](int k, int ci, const Window<-1, KWB, OFF> &win, float (&v)[KWB]) {
             const long long at = base + ci * q.SP;
             if (k == 2) win.template load<float>(gt1 + at, v);
             else win.template load<T>((k ? t1 : x) + at, v);
         });
+        finish(t, pos, acc);
+    }
+    NDC_HD void finish(const Unit &t, long long pos, const float (&acc)[kNin][NB]) const
+    {
+        const long long bg = (long long)t.b * q.G + t.g;
 #pragma unroll
         for (int c = 0; c < NB; ++c) {
             const int i = t.c0 + c;
@@ -325,7 +361,7 @@ template <typename T, int STAGE, int NB, int KWB, typename OFF> struct Ratio {
                 gn[idx] = a;
                 gd[idx] = -(a * n) * inv;
             } else {
-                float r = Elem<T>::load(gout + idx) * n / d + acc[2][c];
+                float r = Elem<T>::load(gout + idx) * n / d + acc[kNin - 1][c];
                 if (q.relu && zv + bv <= 0.f) r = 0.f;   // a NaN passes, as through torch.relu's backward
                 Elem<T>::store(out + idx, r);
             }

@@ -1,0 +1,276 @@
+// The direct kernels' convolutions from boxes in LDS: filters of 3 x 3 or 5 x 5 taps in the last two axes (any number
+// in the first), the functors of ndc_direct.h.
+//
+// A workgroup makes a box of positions for one unit (sample, group, block of output channels), a thread one position or
+// two of neighbouring rows.  It stages the box with its halo, zeros outside the volume, for as many input channels as
+// its LDS share takes, and those channels' weights in the order they are used; then every thread runs over channels and
+// taps without a bounds check, an address or a load from memory, both factors of a product in vector registers (3.3
+// clocks a multiply-add, 4.4 with one in a scalar register).  Two rows a thread share the weights of a row and the
+// window rows between them.  Without boxes a thread waits for the loads of every tap row, some twenty round trips to the
+// L2 in a row, which is what small launches spent their time on; here it is one round trip per group of channels.
+// What bounds them now: the multiply-adds of large launches; in small ones the launch, that round trip, the products of
+// the one or two wavefronts a SIMD has and the epilogue follow each other.
+// us, one position at a time (ndc_direct.h) -> boxes, float32: 4 groups of 4 and 8 channels on 2 x 24^3, t1 30 -> 22,
+// the forward's ratio 26 -> 17, gn and gd 26 -> 17, gx and gt1 25 -> 23, gz 36 -> 23; forward and backward in all
+// 194 -> 154 (the layer's call 206 -> 166), 2 groups with 5^3 taps on 12 x 13 x 15 438 -> 247, 16 channels 1 -> 2 on 2 x 24^3 122 -> 94, 64 channels
+// 1 -> 2 with 5 x 5 taps on 4 x 128^2 618 -> 452, 16 groups of 4 and 8 on 2 x 48 x 50 x 46 2838 -> 2538; behind in none of
+// 19 layers measured (0.56 to 0.93 of the time).
+#pragma once
+
+#include "ndc_direct.h"
+#include "ndc_exec.h"
+
+#include <cstring>
+
+namespace ndc {
+namespace direct {
+
+struct Box {
+    int NR;                  // rows of positions a thread makes, 1 or 2
+    int TD, TH, TW, HP;      // positions of a workgroup, and how many threads share their rows of a plane
+    int SD, SH, SW, SV;      // staged extents and their product
+    int nd, nh, nw, tiles;   // boxes per axis and volume
+    int chunk;               // input channels staged at once
+    int NT;                  // threads of a workgroup
+    uint32_t over_sw, over_sh;   // 2^32 / SW and 2^32 / SH, rounded up (see quotient)
+};
+
+// v / d from o = 2^32 / d rounded up: exact while v * d < 2^32 (d > 1), and staged extents are below 2^16
+static NDC_HD int quotient(int v, uint32_t o) { return (int)(((uint64_t)(uint32_t)v * o) >> 32); }
+
+static NDC_HD int box_weights(const KGeom &q, int nb) { return q.KT * nb; }
+// words of LDS: the staged channels of the inputs, the weights from a multiple of four words on
+static NDC_HD int box_values(const Box &t, int nin) { return (nin * t.chunk * t.SV + 3) / 4 * 4; }
+
+template <class F, int K, int NR> struct Tiled {
+    static constexpr int NIN = F::kNin, NB = F::kNB, ROW = NB * K;
+    static_assert(F::kKWB == K, "a tap row at a time");
+    struct Params {
+        F f;
+        Box t;
+    };
+    struct State {
+        float acc[NR][NIN][NB];
+        int at, pos, live, live1;
+    };
+    static int lds_floats(const KGeom &q, const Box &t) { return box_values(t, NIN) + t.chunk * box_weights(q, NB); }
+
+    template <class Exec> static NDC_D void run(Exec &ex, const Params &p, int block)
+    {
+        const F &f = p.f;
+        const Box t = p.t;
+        const KGeom &q = f.q;
+        const int u = block / t.tiles, tile = block - u * t.tiles;
+        const int iw = tile % t.nw, r0 = tile / t.nw, d0 = r0 / t.nh * t.TD, h0 = r0 % t.nh * t.TH, w0 = iw * t.TW;
+        const Unit un(u, q.G, f.blocks, NB);
+        const int cin = F::kAdj ? q.m : q.sc, cout = F::kAdj ? q.sc : q.m, rows = q.kD * K, wbase = box_values(t, NIN);
+        const float *hg = f.hf + (long long)un.g * q.m * q.sc * q.KT;
+
+        ex.each([&](State &st, int tid) NDC_LAMBDA {
+            const int w = tid % t.TW, r = tid / t.TW, h = r % t.HP * NR, d = r / t.HP;
+            st.live = d < t.TD && d0 + d < q.D && h0 + h < q.H && w0 + w < q.W;
+            st.live1 = st.live && h + 1 < t.TH && h0 + h + 1 < q.H;
+            st.at = (d * t.SH + h) * t.SW + w;
+            st.pos = ((d0 + d) * q.H + h0 + h) * q.W + w0 + w;
+#pragma unroll
+            for (int n = 0; n < NR; ++n)
+#pragma unroll
+                for (int k = 0; k < NIN; ++k)
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) st.acc[n][k][c] = 0.f;
+        });
+        for (int c0 = 0; c0 < cin; c0 += t.chunk) {
+            const int nc = cin - c0 < t.chunk ? cin - c0 : t.chunk;
+            if (c0) ex.sync();
+            ex.each([&](State &, int tid) NDC_LAMBDA {
+                for (int e = tid; e < t.SV; e += t.NT) {
+                    const int r = quotient(e, t.over_sw), d = quotient(r, t.over_sh);
+                    const int dd = d0 + d - q.pD, hh = h0 + r - d * t.SH - q.pH, ww = w0 + e - r * t.SW - q.pW;
+                    const bool in = (unsigned)dd < (unsigned)q.D && (unsigned)hh < (unsigned)q.H && (unsigned)ww < (unsigned)q.W;
+                    const uint32_t off = in ? ((uint32_t)dd * q.H + hh) * q.W + ww : 0u;
+#pragma unroll 4
+                    for (int ci = 0; ci < nc; ++ci)
+#pragma unroll
+                        for (int k = 0; k < NIN; ++k) {
+                            const float v = f.value(k, un, c0 + ci, off);
+                            ex.st_((k * t.chunk + ci) * t.SV + e, in ? v : 0.f);
+                        }
+                }
+                // weights: [input channel][tap row][output channel][K]; channels past the last repeat the last
+                for (int e = tid; e < nc * rows; e += t.NT) {
+                    float w[ROW];
+                    load_weights(q, hg, un, cout, rows, c0, e, w);
+#pragma unroll
+                    for (int i = 0; i < ROW; ++i) ex.st_(wbase + e * ROW + i, w[i]);
+                }
+            });
+            ex.sync();
+            ex.each([&](State &st, int) NDC_LAMBDA {
+                if (!st.live) return;
+                for (int ci = 0; ci < nc; ++ci)
+                    for (int td = 0; td < q.kD; ++td) {
+                        // (A takes the taps from the far end of the window)
+                        const int sd = F::kAdj ? q.kD - 1 - td : td;
+                        const int wrow = wbase + (ci * q.kD + td) * K * ROW;
+                        float w[NR][ROW];   // row s of the window meets tap rows s, s - 1 of the positions' NR rows
+#pragma unroll
+                        for (int s = 0; s < K + NR - 1; ++s) {
+                            float v[NIN][K];
+                            if (s < K) row_words(ex, wrow + (F::kAdj ? K - 1 - s : s) * ROW, w[s % NR]);
+#pragma unroll
+                            for (int k = 0; k < NIN; ++k) {
+                                const int from = st.at + ((k * t.chunk + ci) * t.SV + (sd * t.SH + s) * t.SW);
+#pragma unroll
+                                for (int j = 0; j < K; ++j) v[k][F::kAdj ? K - 1 - j : j] = ex.ld(from + j);
+                            }
+#pragma unroll
+                            for (int n = 0; n < NR; ++n) {
+                                if (s - n < 0 || s - n >= K) continue;
+#pragma unroll
+                                for (int c = 0; c < NB; ++c)
+#pragma unroll
+                                    for (int j = 0; j < K; ++j)
+#pragma unroll
+                                        for (int k = 0; k < NIN; ++k) st.acc[n][k][c] += v[k][j] * w[(s - n) % NR][c * K + j];
+                            }
+                        }
+                    }
+            });
+        }
+        ex.each([&](State &st, int) NDC_LAMBDA {
+            if (st.live) f.finish(un, st.pos, st.acc[0]);
+            if (NR > 1 && st.live1) f.finish(un, st.pos + q.W, st.acc[NR - 1]);
+        });
+    }
+
+    static NDC_HD void load_weights(const KGeom &q, const float *hg, const Unit &un, int cout, int rows, int c0, int e, float (&w)[ROW])
+    {
+        const int ci = e / rows, row = e - ci * rows;
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+            const int k = un.c0 + c < cout ? un.c0 + c : cout - 1;
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                w[c * K + j] = hg[((F::kAdj ? c0 + ci : k) * q.sc + (F::kAdj ? k : c0 + ci)) * q.KT + row * K + j];
+        }
+    }
+
+    // a row of weights (from a multiple of four words where it is that long)
+    template <class Exec> static NDC_D void row_words(Exec &ex, int at, float (&w)[ROW])
+    {
+        if constexpr (ROW % 4 == 0) {
+#pragma unroll
+            for (int i = 0; i < ROW; i += 4) {
+                uint32_t v[4];
+                ex.ld4a(at + i, v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) w[i + j] = bits_to_float(v[j]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < ROW; ++i) w[i] = ex.ld(at + i);
+        }
+    }
+};
+
+// The box of a launch: the least cost over one or two rows a thread and the boxes that cut an axis into equal parts.
+// The cost is what the busiest CU has to do: products and LDS reads of its SIMDs (dearer where a SIMD has fewer than two
+// wavefronts), the values and 128-byte lines staged, the lines its outputs touch, and a fixed part for every round of
+// workgroups the CU holds at once times the groups of channels.  Its constants were fitted to 70 boxes each of five
+// kernels on seven layers, on which the box it takes is 5 % behind the best one (a box for the most threads alone: 16 %).
+static inline bool choose_box(const KGeom &q, int nin, int nb, int cin, long long units, Box &best)
+{
+    const int K = q.kW, weights = box_weights(q, nb), budget = 10 * 1024, kMaxLds = 160 * 1024;
+    double least = 0;
+    best.NT = 0;
+    for (int nr = 1; nr <= 2; ++nr)
+        for (int pw = 1; pw <= 6 && pw <= q.W; ++pw)
+            for (int ph = 1; ph <= 16 && ph <= q.H; ++ph) {
+                int before = 0;
+                for (int pd = 1; pd <= 32 && pd <= q.D; ++pd) {
+                    Box t;
+                    t.NR = nr;
+                    t.TW = (q.W + pw - 1) / pw, t.TH = (q.H + ph - 1) / ph, t.TD = (q.D + pd - 1) / pd;
+                    if (t.TD == before) continue;
+                    before = t.TD;
+                    t.HP = (t.TH + nr - 1) / nr;
+                    const long long n = (long long)t.TW * t.HP * t.TD;
+                    if (n > 512) continue;
+                    t.NT = (int)((n + 63) / 64 * 64);
+                    t.SD = t.TD + q.kD - 1, t.SH = t.HP * nr + K - 1, t.SW = t.TW + K - 1, t.SV = t.SD * t.SH * t.SW;
+                    t.over_sw = 0xffffffffu / t.SW + 1, t.over_sh = 0xffffffffu / t.SH + 1;
+                    t.chunk = budget / (nin * t.SV + weights);
+                    if (t.chunk < 1) continue;
+                    if (t.chunk > cin) t.chunk = cin;
+                    t.nd = (q.D + t.TD - 1) / t.TD, t.nh = (q.H + t.TH - 1) / t.TH, t.nw = (q.W + t.TW - 1) / t.TW;
+                    t.tiles = t.nd * t.nh * t.nw;
+                    const long long group = (units * t.tiles + 255) / 256;   // workgroups of the busiest CU
+                    const int w = t.NT / 64, lds = 4 * t.chunk * (nin * t.SV + weights);
+                    // wavefronts a SIMD has the registers for, workgroups a CU has the place for
+                    int simd = 512 / (46 + nr * nb * (nin + K) + 2 * nin * K);
+                    simd = simd < 1 ? 1 : simd > 8 ? 8 : simd;
+                    int held = kMaxLds / lds;
+                    if (held * w > 4 * simd) held = 4 * simd / w;
+                    if (held > group) held = (int)group;
+                    if (held < 1) held = 1;
+                    const double per_simd = held * w / 4.0, product = per_simd >= 2 ? 1.1 : 1.1 * (1 + 0.37 * (2 - (per_simd < 1 ? 1 : per_simd)));
+                    const double row = product * nr * nb * K * nin + 0.8 * nb * K + 0.75 * nin * (K + nr - 1);
+                    const double staging = (double)group * cin * nin * (t.SV / 64.0 * 8 + 8.4 * t.SD * t.SH * (t.SW / 32.0 + 1));
+                    const double cost = (double)((group * w + 3) / 4) * cin * (q.KT / K) * row + (held == 1 ? 1.0 : 0.66) * staging +
+                                        group * 40.0 * nb * t.TD * t.TH * (t.TW / 32.0 + 1) +
+                                        (double)((group + held - 1) / held) * ((cin + t.chunk - 1) / t.chunk) * 40e3;
+                    if (!best.NT || cost < least) best = t, least = cost;
+                    if (n < 64) break;
+                }
+            }
+    return best.NT > 0;
+}
+
+// ... of the last sizes a thread saw
+static inline bool box_of(const KGeom &q, int nin, int nb, int cin, long long units, Box &box)
+{
+    if ((q.kW != 3 && q.kW != 5) || q.kH != q.kW || !small_volume(q) || tap_block(q) != q.kW) return false;
+    struct Entry {
+        long long units;
+        int key[8];
+        bool ok;
+        Box box;
+    };
+    static thread_local Entry kept[32];
+    static thread_local int next = 0;
+    const int key[8] = {q.D, q.H, q.W, q.kD, q.kW, nin, nb, cin};
+    for (const Entry &e : kept)
+        if (e.units == units && !memcmp(e.key, key, sizeof key)) {
+            box = e.box;
+            return e.ok;
+        }
+    Entry &e = kept[next];
+    next = (next + 1) % 32;
+    e.ok = choose_box(q, nin, nb, cin, units, e.box);
+    e.units = units;
+    memcpy(e.key, key, sizeof key);
+    box = e.box;
+    return e.ok;
+}
+
+template <class BE, class F, int K, int NR> static int launch_boxes(const F &f, const Box &t, long long units, void *stream)
+{
+    typedef Tiled<F, K, NR> Kernel;
+    const typename Kernel::Params p = {f, t};
+    return BE::template block_kernel<Kernel>(p, (int)(units * t.tiles), t.NT, Kernel::lds_floats(f.q, t), stream);
+}
+
+// a functor over all its units and positions: from tiles where its filter is of that form
+template <class BE, class F> static int launch(const F &f, long long units, void *stream)
+{
+    if constexpr (F::kKWB == 3 || F::kKWB == 5) {
+        constexpr int K = F::kKWB;
+        Box t;
+        if (box_of(f.q, F::kNin, F::kNB, F::kAdj ? f.q.m : f.q.sc, units, t) && units * t.tiles < (1LL << 31))
+            return t.NR == 2 ? launch_boxes<BE, F, K, 2>(f, t, units, stream) : launch_boxes<BE, F, K, 1>(f, t, units, stream);
+    }
+    return BE::weighted_unit(units, f.q.SP, stream, f);
+}
+
+}  // namespace direct
+}  // namespace ndc
