@@ -910,12 +910,14 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
 
 // How ndc_gemm cuts its work: blocks of 32 output rows that a workgroup makes of a 128-voxel tile, or
 // one of the small-grid forms, which slice the channels over the wavefronts (waves <= 0), in tiles of 32
-// rows x 64 voxels or (-1) of 16 rows x 32 voxels: the smaller ones while they are at most two per CU (us, float32 /
-// bf16, 512 -> 128 channels over 1000 voxels, 64 of the larger tiles, 5.7 against 9.4 / 4.8 against 5.6; over 2288,
-// 144 of them, 11.3 against 9.9 / 7.2 against 5.7; 1024 -> 256 over 8 x 256, 256 of them, 25 against 18 / 14.3 against 8.9).
+// rows x 64 voxels or (-1) of 16 rows x 32 voxels: in float32 the smaller ones while they are at most two per CU (us,
+// 512 -> 128 channels over 1000 voxels, 64 of the larger tiles, 5.7 against 9.4; over 2288, 144 of them, 11.3 against
+// 9.9; 1024 -> 256 over 8 x 256, 256 of them, 25 against 18).
 // bf16 is sliced up to four workgroups per CU (128 -> 512 channels over 4096 voxels 8.1 us against 10.2 tiled,
-// over 32 768, 4096 workgroups, 24 against 11.5).  Otherwise as many output rows per workgroup (32 per wavefront) as
-// still leave two workgroups per CU.
+// over 32 768, 4096 workgroups, 24 against 11.5), in the smaller tiles up to four of those per CU (512 -> 128 over 1000
+// 4.8 against 5.6; past two they are behind, 7.2 against 5.7 over 2288, but the two forms add the channels in another
+// order, and results that are rounded to bf16 keep their bits where the line is).  Otherwise as many output rows per
+// workgroup (32 per wavefront) as still leave two workgroups per CU.
 // float32 is sliced up to 600 workgroups (us, sliced / tiled: 512 -> 2048 over 572, 576 of them, 22.1 / 23.1, 512 -> 512
 // over 8 x 256, 512, 17.1 / 17.9; 1024 -> 256 over 2 x 3375, 848, 55 / 43; 256 -> 256 over 8 x 1024, 1024, 19 / 13.7).
 // Otherwise 64 rows a workgroup from 400 of those on (256 -> 256 over 13 824, 432 of them, 19 against 21 with 32 rows;
@@ -923,7 +925,7 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
 static int gemm_waves(long long batch, long long cin, long long cout, long long n, int esz)
 {
     const long long vt = batch * ((n + 127) / 128), small = batch * ((n + 63) / 64) * ((cout + 31) / 32);
-    if (small <= (esz == 4 ? 600 : 1024) && cin % (16 / esz) == 0 && n >= 2) return small <= 128 ? -1 : 0;
+    if (small <= (esz == 4 ? 600 : 1024) && cin % (16 / esz) == 0 && n >= 2) return small <= (esz == 4 ? 128 : 256) ? -1 : 0;
     if (esz == 4) return cout > 32 && vt * ((cout + 63) / 64) >= 400 ? 2 : 1;
     int waves = 4;
     while (waves > 1 && (cout <= 32 * (waves / 2) || vt * ((cout + 32 * waves - 1) / (32 * waves)) < 512)) waves /= 2;

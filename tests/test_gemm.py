@@ -105,6 +105,18 @@ def test_weight_gradient_over_long_rows(rows, cols):
     assert _rel(gw, g[0].double() @ x[0].double().t()) < 1e-5 and _rel(gb, g.double().sum((0, 2))) < 1e-5
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("cin,cout,n", [(64, 256, 1280), (128, 512, 1000), (320, 64, 5000)])
+def test_small_grids_keep_one_order_of_sums(cin, cout, n):
+    """bf16 grids of 129 to 256 tiles of 32 x 64 add their channels in the order of smaller ones: bit-equal columns.
+    (Channels of very different sizes, so that another order rounds otherwise.)"""
+    assert 128 < -(-n // 64) * -(-cout // 32) <= 256
+    lib, (x, _, _, _), w, _ = _setup("cuda", (1, cin, cout, n), torch.bfloat16)
+    x *= torch.logspace(-3, 3, cin, device="cuda").roll(cin // 2)[:, None]
+    half = n // 256 * 128
+    assert torch.equal(ops.gemm(lib, x, w)[0][..., :half], ops.gemm(lib, x[..., :half].contiguous(), w)[0])
+
+
 # rows of 32 and 64 a workgroup, one chain of sums and several; ragged channels, rows and voxels
 PARTS = [(1, 33, 40, 38501), (2, 100, 130, 9001), (1, 32, 64, 52001), (2, 72, 30, 20003), (1, 1030, 96, 13000)]
 
