@@ -150,6 +150,34 @@ def test_parts_of_small_and_large_values(scale):
     assert _rel(gw, torch.matmul(g.double(), x.double().transpose(1, 2)).sum(0)) < 1e-6
 
 
+def _each_within(y, a, b):
+    """Every sum within what a chain of float32 sums may be off (and the least normal number), that of nothing but zeros
+    zero."""
+    want, size = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    off = (y.double() - want).abs() - size * (b.size(-2) + 8) * 2.0 ** -24
+    assert bool((off <= 2.0 ** -126).all()) and bool((y[size == 0] == 0).all())
+
+
+# exponents of x's even and odd voxels, of w's rows 1 and 2, and of w (or g in its place)
+@pytest.mark.gpu
+@pytest.mark.parametrize("voxels,rows,weight", [((0, -118), 0, 0), ((-118, -118), 0, 40), ((-140, -140), 0, 70), ((0, 0), -115, 0),
+                                                ((0, -60), -45, 0), ((90, 90), -118, 0), ((0, -500), -500, 0)])
+def test_parts_of_values_of_very_different_sizes(voxels, rows, weight):
+    """Small values beside others, and against large ones: bf16 parts of them are denormal, or their products' are."""
+    print("case", voxels, rows, weight, flush=True)
+    lib, (x, _, _, g), w, _ = _setup("cuda", (2, 72, 130, 20003), torch.float32)
+    x[..., 0::2] *= 2.0 ** voxels[0]
+    x[..., 1::2] *= 2.0 ** voxels[1]
+    for t in (w, g.transpose(0, 1)):
+        t *= 2.0 ** weight
+        t[1:3] *= 2.0 ** rows
+    x[:, 4] = 0
+    for y in (ops.gemm(lib, x, w)[0], ops.gemm(lib, x, w.t().contiguous(), transposed=True)[0]):
+        _each_within(y, w, x)
+    gw, _ = ops.weight_grad(lib, g, x)
+    _each_within(gw, g.transpose(0, 1).flatten(1), x.transpose(0, 1).flatten(1).t())
+
+
 @pytest.mark.gpu
 def test_parts_of_values_that_are_not_finite():
     """What a float32 product makes of infinities, NaN and values beyond the range of bf16: an infinity's column is
