@@ -69,8 +69,19 @@ template <typename T, bool WT, int MODE> static void tile_gemm_w(TileParams p, i
     const int rows = 32 * waves;   // 32, 64 or 128 output rows per workgroup
     p.tiles_m = (p.cout + rows - 1) / rows;
     p.tiles_n = (int)((p.n + 127) / 128);
-    const dim3 grid(8u * (unsigned)((p.tiles_n * p.batch + 7) / 8) * (unsigned)p.tiles_m);
-    auto launch = [&](auto kernel, int threads) { hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, (hipStream_t)stream, p); };
+    // a launch takes fewer than 2^32 threads: as many samples at a time (2^20 of one voxel into 1024 channels are 2^32)
+    auto launch = [&](auto kernel, unsigned threads) {
+        const long long most = (0xffffffffLL / ((long long)threads * p.tiles_m) - 7) / p.tiles_n, batch = p.batch;
+        TileParams q = p;
+        for (long long b = 0; b < batch; b += q.batch) {
+            q.batch = (int)(batch - b < most ? batch - b : most < 1 ? 1 : most);
+            auto at = [&](auto *t, long long per) { return t ? (decltype(t))((char *)t + b * per * p.n * (long long)sizeof(T)) : t; };
+            q.x = at(p.x, p.cin), q.res = at(p.res, p.cout), q.mask = at(p.mask, p.cout), q.y = at(p.y, p.cout);
+            q.zkeep = at(p.zkeep, p.cout), q.gpart = p.gpart ? p.gpart + b * p.tiles_n * p.cout : nullptr;
+            const dim3 grid(8u * (unsigned)(((long long)p.tiles_n * q.batch + 7) / 8) * (unsigned)p.tiles_m);
+            hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, (hipStream_t)stream, q);
+        }
+    };
     if constexpr (sizeof(T) == 4) {
         // one chain of sums where it is no less exact than the float32 instruction was there (a grid that used to be
         // sliced had chains of eight channels)

@@ -193,6 +193,20 @@ def test_parts_of_values_that_are_not_finite():
         assert _rel(y[ok], want[ok]) < 1e-6
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("transposed", [False, True])
+def test_more_samples_than_a_launch_has_threads_for(transposed):
+    """2^20 samples of a voxel into 1040 channels: 2^32 threads and more, those of the last launch's samples included."""
+    print("case", transposed, flush=True)
+    lib, B, cout = _lib.get_library(), 1 << 20, 1040
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    x, w, bias = (torch.randn(*s, generator=gen, device="cuda") for s in ((B, 1, 1), (cout, 1), (cout,)))
+    y, _ = ops.gemm(lib, x, w.t().contiguous() if transposed else w, bias, None, transposed=transposed)
+    want = torch.addcmul(bias[:, None], w, x)
+    assert float((y - want).abs().max()) < 2e-5        # (products of up to 30)
+    assert bool((y[-16:] != 0).any(dim=(1, 2)).all())
+
+
 def test_refused_arguments():
     lib = hostcheck_library()
     x, w = torch.zeros(1, 8, 4), torch.zeros(6, 8)
