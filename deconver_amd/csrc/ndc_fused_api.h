@@ -28,14 +28,17 @@ namespace fused {
     X(3, 3, 3, 4, 2, 2, 1, 2)        \
     X(3, 3, 3, 4, 2, -2, 2, -2)      \
     X(3, 3, 3, 4, 2, -2, 2, 1)       \
+    X(3, 3, 3, 4, 4, 1, 2, -2)       \
     X(3, 3, 3, 4, 4, 1, 2, 1)        \
     X(3, 3, 3, 4, 2, 1, 1, 1)        \
     X(5, 1, 5, 4, 1, 2, 1, 2)        \
     X(5, 1, 5, 4, 1, -2, 1, -2)      \
+    X(5, 1, 5, 4, 1, -2, 1, 1)       \
     X(5, 1, 5, 4, 1, 1, 1, -2)       \
     X(5, 1, 5, 4, 1, 1, 1, 1)        \
     X(3, 1, 3, 4, 1, 2, 1, 2)        \
     X(3, 1, 3, 4, 1, -2, 1, -2)      \
+    X(3, 1, 3, 4, 1, -2, 1, 1)       \
     X(3, 1, 3, 4, 1, 1, 1, -2)       \
     X(3, 1, 3, 4, 1, 1, 1, 1)
 
@@ -80,9 +83,14 @@ static inline const Tuning &tuning()
 static inline Tuning tuning() { return Tuning{0, 0, 0, 0, 256, 512, 256, 256, 512, 128, 1, 1, 1}; }
 #endif
 
+// where column pairs of rows of any length and alignment are taken (see loose_pairs)
+struct LoosePairs {
+    bool forward, backward;
+};
+
 // first listed row of this filter geometry that the width / alignment allow (and, in a
 // tuning run, that matches the requested register tiles)
-static inline bool find_variant(const KGeom &q, const March &m, int pairs, Variant &v)
+static inline bool find_variant(const KGeom &q, const March &m, int pairs, const LoosePairs &loose, Variant &v)
 {
     if (q.m != 1) return false;
     const Tuning tn = tuning();
@@ -91,17 +99,7 @@ static inline bool find_variant(const KGeom &q, const March &m, int pairs, Varia
     // (measured 16-32 % faster from 16 to 100 columns, 4-15 % slower from 128 on)
     const bool narrow_2d = m.H == 1 && m.W < 128 && !tn.rwf && !tn.rwb;
     const bool even = pairs == kPairs && m.W % 2 == 0 && !narrow_2d;
-    // Loose pairs, where they are ahead of one column a thread (us, float32 / bf16, one column -> pairs).
-    // 3-D: forward 32 channels of 91 x 101 x 87 652 -> 585 / 661 -> 588, of 55 x 61 x 129 557 -> 369 / 556 -> 365, 4 x 128
-    // of 21 x 15 x 23 119 -> 114 / 122 -> 117; backward from 32 columns on (32 of 91 x 101 x 87 1177 -> 1109 / 1117 -> 983,
-    // 64 of 45 x 53 x 77 543 -> 539 / 519 -> 490, 2 x 64 of 33 x 40 x 31 252 -> 256 / 228 -> 241, 512 of 13 x 11 x 9
-    // 72 -> 101).  2-D: backward 8 x 32 of 257 x 255 596 -> 537 / 575 -> 460, 2 x 128 of 301 x 299 1275 -> 996 /
-    // 1342 -> 953; forward up to 256 columns (297 -> 258 / 293 -> 257; 301 x 299 415 -> 431 / 417 -> 443).  3-D rows of more
-    // than 192 leave the backward one workgroup a CU (64 of 30 x 41 x 255 857 -> 1073 / 782 -> 949).
-    // (Rows that one column a thread cannot take stay outside.)
-    const bool plane = m.H == 1;
-    const bool loose_f = pairs >= kLooseForward && !narrow_2d && m.W >= 2 && m.W <= 256;
-    const bool loose_b = pairs >= kLoosePairs && !narrow_2d && m.W >= 32 && m.W <= (plane ? 512 : 192);
+    const bool loose_f = pairs >= kLooseForward && loose.forward, loose_b = pairs >= kLoosePairs && loose.backward;
     auto takes = [&](int rwf, int rwb) {
         return (rwf == 1 || (rwf == 2 ? even : loose_f)) && (rwb == 1 || (rwb == 2 ? even : loose_b));
     };
@@ -271,6 +269,65 @@ static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, cons
     return found;
 }
 
+// Column pairs of rows of any length and alignment, where they are ahead of one column a thread.
+// 3-D: where the cost of their launch says so.  The times of 141 problems (3 to 255 columns, 1 to 1024 channels, 0.1 to 10 M
+// voxels) follow the ratio of the two costs.  Forward, 2 x 2 outputs a thread against 4 x 1: a pair's thread takes 1.02 to
+// 1.09 times as long (a lone wavefront up to 1.03), workgroups of three wavefronts 1.12 times what they are counted as; so
+// pairs below 0.93 (0.965) of the cost.  us, one column -> pairs, float32 / bf16, with that ratio: 192 channels of
+// 23 x 29 x 33 161 -> 99 / 162 -> 99, 0.60; 32 of 55 x 61 x 129 559 -> 371 / 563 -> 364, 0.79; 32 of 91 x 101 x 87 643 -> 585 /
+// 661 -> 582, 0.85; 2 of 104 x 100 x 61 60 -> 55 / 60 -> 56, 0.92; 64 of 45 x 53 x 77 299 -> 300 / 306 -> 319, 0.94; 1024 of
+// 6 x 3 x 7 44 -> 94 / 42 -> 95, 1.00; 16 of 106 x 82 x 73 245 -> 255 / 245 -> 274, 1.06.  Taken, the most behind are 384 of
+// 10 x 30 x 19 (87 -> 91) and 1 of 160 x 157 x 151 (122 -> 123 / 119 -> 126).  Backward, 2 x 2 outputs against 2 x 1: 1.4 (few
+// wavefronts) to 2 times (many), so below 0.54 (1 of 143 x 135 x 135 167 -> 155 / 166 -> 143, 0.49; 64 of 45 x 53 x 77
+// 547 -> 541 / 526 -> 498, 0.52; 1 of 160 x 90 x 159 134 -> 149 / 132 -> 137, 0.65; 8 of 22 x 19 x 41 62 -> 86 / 61 -> 84, 0.94).
+// Not tried below 32 columns; past 192 of them pairs leave the backward one workgroup a CU (64 of 30 x 41 x 255 857 -> 1073 /
+// 782 -> 949).
+// 2-D: where they halve the wavefronts across a row, from 193 columns on (two for four; 161 columns, two for three, forward
+// 5x5 of 256 channels of 119 x 161 110 -> 129 / 110 -> 130), and leave enough of them.  Forward up to 256 columns, 5x5 from 4 M
+// pixels on (256 of 213 x 201 244 -> 215 / 244 -> 217, 32 of 226 x 241 50 -> 57 / 50 -> 59; of 281 x 281 351 -> 351).  Backward
+// up to 512, from 2 M pixels on (3x3: 64 of 442 x 383 357 -> 339 / 357 -> 282, 8 of 378 x 499 53 -> 60 / 53 -> 52; 5x5: 64 of
+// 151 x 223 114 -> 105 / 114 -> 98, 32 of 184 x 201 81 -> 85 / 81 -> 83); of 5x5 rows of 257 to 384 columns, where one column a
+// thread takes five or six wavefronts, any (16 of 226 x 271 132 -> 94 / 132 -> 89), wider ones where segments of eight rows make
+// 2048 wavefronts of four a row (16 of 270 x 401 184 -> 105 / 184 -> 98, 8 of 378 x 499 85 -> 105 / 85 -> 99).
+// (Rows that one column a thread cannot take stay outside.)
+// (true in a host build whose tests send every row they can down these kernels)
+#ifndef NDC_LOOSE_EVERYWHERE
+#define NDC_LOOSE_EVERYWHERE false
+#endif
+static inline LoosePairs loose_pairs(const KGeom &q, const March &m)
+{
+    const long long nbc = (long long)q.B * q.G;
+    const Tuning tn = tuning();
+    if (m.H == 1) {
+        const long long pixels = nbc * m.D * m.W;
+        LoosePairs l = {m.W > 192 && m.W <= 256 && (m.KW == 3 || pixels >= 4000 * 1000), m.W > 192 && m.W <= 512};
+        if (m.KW == 3 || m.W <= 256) l.backward = l.backward && pixels >= 2000 * 1000;
+        else if (m.W > 384) l.backward = l.backward && nbc * 4 * (m.D / 8) >= 2048;
+        if (NDC_LOOSE_EVERYWHERE) l = {m.W >= 128 && m.W <= 256, m.W >= 128 && m.W <= 512};
+        return l;
+    }
+    LoosePairs l = {m.W >= 2 && m.W <= 256, m.W >= 32 && m.W <= 192};
+    if (NDC_LOOSE_EVERYWHERE || tn.rwf || tn.rwb || m.KH != 3 || m.KW != 3) return l;
+    // the cost of pairs as a share of that of single columns (0 where those do not fit, 2 where pairs do not)
+    auto ratio = [&](auto single, auto pair, int RH, const auto &targets, const CostModel &model, Tile &a, Tile &b) {
+        typedef decltype(single) S;
+        typedef decltype(pair) P;
+        if (!cost_tile<S>(m, RH, 1, nbc, targets, 0, 4, model, a)) return 0.0;
+        if (!cost_tile<P>(m, 2, -2, nbc, targets, 0, 4, model, b)) return 2.0;
+        return launch_cost(b, m, nbc, P::lds_floats(b), model) / launch_cost(a, m, nbc, S::lds_floats(a), model);
+    };
+    const int targets_f[4] = {64, 128, tn.threads_f, 512}, targets_b[3] = {128, 256, tn.threads_b};
+    Tile a, b;
+    if (l.forward) {
+        double r = ratio(FwdKernel<3, 3, 3, 4, 4, 1, float>(), FwdKernel<3, 3, 3, 4, 2, -2, float>(), 4, targets_f, kCostFmaF, a, b);
+        if (r > 0 && r < 2) r *= (b.NT == 192 ? 1.12 : 1.0) / (a.NT == 192 ? 1.12 : 1.0);
+        l.forward = r < (r > 0 && a.NT == 64 && b.NT == 64 ? 0.965 : 0.93);
+    }
+    if (l.backward)
+        l.backward = ratio(Bwd1Kernel<3, 3, 3, 4, 2, 1, float>(), Bwd1Kernel<3, 3, 3, 4, 2, -2, float>(), 2, targets_b, kCostFmaB, a, b) < 0.54;
+    return l;
+}
+
 template <int KD, int KH, int KW, int SC, int RHF, int RWF, int RHB, int RWB>
 static inline void plan_lds(Plan &pl, long long nbc)
 {
@@ -297,7 +354,10 @@ static inline bool make_plan_for(const KGeom &q, Plan &pl, int pairs, int dtype,
     pl.mfma1 = pl.mfma2 = pl.mfmaf = false;
     // 32-bit offsets inside one (sample, channel) volume
     if ((long long)q.sc * q.SP >= (1LL << 31)) return false;
-    if (!find_variant(q, pl.m, pairs, pl.v)) return false;
+    // (aligned tensors of an even width have their own pairs)
+    const bool ask = pairs >= kLooseForward && (pairs < kPairs || pl.m.W % 2);
+    const LoosePairs loose = ask ? loose_pairs(q, pl.m) : LoosePairs{false, false};
+    if (!find_variant(q, pl.m, pairs, loose, pl.v)) return false;
     const Tuning tn = tuning();
     if (!make_tile(pl.m, pl.v.RHF, pl.v.RWF, tn.threads_f, pl.tf)) return false;
     if (!make_tile(pl.m, pl.v.RHB, pl.v.RWB, tn.threads_b, pl.tb)) return false;

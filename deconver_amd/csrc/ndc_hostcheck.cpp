@@ -529,6 +529,7 @@ static int host_tiles_2d = 1;
 }  // namespace ndc
 
 #define NDC_TILES_2D ndc::host_tiles_2d
+#define NDC_LOOSE_EVERYWHERE (!ndc::host_tiles_2d)
 #include "ndc_api_impl.h"
 
 // LDS faults (races, out-of-bounds, uninitialised reads) seen by the host execution since
@@ -545,4 +546,16 @@ extern "C" long long ndc_host_faults(char *first, int n)
 }
 
 // Test hook of the host build only: 0 sends every 2-D problem down the marching kernels.
+// columns a thread of the marching kernels makes of this geometry, forward and backward (-2: pairs of any width and
+// alignment); aligned: every tensor is aligned to two elements
+extern "C" int ndc_host_columns(const ndc_geom *g, int aligned, int *forward, int *backward)
+{
+    ndc::KGeom q;
+    ndc::fused::Plan pl;
+    const int st = ndc::make_kgeom(g, q);
+    if (st) return st;
+    if (!ndc::fused::make_plan(q, pl, aligned != 0, g->dtype)) return NDC_ERR_GEOMETRY;
+    *forward = pl.v.RWF, *backward = pl.v.RWB;
+    return NDC_OK;
+}
 extern "C" void ndc_host_tiles_2d(int on) { ndc::host_tiles_2d = on ? 1 : 0; }

@@ -379,12 +379,13 @@ def test_autograd_node_names_its_family_once(matrix_switch):
         assert torch.equal(a, b)
 
 
-# column pairs of rows of any length and alignment (W even: at an odd element): one pair a row, either side of where the
-# backward takes them (32 columns), several wavefronts a row; 2-D marches of large images, in the backward only past 256
+# column pairs of rows of any length and alignment (W even: at an odd element) and the single columns that are taken where
+# those are ahead: short rows, several wavefronts a row, pairs in the forward (33 columns) and in the backward only (129); 2-D
+# marches of large images, in the backward only past 256
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2)])
 @pytest.mark.parametrize("C,ks,sp", [(3, (3, 3, 3), (3, 5, 2)), (3, (3, 3, 3), (6, 7, 31)), (2, (3, 3, 3), (5, 9, 33)),
                                      (2, (3, 3, 3), (4, 6, 64)), (1, (3, 3, 3), (5, 7, 255)), (64, (5, 5), (150, 201)),
-                                     (48, (3, 3), (160, 301))])
+                                     (48, (3, 3), (160, 301)), (4, (3, 3, 3), (6, 8, 33)), (96, (3, 3, 3), (6, 16, 129))])
 def test_pairs_of_any_width_and_alignment(C, ks, sp, dtype, tol):
     print("case", C, ks, sp, dtype, flush=True)
     lib = _lib.get_library()

@@ -96,6 +96,32 @@ def test_pairs_of_any_width_and_alignment(geom, shift, dtype, tol):
     assert host_faults(lib)[0] == 0
 
 
+# (C, kernel, spatial, aligned, columns forward, columns backward): as measured, one column a thread against pairs
+COLUMNS = [
+    (64, (3, 3, 3), (45, 53, 77), True, 1, -2), (32, (3, 3, 3), (91, 101, 87), True, -2, -2),
+    (192, (3, 3, 3), (23, 29, 33), True, -2, 1), (8, (3, 3, 3), (22, 19, 41), True, -2, 1),
+    (1024, (3, 3, 3), (6, 3, 7), True, 1, 1), (1024, (3, 3, 3), (3, 3, 3), True, 1, 1), (16, (3, 3, 3), (106, 82, 73), True, 1, 1),
+    (1, (3, 3, 3), (160, 90, 159), True, 1, 1), (1, (3, 3, 3), (143, 135, 135), True, -2, -2),
+    (64, (3, 3, 3), (30, 41, 255), True, -2, 1), (64, (3, 3, 3), (45, 53, 78), False, 1, -2), (64, (3, 3, 3), (45, 53, 78), True, 2, 2),
+    (256, (5, 5), (119, 161), True, 1, 1), (256, (5, 5), (213, 201), True, -2, -2), (32, (5, 5), (226, 241), True, 1, 1),
+    (64, (5, 5), (151, 223), True, 1, -2), (64, (3, 3), (120, 201), True, -2, 1), (16, (5, 5), (226, 271), True, 1, -2),
+    (16, (5, 5), (270, 401), True, 1, -2), (8, (5, 5), (378, 499), True, 1, 1), (8, (3, 3), (296, 301), True, 1, 1),
+    (64, (3, 3), (442, 383), True, 1, -2),
+]
+
+
+@pytest.mark.parametrize("C,ks,sp,aligned,forward,backward", COLUMNS)
+def test_columns_a_thread_makes(C, ks, sp, aligned, forward, backward):
+    import ctypes
+
+    lib = hostcheck_library()
+    like = torch.empty(1, C, *sp, device="meta")
+    g = ops.make_geom_for(like, torch.empty(C, 4, *ks, device="meta"), C, 1, 4, 1e-16, True)
+    f, b = ctypes.c_int(), ctypes.c_int()
+    assert lib._dll.ndc_host_columns(ctypes.byref(g), int(aligned), ctypes.byref(f), ctypes.byref(b)) == 0
+    assert (f.value, b.value) == (forward, backward)
+
+
 @pytest.mark.parametrize("geom", FUSED_GEOMS)
 @pytest.mark.parametrize("relu,with_bias", [(True, True), (False, False)])
 def test_fused_forward_backward_fp32(geom, relu, with_bias):
