@@ -932,6 +932,15 @@ static int gemm_waves(long long batch, long long cin, long long cout, long long 
     return waves;
 }
 
+// sizes that ndc_gemm takes
+static int gemm_sizes(long long batch, long long cin, long long cout, long long n, int dtype)
+{
+    const int st = gemm_check(batch, cin, cout, n, dtype);
+    if (st) return st;
+    const long long vt = batch * ((n + 127) / 128);
+    return (vt + 8) * 2 * ((cout + 31) / 32 + 8) > 0x7fffffffLL ? (int)NDC_ERR_GEOMETRY : (int)NDC_OK;
+}
+
 // voxels of a tile
 static int gemm_tile(int waves) { return waves > 0 ? 128 : waves ? 32 : 64; }
 
@@ -940,7 +949,7 @@ static int gemm_impl(const void *x, const float *w, int transposed, const float 
                      int dtype, void *stream)
 {
     if (!x || !w || !y) return NDC_ERR_NULL;
-    int st = gemm_check(batch, cin, cout, n, dtype);
+    const int st = gemm_sizes(batch, cin, cout, n, dtype);
     if (st) return st;
     if (mode < NDC_ACT_NONE || mode > NDC_GEMM_GELU_GRAD || mode == 3) return NDC_ERR_GEOMETRY;
     const bool grad = mode == NDC_GEMM_GELU_GRAD, act = mode == NDC_ACT_RELU || mode == NDC_ACT_GELU;
@@ -953,8 +962,6 @@ static int gemm_impl(const void *x, const float *w, int transposed, const float 
         return NDC_ERR_WORKSPACE;
     if (y == x || zkeep == x || (zkeep && zkeep == y)) return NDC_ERR_GEOMETRY;
     const int esz = dtype == NDC_BF16 ? 2 : 4;
-    const long long vt = batch * ((n + 127) / 128);
-    if ((vt + 8) * 2 * ((cout + 31) / 32 + 8) > 0x7fffffffLL) return NDC_ERR_GEOMETRY;
     return ndc::Backend::tile_gemm(x, w, transposed != 0, bias, residual, mask, y, zkeep, gpart, batch, (int)cin, (int)cout, n,
                                    mode, esz, gemm_waves(batch, cin, cout, n, esz), stream);
 }
@@ -968,7 +975,7 @@ int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, c
 
 int64_t ndc_gemm_parts(int64_t batch, int64_t cin, int64_t cout, int64_t n, int dtype)
 {
-    if (gemm_check(batch, cin, cout, n, dtype)) return 0;
+    if (gemm_sizes(batch, cin, cout, n, dtype)) return 0;
     const int tile = gemm_tile(gemm_waves(batch, cin, cout, n, dtype == NDC_BF16 ? 2 : 4));
     return batch * ((n + tile - 1) / tile);
 }

@@ -247,7 +247,7 @@ Matrix saved_weight(const Tensor &w, bool transposed, int64_t cout, const Tensor
 //             library / tiled: 64 -> 256 over 2 x 91 125 voxels 128 / 61, 256 -> 1024 over 2 x 27 000 277 / 212,
 //             512 -> 128 over 8 x 4096 37.7 / 33.9, 128 -> 64 over 8 x 16 384 27.6 / 27.5), but for those from 1024
 //             channels and more between 2 and 12 GFLOP (1024 -> 256 over 8 x 1024 36.9 / 42.2, 2048 -> 512 over
-//             4 x 1000 65 / 82, over 8000, 17 GFLOP, 130 / 118);
+//             4 x 1000 65 / 82, over 8000, 17 GFLOP, 130 / 118) and for sizes that the tiled GEMM refuses;
 //   kLibrary  the rest.
 enum Gemm { kStream, kTiled, kLibrary };
 
@@ -259,7 +259,10 @@ Gemm choose_gemm(const Tensor &x, int64_t cout, bool act_or_keep, bool tail)
     if (stream && B * n >= 2048 * 64) return kStream;
     if (n > (1 << 24)) return stream ? kStream : kLibrary;
     const double flops = 2.0 * (double)B * (double)n * (double)cin * (double)cout;
-    if (!half) return !tail && cin >= 1024 && flops >= 2e9 && flops < 12e9 ? kLibrary : kTiled;
+    if (!half) {
+        const bool library = (cin >= 1024 && flops < 12e9) || !ndc_gemm_parts(B, cin, cout, n, NDC_F32);
+        return !tail && flops >= 2e9 && library ? kLibrary : kTiled;
+    }
     if (flops < 4e9) return kTiled;
     if (tail && cin * cout <= 32 * 1024) return kTiled;
     return stream ? kStream : kLibrary;
@@ -670,7 +673,8 @@ Tensor update(const Tensor &x, const Tensor &z, const Tensor &h, const OptTensor
 // backward 0.180 -> 0.150.
 bool wide_is_tiled(int64_t B, int64_t cin, int64_t cout, int64_t n)
 {
-    if (cin >= cout || B < 1 || n < 1 || B > (1 << 20)) return false;   // (nothing to do, or more than the tiled GEMM takes)
+    // (no parts: nothing to do, or more than the tiled GEMM takes)
+    if (cin >= cout || !ndc_gemm_parts(B, cin, cout, n, NDC_F32)) return false;
     const double columns = (double)B * (double)((n + 63) / 64 * 64), flops = 2.0 * (double)cin * (double)cout * columns;
     return flops < 0.5e9 || (cin <= 128 && flops < 1e9);
 }

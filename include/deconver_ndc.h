@@ -471,7 +471,8 @@ int ndc_gemm(const void *x, const float *w, int transposed, const float *bias, c
  * The NDC_GEMM_GELU_GRAD form with the gradient of `bias`: gz = (W gy) * gelu'(z + bias) for w the
  * (cin, cout) storage of W, and, if gpart is not NULL, gpart[t][c] = the sum of gz over voxel tile t,
  * float32 and taken before gz is rounded to its storage: ndc_gemm_parts(...) * cout floats, every one
- * written.  The gradient of `bias` is the sum over the tiles (ndc_column_sums).
+ * written.  The gradient of `bias` is the sum over the tiles (ndc_column_sums).  0 parts: sizes that
+ * ndc_gemm refuses.
  */
 int64_t ndc_gemm_parts(int64_t batch, int64_t cin, int64_t cout, int64_t n, int dtype);
 int ndc_gemm_gelu_grad(const void *gy, const float *w, const float *bias, const void *z, void *gz,

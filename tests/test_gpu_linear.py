@@ -5,6 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from deconver_amd import _lib, ops
 from deconver_amd.layers import Linear, pointwise_linear
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +111,30 @@ def test_bare_float32_products_that_widen(B, cin, cout, n, tiled, transposed):
     assert float((y.double() - w.double() @ x.double()).norm() / y.double().norm()) < 2e-6     # float32 sums
     lib = torch.bmm(w.expand(B, cout, cin), x)
     assert tiled or (y - lib).abs().max() <= 0 or transposed    # (the library has a kernel of its own for each storage)
+
+
+def test_bare_float32_products_beyond_the_tiled_gemm():
+    """More samples, and more output channels, than the tiled GEMM takes go by the library: forward and input gradient."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn((1 << 20) + 8, 32, 1, generator=g, device="cuda").requires_grad_(True)
+    w = torch.randn(32, 32, generator=g, device="cuda") / 32 ** 0.5
+    y = pointwise_linear(x, w)
+    y.backward(x.detach())
+    for got, m in ((y.detach(), w), (x.grad, w.t())):
+        assert float((got - (x.detach().flatten(1) @ m.t())[..., None]).abs().max()) < 1e-4
+    x, w = torch.randn(1, 1, 3, generator=g, device="cuda"), torch.randn((1 << 20) + 8, 1, generator=g, device="cuda")
+    assert torch.equal(pointwise_linear(x, w), w * x)
+
+
+# ... the route as well as the error: the tiled GEMM's bits, or the library's
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("B,cin,cout,n,tiled", WIDE)
+def test_products_that_widen_go_by_their_rule(B, cin, cout, n, tiled, transposed):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, w = torch.randn(B, cin, n, generator=g, device="cuda"), torch.randn(cout, cin, generator=g, device="cuda") / cin ** 0.5
+    stored = w.t().contiguous() if transposed else w
+    y = pointwise_linear(x, stored, transposed=transposed)
+    if tiled:
+        assert torch.equal(y, ops.gemm(_lib.get_library(), x, stored, transposed=transposed)[0])
+    else:
+        assert torch.equal(y, torch.bmm((stored.t() if transposed else stored).expand(B, cout, cin), x))
