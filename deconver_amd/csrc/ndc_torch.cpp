@@ -1164,7 +1164,9 @@ struct ChannelNorm : public torch::autograd::Function<ChannelNorm> {
                                   scope.stream), "ndc_chnorm_backward");
         if (affine) {
             // (the library's own sum, two launches of 4 us: torch's takes 10 and clears a semaphore ahead of it, 4 more)
-            const Tensor sums = column_sums(partial.view({partial.size(0), 2 * C}), scope.stream).view({C, 2});
+            // Its columns end at 2^22; more than half as many channels take torch's.
+            const Tensor sums = 2 * C > (1 << 22) ? partial.sum(0)
+                                                  : column_sums(partial.view({partial.size(0), 2 * C}), scope.stream).view({C, 2});
             if (need[1]) gw = sums.select(1, 0).to((at::ScalarType)cfg[2]).contiguous();
             if (need[2]) gb = sums.select(1, 1).to((at::ScalarType)cfg[3]).contiguous();
         }

@@ -158,3 +158,15 @@ def test_default_norm_block_on_the_gpu_matches_its_float64_general_route():
     with torch.autocast("cuda", dtype=torch.bfloat16):
         y = blk(x.cuda())
     assert _rel(y.cpu(), ref) <= 2e-2
+
+
+@pytest.mark.gpu
+def test_more_channels_than_a_column_sum_takes():
+    C = (1 << 21) + 1
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    x, gy = (torch.randn(1, C, 2, generator=gen, device="cuda") for _ in range(2))
+    w, b = (torch.full((C,), v, device="cuda", requires_grad=True) for v in (1.0, 0.0))
+    y = _lib.get_native().channel_norm(x, w, b, 1e-5)
+    y.backward(gy)
+    torch.testing.assert_close(b.grad, gy.sum((0, 2)), rtol=1e-6, atol=1e-6)
+    torch.testing.assert_close(w.grad, (gy * y.detach()).sum((0, 2)), rtol=1e-4, atol=1e-4)
