@@ -173,7 +173,12 @@ template <class F, int K, int NR> struct Tiled {
     }
 };
 
-// The box of a launch: the least cost over one or two rows a thread and the boxes that cut an axis into equal parts.
+#ifndef NDC_BOX_WEIGHED
+#define NDC_BOX_WEIGHED()   // (the host build counts the boxes it looks at)
+#endif
+// The box of a launch: the least cost over one or two rows a thread and the boxes that cut an axis into equal parts, of the
+// first axis at most 32, of the second 16, of the last 6.  Volumes of which such parts have more than 512 threads' positions
+// (144^3 and 320^2, not 128^3 and 256^2) have no box.
 // The cost is what the busiest CU has to do: products and LDS reads of its SIMDs (dearer where a SIMD has fewer than two
 // wavefronts), the values and 128-byte lines staged, the lines its outputs touch, and a fixed part for every round of
 // workgroups the CU holds at once times the groups of channels.  Its constants were fitted to 70 boxes each of five
@@ -183,72 +188,99 @@ static inline bool choose_box(const KGeom &q, int nin, int nb, int cin, long lon
     const int K = q.kW, weights = box_weights(q, nb), budget = 10 * 1024, kMaxLds = 160 * 1024;
     double least = 0;
     best.NT = 0;
-    for (int nr = 1; nr <= 2; ++nr)
-        for (int pw = 1; pw <= 6 && pw <= q.W; ++pw)
-            for (int ph = 1; ph <= 16 && ph <= q.H; ++ph) {
-                int before = 0;
-                for (int pd = 1; pd <= 32 && pd <= q.D; ++pd) {
-                    Box t;
-                    t.NR = nr;
-                    t.TW = (q.W + pw - 1) / pw, t.TH = (q.H + ph - 1) / ph, t.TD = (q.D + pd - 1) / pd;
-                    if (t.TD == before) continue;
-                    before = t.TD;
-                    t.HP = (t.TH + nr - 1) / nr;
+    // the extents that equal parts of an axis have, and how many of them it takes
+    struct Parts {
+        int n = 0, extent[32], count[32];
+        Parts(int of, int most)
+        {
+            for (int p = 1; p <= most && p <= of; ++p) {
+                const int e = (of + p - 1) / p;
+                if (n && extent[n - 1] == e) continue;
+                extent[n] = e, count[n++] = (of + e - 1) / e;
+            }
+        }
+    };
+    const Parts pw(q.W, 6), ph(q.H, 16), pd(q.D, 32);
+    auto row_cost = [&](double product, int nr) { return product * nr * nb * K * nin + 0.8 * nb * K + 0.75 * nin * (K + nr - 1); };
+    for (int nr = 1; nr <= 2; ++nr) {
+        // wavefronts a SIMD has the registers for
+        int simd = 512 / (46 + nr * nb * (nin + K) + 2 * nin * K);
+        simd = simd < 1 ? 1 : simd > 8 ? 8 : simd;
+        const double least_row = row_cost(1.1, nr);
+        for (int iw = 0; iw < pw.n; ++iw)
+            for (int ih = 0; ih < ph.n; ++ih) {
+                Box t;
+                t.NR = nr, t.TW = pw.extent[iw], t.TH = ph.extent[ih], t.HP = (t.TH + nr - 1) / nr;
+                t.SH = t.HP * nr + K - 1, t.SW = t.TW + K - 1, t.nh = ph.count[ih], t.nw = pw.count[iw];
+                if (t.TW > 512 || t.HP > 512) continue;
+                for (int id = 0; id < pd.n; ++id) {
+                    t.TD = pd.extent[id], t.nd = pd.count[id], t.tiles = t.nd * t.nh * t.nw;
                     const long long n = (long long)t.TW * t.HP * t.TD;
                     if (n > 512) continue;
+                    NDC_BOX_WEIGHED();
                     t.NT = (int)((n + 63) / 64 * 64);
-                    t.SD = t.TD + q.kD - 1, t.SH = t.HP * nr + K - 1, t.SW = t.TW + K - 1, t.SV = t.SD * t.SH * t.SW;
-                    t.over_sw = 0xffffffffu / t.SW + 1, t.over_sh = 0xffffffffu / t.SH + 1;
-                    t.chunk = budget / (nin * t.SV + weights);
-                    if (t.chunk < 1) continue;
-                    if (t.chunk > cin) t.chunk = cin;
-                    t.nd = (q.D + t.TD - 1) / t.TD, t.nh = (q.H + t.TH - 1) / t.TH, t.nw = (q.W + t.TW - 1) / t.TW;
-                    t.tiles = t.nd * t.nh * t.nw;
+                    t.SD = t.TD + q.kD - 1, t.SV = t.SD * t.SH * t.SW;
+                    const int words = nin * t.SV + weights;   // of a channel
+                    if (words > budget) continue;
                     const long long group = (units * t.tiles + 255) / 256;   // workgroups of the busiest CU
-                    const int w = t.NT / 64, lds = 4 * t.chunk * (nin * t.SV + weights);
-                    // wavefronts a SIMD has the registers for, workgroups a CU has the place for
-                    int simd = 512 / (46 + nr * nb * (nin + K) + 2 * nin * K);
-                    simd = simd < 1 ? 1 : simd > 8 ? 8 : simd;
-                    int held = kMaxLds / lds;
+                    const int w = t.NT / 64;
+                    const double rows = (double)((group * w + 3) / 4) * cin * (q.KT / K);
+                    const double staging = (double)group * cin * nin * (t.SV / 64.0 * 8 + 8.4 * t.SD * t.SH * (t.SW / 32.0 + 1));
+                    const double out = group * 40.0 * nb * t.TD * t.TH * (t.TW / 32.0 + 1);
+                    if (best.NT) {
+                        // the least that it can cost, without the divisions: as many workgroups a CU as registers allow
+                        const double share = w / (4.0 * simd), rounds = group * (share < 1 ? share : 1.0), groups = cin * (double)words * (1.0 / budget);
+                        const double fixed = (rounds > 1 ? rounds : 1.0) * (groups > 1 ? groups : 1.0) * 40e3;
+                        if ((rows * least_row + 0.66 * staging + out + fixed) * (1 - 1e-9) > least) {
+                            if (n < 64) break;
+                            continue;
+                        }
+                    }
+                    t.chunk = budget / words;
+                    if (t.chunk > cin) t.chunk = cin;
+                    int held = kMaxLds / (4 * t.chunk * words);   // workgroups a CU has the place for
                     if (held * w > 4 * simd) held = 4 * simd / w;
                     if (held > group) held = (int)group;
                     if (held < 1) held = 1;
                     const double per_simd = held * w / 4.0, product = per_simd >= 2 ? 1.1 : 1.1 * (1 + 0.37 * (2 - (per_simd < 1 ? 1 : per_simd)));
-                    const double row = product * nr * nb * K * nin + 0.8 * nb * K + 0.75 * nin * (K + nr - 1);
-                    const double staging = (double)group * cin * nin * (t.SV / 64.0 * 8 + 8.4 * t.SD * t.SH * (t.SW / 32.0 + 1));
-                    const double cost = (double)((group * w + 3) / 4) * cin * (q.KT / K) * row + (held == 1 ? 1.0 : 0.66) * staging +
-                                        group * 40.0 * nb * t.TD * t.TH * (t.TW / 32.0 + 1) +
+                    const double cost = rows * row_cost(product, nr) + (held == 1 ? 1.0 : 0.66) * staging + out +
                                         (double)((group + held - 1) / held) * ((cin + t.chunk - 1) / t.chunk) * 40e3;
                     if (!best.NT || cost < least) best = t, least = cost;
                     if (n < 64) break;
                 }
             }
-    return best.NT > 0;
+    }
+    if (!best.NT) return false;
+    best.over_sw = 0xffffffffu / best.SW + 1, best.over_sh = 0xffffffffu / best.SH + 1;
+    return true;
 }
 
-// ... of the last sizes a thread saw
+// ... of the sizes a thread saw last.  A search takes the host 2 to 8 us, and a layer with its backward asks for five: what
+// is kept serves some hundred sizes, so that a network searches once.
 static inline bool box_of(const KGeom &q, int nin, int nb, int cin, long long units, Box &box)
 {
     if ((q.kW != 3 && q.kW != 5) || q.kH != q.kW || !small_volume(q) || tap_block(q) != q.kW) return false;
+    static const int kWords = 10, kEntries = 1024, kWays = 4;
     struct Entry {
-        long long units;
-        int key[8];
+        int key[kWords];   // zeros where nothing is kept (a filter has kW > 0)
         bool ok;
         Box box;
     };
-    static thread_local Entry kept[32];
-    static thread_local int next = 0;
-    const int key[8] = {q.D, q.H, q.W, q.kD, q.kW, nin, nb, cin};
-    for (const Entry &e : kept)
-        if (e.units == units && !memcmp(e.key, key, sizeof key)) {
-            box = e.box;
-            return e.ok;
+    static thread_local Entry kept[kEntries] = {};
+    static thread_local unsigned turn = 0;
+    const int key[kWords] = {q.kW, q.kD, q.D, q.H, q.W, nin, nb, cin, (int)(units >> 32), (int)units};
+    unsigned at = 0;
+    for (int k : key) at = ((at ^ at >> 15) + (unsigned)k) * 0x9e3779b1u;
+    Entry *set = kept + (at >> 16) % (kEntries / kWays) * kWays;
+    int way = 0;
+    for (; way < kWays && set[way].key[0]; ++way)
+        if (!memcmp(set[way].key, key, sizeof(key))) {
+            box = set[way].box;
+            return set[way].ok;
         }
-    Entry &e = kept[next];
-    next = (next + 1) % 32;
+    Entry &e = set[way < kWays ? way : (int)(turn++ % kWays)];
     e.ok = choose_box(q, nin, nb, cin, units, e.box);
-    e.units = units;
-    memcpy(e.key, key, sizeof key);
+    memcpy(e.key, key, sizeof(key));
     box = e.box;
     return e.ok;
 }

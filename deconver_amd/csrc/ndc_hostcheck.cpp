@@ -525,11 +525,14 @@ struct Backend {
 
 // whether small images run tile by tile, as on the GPU, or march
 static int host_tiles_2d = 1;
+// boxes that the direct kernels' search looked at
+static long long host_boxes_weighed = 0;
 
 }  // namespace ndc
 
 #define NDC_TILES_2D ndc::host_tiles_2d
 #define NDC_LOOSE_EVERYWHERE (!ndc::host_tiles_2d)
+#define NDC_BOX_WEIGHED() (++ndc::host_boxes_weighed)
 #include "ndc_api_impl.h"
 
 // LDS faults (races, out-of-bounds, uninitialised reads) seen by the host execution since
@@ -545,7 +548,6 @@ extern "C" long long ndc_host_faults(char *first, int n)
     return total;
 }
 
-// Test hook of the host build only: 0 sends every 2-D problem down the marching kernels.
 // columns a thread of the marching kernels makes of this geometry, forward and backward (-2: pairs of any width and
 // alignment); aligned: every tensor is aligned to two elements
 extern "C" int ndc_host_columns(const ndc_geom *g, int aligned, int *forward, int *backward)
@@ -558,4 +560,19 @@ extern "C" int ndc_host_columns(const ndc_geom *g, int aligned, int *forward, in
     *forward = pl.v.RWF, *backward = pl.v.RWB;
     return NDC_OK;
 }
+
+// The direct kernels' launch for `units` of nb output channels each, nin inputs of cin channels: its workgroups and their
+// threads and rows a thread, or zeros where no box is taken.  Returns the boxes looked at for it.
+extern "C" long long ndc_host_box(const ndc_geom *g, int nin, int nb, int cin, long long units, long long *launch)
+{
+    ndc::KGeom q;
+    ndc::direct::Box t;
+    if (ndc::make_kgeom(g, q)) return -1;
+    const long long before = ndc::host_boxes_weighed;
+    const bool ok = ndc::direct::box_of(q, nin, nb, cin, units, t);
+    launch[0] = ok ? units * t.tiles : 0, launch[1] = ok ? t.NT : 0, launch[2] = ok ? t.NR : 0;
+    return ndc::host_boxes_weighed - before;
+}
+
+// Test hook of the host build only: 0 sends every 2-D problem down the marching kernels.
 extern "C" void ndc_host_tiles_2d(int on) { ndc::host_tiles_2d = on ? 1 : 0; }

@@ -5,7 +5,7 @@ planes; and a filter without boxes that takes its weights from LDS.  Oracle and 
 import pytest
 import torch
 
-from deconver_amd import _lib
+from deconver_amd import _lib, ops
 from tests.helpers import host_faults, hostcheck_library
 from tests.test_direct_blocks import _compare
 
@@ -40,3 +40,48 @@ def test_boxes_on_the_host_build(geom, dtype):
 def test_boxes_on_the_gpu(geom, dtype):
     print("case", geom, dtype, flush=True)
     _compare(_lib.get_library(), geom, dtype, "cuda")
+
+
+# filters of unequal extents and images beyond the boxes: one position at a time, three and five taps, the weights from the
+# scalar unit and from LDS
+UNEQUAL = [(4, 2, 6, (5, 3), (9, 11), 1), (6, 3, 4, (3, 5, 3), (5, 6, 7), 2), (4, 2, 3, (3, 5), (8, 12), 1)]
+WITHOUT = [(4, 2, 6, (3, 3), (384, 256), 1), (16, 16, 4, (3, 3), (384, 256), 2), (16, 16, 4, (5, 3), (64, 64), 8)]
+
+
+@pytest.mark.parametrize("geom", UNEQUAL)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_position_at_a_time_on_the_host_build(geom, dtype):
+    lib = hostcheck_library()
+    _compare(lib, geom, dtype, "cpu")
+    assert host_faults(lib)[0] == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("geom", UNEQUAL + WITHOUT)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_position_at_a_time_on_the_gpu(geom, dtype):
+    print("case", geom, dtype, flush=True)
+    _compare(_lib.get_library(), geom, dtype, "cuda")
+
+
+def _box(sp, ks=(3, 3, 3), nin=1, nb=4, cin=4, units=16):
+    """(boxes looked at, workgroups, threads, rows a thread) of a launch; no workgroups: no box."""
+    import ctypes
+
+    lib = hostcheck_library()
+    like = torch.empty(1, 8, *sp, device="meta")
+    g = ops.make_geom_for(like, torch.empty(8, 8, *ks, device="meta"), 2, 4, 8, 1e-16, True)
+    launch = (ctypes.c_longlong * 3)()
+    lib._dll.ndc_host_box.restype = ctypes.c_longlong
+    looked = lib._dll.ndc_host_box(ctypes.byref(g), nin, nb, cin, ctypes.c_longlong(units), launch)
+    return looked, *launch
+
+
+def test_a_size_is_searched_once():
+    """What the host does for a launch: few boxes looked at, none where none can be, and none for a size it has seen."""
+    sizes = [(20 + k, 24 + k, 22 + 2 * k) for k in range(24)]
+    first = [_box(sp, nin=nin)[0] for sp in sizes for nin in (1, 2, 3)]
+    assert all(0 < n <= 800 for n in first)
+    assert not any(_box(sp, nin=nin)[0] for sp in sizes for nin in (1, 2, 3))
+    for sp, ks in (((160, 160, 160), (3, 3, 3)), ((192, 192, 192), (3, 3, 3)), ((320, 320), (3, 3))):
+        assert _box(sp, ks)[:2] == (0, 0)
