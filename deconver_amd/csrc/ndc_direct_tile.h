@@ -285,6 +285,13 @@ static inline bool box_of(const KGeom &q, int nin, int nb, int cin, long long un
     return e.ok;
 }
 
+// ... if a launch takes them: fewer than 2^32 threads (46 x 1 x 60 positions are six boxes of 512 threads a unit where they
+// were 2816 threads one position at a time)
+static inline bool takes_boxes(const KGeom &q, int nin, int nb, int cin, long long units, Box &box)
+{
+    return box_of(q, nin, nb, cin, units, box) && units * box.tiles < (1LL << 31) && units * box.tiles * box.NT < (1LL << 32);
+}
+
 template <class BE, class F, int K, int NR> static int launch_boxes(const F &f, const Box &t, long long units, void *stream)
 {
     typedef Tiled<F, K, NR> Kernel;
@@ -298,7 +305,7 @@ template <class BE, class F> static int launch(const F &f, long long units, void
     if constexpr (F::kKWB == 3 || F::kKWB == 5) {
         constexpr int K = F::kKWB;
         Box t;
-        if (box_of(f.q, F::kNin, F::kNB, F::kAdj ? f.q.m : f.q.sc, units, t) && units * t.tiles < (1LL << 31))
+        if (takes_boxes(f.q, F::kNin, F::kNB, F::kAdj ? f.q.m : f.q.sc, units, t))
             return t.NR == 2 ? launch_boxes<BE, F, K, 2>(f, t, units, stream) : launch_boxes<BE, F, K, 1>(f, t, units, stream);
     }
     return BE::weighted_unit(units, f.q.SP, stream, f);

@@ -569,7 +569,7 @@ extern "C" long long ndc_host_box(const ndc_geom *g, int nin, int nb, int cin, l
     ndc::direct::Box t;
     if (ndc::make_kgeom(g, q)) return -1;
     const long long before = ndc::host_boxes_weighed;
-    const bool ok = ndc::direct::box_of(q, nin, nb, cin, units, t);
+    const bool ok = ndc::direct::takes_boxes(q, nin, nb, cin, units, t);
     launch[0] = ok ? units * t.tiles : 0, launch[1] = ok ? t.NT : 0, launch[2] = ok ? t.NR : 0;
     return ndc::host_boxes_weighed - before;
 }

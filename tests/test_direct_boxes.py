@@ -85,3 +85,11 @@ def test_a_size_is_searched_once():
     assert not any(_box(sp, nin=nin)[0] for sp in sizes for nin in (1, 2, 3))
     for sp, ks in (((160, 160, 160), (3, 3, 3)), ((192, 192, 192), (3, 3, 3)), ((320, 320), (3, 3))):
         assert _box(sp, ks)[:2] == (0, 0)
+
+
+def test_boxes_of_fewer_threads_than_a_launch_takes():
+    """46 x 1 x 60 positions a unit are 2816 threads one at a time and more in boxes: those reach 2^32 at fewer units."""
+    sp, ks, most = (46, 1, 60), (7, 3, 3), (2 ** 32 - 1) // 2816
+    for units in (1000, most // 2, most * 9 // 10, most):
+        _, groups, threads, _ = _box(sp, ks, 1, 1, 1, units)
+        assert groups * threads < 2 ** 32 and (groups > 0) == (units < most)
