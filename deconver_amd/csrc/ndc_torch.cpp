@@ -247,7 +247,10 @@ Matrix saved_weight(const Tensor &w, bool transposed, int64_t cout, const Tensor
 //             library / tiled: 64 -> 256 over 2 x 91 125 voxels 128 / 61, 256 -> 1024 over 2 x 27 000 277 / 212,
 //             512 -> 128 over 8 x 4096 37.7 / 33.9, 128 -> 64 over 8 x 16 384 27.6 / 27.5), but for those from 1024
 //             channels and more between 2 and 12 GFLOP (1024 -> 256 over 8 x 1024 36.9 / 42.2, 2048 -> 512 over
-//             4 x 1000 65 / 82, over 8000, 17 GFLOP, 130 / 118) and for sizes that the tiled GEMM refuses;
+//             4 x 1000 65 / 82, over 8000, 17 GFLOP, 130 / 118), for samples that fill half a tile's 128 voxels or less
+//             (256 -> 256 over 4197 x 4 130 / 446, over 1050 x 16 59 / 121, over 954 x 64 74 / 115, but over 210 x 80
+//             45 / 39; 128 -> 512 over 1908 x 32 110 / 257; not up to 64 channels, 64 -> 64 over 8393 x 32 109 / 83), and
+//             for sizes that the tiled GEMM refuses;
 //   kLibrary  the rest.
 enum Gemm { kStream, kTiled, kLibrary };
 
@@ -260,7 +263,7 @@ Gemm choose_gemm(const Tensor &x, int64_t cout, bool act_or_keep, bool tail)
     if (n > (1 << 24)) return stream ? kStream : kLibrary;
     const double flops = 2.0 * (double)B * (double)n * (double)cin * (double)cout;
     if (!half) {
-        const bool library = (cin >= 1024 && flops < 12e9) || !ndc_gemm_parts(B, cin, cout, n, NDC_F32);
+        const bool library = (cin >= 1024 && flops < 12e9) || (n <= 64 && cin * cout > 64 * 64) || !ndc_gemm_parts(B, cin, cout, n, NDC_F32);
         return !tail && flops >= 2e9 && library ? kLibrary : kTiled;
     }
     if (flops < 4e9) return kTiled;

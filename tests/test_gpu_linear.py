@@ -138,3 +138,18 @@ def test_products_that_widen_go_by_their_rule(B, cin, cout, n, tiled, transposed
         assert torch.equal(y, ops.gemm(_lib.get_library(), x, stored, transposed=transposed)[0])
     else:
         assert torch.equal(y, torch.bmm((stored.t() if transposed else stored).expand(B, cout, cin), x))
+
+
+# (B, cin, cout, n, by the tiled GEMM): input gradients of 2 GFLOP and more whose samples fill half a tile or less, or more
+@pytest.mark.parametrize("B,cin,cout,n,tiled", [(1050, 256, 256, 16, False), (525, 512, 128, 32, False), (264, 128, 512, 64, False),
+                                                (260, 256, 256, 65, True), (8393, 64, 64, 32, True)])
+def test_input_gradients_of_samples_of_few_voxels(B, cin, cout, n, tiled):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.empty(B, cin, n, device="cuda").requires_grad_(True)
+    w = torch.randn(cout, cin, generator=g, device="cuda") / cin ** 0.5
+    gy = torch.randn(B, cout, n, generator=g, device="cuda")
+    pointwise_linear(x, w).backward(gy)
+    if tiled:
+        assert torch.equal(x.grad, ops.gemm(_lib.get_library(), gy, w, transposed=True)[0])
+    else:
+        assert torch.equal(x.grad, torch.bmm(w.t().expand(B, cin, cout), gy))
