@@ -920,12 +920,16 @@ int ndc_weight_grad(const void *gz, const void *x, float *gw, float *gb, int64_t
 // workgroup (32 per wavefront) as still leave two workgroups per CU.
 // float32 is sliced up to 600 workgroups (us, sliced / tiled: 512 -> 2048 over 572, 576 of them, 22.1 / 23.1, 512 -> 512
 // over 8 x 256, 512, 17.1 / 17.9; 1024 -> 256 over 2 x 3375, 848, 55 / 43; 256 -> 256 over 8 x 1024, 1024, 19 / 13.7).
+// Samples that fill half of a tile or less are sliced, as bf16 is, up to 1024 workgroups and in the smaller tiles up to 256
+// of the larger ones (us, sliced / tiled: 1024 -> 256 over 96 x 4, 768 of them, 39 / 56, over 90 x 32 40 / 56; 256 -> 256 over
+// 96 x 16 13.6 / 18.6; 512 -> 128 over 179 x 64 25 / 33; smaller tiles / larger: 1024 -> 256 over 20 x 2, 160, 12.8 / 15.2).
 // Otherwise 64 rows a workgroup from 400 of those on (256 -> 256 over 13 824, 432 of them, 19 against 21 with 32 rows;
 // 512 -> 128 over 20 000, 314, 31 against 29).
 static int gemm_waves(long long batch, long long cin, long long cout, long long n, int esz)
 {
     const long long vt = batch * ((n + 127) / 128), small = batch * ((n + 63) / 64) * ((cout + 31) / 32);
-    if (small <= (esz == 4 ? 600 : 1024) && cin % (16 / esz) == 0 && n >= 2) return small <= (esz == 4 ? 128 : 256) ? -1 : 0;
+    if (small <= (esz == 4 && n > 64 ? 600 : 1024) && cin % (16 / esz) == 0 && n >= 2)
+        return small <= (esz == 4 && n > 32 ? 128 : 256) ? -1 : 0;
     if (esz == 4) return cout > 32 && vt * ((cout + 63) / 64) >= 400 ? 2 : 1;
     int waves = 4;
     while (waves > 1 && (cout <= 32 * (waves / 2) || vt * ((cout + 32 * waves - 1) / (32 * waves)) < 512)) waves /= 2;

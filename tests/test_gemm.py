@@ -117,6 +117,15 @@ def test_small_grids_keep_one_order_of_sums(cin, cout, n):
     assert torch.equal(ops.gemm(lib, x, w)[0][..., :half], ops.gemm(lib, x[..., :half].contiguous(), w)[0])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,cin,cout,n", [(96, 1024, 256, 16), (180, 512, 128, 64), (24, 1024, 256, 16), (40, 256, 128, 32)])
+def test_small_float32_grids_of_few_voxels_are_sliced(B, cin, cout, n):
+    """601 to 1024 of the larger tiles over samples of at most 64 voxels, 129 to 256 over at most 32: the bits of fewer samples."""
+    lib, (x, _, _, _), w, _ = _setup("cuda", (B, cin, cout, n), torch.float32)
+    few = max(1, 100 // (cout // 32)) if B * cout // 32 <= 256 else B // 2
+    assert torch.equal(ops.gemm(lib, x, w)[0][:few], ops.gemm(lib, x[:few].contiguous(), w)[0])
+
+
 # rows of 32 and 64 a workgroup, one chain of sums and several; ragged channels, rows and voxels
 PARTS = [(1, 33, 40, 38501), (2, 100, 130, 9001), (1, 32, 64, 52001), (2, 72, 30, 20003), (1, 1030, 96, 13000)]
 
