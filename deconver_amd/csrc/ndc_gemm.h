@@ -126,15 +126,14 @@ template <typename T> __device__ inline u32x4 ragged(const T *p, int have)
 //   * the bf16 instruction drops what it shifts out, which leaves its sums 1e-8 .. 1e-7 of their norm too
 //     low, and that adds up in sums over voxels: half of the results are made with the sign turned (every
 //     other voxel; in weight gradients every other split), so that it cancels;
-//   * infinities, and what rounds to one, leave NaN;
-//   * the instruction takes denormal parts for zero, and sums.  What of a value is in such parts is below 3 x 2^-126, so
-//     that a sum of K products misses no more than 2^-124 K (a + b + 1), a and b the largest of its two factors.
-// Where a sum is not finite, or so small that this may count (2^-24 of it and more) and its factors have values other
-// than zero below 2^-102, or some whose product is, a tile is made again by the float32 instruction.  Sums that cancel to
-// zero by themselves are told apart by a look at their factors: one in some 10^7, 2 us for the wavefront that has it.
-// The largest values and the look at the sums take up to 4 % (us, without and with: 512 -> 128 channels over 8 x 4096
-// voxels 37.0 and 37.6, 64 -> 256 over 8 x 16 384 46 and 48, 32 -> 128 over 8 x 65 536 77 and 79, 256 x 64 weight gradient
-// over 8 x 16 384 42.5 and 41.8; a recorded 2-D training step on one 128^2 image 1966 and 1986).
+//   * it takes denormal parts and results for zero: both factors are parted 2^24 times as large, at which every bit of a
+//     float32, the last of a denormal one too, is a normal bf16, and what falls short as a result is below 2^-173;
+//   * infinities, values of 2^104 and products of 2^78 and more leave sums that are not finite: such a tile is made
+//     again by the float32 instruction.
+// (Instead of the scale, a look at the sums and the largest values for what small values may have lost took 1 to 9 % of
+// the kernels, and on volumes with an empty background, where many sums are zero, up to 1.9 times the weight gradients' time:
+// 256 x 64 over 80 x 80 x 72 voxels 140 -> 230 us, 128 x 128 43 -> 56; like this 140 and 43.)
+static constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;   // (of a factor, of a product)
 __device__ inline u32x2 next_part(float (&v)[4])   // four values' next part, which is taken off them
 {
     const u32x2 r = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
@@ -145,90 +144,30 @@ __device__ inline u32x2 next_part(float (&v)[4])   // four values' next part, wh
     }
     return r;
 }
-// ... their first part, of the values with `sign` (a sign bit or nothing) turned: two at a time, and the rest of it by
-// the subtraction
-__device__ inline u32x2 first_part(float (&v)[4], uint32_t sign)
-{
-    const uint32_t both = sign | sign >> 16;
-    const float one = __uint_as_float(0x3f800000u | sign);
-    const u32x2 r = {pack_bf16x2(v[0], v[1]) ^ both, pack_bf16x2(v[2], v[3]) ^ both};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        v[2 * h] = __builtin_fmaf(v[2 * h], one, -__uint_as_float(r[h] << 16));
-        v[2 * h + 1] = __builtin_fmaf(v[2 * h + 1], one, -__uint_as_float(r[h] & 0xffff0000u));
-    }
-    return r;
-}
 // A stage of float32 granules in parts: per part, granules of 8 bf16 (two of the float32 ones), four deep;
 // the rows turned by four per depth, so that a writer's lanes along the depth do not meet a bank twice.
 static const int kPartDepth = 4;
 __device__ inline int part_slot(int rows, int part, int d, int r) { return (part * kPartDepth + d) * rows + (r ^ (4 * d)); }
-__device__ inline void put_parts(u32x4 *lds, int rows, int q, int r, float (&v)[4], uint32_t sign)
+__device__ inline void put_parts(u32x4 *lds, int rows, int q, int r, const float (&g)[4], float scale)
 {
+    float v[4] = {g[0] * scale, g[1] * scale, g[2] * scale, g[3] * scale};
     u32x2 *half = reinterpret_cast<u32x2 *>(lds);
 #pragma unroll
-    for (int p = 0; p < 3; ++p) half[2 * part_slot(rows, p, q >> 1, r) + (q & 1)] = p ? next_part(v) : first_part(v, sign);
+    for (int p = 0; p < 3; ++p) half[2 * part_slot(rows, p, q >> 1, r) + (q & 1)] = next_part(v);
 }
 // granules of 16 bytes per row of a stage of depth D
 template <typename T> constexpr int stage_granules(int depth) { return sizeof(T) == 4 ? 3 * kPartDepth : depth; }
-// the largest of `most` and the sizes of four values (fmaxf turns values from memory quiet first, one by one)
-__device__ inline float largest(float most, const float (&v)[4])
+// whether a wavefront's sums are all finite
+template <int RT, int CT> __device__ inline bool all_finite(const f32x16 (&acc)[RT][CT])
 {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(v[0]), "v"(v[1]));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(v[2]), "v"(v[3]));
-    return most;
-}
-// the largest size of N lanes in the last of them (N: 8 or 64, see wave_sum)
-template <int N> __device__ inline float lanes_largest(float v)
-{
-    auto with = [&](auto ctrl, auto rows) NDC_INLINE {
-        const uint32_t u = __float_as_uint(v);
-        v = __uint_as_float(max(u, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u, decltype(ctrl)::value, decltype(rows)::value, 0xf, true)));
-    };
-    typedef std::integral_constant<int, 0xf> All;
-    with(std::integral_constant<int, 0x111>(), All()), with(std::integral_constant<int, 0x112>(), All());   // row_shr:1, 2
-    with(std::integral_constant<int, 0x114>(), All());                                                      // row_shr:4
-    if constexpr (N == 64) {
-        with(std::integral_constant<int, 0x118>(), All());                                // row_shr:8
-        with(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());   // row_bcast:15 into rows 1 and 3
-        with(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());   // row_bcast:31 into rows 2 and 3
-    }
-    return v;
-}
-// 2^24 times what a sum of k products with factors up to a and b may miss
-__device__ inline float missed(long long k, float a, float b) { return (float)k * 0x1p-100f * (a + b + 1.f); }
-// The smaller of `low` and twice the bits of a value's size less one: zeros are the largest.
-__device__ inline uint32_t lowest(uint32_t low, float v) { return min(low, (__float_as_uint(v) << 1) - 1u); }
-// whether no part and no product of the kept ones is denormal: factors from such values on
-__device__ inline bool exact_from(uint32_t a, uint32_t b)
-{
-    const uint32_t ea = (a + 1u) >> 24, eb = (b + 1u) >> 24;   // (biased exponents)
-    return a == ~0u || b == ~0u || (ea >= 25 && eb >= 25 && ea + eb >= 152);
-}
-// ... of a wavefront's values
-__device__ inline bool wave_exact_from(uint32_t a, uint32_t b)
-{
+    float t = 0.f;
 #pragma unroll
-    for (int o = 1; o < 64; o *= 2) {
-        a = min(a, (uint32_t)__shfl_xor((int)a, o));
-        b = min(b, (uint32_t)__shfl_xor((int)b, o));
-    }
-    return exact_from(a, b);
-}
-// The few small sums of a wavefront, each by the factors it is made of: lanes have `count` of them, the last one's place
-// `at`.  lows(lane, at, a, b): the lowest of this lane's share of those factors.  0: all exact, 1: not, 2: more than
-// a few.
-template <class Lows> __device__ inline int small_sums(int count, int at, Lows lows)
-{
-    uint64_t left = __ballot(count > 0);
-    if (__any(count > 1) || __popcll(left) > 4) return 2;
-    for (; left; left &= left - 1) {
-        const int lane = __ffsll((long long)left) - 1;
-        uint32_t a = ~0u, b = ~0u;
-        lows(lane, __builtin_amdgcn_readlane(at, lane), a, b);
-        if (!wave_exact_from(a, b)) return 1;
-    }
-    return 0;
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) t = __builtin_fmaf(acc[i][j][e], 0.f, t);
+    return !__any(t != 0.f);
 }
 
 // ---------------------------------------------------------------------------- weight gradient
@@ -279,10 +218,10 @@ __global__ void __launch_bounds__(64 * WM * WN, sizeof(T) == 4 ? 2 : 1) wgrad_ke
     const T *A = (const T *)p.a + ((long long)sample * p.rows + m0) * p.n;   // (uniform)
     const T *B = (const T *)p.b + ((long long)sample * p.cols + n0) * p.n;
     const bool want_sums = p.gb != nullptr && n0 == 0;
-    uint32_t sign = F32 && (split & 1) ? 0x80000000u : 0u;   // (of the products, see above)
+    const float scale = F32 && (split & 1) ? -kScale : kScale;   // (of gz, see above)
+    float unscale = split & 1 ? -kUnscale : kUnscale;
     u32x4 ra[NA], rb[NB];
-    float sums[NA], most[NA + NB] = {};   // (float32: the largest values of this thread's rows)
-    __shared__ __attribute__((aligned(16))) float top[F32 ? BM + BN + WM * WN : 1];   // ... of all rows, of a wavefront's of A
+    float sums[NA];
 
     // Rows past the end repeat the last one: what they contribute is never stored.  Addresses are a
     // uniform pointer plus a 32-bit lane offset (the caller keeps a tile's rows below 4 GiB): as
@@ -311,24 +250,23 @@ __global__ void __launch_bounds__(64 * WM * WN, sizeof(T) == 4 ? 2 : 1) wgrad_ke
         for (int i = 0; i < NB; ++i) rb[i] = ragged<T>((const T *)(b + off_b[i]), have);
     };
     auto put = [&](auto parts) NDC_INLINE {
-        auto store = [&](u32x4 *to, int rows, int r, u32x4 g, uint32_t turn, float &m) NDC_INLINE {
+        auto store = [&](u32x4 *to, int rows, int r, u32x4 g, float by) NDC_INLINE {
             if constexpr (decltype(parts)::value) {
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(g[e]);
-                m = largest(m, v);
-                put_parts(to, rows, q, r, v, turn);
+                put_parts(to, rows, q, r, v, by);
             } else {
                 to[slot(rows, q, r)] = g;
             }
         };
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            store(lds, BM, r0 + i * (NT / D), ra[i], sign, most[i]);
+            store(lds, BM, r0 + i * (NT / D), ra[i], scale);
             if (want_sums) sums[i] += G::sum(ra[i]);
         }
 #pragma unroll
-        for (int i = 0; i < NB; ++i) store(lds + BM * LG, BN, r0 + i * (NT / D), rb[i], 0u, most[NA + i]);
+        for (int i = 0; i < NB; ++i) store(lds + BM * LG, BN, r0 + i * (NT / D), rb[i], kScale);
     };
 
     const int lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN, l32 = lane & 31, kb = lane >> 5;
@@ -383,18 +321,11 @@ __global__ void __launch_bounds__(64 * WM * WN, sizeof(T) == 4 ? 2 : 1) wgrad_ke
 #pragma unroll
             for (int j = 0; j < CT; ++j) acc[i][j] = f32x16{};
     };
-    // what the look at the sums reads, with the last stage
-    auto note = [&]() NDC_INLINE {
-        if constexpr (F32) {
-            float rows = 0.f;
-#pragma unroll
-            for (int i = 0; i < NA + NB; ++i) {
-                if (i < NA) rows = __builtin_fmaxf(rows, most[i]);
-                const float m = lanes_largest<D>(most[i]);   // (the lanes of a row)
-                if (q == D - 1) top[i < NA ? r0 + i * (NT / D) : BM + r0 + (i - NA) * (NT / D)] = m;
-            }
-            if (rows = lanes_largest<64>(rows); lane == 63) top[BM + BN + wave] = rows;
-        }
+    auto last = [&](long long k0, auto parts) NDC_INLINE {
+        fetch_ragged(k0);
+        put(parts);
+        __syncthreads();
+        multiply(parts);
     };
     clear();
     const std::bool_constant<F32> parts;
@@ -402,71 +333,24 @@ __global__ void __launch_bounds__(64 * WM * WN, sizeof(T) == 4 ? 2 : 1) wgrad_ke
     if (stages > 0) fetch(k_lo);
     for (int s = 0; s < stages; ++s) {
         put(parts);
-        if (s + 1 == stages) note();
         __syncthreads();
         fetch(k_lo + (long long)(s + 1 < stages ? s + 1 : s) * BK);
         multiply(parts);
         __syncthreads();
     }
-    if (k_lo + (long long)stages * BK < k_hi) {
-        fetch_ragged(k_lo + (long long)stages * BK);
-        put(parts);
-        note();
-        __syncthreads();
-        multiply(parts);
-    }
+    if (k_lo + (long long)stages * BK < k_hi) last(k_lo + (long long)stages * BK, parts);
     if constexpr (F32) {
-        __shared__ int again[WM * WN];
-        float rows = 0.f;
-#pragma unroll
-        for (int w = 0; w < WM * WN; ++w) rows = __builtin_fmaxf(rows, top[BM + BN + w]);
-        float finite = 0.f, least[CT], col[CT];
-        bool small = false;
-#pragma unroll
-        for (int j = 0; j < CT; ++j) {
-            col[j] = top[BM + 32 * (wn * CT + j) + l32];
-            least[j] = __builtin_fabsf(acc[0][j][0]);
-#pragma unroll
-            for (int i = 0; i < RT; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    finite = __builtin_fmaf(acc[i][j][e], 0.f, finite);
-                    least[j] = __builtin_fminf(least[j], __builtin_fabsf(acc[i][j][e]));
-                }
-            small = small || least[j] < missed(k_hi - k_lo, rows, col[j]);
-        }
-        int r = __any(finite != 0.f);
-        if (__builtin_expect(!r && __any(small), 0)) {   // (rows and columns of zeros have sums of zero)
-            int count = 0, at = 0;
-#pragma unroll
-            for (int i = 0; i < RT; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float row = top[32 * (wm * RT + i) + 8 * (e / 4) + 4 * kb + e % 4];
-#pragma unroll
-                    for (int j = 0; j < CT; ++j)
-                        if (__builtin_fabsf(acc[i][j][e]) < missed(k_hi - k_lo, row, col[j]) && __builtin_fminf(row, col[j]) > 0.f)
-                            ++count, at = (32 * (wm * RT + i) + 8 * (e / 4) + 4 * kb + e % 4) << 16 | (32 * (wn * CT + j) + l32);
-                }
-            r = small_sums(count, at, [&](int, int at, uint32_t &a, uint32_t &b) NDC_INLINE {
-                const float *pa = (const float *)A + (long long)min(at >> 16, p.rows - 1 - m0) * p.n;
-                const float *pb = (const float *)B + (long long)min(at & 0xffff, p.cols - 1 - n0) * p.n;
-#pragma unroll 8
-                for (long long k = k_lo + lane; k < k_hi; k += 64) a = lowest(a, pa[k]), b = lowest(b, pb[k]);
-            });
-        }
-        if (lane == 0) again[wave] = r;
+        __shared__ int finite[WM * WN];
+        if (const bool f = all_finite(acc); lane == 0) finite[wave] = f;
         __syncthreads();
+        bool again = false;
 #pragma unroll
-        for (int w = 0; w < WM * WN; ++w) r |= again[w];
-        if (__builtin_expect(r, 0)) {
+        for (int w = 0; w < WM * WN; ++w) again = again || !finite[w];
+        if (__builtin_expect(again, 0)) {
             clear();
-            sign = 0u;
+            unscale = 1.f;
             for (long long k0 = k_lo; k0 < k_hi; k0 += BK) {
-                fetch_ragged(k0);
-                put(std::false_type());
-                __syncthreads();
-                multiply(std::false_type());
+                last(k0, std::false_type());
                 __syncthreads();
             }
         }
@@ -482,7 +366,7 @@ __global__ void __launch_bounds__(64 * WM * WN, sizeof(T) == 4 ? 2 : 1) wgrad_ke
             for (int e = 0; e < 16; ++e) {
                 const int row = m0 + 32 * (wm * RT + i) + 8 * (e / 4) + 4 * kb + e % 4;
                 if (row < p.rows && col < p.cols)
-                    gw[(long long)row * p.cols + col] = F32 ? __uint_as_float(__float_as_uint(acc[i][j][e]) ^ sign) : acc[i][j][e];
+                    gw[(long long)row * p.cols + col] = F32 ? acc[i][j][e] * unscale : acc[i][j][e];
             }
         }
     if (want_sums) {
@@ -897,7 +781,7 @@ __global__ void __launch_bounds__(256, (RT == 2 ? 4 : 5) - CHAINS) parts_kernel(
     constexpr int BM = 32 * RT, BN = 128, BK = 32;
     __shared__ __attribute__((aligned(16))) u32x4 lds[2][BM * 3 * kPartDepth];
     __shared__ __attribute__((aligned(16))) float bias[BM];
-    __shared__ float red[4][BM], top[4];   // (top: the largest value of W that each wavefront met)
+    __shared__ float red[4][BM];
     const int xcd = blockIdx.x & 7, pos = blockIdx.x >> 3;
     const int tile_m = pos % p.tiles_m, vt = (pos / p.tiles_m) * 8 + xcd;   // a voxel tile stays on one XCD
     if (vt >= p.tiles_n * p.batch) return;
@@ -909,8 +793,8 @@ __global__ void __launch_bounds__(256, (RT == 2 ? 4 : 5) - CHAINS) parts_kernel(
     const float *X = (const float *)p.x + (long long)sample * p.cin * p.n + v0;
     // lanes past the end of a row repeat its last voxel, rows past the end the last row: never stored
     const uint32_t xoff = ((uint32_t)(8 * kb) * (uint32_t)p.n + (uint32_t)min(mine, left - 1)) * 4u;
-    const uint32_t sign = (uint32_t)(l32 & 1) << 31;
-    float xr[2][8], rw[RT][4], most_x = 0.f, most_w = 0.f;   // (the largest values met)
+    const float scale = l32 & 1 ? -kScale : kScale;
+    float xr[2][8], rw[RT][4];
     auto weight_at = [&](int i, int &r, int &q) NDC_INLINE {   // granule i of this thread
         const int g = tid + i * 256;
         if (WT) r = g % BM, q = g / BM;   // lanes along the rows of W, contiguous in W^T
@@ -957,37 +841,40 @@ __global__ void __launch_bounds__(256, (RT == 2 ? 4 : 5) - CHAINS) parts_kernel(
     };
     f32x16 acc[RT][1];
     u32x4 xp[2][1][3];
-    auto put = [&](u32x4 *to) NDC_INLINE {
+    // halves: 2, or 1 in a last stage of 16 channels and fewer (us, 16 -> 64 over 98 x 1000 voxels 13.8 with both, 12.5 with one;
+    // with 32 rows the choice costs registers that are not there, 22 -> 29 for 32 channels)
+    auto put = [&](u32x4 *to, int halves) NDC_INLINE {
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
             int r, q;
             weight_at(i, r, q);
-            most_w = largest(most_w, rw[i]);
-            put_parts(to, BM, q, r, rw[i], 0u);
+            put_parts(to, BM, q, r, rw[i], kScale);
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t) {
+            if (t >= halves) continue;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = xr[t][4 * h + e];
-                most_x = largest(most_x, v);
+                for (int e = 0; e < 4; ++e) v[e] = xr[t][4 * h + e] * scale;
 #pragma unroll
                 for (int o = 0; o < 3; ++o) {
-                    const u32x2 w = o ? next_part(v) : first_part(v, sign);
+                    const u32x2 w = next_part(v);
                     xp[t][0][o][2 * h] = w[0], xp[t][0][o][2 * h + 1] = w[1];
                 }
             }
+        }
     };
-    auto multiply = [&](const u32x4 *from) NDC_INLINE {
+    auto multiply = [&](const u32x4 *from, int halves) NDC_INLINE {
         f32x16 sum[RT];
         if constexpr (!CHAINS) {
 #pragma unroll
             for (int i = 0; i < RT; ++i) sum[i] = acc[i][0];
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < 2; ++t) {
+            if (t >= halves) continue;
 #pragma unroll
             for (int o = 2; o >= 0; --o) {   // the least terms first
                 u32x4 fa[RT];
@@ -999,74 +886,31 @@ __global__ void __launch_bounds__(256, (RT == 2 ? 4 : 5) - CHAINS) parts_kernel(
                     for (int i = 0; i < RT; ++i)
                         sum[i] = Gran<bf16_t>::mma(fa[i], xp[t][0][b], CHAINS && t == 0 && o == 2 ? f32x16{} : sum[i]);
             }
+        }
 #pragma unroll
         for (int i = 0; i < RT; ++i) acc[i][0] = CHAINS ? acc[i][0] + sum[i] : sum[i];
     };
 #pragma unroll
     for (int i = 0; i < RT; ++i) acc[i][0] = f32x16{};
     for (int r = tid; r < BM; r += 256) bias[r] = p.bias && m0 + r < p.cout ? p.bias[m0 + r] : 0.f;
-    auto note = [&]() NDC_INLINE {   // what the look at the sums reads, with the last stage
-        if (const float m = lanes_largest<64>(most_w); lane == 63) top[wave] = m;
-    };
     const int stages = p.cin / BK;
     if (stages > 0) fetch(0);
     for (int s = 0; s < stages; ++s) {
-        put(lds[s & 1]);
-        if ((s + 1) * BK == p.cin) note();
+        put(lds[s & 1], 2);
         __syncthreads();
         if (s + 1 < stages) fetch((s + 1) * BK);
-        multiply(lds[s & 1]);
+        multiply(lds[s & 1], 2);
     }
     if (stages * BK < p.cin) {
         fetch_ragged(stages * BK);
-        put(lds[stages & 1]);
-        note();
+        const int halves = RT == 2 && p.cin - stages * BK <= 16 ? 1 : 2;
+        put(lds[stages & 1], halves);
         __syncthreads();
-        multiply(lds[stages & 1]);
+        multiply(lds[stages & 1], halves);
     }
-    most_x = __builtin_fmaxf(most_x, __shfl_xor(most_x, 32));   // (of this lane's voxel; a voxel of zeros has sums of zero)
-    most_w = __builtin_fmaxf(__builtin_fmaxf(top[0], top[1]), __builtin_fmaxf(top[2], top[3]));
-    const float counts = __builtin_fminf(most_x, most_w) > 0.f ? missed(p.cin, most_x, most_w) : 0.f;
-    float finite = 0.f, least = __builtin_fabsf(acc[0][0][0]);
-#pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            finite = __builtin_fmaf(acc[i][0][e], 0.f, finite);
-            least = __builtin_fminf(least, __builtin_fabsf(acc[i][0][e]));
-        }
-    bool again = __any(finite != 0.f);
-    if (__builtin_expect(!again && __any(least < counts), 0)) {   // such sums come about by cancellation too: what values are there?
-        int count = 0, at = 0;
-#pragma unroll
-        for (int i = 0; i < RT; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (__builtin_fabsf(acc[i][0][e]) < counts) ++count, at = 32 * i + 8 * (e / 4) + 4 * kb + e % 4;
-        auto weight = [&](int row, int k) NDC_INLINE {
-            const int m = min(m0 + row, p.cout - 1);
-            return p.w[WT ? (long long)k * p.cout + m : (long long)m * p.cin + k];
-        };
-        int r = small_sums(count, at, [&](int from, int row, uint32_t &a, uint32_t &b) NDC_INLINE {
-            const float *x = X + min(32 * wave + (from & 31), left - 1);
-#pragma unroll 4
-            for (int k = lane; k < p.cin; k += 64) a = lowest(a, x[(long long)k * p.n]), b = lowest(b, weight(row, k));
-        });
-        if (r == 2) {
-            uint32_t low_x = ~0u, low_w = ~0u;
-#pragma unroll 4
-            for (int k = kb; k < p.cin; k += 2) {
-                low_x = lowest(low_x, X[(long long)k * p.n + min(mine, left - 1)]);
-#pragma unroll
-                for (int i = 0; i < RT; ++i) low_w = lowest(low_w, weight(32 * i + l32, k));
-            }
-            r = !wave_exact_from(low_x, low_w);
-        }
-        again = r != 0;
-    }
-    uint32_t turn = sign;
-    if (__builtin_expect(again, 0)) {
-        turn = 0u;
+    float unscale = l32 & 1 ? -kUnscale : kUnscale;
+    if (__builtin_expect(!all_finite(acc), 0)) {
+        unscale = 1.f;
 #pragma unroll
         for (int i = 0; i < RT; ++i) acc[i][0] = f32x16{};
         for (int k0 = 0; k0 < p.cin; k0 += 2) {
@@ -1104,7 +948,7 @@ __global__ void __launch_bounds__(256, (RT == 2 ? 4 : 5) - CHAINS) parts_kernel(
                 }
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float z = __uint_as_float(__float_as_uint(acc[i][0][8 * h + e]) ^ turn);
+                    const float z = acc[i][0][8 * h + e] * unscale;
                     float y;
                     if constexpr (MODE == kGeluGrad) {
                         y = z * epilogue::act_grad<epilogue::kGelu>(rv[e] + bv[e]);

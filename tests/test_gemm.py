@@ -188,6 +188,23 @@ def test_parts_of_values_of_very_different_sizes(voxels, rows, weight):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("one,size,weight", [(3.4e38, 0, -100), (3.4e38, -120, -20), (1.0, 64, 56), (1.0, 50, 64)])
+def test_parts_of_values_near_the_largest(one, size, weight):
+    """A value that rounds to an infinite bf16, beside others and small weights, and products of which a few sums would pass
+    the largest float32 on the way."""
+    print("case", one, size, weight, flush=True)
+    lib, (x, _, _, g), w, _ = _setup("cuda", (2, 72, 130, 20003), torch.float32)
+    x *= 2.0 ** size
+    x[0, 3, 7] = one
+    w *= 2.0 ** weight
+    g *= 2.0 ** (weight - 8)
+    for y in (ops.gemm(lib, x, w)[0], ops.gemm(lib, x, w.t().contiguous(), transposed=True)[0]):
+        _each_within(y, w, x)
+    gw, _ = ops.weight_grad(lib, g, x)
+    _each_within(gw, g.transpose(0, 1).flatten(1), x.transpose(0, 1).flatten(1).t())
+
+
+@pytest.mark.gpu
 def test_parts_of_values_that_are_not_finite():
     """What a float32 product makes of infinities, NaN and values beyond the range of bf16: an infinity's column is
     infinite by the weight's sign, the rest finite."""
