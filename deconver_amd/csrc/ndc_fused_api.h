@@ -270,16 +270,17 @@ static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, cons
 }
 
 // Column pairs of rows of any length and alignment, where they are ahead of one column a thread.
-// 3-D: where the cost of their launch says so.  The times of 141 problems (3 to 255 columns, 1 to 1024 channels, 0.1 to 10 M
-// voxels) follow the ratio of the two costs.  Forward, 2 x 2 outputs a thread against 4 x 1: a pair's thread takes 1.02 to
-// 1.09 times as long (a lone wavefront up to 1.03), workgroups of three wavefronts 1.12 times what they are counted as; so
-// pairs below 0.93 (0.965) of the cost.  us, one column -> pairs, float32 / bf16, with that ratio: 192 channels of
-// 23 x 29 x 33 161 -> 99 / 162 -> 99, 0.60; 32 of 55 x 61 x 129 559 -> 371 / 563 -> 364, 0.79; 32 of 91 x 101 x 87 643 -> 585 /
-// 661 -> 582, 0.85; 2 of 104 x 100 x 61 60 -> 55 / 60 -> 56, 0.92; 64 of 45 x 53 x 77 299 -> 300 / 306 -> 319, 0.94; 1024 of
-// 6 x 3 x 7 44 -> 94 / 42 -> 95, 1.00; 16 of 106 x 82 x 73 245 -> 255 / 245 -> 274, 1.06.  Taken, the most behind are 384 of
-// 10 x 30 x 19 (87 -> 91) and 1 of 160 x 157 x 151 (122 -> 123 / 119 -> 126).  Backward, 2 x 2 outputs against 2 x 1: 1.4 (few
-// wavefronts) to 2 times (many), so below 0.54 (1 of 143 x 135 x 135 167 -> 155 / 166 -> 143, 0.49; 64 of 45 x 53 x 77
-// 547 -> 541 / 526 -> 498, 0.52; 1 of 160 x 90 x 159 134 -> 149 / 132 -> 137, 0.65; 8 of 22 x 19 x 41 62 -> 86 / 61 -> 84, 0.94).
+// 3-D: where the cost of their launch says so.  The times of 200 problems (3 to 255 columns, 1 to 1024 channels, 0.1 to 10 M
+// voxels) follow the ratio of the two costs.  Forward, 2 x 2 outputs a thread against 4 x 1: pairs in workgroups of up to three
+// wavefronts are ahead up to 0.978 of the cost (of 56 problems between 0.93 and that 0.96 of the time, the most behind 1.02),
+// in larger ones, whose threads take 1.02 to 1.09 times as long, up to 0.93; workgroups of three wavefronts count 1.12
+// times.  us, one column -> pairs, float32 / bf16, with that ratio: 192 channels of 23 x 29 x 33 161 -> 99 / 162 -> 99, 0.60; 32
+// of 55 x 61 x 129 559 -> 371 / 563 -> 364, 0.79; 32 of 91 x 101 x 87 643 -> 585 / 661 -> 582, 0.85; 256 of 32 x 31 x 39
+// 226 -> 210, 0.94; 768 of 21 x 24 x 25 279 -> 261, 0.97; 64 of 45 x 53 x 77 299 -> 300 / 306 -> 319, 0.94 with four
+// wavefronts; 1024 of 6 x 3 x 7 44 -> 94 / 42 -> 95, 1.00; 16 of 106 x 82 x 73 245 -> 255 / 245 -> 274, 1.06.  Backward, 2 x 2
+// outputs against 2 x 1: 1.4 (few wavefronts) to 2 times (many), so below 0.549 (1 of 143 x 135 x 135 167 -> 155 / 166 -> 143,
+// 0.49; 64 of 45 x 53 x 77 547 -> 541 / 526 -> 498, 0.52; 256 of 32 x 31 x 39 493 -> 438, 0.545; 32 of 63 x 71 x 81
+// 522 -> 543, 0.550; 1 of 160 x 90 x 159 134 -> 149 / 132 -> 137, 0.65; 8 of 22 x 19 x 41 62 -> 86 / 61 -> 84, 0.94).
 // Not tried below 32 columns; past 192 of them pairs leave the backward one workgroup a CU (64 of 30 x 41 x 255 857 -> 1073 /
 // 782 -> 949).
 // 2-D: where they halve the wavefronts across a row, from 193 columns on (two for four; 161 columns, two for three, forward
@@ -321,10 +322,10 @@ static inline LoosePairs loose_pairs(const KGeom &q, const March &m)
     if (l.forward) {
         double r = ratio(FwdKernel<3, 3, 3, 4, 4, 1, float>(), FwdKernel<3, 3, 3, 4, 2, -2, float>(), 4, targets_f, kCostFmaF, a, b);
         if (r > 0 && r < 2) r *= (b.NT == 192 ? 1.12 : 1.0) / (a.NT == 192 ? 1.12 : 1.0);
-        l.forward = r < (r > 0 && a.NT == 64 && b.NT == 64 ? 0.965 : 0.93);
+        l.forward = r < (r > 0 && b.NT <= 192 ? 0.978 : 0.93);
     }
     if (l.backward)
-        l.backward = ratio(Bwd1Kernel<3, 3, 3, 4, 2, 1, float>(), Bwd1Kernel<3, 3, 3, 4, 2, -2, float>(), 2, targets_b, kCostFmaB, a, b) < 0.54;
+        l.backward = ratio(Bwd1Kernel<3, 3, 3, 4, 2, 1, float>(), Bwd1Kernel<3, 3, 3, 4, 2, -2, float>(), 2, targets_b, kCostFmaB, a, b) < 0.549;
     return l;
 }
 
@@ -454,7 +455,7 @@ static inline bool make_plan_fresh(const KGeom &q, Plan &pl, bool pairs_ok, int 
 }
 
 // A plan is a function of sizes, and a forward and a backward ask for it some ten times (what is
-// supported, workspace sizes, the launches); the search for a launch shape takes 1-2 us.  Each thread
+// supported, workspace sizes, the launches); the search for a launch shape takes 1-5 us.  Each thread
 // keeps the plans of the last sizes it saw: an update of 64 channels of 32^3 plans for 2 us in all
 // instead of 25, which a small layer waits for.
 static inline bool make_plan(const KGeom &q, Plan &pl, bool pairs_ok = true, int dtype = NDC_F32, bool matrix = false)

@@ -122,6 +122,16 @@ def test_columns_a_thread_makes(C, ks, sp, aligned, forward, backward):
     assert (f.value, b.value) == (forward, backward)
 
 
+# ... near the lines in 3-D: workgroups of two, three and four wavefronts of pairs, the backward either side of its own
+NEAR = [(256, (3, 3, 3), (32, 31, 39), True, -2, -2), (768, (3, 3, 3), (21, 24, 25), True, -2, 1),
+        (32, (3, 3, 3), (63, 71, 81), True, 1, 1), (512, (3, 3, 3), (26, 28, 31), True, 1, 1)]
+
+
+@pytest.mark.parametrize("C,ks,sp,aligned,forward,backward", NEAR)
+def test_columns_near_the_lines(C, ks, sp, aligned, forward, backward):
+    test_columns_a_thread_makes(C, ks, sp, aligned, forward, backward)
+
+
 @pytest.mark.parametrize("geom", FUSED_GEOMS)
 @pytest.mark.parametrize("relu,with_bias", [(True, True), (False, False)])
 def test_fused_forward_backward_fp32(geom, relu, with_bias):
