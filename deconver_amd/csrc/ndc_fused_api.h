@@ -289,7 +289,10 @@ static inline bool cost_tile(const March &m, int RH, int RW, long long nbc, cons
 // up to 512, from 2 M pixels on (3x3: 64 of 442 x 383 357 -> 339 / 357 -> 282, 8 of 378 x 499 53 -> 60 / 53 -> 52; 5x5: 64 of
 // 151 x 223 114 -> 105 / 114 -> 98, 32 of 184 x 201 81 -> 85 / 81 -> 83); of 5x5 rows of 257 to 384 columns, where one column a
 // thread takes five or six wavefronts, any (16 of 226 x 271 132 -> 94 / 132 -> 89), wider ones where segments of eight rows make
-// 2048 wavefronts of four a row (16 of 270 x 401 184 -> 105 / 184 -> 98, 8 of 378 x 499 85 -> 105 / 85 -> 99).
+// 2048 wavefronts of four a row (16 of 270 x 401 184 -> 105 / 184 -> 98, 8 of 378 x 499 85 -> 105 / 85 -> 99).  Not where
+// their segments end in a round that is nearly empty: rounds over segments below 0.6 (3x3: 0.9) of the single columns' (5x5,
+// 256 of 207 x 199, 1/4 and 1/2: 476 -> 390 / 470 -> 367, 512 914 -> 730 / 897 -> 686, but 384, 2/3 and 1: 582 -> 701 /
+// 576 -> 656; 3x3, 384 of 200 x 271, 1 and 1: 617 -> 642 / 413 -> 471).
 // (Rows that one column a thread cannot take stay outside.)
 // (true in a host build whose tests send every row they can down these kernels)
 #ifndef NDC_LOOSE_EVERYWHERE
@@ -304,6 +307,17 @@ static inline LoosePairs loose_pairs(const KGeom &q, const March &m)
         LoosePairs l = {m.W > 192 && m.W <= 256 && (m.KW == 3 || pixels >= 4000 * 1000), m.W > 192 && m.W <= 512};
         if (m.KW == 3 || m.W <= 256) l.backward = l.backward && pixels >= 2000 * 1000;
         else if (m.W > 384) l.backward = l.backward && nbc * 4 * (m.D / 8) >= 2048;
+        if (m.KW == 3 || m.W <= 256) {
+            // rounds of the wavefronts that are resident, a segment of the march each
+            auto rounds = [&](int RW) {
+                Tile t;
+                if (!make_tile(m, 1, RW, tn.threads_b, t)) return 0.0;
+                split_march(m, nbc * t.ntile, t, kSplitWavesB);
+                return (double)((nbc * t.ntile * t.nseg * (t.NT / 64) + kSplitWavesB - 1) / kSplitWavesB) / t.nseg;
+            };
+            const double single = rounds(1);
+            l.backward = l.backward && (single == 0.0 || rounds(-2) < (m.KW == 3 ? 0.9 : 0.6) * single);
+        }
         if (NDC_LOOSE_EVERYWHERE) l = {m.W >= 128 && m.W <= 256, m.W >= 128 && m.W <= 512};
         return l;
     }

@@ -122,9 +122,12 @@ def test_columns_a_thread_makes(C, ks, sp, aligned, forward, backward):
     assert (f.value, b.value) == (forward, backward)
 
 
-# ... near the lines in 3-D: workgroups of two, three and four wavefronts of pairs, the backward either side of its own
+# ... near the lines: in 3-D workgroups of two, three and four wavefronts of pairs, the backward either side of its own
 NEAR = [(256, (3, 3, 3), (32, 31, 39), True, -2, -2), (768, (3, 3, 3), (21, 24, 25), True, -2, 1),
-        (32, (3, 3, 3), (63, 71, 81), True, 1, 1), (512, (3, 3, 3), (26, 28, 31), True, 1, 1)]
+        (32, (3, 3, 3), (63, 71, 81), True, 1, 1), (512, (3, 3, 3), (26, 28, 31), True, 1, 1),
+        # ... and in 2-D, where a last round of wavefronts is full and where it is nearly empty
+        (256, (5, 5), (207, 199), True, -2, -2), (384, (5, 5), (207, 199), True, -2, 1), (512, (5, 5), (207, 199), True, -2, -2),
+        (384, (5, 5), (200, 271), True, 1, -2), (384, (3, 3), (207, 199), True, -2, -2), (384, (3, 3), (200, 271), True, 1, 1)]
 
 
 @pytest.mark.parametrize("C,ks,sp,aligned,forward,backward", NEAR)
